@@ -652,6 +652,27 @@ void dgd_fused_forward_f32_cuda(float *k_mem, const float *v_mem, float *q_mem, 
  * cache [cache_len, heads*hd]; q, out [1, heads*hd]; no weights are kept. */
 void swa_single_token_cuda(const uint16_t *q, const uint16_t *k_cache, const uint16_t *v_cache, uint16_t *out,
                            int cache_len, int num_heads, int head_dim, int window_size, int n_persistent);
+/* One whole decode step (core/src/gpu_forward.rs:3377-3492 gpu_single_token_forward) in four launches: projections of
+ * the embedded token, K and V rounded into row `pos` of the bf16 caches [max_len, d], attention over the cache, every
+ * level's one-token step on its carried memory, combine, gate, output projection and unembedding.  Blocks until the
+ * logits are on the host.  Head size 32, 64 or 128, d <= 4096, at most 8 levels.  Returns 0 on success.
+ *   embedding_row [d]; w_* [d, d]; w_unembed [d, vocab]
+ *   level_ptrs    host array, 8 device pointers per level: w_k, w_v, w_q, w_alpha, b_alpha, w_theta, b_theta,
+ *                 memory [heads, hd*hd] (updated in place for an active level)
+ *   level_rule    host array: -1 frozen (y = M q with the raw projection), 0 Hebbian, 1 Delta or Titans (zero
+ *                 momentum at the start of a call), 2 DGD
+ *   level_bounds  host array, 6 per level: alpha floor / ceil, theta floor / ceil, error_clip, m_norm_max
+ *   work          device floats, decode_work_floats_rocm(...) of them
+ *   workspace     host array of 7 device buffers that receive the step's intermediates: embedded [d] f32, q [d] bf16,
+ *                 attention output [d] bf16 and [d] f32, y_combined, gate, gated [d] f32
+ *   logits [vocab] device, logits_host [vocab] pinned host memory */
+int decode_work_floats_rocm(int d, int heads, int levels, int window, int n_persistent);
+int decode_token_rocm(const float *embedding_row, const float *w_q, const float *w_k, const float *w_v, const float *w_o,
+                      const float *w_unembed, const void *const *level_ptrs, const int *level_rule,
+                      const float *level_bounds, int levels, int d, int heads, int vocab, int window, int n_persistent,
+                      int pos, uint16_t *k_cache, uint16_t *v_cache, float *work, void *const *workspace, float *logits,
+                      float *logits_host);
+
 /* Phase-2 kernels of the split chunkwise path (core/src/cuda_ffi.rs:407-453): the recurrence /
  * reverse sweep of chunk `chunk_idx` with the chunk's errors [batch, chunk_size, d] supplied by
  * the caller.  Forward: m_work / s_work [batch, d*d] are the running state (in/out); slot

@@ -11,6 +11,7 @@ libnl_hecate_rocm.so or a torch matmul in the place of the reference's cuBLAS ca
 the token ids in and the logits out, as in the reference.
 """
 import ctypes
+import operator
 from dataclasses import dataclass, field
 from typing import List
 
@@ -130,6 +131,95 @@ class DecodeWorkspace:
         self.attn_out = _zeros(1, d)
         self.y_combined, self.gate, self.gated_out = _zeros(1, d), _zeros(1, d), _zeros(1, d)
         self.logits_gpu = _zeros(1, v)
+        # what the library's one-call step writes: intermediates of its launches, and the logits where the host reads them
+        self.work = _new(0)
+        self.plans = {}
+        self.logits_host = torch.empty(v, dtype=torch.float32, pin_memory=True)
+        self.outputs = (ctypes.c_void_p * 7)(*[t.data_ptr() for t in (
+            self.embedded, self.q_bf16, self.attn_out_bf16, self.attn_out, self.y_combined, self.gate, self.gated_out)])
+
+    def work_for(self, floats):
+        if self.work.numel() < floats:
+            self.work = _new(floats)
+            self.plans.clear()   # they hold the old buffer's address
+        return self.work
+
+
+# level_rule of decode_token_rocm; a Titans level starts every call with zero momentum, so its one-token step is Delta's
+_DECODE_RULE = {"hebbian": 0, "delta": 1, "titans": 1, "dgd": 2}
+
+
+def _decode_plan(params, cfg, active, context, kv_cache, ws, tensors):
+    """The argument block of the one-call step, or None for a model that it does not cover (MLP memories, SwiGLU, other
+    head sizes): those take the step below, operation by operation."""
+    d, nh, hd, v, k = cfg.d_model, cfg.num_heads, cfg.head_dim, cfg.vocab_size, cfg.k
+    if (hd not in (32, 64, 128) or nh * hd != d or d > 4096 or not 1 <= k <= 8 or kv_cache._scratch_k.numel() < d
+            or kv_cache.d != d or ws.logits_host.numel() != v):
+        return None
+    square, vectors = [params.w_q, params.w_k, params.w_v, params.w_o], []
+    rules, bounds = [], []
+    for lv in range(k):
+        lc, lp, mem = cfg.levels[lv], params.levels[lv], context.memory[lv]
+        rule = _DECODE_RULE.get(lc.memory_rule)
+        if rule is None or lc.memory_layers != 1 or (lc.num_heads, lc.head_dim) != (nh, hd):
+            return None
+        if mem.shape != (nh, hd * hd) and (active[lv] or mem[:nh].numel() != nh * hd * hd):
+            return None
+        rules.append(rule if active[lv] else -1)
+        bounds += (lc.alpha_floor, lc.alpha_ceil, lc.theta_floor, lc.theta_ceil, lc.error_clip, lc.m_norm_max)
+        square += (lp.w_k, lp.w_v, lp.w_q)
+        vectors += (lp.w_alpha, lp.w_theta)
+    if (any(t.shape != (d, d) for t in square) or any(t.numel() != 2 * d for t in vectors)
+            or params.w_unembed.shape != (d, v) or params.w_embed.shape != (v, d)):
+        return None
+    for t in tensors:   # contiguous floats; all but the scalar biases are read in 16-byte pieces
+        if t.dtype is torch.bfloat16:
+            continue
+        if t.dtype != torch.float32 or not t.is_cuda or not t.is_contiguous() or (t.numel() > 1 and t.data_ptr() & 15):
+            return None
+    work = ws.work_for(lib.decode_work_floats_rocm(d, nh, k, cfg.window_size, cfg.n_persistent))
+    ptrs = [t.data_ptr() for t in tensors]
+    weights = ptrs[1:6]
+    level_args = ((ctypes.c_void_p * (8 * k))(*ptrs[8:]), (ctypes.c_int * k)(*rules), (ctypes.c_float * (6 * k))(*bounds))
+    tail = (kv_cache.k_cache_bf16.data_ptr(), kv_cache.v_cache_bf16.data_ptr(), work.data_ptr(), ws.outputs,
+            ws.logits_gpu.data_ptr(), ws.logits_host.data_ptr())
+    return weights, level_args, tail
+
+
+def _decode_in_one_call(params, cfg, token_id, pulse, context, kv_cache, ws):
+    """The whole step as one library call -> logits, or None (see _decode_plan).  Checking some forty tensors and level
+    options costs as much as the step's kernels, so the workspace keeps the argument blocks together with what they were
+    made from (addresses, options, pulse) and makes one again when any of it has changed."""
+    k = cfg.k
+    levels, lcfgs = params.levels, cfg.levels
+    tensors = [params.w_embed, params.w_q, params.w_k, params.w_v, params.w_o, params.w_unembed, kv_cache.k_cache_bf16,
+               kv_cache.v_cache_bf16]
+    key = [cfg.d_model, cfg.num_heads, cfg.head_dim, cfg.vocab_size, cfg.window_size, cfg.n_persistent]
+    for lv in range(k):
+        lp, lc = levels[lv], lcfgs[lv]
+        if not hasattr(lp, "w_alpha"):
+            return None
+        tensors += (lp.w_k, lp.w_v, lp.w_q, lp.w_alpha, lp.b_alpha, lp.w_theta, lp.b_theta, context.memory[lv])
+        key += (lc.memory_rule, lc.memory_layers, lc.num_heads, lc.head_dim, lc.alpha_floor, lc.alpha_ceil, lc.theta_floor,
+                lc.theta_ceil, lc.error_clip, lc.m_norm_max)
+    active = tuple(map(bool, pulse.active_levels[:k]))
+    key += map(torch.Tensor.data_ptr, tensors)
+    made_for, plan = ws.plans.get(active, (None, None))
+    # the same tensor objects at the same addresses: their shapes and types are the ones that were checked
+    if made_for is None or made_for[0] != key or not all(map(operator.is_, made_for[1], tensors)):
+        plan = _decode_plan(params, cfg, active, context, kv_cache, ws, tensors)
+        if len(ws.plans) >= 16:
+            ws.plans.clear()
+        ws.plans[active] = ((key, tensors), plan)
+    if plan is None:
+        return None
+    weights, level_args, tail = plan
+    rc = lib.decode_token_rocm(key[6 + 10 * k] + 4 * cfg.d_model * token_id, *weights, *level_args, k, cfg.d_model,
+                               cfg.num_heads, cfg.vocab_size, cfg.window_size, cfg.n_persistent, kv_cache.len, *tail)
+    if rc:
+        raise RuntimeError(f"decode_token_rocm failed ({rc})")
+    kv_cache.len += 1
+    return ws.logits_host.numpy().copy()
 
 
 def _memory_read_only(lp, embedded, memory, n, nh, hd):
@@ -214,6 +304,9 @@ def gpu_single_token_forward(params: GpuMAGParams, cfg: ServeConfig, token_id, p
         raise RuntimeError("KV cache must be populated via prefill first")
     if kv_cache.len >= kv_cache.max_len:
         raise OverflowError(f"KV cache full: {kv_cache.len} >= {kv_cache.max_len}")
+    logits = _decode_in_one_call(params, cfg, token_id, pulse, context, kv_cache, ws)
+    if logits is not None:
+        return logits
     ws.d_input.copy_(torch.tensor([token_id], dtype=torch.int32))
     D.call("embedding_gather_cuda", params.w_embed, ws.d_input, ws.embedded, 1, d)
     q_f32, k_f32, v_f32 = (ws.embedded @ w.t() for w in (params.w_q, params.w_k, params.w_v))

@@ -1,0 +1,58 @@
+"""The one-call decode step (decode_token_rocm) at the edges of its kernels: every head size it serves, windows that end
+on and off an attention slice of 128 keys, an odd vocabulary, a persistent prefix, clamps, clip and norm bound, against
+the CPU composition of the same step (oracle/serving.py)."""
+import types
+
+import numpy as np
+import pytest
+
+from nl_hecate_amd import serving as SG
+from nl_hecate_amd.cms import ContextState, Pulse
+from nl_hecate_amd.ffi import lib
+from nl_hecate_amd.memory_level import LevelConfig
+from oracle import serving as SV
+from tests.gpu_util import assert_close, dev, host
+from tests.test_gpu_serving import gpu_params, model
+
+pytestmark = pytest.mark.gpu
+f32 = np.float32
+
+CASES = [  # rule, active, n_persistent, heads, head size, window, prompt, tokens, vocab, level options
+    ("titans", [True, True, False], 0, 2, 64, 128, 126, 4, 64, {}),
+    ("delta", [True, False], 0, 3, 32, 130, 140, 3, 37, dict(m_norm_max=0.5, error_clip=0.1)),
+    ("titans", [True], 3, 1, 128, 257, 300, 2, 1000, dict(alpha_floor=0.2, theta_ceil=0.03, m_norm_max=0.7)),
+    ("hebbian", [False, True], 0, 2, 32, 7, 5, 4, 4, dict(m_norm_max=0.9)),
+    ("dgd", [True, True, True, False], 1, 4, 64, 16, 1, 3, 130, dict(m_norm_max=1.0, error_clip=0.5)),
+]
+
+
+@pytest.mark.parametrize("rule,active,n_p,nh,hd,window,s,extra,v,opts", CASES)
+def test_one_call_step(rule, active, n_p, nh, hd, window, s, extra, v, opts):
+    print(rule, nh, hd, window, s, v, flush=True)
+    d, k = nh * hd, len(active)
+    p = model(d, v, k, 91 + hd)
+    lcfgs = [LevelConfig(rule, nh, hd, **opts) for _ in range(k)]
+    ocfg = types.SimpleNamespace(d_model=d, num_heads=nh, head_dim=hd, window_size=window, n_persistent=n_p, levels=lcfgs)
+    cfg = SG.ServeConfig(d, v, nh, hd, window, s, lcfgs, n_persistent=n_p, decode_tokens=extra)
+    r = np.random.default_rng(7)
+    ids = r.integers(0, v, s + extra)
+    mem0 = [(0.2 * r.standard_normal((nh, hd, hd))).astype(f32) for _ in range(k)]
+    gp, pulse = gpu_params(p), Pulse(0, list(active))
+    ctx = ContextState([dev(m.reshape(nh, hd * hd)) for m in mem0])
+    _, kv = SG.gpu_prefill_forward(gp, cfg, ids, pulse, ctx)
+    want, mem, kc, vc = SV.forward_all(p, ocfg, ids[:s], active, mem0)
+    scale = np.abs(want).max()
+    ws = SG.DecodeWorkspace(d, v)
+    lib.nlh_kernel_timer_enable(1)
+    for i in range(extra):
+        step = SG.gpu_single_token_forward(gp, cfg, int(ids[s + i]), pulse, ctx, kv, ws)
+        ref, mem, kc, vc = SV.single_token(p, ocfg, int(ids[s + i]), active, mem, kc, vc)
+        assert np.abs(step - ref).max() <= 2e-2 * scale, i     # attention storage in bf16, as the other decode tests
+        assert np.array_equal(host(ws.logits_gpu)[0], step)
+    import ctypes
+    buf = ctypes.create_string_buffer(4096)
+    lib.nlh_kernel_timer_report(buf, 4096)
+    lib.nlh_kernel_timer_enable(0)
+    assert f"decode_logits_kernel:{extra}:".encode() in buf.value, buf.value
+    for lv in range(k):
+        assert_close(f"memory[{lv}]", host(ctx.memory[lv]).reshape(mem[lv].shape), mem[lv], 1e-4)
