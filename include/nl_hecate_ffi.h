@@ -292,13 +292,15 @@ void delta_backward_ckpt_replay_f32_rocm(const float *k_mem, const float *v_mem,
                                          int seq_len, int d, int batch_size, int checkpoint_interval,
                                          float error_clip, float m_norm_max);
 /* One call over all segments (the loop of core/src/gpu_backward.rs:1770-1962 inside the library).  Three forms, chosen
- * per call: (1) head size 64, checkpoint_interval <= 64: the rule in chunk-parallel matrix form on the fp32 matrix
+ * per call: (1) head size 64 or 32, checkpoint_interval <= 64: the rule in chunk-parallel matrix form on the fp32 matrix
  * cores (a triangular solve per segment, an adjoint scan over the segments, gradients per segment), taken where a cost
  * model says it beats (2) at the call's shape (long intervals, or few chains); (2) the fused form: the replayed
  * trajectory stays in LDS and registers (two-level recomputation inside one kernel), checkpoint_interval <= 64;
  * (3) the `_replay_` schedule.  With a finite m_norm_max (1) and (2) end with a device-side test that the bound
  * could not have been reached and leave the call to (3) when it could; with an error clip (1) does the same and
- * (2) is not used. */
+ * (2) is not used.
+ * checkpoint_interval = 1 takes the full trajectory [batch, seq_len+1, d*d] of a forward that ran under these bounds:
+ * form (1), or the reverse sweep of *_backward_f32_cuda. */
 void titans_backward_ckpt_f32_rocm(const float *k_mem, const float *v_mem, const float *q_mem,
                                    const float *alpha, const float *theta, const float *eta,
                                    const float *m_ckpt, const float *s_ckpt, const float *d_y,

@@ -47,9 +47,8 @@ struct FirstSum {
     const float *src[2];   // [batch][chain_stride]: gradient of the initial M / S per chain
     float *tmp;            // [nsum][rows][d*d]
     size_t chain_stride;
-    int batch, per, rows, nsum;
+    int batch, per, rows, nsum, elems;   // elems = d*d, a multiple of 256
 };
-constexpr int kSumElems = 64 * 64;
 
 template <bool HAS_S>
 __global__ __launch_bounds__(64 * kGateWaves) void cw_gates_sweep_kernel(
@@ -58,13 +57,12 @@ __global__ __launch_bounds__(64 * kGateWaves) void cw_gates_sweep_kernel(
     float *__restrict__ d_eta, int s, int C, int nc, int ntask, int sweep_blocks, FirstSum fs) {
     extern __shared__ float smem[];
     if ((int)blockIdx.x >= sweep_blocks) {
-        const int bid = blockIdx.x - sweep_blocks, eb = bid % (kSumElems / 256), y = (bid / (kSumElems / 256)) % fs.rows,
-                  z = bid / ((kSumElems / 256) * fs.rows);
+        const int bid = blockIdx.x - sweep_blocks, nb = fs.elems / 256, eb = bid % nb, y = (bid / nb) % fs.rows, z = bid / (nb * fs.rows);
         const float *st = fs.src[z];
         const int e = eb * 256 + threadIdx.x, b0 = y * fs.per, b1 = min(fs.batch, b0 + fs.per);
         float x = 0.f;
         for (int b = b0; b < b1; b++) x += st[(size_t)b * fs.chain_stride + e];
-        fs.tmp[((size_t)z * fs.rows + y) * kSumElems + e] = x;
+        fs.tmp[((size_t)z * fs.rows + y) * fs.elems + e] = x;
         return;
     }
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
@@ -154,7 +152,7 @@ __global__ __launch_bounds__(64 * kGateWaves) void cw_gates_sweep_kernel(
 void chunkwise_gate_gradients(const float *alpha, const float *eta, const float *pvec, const float *xs,
                               const float *scal, float *d_alpha, float *d_eta, int seq_len, int batch,
                               int chunk_size, bool has_s, const float *dm_first, const float *ds_first,
-                              size_t chain_stride, int per, int nsum, float *tmp) {
+                              size_t chain_stride, int per, int nsum, float *tmp, int elems) {
     const ErrorScope es;
     const int nc = ceil_div(seq_len, chunk_size), ntask = batch * nc;
     const size_t lds = (size_t)kGateWaves * (has_s ? 2 : 1) * GTRI * sizeof(float);
@@ -171,8 +169,8 @@ void chunkwise_gate_gradients(const float *alpha, const float *eta, const float 
     if (es.failed()) return;
     static_assert(64 * kGateWaves == 256, "the sum workgroups take 256 elements each");
     const int sweep_blocks = ceil_div(ntask, kGateWaves), rows = ceil_div(batch, per);
-    const FirstSum fs{{dm_first, ds_first}, tmp, chain_stride, batch, per, rows, nsum};
-    const dim3 grid(sweep_blocks + (kSumElems / 256) * rows * nsum), block(64 * kGateWaves);
+    const FirstSum fs{{dm_first, ds_first}, tmp, chain_stride, batch, per, rows, nsum, elems};
+    const dim3 grid(sweep_blocks + (elems / 256) * rows * nsum), block(64 * kGateWaves);
     KernelTimer kt("cw_gates_sweep_kernel");
     if (has_s)
         hipLaunchKernelGGL(cw_gates_sweep_kernel<true>, grid, block, lds, stream(), alpha, eta, pvec, xs, scal, d_alpha,

@@ -60,6 +60,6 @@ void titans_chunkwise_backward_bf16_tokens_g16(const uint16_t *k_mem, const uint
 void chunkwise_gate_gradients(const float *alpha, const float *eta, const float *pvec, const float *xs,
                               const float *scal, float *d_alpha, float *d_eta, int seq_len, int batch,
                               int chunk_size, bool has_s, const float *dm_first, const float *ds_first,
-                              size_t chain_stride, int per, int nsum, float *tmp);
+                              size_t chain_stride, int per, int nsum, float *tmp, int elems = 64 * 64);
 
 }  // namespace nlh

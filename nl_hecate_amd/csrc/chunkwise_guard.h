@@ -31,7 +31,7 @@ bool couplings_may_fire_tracked(const uint16_t *k, const float *alpha, const flo
                                 float m_norm_max);
 bool couplings_may_fire_tracked(const float *k, const float *alpha, const float *theta, const float *eta,
                                 const ChainTracks &tr, bool has_s, int seq_len, int batch, int chunk_size, float error_clip,
-                                float m_norm_max);
+                                float m_norm_max, int hd = 64);
 
 // For the exact rules and the sequential frozen-M0 kernels: msq_part [batch, parts] holds, per workgroup of a chain,
 // an upper bound of max_t of the sum of squares of its rows of M_t.  true: the bound (plus rounding slack) reaches

@@ -133,7 +133,7 @@ __global__ __launch_bounds__(256) void cw_guard_tracks_kernel(const TOK *__restr
                                                               const float *__restrict__ theta, const float *__restrict__ eta,
                                                               const float *__restrict__ e2, const float *__restrict__ nrm,
                                                               int seq_len, int C, int nc, int nchunks, float clip, float mmax,
-                                                              float split_slack, int *__restrict__ flag) {
+                                                              float split_slack, int hd, int *__restrict__ flag) {
     const int lane = threadIdx.x & 63, task = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (task >= nchunks) return;   // waves are independent: no barrier below
     const int chain = task / nc, c = task % nc, t0 = c * C, L = min(C, seq_len - t0);
@@ -141,9 +141,9 @@ __global__ __launch_bounds__(256) void cw_guard_tracks_kernel(const TOK *__restr
     const size_t tok = (size_t)chain * seq_len + t0 + lane;
     float ksq = 0.f, esq = 0.f, al = 0.f, th = 0.f, et = 0.f;
     if (in) {
-#pragma unroll
-        for (int i = 0; i < HD / 4; i++) {
-            const float4 x = tok4(k, tok * HD + 4 * i);
+#pragma unroll 8
+        for (int i = 0; i < hd / 4; i++) {
+            const float4 x = tok4(k, tok * hd + 4 * i);
             ksq += x.x * x.x + x.y * x.y + x.z * x.z + x.w * x.w;
         }
         esq = e2[(((size_t)chain * 2 + 0) * nc + c) * CW + lane] + e2[(((size_t)chain * 2 + 1) * nc + c) * CW + lane];
@@ -246,7 +246,7 @@ bool norm_bound_exceeded(const float *msq_part, int batch, int parts, float m_no
 template <typename TOK>
 static bool tracked_test(const TOK *k, const float *alpha, const float *theta, const float *eta, const ChainTracks &tr,
                          bool has_s, int seq_len, int batch, int chunk_size, float error_clip, float m_norm_max,
-                         float split_slack) {
+                         float split_slack, int hd) {
     const ErrorScope es;
     int *flag = reinterpret_cast<int *>(scratch(31, 256));
     if (!g_host_flag) check_hip(hipHostMalloc(reinterpret_cast<void **>(&g_host_flag), 256, hipHostMallocDefault), "hipHostMalloc");
@@ -258,10 +258,10 @@ static bool tracked_test(const TOK *k, const float *alpha, const float *theta, c
         const dim3 grid((unsigned)((nchunks + 3) / 4));
         if (has_s)
             hipLaunchKernelGGL((cw_guard_tracks_kernel<TOK, true>), grid, dim3(256), 0, stream(), k, alpha, theta, eta, tr.e2,
-                               tr.nrm, seq_len, chunk_size, nc, nchunks, error_clip, m_norm_max, split_slack, flag);
+                               tr.nrm, seq_len, chunk_size, nc, nchunks, error_clip, m_norm_max, split_slack, hd, flag);
         else
             hipLaunchKernelGGL((cw_guard_tracks_kernel<TOK, false>), grid, dim3(256), 0, stream(), k, alpha, theta, eta, tr.e2,
-                               tr.nrm, seq_len, chunk_size, nc, nchunks, error_clip, m_norm_max, split_slack, flag);
+                               tr.nrm, seq_len, chunk_size, nc, nchunks, error_clip, m_norm_max, split_slack, hd, flag);
         check_launch("cw_guard_tracks_kernel");
     }
     *g_host_flag = 1;
@@ -282,12 +282,12 @@ ChainTracks chain_tracks(int seq_len, int batch, int chunk_size) {
 bool couplings_may_fire_tracked(const uint16_t *k, const float *alpha, const float *theta, const float *eta,
                                 const ChainTracks &tr, bool has_s, int seq_len, int batch, int chunk_size, float error_clip,
                                 float m_norm_max) {
-    return tracked_test(k, alpha, theta, eta, tr, has_s, seq_len, batch, chunk_size, error_clip, m_norm_max, 3.0517578125e-5f);
+    return tracked_test(k, alpha, theta, eta, tr, has_s, seq_len, batch, chunk_size, error_clip, m_norm_max, 3.0517578125e-5f, HD);
 }
 bool couplings_may_fire_tracked(const float *k, const float *alpha, const float *theta, const float *eta,
                                 const ChainTracks &tr, bool has_s, int seq_len, int batch, int chunk_size, float error_clip,
-                                float m_norm_max) {
-    return tracked_test(k, alpha, theta, eta, tr, has_s, seq_len, batch, chunk_size, error_clip, m_norm_max, 0.f);
+                                float m_norm_max, int hd) {
+    return tracked_test(k, alpha, theta, eta, tr, has_s, seq_len, batch, chunk_size, error_clip, m_norm_max, 0.f, hd);
 }
 
 bool couplings_may_fire(const float *k, const float *v, const float *alpha, const float *theta, const float *eta,

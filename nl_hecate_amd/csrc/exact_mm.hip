@@ -1,5 +1,5 @@
 // Backward of the exact Titans / Delta rule from checkpoints every C <= 64 tokens, in chunk-parallel matrix form on
-// the fp32 matrix cores (v_mfma_f32_16x16x4_f32), head size 64.
+// the fp32 matrix cores (v_mfma_f32_16x16x4_f32), head sizes 64 and 32.
 //
 // Semantics are those of core/kernels/titans_backward.cu:66-341 run segment by segment from the checkpoints of
 // core/kernels/titans_forward.cu (the schedule of core/src/gpu_backward.rs:1770-1962) with error_clip and the
@@ -59,7 +59,59 @@ using namespace mmt;
 
 // per chunk, for the scan: Phi_MM, Phi_SM, Phi_MS, Phi_SS (source state, destination state), C_M, C_S
 constexpr size_t kExLocMats = 6;
-constexpr size_t kDD = (size_t)HD * HD;
+constexpr size_t kDD = (size_t)HD * HD;   // a token x token or token x head-size matrix of a chunk in memory
+
+// Staging of a row-major [nrows <= ROWS][D] tile as fetch / commit of mm_tiles.h, for either head size.
+template <int D, int ROWS>
+struct TileD {
+    static constexpr int N = ROWS * D / 4, PER = (N + kThr - 1) / kThr;
+    float4 x[PER];
+};
+template <int D, int ROWS>
+__device__ __forceinline__ void fetch(TileD<D, ROWS> &r, const float *src, int nrows, int tid) {
+    using T = TileD<D, ROWS>;
+#pragma unroll
+    for (int it = 0; it < T::PER; it++) {
+        const int e = it * kThr + tid, rr = e / (D / 4), cc = 4 * (e % (D / 4));
+        r.x[it] = rr < nrows ? *reinterpret_cast<const float4 *>(src + rr * D + cc) : make_float4(0, 0, 0, 0);
+    }
+}
+template <int D, int ROWS>
+__device__ __forceinline__ void commit(float *dst, const TileD<D, ROWS> &r, int tid) {
+    using T = TileD<D, ROWS>;
+#pragma unroll
+    for (int it = 0; it < T::PER; it++) {
+        const int e = it * kThr + tid, rr = e / (D / 4), cc = 4 * (e % (D / 4));
+        if (T::N % kThr == 0 || e < T::N) {
+            float *p = dst + rr * LDM + cc;
+            p[0] = r.x[it].x; p[1] = r.x[it].y; p[2] = r.x[it].z; p[3] = r.x[it].w;
+        }
+    }
+}
+template <int D, int ROWS>
+__device__ __forceinline__ float tile_dot(const TileD<D, ROWS> &a, const TileD<D, ROWS> &b) {
+    float x = 0.f;
+#pragma unroll
+    for (int it = 0; it < TileD<D, ROWS>::PER; it++)
+        x += a.x[it].x * b.x[it].x + a.x[it].y * b.x[it].y + a.x[it].z * b.x[it].z + a.x[it].w * b.x[it].w;
+    return x;
+}
+
+// The scan matrices leave in the order in which the scan's waves take them as the second operand of their product:
+// lane 16 g + n % 16 of the wave for the 16 columns n / 16 takes the contraction indices (D / 4) g + 0 .. D / 4 - 1 of
+// its column as 16-byte pieces of four, and pieces are stored [column tile][piece][lane], so that a load instruction
+// of the scan reads 1 KB of consecutive memory.  A lane of a 16 x 16 accumulator tile (rows 16 ib + 4 (l / 16) + i,
+// columns 16 ct + l % 16) holds exactly one piece.
+template <int D>
+__device__ __forceinline__ void store_operand_tile(float *mat, const f32x4 &t, int ib, int ct, int l) {
+    const int k0 = 16 * ib + 4 * (l >> 4), g = k0 / (D / 4), piece = (k0 % (D / 4)) / 4;
+    *reinterpret_cast<f32x4 *>(mat + ((size_t)(ct * (D / 16) + piece) * 64 + 16 * g + (l & 15)) * 4) = t;
+}
+// The additive terms leave in the accumulator order of the wave that adds them: [row block][column tile][lane].
+template <int D>
+__device__ __forceinline__ void store_acc_tile(float *mat, const f32x4 &t, int ib, int ct, int l) {
+    *reinterpret_cast<f32x4 *>(mat + ((size_t)(ib * (D / 16) + ct) * 64 + l) * 4) = t;
+}
 
 struct ChunkVecs { float wM[CW], wS[CW], am[CW], bm[CW]; };
 __device__ __forceinline__ void chunk_vectors(ChunkVecs &cv, const Coef &cf, int L) {
@@ -73,13 +125,14 @@ __device__ __forceinline__ void chunk_vectors(ChunkVecs &cv, const Coef &cf, int
 }
 
 // ── pass 1: chunk-local matrices ────────────────────────────────────────────
-template <bool TRACK>
+template <int D, bool TRACK>
 __global__ __launch_bounds__(kThr) void ex_local_kernel(
     const float *__restrict__ k, const float *__restrict__ v, const float *__restrict__ q, const float *__restrict__ d_y,
     const float *__restrict__ alpha, const float *__restrict__ theta, const float *__restrict__ eta,
-    const float *__restrict__ m_ckpt, const float *__restrict__ s_ckpt, float *__restrict__ loc, float *__restrict__ locs,
-    float *__restrict__ Tg, float *__restrict__ Ug, float *__restrict__ dUg, int s, int C, int nc, int nck, int has_s,
+    const float *__restrict__ m_ckpt, const float *__restrict__ s_ckpt, float *__restrict__ loc,
+    float *__restrict__ Tg, float *__restrict__ Ug, float *__restrict__ dUg, int s, int C, int nc, int nck, int cstep, int has_s,
     int ntask, ChainTracks tr) {
+    constexpr size_t DD = (size_t)D * D;
     extern __shared__ float smem[];
     float *Ks = smem, *Vs = Ks + MAT, *Qs = Vs + MAT, *Ds = Qs + MAT, *Ms = Ds + MAT, *Ss = Ms + MAT, *Cc = Ss + MAT,
           *B8 = Cc + MAT, *B9 = B8 + MAT;
@@ -88,18 +141,19 @@ __global__ __launch_bounds__(kThr) void ex_local_kernel(
     // Persistent over a contiguous range of chunks.  A workgroup fills the compute unit's LDS, so nothing else would
     // hide its loads: the next chunk's tiles are requested at the start of this chunk's last phase (the longest one,
     // ten products back to back) and land in LDS at the top of the next round.
-    Tile<float> tk, tv, tq, td, tm, ts;
+    TileD<D, 64> tk, tv, tq, td;
+    TileD<D, D> tm, ts;
     Gates gt;
     auto fetch_task = [&](int task, int tid) {
         const int chain = task / nc, ci = task % nc, t0 = ci * C, L = min(C, s - t0);
-        const size_t tok = (size_t)chain * s + t0;
+        const size_t tok = (size_t)chain * s + t0, st = ((size_t)chain * nck + (size_t)ci * cstep) * DD;
         gt = fetch_gates(alpha + tok, theta + tok, eta + tok, L, has_s != 0);
-        fetch(tk, k + tok * HD, L, tid);
-        fetch(tv, v + tok * HD, L, tid);
-        fetch(tq, q + tok * HD, L, tid);
-        fetch(td, d_y + tok * HD, L, tid);
-        fetch(tm, m_ckpt + ((size_t)chain * nck + ci) * kDD, 64, tid);
-        if (has_s) fetch(ts, s_ckpt + ((size_t)chain * nck + ci) * kDD, 64, tid);
+        fetch(tk, k + tok * D, L, tid);
+        fetch(tv, v + tok * D, L, tid);
+        fetch(tq, q + tok * D, L, tid);
+        fetch(td, d_y + tok * D, L, tid);
+        fetch(tm, m_ckpt + st, D, tid);
+        if (has_s) fetch(ts, s_ckpt + st, D, tid);
     };
     const int per = (ntask + (int)gridDim.x - 1) / (int)gridDim.x, task_lo = blockIdx.x * per, task_hi = min(ntask, task_lo + per);
     if (task_lo < task_hi) fetch_task(task_lo, threadIdx.x);
@@ -114,6 +168,9 @@ __global__ __launch_bounds__(kThr) void ex_local_kernel(
     auto MMA = [&](Strip &acc, auto fa, auto fb) { mma(acc, fa, fb, l); };
     auto MMAR = [&](Strip &acc, auto fa, auto fb, int p0, int p1) { mma_range(acc, fa, fb, p0, p1, l); };
     auto MMAT = [&](f32x4 &acc, auto fa, auto fb, int k0) { mma_tile16(acc, fa, fb, k0, l); };
+    // over the head size
+    auto MMD = [&](Strip &acc, auto fa, auto fb) { if constexpr (D == 64) mma(acc, fa, fb, l); else mma_range(acc, fa, fb, 0, D / 32, l); };
+    const bool dcol = D == 64 || nh == 0;   // this wave's strip lies inside a token x head-size product
     auto FORC = [&](Strip &acc, auto f) { for_c(acc, f, l); };
     const int chain = itask / nc, ci = itask % nc, t0 = ci * C, L = min(C, s - t0);
     const size_t task = (size_t)itask;
@@ -134,26 +191,23 @@ __global__ __launch_bounds__(kThr) void ex_local_kernel(
     }
     __syncthreads();
     chunk_vectors(cv, cf, L);
-    if (threadIdx.x == 0) {
-        float *sc = locs + task * 4;
-        sc[0] = cf.a[L - 1]; sc[1] = cf.beta[L - 1]; sc[2] = cf.h[L - 1]; sc[3] = 0.f;
-    }
     {
         Strip g = zero_strip(), km = zero_strip(), ks = zero_strip(), p = zero_strip();
         auto aK = [&](int m, int kk) { return Ks[(m0 + m) * LDM + kk]; };
-        MMA(g, aK, [&](int kk, int n) { return Ks[(n0 + n) * LDM + kk]; });
-        MMA(km, aK, [&](int kk, int n) { return Ms[(n0 + n) * LDM + kk]; });
-        if (has_s) MMA(ks, aK, [&](int kk, int n) { return Ss[(n0 + n) * LDM + kk]; });
-        MMA(p, [&](int m, int kk) { return Qs[(m0 + m) * LDM + kk]; }, [&](int kk, int n) { return Ks[(n0 + n) * LDM + kk]; });
+        MMD(g, aK, [&](int kk, int n) { return Ks[(n0 + n) * LDM + kk]; });
+        if (dcol) MMD(km, aK, [&](int kk, int n) { return Ms[(n0 + n) * LDM + kk]; });
+        if (dcol && has_s) MMD(ks, aK, [&](int kk, int n) { return Ss[(n0 + n) * LDM + kk]; });
+        MMD(p, [&](int m, int kk) { return Qs[(m0 + m) * LDM + kk]; }, [&](int kk, int n) { return Ks[(n0 + n) * LDM + kk]; });
         __syncthreads();   // the vectors are there
 #pragma unroll
         for (int tl = 0; tl < 2; tl++)
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 const int row = m0 + row_of(i, l), col = n0 + 16 * tl + (l & 15);
-                // R in place over V (own strip)
-                float *d = Vs + row * LDM + col;
-                *d = cv.am[row] * km.t[tl][i] + cv.bm[row] * ks.t[tl][i] - *d;
+                if (dcol) {   // R in place over V (own strip)
+                    float *d = Vs + row * LDM + col;
+                    *d = cv.am[row] * km.t[tl][i] + cv.bm[row] * ks.t[tl][i] - *d;
+                }
                 const float nth = -cf.th[col];
                 B8[row * LDM + col] = (col < row) ? nth * Cc[(row - 1) * LDM + col] * g.t[tl][i] : 0.f;   // Lam
                 B9[row * LDM + col] = nth * Cc[row * LDM + col] * p.t[tl][i];                            // W.P
@@ -161,84 +215,18 @@ __global__ __launch_bounds__(kThr) void ex_local_kernel(
     }
     __syncthreads();
     Strip dul = zero_strip();
-    MMA(dul, [&](int m, int kk) { return B9[kk * LDM + m0 + m]; }, [&](int kk, int n) { return Ds[kk * LDM + n0 + n]; });
-    if (w < 4 && l < 16) {
-        // D_b = (I - Lam_bb)^-1 by substitution: lane c holds column c of block b = w
-        const float *A = B8 + (16 * w) * LDM + 16 * w;
-        float x[16];
-#pragma unroll
-        for (int r = 0; r < 16; r++) {
-            float acc = r == l ? 1.f : 0.f;
-#pragma unroll
-            for (int j = 0; j < r; j++) acc = fmaf(A[r * LDM + j], x[j], acc);
-            x[r] = acc;
-        }
-        float *Dd = Ms + (16 * w) * LDM + 16 * w + l;
-#pragma unroll
-        for (int r = 0; r < 16; r++) Dd[r * LDM] = x[r];
-    }
-    __syncthreads();
-    {   // N = D Lam_off -> Ss; dU_loc -> B9 and out
-#pragma unroll
-        for (int tl = 0; tl < 2; tl++) {
-            const int jb = 2 * (w & 1) + tl;
-            f32x4 nacc = {0.f, 0.f, 0.f, 0.f};
-            if (jb < ib)
-                MMAT(nacc, [&](int m, int kk) { return Ms[(m0 + m) * LDM + kk]; },
-                           [&](int kk, int n) { return B8[kk * LDM + 16 * jb + n]; }, 16 * ib);
-#pragma unroll
-            for (int i = 0; i < 4; i++) Ss[(m0 + row_of(i, l)) * LDM + 16 * jb + (l & 15)] = nacc[i];
-        }
-        float *go = dUg + task * kDD;
-        FORC(dul, [&](int r, int c, float &x) {
-            B9[(m0 + r) * LDM + n0 + c] = x;
-            go[(m0 + r) * HD + n0 + c] = x;
-        });
-    }
-    __syncthreads();
-    auto aN = [&](int m, int kk) { return Ss[(m0 + m) * LDM + kk]; };
-    // N is strictly block lower triangular (blocks of 16): its powers need only the block products that can be non-zero
-#pragma unroll
-    for (int tl = 0; tl < 2; tl++) {   // N^2 -> B8
-        const int jb = 2 * (w & 1) + tl;
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-        for (int kb = jb + 1; kb < ib; kb++)
-            MMAT(acc, aN, [&](int kk, int n) { return Ss[kk * LDM + 16 * jb + n]; }, 16 * kb);
-#pragma unroll
-        for (int i = 0; i < 4; i++) B8[(m0 + row_of(i, l)) * LDM + 16 * jb + (l & 15)] = acc[i];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int tl = 0; tl < 2; tl++) {   // X = (I + N)(I + N^2) = I + N + N^2 + N N^2 -> Cc
-        const int jb = 2 * (w & 1) + tl;
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-        for (int kb = jb + 2; kb < ib; kb++)
-            MMAT(acc, aN, [&](int kk, int n) { return B8[kk * LDM + 16 * jb + n]; }, 16 * kb);
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int row = m0 + row_of(i, l), col = 16 * jb + (l & 15);
-            Cc[row * LDM + col] = acc[i] + Ss[row * LDM + col] + B8[row * LDM + col] + (row == col ? 1.f : 0.f);
-        }
-    }
-    __syncthreads();
-    {   // T = X D -> Ss and out
-        float *go = Tg + task * kDD;
-#pragma unroll
-        for (int tl = 0; tl < 2; tl++) {
-            const int jb = 2 * (w & 1) + tl;
-            f32x4 t = {0.f, 0.f, 0.f, 0.f};
-            MMAT(t, [&](int m, int kk) { return Cc[(m0 + m) * LDM + kk]; },
-                       [&](int kk, int n) { return Ms[kk * LDM + 16 * jb + n]; }, 16 * jb);
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int row = m0 + row_of(i, l), col = 16 * jb + (l & 15);
-                Ss[row * LDM + col] = t[i];
-                go[row * HD + col] = t[i];
-            }
-        }
-    }
-    __syncthreads();
-    {   // U = T R -> out;  Z1 = T (am.K) -> B8,  Z2 = T (bm.K) -> Ms
+    if (dcol) MMA(dul, [&](int m, int kk) { return B9[kk * LDM + m0 + m]; }, [&](int kk, int n) { return Ds[kk * LDM + n0 + n]; });
+    float *goT = Tg + task * kDD, *goU = dUg + task * kDD;
+#define INV_L B8
+#define INV_D Ms
+#define INV_N Ss
+#define INV_X Cc
+#define INV_BESIDE_N \
+    if (dcol)        \
+        FORC(dul, [&](int r, int c, float &x) { B9[(m0 + r) * LDM + n0 + c] = x; goU[(m0 + r) * HD + n0 + c] = x; });
+#define INV_OUT(row, col, x) goT[(row) * HD + (col)] = x;
+#include "exact_inverse.h"
+    if (dcol) {   // U = T R -> out;  Z1 = T (am.K) -> B8,  Z2 = T (bm.K) -> Ms
         Strip u = zero_strip(), z1 = zero_strip(), z2 = zero_strip();
         auto aT = [&](int m, int kk) { return Ss[(m0 + m) * LDM + kk]; };
         // T is lower triangular: row block ib contracts over the first ib + 1 blocks of 16 (taken in pairs)
@@ -259,156 +247,154 @@ __global__ __launch_bounds__(kThr) void ex_local_kernel(
                 for (int i = 0; i < 4; i++) eo[row_of(i, l)] = u.t[0][i];
             }
         }
+    } else if (TRACK && row_writer(l)) {   // head size 32 has no second half
+        float *eo = tr.e2 + (((size_t)chain * 2 + nh) * nc + ci) * CW + m0;
+#pragma unroll
+        for (int i = 0; i < 4; i++) eo[row_of(i, l)] = 0.f;
     }
     __syncthreads();
     if (itask + 1 < task_hi) fetch_task(itask + 1, tid);
-    float *out = loc + task * kExLocMats * kDD;
-    auto store = [&](int which, Strip &x) {
-        FORC(x, [&](int r, int c, float &y) { out[(size_t)which * kDD + (m0 + r) * HD + n0 + c] = y; });
-    };
-    // The four scan matrices leave in the order in which the scan's waves take them as the second operand of their
-    // product: lane 16 (k / 16) + n % 16 of the wave for column half n / 32 takes, as its 16-byte piece j = (k % 16) / 2,
-    // the elements (k, n), (k, n + 16), (k + 1, n), (k + 1, n + 16) with k even, n % 32 < 16.  Pieces are stored
-    // [column half][j][lane], so a load instruction of the scan reads 1 KB of consecutive memory.  A lane of this strip
-    // holds two pieces.
-    auto store_operand = [&](int which, const Strip &x) {
-        float *o = out + (size_t)which * kDD + (size_t)(((nh * 8 + 2 * (l >> 4)) * 64 + 16 * ib + (l & 15)) * 4);
-        *reinterpret_cast<float4 *>(o) = make_float4(x.t[0][0], x.t[1][0], x.t[0][1], x.t[1][1]);
-        *reinterpret_cast<float4 *>(o + 64 * 4) = make_float4(x.t[0][2], x.t[1][2], x.t[0][3], x.t[1][3]);
-    };
-    // one product at a time (no unrolling over the outputs): the next chunk's tiles are in registers during this phase
+    float *out = loc + task * kExLocMats * DD;
+    // One product at a time (no unrolling over the outputs): the next chunk's tiles are in registers during this phase.
+    // At head size 32 a wave's strip is half a matrix's rows, so the outputs are dealt to the waves in pairs of strips.
+    const int sib = D == 64 ? ib : w & 1, sn0 = D == 64 ? n0 : 0, sm0 = 16 * sib;
+    const int o0 = D == 64 ? 0 : w >> 1, ostep = D == 64 ? 1 : 4;
+    const float aL = cf.a[L - 1], bL = cf.beta[L - 1], hL = cf.h[L - 1];
+    const bool on_diag = sm0 == sn0 || sm0 == sn0 + 16;
 #pragma unroll 1
-    for (int o = 0; o < (has_s ? 4 : 1); o++) {   // Phi_MM, Phi_SM, Phi_MS, Phi_SS = (w.K)^T Z
+    for (int o = o0; o < (has_s ? 4 : 1); o += ostep) {   // Phi_MM, Phi_SM, Phi_MS, Phi_SS = (w.K)^T Z
         const float *wv = (o & 1) ? cv.wS : cv.wM, *Z = (o & 2) ? Ms : B8;
         Strip x = zero_strip();
-        MMA(x, [&](int m, int kk) { return wv[kk] * Ks[kk * LDM + m0 + m]; }, [&](int kk, int n) { return Z[kk * LDM + n0 + n]; });
-        store_operand(o, x);
+        MMA(x, [&](int m, int kk) { return wv[kk] * Ks[kk * LDM + sm0 + m]; }, [&](int kk, int n) { return Z[kk * LDM + sn0 + n]; });
+        if (on_diag) {   // the chunk's own decay
+            const float dg = o == 0 ? aL : o == 2 ? bL : o == 3 ? hL : 0.f;
+            FORC(x, [&](int r, int c, float &y) { if (sm0 + r == sn0 + c) y += dg; });
+        }
+#pragma unroll
+        for (int tl = 0; tl < 2; tl++) store_operand_tile<D>(out + (size_t)o * DD, x.t[tl], sib, sn0 / 16 + tl, l);
     }
 #pragma unroll 1
-    for (int o = 0; o < (has_s ? 2 : 1); o++) {   // C_M = (a.dY)^T Q + dU_loc^T Z1,  C_S = (beta.dY)^T Q + dU_loc^T Z2
+    for (int o = o0; o < (has_s ? 2 : 1); o += ostep) {   // C_M = (a.dY)^T Q + dU_loc^T Z1,  C_S = (beta.dY)^T Q + dU_loc^T Z2
         const float *vec = o ? cf.beta : cf.a, *Z = o ? Ms : B8;
         Strip x = zero_strip();
-        MMA(x, [&](int m, int kk) { return vec[kk] * Ds[kk * LDM + m0 + m]; }, [&](int kk, int n) { return Qs[kk * LDM + n0 + n]; });
-        MMA(x, [&](int m, int kk) { return B9[kk * LDM + m0 + m]; }, [&](int kk, int n) { return Z[kk * LDM + n0 + n]; });
-        store(4 + o, x);
+        MMA(x, [&](int m, int kk) { return vec[kk] * Ds[kk * LDM + sm0 + m]; }, [&](int kk, int n) { return Qs[kk * LDM + sn0 + n]; });
+        MMA(x, [&](int m, int kk) { return B9[kk * LDM + sm0 + m]; }, [&](int kk, int n) { return Z[kk * LDM + sn0 + n]; });
+#pragma unroll
+        for (int tl = 0; tl < 2; tl++) store_acc_tile<D>(out + (size_t)(4 + o) * DD, x.t[tl], sib, sn0 / 16 + tl, l);
     }
     __syncthreads();   // LDS is rewritten by the next chunk
     }
 }
 constexpr size_t kExLocalLds = 9 * MAT * sizeof(float);
 
-// ── pass 2: reverse scan over the chunks of a chain, one workgroup per 16-row block ──
-//   X1' = a_L X1 + X1 Phi_MM + X2 Phi_SM + C_M,   X2' = beta_L X1 + h_L X2 + X1 Phi_MS + X2 Phi_SS + C_S
-// ends [chain][nc + 1][64*64]: slot c = adjoint of the state at the start of chunk c (slot nc = 0, slot 0 = the
-// gradient of the initial state, also written to first [chain][64*64]).
-// Wave w: destination w / 4, source (w / 2) % 2, column half w % 2: one 16 x 64 x 32 product per step.  The two
-// source waves of a destination strip then finish one 16 x 16 tile of it each (they swap the other tile through
-// LDS), so every wave runs the same instructions: per step 12 loads, then 4 stores.  That matters: the memory
-// counter of this hardware counts loads and stores together and in order, and the wait for the next step's operands
-// at the top of a step can only leave this step's stores in flight if their number is the same on every path
-// (with the stores under a branch the wait was for all of them: 4 of a step's 9 thousand cycles).
-// Without momentum (the Delta rule) there is one state and one matrix: the two source waves split its contraction.
-template <bool HAS_S>
-__global__ __launch_bounds__(kThr) void ex_scan_kernel(const float *__restrict__ loc, const float *__restrict__ locs,
-                                                       float *__restrict__ em, float *__restrict__ es_,
-                                                       float *__restrict__ first_m, float *__restrict__ first_s, int nc) {
-    __shared__ float X1[16 * LDM], X2[16 * LDM], part[8 * 256];
-    // the four row blocks of a chain sit 8 workgroups apart: consecutive workgroups go to consecutive XCDs, so the
-    // four share one XCD's L2 for the chunk matrices they all read
-    const int chain0 = (blockIdx.x & 7) + 8 * (blockIdx.x >> 5), rb0 = (blockIdx.x >> 3) & 3;
-    const bool whole = (int)(blockIdx.x | 31) < (int)gridDim.x;   // a full group of 32 workgroups
-    const int chain = whole ? chain0 : blockIdx.x >> 2, r0 = 16 * (whole ? rb0 : blockIdx.x & 3);
-    const int l = threadIdx.x & 63, w = threadIdx.x >> 6, dst = w >> 2, src = (w >> 1) & 1, half = w & 1;
-    const int col = 32 * half + 16 * src + (l & 15), rw = 4 * (l >> 4);   // the tile this wave finishes: rows rw + i
-    float *emp = em + (size_t)chain * (nc + 1) * kDD, *esp = HAS_S ? es_ + (size_t)chain * (nc + 1) * kDD : nullptr;
-    for (int e = threadIdx.x; e < 16 * 64; e += kThr) {
-        const int rr = e >> 6, cc = e & 63;
-        X1[rr * LDM + cc] = 0.f;
-        X2[rr * LDM + cc] = 0.f;
-        emp[(size_t)nc * kDD + (r0 + rr) * HD + cc] = 0.f;
-        if (HAS_S) esp[(size_t)nc * kDD + (r0 + rr) * HD + cc] = 0.f;
+// ── pass 2: scan over the chunks of a chain, one workgroup per 16-row block ──
+//   X1' = X1 Phi_MM + X2 Phi_SM + C_M,   X2' = X1 Phi_MS + X2 Phi_SS + C_S   (the chunk's decay is on the diagonals)
+// REV: adjoints, last chunk first, from zero; states [chain][nc + 1][D*D]: slot c = adjoint of the state at the start of
+// chunk c (slot nc = 0, slot 0 = the gradient of the initial state, also written to first [chain][D*D]).
+// Forward: the states themselves from the initial ones; chunk c's start state goes to slot c * sstep of the chain's
+// states (the last chunk's end state is left to the pass that walks its tokens).
+// One wave per (destination, 16 columns): both sources' contributions, 2 D / 16 products of 16 x 16 x 16, so a step needs
+// no exchange of partial sums and, with X in two LDS buffers, one barrier.  The second operand comes straight from memory
+// in the lane order of the product (store_operand_tile), the additive term in accumulator order: every load is 1 KB of
+// consecutive memory, requested two steps ahead of its use.  All waves run the same number of loads and stores per step:
+// the memory counter of this hardware counts both in order, and only a fixed number in flight can be waited past.
+// Bound by the step's own chain: LDS read, 2 D / 4 matrix instructions on each of two waves per SIMD, LDS write, barrier.
+// 64 chains x 32 chunks, head size 64: 84 -> 78 us (four source / destination waves that swapped tiles through LDS,
+// two barriers a step and loads one step ahead before).
+template <int D, bool HAS_S, bool REV>
+__global__ __launch_bounds__((HAS_S ? 2 : 1) * D * 4) void ex_scan_kernel(
+    const float *__restrict__ loc, const float *__restrict__ m_initial, const float *__restrict__ s_initial, long long m_stride,
+    float *__restrict__ mst, float *__restrict__ sst, long long state_stride, int sstep, float *__restrict__ first_m,
+    float *__restrict__ first_s, int nc) {
+    constexpr int NS = HAS_S ? 2 : 1, NT = D / 16, NB = D / 16, LDX = D + 4, DD = D * D;
+    __shared__ __align__(16) float X[2][NS][16 * LDX];
+    // the row blocks of a chain sit 8 workgroups apart: consecutive workgroups go to consecutive XCDs, so they share one
+    // XCD's L2 for the chunk matrices they all read
+    const int bx = blockIdx.x, span = 8 * NT;
+    const bool whole = (bx / span + 1) * span <= (int)gridDim.x;   // a full group of workgroups
+    const int chain = whole ? (bx & 7) + 8 * (bx / span) : bx / NT, rb = whole ? (bx >> 3) % NT : bx % NT;
+    const int l = threadIdx.x & 63, w = threadIdx.x >> 6, dst = w / NT, ct = w % NT;
+    const int col = 16 * ct + (l & 15), rw = 4 * (l >> 4);   // this wave's tile: rows 16 rb + rw + i
+    const size_t at = (size_t)(16 * rb + rw) * D + col;      // its first element in a D x D matrix
+    float *st = (dst ? sst : mst) + (size_t)chain * state_stride + at;
+    f32x4 x = {0.f, 0.f, 0.f, 0.f};
+    if (!REV) {
+        const float *in = (dst ? s_initial : m_initial) + (size_t)chain * m_stride + at;
+#pragma unroll
+        for (int i = 0; i < 4; i++) x[i] = in[i * D];
     }
-    const bool active = HAS_S || dst == 0;   // wave-uniform; the idle waves of the Delta rule only keep the barriers
-    constexpr int NB = HAS_S ? 8 : 4;   // 16-byte pieces of the operand per lane and step
-    // The wave's second operand (a 64 x 32 piece of one chunk matrix) comes straight from memory in the lane order
-    // of the product (ex_local_kernel writes it that way), requested a step ahead.
-    float4 bn[NB], bc[NB];
-    f32x4 cn = {0.f, 0.f, 0.f, 0.f}, out = {0.f, 0.f, 0.f, 0.f};
-    float scn = 0.f;   // lanes 4 j + 0, 1, 2: a_L, beta_L, h_L of the next step
-    auto prefetch = [&](int ci) {
-        const float *lc = loc + ((size_t)chain * nc + ci) * kExLocMats * kDD;
-        const float *sc = locs + ((size_t)chain * nc + ci) * 4;
-        const float4 *bp = reinterpret_cast<const float4 *>(lc + (size_t)(HAS_S ? dst * 2 + src : 0) * kDD) +
-                           (half * 8 + (HAS_S ? 0 : 4 * src)) * 64 + l;
 #pragma unroll
-        for (int j = 0; j < NB; j++) bn[j] = bp[j * 64];
-        // a vector load (lane-dependent address) on purpose: a scalar load would join the LDS reads under one counter
-        // that only knows "all done", and the first product of the step would wait for it to come back from memory
-        scn = sc[l & 3];
-        const float *Cm = lc + (4 + dst) * kDD + (r0 + rw) * HD + col;
+    for (int i = 0; i < 4; i++) {
+        X[0][dst][(rw + i) * LDX + col] = x[i];
+        st[(REV ? (size_t)nc * DD : 0) + i * D] = x[i];
+    }
+    struct Step { f32x4 b[NS][NB], c; };
+    const f32x4 *lc = reinterpret_cast<const f32x4 *>(loc) + (size_t)chain * nc * kExLocMats * (DD / 4) + l;
+    auto request = [&](Step &r, int i) {   // step i of the scan (past the end: the last one again, unused)
+        const int ci = REV ? max(nc - 1 - i, 0) : min(i, nc - 1);
+        const f32x4 *p = lc + (size_t)ci * kExLocMats * (DD / 4);
 #pragma unroll
-        for (int i = 0; i < 4; i++) cn[i] = Cm[i * HD];
+        for (int sr = 0; sr < NS; sr++)
+#pragma unroll
+            for (int j = 0; j < NB; j++) r.b[sr][j] = p[(HAS_S ? dst * 2 + sr : 0) * (DD / 4) + (ct * NB + j) * 64];
+        r.c = p[(4 + dst) * (DD / 4) + (rb * NT + ct) * 64];
     };
-    if (active) prefetch(nc - 1);
+    const int steps = REV ? nc : nc - 1;
+    auto step = [&](Step &r, int i) {
+        const float *Xr = X[i & 1][0] + (l & 15) * LDX + (D / 4) * (l >> 4);
+        f32x4 a[NS][NB];
+#pragma unroll
+        for (int sr = 0; sr < NS; sr++)
+#pragma unroll
+            for (int j = 0; j < NB; j++) a[sr][j] = *reinterpret_cast<const f32x4 *>(Xr + sr * 16 * LDX + 4 * j);
+        f32x4 acc[2] = {r.c, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+        for (int j = 0; j < NB; j++)
+#pragma unroll
+            for (int sr = 0; sr < NS; sr++)
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    acc[HAS_S ? sr : e & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[sr][j][e], r.b[sr][j][e], acc[HAS_S ? sr : e & 1], 0, 0, 0);
+        request(r, i + 2);
+        float *Xw = X[(i + 1) & 1][dst] + rw * LDX + col;
+        const size_t slot = REV ? (size_t)(nc - 1 - i) * DD : (size_t)(i + 1) * sstep * DD;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            x[e] = acc[0][e] + acc[1][e];
+            Xw[e * LDX] = x[e];
+            st[slot + e * D] = x[e];
+        }
+        __syncthreads();
+    };
+    Step r0, r1;
+    request(r0, 0);
+    request(r1, 1);
     __syncthreads();
-    float *Xd = dst ? X2 : X1;
-    float *gd = (dst ? esp : emp) + (size_t)(r0 + rw) * HD + col;
-    const float *Xs = ((HAS_S && src) ? X2 : X1) + (l & 15) * LDM + 16 * (l >> 4) + (HAS_S ? 0 : 8 * src);
-    for (int ci = nc - 1; ci >= 0; ci--) {
-        if (active) {
-#pragma unroll
-            for (int j = 0; j < NB; j++) bc[j] = bn[j];
-            const float aL = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, scn), 0)),
-                        bL = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, scn), 1)),
-                        hL = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, scn), 2));
-            const f32x4 ca = cn;
-            if (ci > 0) prefetch(ci - 1);
-            f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-#pragma unroll
-            for (int j = 0; j < NB; j++) {   // contraction indices 16 (l / 16) + 2 j, + 1 (+ 8 for the second Delta wave)
-                const float a0 = Xs[2 * j], a1 = Xs[2 * j + 1];
-                acc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a0, bc[j].x, acc[0], 0, 0, 0);
-                acc[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a0, bc[j].y, acc[1], 0, 0, 0);
-                acc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a1, bc[j].z, acc[0], 0, 0, 0);
-                acc[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a1, bc[j].w, acc[1], 0, 0, 0);
-            }
-            // the tile the partner wave (w ^ 2) finishes goes to LDS; this wave keeps tile `src`
-            const f32x4 mine = src ? acc[1] : acc[0], theirs = src ? acc[0] : acc[1];
-#pragma unroll
-            for (int i = 0; i < 4; i++) part[w * 256 + i * 64 + l] = theirs[i];
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const float x1 = X1[(rw + i) * LDM + col];
-                out[i] = mine[i] + ca[i] + (dst ? bL * x1 + hL * X2[(rw + i) * LDM + col] : aL * x1);
-            }
-        }
-        __syncthreads();   // every read of the old X1 / X2 is done; the partners' tiles are in LDS
-        if (active) {
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                out[i] += part[(w ^ 2) * 256 + i * 64 + l];
-                Xd[(rw + i) * LDM + col] = out[i];
-                gd[(size_t)ci * kDD + i * HD] = out[i];
-            }
-        }
-        __syncthreads();   // the new X1 / X2 are complete
+    int i = 0;
+    for (; i + 2 <= steps; i += 2) {
+        step(r0, i);
+        step(r1, i + 1);
     }
-    if (!active) return;
-    float *gf = (dst ? first_s : first_m) + (size_t)chain * kDD + (size_t)(r0 + rw) * HD + col;
+    if (i < steps) step(r0, i);
+    if (REV) {
+        float *gf = (dst ? first_s : first_m) + (size_t)chain * DD + at;
 #pragma unroll
-    for (int i = 0; i < 4; i++) gf[i * HD] = out[i];
+        for (int e = 0; e < 4; e++) gf[e * D] = x[e];
+    }
 }
 
 // ── pass 3: gradients of one chunk ──────────────────────────────────────────
 //   pvec [chain][token][4] = <M0, J_t>, <S0, J_t>, -theta_t u_t^T dMo k_t, -theta_t u_t^T dSo k_t
 //   xs [chain][chunk][s][t] as above     scal [chunk][4] = <M0, dMo>, <S0, dMo>, <S0, dSo>
+template <int D>
 __global__ __launch_bounds__(kThr) void ex_grads_kernel(
     const float *__restrict__ k, const float *__restrict__ q, const float *__restrict__ d_y, const float *__restrict__ alpha,
     const float *__restrict__ theta, const float *__restrict__ eta, const float *__restrict__ m_ckpt,
     const float *__restrict__ s_ckpt, const float *__restrict__ Tg, const float *__restrict__ Ug,
     const float *__restrict__ dUg, const float *__restrict__ em, const float *__restrict__ es_, float *__restrict__ d_k,
     float *__restrict__ d_v, float *__restrict__ d_q, float *__restrict__ d_theta, float *__restrict__ pvec,
-    float *__restrict__ xs, float *__restrict__ scal, int s, int C, int nc, int nck, int has_s, int ntask) {
+    float *__restrict__ xs, float *__restrict__ scal, int s, int C, int nc, int nck, int cstep, int has_s, int ntask) {
+    constexpr size_t DD = (size_t)D * D;
     extern __shared__ float smem[];
     float *Ks = smem, *Qs = Ks + MAT, *Ds = Qs + MAT, *Ts = Ds + MAT, *Us = Ts + MAT, *A1 = Us + MAT, *A2 = A1 + MAT,
           *Cc = A2 + MAT, *B9 = Cc + MAT;
@@ -419,7 +405,9 @@ __global__ __launch_bounds__(kThr) void ex_grads_kernel(
     __shared__ float dots[3][8];
     // Persistent over a contiguous range of chunks, as ex_local_kernel: the next chunk's nine tiles are requested at the
     // start of this chunk's last phase.
-    Tile<float> tk, tq, td, tt, tu, tdm, tds, tm, ts;
+    TileD<D, 64> tk, tq, td;
+    TileD<64, 64> tt, tu;
+    TileD<D, D> tdm, tds, tm, ts;
     Gates gt;
     // K, Q, dY of the next chunk are requested during this chunk's last phase (more does not fit next to its
     // accumulators); the other six tiles at the top of the chunk, behind two products that need K and Q only
@@ -427,19 +415,19 @@ __global__ __launch_bounds__(kThr) void ex_grads_kernel(
         const int chain = task / nc, ci = task % nc, t0 = ci * C, L = min(C, s - t0);
         const size_t tok = (size_t)chain * s + t0;
         gt = fetch_gates(alpha + tok, theta + tok, eta + tok, L, has_s != 0);
-        fetch(tk, k + tok * HD, L, tid);
-        fetch(tq, q + tok * HD, L, tid);
-        fetch(td, d_y + tok * HD, L, tid);
+        fetch(tk, k + tok * D, L, tid);
+        fetch(tq, q + tok * D, L, tid);
+        fetch(td, d_y + tok * D, L, tid);
     };
     auto fetch_b = [&](int task, int tid) {
         const int chain = task / nc, ci = task % nc;
-        const size_t end = ((size_t)chain * (nc + 1) + ci + 1) * kDD;
+        const size_t end = ((size_t)chain * (nc + 1) + ci + 1) * DD, st = ((size_t)chain * nck + (size_t)ci * cstep) * DD;
         fetch(tt, Tg + (size_t)task * kDD, 64, tid);
-        fetch(tu, Ug + (size_t)task * kDD, 64, tid);
-        fetch(tdm, em + end, 64, tid);
-        if (has_s) fetch(tds, es_ + end, 64, tid);
-        fetch(tm, m_ckpt + ((size_t)chain * nck + ci) * kDD, 64, tid);
-        if (has_s) fetch(ts, s_ckpt + ((size_t)chain * nck + ci) * kDD, 64, tid);
+        fetch(tu, Ug + (size_t)task * kDD, 64, tid);   // at head size 32 the right half is stale memory, never used
+        fetch(tdm, em + end, D, tid);
+        if (has_s) fetch(tds, es_ + end, D, tid);
+        fetch(tm, m_ckpt + st, D, tid);
+        if (has_s) fetch(ts, s_ckpt + st, D, tid);
     };
     const int per = (ntask + (int)gridDim.x - 1) / (int)gridDim.x, task_lo = blockIdx.x * per, task_hi = min(ntask, task_lo + per);
     if (task_lo < task_hi) fetch_a(task_lo, threadIdx.x);
@@ -453,6 +441,8 @@ __global__ __launch_bounds__(kThr) void ex_grads_kernel(
     auto MMA = [&](Strip &acc, auto fa, auto fb) { mma(acc, fa, fb, l); };
     auto MMAR = [&](Strip &acc, auto fa, auto fb, int p0, int p1) { mma_range(acc, fa, fb, p0, p1, l); };
     auto FORC = [&](Strip &acc, auto f) { for_c(acc, f, l); };
+    auto MMD = [&](Strip &acc, auto fa, auto fb) { if constexpr (D == 64) mma(acc, fa, fb, l); else mma_range(acc, fa, fb, 0, D / 32, l); };
+    const bool dcol = D == 64 || nh == 0;   // this wave's strip lies inside a token x head-size product
     const int chain = itask / nc, ci = itask % nc, t0 = ci * C, L = min(C, s - t0);
     const size_t tok = (size_t)chain * s + t0, task = (size_t)itask;
     fetch_b(itask, tid);
@@ -465,8 +455,8 @@ __global__ __launch_bounds__(kThr) void ex_grads_kernel(
     chunk_vectors(cv, cf, L);
     auto aK = [&](int m, int kk) { return Ks[(m0 + m) * LDM + kk]; };
     Strip p = zero_strip(), g = zero_strip();   // Q K^T and K K^T while the other tiles are in flight
-    MMA(p, [&](int m, int kk) { return Qs[(m0 + m) * LDM + kk]; }, [&](int kk, int n) { return Ks[(n0 + n) * LDM + kk]; });
-    MMA(g, aK, [&](int kk, int n) { return Ks[(n0 + n) * LDM + kk]; });
+    MMD(p, [&](int m, int kk) { return Qs[(m0 + m) * LDM + kk]; }, [&](int kk, int n) { return Ks[(n0 + n) * LDM + kk]; });
+    MMD(g, aK, [&](int kk, int n) { return Ks[(n0 + n) * LDM + kk]; });
     {
         commit(Ts, tt, tid);
         commit(Us, tu, tid);
@@ -491,13 +481,13 @@ __global__ __launch_bounds__(kThr) void ex_grads_kernel(
     };
     auto aU = [&](int m, int kk) { return Us[(m0 + m) * LDM + kk]; };
     Strip udm = zero_strip(), uds = zero_strip();
-    {
+    if (dcol) {
         Strip kdm = zero_strip(), kds = zero_strip();
-        MMA(kdm, aK, [&](int kk, int n) { return A1[(n0 + n) * LDM + kk]; });
-        MMA(udm, aU, [&](int kk, int n) { return A1[kk * LDM + n0 + n]; });
+        MMD(kdm, aK, [&](int kk, int n) { return A1[(n0 + n) * LDM + kk]; });
+        MMD(udm, aU, [&](int kk, int n) { return A1[kk * LDM + n0 + n]; });
         if (has_s) {
-            MMA(kds, aK, [&](int kk, int n) { return A2[(n0 + n) * LDM + kk]; });
-            MMA(uds, aU, [&](int kk, int n) { return A2[kk * LDM + n0 + n]; });
+            MMD(kds, aK, [&](int kk, int n) { return A2[(n0 + n) * LDM + kk]; });
+            MMD(uds, aU, [&](int kk, int n) { return A2[kk * LDM + n0 + n]; });
         }
         const float *gi = dUg + task * kDD;
 #pragma unroll
@@ -512,13 +502,15 @@ __global__ __launch_bounds__(kThr) void ex_grads_kernel(
     {
         Strip dr = zero_strip();
         // T^T is upper triangular: row block ib contracts over the blocks ib .. 3 of 16 (taken in pairs)
-        MMAR(dr, [&](int m, int kk) { return Ts[kk * LDM + m0 + m]; }, [&](int kk, int n) { return B9[kk * LDM + n0 + n]; },
-             ib >> 1, 2);
-        FORC(dr, [&](int r, int c, float &x) {
-            if (m0 + r < L) d_v[(tok + m0 + r) * HD + n0 + c] = -x;
-        });
+        if (dcol) {
+            MMAR(dr, [&](int m, int kk) { return Ts[kk * LDM + m0 + m]; }, [&](int kk, int n) { return B9[kk * LDM + n0 + n]; },
+                 ib >> 1, 2);
+            FORC(dr, [&](int r, int c, float &x) {
+                if (m0 + r < L) d_v[(tok + m0 + r) * D + n0 + c] = -x;
+            });
+        }
         __syncthreads();   // T no longer needed
-        FORC(dr, [&](int r, int c, float &x) { Ts[(m0 + r) * LDM + n0 + c] = x; });   // dR
+        if (dcol) FORC(dr, [&](int r, int c, float &x) { Ts[(m0 + r) * LDM + n0 + c] = x; });   // dR
     }
     __syncthreads();
     const float *dRs = Ts;
@@ -526,8 +518,8 @@ __global__ __launch_bounds__(kThr) void ex_grads_kernel(
     {
         Strip dlam = zero_strip(), dyu = zero_strip();
         auto bU = [&](int kk, int n) { return Us[(n0 + n) * LDM + kk]; };
-        MMA(dlam, [&](int m, int kk) { return dRs[(m0 + m) * LDM + kk]; }, bU);
-        MMA(dyu, [&](int m, int kk) { return Ds[(m0 + m) * LDM + kk]; }, bU);
+        MMD(dlam, [&](int m, int kk) { return dRs[(m0 + m) * LDM + kk]; }, bU);
+        MMD(dyu, [&](int m, int kk) { return Ds[(m0 + m) * LDM + kk]; }, bU);
 #pragma unroll
         for (int tl = 0; tl < 2; tl++)
 #pragma unroll
@@ -571,11 +563,11 @@ __global__ __launch_bounds__(kThr) void ex_grads_kernel(
     __syncthreads();
     if (itask + 1 < task_hi) fetch_a(itask + 1, tid);
     const float *M0s = Us, *S0s = Cc, *dPs = B9, *dGs = A1;
-    {
+    if (dcol) {
         Strip dym = zero_strip(), dys = zero_strip(), dq = zero_strip(), r0 = zero_strip(), r1 = zero_strip();
         auto aD = [&](int m, int kk) { return Ds[(m0 + m) * LDM + kk]; };
-        MMA(dym, aD, [&](int kk, int n) { return M0s[kk * LDM + n0 + n]; });
-        if (has_s) MMA(dys, aD, [&](int kk, int n) { return S0s[kk * LDM + n0 + n]; });
+        MMD(dym, aD, [&](int kk, int n) { return M0s[kk * LDM + n0 + n]; });
+        if (has_s) MMD(dys, aD, [&](int kk, int n) { return S0s[kk * LDM + n0 + n]; });
         MMA(dq, [&](int m, int kk) { return dPs[(m0 + m) * LDM + kk]; }, [&](int kk, int n) { return Ks[kk * LDM + n0 + n]; });
 #pragma unroll
         for (int tl = 0; tl < 2; tl++)
@@ -586,12 +578,12 @@ __global__ __launch_bounds__(kThr) void ex_grads_kernel(
                 r0.t[tl][i] = dym.t[tl][i] * qv;
                 r1.t[tl][i] = dys.t[tl][i] * qv;
                 if (row < L)
-                    d_q[(tok + row) * HD + col] = cf.a[row] * dym.t[tl][i] + cf.beta[row] * dys.t[tl][i] + dq.t[tl][i];
+                    d_q[(tok + row) * D + col] = cf.a[row] * dym.t[tl][i] + cf.beta[row] * dys.t[tl][i] + dq.t[tl][i];
             }
         publish(0, r0);
         publish(1, r1);
     }
-    {   // d_k in two halves: fewer accumulators alive at once
+    if (dcol) {   // d_k in two halves: fewer accumulators alive at once
         Strip dk = zero_strip();
         {
             Strip r2 = zero_strip(), r3 = zero_strip();
@@ -613,8 +605,8 @@ __global__ __launch_bounds__(kThr) void ex_grads_kernel(
         {
             Strip drm = zero_strip(), drs = zero_strip(), r4 = zero_strip(), r5 = zero_strip();
             auto aR = [&](int m, int kk) { return dRs[(m0 + m) * LDM + kk]; };
-            MMA(drm, aR, [&](int kk, int n) { return M0s[kk * LDM + n0 + n]; });
-            if (has_s) MMA(drs, aR, [&](int kk, int n) { return S0s[kk * LDM + n0 + n]; });
+            MMD(drm, aR, [&](int kk, int n) { return M0s[kk * LDM + n0 + n]; });
+            if (has_s) MMD(drs, aR, [&](int kk, int n) { return S0s[kk * LDM + n0 + n]; });
 #pragma unroll
             for (int tl = 0; tl < 2; tl++)
 #pragma unroll
@@ -624,7 +616,7 @@ __global__ __launch_bounds__(kThr) void ex_grads_kernel(
                     r4.t[tl][i] = drm.t[tl][i] * kv;
                     r5.t[tl][i] = drs.t[tl][i] * kv;
                     if (row < L)
-                        d_k[(tok + row) * HD + col] = dk.t[tl][i] + cv.am[row] * drm.t[tl][i] + cv.bm[row] * drs.t[tl][i];
+                        d_k[(tok + row) * D + col] = dk.t[tl][i] + cv.am[row] * drm.t[tl][i] + cv.bm[row] * drs.t[tl][i];
                 }
             publish(4, r4);
             publish(5, r5);
@@ -633,7 +625,7 @@ __global__ __launch_bounds__(kThr) void ex_grads_kernel(
     __syncthreads();
     if (tid < L) {
         const int t = tid;
-        auto sum = [&](int which, int row) { return part[which][0][row] + part[which][1][row]; };
+        auto sum = [&](int which, int row) { return D == 64 ? part[which][0][row] + part[which][1][row] : part[which][0][row]; };
         const float g1 = sum(2, t), g2 = sum(3, t);
         const float dam = t + 1 < CW ? sum(4, t + 1) : 0.f, dbm = t + 1 < CW ? sum(5, t + 1) : 0.f;
         d_theta[tok + t] = -(((part_th[0][t] + part_th[1][t]) + (part_th[2][t] + part_th[3][t])) + cf.cl[t] * g1 + cf.bl[t] * g2);
@@ -648,6 +640,90 @@ __global__ __launch_bounds__(kThr) void ex_grads_kernel(
 }
 constexpr size_t kExGradsLds = 9 * MAT * sizeof(float);
 
+// ── the forward of the rule, pass 1: the chunk maps of the state scan ────────
+//   M' = a_L M + beta_L S + U^T (wM.K),  S' = h_L S + U^T (wS.K)  with  U = Z1 M^T + Z2 S^T - T V,  Z1 = T (am.K), Z2 = T (bm.K)
+// so the end state is affine in the start state with the matrices Z^T (w.K): the same scan as the backward's, first chunk
+// first.  Nothing else leaves this pass; the tokens of a chunk are then walked from its start state by the sequential
+// kernel (rule_fwd_kernel with FwdArgs::sub_chunks), all chunks at once.
+template <int D>
+__global__ __launch_bounds__(kThr) void ex_fwd_local_kernel(
+    const float *__restrict__ k, const float *__restrict__ v, const float *__restrict__ alpha, const float *__restrict__ theta,
+    const float *__restrict__ eta, float *__restrict__ loc, int s, int stride, int C, int nc, int has_s) {
+    constexpr size_t DD = (size_t)D * D;
+    extern __shared__ float smem[];
+    float *Ks = smem, *Vs = Ks + MAT, *B8 = Vs + MAT, *Dg = B8 + MAT, *Nn = Dg + MAT, *Cc = Nn + MAT;
+    __shared__ Coef cf;
+    __shared__ ChunkVecs cv;
+    const int tid = threadIdx.x, l = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    NLH_STRIP_ORIGIN_OF(w);
+    const bool dcol = D == 64 || nh == 0;
+    auto MMAT = [&](f32x4 &acc, auto fa, auto fb, int k0) { mma_tile16(acc, fa, fb, k0, l); };
+    const int chain = blockIdx.x / (nc - 1), ci = blockIdx.x % (nc - 1), t0 = ci * C, L = min(C, s - t0);   // the last chunk's map is not needed
+    const size_t tok = (size_t)chain * stride + t0;
+    {
+        TileD<D, 64> tk, tv;
+        fetch(tk, k + tok * D, L, tid);
+        fetch(tv, v + tok * D, L, tid);
+        const Gates gt = fetch_gates(alpha + tok, theta + tok, eta + tok, L, has_s != 0);
+        load_gates(cf, gt);
+        coefficients(cf, gt, L, Cc, nullptr, nullptr);
+        commit(Ks, tk, tid);
+        commit(Vs, tv, tid);
+    }
+    __syncthreads();
+    chunk_vectors(cv, cf, L);
+    {
+        Strip g = zero_strip();
+        auto a = [&](int m, int kk) { return Ks[(m0 + m) * LDM + kk]; };
+        auto b = [&](int kk, int n) { return Ks[(n0 + n) * LDM + kk]; };
+        if constexpr (D == 64) mma(g, a, b, l); else mma_range(g, a, b, 0, D / 32, l);
+        for_c(g, [&](int r, int c, float &x) {
+            const int row = m0 + r, col = n0 + c;
+            B8[row * LDM + col] = (col < row) ? -cf.th[col] * Cc[(row - 1) * LDM + col] * x : 0.f;   // Lam
+        }, l);
+    }
+    __syncthreads();
+#define INV_L B8
+#define INV_D Dg
+#define INV_N Nn
+#define INV_X Cc
+#define INV_BESIDE_N
+#define INV_OUT(row, col, x)
+#include "exact_inverse.h"
+    if (dcol) {   // Z1 -> B8, Z2 -> Dg, T V -> Cc
+        Strip tv = zero_strip(), z1 = zero_strip(), z2 = zero_strip();
+        auto aT = [&](int m, int kk) { return Nn[(m0 + m) * LDM + kk]; };
+        const int pe = (ib >> 1) + 1;
+        mma_range(tv, aT, [&](int kk, int n) { return Vs[kk * LDM + n0 + n]; }, 0, pe, l);
+        mma_range(z1, aT, [&](int kk, int n) { return cv.am[kk] * Ks[kk * LDM + n0 + n]; }, 0, pe, l);
+        if (has_s) mma_range(z2, aT, [&](int kk, int n) { return cv.bm[kk] * Ks[kk * LDM + n0 + n]; }, 0, pe, l);
+        for_c(tv, [&](int r, int c, float &x) { Cc[(m0 + r) * LDM + n0 + c] = x; }, l);
+        for_c(z1, [&](int r, int c, float &x) { B8[(m0 + r) * LDM + n0 + c] = x; }, l);
+        if (has_s) for_c(z2, [&](int r, int c, float &x) { Dg[(m0 + r) * LDM + n0 + c] = x; }, l);
+    }
+    __syncthreads();
+    float *out = loc + ((size_t)chain * nc + ci) * kExLocMats * DD;
+    const int sib = D == 64 ? ib : w & 1, sn0 = D == 64 ? n0 : 0, sm0 = 16 * sib;
+    const int o0 = D == 64 ? 0 : w >> 1, ostep = D == 64 ? 1 : 4;
+    const float aL = cf.a[L - 1], bL = cf.beta[L - 1], hL = cf.h[L - 1];
+#pragma unroll 1
+    for (int o = o0; o < 6; o += ostep) {   // matrix 2 * destination + source, then C_M, C_S
+        if (!has_s && (o == 1 || o == 2 || o == 3 || o == 5)) continue;
+        const float *wv = (o == 2 || o == 3 || o == 5) ? cv.wS : cv.wM, *Z = o >= 4 ? Cc : (o & 1) ? Dg : B8;
+        Strip x = zero_strip();
+        mma(x, [&](int m, int kk) { return Z[kk * LDM + sm0 + m]; }, [&](int kk, int n) { return wv[kk] * Ks[kk * LDM + sn0 + n]; }, l);
+        const float dg = o == 0 ? aL : o == 1 ? bL : o == 3 ? hL : 0.f;
+        for_c(x, [&](int r, int c, float &y) { y = o >= 4 ? -y : sm0 + r == sn0 + c ? y + dg : y; }, l);
+        float *mat = out + (size_t)o * DD;
+#pragma unroll
+        for (int tl = 0; tl < 2; tl++) {
+            if (o < 4) store_operand_tile<D>(mat, x.t[tl], sib, sn0 / 16 + tl, l);
+            else store_acc_tile<D>(mat, x.t[tl], sib, sn0 / 16 + tl, l);
+        }
+    }
+}
+constexpr size_t kExFwdLds = 6 * MAT * sizeof(float);
+
 template <class K>
 void set_lds(K kernel, size_t bytes) {
     check_hip(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -656,91 +732,161 @@ void set_lds(K kernel, size_t bytes) {
 
 }  // namespace
 
-bool exact_backward_mm_applies(int d, int C) { return d == HD && C >= 1 && C <= CW; }
+bool exact_mm_applies(int d, int C) { return (d == 64 || d == 32) && C >= 1 && C <= CW; }
 
-// Cost model from measurements on one MI355X: a chunk costs the two chunk-parallel kernels about 65 us of a compute
-// unit whatever its length, a scan step 2.7 us; the fused sequential kernel walks a chain's tokens at 0.6 us each on a
-// quarter of a compute unit's worth of workgroups (four per chain).
-bool exact_backward_mm_pays(int seq_len, int batch, int C) {
-    const int nc = ceil_div(seq_len, C), cus = compute_units();
-    const double t_mm = (double)ceil_div(batch * nc, cus) * 65.0 + nc * 2.7;
-    const double t_seq = (double)seq_len * 0.6 * ceil_div(batch * 4, cus);
+// A chunk of the matrix form spans as many whole checkpoint intervals as fit into 64 tokens: a chunk costs the same
+// whatever its length, and only the states at chunk starts are read.
+static int chunk_of(int C) { return C * (CW / C); }
+
+// Cost models from measurements on one MI355X (us).  A chunk costs the two chunk-parallel kernels of the backward about
+// 65 us of a compute unit (42 at head size 32) whatever its length, a scan step 1.3; the fused sequential kernel walks a
+// chain's tokens at 0.6 each on a quarter of a compute unit's worth of workgroups (four per chain, one at head size 32),
+// the kernel that reads a whole trajectory at 1.1.  Under a clip or a bound the test on the errors adds two launches to the
+// matrix form where the fused kernel's only adds one on its maxima.
+bool exact_backward_mm_pays(int seq_len, int batch, int d, int C, bool tested) {
+    const int nc = ceil_div(seq_len, chunk_of(C)), cus = compute_units();
+    const double t_mm = (double)ceil_div(batch * nc, cus) * (d == 64 ? 65.0 : 42.0) + nc * 1.3 + (tested ? 20.0 : 10.0);
+    const double t_seq = (double)seq_len * (C == 1 ? 1.1 : 0.6) * ceil_div(batch * (d == 64 ? 4 : 1), cus);
     return t_mm < t_seq;
 }
 
-bool exact_backward_mm(const char *fn, bool has_s, const float *k, const float *v, const float *q, const float *alpha,
-                       const float *theta, const float *eta, const float *m_ckpt, const float *s_ckpt, const float *d_y,
-                       float *d_k, float *d_v, float *d_q, float *d_alpha, float *d_theta, float *d_eta, float *d_m_initial,
-                       float *d_s_initial, int seq_len, int batch, int C, float error_clip, float m_norm_guard) {
+// The sequential forward takes 0.15 a token as long as its workgroups (four per chain, one at head size 32) fit the
+// chip.  The chunk maps cost 24 of a compute unit per chunk (16 at head size 32), a scan step 1.3, and the walk of the
+// chunks' tokens again 0.15 a token for whatever does not run at the same time.
+bool exact_forward_mm_pays(int seq_len, int batch, int d) {
+    const int nc = ceil_div(seq_len, CW), cus = compute_units(), parts = d == 64 ? 4 : 1;
+    if (nc < 3) return false;
+    const double t_mm = (double)ceil_div(batch * (nc - 1), cus) * (d == 64 ? 24.0 : 16.0) + nc * 1.3 + 8.0 +
+                        0.15 * CW * ceil_div((long long)batch * nc * parts, cus);
+    const double t_seq = 0.15 * seq_len * ceil_div(batch * parts, cus);
+    return t_mm < t_seq;
+}
+
+template <int D>
+static void forward_states_t(bool has_s, const float *k, const float *v, const float *alpha, const float *theta, const float *eta,
+                             const float *m_initial, const float *s_initial, long long m_stride, float *m_states, float *s_states,
+                             long long state_stride, int sstep, int seq_len, int input_stride, int batch) {
     const ErrorScope es;
-    if (seq_len <= 0 || batch <= 0 || !exact_backward_mm_applies(HD, C)) {
-        fail("%s: the matrix form needs seq_len=%d and batch=%d positive and a checkpoint interval %d in [1, %d].", fn, seq_len, batch,
-             C, CW);
-        return true;
+    const int nc = ceil_div(seq_len, CW);
+    float *loc = scratch(32, (size_t)batch * nc * kExLocMats * D * D * sizeof(float));
+    static bool attr_set = false;
+    if (!attr_set) {
+        set_lds(ex_fwd_local_kernel<D>, kExFwdLds);
+        attr_set = true;
     }
-    const int nc = ceil_div(seq_len, C), nck = n_ckpt_count(seq_len, C);
+    if (es.failed()) return;
+    {
+        KernelTimer kt("ex_fwd_local_kernel");
+        hipLaunchKernelGGL(ex_fwd_local_kernel<D>, dim3((unsigned)batch * (nc - 1)), dim3(kThr), kExFwdLds, stream(), k, v, alpha, theta,
+                           has_s ? eta : alpha, loc, seq_len, input_stride, CW, nc, (int)has_s);
+        check_launch("ex_fwd_local_kernel");
+    }
+    KernelTimer kt("ex_scan_kernel");
+    const dim3 grid((unsigned)batch * (D / 16));
+    if (has_s)
+        hipLaunchKernelGGL((ex_scan_kernel<D, true, false>), grid, dim3(8 * D), 0, stream(), loc, m_initial, s_initial, m_stride,
+                           m_states, s_states, state_stride, sstep, nullptr, nullptr, nc);
+    else
+        hipLaunchKernelGGL((ex_scan_kernel<D, false, false>), grid, dim3(4 * D), 0, stream(), loc, m_initial, nullptr, m_stride,
+                           m_states, nullptr, state_stride, sstep, nullptr, nullptr, nc);
+    check_launch("ex_scan_kernel");
+}
+
+void exact_forward_states(bool has_s, int d, const float *k, const float *v, const float *alpha, const float *theta, const float *eta,
+                          const float *m_initial, const float *s_initial, long long m_stride, float *m_states, float *s_states,
+                          long long state_stride, int sstep, int seq_len, int input_stride, int batch) {
+    if (d == 64)
+        forward_states_t<64>(has_s, k, v, alpha, theta, eta, m_initial, s_initial, m_stride, m_states, s_states, state_stride, sstep,
+                             seq_len, input_stride, batch);
+    else
+        forward_states_t<32>(has_s, k, v, alpha, theta, eta, m_initial, s_initial, m_stride, m_states, s_states, state_stride, sstep,
+                             seq_len, input_stride, batch);
+}
+
+template <int D>
+static bool backward_mm_t(const char *fn, bool has_s, const float *k, const float *v, const float *q, const float *alpha,
+                          const float *theta, const float *eta, const float *m_ckpt, const float *s_ckpt, const float *d_y,
+                          float *d_k, float *d_v, float *d_q, float *d_alpha, float *d_theta, float *d_eta, float *d_m_initial,
+                          float *d_s_initial, int seq_len, int batch, int interval, float error_clip, float m_norm_guard) {
+    const ErrorScope es;
+    constexpr size_t DD = (size_t)D * D;
+    const int C = chunk_of(interval), cstep = C / interval;
+    const int nc = ceil_div(seq_len, C), nck = interval == 1 ? seq_len + 1 : n_ckpt_count(seq_len, interval);
     const size_t nchunks = (size_t)batch * nc;
     const bool guard = error_clip > 0.f || m_norm_guard > 0.f;
     ChainTracks tracks{nullptr, nullptr};
     if (guard) tracks = chain_tracks(seq_len, batch, C);
-    float *loc = scratch(32, nchunks * kExLocMats * kDD * sizeof(float));
+    float *loc = scratch(32, nchunks * kExLocMats * DD * sizeof(float));
     float *Tg = scratch(33, nchunks * kDD * sizeof(float));
     float *Ug = scratch(34, nchunks * kDD * sizeof(float));
     float *dUg = scratch(35, nchunks * kDD * sizeof(float));
-    float *locs = scratch(4, nchunks * 4 * sizeof(float));
-    float *em = scratch(5, (size_t)batch * (nc + 1) * kDD * sizeof(float));
-    float *esn = has_s ? scratch(6, (size_t)batch * (nc + 1) * kDD * sizeof(float)) : nullptr;
+    float *em = scratch(5, (size_t)batch * (nc + 1) * DD * sizeof(float));
+    float *esn = has_s ? scratch(6, (size_t)batch * (nc + 1) * DD * sizeof(float)) : nullptr;
     float *xs = scratch(7, nchunks * CW * CW * sizeof(float));
     float *pvec = scratch(8, (size_t)batch * seq_len * 4 * sizeof(float));
     float *scal = scratch(9, nchunks * 4 * sizeof(float));
     const int per = 8, rows = ceil_div(batch, per), nsum = has_s ? 2 : 1;
-    float *tmp = scratch(10, (size_t)nsum * rows * kDD * sizeof(float));
-    float *first = scratch(36, (size_t)2 * batch * kDD * sizeof(float));
+    float *tmp = scratch(10, (size_t)nsum * rows * DD * sizeof(float));
+    float *first = scratch(36, (size_t)2 * batch * DD * sizeof(float));
     if (es.failed()) return true;
-    float *first_m = first, *first_s = first + (size_t)batch * kDD;
+    float *first_m = first, *first_s = first + (size_t)batch * DD;
     static bool attr_set = false;
     if (!attr_set) {
-        set_lds(ex_local_kernel<false>, kExLocalLds);
-        set_lds(ex_local_kernel<true>, kExLocalLds);
-        set_lds(ex_grads_kernel, kExGradsLds);
+        set_lds(ex_local_kernel<D, false>, kExLocalLds);
+        set_lds(ex_local_kernel<D, true>, kExLocalLds);
+        set_lds(ex_grads_kernel<D>, kExGradsLds);
         attr_set = true;
     }
     if (es.failed()) return true;
     const int cus = compute_units(), pgrid = nchunks < (size_t)cus ? (int)nchunks : cus;   // one workgroup per compute unit (LDS)
+    const float *et = has_s ? eta : alpha;
     {
         KernelTimer kt("ex_local_kernel");
-        if (guard)
-            hipLaunchKernelGGL(ex_local_kernel<true>, dim3((unsigned)pgrid), dim3(kThr), kExLocalLds, stream(), k, v, q, d_y,
-                               alpha, theta, eta, m_ckpt, s_ckpt, loc, locs, Tg, Ug, dUg, seq_len, C, nc, nck, (int)has_s, (int)nchunks, tracks);
-        else
-            hipLaunchKernelGGL(ex_local_kernel<false>, dim3((unsigned)pgrid), dim3(kThr), kExLocalLds, stream(), k, v, q, d_y,
-                               alpha, theta, eta, m_ckpt, s_ckpt, loc, locs, Tg, Ug, dUg, seq_len, C, nc, nck, (int)has_s, (int)nchunks, tracks);
+        auto kernel = guard ? ex_local_kernel<D, true> : ex_local_kernel<D, false>;
+        hipLaunchKernelGGL(kernel, dim3((unsigned)pgrid), dim3(kThr), kExLocalLds, stream(), k, v, q, d_y, alpha, theta, et,
+                           m_ckpt, s_ckpt, loc, Tg, Ug, dUg, seq_len, C, nc, nck, cstep, (int)has_s, (int)nchunks, tracks);
         check_launch("ex_local_kernel");
     }
     {
         KernelTimer kt("ex_scan_kernel");
+        const dim3 grid((unsigned)batch * (D / 16));
+        const long long stride = (long long)(nc + 1) * DD;
         if (has_s)
-            hipLaunchKernelGGL(ex_scan_kernel<true>, dim3((unsigned)batch * 4), dim3(kThr), 0, stream(), loc, locs, em, esn,
-                               first_m, first_s, nc);
+            hipLaunchKernelGGL((ex_scan_kernel<D, true, true>), grid, dim3(8 * D), 0, stream(), loc, nullptr, nullptr, 0LL, em, esn,
+                               stride, 1, first_m, first_s, nc);
         else
-            hipLaunchKernelGGL(ex_scan_kernel<false>, dim3((unsigned)batch * 4), dim3(kThr), 0, stream(), loc, locs, em, esn,
-                               first_m, first_s, nc);
+            hipLaunchKernelGGL((ex_scan_kernel<D, false, true>), grid, dim3(4 * D), 0, stream(), loc, nullptr, nullptr, 0LL, em, nullptr,
+                               stride, 1, first_m, nullptr, nc);
         check_launch("ex_scan_kernel");
     }
     {
         KernelTimer kt("ex_grads_kernel");
-        hipLaunchKernelGGL(ex_grads_kernel, dim3((unsigned)pgrid), dim3(kThr), kExGradsLds, stream(), k, q, d_y, alpha, theta,
-                           eta, m_ckpt, s_ckpt, Tg, Ug, dUg, em, esn, d_k, d_v, d_q, d_theta, pvec, xs, scal, seq_len, C, nc, nck,
+        hipLaunchKernelGGL(ex_grads_kernel<D>, dim3((unsigned)pgrid), dim3(kThr), kExGradsLds, stream(), k, q, d_y, alpha, theta,
+                           et, m_ckpt, s_ckpt, Tg, Ug, dUg, em, esn, d_k, d_v, d_q, d_theta, pvec, xs, scal, seq_len, C, nc, nck, cstep,
                            (int)has_s, (int)nchunks);
         check_launch("ex_grads_kernel");
     }
-    chunkwise_gate_gradients(alpha, eta, pvec, xs, scal, d_alpha, d_eta, seq_len, batch, C, has_s, first_m, first_s, kDD, per,
-                             nsum, tmp);
+    chunkwise_gate_gradients(alpha, eta, pvec, xs, scal, d_alpha, d_eta, seq_len, batch, C, has_s, first_m, first_s, DD, per,
+                             nsum, tmp, (int)DD);
     if (es.failed()) return true;
-    if (guard && couplings_may_fire_tracked(k, alpha, theta, eta, tracks, has_s, seq_len, batch, C, error_clip, m_norm_guard))
+    if (guard && couplings_may_fire_tracked(k, alpha, theta, eta, tracks, has_s, seq_len, batch, C, error_clip, m_norm_guard, D))
         return false;
-    accumulate_over_batch2(tmp, d_m_initial, has_s ? tmp + (size_t)rows * kDD : nullptr, d_s_initial, rows, (int)kDD);
+    accumulate_over_batch2(tmp, d_m_initial, has_s ? tmp + (size_t)rows * DD : nullptr, d_s_initial, rows, (int)DD);
     return true;
+}
+
+bool exact_backward_mm(const char *fn, bool has_s, int d, const float *k, const float *v, const float *q, const float *alpha,
+                       const float *theta, const float *eta, const float *m_ckpt, const float *s_ckpt, const float *d_y,
+                       float *d_k, float *d_v, float *d_q, float *d_alpha, float *d_theta, float *d_eta, float *d_m_initial,
+                       float *d_s_initial, int seq_len, int batch, int C, float error_clip, float m_norm_guard) {
+    if (seq_len <= 0 || batch <= 0 || !exact_mm_applies(d, C)) {
+        fail("%s: the matrix form needs seq_len=%d and batch=%d positive, head size %d of 64 or 32 and a checkpoint interval %d in [1, %d].",
+             fn, seq_len, batch, d, C, CW);
+        return true;
+    }
+    return (d == 64 ? backward_mm_t<64> : backward_mm_t<32>)(fn, has_s, k, v, q, alpha, theta, eta, m_ckpt, s_ckpt, d_y, d_k, d_v, d_q,
+                                                             d_alpha, d_theta, d_eta, d_m_initial, d_s_initial, seq_len, batch, C,
+                                                             error_clip, m_norm_guard);
 }
 
 }  // namespace nlh

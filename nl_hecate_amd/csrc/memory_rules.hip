@@ -43,7 +43,8 @@ static __global__ void zero_fill_kernel(float *__restrict__ p, size_t n) {
 // errors of a chunk are taken against the chunk-start M; ckpt_interval is the
 // chunk size and the stored checkpoints are the chunk-boundary states.
 // MODE: 0 rows split over workgroups, 1 COUPLED (clip / projection: a chain in one workgroup), 2 as 0 and keeps the
-// bound of max_t |M_t|_F^2 that FwdArgs::msq_part describes.
+// bound of max_t |M_t|_F^2 that FwdArgs::msq_part describes, 3 as 0 over the runs of FwdArgs::sub_chunks (a mode of its
+// own: the straight-line tile code of mode 0 schedules 15 % worse with the runs' conditions in it).
 template <int D, int RPL, bool HAS_S, int STORE, int MODE, bool FROZEN>
 __global__ __launch_bounds__(kThreads) void rule_fwd_kernel(FwdArgs a) {
     constexpr bool COUPLED = MODE == 1, TRACK = MODE == 2;
@@ -66,16 +67,29 @@ __global__ __launch_bounds__(kThreads) void rule_fwd_kernel(FwdArgs a) {
     map_block(a.parts, chain, part);
     const int row_local = (wave * RG + g) * RPL;
     const int row0 = part * ROWS_WG + row_local;
+    // a run of a chain (FwdArgs::sub_chunks): tokens [sub0, sub0 + seq_len) from the state in its slot
+    constexpr bool sub = MODE == 3;
+    int sub0 = 0, seq_len = a.seq_len;
+    bool sub_last = true;
+    if constexpr (sub) {
+        const int run = chain % a.sub_chunks;
+        chain /= a.sub_chunks;
+        sub0 = run * kExactChunk;
+        seq_len = min(kExactChunk, a.seq_len - sub0);
+        sub_last = run == a.sub_chunks - 1;
+    }
 
-    const float *kb = a.k + (size_t)chain * a.input_stride * D;
-    const float *vb = a.v + (size_t)chain * a.input_stride * D;
-    const float *qb = a.q + (size_t)chain * a.input_stride * D;
-    const float *ab = a.alpha + (size_t)chain * a.input_stride;
-    const float *tb = a.theta + (size_t)chain * a.input_stride;
-    const float *eb = HAS_S ? a.eta + (size_t)chain * a.input_stride : nullptr;
-    float *yb = a.y + (size_t)chain * a.seq_len * D;
-    float *mo = a.m_out + (size_t)chain * a.state_stride;
-    float *so = HAS_S ? a.s_out + (size_t)chain * a.state_stride : nullptr;
+    const size_t in0 = (size_t)chain * a.input_stride + sub0;
+    const float *kb = a.k + in0 * D;
+    const float *vb = a.v + in0 * D;
+    const float *qb = a.q + in0 * D;
+    const float *ab = a.alpha + in0;
+    const float *tb = a.theta + in0;
+    const float *eb = HAS_S ? a.eta + in0 : nullptr;
+    float *yb = a.y + ((size_t)chain * a.seq_len + sub0) * D;
+    const size_t slot0 = (size_t)chain * a.state_stride + (size_t)(STORE == STORE_CKPT && sub ? sub0 / a.ckpt_interval : sub0) * DD;
+    float *mo = a.m_out + slot0;
+    float *so = HAS_S ? a.s_out + slot0 : nullptr;
 
     float4 M[RPL], S[RPL], M0[FROZEN ? RPL : 1];
     bool valid[RPL];
@@ -86,10 +100,13 @@ __global__ __launch_bounds__(kThreads) void rule_fwd_kernel(FwdArgs a) {
         S[r] = f4_zero();
         if (valid[r]) {
             size_t off = (size_t)(row0 + r) * D + cb * 4;
-            M[r] = *reinterpret_cast<const float4 *>(a.m_initial + (size_t)chain * a.m_stride + off);
-            if (HAS_S)
-                S[r] = *reinterpret_cast<const float4 *>(a.s_initial + (size_t)chain * a.m_stride + off);
-            if (STORE != STORE_NONE) {
+            const float *mi = sub ? mo : a.m_initial + (size_t)chain * a.m_stride;
+            M[r] = *reinterpret_cast<const float4 *>(mi + off);
+            if (HAS_S) {
+                const float *si = sub ? so : a.s_initial + (size_t)chain * a.m_stride;
+                S[r] = *reinterpret_cast<const float4 *>(si + off);
+            }
+            if (STORE != STORE_NONE && !sub) {
                 *reinterpret_cast<float4 *>(mo + off) = M[r];
                 if (HAS_S) *reinterpret_cast<float4 *>(so + off) = S[r];
             }
@@ -101,7 +118,6 @@ __global__ __launch_bounds__(kThreads) void rule_fwd_kernel(FwdArgs a) {
         for (int r = 0; r < RPL; r++) M0[r] = M[r];
     }
 
-    const int seq_len = a.seq_len;
     const int ntiles = (seq_len + TB - 1) / TB;
     const bool clip_on = COUPLED && a.error_clip > 0.f;
     const bool mn_on = COUPLED && mnorm_active(a.m_norm_max);
@@ -201,7 +217,7 @@ __global__ __launch_bounds__(kThreads) void rule_fwd_kernel(FwdArgs a) {
                 if (STORE == STORE_TRAJ) {
 #pragma unroll
                     for (int r = 0; r < RPL; r++)
-                        if (ALL_VALID || valid[r]) {
+                        if ((ALL_VALID || valid[r]) && (!sub || sub_last || t + 1 < kExactChunk)) {
                             size_t off = (size_t)(t + 1) * DD + (size_t)(row0 + r) * D + cb * 4;
                             *reinterpret_cast<float4 *>(mo + off) = M[r];
                             if (HAS_S) *reinterpret_cast<float4 *>(so + off) = S[r];
@@ -214,7 +230,7 @@ __global__ __launch_bounds__(kThreads) void rule_fwd_kernel(FwdArgs a) {
                         if (STORE == STORE_CKPT) {
 #pragma unroll
                             for (int r = 0; r < RPL; r++)
-                                if (ALL_VALID || valid[r]) {
+                                if ((ALL_VALID || valid[r]) && (!sub || sub_last || t + 1 < kExactChunk)) {
                                     size_t off = (size_t)ckpt_slot * DD + (size_t)(row0 + r) * D + cb * 4;
                                     *reinterpret_cast<float4 *>(mo + off) = M[r];
                                     if (HAS_S) *reinterpret_cast<float4 *>(so + off) = S[r];
@@ -565,6 +581,8 @@ void accumulate_over_batch2(const float *src_a, float *dst_a, const float *src_b
     check_launch("accumulate_over_batch2_kernel");
 }
 
+static int g_exact_form = 0;   // nlh_exact_backward_form
+
 bool coupled_needed(float error_clip, float m_norm_max) {
     return error_clip > 0.f || (m_norm_max > 0.f && m_norm_max < 1e30f);
 }
@@ -599,6 +617,13 @@ template <int D, int RPL, bool HAS_S, int STORE, bool FROZEN>
 static void launch_fwd_c(const FwdArgs &a, int batch, bool coupled) {
     dim3 grid(batch * a.parts), block(kThreads);
     KernelTimer kt("rule_fwd_kernel");
+    if constexpr (!FROZEN && STORE != STORE_NONE && (D == 64 || D == 32)) {
+        if (a.sub_chunks > 1) {
+            hipLaunchKernelGGL((rule_fwd_kernel<D, RPL, HAS_S, STORE, 3, FROZEN>), grid, block, 0, stream(), a);
+            check_launch("rule_fwd_kernel");
+            return;
+        }
+    }
     if (coupled)
         hipLaunchKernelGGL((rule_fwd_kernel<D, RPL, HAS_S, STORE, 1, FROZEN>), grid, block, 0, stream(), a);
     else if (a.msq_part)
@@ -655,6 +680,21 @@ static bool launch_fwd(FwdArgs a, int d, int batch) {
         if (!norm_bound_exceeded(u.msq_part, batch, parts, a.m_norm_max)) return true;
     }
     a.msq_part = nullptr;
+    // few long chains leave the sequential walk's chip idle: chunk-start states by the matrix form's scan, then all
+    // chunks' tokens at once
+    if constexpr (!FROZEN && STORE != STORE_NONE) {
+        const bool kept = STORE == STORE_TRAJ || kExactChunk % a.ckpt_interval == 0;   // the slots of all chunk starts exist
+        if (!coupled && kept && exact_mm_applies(d, 1) && g_exact_form != 2 &&
+            (g_exact_form == 1 ? a.seq_len > kExactChunk : exact_forward_mm_pays(a.seq_len, batch, d))) {
+            const ErrorScope es;
+            const int sstep = STORE == STORE_TRAJ ? kExactChunk : kExactChunk / a.ckpt_interval;
+            exact_forward_states(HAS_S, d, a.k, a.v, a.alpha, a.theta, a.eta, a.m_initial, a.s_initial, a.m_stride, a.m_out, a.s_out,
+                                 a.state_stride, sstep, a.seq_len, a.input_stride, batch);
+            if (es.failed()) return true;
+            a.sub_chunks = ceil_div(a.seq_len, kExactChunk);
+            return launch_fwd_as<HAS_S, STORE, FROZEN>(a, d, batch * a.sub_chunks, false);
+        }
+    }
     return launch_fwd_as<HAS_S, STORE, FROZEN>(a, d, batch, coupled);
 }
 
@@ -835,7 +875,6 @@ static void backward_ckpt_replay(const float *k, const float *v, const float *q,
 
 // One-call checkpointed / chunkwise backward: fused on-chip replay when it
 // covers the case, the replay-through-memory schedule otherwise.
-static int g_exact_form = 0;   // nlh_exact_backward_form
 static void backward_ckpt_any(bool has_s, bool frozen, bool allow_fused,
                               const float *k, const float *v, const float *q,
                               const float *alpha, const float *theta, const float *eta,
@@ -857,22 +896,31 @@ static void backward_ckpt_any(bool has_s, bool frozen, bool allow_fused,
     // directly, and so does a call under a bound right after any other test of a bound that fired.
     const bool coupled = bound || error_clip > 0.f;
     static int skip_left = 0, skip_len = 0;
-    bool try_mm = allow_fused && !frozen && exact_backward_mm_applies(d, C) && g_exact_form != 2 &&
-                  (g_exact_form == 1 || exact_backward_mm_pays(seq_len, batch, C));
+    bool try_mm = allow_fused && !frozen && exact_mm_applies(d, C) && g_exact_form != 2 &&
+                  (g_exact_form == 1 || exact_backward_mm_pays(seq_len, batch, d, C, coupled));
     if (try_mm && coupled) {
         if (!guard_possible()) try_mm = false;
         else if (skip_left > 0) { skip_left--; try_mm = false; }
         else if (error_clip <= 0.f && last_test_fired) try_mm = false;
     }
     if (try_mm) {
-        if (exact_backward_mm(fn, has_s, k, v, q, alpha, theta, eta, m_ckpt, s_ckpt, d_y, d_k, d_v, d_q, d_alpha, d_theta,
+        if (exact_backward_mm(fn, has_s, d, k, v, q, alpha, theta, eta, m_ckpt, s_ckpt, d_y, d_k, d_v, d_q, d_alpha, d_theta,
                               d_eta, d_m_initial, d_s_initial, seq_len, batch, C, error_clip, bound ? m_norm_max : 0.f)) {
             if (coupled) skip_len = 0;
             return;
         }
         skip_len = skip_len ? (skip_len < 64 ? 2 * skip_len : 64) : 1;
         skip_left = skip_len;
-        allow_fused = false;   // the test fired: the fused kernel's own test would fire too
+        if (C > 1) allow_fused = false;   // the test fired: the fused kernel's own test would fire too
+    }
+    if (C == 1 && !frozen && allow_fused) {   // every state is there: nothing to replay
+        if (has_s)
+            titans_backward_f32_cuda(k, v, q, alpha, theta, eta, m_ckpt, s_ckpt, d_y, d_k, d_v, d_q, d_alpha, d_theta, d_eta,
+                                     d_m_initial, d_s_initial, seq_len, d, batch, error_clip);
+        else
+            delta_backward_f32_cuda(k, v, q, alpha, theta, m_ckpt, d_y, d_k, d_v, d_q, d_alpha, d_theta, d_m_initial, seq_len, d,
+                                    batch, error_clip);
+        return;
     }
     if (allow_fused && error_clip <= 0.f && (!bound || guard_possible()) &&
         backward_ckpt_fused(has_s, frozen, k, v, q, alpha, theta, eta, m_ckpt, s_ckpt, d_y, d_k, d_v,

@@ -418,12 +418,12 @@ def gpu_memory_backward(level_params: MemoryLevelParams, cfg: LevelConfig, mem_c
     dah, dth, deh = _zeros(B, s), _zeros(B, s), _zeros(B, s)
     d_m0, d_s0 = _zeros(dd), _zeros(dd)
     clip, mx = cfg.error_clip, cfg.m_norm_max
-    if kind in ("Delta", "DGD"):
-        D.call("delta_backward_f32_cuda", kh, vh, qh, ah, th, c.m_states, dyh, dkh, dvh, dqh, dah, dth, d_m0, s, hd,
-               B, clip)
+    if kind in ("Delta", "DGD"):   # a trajectory is a checkpoint per token; the DGD forward ran without the projection
+        D.call("delta_backward_ckpt_f32_rocm", kh, vh, qh, ah, th, c.m_states, dyh, dkh, dvh, dqh, dah, dth, d_m0, s, hd,
+               B, 1, clip, F32_MAX if kind == "DGD" else mx)
     elif kind == "Titans":
-        D.titans_backward_dd(kh, vh, qh, ah, th, eh, c.m_states, c.s_states, dyh, dkh, dvh, dqh, dah, dth, deh, d_m0,
-                             d_s0, s, hd, B, clip)
+        D.call("titans_backward_ckpt_f32_rocm", kh, vh, qh, ah, th, eh, c.m_states, c.s_states, dyh, dkh, dvh, dqh, dah,
+               dth, deh, d_m0, d_s0, s, hd, B, 1, clip, mx)
     elif kind == "DeltaChunkwise":
         D.call("delta_chunkwise_backward_f32_cuda", kh, vh, qh, ah, th, c.m_states, dyh, dkh, dvh, dqh, dah, dth,
                d_m0, s, hd, B, c.chunk_size, clip, mx)
