@@ -654,6 +654,36 @@ void dgd_fused_forward_f32_cuda(float *k_mem, const float *v_mem, float *q_mem, 
  * cache [cache_len, heads*hd]; q, out [1, heads*hd]; no weights are kept. */
 void swa_single_token_cuda(const uint16_t *q, const uint16_t *k_cache, const uint16_t *v_cache, uint16_t *out,
                            int cache_len, int num_heads, int head_dim, int window_size, int n_persistent);
+/* ── Groups of levels (additions): one launch per step of gpu_memory_forward / gpu_memory_backward for all levels that
+ * run the same rule on the same tokens, and the dense products around them as groups of equal shape.  fp32 throughout.
+ * linear_group: op 0: c_j [m,n] = a_j [m,k] b_j^T [n,k] (bit j of bf16_mask: c_j leaves as bf16);
+ *   op 1: c_0 [m,n] = sum_j a_j [m,k] b_j [k,n];  op 2: c_j [m,n] = a_j^T b_j with a_j [k,m], b_j [k,n].
+ *   Pointer arrays are host arrays of `count` <= 32 device pointers; row lengths multiples of 4. */
+void linear_group_f32_rocm(int op, int count, const float *const *a, const float *const *b, void *const *c,
+                           unsigned bf16_mask, int m, int n, int k);
+/* ptrs: host array of 14 device pointers per level: k, v, q [bs*s, d] (k, q normalised in place), w_alpha, b_alpha,
+ * w_theta, b_theta, w_eta, b_eta, then written: k_norms, q_norms, alpha, theta, eta [bs*s].  bounds: 4 per level: alpha
+ * floor / ceil, theta floor / ceil.  *_heads [levels*bs*nh, s, hd], [levels*bs*nh, s].  q_heads null: no q (its pointers
+ * are not read); eta_heads null: no momentum gate.  Width nh*hd at most 1024. */
+void level_group_inputs_f32_rocm(const void *const *ptrs, const float *bounds, int levels, float *k_heads, float *v_heads,
+                                 float *q_heads, float *alpha_heads, float *theta_heads, float *eta_heads, int bs, int s,
+                                 int nh, int hd, float eps);
+/* ptrs: 17 per level: k, v, q (normalised), k_norms, q_norms, alpha, theta, eta, then written: d_k, d_v, d_q [bs*s, d]
+ * with respect to the raw projections, d_w_alpha, d_b_alpha, d_w_theta, d_b_theta, d_w_eta, d_b_eta. */
+void level_group_grads_f32_rocm(const void *const *ptrs, const float *bounds, int levels, const float *d_k_heads,
+                                const float *d_v_heads, const float *d_q_heads, const float *d_alpha_heads,
+                                const float *d_theta_heads, const float *d_eta_heads, int bs, int s, int nh, int hd,
+                                float eps);
+/* initial [levels*chains, dd] = the levels' carried memories [chains, dd] */
+void level_group_states_gather_rocm(const float *const *contexts, int levels, float *initial, int chains, int dd);
+/* contexts[l] [chains, dd] = the states at states + chain * stride, clamped to Frobenius norm m_norm_max[l] */
+void level_group_states_final_rocm(const float *states, long long stride, float *const *contexts, const float *m_norm_max,
+                                   int levels, int chains, int dd);
+/* out [levels][bs*nh, s, hd] = the token-major x [bs*s, nh*hd], head-major, once per level */
+void level_group_heads_repeat_rocm(const float *x, float *out, int bs, int s, int nh, int hd, int levels);
+/* y_i += alpha * x_i for `count` tensors (host arrays of device pointers and sizes) */
+void saxpy_multi_rocm(float alpha, const float *const *x, float *const *y, const int *n, int count);
+
 /* One whole decode step (core/src/gpu_forward.rs:3377-3492 gpu_single_token_forward) in four launches: projections of
  * the embedded token, K and V rounded into row `pos` of the bf16 caches [max_len, d], attention over the cache, every
  * level's one-token step on its carried memory, combine, gate, output projection and unembedding.  Blocks until the

@@ -15,13 +15,15 @@ L2 normalisation of k and q, gate projections with their clamps, per-head layout
 memory carried into `context_m` under its Frobenius clamp; backward: the rule's backward per head, gate
 gradients summed over heads and masked where a gate sat on a clamp bound, back to token layout,
 normalisation backward, projection and gate weight gradients, d_embedded.  Tensors are float32 CUDA
-tensors (torch stands in for GpuBuf); every step is a call into libnl_hecate_rocm.so or a torch matmul
-for the projections (cublas_matmul_*_dd in the reference) — nothing is computed on the host.
+tensors (torch stands in for GpuBuf); every step is a call into libnl_hecate_rocm.so or, for the levels that do
+not run as a group, a torch matmul for the projections (cublas_matmul_*_dd in the reference) — nothing is computed
+on the host.  Delta, Titans and DGD levels with equal options run as one batch (forward_group, backward_group).
 
 Where the reference loops single-chain kernels over heads and refuses batch_size > 1 (checkpointed
 variants, gpu_forward.rs:1608-1703), the batched entry points of the library take every chain at once
 and any batch size.
 """
+import ctypes
 from dataclasses import dataclass, field
 from typing import Optional
 
@@ -29,6 +31,7 @@ import numpy as np
 import torch
 
 from . import dispatch as D
+from .ffi import lib
 from .mag_layer import MemoryLevelParams
 
 F32_MAX = 3.4028234663852886e38
@@ -104,6 +107,8 @@ class GpuMemoryCache:
     up_buf: Optional[torch.Tensor] = None
     fused_buf: Optional[torch.Tensor] = None
     cache_buf: Optional[torch.Tensor] = None
+    group: Optional["LevelGroup"] = None      # the batch of levels this one ran in, and its place there
+    group_index: int = 0
 
     def dgd_delta_norm(self, s, d, batch_size, num_heads):
         """|M k - v|_2 of the last token against the memory that token was written into
@@ -192,9 +197,13 @@ class LevelGrads:
     d_down_proj: Optional[torch.Tensor] = None
 
     @staticmethod
-    def zeros(d, device="cuda", intermediate=0):
+    def zeros(d, device="cuda", intermediate=0, cleared=True):
+        """One buffer behind all tensors; cleared=False where a backward of every gate writes all of them."""
+        sizes = [d * d] * 3 + [2 * d, 4] * 3
+        flat = (torch.zeros if cleared else torch.empty)(sum(sizes), dtype=torch.float32, device=device)
+        wk, wv, wq, wa, ba, wt, bt, we, be = flat.split(sizes)
+        g = LevelGrads(wk.view(d, d), wv.view(d, d), wq.view(d, d), wa, ba[:1], wt, bt[:1], we, be[:1])
         z = lambda *sh: torch.zeros(*sh, dtype=torch.float32, device=device)
-        g = LevelGrads(z(d, d), z(d, d), z(d, d), z(2 * d), z(1), z(2 * d), z(1), z(2 * d), z(1))
         if intermediate:
             g.d_gate_proj, g.d_up_proj, g.d_down_proj = z(intermediate, d), z(intermediate, d), z(d, intermediate)
         return g
@@ -252,6 +261,158 @@ def _sum_heads(cfg, g, bs, s):
     return out
 
 
+# ── levels as one batch ──────────────────────────────────────────────────────
+# Levels that run the same rule with the same options on the same tokens are independent memories: their projections are
+# one group of products, their glue one launch per step, and the rule one batch of levels * batch * heads chains.
+
+class LevelGroup:
+    """What a grouped forward leaves for the grouped backward: the head-major inputs of the rule, all levels stacked."""
+    __slots__ = ("heads", "gates", "m_states", "s_states", "interval", "levels", "kind")
+
+    def __init__(self, heads, gates, m_states, s_states, interval, levels, kind):
+        self.heads, self.gates, self.m_states, self.s_states = heads, gates, m_states, s_states
+        self.interval, self.levels, self.kind = interval, levels, kind
+
+
+def group_key(cfg, level_params, d, bs):
+    """Levels with equal keys can run as one batch; None: the level takes its own path."""
+    if (cfg.memory_rule not in ("titans", "delta", "dgd") or cfg.memory_layers != 1 or d > 1024 or cfg.head_dim % 4
+            or cfg.num_heads * cfg.head_dim != d or (cfg.proxy and cfg.memory_rule == "dgd")):
+        return None
+    for t in (level_params.w_k, level_params.w_v, level_params.w_q, level_params.w_alpha, level_params.w_theta,
+              level_params.w_eta):
+        if t.dtype != torch.float32 or not t.is_contiguous() or t.data_ptr() & 15:
+            return None
+    return (cfg.memory_rule, cfg.num_heads, cfg.head_dim, cfg.checkpoint_interval, cfg.proxy, cfg.chunk_size, cfg.error_clip,
+            cfg.m_norm_max)
+
+
+def _plain(t):
+    """Contiguous floats at a 16-byte boundary, which the grouped kernels read."""
+    return t.dtype == torch.float32 and t.is_contiguous() and not t.data_ptr() & 15
+
+
+def _ptrs(tensors):
+    return (ctypes.c_void_p * len(tensors))(*[t.data_ptr() for t in tensors])
+
+
+def _bounds(cfgs):
+    return (ctypes.c_float * (4 * len(cfgs)))(*[x for c in cfgs for x in (c.alpha_floor, c.alpha_ceil, c.theta_floor,
+                                                                          c.theta_ceil)])
+
+
+def linear_group(op, a, b, c, m, n, k, bf16_mask=0):
+    """Products of equal shape in one launch (linear_group_f32_rocm), 32 at a time."""
+    if op == 1:
+        lib.linear_group_f32_rocm(1, len(a), _ptrs(a), _ptrs(b), _ptrs(c), 0, m, n, k)
+        return
+    for i in range(0, len(a), 32):
+        lib.linear_group_f32_rocm(op, len(a[i:i + 32]), _ptrs(a[i:i + 32]), _ptrs(b[i:i + 32]), _ptrs(c[i:i + 32]),
+                                  (bf16_mask >> i) & 0xffffffff, m, n, k)
+
+
+def forward_group(params, cfgs, embedded, contexts, s, d, bs, extra=()):
+    """gpu_memory_forward of a group of levels.  extra: (weight, output) pairs of further projections of `embedded` (a bf16
+    output is rounded at the store).  Returns (y [levels, bs*s, d], [cache per level])."""
+    cfg, L = cfgs[0], len(cfgs)
+    nh, hd = cfg.num_heads, cfg.head_dim
+    n, B, dd = bs * s, bs * nh, hd * hd
+    titans = cfg.memory_rule == "titans"
+    proj = _new(3 * L, n, d)
+    mem = list(proj.unbind(0))
+    linear_group(0, [embedded] * (3 * L + len(extra)),
+                 [w for lp in params for w in (lp.w_k, lp.w_v, lp.w_q)] + [w for w, _ in extra], mem + [o for _, o in extra],
+                 n, d, d, sum(1 << (3 * L + i) for i, (_, o) in enumerate(extra) if o.dtype == torch.bfloat16))
+    gate = _new(5 * L, n)
+    rows = list(gate.unbind(0))   # per level: k_norms, q_norms, alpha, theta, eta
+    heads, gates = _new(3, L * B, s, hd), _new(3 if titans else 2, L * B, s)
+    h0, g0 = heads.data_ptr(), gates.data_ptr()
+    hs, gs = 4 * L * B * s * hd, 4 * L * B * s
+    lib.level_group_inputs_f32_rocm(
+        _ptrs([t for i, lp in enumerate(params) for t in (*mem[3 * i:3 * i + 3], lp.w_alpha, lp.b_alpha, lp.w_theta,
+                                                         lp.b_theta, lp.w_eta, lp.b_eta, *rows[5 * i:5 * i + 5])]),
+        _bounds(cfgs), L, h0, h0 + hs, h0 + 2 * hs, g0, g0 + gs, g0 + 2 * gs if titans else None, bs, s, nh, hd, 1e-8)
+    initial = contexts[0]
+    if L > 1:
+        initial = _new(L * B, dd)
+        lib.level_group_states_gather_rocm(_ptrs(contexts), L, initial.data_ptr(), B, dd)
+    yh, clip, mx, C = _new(L * B, s, hd), cfg.error_clip, F32_MAX if cfg.memory_rule == "dgd" else cfg.m_norm_max, cfg.checkpoint_interval
+    interval, form = 1, "" if C is None else "Ckpt"
+    if C is not None:
+        interval, slots = C, 1 + -(-s // C)
+    elif cfg.proxy:
+        interval, form = cfg.chunk_size or s, "Chunkwise"
+        slots = -(-s // interval) + 1
+    else:
+        slots = s + 1
+    m_states = _new(L * B, slots, dd)
+    s_states = _new(L * B, slots, dd) if titans else None
+    q = [h0, h0 + hs, h0 + 2 * hs, g0, g0 + gs]
+    if titans:
+        q += [g0 + 2 * gs, initial.data_ptr(), _zeros(L * B, dd).data_ptr(), m_states.data_ptr(), s_states.data_ptr(), yh.data_ptr()]
+    else:
+        q += [initial.data_ptr(), m_states.data_ptr(), yh.data_ptr()]
+    rule = "titans" if titans else "delta"
+    if form == "Ckpt":
+        getattr(lib, rule + "_forward_ckpt_batched_f32_rocm")(*q, s, hd, L * B, interval, clip, mx)
+    elif form == "Chunkwise":
+        getattr(lib, rule + "_chunkwise_forward_f32_cuda")(*q, s, hd, L * B, interval, clip, mx)
+    else:
+        getattr(lib, rule + "_forward_f32_cuda")(*q, s, hd, L * B, s, dd, clip, mx)
+    # copy_final_m_batch + m_norm_clamp_batch_f32_cuda (gpu_forward.rs:2824, :1431)
+    lib.level_group_states_final_rocm(m_states.data_ptr() + 4 * (slots - 1) * dd, slots * dd, _ptrs(contexts),
+                                      (ctypes.c_float * L)(*[c.m_norm_max for c in cfgs]), L, B, dd)
+    y = _new(L, n, d)
+    lib.transpose_heads_f32_cuda(yh.data_ptr(), y.data_ptr(), L * bs, s, nh, hd, 0)
+    kind = {"delta": "Delta", "titans": "Titans", "dgd": "DGD"}[cfg.memory_rule] + form
+    group = LevelGroup(heads, gates, m_states, s_states, interval, L, kind)
+    more = {"": {}, "Ckpt": dict(checkpoint_interval=C), "Chunkwise": dict(chunk_size=interval, num_chunks=slots - 1)}[form]
+    mst = m_states.split(B)
+    sst = s_states.split(B) if titans else [None] * L
+    caches = [GpuMemoryCache(kind, k_mem=mem[3 * i], v_mem=mem[3 * i + 1], q_mem=mem[3 * i + 2], k_norms=rows[5 * i],
+                             q_norms=rows[5 * i + 1], alpha=rows[5 * i + 2], theta=rows[5 * i + 3],
+                             eta=rows[5 * i + 4] if titans else None, m_states=mst[i], s_states=sst[i], group=group,
+                             group_index=i, **more) for i in range(L)]
+    return y, caches
+
+
+def backward_group(params, cfgs, caches, d_y, embedded, level_grads, s, d, bs, extra=()):
+    """gpu_memory_backward of a whole group: every level sees the same d_y [bs*s, d].  extra: (gradient, weight, weight
+    gradient) of further projections of `embedded`.  Fills the gradients and returns the sum of all input gradients."""
+    cfg, L, g = cfgs[0], len(cfgs), caches[0].group
+    nh, hd = cfg.num_heads, cfg.head_dim
+    n, B, dd = bs * s, bs * nh, hd * hd
+    titans = cfg.memory_rule == "titans"
+    dyh = _new(L * B, s, hd)
+    lib.level_group_heads_repeat_rocm(d_y.data_ptr(), dyh.data_ptr(), bs, s, nh, hd, L)
+    dh, dg, d_init = _new(3, L * B, s, hd), _new(3 if titans else 2, L * B, s), _zeros(2, dd)
+    h0, g0, e0, f0, i0 = (t.data_ptr() for t in (g.heads, g.gates, dh, dg, d_init))
+    hs, gs = 4 * L * B * s * hd, 4 * L * B * s
+    clip, mx = cfg.error_clip, F32_MAX if cfg.memory_rule == "dgd" else cfg.m_norm_max
+    if titans:
+        args = [h0, h0 + hs, h0 + 2 * hs, g0, g0 + gs, g0 + 2 * gs, g.m_states.data_ptr(), g.s_states.data_ptr(), dyh.data_ptr(),
+                e0, e0 + hs, e0 + 2 * hs, f0, f0 + gs, f0 + 2 * gs, i0, i0 + 4 * dd]
+    else:
+        args = [h0, h0 + hs, h0 + 2 * hs, g0, g0 + gs, g.m_states.data_ptr(), dyh.data_ptr(), e0, e0 + hs, e0 + 2 * hs, f0, f0 + gs, i0]
+    rule = "titans" if titans else "delta"
+    fn = rule + ("_chunkwise_backward_f32_cuda" if g.kind.endswith("Chunkwise") else "_backward_ckpt_f32_rocm")
+    getattr(lib, fn)(*args, s, hd, L * B, g.interval, clip, mx)
+    raw = list(_new(3 * L, n, d).unbind(0))   # d_k, d_v, d_q of the raw projections, per level
+    ptrs = []
+    for i, (c, lg) in enumerate(zip(caches, level_grads)):
+        eta = c.eta if titans else c.alpha     # not read without the momentum gate
+        ptrs += (c.k_mem, c.v_mem, c.q_mem, c.k_norms, c.q_norms, c.alpha, c.theta, eta, *raw[3 * i:3 * i + 3], lg.d_w_alpha,
+                 lg.d_b_alpha, lg.d_w_theta, lg.d_b_theta, lg.d_w_eta, lg.d_b_eta)
+    lib.level_group_grads_f32_rocm(_ptrs(ptrs), _bounds(cfgs), L, e0, e0 + hs, e0 + 2 * hs, f0, f0 + gs,
+                                   f0 + 2 * gs if titans else None, bs, s, nh, hd, 1e-8)
+    up = raw + [x for x, _, _ in extra]
+    linear_group(2, up, [embedded] * len(up),
+                 [w for lg in level_grads for w in (lg.d_w_k_mem, lg.d_w_v_mem, lg.d_w_q_mem)] + [w for _, _, w in extra], d, d, n)
+    d_embedded = _new(n, d)
+    linear_group(1, up, [w for lp in params for w in (lp.w_k, lp.w_v, lp.w_q)] + [w for _, w, _ in extra], [d_embedded], n, d, d)
+    return d_embedded
+
+
 def gpu_memory_forward(level_params: MemoryLevelParams, cfg: LevelConfig, embedded, context_m, s, d, batch_size):
     """embedded [bs*s, d]; context_m [bs*nh, hd*hd]: the level's carried memory per (batch, head), read as the
     initial state and overwritten with the final one.  Returns (y [bs*s, d], GpuMemoryCache)."""
@@ -275,6 +436,9 @@ def gpu_memory_forward(level_params: MemoryLevelParams, cfg: LevelConfig, embedd
             raise ValueError(f"{rule} forward with batch_size > 1 is not supported")
     elif not cfg.is_mlp_mem:
         assert tuple(context_m.shape) == (B, dd)
+    if group_key(cfg, lp, d, bs) is not None and _plain(embedded) and _plain(context_m):
+        y, caches = forward_group([lp], [cfg], embedded, [context_m], s, d, bs)
+        return y[0], caches[0]
     k_mem, v_mem, q_mem = embedded @ lp.w_k.t(), embedded @ lp.w_v.t(), embedded @ lp.w_q.t()
     k_norms, q_norms = _new(n), _new(n)
     D.call("l2_normalize_rows_f32_cuda", k_mem, k_norms, n, d, 1e-8)
@@ -408,6 +572,9 @@ def gpu_memory_backward(level_params: MemoryLevelParams, cfg: LevelConfig, mem_c
         return d_x
     if kind == "Mlp":
         return _mlp_backward(level_params, cfg, c, d_y, embedded, level_grads, s, d, bs)
+    if (c.group is not None and c.group.levels == 1 and group_key(cfg, level_params, d, bs) is not None and _plain(d_y)
+            and _plain(embedded)):
+        return backward_group([level_params], [cfg], [c], d_y, embedded, [level_grads], s, d, bs)
     has_theta, has_eta = not kind.startswith("Hebbian"), kind.startswith("Titans")
     dyh = _heads(cfg, d_y, bs, s)
     kh, vh, qh = (_heads(cfg, t, bs, s) for t in (c.k_mem, c.v_mem, c.q_mem))

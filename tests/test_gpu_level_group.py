@@ -1,0 +1,111 @@
+"""Groups of levels as one batch (csrc/level_group.hip, csrc/gemm_f32.hip): the grouped products at the edges of their
+tiles and splits against float64, the multi-tensor update, the register-held cross-entropy rows, and a grouped training
+step against the same step level by level (whose parity with the oracle has its own tests)."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from nl_hecate_amd import cms_model as GM
+from nl_hecate_amd import dispatch as D
+from nl_hecate_amd import memory_level as ML
+from nl_hecate_amd.ffi import lib
+from tests.gpu_util import dev, host
+from tests.test_gpu_cms_model import gpu_model, setup
+from nl_hecate_amd.cms import ContextState, Pulse
+
+pytestmark = pytest.mark.gpu
+f32 = np.float32
+
+
+@pytest.mark.parametrize("op,count,m,n,k", [(0, 1, 1, 4, 4), (0, 3, 65, 36, 100), (0, 2, 300, 260, 64), (0, 17, 129, 64, 32),
+                                            (0, 1, 70, 64, 8000), (1, 1, 5, 4, 4), (1, 7, 130, 128, 96), (1, 15, 512, 256, 256),
+                                            (2, 4, 64, 132, 777), (2, 1, 4, 4, 1), (2, 33, 32, 64, 50)])
+def test_grouped_products(op, count, m, n, k):
+    print(op, count, m, n, k, flush=True)
+    r = np.random.default_rng(m + n + k)
+    shp_a, shp_b = {0: ((m, k), (n, k)), 1: ((m, k), (k, n)), 2: ((k, m), (k, n))}[op]
+    A = [r.standard_normal(shp_a).astype(f32) for _ in range(count)]
+    B = [r.standard_normal(shp_b).astype(f32) for _ in range(count)]
+    a, b = [dev(x) for x in A], [dev(x) for x in B]
+    c = [torch.full((m, n), 7.5, device="cuda") for _ in range(1 if op == 1 else count)]
+    ML.linear_group(op, a, b, c, m, n, k)
+    want = {0: lambda: [x.astype(np.float64) @ y.T for x, y in zip(A, B)],
+            1: lambda: [sum(x.astype(np.float64) @ y for x, y in zip(A, B))],
+            2: lambda: [x.T.astype(np.float64) @ y for x, y in zip(A, B)]}[op]()
+    terms = k * (count if op == 1 else 1)
+    for got, w in zip(c, want):
+        # fp32 sums of `terms` products of unit normals: rounding grows like sqrt(terms) ulps of sums of size sqrt(terms)
+        assert np.abs(host(got) - w).max() <= 8 * 2 ** -24 * terms + 1e-6
+    if op == 0:
+        half = [torch.zeros(m, n, dtype=torch.bfloat16, device="cuda") for _ in range(count)]
+        ML.linear_group(0, a, b, half, m, n, k, (1 << count) - 1)
+        for h, got in zip(half, c):
+            assert (h.float() - got).abs().max().item() <= 2 ** -7 * got.abs().max().item()
+
+
+def test_saxpy_multi():
+    r = np.random.default_rng(3)
+    sizes = [1, 3, 4096, 4097, 5, 100000, 64] * 10
+    x, y = [[r.standard_normal(n).astype(f32) for n in sizes] for _ in range(2)]
+    xd, yd = [dev(t) for t in x], [dev(t) for t in y]
+    shifted = torch.zeros(8, device="cuda")   # an operand that is not at a 16-byte boundary
+    xd.append(dev(np.arange(5, dtype=f32)))
+    yd.append(shifted[1:6])
+    n = [t.numel() for t in xd]
+    lib.saxpy_multi_rocm(-0.25, ML._ptrs(xd), ML._ptrs(yd), (ctypes.c_int * len(n))(*n), len(n))
+    for a, b, g in zip(x, y, yd):
+        assert np.array_equal(host(g), (b + f32(-0.25) * a)) or np.abs(host(g) - (b - 0.25 * a)).max() <= 2 ** -23 * np.abs(b).max() * 2
+    assert np.array_equal(host(shifted), np.array([0, 0, -0.25, -0.5, -0.75, -1.0, 0, 0], f32))
+
+
+@pytest.mark.parametrize("s,v", [(5, 1024), (3, 8192), (4, 8196), (2, 32768), (3, 16388), (2, 32772)])
+def test_cross_entropy_rows(s, v):
+    r = np.random.default_rng(v)
+    x = (4 * r.standard_normal((s, v))).astype(f32)
+    t = r.integers(0, v, s).astype(np.int32)
+    t[0] = v - 1
+    if s > 2:
+        t[1] = -1
+    loss, g = torch.zeros(1, device="cuda"), torch.full((s, v), 3.0, device="cuda")
+    D.call("cross_entropy_forward_cuda", dev(x), dev(t), loss, s, v)
+    D.call("cross_entropy_backward_cuda", dev(x), dev(t), g, s, v, 0.5)
+    p = np.exp(x.astype(np.float64) - x.max(1, keepdims=True))
+    p /= p.sum(1, keepdims=True)
+    ok = t >= 0
+    want = -np.log(p[np.arange(s), t])[ok].sum()
+    assert abs(loss.item() - want) <= 1e-5 * want
+    p[np.arange(s), t] -= 1
+    assert np.abs(host(g) - 0.5 * p * ok[:, None]).max() <= 1e-6
+
+
+@pytest.mark.parametrize("rule,k,nh,hd,s,bs,kw", [
+    ("titans", 3, 2, 32, 70, 2, {}),
+    ("delta", 2, 4, 8, 33, 1, dict(alpha_floor=0.3, theta_ceil=0.04, m_norm_max=0.8)),
+    ("titans", 2, 3, 4, 40, 1, dict(checkpoint_interval=8, alpha_ceil=0.4)),
+    ("dgd", 2, 2, 16, 50, 1, dict(error_clip=0.2)),
+    ("titans", 2, 10, 64, 130, 1, dict(proxy=True, chunk_size=64, m_norm_max=50.0))])
+def test_grouped_step_against_level_by_level(rule, k, nh, hd, s, bs, kw, monkeypatch):
+    print(rule, k, nh, hd, s, bs, flush=True)
+    cfg, _, p, mem = setup(rule, k, nh, hd, 60, s, 16, bs=bs, **kw)
+    ids = [int(t) for t in np.random.default_rng(1).integers(0, 60, bs * s)]
+    out = []
+    for grouped in (True, False):
+        if not grouped:
+            for mod in (GM, ML):
+                monkeypatch.setattr(mod, "group_key", lambda *a: None)
+        gp, _ = gpu_model(p)
+        ctx = ContextState([dev(m.reshape(m.shape[0], hd * hd)) for m in mem])
+        loss, cache = GM.gpu_cms_forward(gp, cfg, ids, ids[1:] + ids[:1], Pulse(0, [True] * k), ctx)
+        assert (cache["memory_caches"][0].group is not None) == grouped
+        g = GM.gpu_cms_backward(gp, cfg, cache)
+        GM.gpu_weight_update(gp, g, 0.1)
+        vals = [torch.tensor([loss]), g.d_w_embed, g.d_w_q, g.d_w_k, g.d_w_v, g.d_w_o, g.d_w_unembed, gp.w_q, gp.w_embed, *ctx.memory]
+        for lg, lp, mc in zip(g.levels, gp.levels, cache["memory_caches"]):
+            vals += [lg.d_w_k_mem, lg.d_w_v_mem, lg.d_w_q_mem, lg.d_w_alpha, lg.d_b_alpha, lg.d_w_theta, lg.d_b_theta, lg.d_w_eta,
+                     lg.d_b_eta, lp.w_alpha, lp.w_k, mc.k_mem, mc.q_mem, mc.alpha, mc.theta, mc.m_states]
+        out.append([host(x) for x in vals])
+    for i, (a, b) in enumerate(zip(*out)):
+        # the attention's q, k, v may round to neighbouring bf16 where the products' sums differ in their last bits
+        assert np.abs(a - b).max() <= 2e-3 * max(np.abs(b).max(), 1e-6), i
