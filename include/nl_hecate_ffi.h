@@ -267,6 +267,15 @@ void delta_forward_ckpt_batched_f32_rocm(const float *k_mem, const float *v_mem,
                                          float error_clip, float m_norm_max);
 
 
+/* The states after the last token, without outputs or trajectory (no clip, no projection): what a prompt leaves in a
+ * memory.  k, v [batch, seq_len, d], gates [batch, seq_len], m_initial / m_final [batch, d*d]; s_initial may be null
+ * (zero momentum). */
+void titans_final_states_f32_rocm(const float *k_mem, const float *v_mem, const float *alpha, const float *theta,
+                                  const float *eta, const float *m_initial, const float *s_initial, float *m_final,
+                                  int seq_len, int d, int batch_size);
+void delta_final_states_f32_rocm(const float *k_mem, const float *v_mem, const float *alpha, const float *theta,
+                                 const float *m_initial, float *m_final, int seq_len, int d, int batch_size);
+
 /* ── Checkpointed backward (addition) ───────────────────────────────────────
  * Replaces the host loop titans_backward_checkpointed /
  * delta_backward_checkpointed (core/src/gpu_backward.rs:1770-1962): one call

@@ -34,7 +34,7 @@ struct DecLevel {
     float *memory;               // [heads, hd*hd]
     float *k, *v, *q, *y;        // [d] each, in the work buffer
     float alpha_floor, alpha_ceil, theta_floor, theta_ceil, clip, m_norm;
-    int rule;                    // -1 frozen (read only), 0 Hebbian, 1 Delta / Titans, 2 DGD
+    int rule;                    // -1 frozen (read only), 0 Hebbian, 1 Delta / Titans, 2 DGD, 3 read with the normalised q
 };
 struct DecArgs {
     const float *x;              // the token's embedding row
@@ -56,6 +56,8 @@ __device__ __forceinline__ uint16_t f2bf(float x) {   // round to nearest even; 
 }
 __device__ __forceinline__ float dot4(const float4 &a, const float4 &b) { return a.x * b.x + a.y * b.y + a.z * b.z + a.w * b.w; }
 
+__host__ __device__ inline bool reads_only(int rule) { return rule < 0 || rule == 3; }
+
 // Segments of d rows in the order: attention q, k, v, then per active level k, v, q, per frozen level q.
 __global__ __launch_bounds__(kDecThr) void decode_project_kernel(DecArgs a) {
     const int lane = threadIdx.x & 63, wave = (blockIdx.x * kDecThr + threadIdx.x) >> 6;
@@ -69,12 +71,12 @@ __global__ __launch_bounds__(kDecThr) void decode_project_kernel(DecArgs a) {
     else {
         int s = seg - 3, l = 0;
         for (; l < a.levels; l++) {
-            const int n = a.lv[l].rule < 0 ? 1 : 3;
+            const int n = reads_only(a.lv[l].rule) ? 1 : 3;
             if (s < n) break;
             s -= n;
         }
         if (l == a.levels) return;
-        if (a.lv[l].rule < 0) s = 2;
+        if (reads_only(a.lv[l].rule)) s = 2;
         w = s == 0 ? a.lv[l].w_k : s == 1 ? a.lv[l].w_v : a.lv[l].w_q;
         out = s == 0 ? a.lv[l].k : s == 1 ? a.lv[l].v : a.lv[l].q;
     }
@@ -136,10 +138,15 @@ __device__ __forceinline__ void level_head(const DecArgs &a, int l, int h, float
 #pragma unroll
     for (int i = 0; i < NP; i++) qv[i] = qh[LPR * i];
     float y = 0.f;
-    if (lv.rule < 0) {   // frozen: y = M q with the raw projection
+    if (reads_only(lv.rule)) {   // y = M q, with the raw projection for a frozen level
+        float n2[1] = {0.f};
+        if (lv.rule == 3) {
+            for (int i = tid; i < d; i += kDecThr) n2[0] += lv.q[i] * lv.q[i];
+            block_sums(n2, red);
+        }
 #pragma unroll
         for (int i = 0; i < NP; i++) y += dot4(m[i], qv[i]);
-        y = group_allreduce<LPR>(y);
+        y = group_allreduce<LPR>(y) * (lv.rule == 3 ? 1.f / fmaxf(sqrtf(n2[0]), 1e-8f) : 1.f);
         if (c == 0) lv.y[hoff + row] = y;
         return;
     }
@@ -469,7 +476,7 @@ int decode_token_rocm(const float *embedding_row, const float *w_q, const float 
         p += 4 * d;
         lv.alpha_floor = b[0]; lv.alpha_ceil = b[1]; lv.theta_floor = b[2]; lv.theta_ceil = b[3]; lv.clip = b[4]; lv.m_norm = b[5];
         lv.rule = level_rule[l];
-        segs += lv.rule < 0 ? 1 : 3;
+        segs += reads_only(lv.rule) ? 1 : 3;
     }
     a.part_o = p; p += (size_t)a.slices * d;
     a.part_ml = p; p += (size_t)a.slices * heads * 2;

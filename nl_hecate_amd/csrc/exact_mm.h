@@ -18,10 +18,11 @@ bool exact_backward_mm(const char *fn, bool has_s, int d, const float *k, const 
                        float *d_s_initial, int seq_len, int batch, int C, float error_clip, float m_norm_guard);
 
 // Forward: the states at the starts of all 64-token chunks, chunk c's at element offset c * sstep * d*d of its chain's
-// m_states / s_states (chain stride state_stride), from the initial states (chain stride m_stride).  No clip, no
-// projection.  The chunks' tokens are then independent walks (FwdArgs::sub_chunks).
+// m_states / s_states (chain stride state_stride), from the initial states (chain stride m_stride; s_initial null: zero).
+// No clip, no projection.  The chunks' tokens are then independent walks (FwdArgs::sub_chunks).  sstep 0: the states after
+// the last token instead.
 constexpr int kExactChunk = 64;
-bool exact_forward_mm_pays(int seq_len, int batch, int d);
+bool exact_forward_mm_pays(int seq_len, int batch, int d, bool final_only);
 void exact_forward_states(bool has_s, int d, const float *k, const float *v, const float *alpha, const float *theta, const float *eta,
                           const float *m_initial, const float *s_initial, long long m_stride, float *m_states, float *s_states,
                           long long state_stride, int sstep, int seq_len, int input_stride, int batch);

@@ -292,7 +292,7 @@ constexpr size_t kExLocalLds = 9 * MAT * sizeof(float);
 // REV: adjoints, last chunk first, from zero; states [chain][nc + 1][D*D]: slot c = adjoint of the state at the start of
 // chunk c (slot nc = 0, slot 0 = the gradient of the initial state, also written to first [chain][D*D]).
 // Forward: the states themselves from the initial ones; chunk c's start state goes to slot c * sstep of the chain's
-// states (the last chunk's end state is left to the pass that walks its tokens).
+// states, for as many chunks as there are steps (sstep 0: only the last one stays).
 // One wave per (destination, 16 columns): both sources' contributions, 2 D / 16 products of 16 x 16 x 16, so a step needs
 // no exchange of partial sums and, with X in two LDS buffers, one barrier.  The second operand comes straight from memory
 // in the lane order of the product (store_operand_tile), the additive term in accumulator order: every load is 1 KB of
@@ -305,7 +305,7 @@ template <int D, bool HAS_S, bool REV>
 __global__ __launch_bounds__((HAS_S ? 2 : 1) * D * 4) void ex_scan_kernel(
     const float *__restrict__ loc, const float *__restrict__ m_initial, const float *__restrict__ s_initial, long long m_stride,
     float *__restrict__ mst, float *__restrict__ sst, long long state_stride, int sstep, float *__restrict__ first_m,
-    float *__restrict__ first_s, int nc) {
+    float *__restrict__ first_s, int nc, int steps) {
     constexpr int NS = HAS_S ? 2 : 1, NT = D / 16, NB = D / 16, LDX = D + 4, DD = D * D;
     __shared__ __align__(16) float X[2][NS][16 * LDX];
     // the row blocks of a chain sit 8 workgroups apart: consecutive workgroups go to consecutive XCDs, so they share one
@@ -319,9 +319,12 @@ __global__ __launch_bounds__((HAS_S ? 2 : 1) * D * 4) void ex_scan_kernel(
     float *st = (dst ? sst : mst) + (size_t)chain * state_stride + at;
     f32x4 x = {0.f, 0.f, 0.f, 0.f};
     if (!REV) {
-        const float *in = (dst ? s_initial : m_initial) + (size_t)chain * m_stride + at;
+        const float *in = dst ? s_initial : m_initial;
+        if (in) {   // no initial momentum: zero
+            in += (size_t)chain * m_stride + at;
 #pragma unroll
-        for (int i = 0; i < 4; i++) x[i] = in[i * D];
+            for (int i = 0; i < 4; i++) x[i] = in[i * D];
+        }
     }
 #pragma unroll
     for (int i = 0; i < 4; i++) {
@@ -339,7 +342,6 @@ __global__ __launch_bounds__((HAS_S ? 2 : 1) * D * 4) void ex_scan_kernel(
             for (int j = 0; j < NB; j++) r.b[sr][j] = p[(HAS_S ? dst * 2 + sr : 0) * (DD / 4) + (ct * NB + j) * 64];
         r.c = p[(4 + dst) * (DD / 4) + (rb * NT + ct) * 64];
     };
-    const int steps = REV ? nc : nc - 1;
     auto step = [&](Step &r, int i) {
         const float *Xr = X[i & 1][0] + (l & 15) * LDX + (D / 4) * (l >> 4);
         f32x4 a[NS][NB];
@@ -648,7 +650,7 @@ constexpr size_t kExGradsLds = 9 * MAT * sizeof(float);
 template <int D>
 __global__ __launch_bounds__(kThr) void ex_fwd_local_kernel(
     const float *__restrict__ k, const float *__restrict__ v, const float *__restrict__ alpha, const float *__restrict__ theta,
-    const float *__restrict__ eta, float *__restrict__ loc, int s, int stride, int C, int nc, int has_s) {
+    const float *__restrict__ eta, float *__restrict__ loc, int s, int stride, int C, int nc, int maps, int has_s) {
     constexpr size_t DD = (size_t)D * D;
     extern __shared__ float smem[];
     float *Ks = smem, *Vs = Ks + MAT, *B8 = Vs + MAT, *Dg = B8 + MAT, *Nn = Dg + MAT, *Cc = Nn + MAT;
@@ -658,7 +660,7 @@ __global__ __launch_bounds__(kThr) void ex_fwd_local_kernel(
     NLH_STRIP_ORIGIN_OF(w);
     const bool dcol = D == 64 || nh == 0;
     auto MMAT = [&](f32x4 &acc, auto fa, auto fb, int k0) { mma_tile16(acc, fa, fb, k0, l); };
-    const int chain = blockIdx.x / (nc - 1), ci = blockIdx.x % (nc - 1), t0 = ci * C, L = min(C, s - t0);   // the last chunk's map is not needed
+    const int chain = blockIdx.x / maps, ci = blockIdx.x % maps, t0 = ci * C, L = min(C, s - t0);
     const size_t tok = (size_t)chain * stride + t0;
     {
         TileD<D, 64> tk, tv;
@@ -739,25 +741,26 @@ bool exact_mm_applies(int d, int C) { return (d == 64 || d == 32) && C >= 1 && C
 static int chunk_of(int C) { return C * (CW / C); }
 
 // Cost models from measurements on one MI355X (us).  A chunk costs the two chunk-parallel kernels of the backward about
-// 65 us of a compute unit (42 at head size 32) whatever its length, a scan step 1.3; the fused sequential kernel walks a
+// 65 us of a compute unit (42 at head size 32) whatever its length, a scan step 2.0 (0.5); the fused sequential kernel walks a
 // chain's tokens at 0.6 each on a quarter of a compute unit's worth of workgroups (four per chain, one at head size 32),
 // the kernel that reads a whole trajectory at 1.1.  Under a clip or a bound the test on the errors adds two launches to the
 // matrix form where the fused kernel's only adds one on its maxima.
 bool exact_backward_mm_pays(int seq_len, int batch, int d, int C, bool tested) {
     const int nc = ceil_div(seq_len, chunk_of(C)), cus = compute_units();
-    const double t_mm = (double)ceil_div(batch * nc, cus) * (d == 64 ? 65.0 : 42.0) + nc * 1.3 + (tested ? 20.0 : 10.0);
+    const double t_mm = (double)ceil_div(batch * nc, cus) * (d == 64 ? 65.0 : 42.0) + nc * (d == 64 ? 2.0 : 0.5) + (tested ? 20.0 : 10.0);
     const double t_seq = (double)seq_len * (C == 1 ? 1.1 : 0.6) * ceil_div(batch * (d == 64 ? 4 : 1), cus);
     return t_mm < t_seq;
 }
 
-// The sequential forward takes 0.15 a token as long as its workgroups (four per chain, one at head size 32) fit the
-// chip.  The chunk maps cost 24 of a compute unit per chunk (16 at head size 32), a scan step 1.3, and the walk of the
-// chunks' tokens again 0.15 a token for whatever does not run at the same time.
-bool exact_forward_mm_pays(int seq_len, int batch, int d) {
+// The sequential forward takes 0.15 a token (0.19 where it keeps a trajectory) as long as its workgroups (four per chain,
+// one at head size 32) fit the chip.  The chunk maps cost 26 of a compute unit per chunk (17 at head size 32), a scan
+// step 2.0 (0.5), and, unless only the final states are wanted, the walk of the chunks' tokens again 0.15 a token for
+// whatever does not run at the same time.
+bool exact_forward_mm_pays(int seq_len, int batch, int d, bool final_only) {
     const int nc = ceil_div(seq_len, CW), cus = compute_units(), parts = d == 64 ? 4 : 1;
-    if (nc < 3) return false;
-    const double t_mm = (double)ceil_div(batch * (nc - 1), cus) * (d == 64 ? 24.0 : 16.0) + nc * 1.3 + 8.0 +
-                        0.15 * CW * ceil_div((long long)batch * nc * parts, cus);
+    if (nc < 2) return false;
+    double t_mm = (double)ceil_div(batch * (final_only ? nc : nc - 1), cus) * (d == 64 ? 26.0 : 17.0) + nc * (d == 64 ? 2.0 : 0.5) + 8.0;
+    if (!final_only) t_mm += 0.15 * CW * ceil_div((long long)batch * nc * parts, cus);
     const double t_seq = 0.15 * seq_len * ceil_div(batch * parts, cus);
     return t_mm < t_seq;
 }
@@ -767,7 +770,8 @@ static void forward_states_t(bool has_s, const float *k, const float *v, const f
                              const float *m_initial, const float *s_initial, long long m_stride, float *m_states, float *s_states,
                              long long state_stride, int sstep, int seq_len, int input_stride, int batch) {
     const ErrorScope es;
-    const int nc = ceil_div(seq_len, CW);
+    // to the starts of all chunks, or (sstep 0) through the last one to the end
+    const int nc = ceil_div(seq_len, CW), maps = sstep ? nc - 1 : nc;
     float *loc = scratch(32, (size_t)batch * nc * kExLocMats * D * D * sizeof(float));
     static bool attr_set = false;
     if (!attr_set) {
@@ -777,30 +781,26 @@ static void forward_states_t(bool has_s, const float *k, const float *v, const f
     if (es.failed()) return;
     {
         KernelTimer kt("ex_fwd_local_kernel");
-        hipLaunchKernelGGL(ex_fwd_local_kernel<D>, dim3((unsigned)batch * (nc - 1)), dim3(kThr), kExFwdLds, stream(), k, v, alpha, theta,
-                           has_s ? eta : alpha, loc, seq_len, input_stride, CW, nc, (int)has_s);
+        hipLaunchKernelGGL(ex_fwd_local_kernel<D>, dim3((unsigned)batch * maps), dim3(kThr), kExFwdLds, stream(), k, v, alpha, theta,
+                           has_s ? eta : alpha, loc, seq_len, input_stride, CW, nc, maps, (int)has_s);
         check_launch("ex_fwd_local_kernel");
     }
     KernelTimer kt("ex_scan_kernel");
     const dim3 grid((unsigned)batch * (D / 16));
     if (has_s)
         hipLaunchKernelGGL((ex_scan_kernel<D, true, false>), grid, dim3(8 * D), 0, stream(), loc, m_initial, s_initial, m_stride,
-                           m_states, s_states, state_stride, sstep, nullptr, nullptr, nc);
+                           m_states, s_states, state_stride, sstep, nullptr, nullptr, nc, maps);
     else
         hipLaunchKernelGGL((ex_scan_kernel<D, false, false>), grid, dim3(4 * D), 0, stream(), loc, m_initial, nullptr, m_stride,
-                           m_states, nullptr, state_stride, sstep, nullptr, nullptr, nc);
+                           m_states, nullptr, state_stride, sstep, nullptr, nullptr, nc, maps);
     check_launch("ex_scan_kernel");
 }
 
 void exact_forward_states(bool has_s, int d, const float *k, const float *v, const float *alpha, const float *theta, const float *eta,
                           const float *m_initial, const float *s_initial, long long m_stride, float *m_states, float *s_states,
                           long long state_stride, int sstep, int seq_len, int input_stride, int batch) {
-    if (d == 64)
-        forward_states_t<64>(has_s, k, v, alpha, theta, eta, m_initial, s_initial, m_stride, m_states, s_states, state_stride, sstep,
-                             seq_len, input_stride, batch);
-    else
-        forward_states_t<32>(has_s, k, v, alpha, theta, eta, m_initial, s_initial, m_stride, m_states, s_states, state_stride, sstep,
-                             seq_len, input_stride, batch);
+    (d == 64 ? forward_states_t<64> : forward_states_t<32>)(has_s, k, v, alpha, theta, eta, m_initial, s_initial, m_stride, m_states,
+                                                            s_states, state_stride, sstep, seq_len, input_stride, batch);
 }
 
 template <int D>
@@ -853,10 +853,10 @@ static bool backward_mm_t(const char *fn, bool has_s, const float *k, const floa
         const long long stride = (long long)(nc + 1) * DD;
         if (has_s)
             hipLaunchKernelGGL((ex_scan_kernel<D, true, true>), grid, dim3(8 * D), 0, stream(), loc, nullptr, nullptr, 0LL, em, esn,
-                               stride, 1, first_m, first_s, nc);
+                               stride, 1, first_m, first_s, nc, nc);
         else
             hipLaunchKernelGGL((ex_scan_kernel<D, false, true>), grid, dim3(4 * D), 0, stream(), loc, nullptr, nullptr, 0LL, em, nullptr,
-                               stride, 1, first_m, nullptr, nc);
+                               stride, 1, first_m, nullptr, nc, nc);
         check_launch("ex_scan_kernel");
     }
     {

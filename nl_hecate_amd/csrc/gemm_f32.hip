@@ -69,17 +69,11 @@ struct Operand {
             }
         }
     }
-    // this lane's eight contraction indices (8 (l / 16) + 0..7) of row r
-    static __device__ __forceinline__ void read(float (&v)[8], const float *s, int r, int l) {
-        const int kb = 8 * (l >> 4);
-        if constexpr (KC) {
-            const f32x4 p = *reinterpret_cast<const f32x4 *>(s + r * LD + kb), q = *reinterpret_cast<const f32x4 *>(s + r * LD + kb + 4);
-#pragma unroll
-            for (int i = 0; i < 4; i++) { v[i] = p[i]; v[4 + i] = q[i]; }
-        } else {
-#pragma unroll
-            for (int i = 0; i < 8; i++) v[i] = s[(kb + i) * LD + r];
-        }
+    // half h (four) of this lane's contraction indices, 8 (l / 16) + 4 h + 0..3, of row r
+    static __device__ __forceinline__ f32x4 read(const float *s, int r, int h, int l) {
+        const int kb = 8 * (l >> 4) + 4 * h;
+        if constexpr (KC) return *reinterpret_cast<const f32x4 *>(s + r * LD + kb);
+        else return f32x4{s[kb * LD + r], s[(kb + 1) * LD + r], s[(kb + 2) * LD + r], s[(kb + 3) * LD + r]};
     }
 };
 
@@ -115,18 +109,23 @@ __global__ __launch_bounds__(64 * WM * WN) void group_gemm_kernel(GroupArgs g) {
         rb.store(sb[buf]);
         __syncthreads();   // the buffer is complete; the other one's readers are past their products
         if (s + 1 < s1) load(s + 1);
-        float av[TM][8], bv[TN][8];
+        f32x4 av[2][TM], bv[2][TN];
 #pragma unroll
-        for (int i = 0; i < TM; i++) OA::read(av[i], sa[buf], wm + 16 * i + (l & 15), l);
+        for (int h = 0; h < 2; h++) {   // the second half is read while the first one's products run
 #pragma unroll
-        for (int j = 0; j < TN; j++) OB::read(bv[j], sb[buf], wn + 16 * j + (l & 15), l);
+            for (int i = 0; i < TM; i++) av[h][i] = OA::read(sa[buf], wm + 16 * i + (l & 15), h, l);
 #pragma unroll
-        for (int kk = 0; kk < 8; kk++)
+            for (int j = 0; j < TN; j++) bv[h][j] = OB::read(sb[buf], wn + 16 * j + (l & 15), h, l);
+        }
 #pragma unroll
-            for (int i = 0; i < TM; i++)
+        for (int h = 0; h < 2; h++)
 #pragma unroll
-                for (int j = 0; j < TN; j++)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[i][kk], bv[j][kk], acc[i][j], 0, 0, 0);
+            for (int e = 0; e < 4; e++)
+#pragma unroll
+                for (int i = 0; i < TM; i++)
+#pragma unroll
+                    for (int j = 0; j < TN; j++)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[h][i][e], bv[h][j][e], acc[i][j], 0, 0, 0);
     }
     const bool part = g.splits > 1, b16 = OP == 0 && ((g.bf16_mask >> blockIdx.y) & 1);
     float *c = part ? g.part + (size_t)blockIdx.z * g.m * g.n : reinterpret_cast<float *>(g.c[OP == 1 ? 0 : blockIdx.y]);
@@ -187,9 +186,9 @@ extern "C" void linear_group_f32_rocm(int op, int count, const float *const *a, 
     }
     g.bf16_mask = op == 0 ? bf16_mask : 0;
     g.count = count; g.m = m; g.n = n; g.k = k; g.splits = 1;
-    // Tile and split: one workgroup of the large tile keeps the matrix cores of a compute unit at about 0.85 of their
-    // rate and moves half the bytes per flop, the small one at about 0.6; what decides is how many rounds of the chip
-    // either needs.  A sum over products (op 1) and a single product with a long contraction have few output tiles: their
+    // Tile and split: the large tile keeps the matrix cores of a compute unit at about 0.9 of their rate, three or four
+    // workgroups of the small one at about 0.82 (4096^3: 128 and 114 of 140 TFLOP/s); what decides is how much work the
+    // fullest compute unit gets.  A sum over products (op 1) and a single product with a long contraction have few output tiles: their
     // contraction is split until one (large tile) or two workgroups per compute unit are there.
     const int cus = compute_units(), ny = op == 1 ? 1 : count;
     const int big_tiles = ceil_div(m, 128) * ceil_div(n, 128), small_tiles = ceil_div(m, 64) * ceil_div(n, 64);
@@ -200,8 +199,8 @@ extern "C" void linear_group_f32_rocm(int op, int count, const float *const *a, 
         return s < 1 ? 1 : (s > 16 ? 16 : s);
     };
     const int sb = splits_of(big_tiles, 1), ss = splits_of(small_tiles, 2);
-    const double t_big = (double)ceil_div((long long)big_tiles * ny * sb, cus) * ceil_div(total, sb) * 4096 / 0.85;
-    const double t_small = (double)ceil_div((long long)small_tiles * ny * ss, cus) * ceil_div(total, ss) * 1024 / 0.60;
+    const double t_big = (double)ceil_div((long long)big_tiles * ny * sb, cus) * ceil_div(total, sb) * 4096 / 0.90;
+    const double t_small = (double)ceil_div((long long)small_tiles * ny * ss, cus) * ceil_div(total, ss) * 1024 / 0.82;
     const bool big = t_big < t_small;
     g.splits = big ? sb : ss;
     g.tiles_n = ceil_div(n, big ? 128 : 64);

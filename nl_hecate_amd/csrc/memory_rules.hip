@@ -685,7 +685,7 @@ static bool launch_fwd(FwdArgs a, int d, int batch) {
     if constexpr (!FROZEN && STORE != STORE_NONE) {
         const bool kept = STORE == STORE_TRAJ || kExactChunk % a.ckpt_interval == 0;   // the slots of all chunk starts exist
         if (!coupled && kept && exact_mm_applies(d, 1) && g_exact_form != 2 &&
-            (g_exact_form == 1 ? a.seq_len > kExactChunk : exact_forward_mm_pays(a.seq_len, batch, d))) {
+            (g_exact_form == 1 ? a.seq_len > kExactChunk : exact_forward_mm_pays(a.seq_len, batch, d, false))) {
             const ErrorScope es;
             const int sstep = STORE == STORE_TRAJ ? kExactChunk : kExactChunk / a.ckpt_interval;
             exact_forward_states(HAS_S, d, a.k, a.v, a.alpha, a.theta, a.eta, a.m_initial, a.s_initial, a.m_stride, a.m_out, a.s_out,
@@ -940,8 +940,51 @@ static void backward_ckpt_any(bool has_s, bool frozen, bool allow_fused,
 
 using namespace nlh;
 
+// The state after the last token only: no outputs, no trajectory (a prompt that fills the memories).
+template <bool HAS_S>
+static void final_states(const char *fn, const float *k, const float *v, const float *alpha, const float *theta, const float *eta,
+                         const float *m_initial, const float *s_initial, float *m_final, int seq_len, int d, int batch) {
+    const ErrorScope es;
+    if (!check_dims(fn, seq_len, d, batch) || batch == 0) return;
+    if (seq_len == 0) { fail("%s: seq_len=0.", fn); return; }
+    const size_t dd = (size_t)d * d;
+    // three launches of the matrix form against one walk at 0.15 us a token (see exact_forward_mm_pays)
+    if (exact_mm_applies(d, 1) && g_exact_form != 2 && (g_exact_form == 1 || exact_forward_mm_pays(seq_len, batch, d, true))) {
+        float *sf = HAS_S ? scratch(9, (size_t)batch * dd * sizeof(float)) : nullptr;
+        if (es.failed()) return;
+        exact_forward_states(HAS_S, d, k, v, alpha, theta, eta, m_initial, s_initial, (long long)dd, m_final, sf, (long long)dd, 0, seq_len,
+                             seq_len, batch);
+        return;
+    }
+    float *m2 = scratch(5, 2 * batch * dd * sizeof(float)), *s2 = HAS_S ? scratch(6, 3 * batch * dd * sizeof(float)) : nullptr;
+    float *y = scratch(7, (size_t)batch * seq_len * d * sizeof(float));
+    if (es.failed()) return;
+    if (HAS_S && !s_initial) {
+        float *z = s2 + 2 * batch * dd;
+        hipLaunchKernelGGL(zero_fill_kernel, dim3(ceil_div(batch * dd, 256)), dim3(256), 0, stream(), z, (size_t)batch * dd);
+        check_launch("zero_fill_kernel");
+        s_initial = z;
+    }
+    FwdArgs a{k, v, k, alpha, theta, eta, m_initial, s_initial, m2, s2, y, seq_len, seq_len, seq_len, 1, (long long)dd,
+              (long long)(2 * dd), 0.f, 0.f};
+    if (!launch_fwd<HAS_S, STORE_CKPT>(a, d, batch)) { unsupported(fn, d, false); return; }
+    check_hip(hipMemcpy2DAsync(m_final, dd * sizeof(float), m2 + dd, 2 * dd * sizeof(float), dd * sizeof(float), batch,
+                               hipMemcpyDeviceToDevice, stream()), fn);
+}
+
 // ───────────────────────────── C ABI ───────────────────────────────────────
 extern "C" {
+
+void titans_final_states_f32_rocm(const float *k_mem, const float *v_mem, const float *alpha, const float *theta, const float *eta,
+                                  const float *m_initial, const float *s_initial, float *m_final, int seq_len, int d, int batch_size) {
+    final_states<true>("titans_final_states_f32_rocm", k_mem, v_mem, alpha, theta, eta, m_initial, s_initial, m_final, seq_len, d,
+                       batch_size);
+}
+void delta_final_states_f32_rocm(const float *k_mem, const float *v_mem, const float *alpha, const float *theta,
+                                 const float *m_initial, float *m_final, int seq_len, int d, int batch_size) {
+    final_states<false>("delta_final_states_f32_rocm", k_mem, v_mem, alpha, theta, nullptr, m_initial, nullptr, m_final, seq_len, d,
+                        batch_size);
+}
 
 int nlh_exact_backward_form(int mode) {
     const int prev = g_exact_form;

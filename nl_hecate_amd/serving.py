@@ -15,13 +15,14 @@ import operator
 from dataclasses import dataclass, field
 from typing import List
 
+import numpy as np
 import torch
 
 from . import dispatch as D
 from .cms import ContextState, Pulse
 from .ffi import lib
 from .mag_layer import MemoryLevelParams
-from .memory_level import LevelConfig, gpu_memory_forward
+from .memory_level import F32_MAX, LevelConfig, _plain, _ptrs, gpu_memory_forward, group_key, linear_group
 
 
 def _new(*shape, dtype=torch.float32):
@@ -67,11 +68,9 @@ class GpuKVCache:
     """bf16 K and V of every position so far, [max_len, d] each, with a conversion scratch sized once."""
 
     def __init__(self, max_len, d, scratch_tokens):
-        self.k_cache_bf16 = _zeros(max_len, d, dtype=torch.bfloat16)
-        self.v_cache_bf16 = _zeros(max_len, d, dtype=torch.bfloat16)
+        self.k_cache_bf16, self.v_cache_bf16 = _zeros(2, max_len, d, dtype=torch.bfloat16).unbind(0)
         self.len, self.max_len, self.d = 0, max_len, d
-        self._scratch_k = _zeros(scratch_tokens * d, dtype=torch.bfloat16)
-        self._scratch_v = _zeros(scratch_tokens * d, dtype=torch.bfloat16)
+        self._scratch_k, self._scratch_v = _new(2, scratch_tokens * d, dtype=torch.bfloat16).unbind(0)
 
     def append_f32(self, k_f32, v_f32, n_tokens):
         """:3017-3053: convert into the scratch, copy behind the filled positions."""
@@ -263,12 +262,98 @@ def _combine_gate(ys, attn_out, y_combined, gate, gated, n):
                               gated.data_ptr(), n)
 
 
+def _prefill_in_batch(params, cfg, input_ids, pulse, context):
+    """A prompt leaves three things behind: K and V of every token, the levels' memories after the last token, and the
+    logits of the last position.  So only k, v and the gates are formed for every token (one group of products, one pass
+    of glue over all active levels), the memories go straight to their final states, and the last position is one decode
+    step that reads them: attention, combine, gate, output projection and unembedding of one token.  Exact Delta, Titans
+    and DGD levels without clip or bound and frozen matrix levels; None: anything else takes the step below."""
+    s, d, nh, hd, v, k = cfg.seq_len, cfg.d_model, cfg.num_heads, cfg.head_dim, cfg.vocab_size, cfg.k
+    if hd not in (32, 64, 128) or nh * hd != d or d > 1024 or not 1 <= k <= 8 or s < 1 or params.w_embed.shape != (v, d):
+        return None
+    active = [lv for lv in range(k) if pulse.active_levels[lv]]
+    keys = {group_key(cfg.levels[lv], params.levels[lv], d, 1) for lv in active}
+    if len(keys) > 1 or None in keys:
+        return None
+    for lv in range(k):
+        lc, lp, mem = cfg.levels[lv], params.levels[lv], context.memory[lv]
+        if (_DECODE_RULE.get(lc.memory_rule) is None or lc.memory_layers != 1 or (lc.num_heads, lc.head_dim) != (nh, hd)
+                or not _plain(mem) or mem.shape != (nh, hd * hd)):
+            return None
+        if pulse.active_levels[lv] and (lc.error_clip > 0 or 0 < lc.m_norm_max < 1e30 or lc.proxy):
+            return None
+        if any(not _plain(t) for t in (lp.w_k, lp.w_v, lp.w_q)):
+            return None
+    if any(not _plain(w) for w in (params.w_embed, params.w_q, params.w_k, params.w_v, params.w_o, params.w_unembed)):
+        return None
+    host_ids = torch.empty(s, dtype=torch.int32, pin_memory=True)
+    ids = host_ids.numpy()
+    ids[:] = np.asarray(input_ids[:s].cpu() if isinstance(input_ids, torch.Tensor) else input_ids[:s])
+    last = int(ids[s - 1])
+    if ids.min() < 0 or ids.max() >= v:
+        return None
+    embedded = _new(s, d)
+    lib.embedding_gather_cuda(params.w_embed.data_ptr(), host_ids.cuda(non_blocking=True).data_ptr(), embedded.data_ptr(), s, d)
+    kv_cache = GpuKVCache(s + cfg.decode_tokens, d, s)
+    L = len(active)
+    mem = list(_new(max(2 * L, 1), s, d).unbind(0))[:2 * L]
+    weights = [w for lv in active for w in (params.levels[lv].w_k, params.levels[lv].w_v)] + [params.w_k, params.w_v]
+    linear_group(0, [embedded] * (2 * L + 2), weights, mem + [kv_cache.k_cache_bf16, kv_cache.v_cache_bf16], s, d, d, 3 << (2 * L))
+    kv_cache.len = s
+    if L:
+        cfgs, lps = [cfg.levels[lv] for lv in active], [params.levels[lv] for lv in active]
+        titans = cfgs[0].memory_rule == "titans"
+        heads, gates = _new(2, L * nh, s, hd), _new(3 if titans else 2, L * nh, s)
+        rows = list(_new(4 * L, s).unbind(0))
+        h0, g0 = heads.data_ptr(), gates.data_ptr()
+        hs, gs = 4 * L * nh * s * hd, 4 * L * nh * s
+        lib.level_group_inputs_f32_rocm(
+            _ptrs([t for i, lp in enumerate(lps) for t in (
+                mem[2 * i], mem[2 * i + 1], mem[2 * i], lp.w_alpha, lp.b_alpha, lp.w_theta, lp.b_theta, lp.w_eta, lp.b_eta,
+                rows[4 * i], rows[4 * i], rows[4 * i + 1], rows[4 * i + 2], rows[4 * i + 3])]),
+            (ctypes.c_float * (4 * L))(*[x for c in cfgs for x in (c.alpha_floor, c.alpha_ceil, c.theta_floor, c.theta_ceil)]), L,
+            h0, h0 + hs, None, g0, g0 + gs, g0 + 2 * gs if titans else None, 1, s, nh, hd, 1e-8)
+        contexts = [context.memory[lv] for lv in active]
+        states = contexts[0]
+        if L > 1:
+            states = _new(L * nh, hd * hd)
+            lib.level_group_states_gather_rocm(_ptrs(contexts), L, states.data_ptr(), nh, hd * hd)
+        if titans:
+            lib.titans_final_states_f32_rocm(h0, h0 + hs, g0, g0 + gs, g0 + 2 * gs, states.data_ptr(), None, states.data_ptr(), s, hd,
+                                             L * nh)
+        else:
+            lib.delta_final_states_f32_rocm(h0, h0 + hs, g0, g0 + gs, states.data_ptr(), states.data_ptr(), s, hd, L * nh)
+        if L > 1:
+            lib.level_group_states_final_rocm(states.data_ptr(), hd * hd, _ptrs(contexts), (ctypes.c_float * L)(*[F32_MAX] * L), L,
+                                              nh, hd * hd)
+    # the last position as a decode step at a cache row that holds its K and V already
+    level_ptrs = [t.data_ptr() for lv in range(k) for lp in (params.levels[lv],) for t in (
+        lp.w_k, lp.w_v, lp.w_q, lp.w_alpha, lp.b_alpha, lp.w_theta, lp.b_theta, context.memory[lv])]
+    work = _new(lib.decode_work_floats_rocm(d, nh, k, cfg.window_size, cfg.n_persistent) + 7 * d + v)
+    w0 = work.data_ptr()
+    row, step = w0 + 4 * (work.numel() - 7 * d - v) // 16 * 16, 4 * d
+    outputs = (ctypes.c_void_p * 7)(*[row + i * step for i in range(7)])
+    logits = torch.empty(v, dtype=torch.float32, pin_memory=True)
+    rc = lib.decode_token_rocm(
+        params.w_embed.data_ptr() + 4 * d * last, params.w_q.data_ptr(), params.w_k.data_ptr(), params.w_v.data_ptr(),
+        params.w_o.data_ptr(), params.w_unembed.data_ptr(), (ctypes.c_void_p * (8 * k))(*level_ptrs),
+        (ctypes.c_int * k)(*[3 if pulse.active_levels[lv] else -1 for lv in range(k)]), (ctypes.c_float * (6 * k))(), k, d, nh, v,
+        cfg.window_size, cfg.n_persistent, s - 1, kv_cache.k_cache_bf16.data_ptr(), kv_cache.v_cache_bf16.data_ptr(), w0, outputs,
+        row + 7 * step, logits.data_ptr())
+    if rc:
+        raise RuntimeError(f"decode_token_rocm failed ({rc})")
+    return logits.numpy().copy(), kv_cache
+
+
 def gpu_prefill_forward(params: GpuMAGParams, cfg: ServeConfig, input_ids, pulse: Pulse, context: ContextState):
     """-> (logits of the last prompt position [vocab] on the host, GpuKVCache holding the prompt)."""
     s, d, nh, hd = cfg.seq_len, cfg.d_model, cfg.num_heads, cfg.head_dim
     assert d == nh * hd
     assert not cfg.residual, "gpu_prefill_forward: residual=true is not served by the cached-generation path"
     assert len(input_ids) >= s
+    done = _prefill_in_batch(params, cfg, input_ids, pulse, context)
+    if done is not None:
+        return done
     ids = torch.tensor([int(t) for t in input_ids[:s]], dtype=torch.int32).cuda()
     embedded = _new(s, d)
     D.call("embedding_gather_cuda", params.w_embed, ids, embedded, s, d)

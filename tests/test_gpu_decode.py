@@ -56,3 +56,37 @@ def test_one_call_step(rule, active, n_p, nh, hd, window, s, extra, v, opts):
     assert f"decode_logits_kernel:{extra}:".encode() in buf.value, buf.value
     for lv in range(k):
         assert_close(f"memory[{lv}]", host(ctx.memory[lv]).reshape(mem[lv].shape), mem[lv], 1e-4)
+
+
+@pytest.mark.parametrize("rule,active,n_p,nh,hd,window,s,v,opts", [
+    ("titans", [True, True, True], 0, 2, 64, 100, 200, 64, {}),          # final states by the chunk maps' scan
+    ("titans", [True, False], 2, 3, 32, 64, 65, 33, dict(alpha_floor=0.2)),
+    ("delta", [True, True], 0, 2, 32, 16, 193, 40, dict(theta_ceil=0.05)),
+    ("dgd", [True], 0, 1, 128, 8, 7, 12, {}),
+    ("titans", [False, False], 0, 2, 64, 8, 3, 8, {})])
+def test_prefill_in_one_batch(rule, active, n_p, nh, hd, window, s, v, opts):
+    """Prompts through the batched path (no per-token outputs, memories straight to their final states)."""
+    print(rule, active, nh, hd, s, flush=True)
+    d, k = nh * hd, len(active)
+    p = model(d, v, k, 17 + s)
+    lcfgs = [LevelConfig(rule, nh, hd, **opts) for _ in range(k)]
+    ocfg = types.SimpleNamespace(d_model=d, num_heads=nh, head_dim=hd, window_size=window, n_persistent=n_p, levels=lcfgs)
+    cfg = SG.ServeConfig(d, v, nh, hd, window, s, lcfgs, n_persistent=n_p, decode_tokens=1)
+    r = np.random.default_rng(11)
+    ids = r.integers(0, v, s + 1)
+    mem0 = [(0.2 * r.standard_normal((nh, hd, hd))).astype(f32) for _ in range(k)]
+    gp, pulse = gpu_params(p), Pulse(0, list(active))
+    ctx = ContextState([dev(m.reshape(nh, hd * hd)) for m in mem0])
+    prev = lib.nlh_exact_backward_form(1)   # the matrix form wherever it applies
+    assert SG._prefill_in_batch(gp, cfg, ids, pulse, ContextState([m.clone() for m in ctx.memory])) is not None
+    logits, kv = SG.gpu_prefill_forward(gp, cfg, ids, pulse, ctx)
+    lib.nlh_exact_backward_form(prev)
+    want, mem, kc, vc = SV.forward_all(p, ocfg, ids[:s], active, mem0)
+    assert np.abs(logits - want[s - 1]).max() <= 2e-2 * np.abs(want).max()
+    assert kv.len == s and kv.max_len == s + 1
+    for got, ref in ((kv.k_cache_bf16, kc), (kv.v_cache_bf16, vc)):
+        a, b = host(got.float())[:s], SV.orc.bf16_to_f32(ref)
+        assert np.abs(a - b).max() <= 2 ** -7 * np.abs(b).max()
+        assert not host(got.float())[s:].any()
+    for lv in range(k):
+        assert_close(f"memory[{lv}]", host(ctx.memory[lv]).reshape(mem[lv].shape), mem[lv], 1e-4)
