@@ -29,6 +29,10 @@
 // The algebra is written out and checked against the reference's token loops in float64 in tests/np_rules.py
 // (titans_exact_chunk_backward).
 //
+// FROZEN: the frozen-M0 chunkwise rule (core/kernels/titans_chunkwise_backward.cu) in the same kernels: its errors are
+// taken against the chunk-start memory, i.e. T = I, am = 1, bm = 0, and the terms through Lam are absent.  Serves head
+// size 32, which the chunkwise matrix kernels of chunkwise_mm.hip do not have.
+//
 // Under a finite m_norm_max / error clip the pass also leaves the ChainTracks of chunkwise_chain.h behind (|u_t|^2 per
 // token, sums of squares of the checkpoints); the caller tests on them whether a coupling could have fired.
 #include <hip/hip_runtime.h>
@@ -114,18 +118,19 @@ __device__ __forceinline__ void store_acc_tile(float *mat, const f32x4 &t, int i
 }
 
 struct ChunkVecs { float wM[CW], wS[CW], am[CW], bm[CW]; };
+template <bool FROZEN>
 __device__ __forceinline__ void chunk_vectors(ChunkVecs &cv, const Coef &cf, int L) {
     const int j = threadIdx.x;
     if (j < CW) {
         cv.wM[j] = -cf.th[j] * cf.cl[j];
         cv.wS[j] = -cf.th[j] * cf.bl[j];
-        cv.am[j] = j == 0 ? 1.f : (j < L ? cf.a[j - 1] : 0.f);
-        cv.bm[j] = (j == 0 || j >= L) ? 0.f : cf.beta[j - 1];
+        cv.am[j] = FROZEN ? 1.f : j == 0 ? 1.f : (j < L ? cf.a[j - 1] : 0.f);
+        cv.bm[j] = (FROZEN || j == 0 || j >= L) ? 0.f : cf.beta[j - 1];
     }
 }
 
 // ── pass 1: chunk-local matrices ────────────────────────────────────────────
-template <int D, bool TRACK>
+template <int D, bool FROZEN, bool TRACK>
 __global__ __launch_bounds__(kThr) void ex_local_kernel(
     const float *__restrict__ k, const float *__restrict__ v, const float *__restrict__ q, const float *__restrict__ d_y,
     const float *__restrict__ alpha, const float *__restrict__ theta, const float *__restrict__ eta,
@@ -190,13 +195,13 @@ __global__ __launch_bounds__(kThr) void ex_local_kernel(
         }
     }
     __syncthreads();
-    chunk_vectors(cv, cf, L);
+    chunk_vectors<FROZEN>(cv, cf, L);
     {
         Strip g = zero_strip(), km = zero_strip(), ks = zero_strip(), p = zero_strip();
         auto aK = [&](int m, int kk) { return Ks[(m0 + m) * LDM + kk]; };
-        MMD(g, aK, [&](int kk, int n) { return Ks[(n0 + n) * LDM + kk]; });
+        if (!FROZEN) MMD(g, aK, [&](int kk, int n) { return Ks[(n0 + n) * LDM + kk]; });
         if (dcol) MMD(km, aK, [&](int kk, int n) { return Ms[(n0 + n) * LDM + kk]; });
-        if (dcol && has_s) MMD(ks, aK, [&](int kk, int n) { return Ss[(n0 + n) * LDM + kk]; });
+        if (!FROZEN && dcol && has_s) MMD(ks, aK, [&](int kk, int n) { return Ss[(n0 + n) * LDM + kk]; });
         MMD(p, [&](int m, int kk) { return Qs[(m0 + m) * LDM + kk]; }, [&](int kk, int n) { return Ks[(n0 + n) * LDM + kk]; });
         __syncthreads();   // the vectors are there
 #pragma unroll
@@ -206,10 +211,10 @@ __global__ __launch_bounds__(kThr) void ex_local_kernel(
                 const int row = m0 + row_of(i, l), col = n0 + 16 * tl + (l & 15);
                 if (dcol) {   // R in place over V (own strip)
                     float *d = Vs + row * LDM + col;
-                    *d = cv.am[row] * km.t[tl][i] + cv.bm[row] * ks.t[tl][i] - *d;
+                    *d = FROZEN ? km.t[tl][i] - *d : cv.am[row] * km.t[tl][i] + cv.bm[row] * ks.t[tl][i] - *d;
                 }
                 const float nth = -cf.th[col];
-                B8[row * LDM + col] = (col < row) ? nth * Cc[(row - 1) * LDM + col] * g.t[tl][i] : 0.f;   // Lam
+                if (!FROZEN) B8[row * LDM + col] = (col < row) ? nth * Cc[(row - 1) * LDM + col] * g.t[tl][i] : 0.f;   // Lam
                 B9[row * LDM + col] = nth * Cc[row * LDM + col] * p.t[tl][i];                            // W.P
             }
     }
@@ -217,6 +222,25 @@ __global__ __launch_bounds__(kThr) void ex_local_kernel(
     Strip dul = zero_strip();
     if (dcol) MMA(dul, [&](int m, int kk) { return B9[kk * LDM + m0 + m]; }, [&](int kk, int n) { return Ds[kk * LDM + n0 + n]; });
     float *goT = Tg + task * kDD, *goU = dUg + task * kDD;
+    auto track = [&](Strip &u) {   // squared error norm of the strip's 16 tokens over its 32 memory rows
+        FORC(u, [&](int, int, float &x) { x *= x; });
+        strip_row_sums(u);
+        if (row_writer(l)) {
+            float *eo = tr.e2 + (((size_t)chain * 2 + nh) * nc + ci) * CW + m0;
+#pragma unroll
+            for (int i = 0; i < 4; i++) eo[row_of(i, l)] = u.t[0][i];
+        }
+    };
+    if constexpr (FROZEN) {   // U = R, Z1 = K
+        __syncthreads();      // W.P is read
+        if (dcol) {
+            Strip u;
+            float *go = Ug + task * kDD;
+            FORC(dul, [&](int r, int c, float &x) { B9[(m0 + r) * LDM + n0 + c] = x; goU[(m0 + r) * HD + n0 + c] = x; });
+            FORC(u, [&](int r, int c, float &x) { x = Vs[(m0 + r) * LDM + n0 + c]; go[(m0 + r) * HD + n0 + c] = x; });
+            if (TRACK) track(u);
+        }
+    } else {
 #define INV_L B8
 #define INV_D Ms
 #define INV_N Ss
@@ -238,16 +262,10 @@ __global__ __launch_bounds__(kThr) void ex_local_kernel(
         FORC(u, [&](int r, int c, float &x) { go[(m0 + r) * HD + n0 + c] = x; });
         FORC(z1, [&](int r, int c, float &x) { B8[(m0 + r) * LDM + n0 + c] = x; });
         if (has_s) FORC(z2, [&](int r, int c, float &x) { Ms[(m0 + r) * LDM + n0 + c] = x; });
-        if (TRACK) {   // squared error norm of the strip's 16 tokens over its 32 memory rows
-            FORC(u, [&](int, int, float &x) { x *= x; });
-            strip_row_sums(u);
-            if (row_writer(l)) {
-                float *eo = tr.e2 + (((size_t)chain * 2 + nh) * nc + ci) * CW + m0;
-#pragma unroll
-                for (int i = 0; i < 4; i++) eo[row_of(i, l)] = u.t[0][i];
-            }
-        }
-    } else if (TRACK && row_writer(l)) {   // head size 32 has no second half
+        if (TRACK) track(u);
+    }
+    }
+    if (TRACK && !dcol && row_writer(l)) {   // head size 32 has no second half
         float *eo = tr.e2 + (((size_t)chain * 2 + nh) * nc + ci) * CW + m0;
 #pragma unroll
         for (int i = 0; i < 4; i++) eo[row_of(i, l)] = 0.f;
@@ -263,9 +281,10 @@ __global__ __launch_bounds__(kThr) void ex_local_kernel(
     const bool on_diag = sm0 == sn0 || sm0 == sn0 + 16;
 #pragma unroll 1
     for (int o = o0; o < (has_s ? 4 : 1); o += ostep) {   // Phi_MM, Phi_SM, Phi_MS, Phi_SS = (w.K)^T Z
-        const float *wv = (o & 1) ? cv.wS : cv.wM, *Z = (o & 2) ? Ms : B8;
+        const float *wv = (o & 1) ? cv.wS : cv.wM, *Z = FROZEN ? Ks : (o & 2) ? Ms : B8;
         Strip x = zero_strip();
-        MMA(x, [&](int m, int kk) { return wv[kk] * Ks[kk * LDM + sm0 + m]; }, [&](int kk, int n) { return Z[kk * LDM + sn0 + n]; });
+        if (!(FROZEN && (o & 2)))
+            MMA(x, [&](int m, int kk) { return wv[kk] * Ks[kk * LDM + sm0 + m]; }, [&](int kk, int n) { return Z[kk * LDM + sn0 + n]; });
         if (on_diag) {   // the chunk's own decay
             const float dg = o == 0 ? aL : o == 2 ? bL : o == 3 ? hL : 0.f;
             FORC(x, [&](int r, int c, float &y) { if (sm0 + r == sn0 + c) y += dg; });
@@ -275,10 +294,11 @@ __global__ __launch_bounds__(kThr) void ex_local_kernel(
     }
 #pragma unroll 1
     for (int o = o0; o < (has_s ? 2 : 1); o += ostep) {   // C_M = (a.dY)^T Q + dU_loc^T Z1,  C_S = (beta.dY)^T Q + dU_loc^T Z2
-        const float *vec = o ? cf.beta : cf.a, *Z = o ? Ms : B8;
+        const float *vec = o ? cf.beta : cf.a, *Z = FROZEN ? Ks : o ? Ms : B8;
         Strip x = zero_strip();
         MMA(x, [&](int m, int kk) { return vec[kk] * Ds[kk * LDM + sm0 + m]; }, [&](int kk, int n) { return Qs[kk * LDM + sn0 + n]; });
-        MMA(x, [&](int m, int kk) { return B9[kk * LDM + sm0 + m]; }, [&](int kk, int n) { return Z[kk * LDM + sn0 + n]; });
+        if (!(FROZEN && o))
+            MMA(x, [&](int m, int kk) { return B9[kk * LDM + sm0 + m]; }, [&](int kk, int n) { return Z[kk * LDM + sn0 + n]; });
 #pragma unroll
         for (int tl = 0; tl < 2; tl++) store_acc_tile<D>(out + (size_t)(4 + o) * DD, x.t[tl], sib, sn0 / 16 + tl, l);
     }
@@ -388,7 +408,7 @@ __global__ __launch_bounds__((HAS_S ? 2 : 1) * D * 4) void ex_scan_kernel(
 // ── pass 3: gradients of one chunk ──────────────────────────────────────────
 //   pvec [chain][token][4] = <M0, J_t>, <S0, J_t>, -theta_t u_t^T dMo k_t, -theta_t u_t^T dSo k_t
 //   xs [chain][chunk][s][t] as above     scal [chunk][4] = <M0, dMo>, <S0, dMo>, <S0, dSo>
-template <int D>
+template <int D, bool FROZEN>
 __global__ __launch_bounds__(kThr) void ex_grads_kernel(
     const float *__restrict__ k, const float *__restrict__ q, const float *__restrict__ d_y, const float *__restrict__ alpha,
     const float *__restrict__ theta, const float *__restrict__ eta, const float *__restrict__ m_ckpt,
@@ -424,7 +444,7 @@ __global__ __launch_bounds__(kThr) void ex_grads_kernel(
     auto fetch_b = [&](int task, int tid) {
         const int chain = task / nc, ci = task % nc;
         const size_t end = ((size_t)chain * (nc + 1) + ci + 1) * DD, st = ((size_t)chain * nck + (size_t)ci * cstep) * DD;
-        fetch(tt, Tg + (size_t)task * kDD, 64, tid);
+        if (!FROZEN) fetch(tt, Tg + (size_t)task * kDD, 64, tid);
         fetch(tu, Ug + (size_t)task * kDD, 64, tid);   // at head size 32 the right half is stale memory, never used
         fetch(tdm, em + end, D, tid);
         if (has_s) fetch(tds, es_ + end, D, tid);
@@ -454,13 +474,13 @@ __global__ __launch_bounds__(kThr) void ex_grads_kernel(
     commit(Qs, tq, tid);
     commit(Ds, td, tid);
     __syncthreads();
-    chunk_vectors(cv, cf, L);
+    chunk_vectors<FROZEN>(cv, cf, L);
     auto aK = [&](int m, int kk) { return Ks[(m0 + m) * LDM + kk]; };
     Strip p = zero_strip(), g = zero_strip();   // Q K^T and K K^T while the other tiles are in flight
     MMD(p, [&](int m, int kk) { return Qs[(m0 + m) * LDM + kk]; }, [&](int kk, int n) { return Ks[(n0 + n) * LDM + kk]; });
-    MMD(g, aK, [&](int kk, int n) { return Ks[(n0 + n) * LDM + kk]; });
+    if (!FROZEN) MMD(g, aK, [&](int kk, int n) { return Ks[(n0 + n) * LDM + kk]; });
     {
-        commit(Ts, tt, tid);
+        if (!FROZEN) commit(Ts, tt, tid);
         commit(Us, tu, tid);
         commit(A1, tdm, tid);
         if (has_s) commit(A2, tds, tid);
@@ -497,11 +517,16 @@ __global__ __launch_bounds__(kThr) void ex_grads_kernel(
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 const int row = m0 + row_of(i, l), col = n0 + 16 * tl + (l & 15);
-                B9[row * LDM + col] = gi[row * HD + col] + cv.wM[row] * kdm.t[tl][i] + cv.wS[row] * kds.t[tl][i];   // dU
+                const float du = gi[row * HD + col] + cv.wM[row] * kdm.t[tl][i] + cv.wS[row] * kds.t[tl][i];
+                B9[row * LDM + col] = du;   // dU
+                if constexpr (FROZEN) {     // dR = dU
+                    Ts[row * LDM + col] = du;
+                    if (row < L) d_v[(tok + row) * D + col] = -du;
+                }
             }
     }
     __syncthreads();   // dU complete; dMo, dSo no longer needed
-    {
+    if constexpr (!FROZEN) {
         Strip dr = zero_strip();
         // T^T is upper triangular: row block ib contracts over the blocks ib .. 3 of 16 (taken in pairs)
         if (dcol) {
@@ -513,14 +538,14 @@ __global__ __launch_bounds__(kThr) void ex_grads_kernel(
         }
         __syncthreads();   // T no longer needed
         if (dcol) FORC(dr, [&](int r, int c, float &x) { Ts[(m0 + r) * LDM + n0 + c] = x; });   // dR
+        __syncthreads();
     }
-    __syncthreads();
     const float *dRs = Ts;
     Strip dwa;
     {
         Strip dlam = zero_strip(), dyu = zero_strip();
         auto bU = [&](int kk, int n) { return Us[(n0 + n) * LDM + kk]; };
-        MMD(dlam, [&](int m, int kk) { return dRs[(m0 + m) * LDM + kk]; }, bU);
+        if (!FROZEN) MMD(dlam, [&](int m, int kk) { return dRs[(m0 + m) * LDM + kk]; }, bU);
         MMD(dyu, [&](int m, int kk) { return Ds[(m0 + m) * LDM + kk]; }, bU);
 #pragma unroll
         for (int tl = 0; tl < 2; tl++)
@@ -532,10 +557,12 @@ __global__ __launch_bounds__(kThr) void ex_grads_kernel(
                 const float lam = (col < row && row < L) ? dlam.t[tl][i] : 0.f;
                 const float yu = (col <= row && row < L) ? dyu.t[tl][i] : 0.f;
                 B9[row * LDM + col] = nth * c0 * yu;            // dP = W . tril(dY U^T)
-                A2[row * LDM + col] = lam * g.t[tl][i];         // dLam . G, read one row down below
-                const float dg = nth * c1 * lam;                // dG, stored symmetrised
-                if (col < row) { A1[row * LDM + col] = dg; A1[col * LDM + row] = dg; }
-                if (col == row) A1[row * LDM + col] = 0.f;
+                if constexpr (!FROZEN) {
+                    A2[row * LDM + col] = lam * g.t[tl][i];     // dLam . G, read one row down below
+                    const float dg = nth * c1 * lam;            // dG, stored symmetrised
+                    if (col < row) { A1[row * LDM + col] = dg; A1[col * LDM + row] = dg; }
+                    if (col == row) A1[row * LDM + col] = 0.f;
+                }
                 dwa.t[tl][i] = yu * p.t[tl][i];
             }
     }
@@ -548,7 +575,7 @@ __global__ __launch_bounds__(kThr) void ex_grads_kernel(
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 const int row = m0 + row_of(i, l), col = n0 + 16 * tl + (l & 15);
-                const float dw = dwa.t[tl][i] + (row + 1 < CW ? A2[(row + 1) * LDM + col] : 0.f);
+                const float dw = dwa.t[tl][i] + (!FROZEN && row + 1 < CW ? A2[(row + 1) * LDM + col] : 0.f);
                 xo[col * CW + row] = -cf.th[col] * dw;          // [s][t]
                 cs[tl] = fmaf(dw, Cc[row * LDM + col], cs[tl]);
             }
@@ -590,7 +617,7 @@ __global__ __launch_bounds__(kThr) void ex_grads_kernel(
         {
             Strip r2 = zero_strip(), r3 = zero_strip();
             MMA(dk, [&](int m, int kk) { return dPs[kk * LDM + m0 + m]; }, [&](int kk, int n) { return Qs[kk * LDM + n0 + n]; });
-            MMA(dk, [&](int m, int kk) { return dGs[(m0 + m) * LDM + kk]; }, [&](int kk, int n) { return Ks[kk * LDM + n0 + n]; });
+            if (!FROZEN) MMA(dk, [&](int m, int kk) { return dGs[(m0 + m) * LDM + kk]; }, [&](int kk, int n) { return Ks[kk * LDM + n0 + n]; });
 #pragma unroll
             for (int tl = 0; tl < 2; tl++)
 #pragma unroll
@@ -608,7 +635,7 @@ __global__ __launch_bounds__(kThr) void ex_grads_kernel(
             Strip drm = zero_strip(), drs = zero_strip(), r4 = zero_strip(), r5 = zero_strip();
             auto aR = [&](int m, int kk) { return dRs[(m0 + m) * LDM + kk]; };
             MMD(drm, aR, [&](int kk, int n) { return M0s[kk * LDM + n0 + n]; });
-            if (has_s) MMD(drs, aR, [&](int kk, int n) { return S0s[kk * LDM + n0 + n]; });
+            if (!FROZEN && has_s) MMD(drs, aR, [&](int kk, int n) { return S0s[kk * LDM + n0 + n]; });
 #pragma unroll
             for (int tl = 0; tl < 2; tl++)
 #pragma unroll
@@ -620,8 +647,10 @@ __global__ __launch_bounds__(kThr) void ex_grads_kernel(
                     if (row < L)
                         d_k[(tok + row) * D + col] = dk.t[tl][i] + cv.am[row] * drm.t[tl][i] + cv.bm[row] * drs.t[tl][i];
                 }
-            publish(4, r4);
-            publish(5, r5);
+            if constexpr (!FROZEN) {
+                publish(4, r4);
+                publish(5, r5);
+            }
         }
     }
     __syncthreads();
@@ -629,7 +658,7 @@ __global__ __launch_bounds__(kThr) void ex_grads_kernel(
         const int t = tid;
         auto sum = [&](int which, int row) { return D == 64 ? part[which][0][row] + part[which][1][row] : part[which][0][row]; };
         const float g1 = sum(2, t), g2 = sum(3, t);
-        const float dam = t + 1 < CW ? sum(4, t + 1) : 0.f, dbm = t + 1 < CW ? sum(5, t + 1) : 0.f;
+        const float dam = !FROZEN && t + 1 < CW ? sum(4, t + 1) : 0.f, dbm = !FROZEN && t + 1 < CW ? sum(5, t + 1) : 0.f;
         d_theta[tok + t] = -(((part_th[0][t] + part_th[1][t]) + (part_th[2][t] + part_th[3][t])) + cf.cl[t] * g1 + cf.bl[t] * g2);
         float *pv = pvec + (tok + t) * 4;
         pv[0] = sum(0, t) + dam;
@@ -647,7 +676,7 @@ constexpr size_t kExGradsLds = 9 * MAT * sizeof(float);
 // so the end state is affine in the start state with the matrices Z^T (w.K): the same scan as the backward's, first chunk
 // first.  Nothing else leaves this pass; the tokens of a chunk are then walked from its start state by the sequential
 // kernel (rule_fwd_kernel with FwdArgs::sub_chunks), all chunks at once.
-template <int D>
+template <int D, bool FROZEN>
 __global__ __launch_bounds__(kThr) void ex_fwd_local_kernel(
     const float *__restrict__ k, const float *__restrict__ v, const float *__restrict__ alpha, const float *__restrict__ theta,
     const float *__restrict__ eta, float *__restrict__ loc, int s, int stride, int C, int nc, int maps, int has_s) {
@@ -673,7 +702,8 @@ __global__ __launch_bounds__(kThr) void ex_fwd_local_kernel(
         commit(Vs, tv, tid);
     }
     __syncthreads();
-    chunk_vectors(cv, cf, L);
+    chunk_vectors<FROZEN>(cv, cf, L);
+    if constexpr (!FROZEN) {
     {
         Strip g = zero_strip();
         auto a = [&](int m, int kk) { return Ks[(m0 + m) * LDM + kk]; };
@@ -704,6 +734,7 @@ __global__ __launch_bounds__(kThr) void ex_fwd_local_kernel(
         if (has_s) for_c(z2, [&](int r, int c, float &x) { Dg[(m0 + r) * LDM + n0 + c] = x; }, l);
     }
     __syncthreads();
+    } else __syncthreads();   // the vectors are there
     float *out = loc + ((size_t)chain * nc + ci) * kExLocMats * DD;
     const int sib = D == 64 ? ib : w & 1, sn0 = D == 64 ? n0 : 0, sm0 = 16 * sib;
     const int o0 = D == 64 ? 0 : w >> 1, ostep = D == 64 ? 1 : 4;
@@ -711,9 +742,10 @@ __global__ __launch_bounds__(kThr) void ex_fwd_local_kernel(
 #pragma unroll 1
     for (int o = o0; o < 6; o += ostep) {   // matrix 2 * destination + source, then C_M, C_S
         if (!has_s && (o == 1 || o == 2 || o == 3 || o == 5)) continue;
-        const float *wv = (o == 2 || o == 3 || o == 5) ? cv.wS : cv.wM, *Z = o >= 4 ? Cc : (o & 1) ? Dg : B8;
+        const float *wv = (o == 2 || o == 3 || o == 5) ? cv.wS : cv.wM;
+        const float *Z = FROZEN ? (o >= 4 ? Vs : Ks) : o >= 4 ? Cc : (o & 1) ? Dg : B8;   // FROZEN: Z1 = K, Z2 = 0, T V = V
         Strip x = zero_strip();
-        mma(x, [&](int m, int kk) { return Z[kk * LDM + sm0 + m]; }, [&](int kk, int n) { return wv[kk] * Ks[kk * LDM + sn0 + n]; }, l);
+        if (!(FROZEN && (o == 1 || o == 3))) mma(x, [&](int m, int kk) { return Z[kk * LDM + sm0 + m]; }, [&](int kk, int n) { return wv[kk] * Ks[kk * LDM + sn0 + n]; }, l);
         const float dg = o == 0 ? aL : o == 1 ? bL : o == 3 ? hL : 0.f;
         for_c(x, [&](int r, int c, float &y) { y = o >= 4 ? -y : sm0 + r == sn0 + c ? y + dg : y; }, l);
         float *mat = out + (size_t)o * DD;
@@ -745,8 +777,8 @@ static int chunk_of(int C) { return C * (CW / C); }
 // chain's tokens at 0.6 each on a quarter of a compute unit's worth of workgroups (four per chain, one at head size 32),
 // the kernel that reads a whole trajectory at 1.1.  Under a clip or a bound the test on the errors adds two launches to the
 // matrix form where the fused kernel's only adds one on its maxima.
-bool exact_backward_mm_pays(int seq_len, int batch, int d, int C, bool tested) {
-    const int nc = ceil_div(seq_len, chunk_of(C)), cus = compute_units();
+bool exact_backward_mm_pays(int seq_len, int batch, int d, int C, bool tested, bool frozen) {
+    const int nc = ceil_div(seq_len, frozen ? C : chunk_of(C)), cus = compute_units();
     const double t_mm = (double)ceil_div(batch * nc, cus) * (d == 64 ? 65.0 : 42.0) + nc * (d == 64 ? 2.0 : 0.5) + (tested ? 20.0 : 10.0);
     const double t_seq = (double)seq_len * (C == 1 ? 1.1 : 0.6) * ceil_div(batch * (d == 64 ? 4 : 1), cus);
     return t_mm < t_seq;
@@ -756,33 +788,33 @@ bool exact_backward_mm_pays(int seq_len, int batch, int d, int C, bool tested) {
 // one at head size 32) fit the chip.  The chunk maps cost 26 of a compute unit per chunk (17 at head size 32), a scan
 // step 2.0 (0.5), and, unless only the final states are wanted, the walk of the chunks' tokens again 0.15 a token for
 // whatever does not run at the same time.
-bool exact_forward_mm_pays(int seq_len, int batch, int d, bool final_only) {
-    const int nc = ceil_div(seq_len, CW), cus = compute_units(), parts = d == 64 ? 4 : 1;
+bool exact_forward_mm_pays(int seq_len, int batch, int d, bool final_only, int run) {
+    const int nc = ceil_div(seq_len, run), cus = compute_units(), parts = d == 64 ? 4 : 1;
     if (nc < 2) return false;
     double t_mm = (double)ceil_div(batch * (final_only ? nc : nc - 1), cus) * (d == 64 ? 26.0 : 17.0) + nc * (d == 64 ? 2.0 : 0.5) + 8.0;
-    if (!final_only) t_mm += 0.15 * CW * ceil_div((long long)batch * nc * parts, cus);
+    if (!final_only) t_mm += 0.15 * run * ceil_div((long long)batch * nc * parts, cus);
     const double t_seq = 0.15 * seq_len * ceil_div(batch * parts, cus);
     return t_mm < t_seq;
 }
 
-template <int D>
+template <int D, bool FROZEN>
 static void forward_states_t(bool has_s, const float *k, const float *v, const float *alpha, const float *theta, const float *eta,
                              const float *m_initial, const float *s_initial, long long m_stride, float *m_states, float *s_states,
-                             long long state_stride, int sstep, int seq_len, int input_stride, int batch) {
+                             long long state_stride, int sstep, int seq_len, int input_stride, int batch, int C) {
     const ErrorScope es;
     // to the starts of all chunks, or (sstep 0) through the last one to the end
-    const int nc = ceil_div(seq_len, CW), maps = sstep ? nc - 1 : nc;
+    const int nc = ceil_div(seq_len, C), maps = sstep ? nc - 1 : nc;
     float *loc = scratch(32, (size_t)batch * nc * kExLocMats * D * D * sizeof(float));
     static bool attr_set = false;
     if (!attr_set) {
-        set_lds(ex_fwd_local_kernel<D>, kExFwdLds);
+        set_lds(ex_fwd_local_kernel<D, FROZEN>, kExFwdLds);
         attr_set = true;
     }
     if (es.failed()) return;
     {
         KernelTimer kt("ex_fwd_local_kernel");
-        hipLaunchKernelGGL(ex_fwd_local_kernel<D>, dim3((unsigned)batch * maps), dim3(kThr), kExFwdLds, stream(), k, v, alpha, theta,
-                           has_s ? eta : alpha, loc, seq_len, input_stride, CW, nc, maps, (int)has_s);
+        hipLaunchKernelGGL((ex_fwd_local_kernel<D, FROZEN>), dim3((unsigned)batch * maps), dim3(kThr), kExFwdLds, stream(), k, v, alpha, theta,
+                           has_s ? eta : alpha, loc, seq_len, input_stride, C, nc, maps, (int)has_s);
         check_launch("ex_fwd_local_kernel");
     }
     KernelTimer kt("ex_scan_kernel");
@@ -796,21 +828,22 @@ static void forward_states_t(bool has_s, const float *k, const float *v, const f
     check_launch("ex_scan_kernel");
 }
 
-void exact_forward_states(bool has_s, int d, const float *k, const float *v, const float *alpha, const float *theta, const float *eta,
-                          const float *m_initial, const float *s_initial, long long m_stride, float *m_states, float *s_states,
-                          long long state_stride, int sstep, int seq_len, int input_stride, int batch) {
-    (d == 64 ? forward_states_t<64> : forward_states_t<32>)(has_s, k, v, alpha, theta, eta, m_initial, s_initial, m_stride, m_states,
-                                                            s_states, state_stride, sstep, seq_len, input_stride, batch);
+void exact_forward_states(bool has_s, bool frozen, int d, int run, const float *k, const float *v, const float *alpha, const float *theta,
+                          const float *eta, const float *m_initial, const float *s_initial, long long m_stride, float *m_states,
+                          float *s_states, long long state_stride, int sstep, int seq_len, int input_stride, int batch) {
+    auto fn = frozen ? forward_states_t<32, true> : d == 64 ? forward_states_t<64, false> : forward_states_t<32, false>;
+    fn(has_s, k, v, alpha, theta, eta, m_initial, s_initial, m_stride, m_states, s_states, state_stride, sstep, seq_len, input_stride,
+       batch, run);
 }
 
-template <int D>
+template <int D, bool FROZEN>
 static bool backward_mm_t(const char *fn, bool has_s, const float *k, const float *v, const float *q, const float *alpha,
                           const float *theta, const float *eta, const float *m_ckpt, const float *s_ckpt, const float *d_y,
                           float *d_k, float *d_v, float *d_q, float *d_alpha, float *d_theta, float *d_eta, float *d_m_initial,
                           float *d_s_initial, int seq_len, int batch, int interval, float error_clip, float m_norm_guard) {
     const ErrorScope es;
     constexpr size_t DD = (size_t)D * D;
-    const int C = chunk_of(interval), cstep = C / interval;
+    const int C = FROZEN ? interval : chunk_of(interval), cstep = C / interval;   // a frozen chunk is what the caller says
     const int nc = ceil_div(seq_len, C), nck = interval == 1 ? seq_len + 1 : n_ckpt_count(seq_len, interval);
     const size_t nchunks = (size_t)batch * nc;
     const bool guard = error_clip > 0.f || m_norm_guard > 0.f;
@@ -832,9 +865,9 @@ static bool backward_mm_t(const char *fn, bool has_s, const float *k, const floa
     float *first_m = first, *first_s = first + (size_t)batch * DD;
     static bool attr_set = false;
     if (!attr_set) {
-        set_lds(ex_local_kernel<D, false>, kExLocalLds);
-        set_lds(ex_local_kernel<D, true>, kExLocalLds);
-        set_lds(ex_grads_kernel<D>, kExGradsLds);
+        set_lds(ex_local_kernel<D, FROZEN, false>, kExLocalLds);
+        set_lds(ex_local_kernel<D, FROZEN, true>, kExLocalLds);
+        set_lds(ex_grads_kernel<D, FROZEN>, kExGradsLds);
         attr_set = true;
     }
     if (es.failed()) return true;
@@ -842,7 +875,7 @@ static bool backward_mm_t(const char *fn, bool has_s, const float *k, const floa
     const float *et = has_s ? eta : alpha;
     {
         KernelTimer kt("ex_local_kernel");
-        auto kernel = guard ? ex_local_kernel<D, true> : ex_local_kernel<D, false>;
+        auto kernel = guard ? ex_local_kernel<D, FROZEN, true> : ex_local_kernel<D, FROZEN, false>;
         hipLaunchKernelGGL(kernel, dim3((unsigned)pgrid), dim3(kThr), kExLocalLds, stream(), k, v, q, d_y, alpha, theta, et,
                            m_ckpt, s_ckpt, loc, Tg, Ug, dUg, seq_len, C, nc, nck, cstep, (int)has_s, (int)nchunks, tracks);
         check_launch("ex_local_kernel");
@@ -861,7 +894,7 @@ static bool backward_mm_t(const char *fn, bool has_s, const float *k, const floa
     }
     {
         KernelTimer kt("ex_grads_kernel");
-        hipLaunchKernelGGL(ex_grads_kernel<D>, dim3((unsigned)pgrid), dim3(kThr), kExGradsLds, stream(), k, q, d_y, alpha, theta,
+        hipLaunchKernelGGL((ex_grads_kernel<D, FROZEN>), dim3((unsigned)pgrid), dim3(kThr), kExGradsLds, stream(), k, q, d_y, alpha, theta,
                            et, m_ckpt, s_ckpt, Tg, Ug, dUg, em, esn, d_k, d_v, d_q, d_theta, pvec, xs, scal, seq_len, C, nc, nck, cstep,
                            (int)has_s, (int)nchunks);
         check_launch("ex_grads_kernel");
@@ -875,7 +908,7 @@ static bool backward_mm_t(const char *fn, bool has_s, const float *k, const floa
     return true;
 }
 
-bool exact_backward_mm(const char *fn, bool has_s, int d, const float *k, const float *v, const float *q, const float *alpha,
+bool exact_backward_mm(const char *fn, bool has_s, bool frozen, int d, const float *k, const float *v, const float *q, const float *alpha,
                        const float *theta, const float *eta, const float *m_ckpt, const float *s_ckpt, const float *d_y,
                        float *d_k, float *d_v, float *d_q, float *d_alpha, float *d_theta, float *d_eta, float *d_m_initial,
                        float *d_s_initial, int seq_len, int batch, int C, float error_clip, float m_norm_guard) {
@@ -884,9 +917,9 @@ bool exact_backward_mm(const char *fn, bool has_s, int d, const float *k, const 
              fn, seq_len, batch, d, C, CW);
         return true;
     }
-    return (d == 64 ? backward_mm_t<64> : backward_mm_t<32>)(fn, has_s, k, v, q, alpha, theta, eta, m_ckpt, s_ckpt, d_y, d_k, d_v, d_q,
-                                                             d_alpha, d_theta, d_eta, d_m_initial, d_s_initial, seq_len, batch, C,
-                                                             error_clip, m_norm_guard);
+    auto run = frozen ? backward_mm_t<32, true> : d == 64 ? backward_mm_t<64, false> : backward_mm_t<32, false>;
+    return run(fn, has_s, k, v, q, alpha, theta, eta, m_ckpt, s_ckpt, d_y, d_k, d_v, d_q, d_alpha, d_theta, d_eta, d_m_initial,
+               d_s_initial, seq_len, batch, C, error_clip, m_norm_guard);
 }
 
 }  // namespace nlh

@@ -43,11 +43,12 @@ static __global__ void zero_fill_kernel(float *__restrict__ p, size_t n) {
 // errors of a chunk are taken against the chunk-start M; ckpt_interval is the
 // chunk size and the stored checkpoints are the chunk-boundary states.
 // MODE: 0 rows split over workgroups, 1 COUPLED (clip / projection: a chain in one workgroup), 2 as 0 and keeps the
-// bound of max_t |M_t|_F^2 that FwdArgs::msq_part describes, 3 as 0 over the runs of FwdArgs::sub_chunks (a mode of its
-// own: the straight-line tile code of mode 0 schedules 15 % worse with the runs' conditions in it).
+// bound of max_t |M_t|_F^2 that FwdArgs::msq_part describes, 3 and 4 as 0 and 2 over the runs of FwdArgs::sub_chunks (modes
+// of their own: the straight-line tile code of mode 0 schedules 15 % worse with the runs' conditions in it; the bound is
+// per run).
 template <int D, int RPL, bool HAS_S, int STORE, int MODE, bool FROZEN>
 __global__ __launch_bounds__(kThreads) void rule_fwd_kernel(FwdArgs a) {
-    constexpr bool COUPLED = MODE == 1, TRACK = MODE == 2;
+    constexpr bool COUPLED = MODE == 1, TRACK = MODE == 2 || MODE == 4;
     constexpr int LPR = D / 4;          // lanes per row
     constexpr int RG = 64 / LPR;        // row groups per wave
     constexpr int ROWS_WG = kWaves * RG * RPL;
@@ -68,14 +69,14 @@ __global__ __launch_bounds__(kThreads) void rule_fwd_kernel(FwdArgs a) {
     const int row_local = (wave * RG + g) * RPL;
     const int row0 = part * ROWS_WG + row_local;
     // a run of a chain (FwdArgs::sub_chunks): tokens [sub0, sub0 + seq_len) from the state in its slot
-    constexpr bool sub = MODE == 3;
-    int sub0 = 0, seq_len = a.seq_len;
+    constexpr bool sub = MODE >= 3;
+    int run = 0, sub0 = 0, seq_len = a.seq_len;
     bool sub_last = true;
     if constexpr (sub) {
-        const int run = chain % a.sub_chunks;
+        run = chain % a.sub_chunks;
         chain /= a.sub_chunks;
-        sub0 = run * kExactChunk;
-        seq_len = min(kExactChunk, a.seq_len - sub0);
+        sub0 = run * a.run_len;
+        seq_len = min(a.run_len, a.seq_len - sub0);
         sub_last = run == a.sub_chunks - 1;
     }
 
@@ -217,7 +218,7 @@ __global__ __launch_bounds__(kThreads) void rule_fwd_kernel(FwdArgs a) {
                 if (STORE == STORE_TRAJ) {
 #pragma unroll
                     for (int r = 0; r < RPL; r++)
-                        if ((ALL_VALID || valid[r]) && (!sub || sub_last || t + 1 < kExactChunk)) {
+                        if ((ALL_VALID || valid[r]) && (!sub || sub_last || t + 1 < a.run_len)) {
                             size_t off = (size_t)(t + 1) * DD + (size_t)(row0 + r) * D + cb * 4;
                             *reinterpret_cast<float4 *>(mo + off) = M[r];
                             if (HAS_S) *reinterpret_cast<float4 *>(so + off) = S[r];
@@ -230,7 +231,7 @@ __global__ __launch_bounds__(kThreads) void rule_fwd_kernel(FwdArgs a) {
                         if (STORE == STORE_CKPT) {
 #pragma unroll
                             for (int r = 0; r < RPL; r++)
-                                if ((ALL_VALID || valid[r]) && (!sub || sub_last || t + 1 < kExactChunk)) {
+                                if ((ALL_VALID || valid[r]) && (!sub || sub_last || t + 1 < a.run_len)) {
                                     size_t off = (size_t)ckpt_slot * DD + (size_t)(row0 + r) * D + cb * 4;
                                     *reinterpret_cast<float4 *>(mo + off) = M[r];
                                     if (HAS_S) *reinterpret_cast<float4 *>(so + off) = S[r];
@@ -260,7 +261,7 @@ __global__ __launch_bounds__(kThreads) void rule_fwd_kernel(FwdArgs a) {
     if (ntiles > 0) flush_y(ntiles - 1);
     if (TRACK) {
         const float tot = block_allreduce(nmax, sred[0], tid);
-        if (tid == 0) a.msq_part[chain * a.parts + part] = tot;
+        if (tid == 0) a.msq_part[(sub ? chain * a.sub_chunks + run : chain) * a.parts + part] = tot;
     }
 }
 
@@ -617,9 +618,10 @@ template <int D, int RPL, bool HAS_S, int STORE, bool FROZEN>
 static void launch_fwd_c(const FwdArgs &a, int batch, bool coupled) {
     dim3 grid(batch * a.parts), block(kThreads);
     KernelTimer kt("rule_fwd_kernel");
-    if constexpr (!FROZEN && STORE != STORE_NONE && (D == 64 || D == 32)) {
+    if constexpr (STORE != STORE_NONE && (D == 64 || D == 32)) {
         if (a.sub_chunks > 1) {
-            hipLaunchKernelGGL((rule_fwd_kernel<D, RPL, HAS_S, STORE, 3, FROZEN>), grid, block, 0, stream(), a);
+            if (a.msq_part) hipLaunchKernelGGL((rule_fwd_kernel<D, RPL, HAS_S, STORE, 4, FROZEN>), grid, block, 0, stream(), a);
+            else hipLaunchKernelGGL((rule_fwd_kernel<D, RPL, HAS_S, STORE, 3, FROZEN>), grid, block, 0, stream(), a);
             check_launch("rule_fwd_kernel");
             return;
         }
@@ -666,36 +668,46 @@ static bool launch_fwd_as(FwdArgs a, int d, int batch, bool coupled) {
 // error clip, the uncoupled kernels run first and keep an upper bound of max_t |M_t|_F^2 per workgroup; when the
 // bound stays below m_norm_max^2 no projection could have fired and their results are the coupled kernels' (one
 // 4-byte read-back and a stream synchronisation decide); otherwise the coupled kernels run and overwrite everything.
+// Few long chains leave the sequential walk's chip idle: where it pays the uncoupled kernels run over independent runs of
+// every chain, from chunk-start states by the matrix form's scan (exact_mm.h).  tracked_rows: leave the bound's partial
+// maxima in scratch 23, that many rows of them.
+template <bool HAS_S, int STORE, bool FROZEN>
+static bool launch_fwd_uncoupled(FwdArgs a, int d, int batch, int *tracked_rows) {
+    const ErrorScope es;
+    int rows = batch;
+    if constexpr (STORE != STORE_NONE) {
+        const int run = FROZEN ? a.ckpt_interval : kExactChunk;
+        const bool kept = FROZEN || STORE == STORE_TRAJ || kExactChunk % a.ckpt_interval == 0;   // the slots of all run starts exist
+        if (kept && exact_mm_applies(d, FROZEN ? run : 1) && !(FROZEN && d == 64) && g_exact_form != 2 &&
+            (g_exact_form == 1 ? a.seq_len > run : exact_forward_mm_pays(a.seq_len, batch, d, false, run))) {
+            const int sstep = FROZEN ? 1 : STORE == STORE_TRAJ ? run : run / a.ckpt_interval;
+            exact_forward_states(HAS_S, FROZEN, d, run, a.k, a.v, a.alpha, a.theta, a.eta, a.m_initial, a.s_initial, a.m_stride, a.m_out,
+                                 a.s_out, a.state_stride, sstep, a.seq_len, a.input_stride, batch);
+            a.sub_chunks = ceil_div(a.seq_len, run);
+            a.run_len = run;
+            rows *= a.sub_chunks;
+        }
+    }
+    if (tracked_rows) {
+        a.msq_part = scratch(23, (size_t)rows * ceil_div(d, rows_per_wg(d, pick_rpl(d, rows, false))) * sizeof(float));
+        *tracked_rows = rows;
+    }
+    return es.failed() || launch_fwd_as<HAS_S, STORE, FROZEN>(a, d, rows, false);
+}
+
 template <bool HAS_S, int STORE, bool FROZEN = false>
 static bool launch_fwd(FwdArgs a, int d, int batch) {
     const bool coupled = coupled_needed(a.error_clip, a.m_norm_max);
-    if (coupled && a.error_clip <= 0.f && tiled_size(d) && guard_possible()) {
+    if (!coupled) return launch_fwd_uncoupled<HAS_S, STORE, FROZEN>(a, d, batch, nullptr);
+    if (a.error_clip <= 0.f && tiled_size(d) && guard_possible()) {
         const ErrorScope es;
-        FwdArgs u = a;
-        const int rpl = pick_rpl(d, batch, false), parts = ceil_div(d, rows_per_wg(d, rpl));
-        u.msq_part = scratch(23, (size_t)batch * parts * sizeof(float));
+        int rows = 0;
+        launch_fwd_uncoupled<HAS_S, STORE, FROZEN>(a, d, batch, &rows);
         if (es.failed()) return true;
-        launch_fwd_as<HAS_S, STORE, FROZEN>(u, d, batch, false);
-        if (es.failed()) return true;
-        if (!norm_bound_exceeded(u.msq_part, batch, parts, a.m_norm_max)) return true;
+        const int parts = ceil_div(d, rows_per_wg(d, pick_rpl(d, rows, false)));
+        if (!norm_bound_exceeded(scratch(23, (size_t)rows * parts * sizeof(float)), rows, parts, a.m_norm_max)) return true;
     }
-    a.msq_part = nullptr;
-    // few long chains leave the sequential walk's chip idle: chunk-start states by the matrix form's scan, then all
-    // chunks' tokens at once
-    if constexpr (!FROZEN && STORE != STORE_NONE) {
-        const bool kept = STORE == STORE_TRAJ || kExactChunk % a.ckpt_interval == 0;   // the slots of all chunk starts exist
-        if (!coupled && kept && exact_mm_applies(d, 1) && g_exact_form != 2 &&
-            (g_exact_form == 1 ? a.seq_len > kExactChunk : exact_forward_mm_pays(a.seq_len, batch, d, false))) {
-            const ErrorScope es;
-            const int sstep = STORE == STORE_TRAJ ? kExactChunk : kExactChunk / a.ckpt_interval;
-            exact_forward_states(HAS_S, d, a.k, a.v, a.alpha, a.theta, a.eta, a.m_initial, a.s_initial, a.m_stride, a.m_out, a.s_out,
-                                 a.state_stride, sstep, a.seq_len, a.input_stride, batch);
-            if (es.failed()) return true;
-            a.sub_chunks = ceil_div(a.seq_len, kExactChunk);
-            return launch_fwd_as<HAS_S, STORE, FROZEN>(a, d, batch * a.sub_chunks, false);
-        }
-    }
-    return launch_fwd_as<HAS_S, STORE, FROZEN>(a, d, batch, coupled);
+    return launch_fwd_as<HAS_S, STORE, FROZEN>(a, d, batch, true);
 }
 
 template <int D, int RPL, bool HAS_S, bool FROZEN>
@@ -896,15 +908,16 @@ static void backward_ckpt_any(bool has_s, bool frozen, bool allow_fused,
     // directly, and so does a call under a bound right after any other test of a bound that fired.
     const bool coupled = bound || error_clip > 0.f;
     static int skip_left = 0, skip_len = 0;
-    bool try_mm = allow_fused && !frozen && exact_mm_applies(d, C) && g_exact_form != 2 &&
-                  (g_exact_form == 1 || exact_backward_mm_pays(seq_len, batch, d, C, coupled));
+    // (the frozen rule at head size 64 has matrix kernels of its own, which its entry points call before this)
+    bool try_mm = (allow_fused || frozen) && !(frozen && d == 64) && exact_mm_applies(d, C) && g_exact_form != 2 &&
+                  (g_exact_form == 1 || exact_backward_mm_pays(seq_len, batch, d, C, coupled, frozen));
     if (try_mm && coupled) {
         if (!guard_possible()) try_mm = false;
         else if (skip_left > 0) { skip_left--; try_mm = false; }
         else if (error_clip <= 0.f && last_test_fired) try_mm = false;
     }
     if (try_mm) {
-        if (exact_backward_mm(fn, has_s, d, k, v, q, alpha, theta, eta, m_ckpt, s_ckpt, d_y, d_k, d_v, d_q, d_alpha, d_theta,
+        if (exact_backward_mm(fn, has_s, frozen, d, k, v, q, alpha, theta, eta, m_ckpt, s_ckpt, d_y, d_k, d_v, d_q, d_alpha, d_theta,
                               d_eta, d_m_initial, d_s_initial, seq_len, batch, C, error_clip, bound ? m_norm_max : 0.f)) {
             if (coupled) skip_len = 0;
             return;
@@ -949,10 +962,10 @@ static void final_states(const char *fn, const float *k, const float *v, const f
     if (seq_len == 0) { fail("%s: seq_len=0.", fn); return; }
     const size_t dd = (size_t)d * d;
     // three launches of the matrix form against one walk at 0.15 us a token (see exact_forward_mm_pays)
-    if (exact_mm_applies(d, 1) && g_exact_form != 2 && (g_exact_form == 1 || exact_forward_mm_pays(seq_len, batch, d, true))) {
+    if (exact_mm_applies(d, 1) && g_exact_form != 2 && (g_exact_form == 1 || exact_forward_mm_pays(seq_len, batch, d, true, kExactChunk))) {
         float *sf = HAS_S ? scratch(9, (size_t)batch * dd * sizeof(float)) : nullptr;
         if (es.failed()) return;
-        exact_forward_states(HAS_S, d, k, v, alpha, theta, eta, m_initial, s_initial, (long long)dd, m_final, sf, (long long)dd, 0, seq_len,
+        exact_forward_states(HAS_S, false, d, kExactChunk, k, v, alpha, theta, eta, m_initial, s_initial, (long long)dd, m_final, sf, (long long)dd, 0, seq_len,
                              seq_len, batch);
         return;
     }

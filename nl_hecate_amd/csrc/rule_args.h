@@ -15,10 +15,10 @@ struct FwdArgs {
     // uncoupled kernels only, may be null: [batch * parts] upper bounds of max_t sum(M_t^2) over the workgroup's rows
     // (every lane keeps the largest sum of squares its own elements reached; the lanes' maxima are added up)
     float *msq_part;
-    // > 1: every chain is walked as that many independent runs of 64 tokens (the last may be shorter), run c from the
+    // > 1: every chain is walked as that many independent runs of run_len tokens (the last may be shorter), run c from the
     // state that already stands at its slot of m_out / s_out (exact_mm.h).  A run leaves the slot of its own start and of
     // the next run's start alone.
-    int sub_chunks;
+    int sub_chunks, run_len;
 };
 
 enum { STORE_NONE = 0, STORE_TRAJ = 1, STORE_CKPT = 2 };

@@ -9,6 +9,7 @@ from nl_hecate_amd import dispatch as D
 from nl_hecate_amd.ffi import lib
 from oracle import pyoracle as orc
 from tests.gpu_util import assert_close, dev, host, rule_inputs, zeros
+from tests.test_gpu_chunkwise import gpu_chunkwise, oracle_chunkwise
 from tests.test_gpu_exact_mm import F32_MAX, check, gpu_backward, kernels_run, oracle_pair
 
 pytestmark = pytest.mark.gpu
@@ -96,3 +97,20 @@ def test_titans_forward(B, s, d, C):
         assert_close("y", host(y)[b], yo, 1e-4)
         assert_close("m", host(mc)[b], ms.reshape(n, -1), 1e-4)
         assert_close("s", host(sc)[b], ss.reshape(n, -1), 1e-4)
+
+
+@pytest.mark.parametrize("has_s", [True, False])
+@pytest.mark.parametrize("B,s,C,bound", [(3, 130, 64, F32_MAX), (2, 200, 20, F32_MAX), (9, 65, 16, F32_MAX), (1, 40, 1, F32_MAX),
+                                         (2, 64, 64, F32_MAX), (3, 150, 32, 1e4)])
+def test_frozen_rule_at_head_size_32(has_s, B, s, C, bound):
+    """The frozen-M0 chunkwise rule in the same kernels; its chunks are the caller's (one chunk: the plain walk forward)."""
+    print(has_s, B, s, C, bound, flush=True)
+    x = rule_inputs(B, s, 32, seed=11 + s + C, m0_scale=0.05)
+    (fo, go), got = oracle_chunkwise(x, C, has_s, mx=bound), []
+    gpu_chunkwise(x, C, has_s, mx=bound)   # a test that fired in an earlier call sends the next one to the sequential kernels
+    ran = kernels_run(lambda: got.extend(gpu_chunkwise(x, C, has_s, mx=bound)))
+    assert "ex_grads_kernel" in ran and ("ex_fwd_local_kernel" in ran) == (s > C), ran
+    for n in ("y", "mc") + (("sc",) if has_s else ()):
+        assert_close(n, got[0][n], fo[n], 1e-4)
+    for n in go:
+        assert_close(n, got[1][n], go[n], 1e-4)
