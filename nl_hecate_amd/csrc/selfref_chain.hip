@@ -1,0 +1,536 @@
+// HOPE self-referential memory, forward for chunks of up to 64 tokens, as three launches.
+//
+// With the snapshot F_c of the chunk's start every memory moves by one outer product a token,
+//     M_c <- (1-a_t) M_c + th_t w_c,t k_t^T,    w_c,t = v_t - F_c k_t   (self-generated values: F_c (v_t - k_t)),
+// and only k_t = M_k x_t, v_t = M_v x_t and the gates (means over the rows of M_alpha x_t, M_eta x_t) feed back into
+// the recurrence.  So the part that is bound to one workgroup per chain carries M_k, M_v and the row means of M_alpha,
+// M_eta, M_v; what hangs off it (the other four memories, q_t = M_q x_t and y_t = M_mem q_t) is left to kernels that
+// use the whole chip:
+//   selfref_chain_kernel  one workgroup per chain:               k, v, gates, snapshots of M_k, M_v
+//   selfref_scan_kernel   one workgroup per (chain, memory):     M_q, M_eta, M_alpha, M_mem chunk by chunk
+//   selfref_read_kernel   one workgroup per (chain, chunk):      q and y from the snapshots
+#include <hip/hip_runtime.h>
+
+#include <utility>
+
+#include "../../include/nl_hecate_ffi.h"
+#include "lane_ops.h"
+#include "quad_rows.h"
+#include "runtime.h"
+#include "selfref_chunk.h"
+
+namespace nlh {
+namespace {
+
+__device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ float lane_from(int byte_addr, float x) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(byte_addr, __builtin_bit_cast(int, x)));
+}
+__device__ __forceinline__ float lane_value(float x, int lane) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), lane));
+}
+template <int LANE>
+__device__ __forceinline__ void set_lane(float &x, float uniform) {
+    asm("v_writelane_b32 %0, %1, %2" : "+v"(x) : "s"(uniform), "n"(LANE));
+}
+template <int Q>
+__device__ __forceinline__ float quad_lane(float x) { return dpp_mov<Q * 0x55>(x); }
+// The gates without a branch: the argument is uniform and the value is needed at once.
+__device__ __forceinline__ float sr_sigmoid_select(float x) {
+    const float y = __builtin_amdgcn_rcpf(1.f + __expf(-x));
+    return x >= 15.f ? 1.f : x <= -15.f ? 0.f : y;
+}
+__device__ __forceinline__ float sr_softplus_select(float x) {
+    constexpr float ln2 = 0x1.62e43p-1f, ln2_rest = -0x1.05c61p-29f;  // ln 2 in two parts
+    const float l = __builtin_amdgcn_logf(1.f + __expf(x)), p = l * ln2;
+    const float y = p + fmaf(l, ln2_rest, fmaf(l, ln2, -p));
+    return x >= 15.f ? x : x <= -15.f ? 0.f : y;
+}
+
+// f(0), f(1), ... with the argument as a type, until one returns false
+template <class Fn, int... I>
+__device__ __forceinline__ void while_true(Fn &f, std::integer_sequence<int, I...>) {
+    (void)(f(std::integral_constant<int, I>{}) && ...);
+}
+
+// ── the recurrence ───────────────────────────────────────────────────────────────────────────────────────────────
+// Tiles of 16 tokens.  At a tile's start P_c = M_c X^T for the whole tile comes off the matrix cores; inside the tile
+// token t adds its outer product to the later columns only, P_c[t'] = (1-a_t) P_c[t'] + th_t w_c,t (k_t . x_t'), so a
+// token needs k_t in all waves (one LDS exchange), the products F_k k_t, F_v k_t and the dots of k_t with the tile's x
+// and with the row means; at the tile's end M_c takes the 16 outer products on the matrix cores.
+//
+// Two lane layouts, one a permutation of the other's lanes: the matrix cores' (ml, kg) = (lane % 16, lane / 16) and the
+// quads' (r, cq) = (lane / 4, lane % 4).  Lane (ml, kg) holds row ml of the wave's 16 rows, columns 16 kt + 4 kg + v,
+// which is at once operand and result of the two products (the contraction index runs over (v, kt) in any order);
+// lane (r, cq) holds row r, columns 16 kt + 4 cq + v of F, so that a product with a vector is 16 fused
+// multiply-adds and two DPP adds.  Tokens of a tile go to the matrix cores in the order sigma(4 a + b) = 4 b + a:
+// lane cq then owns the columns t' = 4 j + cq of P, and column group j is finished with token 4 j + 3.
+// The row means are rows 0 (alpha), 1 (eta) and 2 (v) of a third matrix that every wave carries.
+//
+// Bound by the issue rate of one wave per SIMD (155 instructions a token) and the exchange once a token.  64 chains of
+// 2048 tokens, head size 64, chunks of 64: 1.19 ms, with the two kernels below 1.46 ms; one kernel that formed all
+// products of a token with all six memories in sequence (it serves longer chunks, selfref.hip) takes 2.30 ms.  Chunks of
+// 1, 4, 8, 16 tokens at 64 chains of 512: 6.65, 2.05, 1.28, 0.88 ms there, 3.47, 1.07, 0.67, 0.46 ms here.
+__host__ __device__ constexpr int sigma(int t) { return 4 * (t & 3) + (t >> 2); }
+
+template <int D, bool SG>
+__global__ __launch_bounds__(4 * D) void selfref_chain_kernel(
+    float *__restrict__ mems, const float *__restrict__ emb, float *__restrict__ k_cache, float *__restrict__ v_cache,
+    float *__restrict__ alpha_cache, float *__restrict__ theta_cache, float *__restrict__ amean_cache,
+    float *__restrict__ emean_cache, float *__restrict__ frozen, int s, int C, int nc) {
+    constexpr int KT = D / 16, NW = D / 16, DD = D * D, LD = D + 16, V4 = D / 4;
+    __shared__ __align__(16) float xt[2][kTB * LD];
+    __shared__ __align__(16) float Kt[2][kTB * LD], Vt[2][kTB * LD];  // the tile's k, v: exchange and operand
+    __shared__ __align__(16) float Ut[SG ? kTB * LD : 4];             // k - v, exchange only
+    __shared__ __align__(16) float Sx[NW][kTB];
+    __shared__ __align__(16) float mean[3][D];
+
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, wr = 16 * wave;
+    const int ml = lane & 15, kg = lane >> 4, r = lane >> 2, cq = lane & 3;
+    const int to_quad = 4 * (r + 16 * cq), to_mm = 4 * (4 * ml + kg);  // source lanes of the two permutations, in bytes
+    const size_t b = blockIdx.x, tok0 = b * (size_t)s;
+    float *mb = mems + b * 6 * DD;
+
+    // M_k, M_v and the row means in the matrix cores' layout; row means of M_alpha, M_eta, M_v
+    f32x4 M[3][KT];
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
+#pragma unroll
+        for (int kt = 0; kt < KT; kt++)
+            M[c][kt] = *reinterpret_cast<const f32x4 *>(mb + c * DD + (wr + ml) * D + 16 * kt + 4 * kg);
+    }
+    for (int e = tid; e < 3 * D; e += 4 * D) {
+        const int which = e / D;
+        const float *src = mb + (which == 0 ? 4 : which == 1 ? 3 : 1) * DD + e % D;
+        float a = 0.f;
+#pragma unroll 8
+        for (int c = 0; c < D; c++) a += src[c * D];
+        mean[which][e % D] = a * (1.f / D);
+    }
+    // the rows of a partial tile behind its last token enter the end-of-tile product times zero
+    for (int e = tid; e < kTB * LD; e += 4 * D) Kt[0][e] = Kt[1][e] = 0.f;
+
+    const int stt = tid / V4, sj = (tid % V4) * 4;  // staging slot: token, column
+    auto load_x = [&](int t, int n) -> float4 {
+        return stt < n ? *reinterpret_cast<const float4 *>(emb + (tok0 + t + stt) * D + sj) : make_float4(0, 0, 0, 0);
+    };
+    // first token behind the tile that starts at t
+    auto tile_end = [&](int t) { return min(min(t + kTB, (t / C + 1) * C), s); };
+    int te = tile_end(0);
+    *reinterpret_cast<float4 *>(&xt[0][stt * LD + sj]) = load_x(0, te);
+    float4 xnext = te < s ? load_x(te, tile_end(te) - te) : make_float4(0, 0, 0, 0);
+    __syncthreads();
+#pragma unroll
+    for (int kt = 0; kt < KT; kt++)
+        M[2][kt] = ml < 3 ? *reinterpret_cast<const f32x4 *>(&mean[ml < 3 ? ml : 0][16 * kt + 4 * kg])
+                          : f32x4{0.f, 0.f, 0.f, 0.f};
+
+    float F[3][4 * KT];
+    int chunk_t = 0, ci = 0;
+    for (int tb = 0, buf = 0; tb < s; tb = te, buf ^= 1) {
+        te = tile_end(tb);
+        const int nt = te - tb;
+        float *Kb = Kt[buf], *Vb = Vt[buf];
+        if (tb == chunk_t) {  // snapshot
+            float *fb = frozen + (b * nc + ci) * (size_t)6 * DD;
+#pragma unroll
+            for (int c = 0; c < 3; c++) {
+#pragma unroll
+                for (int kt = 0; kt < KT; kt++) {
+                    if (c < 2) *reinterpret_cast<f32x4 *>(fb + c * DD + (wr + ml) * D + 16 * kt + 4 * kg) = M[c][kt];
+#pragma unroll
+                    for (int v = 0; v < 4; v++) F[c][4 * kt + v] = lane_from(to_quad, M[c][kt][v]);
+                }
+            }
+            ci++;
+            chunk_t += C;
+        }
+        // the next tile's x: requested a tile ago, visible after this tile's first exchange
+        if (te < s) {
+            *reinterpret_cast<float4 *>(&xt[buf ^ 1][stt * LD + sj]) = xnext;
+            const int t2 = tile_end(te);
+            if (t2 < s) xnext = load_x(t2, tile_end(t2) - t2);
+        }
+        float P[3][4], X[4 * KT];
+        {
+            f32x4 acc[3] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+            for (int kt = 0; kt < KT; kt++) {
+                const f32x4 xa = *reinterpret_cast<const f32x4 *>(&xt[buf][sigma(ml) * LD + 16 * kt + 4 * kg]);
+                const f32x4 xq = *reinterpret_cast<const f32x4 *>(&xt[buf][sigma(r) * LD + 16 * kt + 4 * cq]);
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    X[4 * kt + v] = xq[v];
+#pragma unroll
+                    for (int c = 0; c < 3; c++) acc[c] = mfma4(xa[v], M[c][kt][v], acc[c]);
+                }
+            }
+#pragma unroll
+            for (int c = 0; c < 3; c++) {
+#pragma unroll
+                for (int v = 0; v < 4; v++) P[c][v] = lane_from(to_quad, acc[c][v]);
+            }
+        }
+        float W[3][4], cs[4], keep_tile = 1.f;  // w_c of token 4 j + cq, th times the retention since, of the whole tile
+#pragma unroll
+        for (int j = 0; j < 4; j++) W[0][j] = W[1][j] = W[2][j] = cs[j] = 0.f;
+        float k = quad_lane<0>(P[0][0]), v = quad_lane<0>(P[1][0]);
+        float am = lane_value(P[2][0], 0), em = lane_value(P[2][0], 4), vm = lane_value(P[2][0], 8);
+        // lane t keeps token t's gate means for the caches; what token t - 1 adds to the columns behind t is added while
+        // token t's exchange is under way
+        float s_am = 0.f, s_em = 0.f;
+        float pw[3] = {0.f, 0.f, 0.f}, pkeep = 1.f;
+        float *const out = (SG ? (cq == 0 ? Kb : cq == 1 ? Vb : Ut) : (cq & 1) ? Vb : Kb) + wr + r;
+
+        auto step = [&](auto T) __attribute__((always_inline)) -> bool {
+            constexpr int t = decltype(T)::value, J = t / 4, Q = t % 4;
+            // every lane of a quad writes, so that no lane is masked out
+            float val = k;
+            if (SG) {
+                const float u = k - v;
+                val = cq == 1 ? v : u;
+                val = cq == 0 ? k : val;
+            } else {
+                val = (cq & 1) ? v : k;
+            }
+            out[t * LD] = val;
+            lds_barrier();
+            float kc[4 * KT], uc[4 * KT];
+            f32x4 ps = f32x4{0.f, 0.f, 0.f, 0.f};
+            if (t > 0 && t + 1 < kTB) ps = *reinterpret_cast<const f32x4 *>(&Sx[wave][4 * cq]);
+#pragma unroll
+            for (int kt = 0; kt < KT; kt++) {
+                const f32x4 k4 = *reinterpret_cast<const f32x4 *>(Kb + t * LD + 16 * kt + 4 * cq);
+                f32x4 u4 = k4;
+                if (SG) u4 = *reinterpret_cast<const f32x4 *>(Ut + t * LD + 16 * kt + 4 * cq);
+#pragma unroll
+                for (int i = 0; i < 4; i++) { kc[4 * kt + i] = k4[i]; uc[4 * kt + i] = u4[i]; }
+            }
+            __builtin_amdgcn_sched_barrier(0);  // what follows runs while the reads are under way, not ahead of the barrier
+            if constexpr (t > 0 && t + 1 < kTB) {
+#pragma unroll
+                for (int j = (t + 1) / 4; j < 4; j++) {
+#pragma unroll
+                    for (int c = 0; c < 3; c++) {
+                        P[c][j] = fmaf(pw[c], ps[j], pkeep * P[c][j]);
+                        asm volatile("" : "+v"(P[c][j]));  // here, not when the column is needed
+                    }
+                }
+            }
+            set_lane<t>(s_am, am);
+            set_lane<t>(s_em, em);
+            const float alpha = sr_sigmoid_select(am), theta = sr_softplus_select(em), keep = 1.f - alpha;
+            const float S = quad_allreduce(dotn<4 * KT>(X, kc));  // row r: k_t . x of token sigma(r)
+            float w[3];  // w_c,t (self-generated values: its negative)
+#pragma unroll
+            for (int c = 0; c < 3; c++) {
+                w[c] = quad_allreduce(dotn<4 * KT>(F[c], uc));
+                if (!SG) w[c] = (c == 2 ? vm : v) - w[c];
+            }
+            const float th = SG ? -theta : theta;
+#pragma unroll
+            for (int j = 0; j <= J; j++) cs[j] *= keep;
+            keep_tile *= keep;
+            cs[J] = cq == Q ? th : cs[J];
+#pragma unroll
+            for (int c = 0; c < 3; c++) W[c][J] = cq == Q ? w[c] : W[c][J];
+            if constexpr (t + 1 < kTB) {
+                constexpr int J1 = (t + 1) / 4, Q1 = (t + 1) % 4;
+                const float s1 = lane_value(S, 4 * sigma(t + 1));
+#pragma unroll
+                for (int c = 0; c < 3; c++) pw[c] = th * w[c];
+                pkeep = keep;
+                k = fmaf(pw[0], s1, keep * quad_lane<Q1>(P[0][J1]));
+                v = fmaf(pw[1], s1, keep * quad_lane<Q1>(P[1][J1]));
+                const float m = fmaf(pw[2], s1, keep * P[2][J1]);
+                am = lane_value(m, Q1);
+                em = lane_value(m, 4 + Q1);
+                vm = lane_value(m, 8 + Q1);
+                if (t + 2 < kTB) Sx[wave][r] = S;  // the wave's own; read back behind the next exchange
+            }
+            return t + 1 < nt;
+        };
+        while_true(step, std::make_integer_sequence<int, kTB>{});
+
+        // M_c <- keep M_c + sum_t cs_t w_c,t k_t^T; every wave has written its part of Kb, Vb
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+#pragma unroll
+            for (int kt = 0; kt < KT; kt++) M[c][kt] *= keep_tile;
+#pragma unroll
+            for (int j = 0; j < 4; j++) W[c][j] = lane_from(to_mm, W[c][j] * cs[j]);
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            if (4 * j < nt) {
+#pragma unroll
+                for (int kt = 0; kt < KT; kt++) {
+                    const float a = Kb[(4 * j + kg) * LD + 16 * kt + ml];
+#pragma unroll
+                    for (int c = 0; c < 3; c++) M[c][kt] = mfma4(a, W[c][j], M[c][kt]);
+                }
+            }
+        }
+        if (stt < nt) {
+            const size_t o = (tok0 + tb + stt) * D + sj;
+            *reinterpret_cast<float4 *>(k_cache + o) = *reinterpret_cast<const float4 *>(Kb + stt * LD + sj);
+            *reinterpret_cast<float4 *>(v_cache + o) = *reinterpret_cast<const float4 *>(Vb + stt * LD + sj);
+        }
+        if (tid < nt) {
+            const size_t o = tok0 + tb + tid;
+            alpha_cache[o] = sr_sigmoid_select(s_am); theta_cache[o] = sr_softplus_select(s_em);
+            amean_cache[o] = s_am; emean_cache[o] = s_em;
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
+#pragma unroll
+        for (int kt = 0; kt < KT; kt++)
+            *reinterpret_cast<f32x4 *>(mb + c * DD + (wr + ml) * D + 16 * kt + 4 * kg) = M[c][kt];
+    }
+}
+
+// ── the other memories ───────────────────────────────────────────────────────────────────────────────────────────
+// Chunk by chunk F <- A_L F + sum_s c_s (v_s - F k_s) k_s^T with c_s = th_s prod_{r>s} (1-a_r), both products on the
+// fp32 matrix cores; a wave owns 16 rows, its lane (ml, kg) row ml, columns 16 kt + 4 kg + v, which serves as operand
+// and as result.  The next chunk's k, v, gates are requested before the products of the current one.
+template <int D, bool SG>
+__global__ __launch_bounds__(4 * D) void selfref_scan_kernel(
+    float *__restrict__ mems, const float *__restrict__ k_cache, const float *__restrict__ v_cache,
+    const float *__restrict__ alpha_cache, const float *__restrict__ theta_cache, float *__restrict__ frozen, int s,
+    int C, int nc, int batch) {
+    constexpr int KT = D / 16, ST = kLrC / 16, DD = D * D, NT = 4 * D, LD = D + 4, V4 = D / 4;
+    constexpr int LOADS = kLrC * V4 / NT;  // 4 at every D
+    __shared__ __align__(16) float Ks[2][kLrC * LD], Us[2][kLrC * LD];  // k and v (self-generated values: k - v)
+    __shared__ float cs[2][kLrC], keep_chunk[2];
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, wr = 16 * wave, ml = lane & 15, kg = lane >> 4;
+    const size_t b = blockIdx.x % batch, tok0 = b * (size_t)s;  // the four memories of a chain share an XCD's L2
+    const int comp = 2 + blockIdx.x / batch;
+    float *mb = mems + (b * 6 + comp) * DD + (wr + ml) * D + 4 * kg;
+    f32x4 F[KT];
+#pragma unroll
+    for (int kt = 0; kt < KT; kt++) F[kt] = *reinterpret_cast<const f32x4 *>(mb + 16 * kt);
+
+    float4 nk[LOADS], nv[LOADS];
+    float nal = 0.f, nth = 0.f;
+    auto request = [&](int ci) {
+        const int t0 = ci * C, L = min(C, s - t0);
+#pragma unroll
+        for (int i = 0; i < LOADS; i++) {
+            const int e = tid + i * NT, li = e / V4, j = (e % V4) * 4;
+            const size_t o = (tok0 + t0 + li) * D + j;
+            nk[i] = li < L ? *reinterpret_cast<const float4 *>(k_cache + o) : make_float4(0, 0, 0, 0);
+            nv[i] = li < L ? *reinterpret_cast<const float4 *>(v_cache + o) : make_float4(0, 0, 0, 0);
+        }
+        if (wave == 0) {
+            nal = lane < L ? alpha_cache[tok0 + t0 + lane] : 0.f;
+            nth = lane < L ? theta_cache[tok0 + t0 + lane] : 0.f;
+        }
+    };
+    auto stage = [&](int buf) {
+#pragma unroll
+        for (int i = 0; i < LOADS; i++) {
+            const int e = tid + i * NT, li = e / V4, j = (e % V4) * 4;
+            *reinterpret_cast<float4 *>(&Ks[buf][li * LD + j]) = nk[i];
+            *reinterpret_cast<float4 *>(&Us[buf][li * LD + j]) =
+                SG ? make_float4(nk[i].x - nv[i].x, nk[i].y - nv[i].y, nk[i].z - nv[i].z, nk[i].w - nv[i].w) : nv[i];
+        }
+        if (wave == 0) {  // products of the retentions behind each token
+            float x = 1.f - nal;
+#pragma unroll
+            for (int off = 1; off < 64; off *= 2) {
+                const float y = __shfl_down(x, off, 64);
+                if (lane + off < 64) x *= y;
+            }
+            const float behind = __shfl_down(x, 1, 64);
+            cs[buf][lane] = nth * (lane < 63 ? behind : 1.f);
+            if (lane == 0) keep_chunk[buf] = x;
+        }
+    };
+    request(0);
+    stage(0);
+    __syncthreads();
+    for (int ci = 0; ci < nc; ci++) {
+        const int buf = ci & 1, L = min(C, s - ci * C);
+        if (ci + 1 < nc) request(ci + 1);
+        float *fb = frozen + ((b * nc + ci) * 6 + comp) * (size_t)DD + (wr + ml) * D + 4 * kg;
+#pragma unroll
+        for (int kt = 0; kt < KT; kt++) *reinterpret_cast<f32x4 *>(fb + 16 * kt) = F[kt];
+        const float *K = Ks[buf], *U = Us[buf];
+        f32x4 w[ST], N[KT];
+        const float keep = keep_chunk[buf];
+#pragma unroll
+        for (int kt = 0; kt < KT; kt++) N[kt] = F[kt] * keep;
+#pragma unroll
+        for (int st = 0; st < ST; st++) {
+            w[st] = f32x4{0.f, 0.f, 0.f, 0.f};
+            if (16 * st >= L) continue;
+#pragma unroll
+            for (int kt = 0; kt < KT; kt++) {
+                const f32x4 a = *reinterpret_cast<const f32x4 *>((SG ? U : K) + (16 * st + ml) * LD + 16 * kt + 4 * kg);
+#pragma unroll
+                for (int v = 0; v < 4; v++) w[st] = mfma4(a[v], F[kt][v], w[st]);
+            }
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int t = 16 * st + 4 * kg + v;
+                w[st][v] = cs[buf][t] * ((SG ? 0.f : U[t * LD + wr + ml]) - w[st][v]);
+            }
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+#pragma unroll
+                for (int kt = 0; kt < KT; kt++)
+                    N[kt] = mfma4(K[(16 * st + 4 * kg + v) * LD + 16 * kt + ml], w[st][v], N[kt]);
+            }
+        }
+#pragma unroll
+        for (int kt = 0; kt < KT; kt++) F[kt] = N[kt];
+        if (ci + 1 < nc) stage(buf ^ 1);
+        __syncthreads();
+    }
+#pragma unroll
+    for (int kt = 0; kt < KT; kt++) *reinterpret_cast<f32x4 *>(mb + 16 * kt) = F[kt];
+}
+
+// ── reads ────────────────────────────────────────────────────────────────────────────────────────────────────────
+// q_t = F_q (G_t x_t) + H_t x_t, y_t = F_mem (G_t q_t) + H_t q_t with the shared factors in their explicit form
+// (selfref_chunk.h).  A wave takes 16 tokens through both reads by itself: the scores with the earlier keys, masked and
+// scaled, are the operand of G and H at once; its rows change layout through its own 16 rows of LDS without a barrier.
+template <int D, bool SG>
+__global__ __launch_bounds__(4 * D) void selfref_read_kernel(
+    const float *__restrict__ emb, const float *__restrict__ k_cache, const float *__restrict__ v_cache,
+    const float *__restrict__ alpha_cache, const float *__restrict__ theta_cache, const float *__restrict__ frozen,
+    float *__restrict__ q_cache, float *__restrict__ y, int s, int C, int nc) {
+    constexpr int KT = D / 16, NW = D / 16, DD = D * D, KL = D + 4;
+    extern __shared__ __align__(16) float chunk_lds[];
+    const ChunkLds<D> m(chunk_lds);
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, ml = lane & 15, kg = lane >> 4;
+    float *row = m.tiles + wave * kTB * kWL;  // the wave's rows
+    const int ci = blockIdx.x % nc;
+    const size_t b = blockIdx.x / nc, chunk = blockIdx.x, tok0 = b * (size_t)s;
+    const int t0 = ci * C, L = min(C, s - t0);
+    chunk_setup<D, SG>(m, k_cache, v_cache, alpha_cache, theta_cache, tok0, t0, L, tid);
+    const float *UC = SG ? m.XC : m.KC;
+
+    for (int tile = wave; tile * kTB < L; tile += NW) {
+        const int li0 = tile * kTB, nt = min(kTB, L - li0);
+        const size_t o0 = (tok0 + t0 + li0) * D;
+        f32x4 a[KT], in[KT];  // the read's argument: as operand, and row 4 kg + v, column 16 jt + ml
+#pragma unroll
+        for (int kt = 0; kt < KT; kt++) {
+            a[kt] = ml < nt ? *reinterpret_cast<const f32x4 *>(emb + o0 + (size_t)ml * D + 16 * kt + 4 * kg)
+                            : f32x4{0.f, 0.f, 0.f, 0.f};
+            *reinterpret_cast<f32x4 *>(row + ml * kWL + 16 * kt + 4 * kg) = a[kt];
+        }
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int jt = 0; jt < KT; jt++) {
+#pragma unroll
+            for (int v = 0; v < 4; v++) in[jt][v] = row[(4 * kg + v) * kWL + 16 * jt + ml];
+        }
+#pragma unroll
+        for (int pass = 0; pass < 2; pass++) {
+            const float *Fp = frozen + (chunk * 6 + (pass ? 5 : 2)) * DD;
+            __builtin_amdgcn_wave_barrier();
+            for (int st = 0; st <= tile; st++) {
+                f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int kt = 0; kt < KT; kt++) {
+                    const f32x4 kk = *reinterpret_cast<const f32x4 *>(m.KC + (16 * st + ml) * KL + 16 * kt + 4 * kg);
+#pragma unroll
+                    for (int v = 0; v < 4; v++) acc = mfma4(a[kt][v], kk[v], acc);
+                }
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    const int tt = 4 * kg + v, li = li0 + tt, s1 = 16 * st + ml;
+                    row[tt * kWL + s1] = (tt < nt && s1 < li) ? m.CT[li * kLrC + s1] * acc[v] : 0.f;
+                }
+            }
+            __builtin_amdgcn_wave_barrier();
+            f32x4 g[KT], h[KT];
+#pragma unroll
+            for (int jt = 0; jt < KT; jt++) g[jt] = h[jt] = f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int st = 0; st <= tile; st++) {
+                const f32x4 w = *reinterpret_cast<const f32x4 *>(row + ml * kWL + 16 * st + 4 * kg);
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+#pragma unroll
+                    for (int jt = 0; jt < KT; jt++) {
+                        const int o = (16 * st + 4 * kg + v) * KL + 16 * jt + ml;
+                        g[jt] = mfma4(w[v], UC[o], g[jt]);
+                        if (!SG) h[jt] = mfma4(w[v], m.XC[o], h[jt]);
+                    }
+                }
+            }
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int jt = 0; jt < KT; jt++) {
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    const int tt = 4 * kg + v;
+                    row[tt * kWL + 16 * jt + ml] = tt < nt ? fmaf(m.cA[li0 + tt], in[jt][v], -g[jt][v]) : 0.f;
+                }
+            }
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int kt = 0; kt < KT; kt++) a[kt] = *reinterpret_cast<const f32x4 *>(row + ml * kWL + 16 * kt + 4 * kg);
+#pragma unroll
+            for (int jt = 0; jt < KT; jt++) {
+#pragma unroll
+                for (int kt = 0; kt < KT; kt++) {
+                    const f32x4 f = *reinterpret_cast<const f32x4 *>(Fp + (16 * jt + ml) * D + 16 * kt + 4 * kg);
+#pragma unroll
+                    for (int v = 0; v < 4; v++) h[jt] = mfma4(a[kt][v], f[v], h[jt]);
+                }
+                float *dst = pass ? y : q_cache;
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    in[jt][v] = h[jt][v];
+                    if (4 * kg + v < nt) dst[o0 + (size_t)(4 * kg + v) * D + 16 * jt + ml] = h[jt][v];
+                }
+            }
+            if (pass == 0) {  // q becomes the second read's argument
+                __builtin_amdgcn_wave_barrier();
+#pragma unroll
+                for (int jt = 0; jt < KT; jt++) {
+#pragma unroll
+                    for (int v = 0; v < 4; v++) row[(4 * kg + v) * kWL + 16 * jt + ml] = in[jt][v];
+                }
+                __builtin_amdgcn_wave_barrier();
+#pragma unroll
+                for (int kt = 0; kt < KT; kt++)
+                    a[kt] = *reinterpret_cast<const f32x4 *>(row + ml * kWL + 16 * kt + 4 * kg);
+            }
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
+}
+
+template <int D, bool SG>
+void launch(const SelfrefForward &a) {
+    const dim3 block(4 * D);
+    hipLaunchKernelGGL((selfref_chain_kernel<D, SG>), dim3(a.batch), block, 0, stream(), a.mems, a.emb, a.k, a.v, a.alpha,
+                       a.theta, a.amean, a.emean, a.frozen, a.s, a.C, a.nc);
+    check_launch("selfref_chain_kernel");
+    hipLaunchKernelGGL((selfref_scan_kernel<D, SG>), dim3(4 * a.batch), block, 0, stream(), a.mems, a.k, a.v, a.alpha,
+                       a.theta, a.frozen, a.s, a.C, a.nc, a.batch);
+    check_launch("selfref_scan_kernel");
+    const size_t lds = (chunk_lds_floats<D>(0) + D / 16 * kTB * kWL) * sizeof(float);
+    check_hip(hipFuncSetAttribute(reinterpret_cast<const void *>(selfref_read_kernel<D, SG>),
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds), "dynamic LDS size");
+    hipLaunchKernelGGL((selfref_read_kernel<D, SG>), dim3(a.batch * a.nc), block, lds, stream(), a.emb, a.k, a.v, a.alpha,
+                       a.theta, a.frozen, a.q, a.y, a.s, a.C, a.nc);
+    check_launch("selfref_read_kernel");
+}
+
+}  // namespace
+
+void selfref_forward_chain(const SelfrefForward &a) {
+    if (a.d == 16) a.sg ? launch<16, true>(a) : launch<16, false>(a);
+    else if (a.d == 32) a.sg ? launch<32, true>(a) : launch<32, false>(a);
+    else a.sg ? launch<64, true>(a) : launch<64, false>(a);
+}
+
+}  // namespace nlh

@@ -1,0 +1,104 @@
+// Tables of one chunk shared by the chunk-parallel kernels of the HOPE self-referential memory, its gate
+// functions and the entry of the chain-resident forward (selfref_chain.hip).
+#pragma once
+#include <hip/hip_runtime.h>
+
+namespace nlh {
+
+constexpr int kTB = 16;  // tokens staged in LDS at a time
+using f32x4 = float __attribute__((ext_vector_type(4)));
+
+// core/src/tensor.rs:202-207, 221-227.  The gates sit on the per-token critical path of the forward,
+// so exp, log and the reciprocal are the hardware approximations (v_exp_f32, v_log_f32, v_rcp_f32: about
+// one ulp each, three orders of magnitude inside the parity bar) instead of the library routines.
+__device__ __forceinline__ float sr_sigmoid(float x) {
+    if (x >= 15.f) return 1.f;
+    if (x <= -15.f) return 0.f;
+    return __builtin_amdgcn_rcpf(1.f + __expf(-x));
+}
+__device__ __forceinline__ float sr_softplus(float x) {
+    if (x >= 15.f) return x;
+    if (x <= -15.f) return 0.f;
+    return __logf(1.f + __expf(x));
+}
+
+// Chunks of up to kLrC tokens use the explicit form of the shared factors,
+//     G_t = A_t I - sum_{s<t} c_ts u_s k_s^T,   H_t = sum_{s<t} c_ts v_s k_s^T,
+//     A_t = prod_{r<t} (1-a_r),   c_ts = th_s prod_{s<r<t} (1-a_r),
+// so that no G_t, H_t is ever written to memory: products G_t^T y, H_t^T y of a
+// tile of tokens become two small LDS-resident matrix products, and the inner
+// product <G_t, dG_{t+1}> + <H_t, dH_{t+1}> the alpha gradient needs follows
+// from a scalar recurrence (see the reverse sweep).
+constexpr int kLrC = 64;
+
+constexpr int kWL = kLrC + 4;
+
+
+// LDS of the chunk-parallel kernels: the chunk's keys KC and u = k - v (or v) XC, rows of stride D + 4;
+// the table c_ts; one tile of products Wt; gates and the vectors c_L, A (kLrC + 1 entries).
+template <int D>
+struct ChunkLds {
+    static constexpr int KL = D + 4;
+    float *KC, *XC, *CT, *Wt, *cal, *cth, *cL, *cA, *tiles;
+    __device__ explicit ChunkLds(float *base) {
+        KC = base; XC = KC + kLrC * KL; CT = XC + kLrC * KL; Wt = CT + kLrC * kLrC;
+        cal = Wt + kTB * kWL; cth = cal + kLrC; cL = cth + kLrC; cA = cL + kLrC; tiles = cA + 2 * kLrC;
+    }
+};
+
+// Stages the chunk [t0, t0 + L) and builds its tables; ends with a barrier.
+template <int D, bool SG>
+__device__ __forceinline__ void chunk_setup(const ChunkLds<D> &m, const float *__restrict__ k_cache,
+                                            const float *__restrict__ v_cache, const float *__restrict__ alpha_cache,
+                                            const float *__restrict__ theta_cache, size_t tok0, int t0, int L, int tid) {
+    constexpr int NT = 4 * D, V4 = D / 4, KL = D + 4;
+    for (int e = tid; e < L * V4; e += NT) {
+        const int li = e / V4, j = (e % V4) * 4;
+        const size_t o = (tok0 + t0 + li) * D + j;
+        const float4 k4 = *reinterpret_cast<const float4 *>(k_cache + o);
+        const float4 v4 = *reinterpret_cast<const float4 *>(v_cache + o);
+        *reinterpret_cast<float4 *>(m.KC + li * KL + j) = k4;
+        *reinterpret_cast<float4 *>(m.XC + li * KL + j) =
+            SG ? make_float4(k4.x - v4.x, k4.y - v4.y, k4.z - v4.z, k4.w - v4.w) : v4;
+    }
+    // rows behind a short chunk's last token enter the products of lowrank_tile times zero
+    for (int e = L * KL + tid; e < kLrC * KL; e += NT) { m.KC[e] = 0.f; m.XC[e] = 0.f; }
+    for (int e = tid; e < L; e += NT) { m.cal[e] = alpha_cache[tok0 + t0 + e]; m.cth[e] = theta_cache[tok0 + t0 + e]; }
+    __syncthreads();
+    if (tid < 64) {
+        // lane t-1 builds row t of c (row L is c_L) from its diagonal leftwards:
+        // c_{t,s} = th_s P, P = prod_{s<r<t} (1-a_r); P ends as A_t.  s runs in lock step
+        // over the wave, so the gate reads are broadcasts that do not depend on the products.
+        const int t = tid + 1;
+        float P = 1.f;
+#pragma unroll 8
+        for (int s1 = kLrC - 1; s1 >= 0; s1--) {
+            const float th_s = s1 < L ? m.cth[s1] : 0.f, keep_s = s1 < L ? 1.f - m.cal[s1] : 1.f;
+            if (s1 < t && t <= L) {
+                if (t < L) m.CT[t * kLrC + s1] = th_s * P;
+                else m.cL[s1] = th_s * P;
+                P *= keep_s;
+            }
+        }
+        if (t <= L) m.cA[t] = P;
+        if (t > L) m.cL[tid] = 0.f;  // c_Ls behind the chunk's last token (tid >= L)
+        if (tid == 0) m.cA[0] = 1.f;
+    }
+    __syncthreads();
+}
+
+template <int D>
+constexpr int chunk_lds_floats(int tiles) { return 2 * kLrC * (D + 4) + kLrC * kLrC + kTB * kWL + 5 * kLrC + tiles * kTB * (D + 4); }
+
+// Forward for chunks of up to kLrC tokens at head sizes 16, 32 and 64; arguments as in
+// selfref_chunkwise_forward_f32_rocm, nc chunks of C tokens.  Takes no scratch memory.
+struct SelfrefForward {
+    float *mems;
+    const float *emb;
+    float *y, *k, *v, *q, *alpha, *theta, *amean, *emean, *frozen;
+    int s, d, batch, C, nc;
+    bool sg;
+};
+void selfref_forward_chain(const SelfrefForward &a);
+
+}  // namespace nlh
