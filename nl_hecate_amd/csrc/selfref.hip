@@ -296,11 +296,11 @@ __device__ __forceinline__ void lowrank_tile(const float *a1, const float *L1, c
 }
 
 // Chunk-parallel first pass of the backward (chunks of up to kLrC tokens): one workgroup per
-// (chain, chunk).  Per token g = G x, p = G q, dp = F_mem^T dy, dq = G^T dp + H^T dy (and H x, H q
-// without self-generated values) into rp [B, s, RS, D]; per chunk the transposed F_k, F_v, F_q
+// (chain, chunk), without self-generated values (with them: selfref_sweep.hip).  Per token g = G x, p = G q,
+// dp = F_mem^T dy, dq = G^T dp + H^T dy, H x, H q into rp [B, s, RS, D]; per chunk the transposed F_k, F_v, F_q
 // (ftt [B, nc, 3, D, D]), the column sums of F_eta, F_alpha (csv [B, nc, 2, D]) and G_L, H_L
 // (gl, hl [B, nc, D, D]; not for a chain's last chunk, whose boundary carries no gradient).
-template <int D, bool SG>
+template <int D>
 __global__ __launch_bounds__(4 * D) void selfref_bwd_chunks_kernel(
     const float *__restrict__ emb, const float *__restrict__ d_y, const float *__restrict__ k_cache,
     const float *__restrict__ v_cache, const float *__restrict__ q_cache,
@@ -308,7 +308,7 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_chunks_kernel(
     const float *__restrict__ frozen, float *__restrict__ rp, float *__restrict__ ftt, float *__restrict__ csv,
     float *__restrict__ gl, float *__restrict__ hl, int s, int C, int nc) {
     constexpr int NT = 4 * D, DD = D * D, V4 = D / 4, TL = D + 4, KL = D + 4, JT = D / 16, FL = D + 1;
-    constexpr int RS = SG ? 4 : 6;
+    constexpr int RS = 6;
     extern __shared__ __align__(16) float chunk_lds[];
     const ChunkLds<D> m(chunk_lds);
     float *tX = m.tiles, *tQ = tX + kTB * TL, *tDY = tQ + kTB * TL, *tDP = tDY + kTB * TL;
@@ -348,7 +348,7 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_chunks_kernel(
         }
         __syncthreads();
     }
-    chunk_setup<D, SG>(m, k_cache, v_cache, alpha_cache, theta_cache, tok0, t0, L, tid);
+    chunk_setup<D, false>(m, k_cache, v_cache, alpha_cache, theta_cache, tok0, t0, L, tid);
 
     const float *Fm = fz + 5 * DD;
     const int stt = tid / V4, sj = (tid % V4) * 4;
@@ -377,15 +377,15 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_chunks_kernel(
             }
         }
         // g = G x, p = G q
-        lowrank_tile<D, true, false>(tX, m.KC, nullptr, nullptr, SG ? m.XC : m.KC, li0, nt, m.CT, m.cA, m.Wt, rp_t,
+        lowrank_tile<D, true, false>(tX, m.KC, nullptr, nullptr, m.KC, li0, nt, m.CT, m.cA, m.Wt, rp_t,
                                      (size_t)RS * D, tid);
         __syncthreads();
-        lowrank_tile<D, true, false>(tQ, m.KC, nullptr, nullptr, SG ? m.XC : m.KC, li0, nt, m.CT, m.cA, m.Wt,
+        lowrank_tile<D, true, false>(tQ, m.KC, nullptr, nullptr, m.KC, li0, nt, m.CT, m.cA, m.Wt,
                                      rp_t + D, (size_t)RS * D, tid);
         __syncthreads();
-        lowrank_tile<D, true, !SG>(tDP, SG ? m.XC : m.KC, tDY, m.XC, m.KC, li0, nt, m.CT, m.cA, m.Wt, rp_t + 2 * D,
+        lowrank_tile<D, true, true>(tDP, m.KC, tDY, m.XC, m.KC, li0, nt, m.CT, m.cA, m.Wt, rp_t + 2 * D,
                                    (size_t)RS * D, tid);
-        if (!SG) {  // H x and H q for the scalar recurrence of the reverse sweep
+        {  // H x and H q for the scalar recurrence of the reverse sweep
             __syncthreads();
             lowrank_tile<D, false, true>(nullptr, nullptr, tX, m.KC, m.XC, li0, nt, m.CT, m.cA, m.Wt, rp_t + 4 * D,
                                          (size_t)RS * D, tid);
@@ -399,16 +399,16 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_chunks_kernel(
         f32x4 g_acc[JT], h_acc[JT];
 #pragma unroll
         for (int jt = 0; jt < JT; jt++) g_acc[jt] = h_acc[jt] = f32x4{0.f, 0.f, 0.f, 0.f};
-        const float *UC = SG ? m.XC : m.KC;
+        const float *UC = m.KC;
         const int kend = (L + 3) & ~3;
         for (int k0 = 0; k0 < kend; k0 += 4) {
             const float cl = m.cL[k0 + kg];
-            const float au = UC[(k0 + kg) * KL + wr + ml] * cl, avv = SG ? 0.f : m.XC[(k0 + kg) * KL + wr + ml] * cl;
+            const float au = UC[(k0 + kg) * KL + wr + ml] * cl, avv = m.XC[(k0 + kg) * KL + wr + ml] * cl;
 #pragma unroll
             for (int jt = 0; jt < JT; jt++) {
                 const float kb = m.KC[(k0 + kg) * KL + 16 * jt + ml];
                 g_acc[jt] = __builtin_amdgcn_mfma_f32_16x16x4f32(au, kb, g_acc[jt], 0, 0, 0);
-                if (!SG) h_acc[jt] = __builtin_amdgcn_mfma_f32_16x16x4f32(avv, kb, h_acc[jt], 0, 0, 0);
+                h_acc[jt] = __builtin_amdgcn_mfma_f32_16x16x4f32(avv, kb, h_acc[jt], 0, 0, 0);
             }
         }
         const float aL = m.cA[L];
@@ -418,7 +418,7 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_chunks_kernel(
             for (int v = 0; v < 4; v++) {
                 const int row = wr + 4 * kg + v, col = 16 * jt + ml;
                 gl[chunk * DD + row * D + col] = (row == col ? aL : 0.f) - g_acc[jt][v];
-                if (!SG) hl[chunk * DD + row * D + col] = h_acc[jt][v];
+                hl[chunk * DD + row * D + col] = h_acc[jt][v];
             }
         }
     }
@@ -1068,13 +1068,17 @@ void launch_bwd_sg(const BwdArgs &a) {
                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes), "dynamic LDS size");
     };
     if (a.lowrank) {
-        const size_t lds1 = chunk_lds_floats<D>(4) * sizeof(float), lds3 = chunk_lds_floats<D>(2) * sizeof(float);
-        set_lds(selfref_bwd_chunks_kernel<D, SG>, lds1);
-        hipLaunchKernelGGL((selfref_bwd_chunks_kernel<D, SG>), dim3(a.batch * a.nc), block, lds1, stream(), a.emb,
-                           a.dy, a.kc, a.vc, a.qc, a.al, a.th, a.frozen, a.rp, a.ftt, a.csv, a.gtraj, a.htraj, a.s,
-                           a.C, a.nc);
-        check_launch("selfref_bwd_chunks_kernel");
-        {
+        const size_t lds3 = chunk_lds_floats<D>(2) * sizeof(float);
+        if constexpr (SG) {
+            selfref_backward_sweep({a.emb, a.dy, a.kc, a.vc, a.qc, a.al, a.th, a.am, a.em, a.frozen, a.d_emb, a.d_mems,
+                                    a.gtraj, a.rp, a.ftt, a.csv, a.s, D, a.batch, a.C, a.nc});
+        } else {
+            const size_t lds1 = chunk_lds_floats<D>(4) * sizeof(float);
+            set_lds(selfref_bwd_chunks_kernel<D>, lds1);
+            hipLaunchKernelGGL((selfref_bwd_chunks_kernel<D>), dim3(a.batch * a.nc), block, lds1, stream(), a.emb,
+                               a.dy, a.kc, a.vc, a.qc, a.al, a.th, a.frozen, a.rp, a.ftt, a.csv, a.gtraj, a.htraj,
+                               a.s, a.C, a.nc);
+            check_launch("selfref_bwd_chunks_kernel");
             KernelTimer kt("selfref_bwd_kernel");
             hipLaunchKernelGGL((selfref_bwd_kernel<D, SG, true>), dim3(a.batch), block, 0, stream(), a.emb, a.dy,
                                a.kc, a.vc, a.qc, a.al, a.th, a.am, a.em, a.frozen, a.d_emb, a.d_mems, a.gtraj,
@@ -1177,9 +1181,10 @@ extern "C" void selfref_chunkwise_backward_f32_rocm(const float *embedded, const
     a.batch = batch_size; a.s = seq_len; a.C = C; a.nc = nc; a.sg = sg; a.lowrank = lowrank;
     a.gtraj = scratch(0, lowrank ? chunks * dd * sizeof(float) : traj_bytes);
     a.htraj = sg ? nullptr : scratch(1, lowrank ? chunks * dd * sizeof(float) : traj_bytes);
-    a.rp = scratch(2, tokens * ((lowrank && !sg) ? 6 : 4) * d * sizeof(float));
+    // with self-generated values on the low-rank path rp and ftt are the tokens' and the chunks' part of selfref_sweep.hip
+    a.rp = scratch(2, tokens * (lowrank ? (sg ? sweep_token_floats(d) : 6 * d) : 4 * d) * sizeof(float));
     if (lowrank) {
-        a.ftt = scratch(3, chunks * 3 * dd * sizeof(float));
+        a.ftt = scratch(3, chunks * (sg ? 4 : 3) * dd * sizeof(float));
         a.csv = scratch(4, chunks * 2 * d * sizeof(float));
         a.dh = sg ? nullptr : scratch(5, tokens * d * sizeof(float));
     }

@@ -46,8 +46,9 @@ struct ChunkLds {
     }
 };
 
-// Stages the chunk [t0, t0 + L) and builds its tables; ends with a barrier.
-template <int D, bool SG>
+// Stages the chunk [t0, t0 + L) and builds its tables; ends with a barrier.  Without THETA the table holds
+// prod_{s<r<t} (1-a_r) alone.
+template <int D, bool SG, bool THETA = true>
 __device__ __forceinline__ void chunk_setup(const ChunkLds<D> &m, const float *__restrict__ k_cache,
                                             const float *__restrict__ v_cache, const float *__restrict__ alpha_cache,
                                             const float *__restrict__ theta_cache, size_t tok0, int t0, int L, int tid) {
@@ -75,7 +76,7 @@ __device__ __forceinline__ void chunk_setup(const ChunkLds<D> &m, const float *_
         for (int s1 = kLrC - 1; s1 >= 0; s1--) {
             const float th_s = s1 < L ? m.cth[s1] : 0.f, keep_s = s1 < L ? 1.f - m.cal[s1] : 1.f;
             if (s1 < t && t <= L) {
-                if (t < L) m.CT[t * kLrC + s1] = th_s * P;
+                if (t < L) m.CT[t * kLrC + s1] = THETA ? th_s * P : P;
                 else m.cL[s1] = th_s * P;
                 P *= keep_s;
             }
@@ -100,5 +101,16 @@ struct SelfrefForward {
     bool sg;
 };
 void selfref_forward_chain(const SelfrefForward &a);
+
+// Backward under self-generated values for the same chunks and head sizes, up to dg (in d_emb) and d_mems; the last
+// pass, d_x = G^T dg, is the caller's.  gl: [chunks, d, d] scratch; tok: [tokens, 3 d + 16 + 2]; outer: [chunks, 4, d, d];
+// csv: [chunks, 2, d].
+struct SelfrefSweep {
+    const float *emb, *d_y, *k, *v, *q, *alpha, *theta, *amean, *emean, *frozen;
+    float *d_emb, *d_mems, *gl, *tok, *outer, *csv;
+    int s, d, batch, C, nc;
+};
+constexpr int sweep_token_floats(int d) { return 3 * d + 16 + 2; }
+void selfref_backward_sweep(const SelfrefSweep &a);
 
 }  // namespace nlh

@@ -1,0 +1,813 @@
+// HOPE self-referential memory with self-generated values: the backward for chunks of up to 64 tokens.
+//
+// Inside a chunk (G, dG as in selfref.hip; W_t = dG_{t+1} k_t, Z_t = dG_{t+1}^T u_t, u = k - v)
+//     dk_t = -th_t (Z_t + W_t),  dv_t = th_t W_t,  dth_t = -u_t . W_t,
+//     dg_t = F_k^T dk_t + F_v^T dv_t + F_q^T dq_t + de_t csE + da_t csA,   dG_t = (1-a_t) dG_{t+1} + dg_t x_t^T + dp_t q_t^T.
+// The part of dG that dp q^T drives depends on nothing the sweep produces, so its W, Z, and with them a first part of
+// dk, dv, dth and dg, come from selfref_bwd_prepare_kernel (one workgroup per chunk, the whole chip), as do the outer
+// products of those parts that make up dF.  What is left for selfref_bwd_sweep_kernel (one workgroup per chain) is the
+// part that dg x^T and the chunk boundary drive, carried as Y_s = F_k^T Z_s + (F_k - F_v)^T W_s:
+//     Y_s <- (1-a_t) Y_s + (F_k^T x_t) (dg_t . u_s) + ((F_k - F_v)^T dg_t) (x_t . k_s)      for the earlier tokens s of a tile
+//     dg_s = dg0_s - th_s Y_s + de_s csE + da_s csA
+// so that a token takes one exchange (dg_t), one product with a matrix and the dots of dg_t with the tile's u_s.
+#include <hip/hip_runtime.h>
+
+#include <utility>
+
+#include "../../include/nl_hecate_ffi.h"
+#include "lane_ops.h"
+#include "quad_rows.h"
+#include "runtime.h"
+#include "selfref_chunk.h"
+
+namespace nlh {
+namespace {
+
+__device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ float lane_from(int byte_addr, float x) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(byte_addr, __builtin_bit_cast(int, x)));
+}
+__device__ __forceinline__ float lane_value(float x, int lane) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), lane));
+}
+__host__ __device__ constexpr int sigma(int t) { return 4 * (t & 3) + (t >> 2); }
+constexpr f32x4 kZero = {0.f, 0.f, 0.f, 0.f};
+
+// Sum over the 16 lanes of a DPP row.
+__device__ __forceinline__ float row_sum(float x) { return group_allreduce<16>(x); }
+
+// ── what does not depend on the sweep ────────────────────────────────────────────────────────────────────────────
+// LDS: the chunk's k and u, the table of retentions, the masked scores of q with the earlier k and of dp with the
+// earlier u (negative), dp, and 16 rows of every wave's own for changes of layout.  The first five make room for
+// q, then for dk0, dv0, dq, g, p as the operands of the outer products.
+template <int D>
+struct PrepareLds {
+    static constexpr int KL = D + 4, NW = D / 16;
+    static constexpr int wq = 0, wd = wq + kLrC * kWL, dp = wd + kLrC * kWL, rows = dp + kLrC * KL,
+                         floats = rows + NW * kTB * kWL;
+};
+
+template <int D>
+__global__ __launch_bounds__(4 * D) void selfref_bwd_prepare_kernel(
+    const float *__restrict__ emb, const float *__restrict__ d_y, const float *__restrict__ k_cache,
+    const float *__restrict__ v_cache, const float *__restrict__ q_cache, const float *__restrict__ alpha_cache,
+    const float *__restrict__ theta_cache, const float *__restrict__ frozen, float *__restrict__ gl,
+    float *__restrict__ tok, float *__restrict__ outer, float *__restrict__ csv, int s, int C, int nc) {
+    constexpr int KT = D / 16, NW = D / 16, NT = 4 * D, DD = D * D, KL = D + 4, V4 = D / 4, TPW = 4 / NW;
+    constexpr int TF = sweep_token_floats(D);
+    using P = PrepareLds<D>;
+    extern __shared__ __align__(16) float lds[];
+    const ChunkLds<D> m(lds);
+    float *Wq = m.tiles + P::wq, *Wd = m.tiles + P::wd, *DP = m.tiles + P::dp;
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, ml = lane & 15, kg = lane >> 4, wr = 16 * wave;
+    float *row = m.tiles + P::rows + wave * kTB * kWL;
+    const int ci = blockIdx.x % nc;
+    const size_t b = blockIdx.x / nc, chunk = blockIdx.x, tok0 = b * (size_t)s;
+    const int t0 = ci * C, L = min(C, s - t0), ntile = (L + kTB - 1) / kTB;
+    const float *fz = frozen + chunk * 6 * DD;
+
+    for (int e = tid; e < 2 * D; e += NT) {  // column sums of F_eta, F_alpha
+        const float *src = fz + (size_t)(3 + e / D) * DD + (e % D);
+        float a = 0.f;
+#pragma unroll 8
+        for (int c = 0; c < D; c++) a += src[c * D];
+        csv[chunk * 2 * D + e] = a;
+    }
+    // scores that no token of the chunk has, and rows behind its last token, enter products times zero
+    for (int e = tid; e < 2 * kLrC * kWL + kLrC * KL; e += NT) Wq[e] = 0.f;
+    chunk_setup<D, true, false>(m, k_cache, v_cache, alpha_cache, theta_cache, tok0, t0, L, tid);
+    for (int e = L + tid; e < kLrC; e += NT) m.cth[e] = 0.f;
+    __syncthreads();
+
+    // a wave's rows: 16 tokens as operand rows (token ml, dims 16 kt + 4 kg + v) or as results (token 4 kg + v, dim
+    // 16 jt + ml)
+    auto put = [&](const f32x4(&x)[KT]) {
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int jt = 0; jt < KT; jt++) {
+#pragma unroll
+            for (int v = 0; v < 4; v++) row[(4 * kg + v) * kWL + 16 * jt + ml] = x[jt][v];
+        }
+        __builtin_amdgcn_wave_barrier();
+    };
+    auto as_operand = [&](f32x4(&a)[KT]) {
+#pragma unroll
+        for (int kt = 0; kt < KT; kt++) a[kt] = *reinterpret_cast<const f32x4 *>(row + ml * kWL + 16 * kt + 4 * kg);
+    };
+
+    f32x4 g[TPW][KT], p[TPW][KT], dq[TPW][KT];
+#pragma unroll
+    for (int i = 0; i < TPW; i++) {
+        const int tile = wave + i * NW, li0 = tile * kTB, nt = min(kTB, L - li0);
+#pragma unroll
+        for (int jt = 0; jt < KT; jt++) g[i][jt] = p[i][jt] = dq[i][jt] = kZero;
+        if (tile >= ntile) continue;
+        const size_t tk = tok0 + t0 + li0;
+        auto load = [&](const float *src, f32x4(&a)[KT]) {
+#pragma unroll
+            for (int kt = 0; kt < KT; kt++)
+                a[kt] = ml < nt ? *reinterpret_cast<const f32x4 *>(src + (tk + ml) * D + 16 * kt + 4 * kg) : kZero;
+        };
+        // out = A x - sum_s th_s c_ts (x_t . L_s) R_s; the scores without th go to sc (negative with NEG)
+        auto low_rank = [&](const f32x4(&a)[KT], const float *Lr, const float *R, float *sc, float sign, float *gam,
+                            f32x4(&out)[KT]) {
+            for (int st = 0; st <= tile; st++) {
+                f32x4 acc = kZero;
+#pragma unroll
+                for (int kt = 0; kt < KT; kt++) {
+                    const f32x4 l = *reinterpret_cast<const f32x4 *>(Lr + (16 * st + ml) * KL + 16 * kt + 4 * kg);
+#pragma unroll
+                    for (int v = 0; v < 4; v++) acc = mfma4(a[kt][v], l[v], acc);
+                }
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    const int tt = 4 * kg + v, li = li0 + tt, s1 = 16 * st + ml;
+                    const bool on = tt < nt && s1 < li;
+                    sc[tt * kWL + s1] = on ? sign * m.CT[li * kLrC + s1] * acc[v] : 0.f;
+                    // x_t . k_s of the tile's own tokens, in the order sigma
+                    if (gam && st == tile && tt < nt) gam[(size_t)tt * TF + sigma(ml)] = on ? acc[v] : 0.f;
+                }
+            }
+            __builtin_amdgcn_wave_barrier();
+            f32x4 acc[KT];
+#pragma unroll
+            for (int jt = 0; jt < KT; jt++) acc[jt] = kZero;
+            for (int st = 0; st <= tile; st++) {
+                const f32x4 w = *reinterpret_cast<const f32x4 *>(sc + ml * kWL + 16 * st + 4 * kg);
+                const f32x4 th = *reinterpret_cast<const f32x4 *>(m.cth + 16 * st + 4 * kg);
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+#pragma unroll
+                    for (int jt = 0; jt < KT; jt++)
+                        acc[jt] = mfma4(sign * w[v] * th[v], R[(16 * st + 4 * kg + v) * KL + 16 * jt + ml], acc[jt]);
+                }
+            }
+#pragma unroll
+            for (int jt = 0; jt < KT; jt++) {
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    const int tt = 4 * kg + v;
+                    out[jt][v] = tt < nt ? fmaf(m.cA[li0 + tt], out[jt][v], -acc[jt][v]) : 0.f;
+                }
+            }
+            __builtin_amdgcn_wave_barrier();
+        };
+        auto as_result = [&](const f32x4(&a)[KT], f32x4(&x)[KT]) {
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int kt = 0; kt < KT; kt++) *reinterpret_cast<f32x4 *>(row + ml * kWL + 16 * kt + 4 * kg) = a[kt];
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int jt = 0; jt < KT; jt++) {
+#pragma unroll
+                for (int v = 0; v < 4; v++) x[jt][v] = row[(4 * kg + v) * kWL + 16 * jt + ml];
+            }
+            __builtin_amdgcn_wave_barrier();
+        };
+        f32x4 a[KT];
+        float *out = tok + tk * TF;
+        load(emb, a);  // g = G x
+        as_result(a, g[i]);
+        low_rank(a, m.KC, m.XC, row, 1.f, out + 3 * D, g[i]);
+        load(q_cache, a);  // p = G q
+        as_result(a, p[i]);
+        low_rank(a, m.KC, m.XC, Wq + li0 * kWL, 1.f, nullptr, p[i]);
+        load(d_y, a);  // dp = F_mem^T dy, dq = G^T dp
+        f32x4 dp[KT];
+#pragma unroll
+        for (int jt = 0; jt < KT; jt++) {
+            dp[jt] = kZero;
+#pragma unroll
+            for (int kt = 0; kt < KT; kt++) {
+#pragma unroll
+                for (int v = 0; v < 4; v++)
+                    dp[jt] = mfma4(a[kt][v], fz[5 * DD + (16 * kt + 4 * kg + v) * D + 16 * jt + ml], dp[jt]);
+            }
+        }
+        float pp[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int jt = 0; jt < KT; jt++) {
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                DP[(li0 + 4 * kg + v) * KL + 16 * jt + ml] = dp[jt][v];
+                pp[v] = fmaf(dp[jt][v], p[i][jt][v], pp[v]);
+            }
+        }
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            pp[v] = row_sum(pp[v]);
+            if (ml == 0 && 4 * kg + v < nt) out[(size_t)(4 * kg + v) * TF + 3 * D + 17] = pp[v];
+        }
+        put(dp);
+        as_operand(a);
+#pragma unroll
+        for (int jt = 0; jt < KT; jt++) dq[i][jt] = dp[jt];
+        low_rank(a, m.XC, m.KC, Wd + li0 * kWL, -1.f, nullptr, dq[i]);
+#pragma unroll
+        for (int jt = 0; jt < KT; jt++) {
+#pragma unroll
+            for (int v = 0; v < 4; v++)
+                if (4 * kg + v < nt) out[(size_t)(4 * kg + v) * TF + 16 * jt + ml] = g[i][jt][v];
+        }
+    }
+    if (ci < nc - 1) {  // G_L = A_L I - sum_s c_Ls u_s k_s^T; wave w takes rows 16 w ..
+        f32x4 acc[KT];
+#pragma unroll
+        for (int jt = 0; jt < KT; jt++) acc[jt] = kZero;
+        const int kend = (L + 3) & ~3;
+        for (int k0 = 0; k0 < kend; k0 += 4) {
+            const float au = m.XC[(k0 + kg) * KL + wr + ml] * m.cL[k0 + kg];
+#pragma unroll
+            for (int jt = 0; jt < KT; jt++) acc[jt] = mfma4(au, m.KC[(k0 + kg) * KL + 16 * jt + ml], acc[jt]);
+        }
+        const float aL = m.cA[L];
+#pragma unroll
+        for (int jt = 0; jt < KT; jt++) {
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int r = wr + 4 * kg + v, c = 16 * jt + ml;
+                gl[chunk * DD + r * D + c] = (r == c ? aL : 0.f) - acc[jt][v];
+            }
+        }
+    }
+    __syncthreads();
+    float *Q = m.KC;
+    for (int e = tid; e < L * V4; e += NT) {
+        const int li = e / V4, j = (e % V4) * 4;
+        *reinterpret_cast<float4 *>(Q + li * KL + j) =
+            *reinterpret_cast<const float4 *>(q_cache + (tok0 + t0 + li) * D + j);
+    }
+    __syncthreads();
+    f32x4 dk[TPW][KT], dv[TPW][KT];
+#pragma unroll
+    for (int i = 0; i < TPW; i++) {
+        const int tile = wave + i * NW, li0 = tile * kTB, nt = min(kTB, L - li0);
+#pragma unroll
+        for (int jt = 0; jt < KT; jt++) dk[i][jt] = dv[i][jt] = kZero;
+        if (tile >= ntile) continue;
+        const size_t tk = tok0 + t0 + li0;
+        float *out = tok + tk * TF;
+        // W_s = sum_t c_ts (q_t . k_s) dp_t, -Z_s = -sum_t c_ts (dp_t . u_s) q_t over the later tokens
+        for (int st = tile; st < ntile; st++) {
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int t = 16 * st + 4 * kg + v;
+                const float wq = Wq[t * kWL + li0 + ml], wd = Wd[t * kWL + li0 + ml];
+#pragma unroll
+                for (int jt = 0; jt < KT; jt++) {
+                    dv[i][jt] = mfma4(wq, DP[t * KL + 16 * jt + ml], dv[i][jt]);
+                    dk[i][jt] = mfma4(wd, Q[t * KL + 16 * jt + ml], dk[i][jt]);
+                }
+            }
+        }
+        float uw[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int jt = 0; jt < KT; jt++) {
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int li = li0 + 4 * kg + v;
+                uw[v] = fmaf(m.XC[li * KL + 16 * jt + ml], dv[i][jt][v], uw[v]);
+                const float th = m.cth[li];
+                dk[i][jt][v] = th * (dk[i][jt][v] - dv[i][jt][v]);
+                dv[i][jt][v] *= th;
+            }
+        }
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            uw[v] = row_sum(uw[v]);
+            if (ml == 0 && 4 * kg + v < nt) out[(size_t)(4 * kg + v) * TF + 3 * D + 16] = -uw[v];
+        }
+        // dg0 = F_k^T dk + F_v^T dv + F_q^T dq, and F_k^T x
+        f32x4 dg[KT], fx[KT], ak[KT], av[KT], aq[KT], ax[KT];
+        put(dk[i]);
+        as_operand(ak);
+        put(dv[i]);
+        as_operand(av);
+        put(dq[i]);
+        as_operand(aq);
+#pragma unroll
+        for (int kt = 0; kt < KT; kt++)
+            ax[kt] = ml < nt ? *reinterpret_cast<const f32x4 *>(emb + (tk + ml) * D + 16 * kt + 4 * kg) : kZero;
+#pragma unroll
+        for (int jt = 0; jt < KT; jt++) {
+            dg[jt] = fx[jt] = kZero;
+#pragma unroll
+            for (int kt = 0; kt < KT; kt++) {
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    const float *f = fz + (16 * kt + 4 * kg + v) * D + 16 * jt + ml;
+                    dg[jt] = mfma4(ak[kt][v], f[0], dg[jt]);
+                    fx[jt] = mfma4(ax[kt][v], f[0], fx[jt]);
+                    dg[jt] = mfma4(av[kt][v], f[DD], dg[jt]);
+                    dg[jt] = mfma4(aq[kt][v], f[2 * DD], dg[jt]);
+                }
+            }
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                if (4 * kg + v < nt) {
+                    float *o = out + (size_t)(4 * kg + v) * TF + 16 * jt + ml;
+                    o[D] = dg[jt][v];
+                    o[2 * D] = fx[jt][v];
+                }
+            }
+        }
+    }
+    // outer products: dF_k, dF_v, dF_q with g, dF_mem with p; stored as the sweep's lanes hold them
+    __syncthreads();
+    float *Es = lds;  // dk, dv, dq, g, p: rows of stride KL, in front of the waves' own rows
+#pragma unroll
+    for (int i = 0; i < TPW; i++) {
+        const int li0 = (wave + i * NW) * kTB;
+#pragma unroll
+        for (int jt = 0; jt < KT; jt++) {
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                float *e = Es + (li0 + 4 * kg + v) * KL + 16 * jt + ml;
+                e[0] = dk[i][jt][v];
+                e[kLrC * KL] = dv[i][jt][v];
+                e[2 * kLrC * KL] = dq[i][jt][v];
+                e[3 * kLrC * KL] = g[i][jt][v];
+                e[4 * kLrC * KL] = p[i][jt][v];
+            }
+        }
+    }
+    __syncthreads();
+    f32x4 o[4][KT];
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+#pragma unroll
+        for (int jt = 0; jt < KT; jt++) o[c][jt] = kZero;
+    }
+    for (int k0 = 0; k0 < 16 * ntile; k0 += 4) {
+        const int li = k0 + kg;
+        const float *e = Es + li * KL;
+        const float ak = e[wr + ml], av = e[kLrC * KL + wr + ml], aq = e[2 * kLrC * KL + wr + ml];
+        const float ay = li < L ? d_y[(tok0 + t0 + li) * D + wr + ml] : 0.f;
+#pragma unroll
+        for (int jt = 0; jt < KT; jt++) {
+            const float bg = e[3 * kLrC * KL + 16 * jt + ml], bp = e[4 * kLrC * KL + 16 * jt + ml];
+            o[0][jt] = mfma4(ak, bg, o[0][jt]);
+            o[1][jt] = mfma4(av, bg, o[1][jt]);
+            o[2][jt] = mfma4(aq, bg, o[2][jt]);
+            o[3][jt] = mfma4(ay, bp, o[3][jt]);
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+#pragma unroll
+        for (int jt = 0; jt < KT; jt++)
+            *reinterpret_cast<f32x4 *>(outer + (chunk * 4 + c) * DD + ((size_t)(wave * KT + jt) * 64 + lane) * 4) = o[c][jt];
+    }
+}
+
+// ── the sweep ────────────────────────────────────────────────────────────────────────────────────────────────────
+// f(15), f(14), ... f(0) with the argument as a type
+template <class Fn, int... I>
+__device__ __forceinline__ void downwards(Fn &f, std::integer_sequence<int, I...>) {
+    (f(std::integral_constant<int, kTB - 1 - I>{}), ...);
+}
+
+// acc + sum_i m[i] x_i with x spread over the DPP rows: lane i of row kg holds x_i for the row's lanes.
+template <int N, int I = 0>
+__device__ __forceinline__ float dot_spread(const float (&m)[N], float x, float acc) {
+    if constexpr (I == N) return acc;
+    else return dot_spread<N, I + 1>(m, x, fmaf(dpp_mov<0x150 + I>(x), m[I], acc));  // row_newbcast: lane I of the row
+}
+
+// Sums over the four DPP rows of three values at once, every lane receives them.
+__device__ __forceinline__ void across_rows3(float &a, float &b, float &c) {
+    float a1 = a, b1 = b, c1 = c;
+    asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\tv_permlane32_swap_b32 %2, %3\n\tv_permlane32_swap_b32 %4, %5"
+                 : "+v"(a), "+v"(a1), "+v"(b), "+v"(b1), "+v"(c), "+v"(c1));
+    a += a1; b += b1; c += c1;
+    a1 = a; b1 = b; c1 = c;
+    asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\tv_permlane16_swap_b32 %2, %3\n\tv_permlane16_swap_b32 %4, %5"
+                 : "+v"(a), "+v"(a1), "+v"(b), "+v"(b1), "+v"(c), "+v"(c1));
+    a += a1; b += b1; c += c1;
+}
+
+// One workgroup per chain, a wave per 16 rows.  Lane (ml, kg) = (lane % 16, lane / 16) holds of every matrix row ml of
+// the wave's rows, columns CP kg + i (CP = D / 4): operand and result of the tile products (the contraction index runs
+// over (i, kg)), and the coefficients of a product with a vector whose element CP kg + i is broadcast from lane i of
+// DPP row kg.  dG is kept a second time by columns (dGT).  Tokens of a tile are result rows in the order sigma, so that
+// lane kg owns the columns s = 4 v + kg of Y.
+template <int D>
+__global__ __launch_bounds__(4 * D) void selfref_bwd_sweep_kernel(
+    const float *__restrict__ emb, const float *__restrict__ k_cache, const float *__restrict__ v_cache,
+    const float *__restrict__ alpha_cache, const float *__restrict__ theta_cache, const float *__restrict__ amean_cache,
+    const float *__restrict__ emean_cache, const float *__restrict__ frozen, const float *__restrict__ gl,
+    const float *__restrict__ tok, const float *__restrict__ outer, const float *__restrict__ csv,
+    float *__restrict__ d_emb, float *__restrict__ d_mems, int s, int C, int nc) {
+    constexpr int CP = D / 4, KT = D / 16, JT = D / 16, NT = 4 * D, NW = D / 16, DD = D * D, V4 = D / 4, LD = D + 4;
+    constexpr int TF = sweep_token_floats(D), TILE = kTB * LD;
+    enum { A_K, A_U, A_X, A_G, A_DG0, A_FX, A_DG, A_W, A_Z, A_COUNT };
+    constexpr int RAW = A_COUNT * TILE > 3 * D * LD ? A_COUNT * TILE : 3 * D * LD;
+    __shared__ __align__(16) float raw[RAW];
+    __shared__ __align__(16) float gam[kTB * kTB];   // x_t . k_s, s in the order sigma
+    __shared__ __align__(16) float sc[kTB][8];       // alpha, theta, sigmoid' / (d keep), softplus' / d, dth0, dp . p
+    __shared__ __align__(16) float Sx[NW][kTB], Cx[NW][kTB];
+    __shared__ __align__(16) float av[2][D];
+    __shared__ float dEA[2][kTB], sp[NW];
+#define T_(a, t, i) raw[(a) * TILE + (t) * LD + (i)]
+
+    const int tid = threadIdx.x, r = tid >> 2, cq = tid & 3, wave = tid >> 6, lane = tid & 63;
+    const int ml = lane & 15, kg = lane >> 4, wr = 16 * wave, c0 = cq * CP;
+    const size_t b = blockIdx.x, tok0 = b * (size_t)s;
+    const int stt = tid / V4, sj = (tid % V4) * 4;      // staging slot: token, column
+    const int ve = CP * kg + ml % CP;                   // the vector element a lane holds
+    const int tcol = CP * (ml >> 2) + (ml & 3);         // column of result row ml of block 0; block kt: + 4 kt
+    const int my_s = sigma(ml);                         // token of operand row ml
+
+    f32x4 dFm[4][JT], accEA = kZero;
+    float dG[CP], dGT[CP], sig = 0.f;
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+#pragma unroll
+        for (int jt = 0; jt < JT; jt++) dFm[c][jt] = kZero;
+    }
+#pragma unroll
+    for (int i = 0; i < CP; i++) dG[i] = dGT[i] = 0.f;
+    if (tid < NW * kTB) (&Sx[0][0])[tid] = 0.f;
+
+    float4 pf_k, pf_v, pf_x, pf_g, pf_dg, pf_fx, pf_gam;
+    float pf_s[6];
+    pf_k = pf_v = pf_x = pf_g = pf_dg = pf_fx = pf_gam = make_float4(0, 0, 0, 0);
+#pragma unroll
+    for (int i = 0; i < 6; i++) pf_s[i] = 0.f;
+    // Inputs of a tile, requested one tile ahead; rows behind the chunk's last token are zeros.
+    auto request = [&](int first, int nt) {
+        const float4 z = make_float4(0, 0, 0, 0);
+        const size_t o = (tok0 + first + stt) * D + sj;
+        const float *tp = tok + (tok0 + first + stt) * TF;
+        const bool on = stt < nt;
+        auto two = [&](const float *q) {  // rows of tok are 8 bytes aligned
+            const float2 lo = *reinterpret_cast<const float2 *>(q), hi = *reinterpret_cast<const float2 *>(q + 2);
+            return make_float4(lo.x, lo.y, hi.x, hi.y);
+        };
+        pf_k = on ? *reinterpret_cast<const float4 *>(k_cache + o) : z;
+        pf_v = on ? *reinterpret_cast<const float4 *>(v_cache + o) : z;
+        pf_x = on ? *reinterpret_cast<const float4 *>(emb + o) : z;
+        pf_g = on ? two(tp + sj) : z;
+        pf_dg = on ? two(tp + D + sj) : z;
+        pf_fx = on ? two(tp + 2 * D + sj) : z;
+        if (tid < 64) pf_gam = tid / 4 < nt ? two(tok + (tok0 + first + tid / 4) * TF + 3 * D + 4 * (tid % 4)) : z;
+        if (tid < nt) {
+            const size_t e = tok0 + first + tid;
+            pf_s[0] = alpha_cache[e]; pf_s[1] = theta_cache[e]; pf_s[2] = amean_cache[e]; pf_s[3] = emean_cache[e];
+            pf_s[4] = tok[e * TF + 3 * D + 16]; pf_s[5] = tok[e * TF + 3 * D + 17];
+        }
+    };
+
+    for (int ci = nc - 1; ci >= 0; ci--) {
+        const int t0 = ci * C, L = min(C, s - t0), ntile = (L + kTB - 1) / kTB;
+        const size_t chunk = b * nc + ci;
+        const float *fz = frozen + chunk * 6 * DD;
+        request(t0 + (ntile - 1) * kTB, L - (ntile - 1) * kTB);
+        // rows of F_k^T and (F_k - F_v)^T, column sums of F_eta, F_alpha
+        float FTk[CP], FTu[CP];
+#pragma unroll
+        for (int i = 0; i < CP; i++) {
+            const float *f = fz + (CP * kg + i) * D + wr + ml;
+            FTk[i] = f[0];
+            FTu[i] = f[DD];
+        }
+        const float csE = csv[chunk * 2 * D + wr + ml], csA = csv[chunk * 2 * D + D + wr + ml];
+        __syncthreads();
+        sig = 0.f;
+        if (ci < nc - 1) {
+            // Chunk boundary: gradients of F'_c = F_c G_L flow into dG_L = sum_c F_c^T dF'_c and dF_c = dF'_c G_L^T, on
+            // the matrix cores; the rows of dF_eta, dF_alpha are all equal (rank-1 terms of dG_L).
+            float *Fs = raw, *Bm = raw + D * LD, *GLT = raw + 2 * D * LD;
+            float G[CP], q[CP];
+            lds_read<CP>(G, gl + chunk * DD + r * D + c0);
+#pragma unroll
+            for (int i = 0; i < CP; i++) GLT[(c0 + i) * LD + r] = G[i];
+            if (kg == 0) { av[0][wr + ml] = accEA[0]; av[1][wr + ml] = accEA[1]; }
+            __syncthreads();
+            {
+                float eE[CP], eA[CP];
+                lds_read<CP>(eE, &av[0][c0]);
+                lds_read<CP>(eA, &av[1][c0]);
+                const float e = csv[chunk * 2 * D + r], a = csv[chunk * 2 * D + D + r];
+#pragma unroll
+                for (int i = 0; i < CP; i++) q[i] = e * eE[i] + a * eA[i];
+            }
+            f32x4 accG[JT], fnext[JT];
+#pragma unroll
+            for (int i = 0; i < JT; i++) {
+                const int e = tid + i * NT;
+                accG[i] = kZero;
+                fnext[i] = *reinterpret_cast<const f32x4 *>(fz + (e / V4) * D + (e % V4) * 4);
+            }
+#pragma unroll
+            for (int comp = 0; comp < 4; comp++) {
+                __syncthreads();
+#pragma unroll
+                for (int i = 0; i < JT; i++) {
+                    const int e = tid + i * NT;
+                    *reinterpret_cast<f32x4 *>(Fs + (e / V4) * LD + (e % V4) * 4) = fnext[i];
+                }
+                if (comp < 3) {
+                    const float *nf = fz + (size_t)(comp < 2 ? comp + 1 : 5) * DD;
+#pragma unroll
+                    for (int i = 0; i < JT; i++) {
+                        const int e = tid + i * NT;
+                        fnext[i] = *reinterpret_cast<const f32x4 *>(nf + (e / V4) * D + (e % V4) * 4);
+                    }
+                }
+#pragma unroll
+                for (int jt = 0; jt < JT; jt++) {
+#pragma unroll
+                    for (int v = 0; v < 4; v++) Bm[(wr + 4 * kg + v) * LD + 16 * jt + ml] = dFm[comp][jt][v];
+                }
+                // the sum over the chunk's tokens that prepare left, behind the products that need dF'_c alone
+                f32x4 accN[JT];
+#pragma unroll
+                for (int jt = 0; jt < JT; jt++) accN[jt] = kZero;
+                __syncthreads();
+#pragma unroll 4
+                for (int k0 = 0; k0 < D; k0 += 4) {
+                    const float a1 = Fs[(k0 + kg) * LD + wr + ml];   // (F_c^T)[row][k]
+                    const float a2 = Bm[(wr + ml) * LD + k0 + kg];   // dF'_c[row][k]
+#pragma unroll
+                    for (int jt = 0; jt < JT; jt++) {
+                        accG[jt] = mfma4(a1, Bm[(k0 + kg) * LD + 16 * jt + ml], accG[jt]);
+                        accN[jt] = mfma4(a2, GLT[(k0 + kg) * LD + 16 * jt + ml], accN[jt]);
+                    }
+                }
+#pragma unroll
+                for (int jt = 0; jt < JT; jt++) dFm[comp][jt] = accN[jt];
+            }
+            {   // accE <- G_L accE, accA <- G_L accA: rows 0 and 1 of one more product
+                f32x4 accV = kZero;
+#pragma unroll 4
+                for (int k0 = 0; k0 < D; k0 += 4) {
+                    const float a = ml < 2 ? av[ml][k0 + kg] : 0.f;
+                    accV = mfma4(a, GLT[(k0 + kg) * LD + wr + ml], accV);
+                }
+                accEA = accV;
+            }
+            __syncthreads();  // every wave has read Bm
+#pragma unroll
+            for (int jt = 0; jt < JT; jt++) {
+#pragma unroll
+                for (int v = 0; v < 4; v++) Bm[(wr + 4 * kg + v) * LD + 16 * jt + ml] = accG[jt][v];
+            }
+            __builtin_amdgcn_wave_barrier();
+            float t[CP];
+            lds_read<CP>(t, Bm + r * LD + c0);
+#pragma unroll
+            for (int i = 0; i < CP; i++) t[i] += q[i];
+            vec_store<CP>(Bm + r * LD + c0, t);
+            // sigma_L = <G_L, dG_L>; then (1-a_t) <G_t, dG_{t+1}> = sigma_{t+1} + th_t u.W_t and
+            // sigma_t = that + dg.g + dp.p carry the inner product the gradient of alpha needs
+            const float part = wave_allreduce(dotn<CP>(G, t));
+            if (lane == 0) sp[wave] = part;
+            __syncthreads();
+#pragma unroll
+            for (int w = 0; w < NW; w++) sig += sp[w];
+            lds_read<CP>(dG, Bm + (wr + ml) * LD + CP * kg);
+#pragma unroll
+            for (int i = 0; i < CP; i++) dGT[i] = Bm[(CP * kg + i) * LD + wr + ml];
+        }
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+#pragma unroll
+            for (int jt = 0; jt < JT; jt++)
+                dFm[c][jt] += *reinterpret_cast<const f32x4 *>(outer + (chunk * 4 + c) * DD +
+                                                               ((size_t)(wave * JT + jt) * 64 + lane) * 4);
+        }
+#pragma unroll
+        for (int i = 0; i < CP; i++) FTu[i] = FTk[i] - FTu[i];
+
+        for (int tile = ntile - 1; tile >= 0; tile--) {
+            const int tb = t0 + tile * kTB, nt = min(kTB, t0 + L - tb);
+            __syncthreads();
+            *reinterpret_cast<float4 *>(&T_(A_K, stt, sj)) = pf_k;
+            *reinterpret_cast<float4 *>(&T_(A_U, stt, sj)) =
+                make_float4(pf_k.x - pf_v.x, pf_k.y - pf_v.y, pf_k.z - pf_v.z, pf_k.w - pf_v.w);
+            *reinterpret_cast<float4 *>(&T_(A_X, stt, sj)) = pf_x;
+            *reinterpret_cast<float4 *>(&T_(A_G, stt, sj)) = pf_g;
+            *reinterpret_cast<float4 *>(&T_(A_DG0, stt, sj)) = pf_dg;
+            *reinterpret_cast<float4 *>(&T_(A_FX, stt, sj)) = pf_fx;
+            *reinterpret_cast<float4 *>(&T_(A_DG, stt, sj)) = make_float4(0, 0, 0, 0);
+            if (tid < 64) *reinterpret_cast<float4 *>(&gam[4 * tid]) = pf_gam;
+            if (tid < kTB) {
+                const float sa = sr_sigmoid(pf_s[2]), keep = 1.f - pf_s[0];
+                sc[tid][0] = pf_s[0];
+                sc[tid][1] = tid < nt ? pf_s[1] : 0.f;
+                // a saturated gate (keep = 0) has no gradient
+                sc[tid][2] = keep > 0.f ? sa * (1.f - sa) * (1.f / D) / keep : 0.f;
+                sc[tid][3] = sr_sigmoid(pf_s[3]) * (1.f / D);
+                sc[tid][4] = pf_s[4];
+                sc[tid][5] = pf_s[5];
+                dEA[0][tid] = dEA[1][tid] = 0.f;
+            }
+            __syncthreads();
+            if (tile > 0) request(tb - kTB, kTB);
+
+            // W = dG K, Z = dG^T U, Y = F_k^T Z + (F_k - F_v)^T W of the whole tile; T_s = u_s . W_s
+            f32x4 W = kZero, Z = kZero, Y = kZero;
+            float U[CP], T = 0.f;
+#pragma unroll
+            for (int i = 0; i < CP; i += 4) {
+                const f32x4 k4 = *reinterpret_cast<const f32x4 *>(&T_(A_K, my_s, CP * kg + i));
+                const f32x4 u4 = *reinterpret_cast<const f32x4 *>(&T_(A_U, my_s, CP * kg + i));
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    U[i + v] = u4[v];
+                    W = mfma4(k4[v], dG[i + v], W);
+                    Z = mfma4(u4[v], dGT[i + v], Z);
+                }
+            }
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                T_(A_W, 4 * v + kg, wr + ml) = W[v];
+                T_(A_Z, 4 * v + kg, wr + ml) = Z[v];
+            }
+            lds_barrier();
+#pragma unroll
+            for (int i = 0; i < CP; i += 4) {
+                const f32x4 w4 = *reinterpret_cast<const f32x4 *>(&T_(A_W, my_s, CP * kg + i));
+                const f32x4 z4 = *reinterpret_cast<const f32x4 *>(&T_(A_Z, my_s, CP * kg + i));
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    T = fmaf(U[i + v], w4[v], T);
+                    Y = mfma4(z4[v], FTk[i + v], Y);
+                    Y = mfma4(w4[v], FTu[i + v], Y);
+                }
+            }
+            T = swapadd32(T, T);
+            T = swapadd16(T, T);
+
+            // a_ts = dg_t . u_s for t = 4 j + kg, and prod_{s<r<t} (1-a_r); the same product over the whole tile above s;
+            // prod_{r<t} (1-a_r) for t = 4 j + kg
+            float at[4], ct[4], above = 1.f, below[4], keep_tile = 1.f;
+#pragma unroll
+            for (int j = 0; j < 4; j++) at[j] = ct[j] = below[j] = 0.f;
+            float ybc = 0.f, uw = 0.f, pkeep = 1.f, pfx = 0.f, pm = 0.f;
+            f32x4 pgam = kZero;
+
+            auto step = [&](auto TT) __attribute__((always_inline)) {
+                constexpr int t = decltype(TT)::value, J = t / 4, Q = t % 4;
+                if (t >= nt) return;
+                if (t == nt - 1) {
+                    ybc = lane_from(4 * (ml + 16 * Q), Y[J]);
+                    uw = lane_value(T, sigma(t));
+                }
+                const f32x4 s0 = *reinterpret_cast<const f32x4 *>(&sc[t][0]);
+                const float2 s1 = *reinterpret_cast<const float2 *>(&sc[t][4]);
+                const float th = s0[1], keep = 1.f - s0[0];
+                const float dth = s1.x - uw, keepalp = fmaf(-th, dth, sig);
+                const float da = -keepalp * s0[2], de = dth * s0[3];
+                const float dg = fmaf(-th, ybc, T_(A_DG0, t, wr + ml)) + de * csE + da * csA;
+                T_(A_DG, t, wr + ml) = dg;
+                if (tid == 0) { dEA[0][t] = de; dEA[1][t] = da; }
+                lds_barrier();
+                const float dgv = T_(A_DG, t, ve), gv = T_(A_G, t, ve);
+                const f32x4 ps = *reinterpret_cast<const f32x4 *>(&Sx[wave][4 * kg]);
+                const float gml = gam[t * kTB + ml], fx = T_(A_FX, t, wr + ml);
+                const f32x4 g4 = *reinterpret_cast<const f32x4 *>(&gam[t * kTB + 4 * kg]);
+                __builtin_amdgcn_sched_barrier(0);  // what follows runs while the reads are under way
+                float yold = 0.f;
+                if constexpr (t > 0) {
+                    constexpr int J1 = (t - 1) / 4, Q1 = (t - 1) % 4;
+#pragma unroll
+                    for (int v = 0; v <= J1; v++) Y[v] = fmaf(pm, pgam[v], fmaf(pfx, ps[v], pkeep * Y[v]));
+                    yold = lane_from(4 * (ml + 16 * Q1), Y[J1]);
+                }
+                float gg = (CP == 16 || ml < CP) ? dgv * gv : 0.f;
+                float mv = dot_spread<CP>(FTu, dgv, 0.f), a = dot_spread<CP>(U, dgv, 0.f);
+                gg = row_sum(gg);
+                across_rows3(mv, a, gg);
+                sig = keepalp + gg + s1.y;
+                T = fmaf(a, gml, keep * T);
+                if constexpr (t > 0) {
+                    constexpr int P1 = sigma(t - 1);
+                    const float a1 = lane_value(a, P1), g1 = lane_value(gml, P1);
+                    ybc = fmaf(mv, g1, fmaf(fx, a1, keep * yold));
+                    uw = lane_value(T, P1);
+                    Sx[wave][ml] = a;
+                    pkeep = keep; pfx = fx; pm = mv; pgam = g4;
+                }
+                // tables of the tile's end: the retention of token t counts for the pairs around it
+                const float km = my_s < t ? keep : 1.f;
+                above *= km;
+#pragma unroll
+                for (int j = J; j < 4; j++) { ct[j] *= km; below[j] *= keep; }
+                keep_tile *= keep;
+                const bool mine = kg == Q;
+                below[J] = mine ? 1.f : below[J];
+                at[J] = mine ? a : at[J];
+                ct[J] = mine ? (my_s < t ? 1.f : 0.f) : ct[J];
+            };
+            downwards(step, std::make_integer_sequence<int, kTB>{});
+
+            // W_s, Z_s at their own tokens: what the tile started with under the retentions above s, plus the tile's own
+            // pairs; dk = -th (Z + W), dv = th W are the operands of the outer products as they stand
+            Cx[wave][ml] = above;
+            __builtin_amdgcn_wave_barrier();
+            const f32x4 top = *reinterpret_cast<const f32x4 *>(&Cx[wave][4 * kg]);
+            W *= top;
+            Z *= top;
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const int t = 4 * j + kg;
+                W = mfma4(ct[j] * gam[t * kTB + ml], T_(A_DG, t, wr + ml), W);
+                Z = mfma4(ct[j] * at[j], T_(A_X, t, wr + ml), Z);
+            }
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int t = 4 * v + kg;
+                const float th = sc[t][1], dv = th * W[v], dk = -th * (Z[v] + W[v]);
+                const float ea = ml < 2 ? dEA[ml][t] : 0.f;
+#pragma unroll
+                for (int jt = 0; jt < JT; jt++) {
+                    const float g = T_(A_G, t, 16 * jt + ml);
+                    dFm[0][jt] = mfma4(dk, g, dFm[0][jt]);
+                    dFm[1][jt] = mfma4(dv, g, dFm[1][jt]);
+                }
+                accEA = mfma4(ea, T_(A_G, t, wr + ml), accEA);
+            }
+            if (tile > 0) {  // the chunk's first tile has no use for its dG: G_0 = I
+                f32x4 n[KT], nT[KT];
+#pragma unroll
+                for (int kt = 0; kt < KT; kt++) {
+#pragma unroll
+                    for (int v = 0; v < 4; v++) {
+                        n[kt][v] = keep_tile * dG[4 * kt + v];
+                        nT[kt][v] = keep_tile * dGT[4 * kt + v];
+                    }
+                }
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const int t = 4 * j + kg;
+                    const float bg = below[j] * T_(A_DG, t, wr + ml), bx = below[j] * T_(A_X, t, wr + ml);
+#pragma unroll
+                    for (int kt = 0; kt < KT; kt++) {
+                        n[kt] = mfma4(T_(A_X, t, tcol + 4 * kt), bg, n[kt]);
+                        nT[kt] = mfma4(T_(A_DG, t, tcol + 4 * kt), bx, nT[kt]);
+                    }
+                }
+#pragma unroll
+                for (int kt = 0; kt < KT; kt++) {
+#pragma unroll
+                    for (int v = 0; v < 4; v++) { dG[4 * kt + v] = n[kt][v]; dGT[4 * kt + v] = nT[kt][v]; }
+                }
+            }
+            if (stt < nt)
+                *reinterpret_cast<float4 *>(d_emb + (tok0 + tb + stt) * D + sj) =
+                    *reinterpret_cast<const float4 *>(&T_(A_DG, stt, sj));
+        }
+    }
+    // gradients of the initial memories
+    float *dmb = d_mems + b * 6 * DD;
+#pragma unroll
+    for (int comp = 0; comp < 4; comp++) {
+        float *dst = dmb + (comp < 3 ? comp : 5) * DD;
+#pragma unroll
+        for (int jt = 0; jt < JT; jt++) {
+#pragma unroll
+            for (int v = 0; v < 4; v++) dst[(wr + 4 * kg + v) * D + 16 * jt + ml] = dFm[comp][jt][v];
+        }
+    }
+    __syncthreads();
+    if (kg == 0) { av[0][wr + ml] = accEA[0]; av[1][wr + ml] = accEA[1]; }
+    __syncthreads();
+    {
+        float eE[CP], eA[CP];
+        lds_read<CP>(eE, &av[0][c0]);
+        lds_read<CP>(eA, &av[1][c0]);
+        vec_store<CP>(dmb + 3 * DD + r * D + c0, eE);
+        vec_store<CP>(dmb + 4 * DD + r * D + c0, eA);
+    }
+#undef T_
+}
+
+template <int D>
+void launch(const SelfrefSweep &a) {
+    constexpr size_t lds = (chunk_lds_floats<D>(0) + PrepareLds<D>::floats) * sizeof(float);
+    static_assert(5 * kLrC * (D + 4) <= chunk_lds_floats<D>(0) + PrepareLds<D>::rows, "operands of the outer products");
+    static_assert(lds <= 160 * 1024, "LDS");
+    check_hip(hipFuncSetAttribute(reinterpret_cast<const void *>(selfref_bwd_prepare_kernel<D>),
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds), "dynamic LDS size");
+    hipLaunchKernelGGL((selfref_bwd_prepare_kernel<D>), dim3(a.batch * a.nc), dim3(4 * D), lds, stream(), a.emb, a.d_y, a.k,
+                       a.v, a.q, a.alpha, a.theta, a.frozen, a.gl, a.tok, a.outer, a.csv, a.s, a.C, a.nc);
+    check_launch("selfref_bwd_prepare_kernel");
+    KernelTimer kt("selfref_bwd_kernel");
+    hipLaunchKernelGGL((selfref_bwd_sweep_kernel<D>), dim3(a.batch), dim3(4 * D), 0, stream(), a.emb, a.k, a.v, a.alpha,
+                       a.theta, a.amean, a.emean, a.frozen, a.gl, a.tok, a.outer, a.csv, a.d_emb, a.d_mems, a.s, a.C, a.nc);
+    check_launch("selfref_bwd_sweep_kernel");
+}
+
+}  // namespace
+
+void selfref_backward_sweep(const SelfrefSweep &a) {
+    if (a.d == 16) launch<16>(a);
+    else if (a.d == 32) launch<32>(a);
+    else launch<64>(a);
+}
+
+}  // namespace nlh
