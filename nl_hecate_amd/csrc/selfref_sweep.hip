@@ -12,7 +12,7 @@
 // so that a token takes one exchange (dg_t), one product with a matrix and the dots of dg_t with the tile's u_s.
 #include <hip/hip_runtime.h>
 
-#include <utility>
+#include <type_traits>
 
 #include "../../include/nl_hecate_ffi.h"
 #include "lane_ops.h"
@@ -363,17 +363,32 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_prepare_kernel(
 }
 
 // ── the sweep ────────────────────────────────────────────────────────────────────────────────────────────────────
-// f(15), f(14), ... f(0) with the argument as a type
-template <class Fn, int... I>
-__device__ __forceinline__ void downwards(Fn &f, std::integer_sequence<int, I...>) {
-    (f(std::integral_constant<int, kTB - 1 - I>{}), ...);
+// f(4 J + 3) ... f(4 J) with the argument as a type, if the tile has tokens there
+template <int J, class Fn>
+__device__ __forceinline__ void four_down(Fn &f, int nt) {
+    if (4 * J < nt) {
+        f(std::integral_constant<int, 4 * J + 3>{});
+        f(std::integral_constant<int, 4 * J + 2>{});
+        f(std::integral_constant<int, 4 * J + 1>{});
+        f(std::integral_constant<int, 4 * J>{});
+    }
 }
 
-// acc + sum_i m[i] x_i with x spread over the DPP rows: lane i of row kg holds x_i for the row's lanes.
+// acc += m x_I with x spread over the DPP rows: lane i of row kg holds x_i for the row's lanes.  In assembly because the
+// compiler moves a broadcast that two products share into a register of its own first.
+template <int I>
+__device__ __forceinline__ void fmac_spread(float &acc, float x, float m) {
+    asm("v_fmac_f32_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "+v"(acc) : "v"(x), "v"(m), "n"(I));
+}
+// Two dots with x at once, two chains each.  x has to come from memory: a vector instruction that wrote it would need
+// two wait states in front of the first broadcast.
 template <int N, int I = 0>
-__device__ __forceinline__ float dot_spread(const float (&m)[N], float x, float acc) {
-    if constexpr (I == N) return acc;
-    else return dot_spread<N, I + 1>(m, x, fmaf(dpp_mov<0x150 + I>(x), m[I], acc));  // row_newbcast: lane I of the row
+__device__ __forceinline__ void dots_spread(const float (&m)[N], const float (&n)[N], float x, float (&dm)[2], float (&dn)[2]) {
+    if constexpr (I < N) {
+        fmac_spread<I>(dm[I & 1], x, m[I]);
+        fmac_spread<I>(dn[I & 1], x, n[I]);
+        dots_spread<N, I + 1>(m, n, x, dm, dn);
+    }
 }
 
 // Sums over the four DPP rows of three values at once, every lane receives them.
@@ -409,7 +424,7 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_sweep_kernel(
     __shared__ __align__(16) float sc[kTB][8];       // alpha, theta, sigmoid' / (d keep), softplus' / d, dth0, dp . p
     __shared__ __align__(16) float Sx[NW][kTB], Cx[NW][kTB];
     __shared__ __align__(16) float av[2][D];
-    __shared__ float dEA[2][kTB], sp[NW];
+    __shared__ float sp[NW];
 #define T_(a, t, i) raw[(a) * TILE + (t) * LD + (i)]
 
     const int tid = threadIdx.x, r = tid >> 2, cq = tid & 3, wave = tid >> 6, lane = tid & 63;
@@ -474,7 +489,16 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_sweep_kernel(
             FTu[i] = f[DD];
         }
         const float csE = csv[chunk * 2 * D + wr + ml], csA = csv[chunk * 2 * D + D + wr + ml];
-        __syncthreads();
+        f32x4 sums[4][JT];  // what the chunk's tokens add to dF whatever the sweep finds
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+#pragma unroll
+            for (int jt = 0; jt < JT; jt++)
+                sums[c][jt] = *reinterpret_cast<const f32x4 *>(outer + (chunk * 4 + c) * DD +
+                                                               ((size_t)(wave * JT + jt) * 64 + lane) * 4);
+        }
+        // LDS-only barriers from here on: the requests above and the stores of dg stay under way across them
+        lds_barrier();
         sig = 0.f;
         if (ci < nc - 1) {
             // Chunk boundary: gradients of F'_c = F_c G_L flow into dG_L = sum_c F_c^T dF'_c and dF_c = dF'_c G_L^T, on
@@ -485,7 +509,7 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_sweep_kernel(
 #pragma unroll
             for (int i = 0; i < CP; i++) GLT[(c0 + i) * LD + r] = G[i];
             if (kg == 0) { av[0][wr + ml] = accEA[0]; av[1][wr + ml] = accEA[1]; }
-            __syncthreads();
+            lds_barrier();
             {
                 float eE[CP], eA[CP];
                 lds_read<CP>(eE, &av[0][c0]);
@@ -503,7 +527,7 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_sweep_kernel(
             }
 #pragma unroll
             for (int comp = 0; comp < 4; comp++) {
-                __syncthreads();
+                lds_barrier();
 #pragma unroll
                 for (int i = 0; i < JT; i++) {
                     const int e = tid + i * NT;
@@ -522,11 +546,10 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_sweep_kernel(
 #pragma unroll
                     for (int v = 0; v < 4; v++) Bm[(wr + 4 * kg + v) * LD + 16 * jt + ml] = dFm[comp][jt][v];
                 }
-                // the sum over the chunk's tokens that prepare left, behind the products that need dF'_c alone
                 f32x4 accN[JT];
 #pragma unroll
                 for (int jt = 0; jt < JT; jt++) accN[jt] = kZero;
-                __syncthreads();
+                lds_barrier();
 #pragma unroll 4
                 for (int k0 = 0; k0 < D; k0 += 4) {
                     const float a1 = Fs[(k0 + kg) * LD + wr + ml];   // (F_c^T)[row][k]
@@ -549,7 +572,7 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_sweep_kernel(
                 }
                 accEA = accV;
             }
-            __syncthreads();  // every wave has read Bm
+            lds_barrier();  // every wave has read Bm
 #pragma unroll
             for (int jt = 0; jt < JT; jt++) {
 #pragma unroll
@@ -565,7 +588,7 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_sweep_kernel(
             // sigma_t = that + dg.g + dp.p carry the inner product the gradient of alpha needs
             const float part = wave_allreduce(dotn<CP>(G, t));
             if (lane == 0) sp[wave] = part;
-            __syncthreads();
+            lds_barrier();
 #pragma unroll
             for (int w = 0; w < NW; w++) sig += sp[w];
             lds_read<CP>(dG, Bm + (wr + ml) * LD + CP * kg);
@@ -575,16 +598,14 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_sweep_kernel(
 #pragma unroll
         for (int c = 0; c < 4; c++) {
 #pragma unroll
-            for (int jt = 0; jt < JT; jt++)
-                dFm[c][jt] += *reinterpret_cast<const f32x4 *>(outer + (chunk * 4 + c) * DD +
-                                                               ((size_t)(wave * JT + jt) * 64 + lane) * 4);
+            for (int jt = 0; jt < JT; jt++) dFm[c][jt] += sums[c][jt];
         }
 #pragma unroll
         for (int i = 0; i < CP; i++) FTu[i] = FTk[i] - FTu[i];
 
         for (int tile = ntile - 1; tile >= 0; tile--) {
             const int tb = t0 + tile * kTB, nt = min(kTB, t0 + L - tb);
-            __syncthreads();
+            lds_barrier();
             *reinterpret_cast<float4 *>(&T_(A_K, stt, sj)) = pf_k;
             *reinterpret_cast<float4 *>(&T_(A_U, stt, sj)) =
                 make_float4(pf_k.x - pf_v.x, pf_k.y - pf_v.y, pf_k.z - pf_v.z, pf_k.w - pf_v.w);
@@ -596,16 +617,16 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_sweep_kernel(
             if (tid < 64) *reinterpret_cast<float4 *>(&gam[4 * tid]) = pf_gam;
             if (tid < kTB) {
                 const float sa = sr_sigmoid(pf_s[2]), keep = 1.f - pf_s[0];
-                sc[tid][0] = pf_s[0];
-                sc[tid][1] = tid < nt ? pf_s[1] : 0.f;
+                const bool on = tid < nt;  // zeros behind the last token: it passes everything on as it is
+                sc[tid][0] = on ? pf_s[0] : 0.f;
+                sc[tid][1] = on ? pf_s[1] : 0.f;
                 // a saturated gate (keep = 0) has no gradient
-                sc[tid][2] = keep > 0.f ? sa * (1.f - sa) * (1.f / D) / keep : 0.f;
-                sc[tid][3] = sr_sigmoid(pf_s[3]) * (1.f / D);
-                sc[tid][4] = pf_s[4];
-                sc[tid][5] = pf_s[5];
-                dEA[0][tid] = dEA[1][tid] = 0.f;
+                sc[tid][2] = on && keep > 0.f ? sa * (1.f - sa) * (1.f / D) / keep : 0.f;
+                sc[tid][3] = on ? sr_sigmoid(pf_s[3]) * (1.f / D) : 0.f;
+                sc[tid][4] = on ? pf_s[4] : 0.f;
+                sc[tid][5] = on ? pf_s[5] : 0.f;
             }
-            __syncthreads();
+            lds_barrier();
             if (tile > 0) request(tb - kTB, kTB);
 
             // W = dG K, Z = dG^T U, Y = F_k^T Z + (F_k - F_v)^T W of the whole tile; T_s = u_s . W_s
@@ -644,54 +665,34 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_sweep_kernel(
 
             // a_ts = dg_t . u_s for t = 4 j + kg, and prod_{s<r<t} (1-a_r); the same product over the whole tile above s;
             // prod_{r<t} (1-a_r) for t = 4 j + kg
-            float at[4], ct[4], above = 1.f, below[4], keep_tile = 1.f;
+            float at[4], ct[4], et[4], above = 1.f, below[4], keep_tile = 1.f;
 #pragma unroll
-            for (int j = 0; j < 4; j++) at[j] = ct[j] = below[j] = 0.f;
-            float ybc = 0.f, uw = 0.f, pkeep = 1.f, pfx = 0.f, pm = 0.f;
-            f32x4 pgam = kZero;
+            for (int j = 0; j < 4; j++) at[j] = ct[j] = et[j] = below[j] = 0.f;
+            // groups of four tokens; the first one ends behind the last token at most
+            const int first_j = (nt - 1) >> 2;
+            float ybc = lane_from(4 * (ml + 48), first_j == 3 ? Y[3] : first_j == 2 ? Y[2] : first_j == 1 ? Y[1] : Y[0]);
+            float uw = lane_value(T, sigma(3) + first_j), pkeep = 1.f, pfx = 0.f, pm = 0.f;
+            f32x4 pgam = kZero, s0 = *reinterpret_cast<const f32x4 *>(&sc[4 * first_j + 3][0]);
+            float2 s1 = *reinterpret_cast<const float2 *>(&sc[4 * first_j + 3][4]);
+            float dg0 = T_(A_DG0, 4 * first_j + 3, wr + ml);
 
             auto step = [&](auto TT) __attribute__((always_inline)) {
                 constexpr int t = decltype(TT)::value, J = t / 4, Q = t % 4;
-                if (t >= nt) return;
-                if (t == nt - 1) {
-                    ybc = lane_from(4 * (ml + 16 * Q), Y[J]);
-                    uw = lane_value(T, sigma(t));
-                }
-                const f32x4 s0 = *reinterpret_cast<const f32x4 *>(&sc[t][0]);
-                const float2 s1 = *reinterpret_cast<const float2 *>(&sc[t][4]);
-                const float th = s0[1], keep = 1.f - s0[0];
+                const float th = s0[1], keep = 1.f - s0[0], sig0 = s1.y;
                 const float dth = s1.x - uw, keepalp = fmaf(-th, dth, sig);
                 const float da = -keepalp * s0[2], de = dth * s0[3];
-                const float dg = fmaf(-th, ybc, T_(A_DG0, t, wr + ml)) + de * csE + da * csA;
-                T_(A_DG, t, wr + ml) = dg;
-                if (tid == 0) { dEA[0][t] = de; dEA[1][t] = da; }
+                T_(A_DG, t, wr + ml) = fmaf(da, csA, fmaf(de, csE, fmaf(-th, ybc, dg0)));
                 lds_barrier();
                 const float dgv = T_(A_DG, t, ve), gv = T_(A_G, t, ve);
                 const f32x4 ps = *reinterpret_cast<const f32x4 *>(&Sx[wave][4 * kg]);
                 const float gml = gam[t * kTB + ml], fx = T_(A_FX, t, wr + ml);
                 const f32x4 g4 = *reinterpret_cast<const f32x4 *>(&gam[t * kTB + 4 * kg]);
+                if constexpr (t > 0) {
+                    s0 = *reinterpret_cast<const f32x4 *>(&sc[t - 1][0]);
+                    s1 = *reinterpret_cast<const float2 *>(&sc[t - 1][4]);
+                    dg0 = T_(A_DG0, t - 1, wr + ml);
+                }
                 __builtin_amdgcn_sched_barrier(0);  // what follows runs while the reads are under way
-                float yold = 0.f;
-                if constexpr (t > 0) {
-                    constexpr int J1 = (t - 1) / 4, Q1 = (t - 1) % 4;
-#pragma unroll
-                    for (int v = 0; v <= J1; v++) Y[v] = fmaf(pm, pgam[v], fmaf(pfx, ps[v], pkeep * Y[v]));
-                    yold = lane_from(4 * (ml + 16 * Q1), Y[J1]);
-                }
-                float gg = (CP == 16 || ml < CP) ? dgv * gv : 0.f;
-                float mv = dot_spread<CP>(FTu, dgv, 0.f), a = dot_spread<CP>(U, dgv, 0.f);
-                gg = row_sum(gg);
-                across_rows3(mv, a, gg);
-                sig = keepalp + gg + s1.y;
-                T = fmaf(a, gml, keep * T);
-                if constexpr (t > 0) {
-                    constexpr int P1 = sigma(t - 1);
-                    const float a1 = lane_value(a, P1), g1 = lane_value(gml, P1);
-                    ybc = fmaf(mv, g1, fmaf(fx, a1, keep * yold));
-                    uw = lane_value(T, P1);
-                    Sx[wave][ml] = a;
-                    pkeep = keep; pfx = fx; pm = mv; pgam = g4;
-                }
                 // tables of the tile's end: the retention of token t counts for the pairs around it
                 const float km = my_s < t ? keep : 1.f;
                 above *= km;
@@ -700,10 +701,40 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_sweep_kernel(
                 keep_tile *= keep;
                 const bool mine = kg == Q;
                 below[J] = mine ? 1.f : below[J];
-                at[J] = mine ? a : at[J];
                 ct[J] = mine ? (my_s < t ? 1.f : 0.f) : ct[J];
+                et[J] = mine ? (ml == 0 ? de : da) : et[J];
+                float yold = 0.f;
+                if constexpr (t > 0) {
+                    constexpr int J1 = (t - 1) / 4, Q1 = (t - 1) % 4;
+#pragma unroll
+                    for (int v = 0; v <= J1; v++) {
+                        Y[v] = fmaf(pm, pgam[v], fmaf(pfx, ps[v], pkeep * Y[v]));
+                        asm volatile("" : "+v"(Y[v]));
+                    }
+                    yold = keep * lane_from(4 * (ml + 16 * Q1), Y[J1]);
+                }
+                float gg = row_sum((CP == 16 || ml < CP) ? dgv * gv : 0.f);
+                float m2[2] = {0.f, 0.f}, a2[2] = {0.f, 0.f};
+                dots_spread<CP>(FTu, U, dgv, m2, a2);
+                float mv = m2[0] + m2[1], a = a2[0] + a2[1];
+                across_rows3(mv, a, gg);
+                asm volatile("" ::"v"(ps), "v"(g4));  // whole: an element without a use is not to be overwritten early
+                sig = keepalp + gg + sig0;
+                T = fmaf(a, gml, keep * T);
+                if constexpr (t > 0) {
+                    constexpr int P1 = sigma(t - 1);
+                    const float a1 = lane_value(a, P1), g1 = lane_value(gml, P1);
+                    ybc = fmaf(mv, g1, fmaf(fx, a1, yold));
+                    uw = lane_value(T, P1);
+                    Sx[wave][ml] = a;
+                    pkeep = keep; pfx = fx; pm = mv; pgam = g4;
+                }
+                at[J] = mine ? a : at[J];
             };
-            downwards(step, std::make_integer_sequence<int, kTB>{});
+            four_down<3>(step, nt);
+            four_down<2>(step, nt);
+            four_down<1>(step, nt);
+            four_down<0>(step, nt);
 
             // W_s, Z_s at their own tokens: what the tile started with under the retentions above s, plus the tile's own
             // pairs; dk = -th (Z + W), dv = th W are the operands of the outer products as they stand
@@ -722,7 +753,7 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_sweep_kernel(
             for (int v = 0; v < 4; v++) {
                 const int t = 4 * v + kg;
                 const float th = sc[t][1], dv = th * W[v], dk = -th * (Z[v] + W[v]);
-                const float ea = ml < 2 ? dEA[ml][t] : 0.f;
+                const float ea = ml < 2 ? et[v] : 0.f;
 #pragma unroll
                 for (int jt = 0; jt < JT; jt++) {
                     const float g = T_(A_G, t, 16 * jt + ml);
