@@ -103,14 +103,14 @@ struct SelfrefForward {
 void selfref_forward_chain(const SelfrefForward &a);
 
 // Backward under self-generated values for the same chunks and head sizes, up to dg (in d_emb) and d_mems; the last
-// pass, d_x = G^T dg, is the caller's.  gl: [chunks, d, d] scratch; tok: [tokens, 3 d + 16 + 2]; outer: [chunks, 4, d, d];
+// pass, d_x = G^T dg, is the caller's.  gl: [chunks, d, d] scratch; tok: [tokens, 3 d + 16 + 6]; outer: [chunks, 4, d, d];
 // csv: [chunks, 2, d].
 struct SelfrefSweep {
     const float *emb, *d_y, *k, *v, *q, *alpha, *theta, *amean, *emean, *frozen;
     float *d_emb, *d_mems, *gl, *tok, *outer, *csv;
     int s, d, batch, C, nc;
 };
-constexpr int sweep_token_floats(int d) { return 3 * d + 16 + 2; }
+constexpr int sweep_token_floats(int d) { return 3 * d + 16 + 6; }
 void selfref_backward_sweep(const SelfrefSweep &a);
 
 }  // namespace nlh

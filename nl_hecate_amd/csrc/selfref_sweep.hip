@@ -53,7 +53,8 @@ template <int D>
 __global__ __launch_bounds__(4 * D) void selfref_bwd_prepare_kernel(
     const float *__restrict__ emb, const float *__restrict__ d_y, const float *__restrict__ k_cache,
     const float *__restrict__ v_cache, const float *__restrict__ q_cache, const float *__restrict__ alpha_cache,
-    const float *__restrict__ theta_cache, const float *__restrict__ frozen, float *__restrict__ gl,
+    const float *__restrict__ theta_cache, const float *__restrict__ amean_cache,
+    const float *__restrict__ emean_cache, const float *__restrict__ frozen, float *__restrict__ gl,
     float *__restrict__ tok, float *__restrict__ outer, float *__restrict__ csv, int s, int C, int nc) {
     constexpr int KT = D / 16, NW = D / 16, NT = 4 * D, DD = D * D, KL = D + 4, V4 = D / 4, TPW = 4 / NW;
     constexpr int TF = sweep_token_floats(D);
@@ -74,6 +75,16 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_prepare_kernel(
 #pragma unroll 8
         for (int c = 0; c < D; c++) a += src[c * D];
         csv[chunk * 2 * D + e] = a;
+    }
+    for (int e = tid; e < L; e += NT) {  // the sweep's scalars of a token
+        const size_t i = tok0 + t0 + e;
+        const float al = alpha_cache[i], keep = 1.f - al, sa = sr_sigmoid(amean_cache[i]);
+        float *o = tok + i * TF + 3 * D + 16;
+        o[0] = al;
+        o[1] = theta_cache[i];
+        // sigmoid' of the mean over d keep (the sweep forms keep <G_t, dG_{t+1}>): a saturated gate has no gradient
+        o[2] = keep > 0.f ? sa * (1.f - sa) * (1.f / D) / keep : 0.f;
+        o[3] = sr_sigmoid(emean_cache[i]) * (1.f / D);  // softplus' of the mean over d
     }
     // scores that no token of the chunk has, and rows behind its last token, enter products times zero
     for (int e = tid; e < 2 * kLrC * kWL + kLrC * KL; e += NT) Wq[e] = 0.f;
@@ -198,7 +209,7 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_prepare_kernel(
 #pragma unroll
         for (int v = 0; v < 4; v++) {
             pp[v] = row_sum(pp[v]);
-            if (ml == 0 && 4 * kg + v < nt) out[(size_t)(4 * kg + v) * TF + 3 * D + 17] = pp[v];
+            if (ml == 0 && 4 * kg + v < nt) out[(size_t)(4 * kg + v) * TF + 3 * D + 21] = pp[v];
         }
         put(dp);
         as_operand(a);
@@ -277,7 +288,7 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_prepare_kernel(
 #pragma unroll
         for (int v = 0; v < 4; v++) {
             uw[v] = row_sum(uw[v]);
-            if (ml == 0 && 4 * kg + v < nt) out[(size_t)(4 * kg + v) * TF + 3 * D + 16] = -uw[v];
+            if (ml == 0 && 4 * kg + v < nt) out[(size_t)(4 * kg + v) * TF + 3 * D + 20] = -uw[v];
         }
         // dg0 = F_k^T dk + F_v^T dv + F_q^T dq, and F_k^T x
         f32x4 dg[KT], fx[KT], ak[KT], av[KT], aq[KT], ax[KT];
@@ -340,18 +351,21 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_prepare_kernel(
 #pragma unroll
         for (int jt = 0; jt < KT; jt++) o[c][jt] = kZero;
     }
-    for (int k0 = 0; k0 < 16 * ntile; k0 += 4) {
-        const int li = k0 + kg;
-        const float *e = Es + li * KL;
-        const float ak = e[wr + ml], av = e[kLrC * KL + wr + ml], aq = e[2 * kLrC * KL + wr + ml];
-        const float ay = li < L ? d_y[(tok0 + t0 + li) * D + wr + ml] : 0.f;
+    for (int st = 0; st < ntile; st++) {
 #pragma unroll
-        for (int jt = 0; jt < KT; jt++) {
-            const float bg = e[3 * kLrC * KL + 16 * jt + ml], bp = e[4 * kLrC * KL + 16 * jt + ml];
-            o[0][jt] = mfma4(ak, bg, o[0][jt]);
-            o[1][jt] = mfma4(av, bg, o[1][jt]);
-            o[2][jt] = mfma4(aq, bg, o[2][jt]);
-            o[3][jt] = mfma4(ay, bp, o[3][jt]);
+        for (int v = 0; v < 4; v++) {
+            const int li = 16 * st + 4 * kg + v;
+            const float *e = Es + li * KL;
+            const float ak = e[wr + ml], av = e[kLrC * KL + wr + ml], aq = e[2 * kLrC * KL + wr + ml];
+            const float ay = li < L ? d_y[(tok0 + t0 + li) * D + wr + ml] : 0.f;
+#pragma unroll
+            for (int jt = 0; jt < KT; jt++) {
+                const float bg = e[3 * kLrC * KL + 16 * jt + ml], bp = e[4 * kLrC * KL + 16 * jt + ml];
+                o[0][jt] = mfma4(ak, bg, o[0][jt]);
+                o[1][jt] = mfma4(av, bg, o[1][jt]);
+                o[2][jt] = mfma4(aq, bg, o[2][jt]);
+                o[3][jt] = mfma4(ay, bp, o[3][jt]);
+            }
         }
     }
 #pragma unroll
@@ -411,15 +425,16 @@ __device__ __forceinline__ void across_rows3(float &a, float &b, float &c) {
 template <int D>
 __global__ __launch_bounds__(4 * D) void selfref_bwd_sweep_kernel(
     const float *__restrict__ emb, const float *__restrict__ k_cache, const float *__restrict__ v_cache,
-    const float *__restrict__ alpha_cache, const float *__restrict__ theta_cache, const float *__restrict__ amean_cache,
-    const float *__restrict__ emean_cache, const float *__restrict__ frozen, const float *__restrict__ gl,
-    const float *__restrict__ tok, const float *__restrict__ outer, const float *__restrict__ csv,
-    float *__restrict__ d_emb, float *__restrict__ d_mems, int s, int C, int nc) {
+    const float *__restrict__ frozen, const float *__restrict__ gl, const float *__restrict__ tok,
+    const float *__restrict__ outer, const float *__restrict__ csv, float *__restrict__ d_emb,
+    float *__restrict__ d_mems, int s, int C, int nc) {
     constexpr int CP = D / 4, KT = D / 16, JT = D / 16, NT = 4 * D, NW = D / 16, DD = D * D, V4 = D / 4, LD = D + 4;
     constexpr int TF = sweep_token_floats(D), TILE = kTB * LD;
-    enum { A_K, A_U, A_X, A_G, A_DG0, A_FX, A_DG, A_W, A_Z, A_COUNT };
+    enum { A_K, A_U, A_X, A_DG0, A_FX, A_DG, A_W, A_Z, A_COUNT };
     constexpr int RAW = A_COUNT * TILE > 3 * D * LD ? A_COUNT * TILE : 3 * D * LD;
     __shared__ __align__(16) float raw[RAW];
+    constexpr int LG = D + 16;                       // rows 4 v + kg of g fall on different banks for the four kg
+    __shared__ __align__(16) float tg[kTB * LG];     // g
     __shared__ __align__(16) float gam[kTB * kTB];   // x_t . k_s, s in the order sigma
     __shared__ __align__(16) float sc[kTB][8];       // alpha, theta, sigmoid' / (d keep), softplus' / d, dth0, dp . p
     __shared__ __align__(16) float Sx[NW][kTB], Cx[NW][kTB];
@@ -468,10 +483,10 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_sweep_kernel(
         pf_dg = on ? two(tp + D + sj) : z;
         pf_fx = on ? two(tp + 2 * D + sj) : z;
         if (tid < 64) pf_gam = tid / 4 < nt ? two(tok + (tok0 + first + tid / 4) * TF + 3 * D + 4 * (tid % 4)) : z;
-        if (tid < nt) {
-            const size_t e = tok0 + first + tid;
-            pf_s[0] = alpha_cache[e]; pf_s[1] = theta_cache[e]; pf_s[2] = amean_cache[e]; pf_s[3] = emean_cache[e];
-            pf_s[4] = tok[e * TF + 3 * D + 16]; pf_s[5] = tok[e * TF + 3 * D + 17];
+        if (tid < kTB) {  // zeros behind the last token: it passes everything on as it is
+            const float *e = tok + (tok0 + first + min(tid, nt - 1)) * TF + 3 * D + 16;
+#pragma unroll
+            for (int i = 0; i < 6; i++) pf_s[i] = tid < nt ? e[i] : 0.f;
         }
     };
 
@@ -479,6 +494,17 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_sweep_kernel(
         const int t0 = ci * C, L = min(C, s - t0), ntile = (L + kTB - 1) / kTB;
         const size_t chunk = b * nc + ci;
         const float *fz = frozen + chunk * 6 * DD;
+        // in the order of their use: G_L and F_k for the boundary, then what the tiles read
+        float G[CP];
+        f32x4 fnext[JT];
+        if (ci < nc - 1) {
+            lds_read<CP>(G, gl + chunk * DD + r * D + c0);
+#pragma unroll
+            for (int i = 0; i < JT; i++) {
+                const int e = tid + i * NT;
+                fnext[i] = *reinterpret_cast<const f32x4 *>(fz + (e / V4) * D + (e % V4) * 4);
+            }
+        }
         request(t0 + (ntile - 1) * kTB, L - (ntile - 1) * kTB);
         // rows of F_k^T and (F_k - F_v)^T, column sums of F_eta, F_alpha
         float FTk[CP], FTu[CP];
@@ -504,8 +530,7 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_sweep_kernel(
             // Chunk boundary: gradients of F'_c = F_c G_L flow into dG_L = sum_c F_c^T dF'_c and dF_c = dF'_c G_L^T, on
             // the matrix cores; the rows of dF_eta, dF_alpha are all equal (rank-1 terms of dG_L).
             float *Fs = raw, *Bm = raw + D * LD, *GLT = raw + 2 * D * LD;
-            float G[CP], q[CP];
-            lds_read<CP>(G, gl + chunk * DD + r * D + c0);
+            float q[CP];
 #pragma unroll
             for (int i = 0; i < CP; i++) GLT[(c0 + i) * LD + r] = G[i];
             if (kg == 0) { av[0][wr + ml] = accEA[0]; av[1][wr + ml] = accEA[1]; }
@@ -518,13 +543,9 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_sweep_kernel(
 #pragma unroll
                 for (int i = 0; i < CP; i++) q[i] = e * eE[i] + a * eA[i];
             }
-            f32x4 accG[JT], fnext[JT];
+            f32x4 accG[JT];
 #pragma unroll
-            for (int i = 0; i < JT; i++) {
-                const int e = tid + i * NT;
-                accG[i] = kZero;
-                fnext[i] = *reinterpret_cast<const f32x4 *>(fz + (e / V4) * D + (e % V4) * 4);
-            }
+            for (int i = 0; i < JT; i++) accG[i] = kZero;
 #pragma unroll
             for (int comp = 0; comp < 4; comp++) {
                 lds_barrier();
@@ -550,14 +571,19 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_sweep_kernel(
 #pragma unroll
                 for (int jt = 0; jt < JT; jt++) accN[jt] = kZero;
                 lds_barrier();
-#pragma unroll 4
-                for (int k0 = 0; k0 < D; k0 += 4) {
-                    const float a1 = Fs[(k0 + kg) * LD + wr + ml];   // (F_c^T)[row][k]
-                    const float a2 = Bm[(wr + ml) * LD + k0 + kg];   // dF'_c[row][k]
+                // contraction in the order 16 c + 4 kg + v: rows 4 apart put the four kg of a read on different banks
 #pragma unroll
-                    for (int jt = 0; jt < JT; jt++) {
-                        accG[jt] = mfma4(a1, Bm[(k0 + kg) * LD + 16 * jt + ml], accG[jt]);
-                        accN[jt] = mfma4(a2, GLT[(k0 + kg) * LD + 16 * jt + ml], accN[jt]);
+                for (int c = 0; c < KT; c++) {
+                    const f32x4 a2 = *reinterpret_cast<const f32x4 *>(Bm + (wr + ml) * LD + 16 * c + 4 * kg);  // dF'_c
+#pragma unroll
+                    for (int v = 0; v < 4; v++) {
+                        const int k = 16 * c + 4 * kg + v;
+                        const float a1 = Fs[k * LD + wr + ml];  // F_c^T
+#pragma unroll
+                        for (int jt = 0; jt < JT; jt++) {
+                            accG[jt] = mfma4(a1, Bm[k * LD + 16 * jt + ml], accG[jt]);
+                            accN[jt] = mfma4(a2[v], GLT[k * LD + 16 * jt + ml], accN[jt]);
+                        }
                     }
                 }
 #pragma unroll
@@ -565,10 +591,11 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_sweep_kernel(
             }
             {   // accE <- G_L accE, accA <- G_L accA: rows 0 and 1 of one more product
                 f32x4 accV = kZero;
-#pragma unroll 4
-                for (int k0 = 0; k0 < D; k0 += 4) {
-                    const float a = ml < 2 ? av[ml][k0 + kg] : 0.f;
-                    accV = mfma4(a, GLT[(k0 + kg) * LD + wr + ml], accV);
+#pragma unroll
+                for (int c = 0; c < KT; c++) {
+                    const f32x4 a = ml < 2 ? *reinterpret_cast<const f32x4 *>(&av[ml][16 * c + 4 * kg]) : kZero;
+#pragma unroll
+                    for (int v = 0; v < 4; v++) accV = mfma4(a[v], GLT[(16 * c + 4 * kg + v) * LD + wr + ml], accV);
                 }
                 accEA = accV;
             }
@@ -610,27 +637,20 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_sweep_kernel(
             *reinterpret_cast<float4 *>(&T_(A_U, stt, sj)) =
                 make_float4(pf_k.x - pf_v.x, pf_k.y - pf_v.y, pf_k.z - pf_v.z, pf_k.w - pf_v.w);
             *reinterpret_cast<float4 *>(&T_(A_X, stt, sj)) = pf_x;
-            *reinterpret_cast<float4 *>(&T_(A_G, stt, sj)) = pf_g;
+            *reinterpret_cast<float4 *>(&tg[stt * LG + sj]) = pf_g;
             *reinterpret_cast<float4 *>(&T_(A_DG0, stt, sj)) = pf_dg;
             *reinterpret_cast<float4 *>(&T_(A_FX, stt, sj)) = pf_fx;
             *reinterpret_cast<float4 *>(&T_(A_DG, stt, sj)) = make_float4(0, 0, 0, 0);
             if (tid < 64) *reinterpret_cast<float4 *>(&gam[4 * tid]) = pf_gam;
             if (tid < kTB) {
-                const float sa = sr_sigmoid(pf_s[2]), keep = 1.f - pf_s[0];
-                const bool on = tid < nt;  // zeros behind the last token: it passes everything on as it is
-                sc[tid][0] = on ? pf_s[0] : 0.f;
-                sc[tid][1] = on ? pf_s[1] : 0.f;
-                // a saturated gate (keep = 0) has no gradient
-                sc[tid][2] = on && keep > 0.f ? sa * (1.f - sa) * (1.f / D) / keep : 0.f;
-                sc[tid][3] = on ? sr_sigmoid(pf_s[3]) * (1.f / D) : 0.f;
-                sc[tid][4] = on ? pf_s[4] : 0.f;
-                sc[tid][5] = on ? pf_s[5] : 0.f;
+                *reinterpret_cast<f32x4 *>(&sc[tid][0]) = f32x4{pf_s[0], pf_s[1], pf_s[2], pf_s[3]};
+                *reinterpret_cast<float2 *>(&sc[tid][4]) = make_float2(pf_s[4], pf_s[5]);
             }
             lds_barrier();
             if (tile > 0) request(tb - kTB, kTB);
 
             // W = dG K, Z = dG^T U, Y = F_k^T Z + (F_k - F_v)^T W of the whole tile; T_s = u_s . W_s
-            f32x4 W = kZero, Z = kZero, Y = kZero;
+            f32x4 W = kZero, Z = kZero, Y = kZero, Y2 = kZero;
             float U[CP], T = 0.f;
 #pragma unroll
             for (int i = 0; i < CP; i += 4) {
@@ -657,9 +677,10 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_sweep_kernel(
                 for (int v = 0; v < 4; v++) {
                     T = fmaf(U[i + v], w4[v], T);
                     Y = mfma4(z4[v], FTk[i + v], Y);
-                    Y = mfma4(w4[v], FTu[i + v], Y);
+                    Y2 = mfma4(w4[v], FTu[i + v], Y2);
                 }
             }
+            Y += Y2;
             T = swapadd32(T, T);
             T = swapadd16(T, T);
 
@@ -683,7 +704,7 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_sweep_kernel(
                 const float da = -keepalp * s0[2], de = dth * s0[3];
                 T_(A_DG, t, wr + ml) = fmaf(da, csA, fmaf(de, csE, fmaf(-th, ybc, dg0)));
                 lds_barrier();
-                const float dgv = T_(A_DG, t, ve), gv = T_(A_G, t, ve);
+                const float dgv = T_(A_DG, t, ve), gv = tg[t * LG + ve];
                 const f32x4 ps = *reinterpret_cast<const f32x4 *>(&Sx[wave][4 * kg]);
                 const float gml = gam[t * kTB + ml], fx = T_(A_FX, t, wr + ml);
                 const f32x4 g4 = *reinterpret_cast<const f32x4 *>(&gam[t * kTB + 4 * kg]);
@@ -756,11 +777,11 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_sweep_kernel(
                 const float ea = ml < 2 ? et[v] : 0.f;
 #pragma unroll
                 for (int jt = 0; jt < JT; jt++) {
-                    const float g = T_(A_G, t, 16 * jt + ml);
+                    const float g = tg[t * LG + 16 * jt + ml];
                     dFm[0][jt] = mfma4(dk, g, dFm[0][jt]);
                     dFm[1][jt] = mfma4(dv, g, dFm[1][jt]);
                 }
-                accEA = mfma4(ea, T_(A_G, t, wr + ml), accEA);
+                accEA = mfma4(ea, tg[t * LG + wr + ml], accEA);
             }
             if (tile > 0) {  // the chunk's first tile has no use for its dG: G_0 = I
                 f32x4 n[KT], nT[KT];
@@ -825,11 +846,11 @@ void launch(const SelfrefSweep &a) {
     check_hip(hipFuncSetAttribute(reinterpret_cast<const void *>(selfref_bwd_prepare_kernel<D>),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds), "dynamic LDS size");
     hipLaunchKernelGGL((selfref_bwd_prepare_kernel<D>), dim3(a.batch * a.nc), dim3(4 * D), lds, stream(), a.emb, a.d_y, a.k,
-                       a.v, a.q, a.alpha, a.theta, a.frozen, a.gl, a.tok, a.outer, a.csv, a.s, a.C, a.nc);
+                       a.v, a.q, a.alpha, a.theta, a.amean, a.emean, a.frozen, a.gl, a.tok, a.outer, a.csv, a.s, a.C, a.nc);
     check_launch("selfref_bwd_prepare_kernel");
     KernelTimer kt("selfref_bwd_kernel");
-    hipLaunchKernelGGL((selfref_bwd_sweep_kernel<D>), dim3(a.batch), dim3(4 * D), 0, stream(), a.emb, a.k, a.v, a.alpha,
-                       a.theta, a.amean, a.emean, a.frozen, a.gl, a.tok, a.outer, a.csv, a.d_emb, a.d_mems, a.s, a.C, a.nc);
+    hipLaunchKernelGGL((selfref_bwd_sweep_kernel<D>), dim3(a.batch), dim3(4 * D), 0, stream(), a.emb, a.k, a.v, a.frozen,
+                       a.gl, a.tok, a.outer, a.csv, a.d_emb, a.d_mems, a.s, a.C, a.nc);
     check_launch("selfref_bwd_sweep_kernel");
 }
 
