@@ -359,31 +359,52 @@ __global__ __launch_bounds__(4 * D) void selfref_scan_kernel(
 #pragma unroll
         for (int kt = 0; kt < KT; kt++) *reinterpret_cast<f32x4 *>(fb + 16 * kt) = F[kt];
         const float *K = Ks[buf], *U = Us[buf];
-        f32x4 w[ST], N[KT];
+        f32x4 w[ST], N[KT], a[2][ST];
         const float keep = keep_chunk[buf];
+        // Tiles behind the chunk's last token hold zeros.  Operands are read one step ahead: left to the compiler, every
+        // read stands right before its use.
+        auto read_w = [&](int kt, int p) __attribute__((always_inline)) {
 #pragma unroll
-        for (int kt = 0; kt < KT; kt++) N[kt] = F[kt] * keep;
+            for (int st = 0; st < ST; st++)
+                a[p][st] = *reinterpret_cast<const f32x4 *>((SG ? U : K) + (16 * st + ml) * LD + 16 * kt + 4 * kg);
+        };
+        float kb[2][KT];
+        auto read_n = [&](int i, int p) __attribute__((always_inline)) {
+#pragma unroll
+            for (int kt = 0; kt < KT; kt++) kb[p][kt] = K[(16 * (i >> 2) + 4 * kg + (i & 3)) * LD + 16 * kt + ml];
+        };
+        read_w(0, 0);
+#pragma unroll
+        for (int st = 0; st < ST; st++) w[st] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int kt = 0; kt < KT; kt++) {
+            N[kt] = F[kt] * keep;
+            if (kt + 1 < KT) read_w(kt + 1, (kt + 1) & 1);
+            else read_n(0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+#pragma unroll
+                for (int st = 0; st < ST; st++) w[st] = mfma4(a[kt & 1][st][v], F[kt][v], w[st]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
 #pragma unroll
         for (int st = 0; st < ST; st++) {
-            w[st] = f32x4{0.f, 0.f, 0.f, 0.f};
-            if (16 * st >= L) continue;
-#pragma unroll
-            for (int kt = 0; kt < KT; kt++) {
-                const f32x4 a = *reinterpret_cast<const f32x4 *>((SG ? U : K) + (16 * st + ml) * LD + 16 * kt + 4 * kg);
-#pragma unroll
-                for (int v = 0; v < 4; v++) w[st] = mfma4(a[v], F[kt][v], w[st]);
-            }
 #pragma unroll
             for (int v = 0; v < 4; v++) {
                 const int t = 16 * st + 4 * kg + v;
                 w[st][v] = cs[buf][t] * ((SG ? 0.f : U[t * LD + wr + ml]) - w[st][v]);
             }
+        }
 #pragma unroll
-            for (int v = 0; v < 4; v++) {
+        for (int i = 0; i < 4 * ST; i++) {
+            if (16 * (i >> 2) >= L) break;
+            if (i + 1 < 4 * ST) read_n(i + 1, (i + 1) & 1);
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int kt = 0; kt < KT; kt++)
-                    N[kt] = mfma4(K[(16 * st + 4 * kg + v) * LD + 16 * kt + ml], w[st][v], N[kt]);
-            }
+            for (int kt = 0; kt < KT; kt++) N[kt] = mfma4(kb[i & 1][kt], w[i >> 2][i & 3], N[kt]);
+            __builtin_amdgcn_sched_barrier(0);
         }
 #pragma unroll
         for (int kt = 0; kt < KT; kt++) F[kt] = N[kt];
@@ -476,13 +497,21 @@ __global__ __launch_bounds__(4 * D) void selfref_read_kernel(
             __builtin_amdgcn_wave_barrier();
 #pragma unroll
             for (int kt = 0; kt < KT; kt++) a[kt] = *reinterpret_cast<const f32x4 *>(row + ml * kWL + 16 * kt + 4 * kg);
+            f32x4 f[2][KT];  // the next 16 rows of the snapshot are requested before the products of the current ones
+            auto request = [&](int jt, int w) __attribute__((always_inline)) {
+#pragma unroll
+                for (int kt = 0; kt < KT; kt++)
+                    f[w][kt] = *reinterpret_cast<const f32x4 *>(Fp + (16 * jt + ml) * D + 16 * kt + 4 * kg);
+            };
+            request(0, 0);
 #pragma unroll
             for (int jt = 0; jt < KT; jt++) {
+                if (jt + 1 < KT) request(jt + 1, (jt + 1) & 1);
+                __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                 for (int kt = 0; kt < KT; kt++) {
-                    const f32x4 f = *reinterpret_cast<const f32x4 *>(Fp + (16 * jt + ml) * D + 16 * kt + 4 * kg);
 #pragma unroll
-                    for (int v = 0; v < 4; v++) h[jt] = mfma4(a[kt][v], f[v], h[jt]);
+                    for (int v = 0; v < 4; v++) h[jt] = mfma4(a[kt][v], f[jt & 1][kt][v], h[jt]);
                 }
                 float *dst = pass ? y : q_cache;
 #pragma unroll

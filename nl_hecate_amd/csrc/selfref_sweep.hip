@@ -72,7 +72,7 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_prepare_kernel(
     for (int e = tid; e < 2 * D; e += NT) {  // column sums of F_eta, F_alpha
         const float *src = fz + (size_t)(3 + e / D) * DD + (e % D);
         float a = 0.f;
-#pragma unroll 8
+#pragma unroll
         for (int c = 0; c < D; c++) a += src[c * D];
         csv[chunk * 2 * D + e] = a;
     }
@@ -85,6 +85,18 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_prepare_kernel(
         // sigmoid' of the mean over d keep (the sweep forms keep <G_t, dG_{t+1}>): a saturated gate has no gradient
         o[2] = keep > 0.f ? sa * (1.f - sa) * (1.f / D) / keep : 0.f;
         o[3] = sr_sigmoid(emean_cache[i]) * (1.f / D);  // softplus' of the mean over d
+    }
+    f32x4 in[3][TPW][KT];  // x, q, dy of the wave's tokens, requested ahead of the tables
+#pragma unroll
+    for (int i = 0; i < TPW; i++) {
+        const int li = (wave + i * NW) * kTB + ml;
+        const size_t o = (tok0 + t0 + min(li, L - 1)) * D + 4 * kg;
+#pragma unroll
+        for (int kt = 0; kt < KT; kt++) {
+            in[0][i][kt] = li < L ? *reinterpret_cast<const f32x4 *>(emb + o + 16 * kt) : kZero;
+            in[1][i][kt] = li < L ? *reinterpret_cast<const f32x4 *>(q_cache + o + 16 * kt) : kZero;
+            in[2][i][kt] = li < L ? *reinterpret_cast<const f32x4 *>(d_y + o + 16 * kt) : kZero;
+        }
     }
     // scores that no token of the chunk has, and rows behind its last token, enter products times zero
     for (int e = tid; e < 2 * kLrC * kWL + kLrC * KL; e += NT) Wq[e] = 0.f;
@@ -111,16 +123,11 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_prepare_kernel(
     f32x4 g[TPW][KT], p[TPW][KT], dq[TPW][KT];
 #pragma unroll
     for (int i = 0; i < TPW; i++) {
-        const int tile = wave + i * NW, li0 = tile * kTB, nt = min(kTB, L - li0);
+        const int tile = wave + i * NW, li0 = tile * kTB, nt = min(kTB, L - li0), tile_i = i;
 #pragma unroll
         for (int jt = 0; jt < KT; jt++) g[i][jt] = p[i][jt] = dq[i][jt] = kZero;
         if (tile >= ntile) continue;
         const size_t tk = tok0 + t0 + li0;
-        auto load = [&](const float *src, f32x4(&a)[KT]) {
-#pragma unroll
-            for (int kt = 0; kt < KT; kt++)
-                a[kt] = ml < nt ? *reinterpret_cast<const f32x4 *>(src + (tk + ml) * D + 16 * kt + 4 * kg) : kZero;
-        };
         // out = A x - sum_s th_s c_ts (x_t . L_s) R_s; the scores without th go to sc (negative with NEG)
         auto low_rank = [&](const f32x4(&a)[KT], const float *Lr, const float *R, float *sc, float sign, float *gam,
                             f32x4(&out)[KT]) {
@@ -179,22 +186,26 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_prepare_kernel(
         };
         f32x4 a[KT];
         float *out = tok + tk * TF;
-        load(emb, a);  // g = G x
-        as_result(a, g[i]);
-        low_rank(a, m.KC, m.XC, row, 1.f, out + 3 * D, g[i]);
-        load(q_cache, a);  // p = G q
-        as_result(a, p[i]);
-        low_rank(a, m.KC, m.XC, Wq + li0 * kWL, 1.f, nullptr, p[i]);
-        load(d_y, a);  // dp = F_mem^T dy, dq = G^T dp
-        f32x4 dp[KT];
+        as_result(in[0][i], g[i]);  // g = G x
+        low_rank(in[0][i], m.KC, m.XC, row, 1.f, out + 3 * D, g[i]);
+        as_result(in[1][i], p[i]);  // p = G q
+        low_rank(in[1][i], m.KC, m.XC, Wq + li0 * kWL, 1.f, nullptr, p[i]);
+        f32x4 dp[KT];  // dp = F_mem^T dy, dq = G^T dp
+        {
+            float f[2][4 * KT];  // the next 16 columns are requested before the products of the current ones
+            auto request = [&](int jt, int w) __attribute__((always_inline)) {
 #pragma unroll
-        for (int jt = 0; jt < KT; jt++) {
-            dp[jt] = kZero;
+                for (int i = 0; i < 4 * KT; i++)
+                    f[w][i] = fz[5 * DD + (16 * (i >> 2) + 4 * kg + (i & 3)) * D + 16 * jt + ml];
+            };
+            request(0, 0);
 #pragma unroll
-            for (int kt = 0; kt < KT; kt++) {
+            for (int jt = 0; jt < KT; jt++) {
+                dp[jt] = kZero;
+                if (jt + 1 < KT) request(jt + 1, (jt + 1) & 1);
+                __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int v = 0; v < 4; v++)
-                    dp[jt] = mfma4(a[kt][v], fz[5 * DD + (16 * kt + 4 * kg + v) * D + 16 * jt + ml], dp[jt]);
+                for (int i = 0; i < 4 * KT; i++) dp[jt] = mfma4(in[2][tile_i][i >> 2][i & 3], f[jt & 1][i], dp[jt]);
             }
         }
         float pp[4] = {0.f, 0.f, 0.f, 0.f};
@@ -254,7 +265,7 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_prepare_kernel(
     f32x4 dk[TPW][KT], dv[TPW][KT];
 #pragma unroll
     for (int i = 0; i < TPW; i++) {
-        const int tile = wave + i * NW, li0 = tile * kTB, nt = min(kTB, L - li0);
+        const int tile = wave + i * NW, li0 = tile * kTB, nt = min(kTB, L - li0), tile_i = i;
 #pragma unroll
         for (int jt = 0; jt < KT; jt++) dk[i][jt] = dv[i][jt] = kZero;
         if (tile >= ntile) continue;
@@ -291,30 +302,37 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_prepare_kernel(
             if (ml == 0 && 4 * kg + v < nt) out[(size_t)(4 * kg + v) * TF + 3 * D + 20] = -uw[v];
         }
         // dg0 = F_k^T dk + F_v^T dv + F_q^T dq, and F_k^T x
-        f32x4 dg[KT], fx[KT], ak[KT], av[KT], aq[KT], ax[KT];
+        f32x4 dg[KT], fx[KT], ak[KT], av[KT], aq[KT];
         put(dk[i]);
         as_operand(ak);
         put(dv[i]);
         as_operand(av);
         put(dq[i]);
         as_operand(aq);
+        float f[2][3][4 * KT];  // the next 16 columns of F_k, F_v, F_q ahead of the products of the current ones
+        auto request = [&](int jt, int w) __attribute__((always_inline)) {
 #pragma unroll
-        for (int kt = 0; kt < KT; kt++)
-            ax[kt] = ml < nt ? *reinterpret_cast<const f32x4 *>(emb + (tk + ml) * D + 16 * kt + 4 * kg) : kZero;
+            for (int c = 0; c < 3; c++) {
+#pragma unroll
+                for (int i = 0; i < 4 * KT; i++)
+                    f[w][c][i] = fz[c * DD + (16 * (i >> 2) + 4 * kg + (i & 3)) * D + 16 * jt + ml];
+            }
+        };
+        request(0, 0);
 #pragma unroll
         for (int jt = 0; jt < KT; jt++) {
+            f32x4 dg2 = kZero;
             dg[jt] = fx[jt] = kZero;
+            if (jt + 1 < KT) request(jt + 1, (jt + 1) & 1);
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int kt = 0; kt < KT; kt++) {
-#pragma unroll
-                for (int v = 0; v < 4; v++) {
-                    const float *f = fz + (16 * kt + 4 * kg + v) * D + 16 * jt + ml;
-                    dg[jt] = mfma4(ak[kt][v], f[0], dg[jt]);
-                    fx[jt] = mfma4(ax[kt][v], f[0], fx[jt]);
-                    dg[jt] = mfma4(av[kt][v], f[DD], dg[jt]);
-                    dg[jt] = mfma4(aq[kt][v], f[2 * DD], dg[jt]);
-                }
+            for (int i = 0; i < 4 * KT; i++) {
+                dg[jt] = mfma4(ak[i >> 2][i & 3], f[jt & 1][0][i], dg[jt]);
+                fx[jt] = mfma4(in[0][tile_i][i >> 2][i & 3], f[jt & 1][0][i], fx[jt]);
+                dg2 = mfma4(av[i >> 2][i & 3], f[jt & 1][1][i], dg2);
+                dg[jt] = mfma4(aq[i >> 2][i & 3], f[jt & 1][2][i], dg[jt]);
             }
+            dg[jt] += dg2;
 #pragma unroll
             for (int v = 0; v < 4; v++) {
                 if (4 * kg + v < nt) {
@@ -326,6 +344,12 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_prepare_kernel(
         }
     }
     // outer products: dF_k, dF_v, dF_q with g, dF_mem with p; stored as the sweep's lanes hold them
+    float dy[kLrC / 4];
+#pragma unroll
+    for (int i = 0; i < kLrC / 4; i++) {
+        const int li = 16 * (i >> 2) + 4 * kg + (i & 3);
+        dy[i] = li < L ? d_y[(tok0 + t0 + li) * D + wr + ml] : 0.f;
+    }
     __syncthreads();
     float *Es = lds;  // dk, dv, dq, g, p: rows of stride KL, in front of the waves' own rows
 #pragma unroll
@@ -351,13 +375,15 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_prepare_kernel(
 #pragma unroll
         for (int jt = 0; jt < KT; jt++) o[c][jt] = kZero;
     }
-    for (int st = 0; st < ntile; st++) {
+#pragma unroll
+    for (int st = 0; st < kLrC / 16; st++) {
+        if (st >= ntile) break;
 #pragma unroll
         for (int v = 0; v < 4; v++) {
             const int li = 16 * st + 4 * kg + v;
             const float *e = Es + li * KL;
             const float ak = e[wr + ml], av = e[kLrC * KL + wr + ml], aq = e[2 * kLrC * KL + wr + ml];
-            const float ay = li < L ? d_y[(tok0 + t0 + li) * D + wr + ml] : 0.f;
+            const float ay = dy[4 * st + v];
 #pragma unroll
             for (int jt = 0; jt < KT; jt++) {
                 const float bg = e[3 * kLrC * KL + 16 * jt + ml], bp = e[4 * kLrC * KL + 16 * jt + ml];
