@@ -69,10 +69,11 @@ __device__ __forceinline__ void while_true(Fn &f, std::integer_sequence<int, I..
 // lane cq then owns the columns t' = 4 j + cq of P, and column group j is finished with token 4 j + 3.
 // The row means are rows 0 (alpha), 1 (eta) and 2 (v) of a third matrix that every wave carries.
 //
-// Bound by the issue rate of one wave per SIMD (155 instructions a token) and the exchange once a token.  64 chains of
-// 2048 tokens, head size 64, chunks of 64: 1.19 ms, with the two kernels below 1.46 ms; one kernel that formed all
-// products of a token with all six memories in sequence (it serves longer chunks, selfref.hip) takes 2.30 ms.  Chunks of
-// 1, 4, 8, 16 tokens at 64 chains of 512: 6.65, 2.05, 1.28, 0.88 ms there, 3.47, 1.07, 0.67, 0.46 ms here.
+// Bound by the issue rate of one wave per SIMD (155 instructions a token at 5.3 clocks, 990 clocks a token with the
+// exchange, 6 % of the time at tile starts and ends each).  64 chains of 2048 tokens, head size 64, chunks of 64: 1.18 ms,
+// with the two kernels below 1.41 ms; one kernel that formed all products of a token with all six memories in sequence
+// (it serves longer chunks, selfref.hip) takes 2.30 ms.  Chunks of 1, 4, 8, 16 tokens at 64 chains of 512: 6.65, 2.05,
+// 1.28, 0.88 ms there, 3.47, 1.07, 0.67, 0.46 ms here.
 __host__ __device__ constexpr int sigma(int t) { return 4 * (t & 3) + (t >> 2); }
 
 template <int D, bool SG>
@@ -419,6 +420,8 @@ __global__ __launch_bounds__(4 * D) void selfref_scan_kernel(
 // q_t = F_q (G_t x_t) + H_t x_t, y_t = F_mem (G_t q_t) + H_t q_t with the shared factors in their explicit form
 // (selfref_chunk.h).  A wave takes 16 tokens through both reads by itself: the scores with the earlier keys, masked and
 // scaled, are the operand of G and H at once; its rows change layout through its own 16 rows of LDS without a barrier.
+// 116 us for 2048 chunks of 64 at head size 64, two workgroups per compute unit; 40 are matrix instructions, the rest the
+// tables at a chunk's start and the four waves' unequal numbers of earlier tokens.
 template <int D, bool SG>
 __global__ __launch_bounds__(4 * D) void selfref_read_kernel(
     const float *__restrict__ emb, const float *__restrict__ k_cache, const float *__restrict__ v_cache,

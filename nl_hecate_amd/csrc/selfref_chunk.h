@@ -67,23 +67,23 @@ __device__ __forceinline__ void chunk_setup(const ChunkLds<D> &m, const float *_
     for (int e = tid; e < L; e += NT) { m.cal[e] = alpha_cache[tok0 + t0 + e]; m.cth[e] = theta_cache[tok0 + t0 + e]; }
     __syncthreads();
     if (tid < 64) {
-        // lane t-1 builds row t of c (row L is c_L) from its diagonal leftwards:
-        // c_{t,s} = th_s P, P = prod_{s<r<t} (1-a_r); P ends as A_t.  s runs in lock step
-        // over the wave, so the gate reads are broadcasts that do not depend on the products.
-        const int t = tid + 1;
-        float P = 1.f;
-#pragma unroll 8
-        for (int s1 = kLrC - 1; s1 >= 0; s1--) {
-            const float th_s = s1 < L ? m.cth[s1] : 0.f, keep_s = s1 < L ? 1.f - m.cal[s1] : 1.f;
-            if (s1 < t && t <= L) {
-                if (t < L) m.CT[t * kLrC + s1] = THETA ? th_s * P : P;
-                else m.cL[s1] = th_s * P;
-                P *= keep_s;
-            }
+        // Lane s builds column s of c downwards, c_{t,s} = th_s prod_{s<r<t} (1-a_r), so that a row's writes fall on 64
+        // banks; the retentions come from the lanes that hold them, and A_t is their running product.
+        const bool on = tid < L;
+        const float th = on ? m.cth[tid] : 0.f, keep = on ? 1.f - m.cal[tid] : 1.f, head = THETA ? th : 1.f;
+        float P = 1.f, A = 1.f, mine = 1.f;
+#pragma unroll
+        for (int t = 0; t < kLrC; t++) {  // retention 1 behind the last token: P and A stay as they are
+            const float k = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, keep), t));
+            const bool behind = tid < t;
+            m.CT[t * kLrC + tid] = behind ? head * P : 0.f;
+            P *= behind ? k : 1.f;
+            mine = tid == t ? A : mine;
+            A *= k;
         }
-        if (t <= L) m.cA[t] = P;
-        if (t > L) m.cL[tid] = 0.f;  // c_Ls behind the chunk's last token (tid >= L)
-        if (tid == 0) m.cA[0] = 1.f;
+        m.cL[tid] = on ? th * P : 0.f;
+        if (on) m.cA[tid] = mine;
+        if (tid == 0) m.cA[L] = A;
     }
     __syncthreads();
 }
