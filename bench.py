@@ -645,7 +645,7 @@ WORKLOAD_SOURCES = {
     "titans_chunkwise_c3_f32_mnorm": ["chunkwise_mm.hip", "chunkwise_gates.hip", "chunkwise_guard.hip", "memory_rules.hip"],
     "titans_exact_c2": ["memory_rules.hip", "exact_mm.hip", "chunkwise_gates.hip"],
     "titans_exact_c2_mnorm": ["memory_rules.hip", "exact_mm.hip", "chunkwise_gates.hip", "chunkwise_guard.hip"],
-    "hope_selfref_c4": ["selfref.hip"],
+    "hope_selfref_c4": ["selfref.hip", "selfref_chain.hip", "selfref_sweep.hip"],
     "swa_c5": _SWA, "swa_stats_c5": _SWA, "swa_c5_hd32": _SWA, "swa_stats_c5_hd32": _SWA,
     "adamw_c5": ["optim.hip", "cms.hip"],
     "hebbian_c2": ["hebbian.hip"],
