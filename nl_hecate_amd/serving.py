@@ -145,6 +145,7 @@ class DecodeWorkspace:
 
 
 # level_rule of decode_token_rocm; a Titans level starts every call with zero momentum, so its one-token step is Delta's
+_DTYPE = operator.attrgetter("dtype")
 _DECODE_RULE = {"hebbian": 0, "delta": 1, "titans": 1, "dgd": 2}
 
 
@@ -187,8 +188,8 @@ def _decode_plan(params, cfg, active, context, kv_cache, ws, tensors):
 
 def _decode_in_one_call(params, cfg, token_id, pulse, context, kv_cache, ws):
     """The whole step as one library call -> logits, or None (see _decode_plan).  Checking some forty tensors and level
-    options costs as much as the step's kernels, so the workspace keeps the argument blocks together with what they were
-    made from (addresses, options, pulse) and makes one again when any of it has changed."""
+    options costs as much as the step's kernels, so the workspace keeps the argument blocks together with everything they
+    were made from (addresses, sizes, strides, types, options, pulse) and makes one again when any of it has changed."""
     k = cfg.k
     levels, lcfgs = params.levels, cfg.levels
     tensors = [params.w_embed, params.w_q, params.w_k, params.w_v, params.w_o, params.w_unembed, kv_cache.k_cache_bf16,
@@ -203,13 +204,16 @@ def _decode_in_one_call(params, cfg, token_id, pulse, context, kv_cache, ws):
                 lc.theta_ceil, lc.error_clip, lc.m_norm_max)
     active = tuple(map(bool, pulse.active_levels[:k]))
     key += map(torch.Tensor.data_ptr, tensors)
+    key += map(torch.Tensor.stride, tensors)   # a tensor can be transposed or resized where it stands
+    key += map(torch.Tensor.size, tensors)
+    key += map(_DTYPE, tensors)
+    key += (kv_cache.d, kv_cache._scratch_k.numel(), ws.logits_host.numel())
     made_for, plan = ws.plans.get(active, (None, None))
-    # the same tensor objects at the same addresses: their shapes and types are the ones that were checked
-    if made_for is None or made_for[0] != key or not all(map(operator.is_, made_for[1], tensors)):
+    if made_for != key:
         plan = _decode_plan(params, cfg, active, context, kv_cache, ws, tensors)
         if len(ws.plans) >= 16:
             ws.plans.clear()
-        ws.plans[active] = ((key, tensors), plan)
+        ws.plans[active] = (key, plan)
     if plan is None:
         return None
     weights, level_args, tail = plan

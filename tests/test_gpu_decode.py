@@ -90,3 +90,36 @@ def test_prefill_in_one_batch(rule, active, n_p, nh, hd, window, s, v, opts):
         assert not host(got.float())[s:].any()
     for lv in range(k):
         assert_close(f"memory[{lv}]", host(ctx.memory[lv]).reshape(mem[lv].shape), mem[lv], 1e-4)
+
+
+@pytest.mark.parametrize("change", ["transpose", "options"])
+def test_step_after_a_change_in_place(change):
+    """The workspace keeps the argument block of a step: a weight transposed where it stands (same tensor, address and
+    shape) or a level's option changed between two steps has to reach the second one."""
+    nh, hd, v, s = 2, 32, 50, 9
+    d = nh * hd
+    r = np.random.default_rng(5)
+    ids = r.integers(0, v, s + 2)
+    mem0 = (0.2 * r.standard_normal((nh, hd * hd))).astype(f32)
+
+    def steps(fresh):
+        gp = gpu_params(model(d, v, 1, 3))
+        cfg = SG.ServeConfig(d, v, nh, hd, 16, s, [LevelConfig("delta", nh, hd)], decode_tokens=2)
+        ctx, pulse = ContextState([dev(mem0)]), Pulse(0, [True])
+        _, kv = SG.gpu_prefill_forward(gp, cfg, ids, pulse, ctx)
+        ws = SG.DecodeWorkspace(d, v)
+        SG.gpu_single_token_forward(gp, cfg, int(ids[s]), pulse, ctx, kv, ws)
+        if change == "transpose":
+            gp.w_q.t_()
+            if fresh:
+                gp.w_q = gp.w_q.contiguous()
+        else:
+            cfg.levels[0].theta_ceil = 0.01
+        if fresh:
+            ws = SG.DecodeWorkspace(d, v)
+        out = SG.gpu_single_token_forward(gp, cfg, int(ids[s + 1]), pulse, ctx, kv, ws)
+        return out, host(ctx.memory[0])
+
+    (a, ma), (b, mb) = steps(False), steps(True)
+    assert np.abs(a - b).max() <= 2e-2 * np.abs(b).max()   # the two routes of a step round their attention to bf16
+    assert_close("memory", ma, mb, 1e-5)
