@@ -16,7 +16,8 @@
 //     G_0 = I, G_{t+1} = (1-a_t) G_t - th_t u_t k_t^T      u = k - v (self-generated
 //     H_0 = 0, H_{t+1} = (1-a_t) H_t + th_t v_t k_t^T       values: H == 0) or u = k
 // so the reverse sweep carries dG, dH (and the six dF) instead of six dM and six
-// dF.  Chunks of up to 64 tokens use the explicit (low-rank) form of G_t, H_t:
+// dF.  Chunks of up to 64 tokens (with self-generated values: selfref_sweep.hip)
+// use the explicit (low-rank) form of G_t, H_t:
 // a chunk-parallel kernel prepares every product that does not depend on the
 // sweep, the sweep kernel keeps only the per-token recurrence, and a second
 // chunk-parallel kernel turns dg, dh into d_x.  Longer chunks replay G_t, H_t
@@ -478,7 +479,8 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_kernel(
     __shared__ __align__(16) float sc[4][kTB];
     __shared__ __align__(16) float av[2][D];
     __shared__ float dEA[2][kTB];  // de_t, da_t of the tile
-    constexpr int RS = (LR && !SG) ? 6 : 4;  // vectors per token kept between the two passes of a chunk
+    static_assert(!(LR && SG), "short chunks with self-generated values: selfref_sweep.hip");
+    constexpr int RS = LR ? 6 : 4;  // vectors per token kept between the two passes of a chunk
 #define T_(a, tt, i) raw[((a) * kTB + (tt)) * TL + (i)]
 
     const int tid = threadIdx.x, r = tid >> 2, cq = tid & 3, wave = tid >> 6, lane = tid & 63;
@@ -819,10 +821,6 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_kernel(
                 *reinterpret_cast<float4 *>(&T_(A_P, stt, sj)) = *reinterpret_cast<const float4 *>(rpt + D);
                 *reinterpret_cast<float4 *>(&T_(A_DQ, stt, sj)) = *reinterpret_cast<const float4 *>(rpt + 2 * D);
                 *reinterpret_cast<float4 *>(&T_(A_DP, stt, sj)) = *reinterpret_cast<const float4 *>(rpt + 3 * D);
-                if (LR && !SG) {
-                    *reinterpret_cast<float4 *>(&T_(A_HX, stt, sj)) = *reinterpret_cast<const float4 *>(rpt + 4 * D);
-                    *reinterpret_cast<float4 *>(&T_(A_HQ, stt, sj)) = *reinterpret_cast<const float4 *>(rpt + 5 * D);
-                }
             }
             if (tid < nt) {
                 const size_t o = tok0 + tb + tid;

@@ -22,15 +22,6 @@
 namespace nlh {
 namespace {
 
-__device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
-__device__ __forceinline__ float lane_from(int byte_addr, float x) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(byte_addr, __builtin_bit_cast(int, x)));
-}
-__device__ __forceinline__ float lane_value(float x, int lane) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), lane));
-}
 template <int LANE>
 __device__ __forceinline__ void set_lane(float &x, float uniform) {
     asm("v_writelane_b32 %0, %1, %2" : "+v"(x) : "s"(uniform), "n"(LANE));
@@ -74,7 +65,6 @@ __device__ __forceinline__ void while_true(Fn &f, std::integer_sequence<int, I..
 // with the two kernels below 1.41 ms; one kernel that formed all products of a token with all six memories in sequence
 // (it serves longer chunks, selfref.hip) takes 2.30 ms.  Chunks of 1, 4, 8, 16 tokens at 64 chains of 512: 6.65, 2.05,
 // 1.28, 0.88 ms there, 3.47, 1.07, 0.67, 0.46 ms here.
-__host__ __device__ constexpr int sigma(int t) { return 4 * (t & 3) + (t >> 2); }
 
 template <int D, bool SG>
 __global__ __launch_bounds__(4 * D) void selfref_chain_kernel(

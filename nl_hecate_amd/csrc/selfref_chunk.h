@@ -8,6 +8,18 @@ namespace nlh {
 constexpr int kTB = 16;  // tokens staged in LDS at a time
 using f32x4 = float __attribute__((ext_vector_type(4)));
 
+__device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ float lane_from(int byte_addr, float x) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(byte_addr, __builtin_bit_cast(int, x)));
+}
+__device__ __forceinline__ float lane_value(float x, int lane) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), lane));
+}
+// The order in which a tile's 16 tokens are rows of a matrix product: result row 4 kg + v is token 4 v + kg.
+__host__ __device__ constexpr int sigma(int t) { return 4 * (t & 3) + (t >> 2); }
+
 // core/src/tensor.rs:202-207, 221-227.  The gates sit on the per-token critical path of the forward,
 // so exp, log and the reciprocal are the hardware approximations (v_exp_f32, v_log_f32, v_rcp_f32: about
 // one ulp each, three orders of magnitude inside the parity bar) instead of the library routines.

@@ -29,16 +29,6 @@
 namespace nlh {
 namespace {
 
-__device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
-__device__ __forceinline__ float lane_from(int byte_addr, float x) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(byte_addr, __builtin_bit_cast(int, x)));
-}
-__device__ __forceinline__ float lane_value(float x, int lane) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), lane));
-}
-__host__ __device__ constexpr int sigma(int t) { return 4 * (t & 3) + (t >> 2); }
 constexpr f32x4 kZero = {0.f, 0.f, 0.f, 0.f};
 
 // Sum over the 16 lanes of a DPP row.
