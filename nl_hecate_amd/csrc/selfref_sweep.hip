@@ -416,8 +416,7 @@ template <int I>
 __device__ __forceinline__ void fmac_spread(float &acc, float x, float m) {
     asm("v_fmac_f32_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "+v"(acc) : "v"(x), "v"(m), "n"(I));
 }
-// Two dots with x at once, two chains each.  x has to come from memory: a vector instruction that wrote it would need
-// two wait states in front of the first broadcast.
+// Two dots with x at once, two chains each.
 template <int N, int I = 0>
 __device__ __forceinline__ void dots_spread(const float (&m)[N], const float (&n)[N], float x, float (&dm)[2], float (&dn)[2]) {
     if constexpr (I < N) {
@@ -758,7 +757,10 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_sweep_kernel(
                 }
                 float gg = row_sum((CP == 16 || ml < CP) ? dgv * gv : 0.f);
                 float m2[2] = {0.f, 0.f}, a2[2] = {0.f, 0.f};
-                dots_spread<CP>(FTu, U, dgv, m2, a2);
+                // two wait states, should a vector instruction (a copy of the compiler's) have written dgv last
+                float spread = dgv;
+                asm("s_nop 1" : "+v"(spread));
+                dots_spread<CP>(FTu, U, spread, m2, a2);
                 float mv = m2[0] + m2[1], a = a2[0] + a2[1];
                 across_rows3(mv, a, gg);
                 asm volatile("" ::"v"(ps), "v"(g4));  // whole: an element without a use is not to be overwritten early
