@@ -389,6 +389,7 @@ def gpu_single_token_forward(params: GpuMAGParams, cfg: ServeConfig, token_id, p
     assert not cfg.residual, "gpu_single_token_forward: residual=true is not served by the cached-generation path"
     if not 0 <= token_id < v:
         raise ValueError(f"token_id {token_id} >= vocab_size {v}")
+    token_id = int(token_id)   # a numpy whole number or a 0-d tensor, as argmax of the logits gives
     if kv_cache.len == 0:
         raise RuntimeError("KV cache must be populated via prefill first")
     if kv_cache.len >= kv_cache.max_len:

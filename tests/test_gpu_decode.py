@@ -5,6 +5,7 @@ import types
 
 import numpy as np
 import pytest
+import torch
 
 from nl_hecate_amd import serving as SG
 from nl_hecate_amd.cms import ContextState, Pulse
@@ -123,3 +124,24 @@ def test_step_after_a_change_in_place(change):
     (a, ma), (b, mb) = steps(False), steps(True)
     assert np.abs(a - b).max() <= 2e-2 * np.abs(b).max()   # the two routes of a step round their attention to bf16
     assert_close("memory", ma, mb, 1e-5)
+
+
+@pytest.mark.parametrize("kind", [np.int64, np.int32, np.uint8, lambda t: torch.tensor(t), lambda t: torch.tensor(t).cuda(), float])
+def test_token_id_of_any_whole_number_type(kind):
+    """The greedy loop passes np.argmax of the logits on: any whole number reaches the embedding row that an int reaches."""
+    nh, hd, v, s = 2, 32, 50, 9
+    d = nh * hd
+    ids = np.random.default_rng(6).integers(0, v, s)
+    gp = gpu_params(model(d, v, 1, 4))
+    cfg = SG.ServeConfig(d, v, nh, hd, 16, s, [LevelConfig("delta", nh, hd)], decode_tokens=2)
+    mem0 = np.zeros((nh, hd * hd), f32)
+
+    def step(token):
+        ctx, pulse = ContextState([dev(mem0)]), Pulse(0, [True])
+        _, kv = SG.gpu_prefill_forward(gp, cfg, ids, pulse, ctx)
+        return SG.gpu_single_token_forward(gp, cfg, token, pulse, ctx, kv, SG.DecodeWorkspace(d, v))
+
+    assert np.array_equal(step(kind(v - 1)), step(v - 1))
+    for bad in (v, -1):
+        with pytest.raises(ValueError):
+            step(np.int64(bad))
