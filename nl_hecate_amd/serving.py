@@ -172,10 +172,11 @@ def _decode_plan(params, cfg, active, context, kv_cache, ws, tensors):
     if (any(t.shape != (d, d) for t in square) or any(t.numel() != 2 * d for t in vectors)
             or params.w_unembed.shape != (d, v) or params.w_embed.shape != (v, d)):
         return None
-    for t in tensors:   # contiguous floats; all but the scalar biases are read in 16-byte pieces
-        if t.dtype is torch.bfloat16:
-            continue
-        if t.dtype != torch.float32 or not t.is_cuda or not t.is_contiguous() or (t.numel() > 1 and t.data_ptr() & 15):
+    # contiguous on the device, read in 16-byte pieces (all but the scalar biases); floats except for the two caches
+    for i, t in enumerate(tensors):
+        cache = i in (6, 7)
+        if (t.dtype != (torch.bfloat16 if cache else torch.float32) or not t.is_cuda or not t.is_contiguous() or t.numel() == 0
+                or (t.numel() > 1 and t.data_ptr() & 15) or (cache and t.numel() < kv_cache.max_len * d)):
             return None
     work = ws.work_for(lib.decode_work_floats_rocm(d, nh, k, cfg.window_size, cfg.n_persistent))
     ptrs = [t.data_ptr() for t in tensors]

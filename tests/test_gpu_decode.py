@@ -145,3 +145,32 @@ def test_token_id_of_any_whole_number_type(kind):
     for bad in (v, -1):
         with pytest.raises(ValueError):
             step(np.int64(bad))
+
+
+def small(rule="delta", levels=1, seed=4):
+    """A prefilled model of two heads of 32 -> (params, config, pulse, context, cache, workspace)."""
+    nh, hd, v, s = 2, 32, 50, 9
+    d = nh * hd
+    gp = gpu_params(model(d, v, levels, seed))
+    cfg = SG.ServeConfig(d, v, nh, hd, 16, s, [LevelConfig(rule, nh, hd) for _ in range(levels)], decode_tokens=2)
+    ctx, pulse = ContextState([dev(np.full((nh, hd * hd), 0.01, f32)) for _ in range(levels)]), Pulse(0, [True] * levels)
+    _, kv = SG.gpu_prefill_forward(gp, cfg, np.random.default_rng(6).integers(0, v, s), pulse, ctx)
+    return gp, cfg, pulse, ctx, kv, SG.DecodeWorkspace(d, v)
+
+
+@pytest.mark.parametrize("which", ["w_q", "w_unembed", "level.w_k", "level.w_alpha", "level.b_alpha", "memory", "short cache",
+                                   "float cache"])
+def test_one_call_step_leaves_other_types_and_sizes_alone(which):
+    """Only the two caches are bf16: any other 16-bit tensor, and a cache of floats or of fewer rows than it says, is left
+    to the step by operations, which refuses it or converts."""
+    gp, cfg, pulse, ctx, kv, ws = small()
+    tensors = [gp.w_embed, gp.w_q, gp.w_k, gp.w_v, gp.w_o, gp.w_unembed, kv.k_cache_bf16, kv.v_cache_bf16]
+    lp = gp.levels[0]
+    names = dict(w_q=1, w_unembed=5) | {"level.w_k": 8, "level.w_alpha": 11, "level.b_alpha": 12, "memory": 15, "short cache": 6,
+                                        "float cache": 7}
+    tensors += [lp.w_k, lp.w_v, lp.w_q, lp.w_alpha, lp.b_alpha, lp.w_theta, lp.b_theta, ctx.memory[0]]
+    plan = lambda: SG._decode_plan(gp, cfg, (True,), ctx, kv, ws, tensors)
+    assert plan() is not None
+    t = tensors[names[which]]
+    tensors[names[which]] = t[:-1] if which == "short cache" else t.float() if which == "float cache" else t.to(torch.bfloat16)
+    assert plan() is None
