@@ -100,8 +100,7 @@ def _level_groups(params, cfg, pulse, bs, context, embedded, d):
         if not pulse.active_levels[lv] or cfg.levels[lv].memory_rule == "swiglu" or _uses_tnt(cfg, lv, bs):
             continue
         key = group_key(cfg.levels[lv], params.levels[lv], d, bs)
-        mem = context.memory[lv]
-        if key is None or not _plain(mem) or tuple(mem.shape) != (bs * cfg.num_heads, cfg.head_dim ** 2):
+        if key is None or not _plain(context.memory[lv], bs * cfg.num_heads, cfg.head_dim ** 2) or not _plain(embedded):
             continue
         by_key.setdefault(key, []).append(lv)
     return [levels[i:i + 8] for levels in by_key.values() for i in range(0, len(levels), 8)]
@@ -214,7 +213,7 @@ def gpu_cms_backward(params: GpuMAGParams, cfg: ModelConfig, cache, collect_outp
     valid = c["valid"]
     d_logits = _new(n, v)
     D.call("cross_entropy_backward_cuda", c["logits"], c["target_ids"], d_logits, n, v, 1.0 / (valid if valid > 0 else 1))
-    if v % 4 == 0 and d % 4 == 0 and _plain(params.w_unembed):   # a contraction over the vocabulary for few output tiles
+    if v % 4 == 0 and d % 4 == 0 and _plain(params.w_unembed, d, v):   # a contraction over the vocabulary for few output tiles
         d_projected = _new(n, d)
         linear_group(0, [d_logits], [params.w_unembed], [d_projected], n, d, v)
     else:
@@ -240,7 +239,8 @@ def gpu_cms_backward(params: GpuMAGParams, cfg: ModelConfig, cache, collect_outp
     for level, mc in enumerate(c["memory_caches"]):
         if mc is not None and getattr(mc, "group", None) is not None:
             groups.setdefault(id(mc.group), []).append(level)
-    groups = [lv for lv in groups.values() if len(lv) == c["memory_caches"][lv[0]].group.levels]
+    groups = [lv for lv in groups.values() if len(lv) == c["memory_caches"][lv[0]].group.levels
+              and all(group_key(cfg.levels[i], params.levels[i], d, bs) is not None for i in lv)]
     grouped = {lv for levels in groups for lv in levels}
 
     def run_group(levels, source, extra=()):
@@ -249,7 +249,7 @@ def gpu_cms_backward(params: GpuMAGParams, cfg: ModelConfig, cache, collect_outp
                               [g.levels[lv] for lv in levels], s, d, bs, extra)
 
     # without the residual path the attention's gradients join the first group's products
-    attn_group = groups[0] if groups and not cfg.residual and all(_plain(w) for w in (params.w_q, params.w_k, params.w_v)) else None
+    attn_group = groups[0] if groups and not cfg.residual and all(_plain(w, d, d) for w in (params.w_q, params.w_k, params.w_v)) else None
     d_mem_input = None
 
     def add_mem(d_emb):

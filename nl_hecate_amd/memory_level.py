@@ -279,17 +279,30 @@ def group_key(cfg, level_params, d, bs):
     if (cfg.memory_rule not in ("titans", "delta", "dgd") or cfg.memory_layers != 1 or d > 1024 or cfg.head_dim % 4
             or cfg.num_heads * cfg.head_dim != d or (cfg.proxy and cfg.memory_rule == "dgd")):
         return None
-    for t in (level_params.w_k, level_params.w_v, level_params.w_q, level_params.w_alpha, level_params.w_theta,
-              level_params.w_eta):
-        if t.dtype != torch.float32 or not t.is_contiguous() or t.data_ptr() & 15:
-            return None
+    lp, gates = level_params, 3 if cfg.memory_rule == "titans" else 2   # the momentum gate is not read without momentum
+    if (not all(_plain(t, d, d) for t in (lp.w_k, lp.w_v, lp.w_q))
+            or not all(_plain(t) and t.numel() == 2 * d for t in (lp.w_alpha, lp.w_theta, lp.w_eta)[:gates])
+            or not all(_floats(t) for t in (lp.b_alpha, lp.b_theta, lp.b_eta)[:gates])):
+        return None
     return (cfg.memory_rule, cfg.num_heads, cfg.head_dim, cfg.checkpoint_interval, cfg.proxy, cfg.chunk_size, cfg.error_clip,
             cfg.m_norm_max)
 
 
-def _plain(t):
-    """Contiguous floats at a 16-byte boundary, which the grouped kernels read."""
-    return t.dtype == torch.float32 and t.is_contiguous() and not t.data_ptr() & 15
+def _floats(t):
+    """Contiguous floats on the device: what D.call asks of a buffer."""
+    return isinstance(t, torch.Tensor) and t.is_cuda and t.dtype == torch.float32 and t.is_contiguous() and t.numel() > 0
+
+
+def _plain(t, *shape):
+    """_floats at a 16-byte boundary, which the grouped kernels read in 16-byte pieces; of this shape, if one is given."""
+    return _floats(t) and not t.data_ptr() & 15 and (not shape or tuple(t.shape) == shape)
+
+
+def _grads_plain(g, d):
+    """The gradients that backward_group writes, momentum gate included."""
+    return (all(_plain(t, d, d) for t in (g.d_w_k_mem, g.d_w_v_mem, g.d_w_q_mem))
+            and all(_floats(t) and t.numel() >= 2 * d for t in (g.d_w_alpha, g.d_w_theta, g.d_w_eta))
+            and all(_floats(t) for t in (g.d_b_alpha, g.d_b_theta, g.d_b_eta)))
 
 
 def _ptrs(tensors):
@@ -299,6 +312,11 @@ def _ptrs(tensors):
 def _bounds(cfgs):
     return (ctypes.c_float * (4 * len(cfgs)))(*[x for c in cfgs for x in (c.alpha_floor, c.alpha_ceil, c.theta_floor,
                                                                           c.theta_ceil)])
+
+
+def _gate_params(lp, titans):
+    """What level_group_inputs_f32_rocm takes of a level's gates; without momentum the last two are not read."""
+    return (lp.w_alpha, lp.b_alpha, lp.w_theta, lp.b_theta) + ((lp.w_eta, lp.b_eta) if titans else (lp.w_alpha, lp.b_alpha))
 
 
 def linear_group(op, a, b, c, m, n, k, bf16_mask=0):
@@ -329,8 +347,7 @@ def forward_group(params, cfgs, embedded, contexts, s, d, bs, extra=()):
     h0, g0 = heads.data_ptr(), gates.data_ptr()
     hs, gs = 4 * L * B * s * hd, 4 * L * B * s
     lib.level_group_inputs_f32_rocm(
-        _ptrs([t for i, lp in enumerate(params) for t in (*mem[3 * i:3 * i + 3], lp.w_alpha, lp.b_alpha, lp.w_theta,
-                                                         lp.b_theta, lp.w_eta, lp.b_eta, *rows[5 * i:5 * i + 5])]),
+        _ptrs([t for i, lp in enumerate(params) for t in (*mem[3 * i:3 * i + 3], *_gate_params(lp, titans), *rows[5 * i:5 * i + 5])]),
         _bounds(cfgs), L, h0, h0 + hs, h0 + 2 * hs, g0, g0 + gs, g0 + 2 * gs if titans else None, bs, s, nh, hd, 1e-8)
     initial = contexts[0]
     if L > 1:
@@ -436,7 +453,7 @@ def gpu_memory_forward(level_params: MemoryLevelParams, cfg: LevelConfig, embedd
             raise ValueError(f"{rule} forward with batch_size > 1 is not supported")
     elif not cfg.is_mlp_mem:
         assert tuple(context_m.shape) == (B, dd)
-    if group_key(cfg, lp, d, bs) is not None and _plain(embedded) and _plain(context_m):
+    if group_key(cfg, lp, d, bs) is not None and _plain(embedded, n, d) and _plain(context_m, B, dd):
         y, caches = forward_group([lp], [cfg], embedded, [context_m], s, d, bs)
         return y[0], caches[0]
     k_mem, v_mem, q_mem = embedded @ lp.w_k.t(), embedded @ lp.w_v.t(), embedded @ lp.w_q.t()
@@ -573,7 +590,7 @@ def gpu_memory_backward(level_params: MemoryLevelParams, cfg: LevelConfig, mem_c
     if kind == "Mlp":
         return _mlp_backward(level_params, cfg, c, d_y, embedded, level_grads, s, d, bs)
     if (c.group is not None and c.group.levels == 1 and group_key(cfg, level_params, d, bs) is not None and _plain(d_y)
-            and _plain(embedded)):
+            and d_y.numel() == n * d and _plain(embedded, n, d) and _grads_plain(level_grads, d)):
         return backward_group([level_params], [cfg], [c], d_y, embedded, [level_grads], s, d, bs)
     has_theta, has_eta = not kind.startswith("Hebbian"), kind.startswith("Titans")
     dyh = _heads(cfg, d_y, bs, s)

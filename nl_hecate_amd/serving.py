@@ -22,7 +22,7 @@ from . import dispatch as D
 from .cms import ContextState, Pulse
 from .ffi import lib
 from .mag_layer import MemoryLevelParams
-from .memory_level import F32_MAX, LevelConfig, _plain, _ptrs, gpu_memory_forward, group_key, linear_group
+from .memory_level import F32_MAX, LevelConfig, _gate_params, _plain, _ptrs, gpu_memory_forward, group_key, linear_group
 
 
 def _new(*shape, dtype=torch.float32):
@@ -314,8 +314,8 @@ def _prefill_in_batch(params, cfg, input_ids, pulse, context):
         hs, gs = 4 * L * nh * s * hd, 4 * L * nh * s
         lib.level_group_inputs_f32_rocm(
             _ptrs([t for i, lp in enumerate(lps) for t in (
-                mem[2 * i], mem[2 * i + 1], mem[2 * i], lp.w_alpha, lp.b_alpha, lp.w_theta, lp.b_theta, lp.w_eta, lp.b_eta,
-                rows[4 * i], rows[4 * i], rows[4 * i + 1], rows[4 * i + 2], rows[4 * i + 3])]),
+                mem[2 * i], mem[2 * i + 1], mem[2 * i], *_gate_params(lp, titans), rows[4 * i], rows[4 * i], rows[4 * i + 1],
+                rows[4 * i + 2], rows[4 * i + 3])]),
             (ctypes.c_float * (4 * L))(*[x for c in cfgs for x in (c.alpha_floor, c.alpha_ceil, c.theta_floor, c.theta_ceil)]), L,
             h0, h0 + hs, None, g0, g0 + gs, g0 + 2 * gs if titans else None, 1, s, nh, hd, 1e-8)
         contexts = [context.memory[lv] for lv in active]
