@@ -174,3 +174,16 @@ def test_one_call_step_leaves_other_types_and_sizes_alone(which):
     t = tensors[names[which]]
     tensors[names[which]] = t[:-1] if which == "short cache" else t.float() if which == "float cache" else t.to(torch.bfloat16)
     assert plan() is None
+
+
+def test_prefill_with_a_padded_unembedding():
+    """Columns past the vocabulary (padding to a round number) come back with the others, as from a plain product."""
+    gp, cfg, pulse, _, _, _ = small()
+    v = cfg.vocab_size
+    ids = np.random.default_rng(8).integers(0, v, cfg.seq_len)
+    memory = lambda: ContextState([dev(np.full((cfg.num_heads, cfg.head_dim ** 2), 0.01, f32))])
+    want, _ = SG.gpu_prefill_forward(gp, cfg, ids, pulse, memory())
+    gp.w_unembed = torch.cat([gp.w_unembed, torch.full((cfg.d_model, 6), 3.0, device="cuda")], 1).contiguous()
+    assert SG._prefill_in_batch(gp, cfg, ids, pulse, memory()) is None
+    got, _ = SG.gpu_prefill_forward(gp, cfg, ids, pulse, memory())
+    assert got.shape == (v + 6,) and np.abs(got[:v] - want).max() <= 2e-2 * np.abs(want).max()
