@@ -74,7 +74,9 @@ __global__ __launch_bounds__(4 * D) void selfref_chain_kernel(
     constexpr int KT = D / 16, NW = D / 16, DD = D * D, LD = D + 16, V4 = D / 4;
     __shared__ __align__(16) float xt[2][kTB * LD];
     __shared__ __align__(16) float Kt[2][kTB * LD], Vt[2][kTB * LD];  // the tile's k, v: exchange and operand
-    __shared__ __align__(16) float Ut[SG ? kTB * LD : 4];             // k - v, exchange only
+    // k - v, exchange only; two as well: a tile of one token has a single barrier, behind which a slow wave still reads its
+    // row while a fast one writes the next tile's first
+    __shared__ __align__(16) float Ut[2][SG ? kTB * LD : 4];
     __shared__ __align__(16) float Sx[NW][kTB];
     __shared__ __align__(16) float mean[3][D];
 
@@ -123,7 +125,7 @@ __global__ __launch_bounds__(4 * D) void selfref_chain_kernel(
     for (int tb = 0, buf = 0; tb < s; tb = te, buf ^= 1) {
         te = tile_end(tb);
         const int nt = te - tb;
-        float *Kb = Kt[buf], *Vb = Vt[buf];
+        float *Kb = Kt[buf], *Vb = Vt[buf], *Ub = Ut[buf];
         if (tb == chunk_t) {  // snapshot
             float *fb = frozen + (b * nc + ci) * (size_t)6 * DD;
 #pragma unroll
@@ -173,7 +175,7 @@ __global__ __launch_bounds__(4 * D) void selfref_chain_kernel(
         // token t's exchange is under way
         float s_am = 0.f, s_em = 0.f;
         float pw[3] = {0.f, 0.f, 0.f}, pkeep = 1.f;
-        float *const out = (SG ? (cq == 0 ? Kb : cq == 1 ? Vb : Ut) : (cq & 1) ? Vb : Kb) + wr + r;
+        float *const out = (SG ? (cq == 0 ? Kb : cq == 1 ? Vb : Ub) : (cq & 1) ? Vb : Kb) + wr + r;
 
         auto step = [&](auto T) __attribute__((always_inline)) -> bool {
             constexpr int t = decltype(T)::value, J = t / 4, Q = t % 4;
@@ -195,7 +197,7 @@ __global__ __launch_bounds__(4 * D) void selfref_chain_kernel(
             for (int kt = 0; kt < KT; kt++) {
                 const f32x4 k4 = *reinterpret_cast<const f32x4 *>(Kb + t * LD + 16 * kt + 4 * cq);
                 f32x4 u4 = k4;
-                if (SG) u4 = *reinterpret_cast<const f32x4 *>(Ut + t * LD + 16 * kt + 4 * cq);
+                if (SG) u4 = *reinterpret_cast<const f32x4 *>(Ub + t * LD + 16 * kt + 4 * cq);
 #pragma unroll
                 for (int i = 0; i < 4; i++) { kc[4 * kt + i] = k4[i]; uc[4 * kt + i] = u4[i]; }
             }

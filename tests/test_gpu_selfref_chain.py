@@ -23,3 +23,20 @@ def test_tile_edges(s, C, d, sg):
     ref = oracle_run(mems, x, dy, C, sg, np.float64)
     for n in ("d_emb", "d_mems"):
         assert_close(n, got[n].reshape(ref[n].shape), ref[n])
+
+
+@pytest.mark.parametrize("C", [1, 17, 33, 49])
+@pytest.mark.parametrize("d", [32, 64])
+def test_tiles_of_one_token(C, d):
+    """Chunks whose last tile is one token: its exchange and the next tile's first stand a single barrier apart, so the
+    waves of a chain must not share the exchanged row between them.  Many chains, equal ones among them: the same bits."""
+    B, s = 96, 3 * C + 1
+    mems, x, dy = inputs(2, s, d, seed=7 * C + d)
+    mems, x, dy = (np.concatenate([a] * (B // 2)) for a in (mems, x, dy))
+    got = gpu_run(mems, x, dy, C, True)
+    for n in ("y", "mems", "k", "v", "alpha", "theta"):
+        a = got[n].reshape(B // 2, -1)
+        assert (a == a[:1]).all(), n
+    want = oracle_run(mems[:2], x[:2], dy[:2], C, True, np.float32)
+    for n in ("y", "k", "v", "alpha", "theta"):
+        assert_close(n, got[n].reshape(B, -1)[:2].reshape(want[n].shape), want[n])
