@@ -171,8 +171,8 @@ __device__ __forceinline__ void level_head(const DecArgs &a, int l, int h, float
     float alpha = 1.f / (1.f + expf(-(s[2] * ki + s[3] + lv.b_alpha[0])));
     const float zt = s[4] * ki + s[5] + lv.b_theta[0];
     float theta = zt > 20.f ? zt : log1pf(expf(zt));
-    alpha = fminf(fmaxf(alpha, lv.alpha_floor), lv.alpha_ceil);
-    theta = fminf(fmaxf(theta, lv.theta_floor), lv.theta_ceil);
+    alpha = clamp_gate(alpha, lv.alpha_floor, lv.alpha_ceil, 1.f);
+    theta = clamp_gate(theta, lv.theta_floor, lv.theta_ceil, FLT_MAX);
     float u = 0.f;
 #pragma unroll
     for (int i = 0; i < NP; i++) { kv[i] = f4_scale(ki, kv[i]); qv[i] = f4_scale(qi, qv[i]); u += dot4(m[i], kv[i]); }

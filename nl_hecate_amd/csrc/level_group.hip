@@ -2,6 +2,7 @@
 // (gpu_memory_forward / gpu_memory_backward, core/src/gpu_forward.rs:1197-1540, core/src/gpu_backward.rs:459-1200,
 // 2047-2117): one launch per step for all levels instead of eleven per level forward and fifteen backward.  Each pass
 // reads and writes every [tokens, d] tensor once; one wave per token where a row is reduced.
+#include <float.h>
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -33,7 +34,7 @@ __device__ __forceinline__ float dot4f(const float4 &a, const float4 &b) { retur
 __device__ __forceinline__ float4 ld4(const float *p, int i4) { return reinterpret_cast<const float4 *>(p)[i4]; }
 __device__ __forceinline__ void st4(float *p, int i4, const float4 &x) { reinterpret_cast<float4 *>(p)[i4] = x; }
 
-// Row norms, gates (clamped), head split of k, v, q and the per-head copies of the gates.  The gate products take the raw
+// Row norms, gates (clamped where a bound is set), head split of k, v, q and the per-head copies of the gates.  The gate products take the raw
 // k and are divided by its norm afterwards, so one sweep over a token's rows serves all eight sums.
 template <int NP, bool HAS_Q, bool HAS_ETA>
 __global__ __launch_bounds__(kThr) void level_inputs_kernel(InArgs a) {
@@ -68,8 +69,8 @@ __global__ __launch_bounds__(kThr) void level_inputs_kernel(InArgs a) {
 #pragma unroll
         for (int i = 0; i < 8; i++) s[i] = wave_allreduce(s[i]);
         const float kn = sqrtf(s[0]), qn = sqrtf(s[1]), ki = 1.f / fmaxf(kn, a.eps), qi = 1.f / fmaxf(qn, a.eps);
-        const float al = fminf(fmaxf(sigmoidf_(s[2] * ki + s[3] + ba), lv.a_lo), lv.a_hi);
-        const float th = fminf(fmaxf(softplusf_(s[4] * ki + s[5] + bt), lv.t_lo), lv.t_hi);
+        const float al = clamp_gate(sigmoidf_(s[2] * ki + s[3] + ba), lv.a_lo, lv.a_hi, 1.f);
+        const float th = clamp_gate(softplusf_(s[4] * ki + s[5] + bt), lv.t_lo, lv.t_hi, FLT_MAX);
         const float et = HAS_ETA ? sigmoidf_(s[6] * ki + s[7] + be) : 0.f;
         const int b = tok / a.s, t = tok - b * a.s;
         const size_t c0 = chain0 + (size_t)b * a.nh;
@@ -356,7 +357,7 @@ void level_group_grads_f32_rocm(const void *const *ptrs, const float *bounds, in
         float *const *p = (float *const *)(ptrs + 17 * l);
         const float *b = bounds + 4 * l;
         a.lv[l] = OutLevel{p[0], p[2], p[3], p[4], p[5], p[6], p[7], p[8], p[9], p[10], b[0], b[1], b[2], b[3],
-                           b[0] > 0.f || b[1] < 1.f, b[2] > 0.f || b[3] < 3.0e38f};
+                           b[0] > 0.f || b[1] < 1.f, b[2] > 0.f || b[3] < FLT_MAX};
         g.lv[l] = GateLevel{p[0], p[1], {p[11], p[13], p[15]}, {p[12], p[14], p[16]}};
     }
     a.dkh = d_k_heads; a.dvh = d_v_heads; a.dqh = d_q_heads; a.dah = d_alpha_heads; a.dth = d_theta_heads; a.deh = d_eta_heads;

@@ -77,4 +77,10 @@ bool backward_ckpt_fused(bool has_s, bool frozen, const float *k, const float *v
                          float *d_m_initial, float *d_s_initial,
                          int seq_len, int d, int batch, int C, float m_norm_guard = 0.f);
 
+// A gate under its configured bounds, as clamp_f32_cuda forms it where the level step calls it: with a bound set only
+// (a NaN of an open gate stays one), the upper bound first.  Open: [0, 1] for alpha, [0, FLT_MAX] for theta.
+__device__ __forceinline__ float clamp_gate(float x, float lo, float hi, float open_hi) {
+    return lo > 0.f || hi < open_hi ? fmaxf(lo, fminf(hi, x)) : x;
+}
+
 }  // namespace nlh

@@ -187,3 +187,28 @@ def test_prefill_with_a_padded_unembedding():
     assert SG._prefill_in_batch(gp, cfg, ids, pulse, memory()) is None
     got, _ = SG.gpu_prefill_forward(gp, cfg, ids, pulse, memory())
     assert got.shape == (v + 6,) and np.abs(got[:v] - want).max() <= 2e-2 * np.abs(want).max()
+
+
+@pytest.mark.parametrize("gate", ["b_alpha", "w_theta"])
+@pytest.mark.parametrize("opts,finite", [({}, False), (dict(alpha_ceil=0.9, theta_ceil=2.0), True),
+                                         (dict(alpha_floor=0.8, alpha_ceil=0.3, theta_floor=0.5, theta_ceil=0.2), True)])
+def test_nan_of_a_gate_parameter(gate, opts, finite):
+    """Without bounds a NaN of a gate's parameters reaches the logits and the memory, of a token and of a prompt; bounds
+    that are set replace it (by the ceiling, or the floor where that is higher), as the clamp of the level step does."""
+    gp, cfg, pulse, ctx, kv, ws = small()
+    clean = host(ctx.memory[0])
+    for k, x in opts.items():
+        setattr(cfg.levels[0], k, x)
+    getattr(gp.levels[0], gate)[0] = float("nan")
+    step = SG.gpu_single_token_forward(gp, cfg, 3, pulse, ctx, kv, ws)
+    assert np.isfinite(step).all() == finite and np.isfinite(host(ctx.memory[0])).all() == finite
+    ids = np.arange(cfg.seq_len)
+    ctx = ContextState([dev(clean)])
+    assert SG._prefill_in_batch(gp, cfg, ids, pulse, ContextState([dev(clean)])) is not None
+    logits, _ = SG.gpu_prefill_forward(gp, cfg, ids, pulse, ctx)
+    assert np.isfinite(logits).all() == finite and np.isfinite(host(ctx.memory[0])).all() == finite
+    if gate == "b_alpha" and finite:   # the same as a bias that drives the gate to that bound
+        gp.levels[0].b_alpha[0] = 1e30
+        want = ContextState([dev(clean)])
+        SG.gpu_prefill_forward(gp, cfg, ids, pulse, want)
+        assert np.array_equal(host(ctx.memory[0]), host(want.memory[0]))

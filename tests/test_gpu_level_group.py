@@ -109,3 +109,56 @@ def test_grouped_step_against_level_by_level(rule, k, nh, hd, s, bs, kw, monkeyp
     for i, (a, b) in enumerate(zip(*out)):
         # the attention's q, k, v may round to neighbouring bf16 where the products' sums differ in their last bits
         assert np.abs(a - b).max() <= 2e-3 * max(np.abs(b).max(), 1e-6), i
+
+
+@pytest.mark.parametrize("gate", ["b_alpha", "b_theta", "w_eta"])
+def test_nan_of_a_gate_parameter_reaches_the_loss(gate):
+    cfg, _, p, mem = setup("titans", 2, 2, 32, 60, 40, 16)
+    ids = [int(t) for t in np.random.default_rng(1).integers(0, 60, 40)]
+    gp, _ = gpu_model(p)
+    getattr(gp.levels[1], gate)[0] = float("nan")
+    ctx = ContextState([dev(m.reshape(m.shape[0], -1)) for m in mem])
+    loss, cache = GM.gpu_cms_forward(gp, cfg, ids, ids, Pulse(0, [True] * 2), ctx)
+    assert cache["memory_caches"][1].group is not None
+    assert np.isnan(loss) and np.isnan(host(ctx.memory[1])).any()
+    g = GM.gpu_cms_backward(gp, cfg, cache)
+    assert np.isnan(host(g.levels[1].d_w_alpha)).any()
+
+
+def test_cross_entropy_rows_of_non_finite_logits():
+    """NaN, both infinities and the type's lowest value among the logits: as the kernel of any vocabulary size."""
+    v, n = 1024, 6
+    x = (3 * np.random.default_rng(2).standard_normal((n, v))).astype(f32)
+    x[0, 5], x[1, 7], x[2, 9] = np.nan, np.inf, -np.inf
+    x[3, :], x[4, :-1] = -np.inf, np.finfo(f32).min
+    out = []
+    for w in (v, v + 1):     # one more column, which weighs nothing: the general kernel
+        xs = np.full((n, w), -np.inf, f32)
+        xs[:, :v] = x
+        row = []
+        for i in range(n):
+            loss, g = torch.zeros(1, device="cuda"), torch.zeros(1, w, device="cuda")
+            t = dev(np.array([11], np.int32))
+            D.call("cross_entropy_forward_cuda", dev(xs[i:i + 1]), t, loss, 1, w)
+            D.call("cross_entropy_backward_cuda", dev(xs[i:i + 1]), t, g, 1, w, 0.5)
+            row.append((host(loss), host(g)[:, :v]))
+        out.append(row)
+    for i, (a, b) in enumerate(zip(*out)):
+        for p, q in zip(a, b):
+            assert np.array_equal(np.isnan(p), np.isnan(q)), i
+            assert np.allclose(p, q, rtol=1e-5, atol=1e-6, equal_nan=True), i
+
+
+@pytest.mark.parametrize("op", [0, 1, 2])
+def test_grouped_products_keep_non_finite_values_in_their_place(op):
+    m, n, k = 72, 68, 36
+    r = np.random.default_rng(9)
+    shp_a, shp_b = {0: ((m, k), (n, k)), 1: ((m, k), (k, n)), 2: ((k, m), (k, n))}[op]
+    A, B = r.standard_normal(shp_a).astype(f32), r.standard_normal(shp_b).astype(f32)
+    A[3, 5], A[6, 1], B[2, 7] = np.nan, np.inf, -np.inf
+    c = torch.zeros(m, n, device="cuda")
+    ML.linear_group(op, [dev(A)], [dev(B)], [c], m, n, k)
+    a, b = {0: (A, B.T), 1: (A, B), 2: (A.T, B)}[op]
+    with np.errstate(invalid="ignore"):
+        want = (a.astype(np.float64)[:, :, None] * b.astype(np.float64)[None]).sum(1)
+    assert np.array_equal(np.isnan(host(c)), np.isnan(want)) and np.array_equal(np.isinf(host(c)), np.isinf(want))
