@@ -450,8 +450,8 @@ class MagLayer:
                                            bs * s * d)
             out = torch.mm(gated, ops["wb"][-d:].t(), out_dtype=torch.float32).view(bs, s, d)
         else:
-            gated = _new(bs, s, d)
-            lib.cms_combine_gate_rocm(ptrs, self.k, attn.to(torch.float32).data_ptr(), None, gate.data_ptr(),
+            gated, attn_f32 = _new(bs, s, d), attn.to(torch.float32)
+            lib.cms_combine_gate_rocm(ptrs, self.k, attn_f32.data_ptr(), None, gate.data_ptr(),
                                       gated.data_ptr(), bs * s * d)
             out = (gated.view(bs * s, d) @ p.w_o.t()).view(bs, s, d)
         cache = dict(x=x, q=q, k=k, v=v, aw=aw, attn=attn, gate=gate, gated=gated, levels=caches, pulse=pulse,

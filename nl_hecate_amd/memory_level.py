@@ -366,7 +366,8 @@ def forward_group(params, cfgs, embedded, contexts, s, d, bs, extra=()):
     s_states = _new(L * B, slots, dd) if titans else None
     q = [h0, h0 + hs, h0 + 2 * hs, g0, g0 + gs]
     if titans:
-        q += [g0 + 2 * gs, initial.data_ptr(), _zeros(L * B, dd).data_ptr(), m_states.data_ptr(), s_states.data_ptr(), yh.data_ptr()]
+        s_initial = _zeros(L * B, dd)   # by name: a tensor that is gone when the call starts is another thread's to take
+        q += [g0 + 2 * gs, initial.data_ptr(), s_initial.data_ptr(), m_states.data_ptr(), s_states.data_ptr(), yh.data_ptr()]
     else:
         q += [initial.data_ptr(), m_states.data_ptr(), yh.data_ptr()]
     rule = "titans" if titans else "delta"

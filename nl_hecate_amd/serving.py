@@ -296,8 +296,8 @@ def _prefill_in_batch(params, cfg, input_ids, pulse, context):
     last = int(ids[s - 1])
     if ids.min() < 0 or ids.max() >= v:
         return None
-    embedded = _new(s, d)
-    lib.embedding_gather_cuda(params.w_embed.data_ptr(), host_ids.cuda(non_blocking=True).data_ptr(), embedded.data_ptr(), s, d)
+    embedded, dev_ids = _new(s, d), host_ids.cuda(non_blocking=True)   # by name: alive until the call has launched
+    lib.embedding_gather_cuda(params.w_embed.data_ptr(), dev_ids.data_ptr(), embedded.data_ptr(), s, d)
     kv_cache = GpuKVCache(s + cfg.decode_tokens, d, s)
     L = len(active)
     mem = list(_new(max(2 * L, 1), s, d).unbind(0))[:2 * L]

@@ -54,3 +54,42 @@ def test_gradient_buffers_that_the_grouped_backward_writes():
                     ("d_w_v_mem", torch.zeros(D // 2, D, device="cuda")), ("d_w_alpha", torch.zeros(D, device="cuda")),
                     ("d_b_theta", torch.zeros(1)), ("d_w_eta", None)):
         assert not ML._grads_plain(dataclasses.replace(ML.LevelGrads.zeros(D), **{name: t}), D), name
+
+
+@pytest.mark.gpu
+def test_tensors_live_until_the_call_has_their_addresses(monkeypatch):
+    """A library call gets addresses and releases the interpreter lock: every tensor behind them has to be alive then, or
+    another thread may be handed its memory.  Looked at from inside the calls: no address of theirs is free memory."""
+    import numpy as np
+
+    from nl_hecate_amd import serving as SG
+    from nl_hecate_amd.cms import ContextState, Pulse
+    from nl_hecate_amd.ffi import lib
+    from tests.test_gpu_serving import gpu_params
+    from tests.test_oracle_serving import model
+
+    def live(address):
+        for seg in torch.cuda.memory_snapshot():
+            at = seg["address"]
+            if at <= address < at + seg["total_size"]:
+                for block in seg["blocks"]:
+                    if at <= address < at + block["size"]:
+                        return block["state"] == "active_allocated"
+                    at += block["size"]
+        return True   # not of this allocator
+
+    names = ("embedding_gather_cuda", "titans_forward_f32_cuda", "titans_final_states_f32_rocm")
+    seen = []
+    for name in names:
+        def call(*args, fn=getattr(lib, name), name=name):
+            seen.append(name)
+            assert all(live(a) for a in args if isinstance(a, int) and a > 1 << 20), name
+            return fn(*args)
+        monkeypatch.setitem(lib.__dict__, name, call)
+    nh, hd, v, s = 2, 32, 50, 40
+    gp = gpu_params(model(nh * hd, v, 1, 3))
+    memory = lambda: torch.zeros(nh, hd * hd, device="cuda")
+    ML.gpu_memory_forward(gp.levels[0], ML.LevelConfig("titans", nh, hd), torch.randn(s, nh * hd, device="cuda"), memory(), s, nh * hd, 1)
+    cfg = SG.ServeConfig(nh * hd, v, nh, hd, 16, s, [ML.LevelConfig("titans", nh, hd)], decode_tokens=2)
+    SG.gpu_prefill_forward(gp, cfg, np.arange(s), Pulse(0, [True]), ContextState([memory()]))
+    assert set(seen) == set(names)
