@@ -279,23 +279,30 @@ def group_key(cfg, level_params, d, bs):
     if (cfg.memory_rule not in ("titans", "delta", "dgd") or cfg.memory_layers != 1 or d > 1024 or cfg.head_dim % 4
             or cfg.num_heads * cfg.head_dim != d or (cfg.proxy and cfg.memory_rule == "dgd")):
         return None
+    # written out: nine tensors a level ahead of the first launch, where a call of _plain each costs half a launch
     lp, gates = level_params, 3 if cfg.memory_rule == "titans" else 2   # the momentum gate is not read without momentum
-    if (not all(_plain(t, d, d) for t in (lp.w_k, lp.w_v, lp.w_q))
-            or not all(_plain(t) and t.numel() == 2 * d for t in (lp.w_alpha, lp.w_theta, lp.w_eta)[:gates])
-            or not all(_floats(t) for t in (lp.b_alpha, lp.b_theta, lp.b_eta)[:gates])):
-        return None
+    f32, square = torch.float32, (d, d)
+    for t in (lp.w_k, lp.w_v, lp.w_q):
+        if t.dtype is not f32 or t.shape != square or not t.is_cuda or not t.is_contiguous() or t.data_ptr() & 15:
+            return None
+    for t in (lp.w_alpha, lp.w_theta, lp.w_eta)[:gates]:
+        if t is None or t.dtype is not f32 or t.numel() != 2 * d or not t.is_cuda or not t.is_contiguous() or t.data_ptr() & 15:
+            return None
+    for t in (lp.b_alpha, lp.b_theta, lp.b_eta)[:gates]:
+        if t is None or t.dtype is not f32 or t.numel() < 1 or not t.is_cuda or not t.is_contiguous():
+            return None
     return (cfg.memory_rule, cfg.num_heads, cfg.head_dim, cfg.checkpoint_interval, cfg.proxy, cfg.chunk_size, cfg.error_clip,
             cfg.m_norm_max)
 
 
 def _floats(t):
     """Contiguous floats on the device: what D.call asks of a buffer."""
-    return isinstance(t, torch.Tensor) and t.is_cuda and t.dtype == torch.float32 and t.is_contiguous() and t.numel() > 0
+    return isinstance(t, torch.Tensor) and t.dtype is torch.float32 and t.is_cuda and t.is_contiguous() and t.numel() > 0
 
 
 def _plain(t, *shape):
     """_floats at a 16-byte boundary, which the grouped kernels read in 16-byte pieces; of this shape, if one is given."""
-    return _floats(t) and not t.data_ptr() & 15 and (not shape or tuple(t.shape) == shape)
+    return _floats(t) and not t.data_ptr() & 15 and (not shape or t.shape == shape)
 
 
 def _grads_plain(g, d):

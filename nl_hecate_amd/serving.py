@@ -283,9 +283,12 @@ def _prefill_in_batch(params, cfg, input_ids, pulse, context):
     for lv in range(k):
         lc, lp, mem = cfg.levels[lv], params.levels[lv], context.memory[lv]
         if (_DECODE_RULE.get(lc.memory_rule) is None or lc.memory_layers != 1 or (lc.num_heads, lc.head_dim) != (nh, hd)
-                or not _plain(mem, nh, hd * hd) or not all(_plain(t, d, d) for t in (lp.w_k, lp.w_v, lp.w_q))):
+                or not _plain(mem, nh, hd * hd)):
             return None
-        if pulse.active_levels[lv] and (lc.error_clip > 0 or 0 < lc.m_norm_max < 1e30 or lc.proxy):
+        if pulse.active_levels[lv]:   # its parameters have a key
+            if lc.error_clip > 0 or 0 < lc.m_norm_max < 1e30 or lc.proxy:
+                return None
+        elif not all(_plain(t, d, d) for t in (lp.w_k, lp.w_v, lp.w_q)):
             return None
     if (not _plain(params.w_embed, v, d) or not _plain(params.w_unembed, d, v)
             or not all(_plain(w, d, d) for w in (params.w_q, params.w_k, params.w_v, params.w_o))):
