@@ -130,12 +130,16 @@ class DecodeWorkspace:
         self.attn_out = _zeros(1, d)
         self.y_combined, self.gate, self.gated_out = _zeros(1, d), _zeros(1, d), _zeros(1, d)
         self.logits_gpu = _zeros(1, v)
-        # what the library's one-call step writes: intermediates of its launches, and the logits where the host reads them
+        # of the library's one-call step: intermediates of its launches, its argument blocks, the logits where the host
+        # reads them
         self.work = _new(0)
         self.plans = {}
         self.logits_host = torch.empty(v, dtype=torch.float32, pin_memory=True)
-        self.outputs = (ctypes.c_void_p * 7)(*[t.data_ptr() for t in (
-            self.embedded, self.q_bf16, self.attn_out_bf16, self.attn_out, self.y_combined, self.gate, self.gated_out)])
+
+    def written(self):
+        """What the one-call step writes besides the logits on the host, in the order of its argument block."""
+        return (self.embedded, self.q_bf16, self.attn_out_bf16, self.attn_out, self.y_combined, self.gate, self.gated_out,
+                self.logits_gpu)
 
     def work_for(self, floats):
         if self.work.numel() < floats:
@@ -154,7 +158,14 @@ def _decode_plan(params, cfg, active, context, kv_cache, ws, tensors):
     head sizes): those take the step below, operation by operation."""
     d, nh, hd, v, k = cfg.d_model, cfg.num_heads, cfg.head_dim, cfg.vocab_size, cfg.k
     if (hd not in (32, 64, 128) or nh * hd != d or d > 4096 or not 1 <= k <= 8 or kv_cache._scratch_k.numel() < d
-            or kv_cache.d != d or ws.logits_host.numel() != v):
+            or kv_cache.d != d):
+        return None
+    for i, t in enumerate(ws.written()):
+        if (t.dtype != (torch.bfloat16 if i in (1, 2) else torch.float32) or not t.is_cuda or not t.is_contiguous()
+                or tuple(t.shape) != (1, v if i == 7 else d) or t.data_ptr() & 15):
+            return None
+    host = ws.logits_host
+    if host.dtype != torch.float32 or host.is_cuda or not host.is_pinned() or not host.is_contiguous() or host.shape != (v,):
         return None
     square, vectors = [params.w_q, params.w_k, params.w_v, params.w_o], []
     rules, bounds = [], []
@@ -182,8 +193,9 @@ def _decode_plan(params, cfg, active, context, kv_cache, ws, tensors):
     ptrs = [t.data_ptr() for t in tensors]
     weights = ptrs[1:6]
     level_args = ((ctypes.c_void_p * (8 * k))(*ptrs[8:]), (ctypes.c_int * k)(*rules), (ctypes.c_float * (6 * k))(*bounds))
-    tail = (kv_cache.k_cache_bf16.data_ptr(), kv_cache.v_cache_bf16.data_ptr(), work.data_ptr(), ws.outputs,
-            ws.logits_gpu.data_ptr(), ws.logits_host.data_ptr())
+    written = [t.data_ptr() for t in ws.written()]
+    tail = (kv_cache.k_cache_bf16.data_ptr(), kv_cache.v_cache_bf16.data_ptr(), work.data_ptr(), (ctypes.c_void_p * 7)(*written[:7]),
+            written[7], ws.logits_host.data_ptr())
     return weights, level_args, tail
 
 
@@ -208,7 +220,10 @@ def _decode_in_one_call(params, cfg, token_id, pulse, context, kv_cache, ws):
     key += map(torch.Tensor.stride, tensors)   # a tensor can be transposed or resized where it stands
     key += map(torch.Tensor.size, tensors)
     key += map(_DTYPE, tensors)
-    key += (kv_cache.d, kv_cache._scratch_k.numel(), ws.logits_host.numel())
+    written = ws.written()
+    key += map(torch.Tensor.data_ptr, written)
+    key += map(torch.Tensor.numel, written)
+    key += (kv_cache.d, kv_cache._scratch_k.numel(), ws.logits_host.numel(), ws.logits_host.data_ptr())
     made_for, plan = ws.plans.get(active, (None, None))
     if made_for != key:
         plan = _decode_plan(params, cfg, active, context, kv_cache, ws, tensors)

@@ -212,3 +212,18 @@ def test_nan_of_a_gate_parameter(gate, opts, finite):
         want = ContextState([dev(clean)])
         SG.gpu_prefill_forward(gp, cfg, ids, pulse, want)
         assert np.array_equal(host(ctx.memory[0]), host(want.memory[0]))
+
+
+@pytest.mark.parametrize("name", ["logits_gpu", "embedded", "gated_out", "attn_out_bf16", "logits_host"])
+def test_step_after_a_workspace_buffer_was_replaced(name):
+    """The kept argument block holds the workspace's addresses: a buffer put in another's place is the one written."""
+    gp, cfg, pulse, ctx, kv, ws = small()
+    first = ctx.memory[0].clone()
+    want = SG.gpu_single_token_forward(gp, cfg, 3, pulse, ctx, kv, ws)
+    old, filled = getattr(ws, name), host(getattr(ws, name).clone().float())
+    setattr(ws, name, torch.zeros_like(old, pin_memory=name == "logits_host"))
+    old.fill_(7.0)
+    ctx.memory[0].copy_(first)
+    kv.len -= 1
+    assert np.array_equal(SG.gpu_single_token_forward(gp, cfg, 3, pulse, ctx, kv, ws), want)
+    assert np.array_equal(host(getattr(ws, name).float()), filled) and (host(old.float()) == 7.0).all()
