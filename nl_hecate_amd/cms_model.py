@@ -26,7 +26,7 @@ from .cms import ContextState, Pulse
 from .ffi import lib
 from .memory_level import (LevelConfig, LevelGrads, _plain, _ptrs, backward_group, forward_group, gpu_memory_backward,
                            gpu_memory_forward, group_key, linear_group)
-from .serving import GpuMAGParams, frozen_level_output
+from .serving import GpuMAGParams, frozen_level_output, host_ids
 from .tnt import ParallelConfig, gpu_tnt_backward, gpu_tnt_forward
 
 LN_EPS = 1e-5
@@ -38,10 +38,6 @@ def _new(*shape, dtype=torch.float32):
 
 def _zeros(*shape, dtype=torch.float32):
     return torch.zeros(*shape, dtype=dtype, device="cuda")
-
-
-def _host_ids(ids):
-    return np.asarray(ids.cpu() if isinstance(ids, torch.Tensor) else ids).astype(np.int32, copy=False)
 
 
 @dataclass
@@ -120,9 +116,9 @@ def gpu_cms_forward(params: GpuMAGParams, cfg: ModelConfig, input_ids, target_id
         raise ValueError("residual=True needs the LayerNorm parameters")
     n = bs * s
     # one pinned buffer for both, copied without waiting for the work in front of it
-    tgt_host = _host_ids(target_ids)
+    tgt_host = host_ids(target_ids)
     both = torch.empty(2 * n, dtype=torch.int32, pin_memory=True)
-    both.numpy()[:n] = _host_ids(input_ids)
+    both.numpy()[:n] = host_ids(input_ids)
     both.numpy()[n:] = tgt_host
     ids, tgt = both.cuda(non_blocking=True).split(n)
     embedded = _new(n, d)

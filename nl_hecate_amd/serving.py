@@ -33,6 +33,20 @@ def _zeros(*shape, dtype=torch.float32):
     return torch.zeros(*shape, dtype=dtype, device="cuda")
 
 
+def host_ids(ids):
+    """Token ids as int32 on the host.  Whatever does not fit is refused, not wrapped; other numbers go through int()."""
+    if isinstance(ids, torch.Tensor):
+        ids = ids.cpu()
+    elif isinstance(ids, (list, tuple)) and ids and isinstance(ids[0], torch.Tensor):
+        ids = [int(t) for t in ids]
+    a = np.asarray(ids)
+    if a.dtype.kind not in "iu":
+        a = np.array([int(t) for t in a], dtype=np.int64 if not a.size else None)
+    if a.dtype.itemsize >= 4 and a.dtype != np.int32 and a.size and not -2 ** 31 <= a.min() <= a.max() < 2 ** 31:
+        raise RuntimeError("token id cannot be converted to int32 without overflow")
+    return a.astype(np.int32, copy=False)
+
+
 @dataclass
 class GpuMAGParams:
     """The tensors the generation path reads (GpuMAGParams: swa block + levels)."""
@@ -308,13 +322,13 @@ def _prefill_in_batch(params, cfg, input_ids, pulse, context):
     if (not _plain(params.w_embed, v, d) or not _plain(params.w_unembed, d, v)
             or not all(_plain(w, d, d) for w in (params.w_q, params.w_k, params.w_v, params.w_o))):
         return None
-    host_ids = torch.empty(s, dtype=torch.int32, pin_memory=True)
-    ids = host_ids.numpy()
-    ids[:] = np.asarray(input_ids[:s].cpu() if isinstance(input_ids, torch.Tensor) else input_ids[:s])
+    pinned = torch.empty(s, dtype=torch.int32, pin_memory=True)
+    ids = pinned.numpy()
+    ids[:] = host_ids(input_ids[:s])
     last = int(ids[s - 1])
     if ids.min() < 0 or ids.max() >= v:
         return None
-    embedded, dev_ids = _new(s, d), host_ids.cuda(non_blocking=True)   # by name: alive until the call has launched
+    embedded, dev_ids = _new(s, d), pinned.cuda(non_blocking=True)   # by name: alive until the call has launched
     lib.embedding_gather_cuda(params.w_embed.data_ptr(), dev_ids.data_ptr(), embedded.data_ptr(), s, d)
     kv_cache = GpuKVCache(s + cfg.decode_tokens, d, s)
     L = len(active)
