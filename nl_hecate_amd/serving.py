@@ -162,6 +162,12 @@ class DecodeWorkspace:
         return self.work
 
 
+def _keys_fit(cfg, pos):
+    """The one-call step merges its slices of 128 keys in 64 KB of LDS: model width + slices * heads floats."""
+    keys = min(pos + 1, cfg.window_size + cfg.n_persistent)
+    return cfg.d_model + -(-keys // 128) * cfg.num_heads <= 16384
+
+
 # level_rule of decode_token_rocm; a Titans level starts every call with zero momentum, so its one-token step is Delta's
 _DTYPE = operator.attrgetter("dtype")
 _DECODE_RULE = {"hebbian": 0, "delta": 1, "titans": 1, "dgd": 2}
@@ -203,7 +209,7 @@ def _decode_plan(params, cfg, active, context, kv_cache, ws, tensors):
         if (t.dtype != (torch.bfloat16 if cache else torch.float32) or not t.is_cuda or not t.is_contiguous() or t.numel() == 0
                 or (t.numel() > 1 and t.data_ptr() & 15) or (cache and t.numel() < kv_cache.max_len * d)):
             return None
-    work = ws.work_for(lib.decode_work_floats_rocm(d, nh, k, cfg.window_size, cfg.n_persistent))
+    work = ws.work_for(lib.decode_work_floats_rocm(d, nh, k, min(cfg.window_size, kv_cache.max_len), cfg.n_persistent))
     ptrs = [t.data_ptr() for t in tensors]
     weights = ptrs[1:6]
     level_args = ((ctypes.c_void_p * (8 * k))(*ptrs[8:]), (ctypes.c_int * k)(*rules), (ctypes.c_float * (6 * k))(*bounds))
@@ -218,6 +224,8 @@ def _decode_in_one_call(params, cfg, token_id, pulse, context, kv_cache, ws):
     options costs as much as the step's kernels, so the workspace keeps the argument blocks together with everything they
     were made from (addresses, sizes, strides, types, options, pulse) and makes one again when any of it has changed."""
     k = cfg.k
+    if not _keys_fit(cfg, kv_cache.len):
+        return None
     levels, lcfgs = params.levels, cfg.levels
     tensors = [params.w_embed, params.w_q, params.w_k, params.w_v, params.w_o, params.w_unembed, kv_cache.k_cache_bf16,
                kv_cache.v_cache_bf16]
@@ -237,7 +245,7 @@ def _decode_in_one_call(params, cfg, token_id, pulse, context, kv_cache, ws):
     written = ws.written()
     key += map(torch.Tensor.data_ptr, written)
     key += map(torch.Tensor.numel, written)
-    key += (kv_cache.d, kv_cache._scratch_k.numel(), ws.logits_host.numel(), ws.logits_host.data_ptr())
+    key += (kv_cache.d, kv_cache.max_len, kv_cache._scratch_k.numel(), ws.logits_host.numel(), ws.logits_host.data_ptr())
     made_for, plan = ws.plans.get(active, (None, None))
     if made_for != key:
         plan = _decode_plan(params, cfg, active, context, kv_cache, ws, tensors)
@@ -305,6 +313,8 @@ def _prefill_in_batch(params, cfg, input_ids, pulse, context):
     s, d, nh, hd, v, k = cfg.seq_len, cfg.d_model, cfg.num_heads, cfg.head_dim, cfg.vocab_size, cfg.k
     if hd not in (32, 64, 128) or nh * hd != d or d > 1024 or not 1 <= k <= 8 or s < 1 or params.w_embed.shape != (v, d):
         return None
+    if not _keys_fit(cfg, s - 1):
+        return None
     active = [lv for lv in range(k) if pulse.active_levels[lv]]
     keys = {group_key(cfg.levels[lv], params.levels[lv], d, 1) for lv in active}
     if len(keys) > 1 or None in keys:
@@ -365,7 +375,7 @@ def _prefill_in_batch(params, cfg, input_ids, pulse, context):
     # the last position as a decode step at a cache row that holds its K and V already
     level_ptrs = [t.data_ptr() for lv in range(k) for lp in (params.levels[lv],) for t in (
         lp.w_k, lp.w_v, lp.w_q, lp.w_alpha, lp.b_alpha, lp.w_theta, lp.b_theta, context.memory[lv])]
-    work = _new(lib.decode_work_floats_rocm(d, nh, k, cfg.window_size, cfg.n_persistent) + 7 * d + v)
+    work = _new(lib.decode_work_floats_rocm(d, nh, k, min(cfg.window_size, s), cfg.n_persistent) + 7 * d + v)
     w0 = work.data_ptr()
     row, step = w0 + 4 * (work.numel() - 7 * d - v) // 16 * 16, 4 * d
     outputs = (ctypes.c_void_p * 7)(*[row + i * step for i in range(7)])

@@ -10,6 +10,7 @@ import torch
 from nl_hecate_amd import serving as SG
 from nl_hecate_amd.cms import ContextState, Pulse
 from nl_hecate_amd.ffi import lib
+from nl_hecate_amd.mag_layer import MemoryLevelParams
 from nl_hecate_amd.memory_level import LevelConfig
 from oracle import serving as SV
 from tests.gpu_util import assert_close, dev, host
@@ -227,3 +228,32 @@ def test_step_after_a_workspace_buffer_was_replaced(name):
     kv.len -= 1
     assert np.array_equal(SG.gpu_single_token_forward(gp, cfg, 3, pulse, ctx, kv, ws), want)
     assert np.array_equal(host(getattr(ws, name).float()), filled) and (host(old.float()) == 7.0).all()
+
+
+def test_windows_past_what_one_call_merges():
+    """head-slices of 128 keys beyond the merge's LDS go step by operations; a window without an end costs no memory."""
+    nh, hd, v, s = 128, 32, 8, 12400    # 97 slices of 128 heads and a width of 4096: 128 floats past 64 KB
+    d = nh * hd
+    cfg = SG.ServeConfig(d, v, nh, hd, 1 << 30, s, [LevelConfig("hebbian", nh, hd)])
+    assert not SG._keys_fit(cfg, s - 1) and SG._keys_fit(cfg, 96 * 128 - 1)
+    g = torch.Generator(device="cuda").manual_seed(1)
+    r = lambda *sh: torch.randn(*sh, generator=g, device="cuda") * 0.02
+    gp = SG.GpuMAGParams(r(v, d), r(d, d), r(d, d), r(d, d), r(d, d), r(d, v),
+                         [MemoryLevelParams(r(d, d), r(d, d), r(d, d), r(2 * d), r(1), r(2 * d), r(1), r(2 * d), r(1))])
+    kv = SG.GpuKVCache(s + 4, d, 1)
+    kv.k_cache_bf16.copy_(r(s + 4, d) * 50)
+    kv.v_cache_bf16.copy_(r(s + 4, d) * 50)
+    out = []
+    for window, start in ((16000, s), (1 << 30, 96 * 128 - 2)):
+        cfg.window_size, kv.len = window, start
+        ws = SG.DecodeWorkspace(d, v)
+        ctx = ContextState([torch.zeros(nh, hd * hd, device="cuda")])
+        out.append(SG.gpu_single_token_forward(gp, cfg, 1, Pulse(0, [True]), ctx, kv, ws))
+        assert bool(ws.plans) == (start < s) and ws.work.numel() < 1 << 20
+        q, keys = (host(x.float()).astype(np.float64) for x in (ws.q_bf16, kv.k_cache_bf16[:start + 1]))
+        w = np.einsum("hc,thc->ht", q.reshape(nh, hd), keys.reshape(-1, nh, hd)) / np.sqrt(hd)
+        w = np.exp(w - w.max(1, keepdims=True))
+        w /= w.sum(1, keepdims=True)
+        want = np.einsum("ht,thc->hc", w, host(kv.v_cache_bf16[:start + 1].float()).reshape(-1, nh, hd))
+        assert np.abs(host(ws.attn_out).reshape(nh, hd) - want).max() <= 2e-2 * np.abs(want).max()
+    assert np.isfinite(out).all()
