@@ -413,24 +413,33 @@ void level_group_heads_repeat_rocm(const float *x, float *out, int bs, int s, in
 }
 
 void saxpy_multi_rocm(float alpha, const float *const *x, float *const *y, const int *n, int count) {
-    for (int c0 = 0; c0 < count; c0 += kMaxSaxpy) {
-        SaxpyArgs a;
-        a.alpha = alpha;
-        a.count = 0;
-        int blocks = 0;
-        for (int i = c0; i < count && i < c0 + kMaxSaxpy; i++) {
-            if (n[i] <= 0) continue;
-            a.x[a.count] = x[i];
-            a.y[a.count] = y[i];
-            a.n[a.count] = n[i];
-            a.first[a.count++] = blocks;
-            blocks += ceil_div(n[i], kSaxpyPer);
-        }
-        if (!blocks) continue;
+    SaxpyArgs a;
+    a.alpha = alpha;
+    a.count = 0;
+    int blocks = 0;
+    auto flush = [&] {
+        if (!blocks) return;
         a.first[a.count] = blocks;
         hipLaunchKernelGGL(saxpy_multi_kernel, dim3(blocks), dim3(kThr), 0, stream(), a);
         check_launch("saxpy_multi_kernel");
+        a.count = blocks = 0;
+    };
+    auto meet = [](const float *p, int np, const float *q, int nq) { return p < q + nq && q < p + np; };
+    for (int i = 0; i < count; i++) {
+        if (n[i] <= 0) continue;
+        // pairs in one launch run beside each other: one that writes or reads what another writes (levels that share their
+        // parameters) comes after it
+        bool apart = a.count == kMaxSaxpy;
+        for (int j = 0; j < a.count && !apart; j++)
+            apart = meet(y[i], n[i], a.y[j], a.n[j]) || meet(x[i], n[i], a.y[j], a.n[j]) || meet(y[i], n[i], a.x[j], a.n[j]);
+        if (apart) flush();
+        a.x[a.count] = x[i];
+        a.y[a.count] = y[i];
+        a.n[a.count] = n[i];
+        a.first[a.count++] = blocks;
+        blocks += ceil_div(n[i], kSaxpyPer);
     }
+    flush();
 }
 
 }  // extern "C"

@@ -60,6 +60,20 @@ def test_saxpy_multi():
     assert np.array_equal(host(shifted), np.array([0, 0, -0.25, -0.5, -0.75, -1.0, 0, 0], f32))
 
 
+def test_saxpy_multi_of_shared_tensors():
+    """A tensor that two pairs update takes both updates, and one that a later pair reads is read updated, as pair by pair."""
+    r = np.random.default_rng(4)
+    y, x = r.standard_normal(9000).astype(f32), [r.standard_normal(9000).astype(f32) for _ in range(3)]
+    for _ in range(5):
+        yd, xd = dev(y), [dev(t) for t in x]
+        ys, xs, n = [yd, yd, yd[4000:], xd[1]], [xd[0], xd[1], xd[2], yd], [9000, 9000, 5000, 9000]
+        lib.saxpy_multi_rocm(0.5, ML._ptrs(xs), ML._ptrs(ys), (ctypes.c_int * 4)(*n), 4)
+        want = (y + f32(0.5) * x[0]) + f32(0.5) * x[1]
+        want[4000:] += f32(0.5) * x[2][:5000]
+        assert np.abs(host(yd) - want).max() <= 2e-6
+        assert np.abs(host(xd[1]) - (x[1] + f32(0.5) * want)).max() <= 2e-6
+
+
 @pytest.mark.parametrize("s,v", [(5, 1024), (3, 8192), (4, 8196), (2, 32768), (3, 16388), (2, 32772)])
 def test_cross_entropy_rows(s, v):
     r = np.random.default_rng(v)
