@@ -92,6 +92,9 @@ def _uses_tnt(cfg, level, bs):
 def _level_groups(params, cfg, pulse, bs, context, embedded, d):
     """The active levels that run as batches (equal options, at most eight to a batch): lists of level numbers."""
     by_key = {}
+    at = [m.data_ptr() for m in context.memory[:cfg.k] if isinstance(m, torch.Tensor) and m.numel()]
+    if len(set(at)) < len(at):   # levels that share a memory take it in turn
+        return []
     for lv in range(cfg.k):
         if not pulse.active_levels[lv] or cfg.levels[lv].memory_rule == "swiglu" or _uses_tnt(cfg, lv, bs):
             continue

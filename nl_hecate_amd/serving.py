@@ -209,6 +209,8 @@ def _decode_plan(params, cfg, active, context, kv_cache, ws, tensors):
         if (t.dtype != (torch.bfloat16 if cache else torch.float32) or not t.is_cuda or not t.is_contiguous() or t.numel() == 0
                 or (t.numel() > 1 and t.data_ptr() & 15) or (cache and t.numel() < kv_cache.max_len * d)):
             return None
+    if len({m.data_ptr() for m in context.memory[:k]}) < k:   # levels that share a memory take it in turn
+        return None
     work = ws.work_for(lib.decode_work_floats_rocm(d, nh, k, min(cfg.window_size, kv_cache.max_len), cfg.n_persistent))
     ptrs = [t.data_ptr() for t in tensors]
     weights = ptrs[1:6]
@@ -329,6 +331,8 @@ def _prefill_in_batch(params, cfg, input_ids, pulse, context):
                 return None
         elif not all(_plain(t, d, d) for t in (lp.w_k, lp.w_v, lp.w_q)):
             return None
+    if len({m.data_ptr() for m in context.memory[:k]}) < k:
+        return None
     if (not _plain(params.w_embed, v, d) or not _plain(params.w_unembed, d, v)
             or not all(_plain(w, d, d) for w in (params.w_q, params.w_k, params.w_v, params.w_o))):
         return None

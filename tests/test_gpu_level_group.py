@@ -176,3 +176,17 @@ def test_grouped_products_keep_non_finite_values_in_their_place(op):
     with np.errstate(invalid="ignore"):
         want = (a.astype(np.float64)[:, :, None] * b.astype(np.float64)[None]).sum(1)
     assert np.array_equal(np.isnan(host(c)), np.isnan(want)) and np.array_equal(np.isinf(host(c)), np.isinf(want))
+
+
+def test_levels_that_share_a_memory_take_it_in_turn():
+    cfg, _, p, mem = setup("delta", 2, 2, 32, 60, 20, 16)
+    ids = [int(t) for t in np.random.default_rng(1).integers(0, 60, 20)]
+    gp, _ = gpu_model(p)
+    one = dev(mem[0].reshape(mem[0].shape[0], -1))
+    first = one.clone()
+    loss, cache = GM.gpu_cms_forward(gp, cfg, ids, ids, Pulse(0, [True] * 2), ContextState([one, one]))
+    # the second level starts from what the first one left
+    y0, c0 = ML.gpu_memory_forward(gp.levels[0], cfg.levels[0], cache["embedded"], first, 20, 64, 1)
+    y1, c1 = ML.gpu_memory_forward(gp.levels[1], cfg.levels[1], cache["embedded"], first, 20, 64, 1)
+    for got, want in ((cache["y_per_level"][0], y0), (cache["y_per_level"][1], y1), (one, first)):
+        assert np.array_equal(host(got), host(want))
