@@ -97,11 +97,16 @@ __global__ __launch_bounds__(64 * WM * WN) void group_gemm_kernel(GroupArgs g) {
         ra.load(g.a[j] + (OP == 2 ? (size_t)k0 * lda + m0 : (size_t)m0 * lda + k0), lda, g.m - m0, ks);
         rb.load(g.b[j] + (OP == 0 ? (size_t)n0 * ldb + k0 : (size_t)k0 * ldb + n0), ldb, g.n - n0, ks);
     };
-    f32x4 acc[TM][TN];
+    // A sum over products adds whole products: one running sum over all of their terms rounds like a contraction of that
+    // length (seven of 1024: 7.6e-7 of the result instead of 5.7e-7).
+    f32x4 acc[TM][TN], sum[OP == 1 ? TM : 1][OP == 1 ? TN : 1];
 #pragma unroll
     for (int i = 0; i < TM; i++)
 #pragma unroll
-        for (int j = 0; j < TN; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int j = 0; j < TN; j++) {
+            acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+            if constexpr (OP == 1) sum[i][j] = acc[i][j];
+        }
     if (s0 < s1) load(s0);
     for (int s = s0; s < s1; s++) {
         const int buf = (s - s0) & 1;
@@ -126,6 +131,20 @@ __global__ __launch_bounds__(64 * WM * WN) void group_gemm_kernel(GroupArgs g) {
 #pragma unroll
                     for (int j = 0; j < TN; j++)
                         acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[h][i][e], bv[h][j][e], acc[i][j], 0, 0, 0);
+        if constexpr (OP == 1) {
+            if ((s + 1) % per_seg == 0 || s + 1 == s1) {
+#pragma unroll
+                for (int i = 0; i < TM; i++)
+#pragma unroll
+                    for (int j = 0; j < TN; j++) { sum[i][j] += acc[i][j]; acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f}; }
+            }
+        }
+    }
+    if constexpr (OP == 1) {
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int j = 0; j < TN; j++) acc[i][j] = sum[i][j];
     }
     const bool part = g.splits > 1, b16 = OP == 0 && ((g.bf16_mask >> blockIdx.y) & 1);
     float *c = part ? g.part + (size_t)blockIdx.z * g.m * g.n : reinterpret_cast<float *>(g.c[OP == 1 ? 0 : blockIdx.y]);

@@ -45,6 +45,20 @@ def test_grouped_products(op, count, m, n, k):
             assert (h.float() - got).abs().max().item() <= 2 ** -7 * got.abs().max().item()
 
 
+@pytest.mark.parametrize("count,m,n,k", [(7, 1000, 1024, 1024), (6, 2000, 512, 512), (12, 512, 512, 512)])
+def test_sum_over_products_rounds_like_products_added_up(count, m, n, k):
+    g = torch.Generator(device="cuda").manual_seed(1)
+    a, b = [[torch.randn(*s, generator=g, device="cuda") for _ in range(count)] for s in ((m, k), (k, n))]
+    c, one = torch.zeros(m, n, device="cuda"), a[0] @ b[0]
+    ML.linear_group(1, a, b, [c], m, n, k)
+    for x, y in zip(a[1:], b[1:]):
+        one.addmm_(x, y)
+    want = sum(x.double() @ y.double() for x, y in zip(a, b))
+    err = lambda t: ((t.double() - want).norm() / want.norm()).item()
+    # each product rounds like one of the library's, and the sums over products add to that on both sides
+    assert err(c) <= 1.05 * err(one)
+
+
 def test_saxpy_multi():
     r = np.random.default_rng(3)
     sizes = [1, 3, 4096, 4097, 5, 100000, 64] * 10
