@@ -50,7 +50,8 @@ struct FirstSum {
     int batch, per, rows, nsum, elems;   // elems = d*d, a multiple of 256
 };
 
-template <bool HAS_S>
+// T: type of the running values and sums (the rows in between are kept in float either way).
+template <bool HAS_S, class T>
 __global__ __launch_bounds__(64 * kGateWaves) void cw_gates_sweep_kernel(
     const float *__restrict__ alpha, const float *__restrict__ eta, const float *__restrict__ pvec,
     const float *__restrict__ xs, const float *__restrict__ scal, float *__restrict__ d_alpha,
@@ -73,17 +74,22 @@ __global__ __launch_bounds__(64 * kGateWaves) void cw_gates_sweep_kernel(
     const size_t tok = (size_t)chain * s + t0;
     const bool in = lane < L;
     const float keep_l = in ? 1.f - alpha[tok + lane] : 1.f;
+    const float alpha_l = in ? alpha[tok + lane] : 0.f;
+    auto keep_at = [&](int t) -> T {
+        if constexpr (sizeof(T) == 8) return 1.0 - (double)bcast(alpha_l, t);
+        else return bcast(keep_l, t);
+    };
     const float eta_l = (HAS_S && in) ? eta[tok + lane] : 0.f;
     const float4 pv = in ? *reinterpret_cast<const float4 *>(pvec + (tok + lane) * 4) : make_float4(0.f, 0.f, 0.f, 0.f);
     const float m0dm = scal[(size_t)task * 4 + 0], s0dm = scal[(size_t)task * 4 + 1], s0ds = scal[(size_t)task * 4 + 2];
     const float *x = xs + (size_t)task * GW * GW + lane;
 
     // ── sweep 1: lane = t ──
-    float u = pv.x, v = pv.y;              // <M_s, dy_t q_t^T>, <S_s, dy_t q_t^T>
-    float um = m0dm, vm = s0dm, vs = s0ds; // <M_s, dMo>, <S_s, dMo>, <S_s, dSo> (wave-uniform)
-    float pum = um, pvm = vm, pvs = vs;    // their values at s = lane - 1
-    U[lane] = u;
-    if (HAS_S) V[lane] = v;
+    T u = pv.x, v = pv.y;                  // <M_s, dy_t q_t^T>, <S_s, dy_t q_t^T>
+    T um = m0dm, vm = s0dm, vs = s0ds;     // <M_s, dMo>, <S_s, dMo>, <S_s, dSo> (wave-uniform)
+    T pum = um, pvm = vm, pvs = vs;        // their values at s = lane - 1
+    U[lane] = (float)u;
+    if (HAS_S) V[lane] = (float)v;
     // The whole column of per-token terms is requested up front.  Row s is used at t >= s only, and the
     // producer leaves out the 16 x 16 tiles that lie entirely below that: those are neither read nor used.
     float xr[GW];
@@ -97,24 +103,23 @@ __global__ __launch_bounds__(64 * kGateWaves) void cw_gates_sweep_kernel(
         }
 #pragma unroll
     for (int sx = 0; sx < GW; sx++) {
-        const float xv = xr[sx];
-        const float kp = bcast(keep_l, sx), g1 = bcast(pv.z, sx);
+        const T xv = xr[sx], kp = keep_at(sx), g1 = bcast(pv.z, sx);
         if (HAS_S) {
-            const float et = bcast(eta_l, sx), g2 = bcast(pv.w, sx);
-            v = fmaf(et, v, xv);
-            vm = fmaf(et, vm, g1);
-            vs = fmaf(et, vs, g2);
+            const T et = bcast(eta_l, sx), g2 = bcast(pv.w, sx);
+            v = fma(et, v, xv);
+            vm = fma(et, vm, g1);
+            vs = fma(et, vs, g2);
         } else {
             v = xv;
             vm = g1;
         }
-        u = fmaf(kp, u, v);
-        um = fmaf(kp, um, vm);
+        u = fma(kp, u, v);
+        um = fma(kp, um, vm);
         if (sx + 1 < GW) {
             // row sx + 1, columns t >= sx + 1; the other lanes store to the spare row (no branch in the sweep)
             const int dst = lane >= sx + 1 ? tri_row(sx + 1) - (sx + 1) + lane : GTRI - GW + lane;
-            U[dst] = u;
-            if (HAS_S) V[dst] = v;
+            U[dst] = (float)u;
+            if (HAS_S) V[dst] = (float)v;
             if (lane == sx + 1) { pum = um; pvm = vm; pvs = vs; }
         }
     }
@@ -123,27 +128,27 @@ __global__ __launch_bounds__(64 * kGateWaves) void cw_gates_sweep_kernel(
     __builtin_amdgcn_wave_barrier();
 
     // ── sweep 2: lane = s; weights r[s][t], c[t][s], bb[s][t] advance with t ──
-    float rho = 1.f, cc = 1.f, bb = 1.f, accA = 0.f, accE = 0.f;
+    T rho = 1, cc = 1, bb = 1, accA = 0, accE = 0;
     // row s seen from column 0: what it reads at t < s belongs to earlier rows and is weighted by zero
     const float *Ur = U + tri_row(lane) - lane, *Vr = V + tri_row(lane) - lane;
     // unrolled by 8 only: fully unrolled, the lane reads of both sweeps (four scalars per step) overflowed the scalar
     // register file and were spilled
 #pragma unroll 8
     for (int t = 0; t < GW; t++) {
-        const float kp = bcast(keep_l, t);
+        const T kp = keep_at(t);
         const bool after = t > lane && t < L, on = t >= lane;   // tokens beyond a short chunk change no weight
-        rho *= after ? kp : 1.f;
-        accA = fmaf(on ? rho : 0.f, Ur[t], accA);
+        rho *= after ? kp : T(1);
+        accA = fma(on ? rho : T(0), T(Ur[t]), accA);
         if (HAS_S) {
-            const float et = bcast(eta_l, t);
-            bb *= after ? et : 1.f;
-            cc = after ? fmaf(kp, cc, bb) : cc;
-            accE = fmaf(on ? cc : 0.f, Vr[t], accE);
+            const T et = bcast(eta_l, t);
+            bb *= after ? et : T(1);
+            cc = after ? fma(kp, cc, bb) : cc;
+            accE = fma(on ? cc : T(0), T(Vr[t]), accE);
         }
     }
     if (in) {
-        d_alpha[tok + lane] = -fmaf(rho, pum, accA);
-        if (HAS_S) d_eta[tok + lane] = accE + cc * pvm + bb * pvs;
+        d_alpha[tok + lane] = -(float)fma(rho, pum, accA);
+        if (HAS_S) d_eta[tok + lane] = (float)(accE + cc * pvm + bb * pvs);
     }
 }
 
@@ -152,18 +157,20 @@ __global__ __launch_bounds__(64 * kGateWaves) void cw_gates_sweep_kernel(
 void chunkwise_gate_gradients(const float *alpha, const float *eta, const float *pvec, const float *xs,
                               const float *scal, float *d_alpha, float *d_eta, int seq_len, int batch,
                               int chunk_size, bool has_s, const float *dm_first, const float *ds_first,
-                              size_t chain_stride, int per, int nsum, float *tmp, int elems) {
+                              size_t chain_stride, int per, int nsum, float *tmp, int elems, bool wide) {
     const ErrorScope es;
     const int nc = ceil_div(seq_len, chunk_size), ntask = batch * nc;
     const size_t lds = (size_t)kGateWaves * (has_s ? 2 : 1) * GTRI * sizeof(float);
     static bool attr_set = false;
     if (!attr_set) {
-        check_hip(hipFuncSetAttribute(reinterpret_cast<const void *>(cw_gates_sweep_kernel<true>),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)(kGateWaves * 2 * GTRI * 4)),
-                  "dynamic LDS size");
-        check_hip(hipFuncSetAttribute(reinterpret_cast<const void *>(cw_gates_sweep_kernel<false>),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)(kGateWaves * GTRI * 4)),
-                  "dynamic LDS size");
+        auto lds_of = [](const void *kernel, int chunks_of) {
+            check_hip(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kGateWaves * chunks_of * GTRI * 4),
+                      "dynamic LDS size");
+        };
+        lds_of(reinterpret_cast<const void *>(cw_gates_sweep_kernel<true, float>), 2);
+        lds_of(reinterpret_cast<const void *>(cw_gates_sweep_kernel<false, float>), 1);
+        lds_of(reinterpret_cast<const void *>(cw_gates_sweep_kernel<true, double>), 2);
+        lds_of(reinterpret_cast<const void *>(cw_gates_sweep_kernel<false, double>), 1);
         attr_set = true;
     }
     if (es.failed()) return;
@@ -172,12 +179,10 @@ void chunkwise_gate_gradients(const float *alpha, const float *eta, const float 
     const FirstSum fs{{dm_first, ds_first}, tmp, chain_stride, batch, per, rows, nsum, elems};
     const dim3 grid(sweep_blocks + (elems / 256) * rows * nsum), block(64 * kGateWaves);
     KernelTimer kt("cw_gates_sweep_kernel");
-    if (has_s)
-        hipLaunchKernelGGL(cw_gates_sweep_kernel<true>, grid, block, lds, stream(), alpha, eta, pvec, xs, scal, d_alpha,
-                           d_eta, seq_len, chunk_size, nc, ntask, sweep_blocks, fs);
-    else
-        hipLaunchKernelGGL(cw_gates_sweep_kernel<false>, grid, block, lds, stream(), alpha, nullptr, pvec, xs, scal,
-                           d_alpha, nullptr, seq_len, chunk_size, nc, ntask, sweep_blocks, fs);
+    auto kernel = has_s ? (wide ? cw_gates_sweep_kernel<true, double> : cw_gates_sweep_kernel<true, float>)
+                        : (wide ? cw_gates_sweep_kernel<false, double> : cw_gates_sweep_kernel<false, float>);
+    hipLaunchKernelGGL(kernel, grid, block, lds, stream(), alpha, has_s ? eta : nullptr, pvec, xs, scal, d_alpha,
+                       has_s ? d_eta : nullptr, seq_len, chunk_size, nc, ntask, sweep_blocks, fs);
     check_launch("cw_gates_sweep_kernel");
 }
 

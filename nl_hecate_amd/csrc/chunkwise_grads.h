@@ -56,10 +56,12 @@ void titans_chunkwise_backward_bf16_tokens_g16(const uint16_t *k_mem, const uint
                                                int batch_size, int chunk_size, int heads, int levels, int d_y_per_level);
 
 // also runs the first stage of the batch sum of the initial-state gradients: tmp [nsum][ceil(batch / per)][64*64]
-// receives the sums of `per` consecutive chains of dm_first (and ds_first when nsum = 2), [batch][chain_stride]
+// receives the sums of `per` consecutive chains of dm_first (and ds_first when nsum = 2), [batch][chain_stride];
+// wide: the sweeps' running values in float64
 void chunkwise_gate_gradients(const float *alpha, const float *eta, const float *pvec, const float *xs,
                               const float *scal, float *d_alpha, float *d_eta, int seq_len, int batch,
                               int chunk_size, bool has_s, const float *dm_first, const float *ds_first,
-                              size_t chain_stride, int per, int nsum, float *tmp, int elems = 64 * 64);
+                              size_t chain_stride, int per, int nsum, float *tmp, int elems = 64 * 64,
+                              bool wide = false);
 
 }  // namespace nlh

@@ -5,7 +5,7 @@
 namespace nlh {
 
 // Backward from states kept every C <= 64 tokens, m_ckpt / s_ckpt [batch][n_ckpt_count(seq_len, C)][d*d] (C = 1: the full
-// trajectory).
+// trajectory).  Sums in float64 at head size 32 and from full trajectories, in fp32 otherwise.
 bool exact_mm_applies(int d, int C);
 // faster than the sequential kernel at this shape (tested: under a clip or a bound)
 bool exact_backward_mm_pays(int seq_len, int batch, int d, int C, bool tested, bool frozen);
@@ -23,7 +23,8 @@ bool exact_backward_mm(const char *fn, bool has_s, bool frozen, int d, const flo
 // (chain stride m_stride; s_initial null: zero).  No clip, no projection.  The runs' tokens are then independent walks
 // (FwdArgs::sub_chunks).  sstep 0: the states after the last token instead.
 constexpr int kExactChunk = 64;
-bool exact_forward_mm_pays(int seq_len, int batch, int d, bool final_only, int run);
+// kept_bytes: states that the walk of the tokens writes
+bool exact_forward_mm_pays(int seq_len, int batch, int d, bool final_only, int run, long long kept_bytes);
 void exact_forward_states(bool has_s, bool frozen, int d, int run, const float *k, const float *v, const float *alpha, const float *theta,
                           const float *eta, const float *m_initial, const float *s_initial, long long m_stride, float *m_states,
                           float *s_states, long long state_stride, int sstep, int seq_len, int input_stride, int batch);

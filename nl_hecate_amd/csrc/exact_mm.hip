@@ -33,10 +33,23 @@
 // taken against the chunk-start memory, i.e. T = I, am = 1, bm = 0, and the terms through Lam are absent.  Serves head
 // size 32, which the chunkwise matrix kernels of chunkwise_mm.hip do not have.
 //
+// P64: which sums are float64 (mm_tiles.h).  The walks that this form stands in for add a row's product up in a tree and
+// are 0.6 to 1.2e-7 off the exact gradients (gates spread over (0, 1); 2 to 4e-7 where the states live for 150 tokens); with
+// fp32 sums throughout the form is at 1.5 to 2.6e-7.  So wherever a walk was replaced, head size 32, full trajectories
+// and the forward's chunk maps, the coefficients' recurrences, the gate sweeps and every product whose rounding reaches a
+// result are float64 sums rounded once: 0.6 to 1.0e-7, each output at or below its walk over spread gates, gates at a
+// model's start and long-lived states.  Left in fp32 are the products that do not show: the inverse, K K^T, K M^T, the maps
+// of the adjoint scan and the products with the adjoint at the chunk's end.  512 tokens of 32 chains, head size 64: first
+// kernel 38 -> 46 us, gradients 38 -> 65, scan 16 -> 23, gates 10 -> 15; head size 32, 777 tokens of 16: 21 -> 25, 24 -> 32,
+// 5 -> 8, 7 -> 9.  Checkpointed head size 64 keeps fp32 sums: it never replaced a more exact path at these entry points, and
+// its two kernels are bound by their products.
+//
 // Under a finite m_norm_max / error clip the pass also leaves the ChainTracks of chunkwise_chain.h behind (|u_t|^2 per
 // token, sums of squares of the checkpoints); the caller tests on them whether a coupling could have fired.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+
+#include <type_traits>
 
 #include "chunkwise_chain.h"
 #include "chunkwise_grads.h"
@@ -60,6 +73,17 @@ using namespace mmt;
 #define NLH_STRIP_ORIGIN() \
     const int w = threadIdx.x >> 6; \
     NLH_STRIP_ORIGIN_OF(w)
+
+// Sums of the products: fp32 or float64 (mm_tiles.h).
+template <bool P64> using real = std::conditional_t<P64, double, float>;
+template <bool P64, class FA, class FB>
+__device__ __forceinline__ void product(Strip &acc, FA a, FB b, int l) {
+    if constexpr (P64) mma_f64(acc, a, b, l); else mma(acc, a, b, l);
+}
+template <bool P64, class FA, class FB>
+__device__ __forceinline__ void product_range(Strip &acc, FA a, FB b, int p0, int p1, int l) {
+    if constexpr (P64) mma_range_f64(acc, a, b, p0, p1, l); else mma_range(acc, a, b, p0, p1, l);
+}
 
 // per chunk, for the scan: Phi_MM, Phi_SM, Phi_MS, Phi_SS (source state, destination state), C_M, C_S
 constexpr size_t kExLocMats = 6;
@@ -130,7 +154,7 @@ __device__ __forceinline__ void chunk_vectors(ChunkVecs &cv, const Coef &cf, int
 }
 
 // ── pass 1: chunk-local matrices ────────────────────────────────────────────
-template <int D, bool FROZEN, bool TRACK>
+template <int D, bool FROZEN, bool TRACK, bool P64>
 __global__ __launch_bounds__(kThr) void ex_local_kernel(
     const float *__restrict__ k, const float *__restrict__ v, const float *__restrict__ q, const float *__restrict__ d_y,
     const float *__restrict__ alpha, const float *__restrict__ theta, const float *__restrict__ eta,
@@ -170,11 +194,12 @@ __global__ __launch_bounds__(kThr) void ex_local_kernel(
     int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     asm volatile("" : "+s"(w));
     NLH_STRIP_ORIGIN_OF(w);
-    auto MMA = [&](Strip &acc, auto fa, auto fb) { mma(acc, fa, fb, l); };
-    auto MMAR = [&](Strip &acc, auto fa, auto fb, int p0, int p1) { mma_range(acc, fa, fb, p0, p1, l); };
+    auto MMA = [&](Strip &acc, auto fa, auto fb) { product<P64>(acc, fa, fb, l); };
+    auto MMAR = [&](Strip &acc, auto fa, auto fb, int p0, int p1) { product_range<P64>(acc, fa, fb, p0, p1, l); };
     auto MMAT = [&](f32x4 &acc, auto fa, auto fb, int k0) { mma_tile16(acc, fa, fb, k0, l); };
     // over the head size
-    auto MMD = [&](Strip &acc, auto fa, auto fb) { if constexpr (D == 64) mma(acc, fa, fb, l); else mma_range(acc, fa, fb, 0, D / 32, l); };
+    auto MMD = [&](Strip &acc, auto fa, auto fb) { if constexpr (D == 64) MMA(acc, fa, fb); else MMAR(acc, fa, fb, 0, D / 32); };
+    auto MMD32 = [&](Strip &acc, auto fa, auto fb) { if constexpr (D == 64) mma(acc, fa, fb, l); else mma_range(acc, fa, fb, 0, D / 32, l); };
     const bool dcol = D == 64 || nh == 0;   // this wave's strip lies inside a token x head-size product
     auto FORC = [&](Strip &acc, auto f) { for_c(acc, f, l); };
     const int chain = itask / nc, ci = itask % nc, t0 = ci * C, L = min(C, s - t0);
@@ -182,7 +207,7 @@ __global__ __launch_bounds__(kThr) void ex_local_kernel(
     (void)t0;
     {
         load_gates(cf, gt);
-        coefficients(cf, gt, L, Cc, nullptr, nullptr);
+        coefficients<real<P64>>(cf, gt, L, Cc, nullptr, nullptr);
         commit(Ks, tk, tid);
         commit(Vs, tv, tid);
         commit(Qs, tq, tid);
@@ -199,9 +224,9 @@ __global__ __launch_bounds__(kThr) void ex_local_kernel(
     {
         Strip g = zero_strip(), km = zero_strip(), ks = zero_strip(), p = zero_strip();
         auto aK = [&](int m, int kk) { return Ks[(m0 + m) * LDM + kk]; };
-        if (!FROZEN) MMD(g, aK, [&](int kk, int n) { return Ks[(n0 + n) * LDM + kk]; });
-        if (dcol) MMD(km, aK, [&](int kk, int n) { return Ms[(n0 + n) * LDM + kk]; });
-        if (!FROZEN && dcol && has_s) MMD(ks, aK, [&](int kk, int n) { return Ss[(n0 + n) * LDM + kk]; });
+        if (!FROZEN) MMD32(g, aK, [&](int kk, int n) { return Ks[(n0 + n) * LDM + kk]; });
+        if (dcol) MMD32(km, aK, [&](int kk, int n) { return Ms[(n0 + n) * LDM + kk]; });
+        if (!FROZEN && dcol && has_s) MMD32(ks, aK, [&](int kk, int n) { return Ss[(n0 + n) * LDM + kk]; });
         MMD(p, [&](int m, int kk) { return Qs[(m0 + m) * LDM + kk]; }, [&](int kk, int n) { return Ks[(n0 + n) * LDM + kk]; });
         __syncthreads();   // the vectors are there
 #pragma unroll
@@ -256,8 +281,8 @@ __global__ __launch_bounds__(kThr) void ex_local_kernel(
         // T is lower triangular: row block ib contracts over the first ib + 1 blocks of 16 (taken in pairs)
         const int pe = (ib >> 1) + 1;
         MMAR(u, aT, [&](int kk, int n) { return Vs[kk * LDM + n0 + n]; }, 0, pe);
-        MMAR(z1, aT, [&](int kk, int n) { return cv.am[kk] * Ks[kk * LDM + n0 + n]; }, 0, pe);
-        if (has_s) MMAR(z2, aT, [&](int kk, int n) { return cv.bm[kk] * Ks[kk * LDM + n0 + n]; }, 0, pe);
+        mma_range(z1, aT, [&](int kk, int n) { return cv.am[kk] * Ks[kk * LDM + n0 + n]; }, 0, pe, l);
+        if (has_s) mma_range(z2, aT, [&](int kk, int n) { return cv.bm[kk] * Ks[kk * LDM + n0 + n]; }, 0, pe, l);
         float *go = Ug + task * kDD;
         FORC(u, [&](int r, int c, float &x) { go[(m0 + r) * HD + n0 + c] = x; });
         FORC(z1, [&](int r, int c, float &x) { B8[(m0 + r) * LDM + n0 + c] = x; });
@@ -284,7 +309,7 @@ __global__ __launch_bounds__(kThr) void ex_local_kernel(
         const float *wv = (o & 1) ? cv.wS : cv.wM, *Z = FROZEN ? Ks : (o & 2) ? Ms : B8;
         Strip x = zero_strip();
         if (!(FROZEN && (o & 2)))
-            MMA(x, [&](int m, int kk) { return wv[kk] * Ks[kk * LDM + sm0 + m]; }, [&](int kk, int n) { return Z[kk * LDM + sn0 + n]; });
+            mma(x, [&](int m, int kk) { return wv[kk] * Ks[kk * LDM + sm0 + m]; }, [&](int kk, int n) { return Z[kk * LDM + sn0 + n]; }, l);
         if (on_diag) {   // the chunk's own decay
             const float dg = o == 0 ? aL : o == 2 ? bL : o == 3 ? hL : 0.f;
             FORC(x, [&](int r, int c, float &y) { if (sm0 + r == sn0 + c) y += dg; });
@@ -296,7 +321,7 @@ __global__ __launch_bounds__(kThr) void ex_local_kernel(
     for (int o = o0; o < (has_s ? 2 : 1); o += ostep) {   // C_M = (a.dY)^T Q + dU_loc^T Z1,  C_S = (beta.dY)^T Q + dU_loc^T Z2
         const float *vec = o ? cf.beta : cf.a, *Z = FROZEN ? Ks : o ? Ms : B8;
         Strip x = zero_strip();
-        MMA(x, [&](int m, int kk) { return vec[kk] * Ds[kk * LDM + sm0 + m]; }, [&](int kk, int n) { return Qs[kk * LDM + sn0 + n]; });
+        MMA(x, [&](int m, int kk) { return (real<P64>)vec[kk] * Ds[kk * LDM + sm0 + m]; }, [&](int kk, int n) { return Qs[kk * LDM + sn0 + n]; });
         if (!(FROZEN && o))
             MMA(x, [&](int m, int kk) { return B9[kk * LDM + sm0 + m]; }, [&](int kk, int n) { return Z[kk * LDM + sn0 + n]; });
 #pragma unroll
@@ -321,7 +346,7 @@ constexpr size_t kExLocalLds = 9 * MAT * sizeof(float);
 // Bound by the step's own chain: LDS read, 2 D / 4 matrix instructions on each of two waves per SIMD, LDS write, barrier.
 // 64 chains x 32 chunks, head size 64: 84 -> 78 us (four source / destination waves that swapped tiles through LDS,
 // two barriers a step and loads one step ahead before).
-template <int D, bool HAS_S, bool REV>
+template <int D, bool HAS_S, bool REV, bool P64>
 __global__ __launch_bounds__((HAS_S ? 2 : 1) * D * 4) void ex_scan_kernel(
     const float *__restrict__ loc, const float *__restrict__ m_initial, const float *__restrict__ s_initial, long long m_stride,
     float *__restrict__ mst, float *__restrict__ sst, long long state_stride, int sstep, float *__restrict__ first_m,
@@ -363,26 +388,30 @@ __global__ __launch_bounds__((HAS_S ? 2 : 1) * D * 4) void ex_scan_kernel(
         r.c = p[(4 + dst) * (DD / 4) + (rb * NT + ct) * 64];
     };
     auto step = [&](Step &r, int i) {
-        const float *Xr = X[i & 1][0] + (l & 15) * LDX + (D / 4) * (l >> 4);
+        const float *Xr = X[i & 1][0] + (P64 ? f64_row(l) : l & 15) * LDX + (D / 4) * (l >> 4);
         f32x4 a[NS][NB];
 #pragma unroll
         for (int sr = 0; sr < NS; sr++)
 #pragma unroll
             for (int j = 0; j < NB; j++) a[sr][j] = *reinterpret_cast<const f32x4 *>(Xr + sr * 16 * LDX + 4 * j);
-        f32x4 acc[2] = {r.c, {0.f, 0.f, 0.f, 0.f}};
+        using Acc = std::conditional_t<P64, f64x4, f32x4>;
+        Acc acc[2] = {Acc{r.c[0], r.c[1], r.c[2], r.c[3]}, Acc{0, 0, 0, 0}};
 #pragma unroll
         for (int j = 0; j < NB; j++)
 #pragma unroll
             for (int sr = 0; sr < NS; sr++)
 #pragma unroll
-                for (int e = 0; e < 4; e++)
-                    acc[HAS_S ? sr : e & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[sr][j][e], r.b[sr][j][e], acc[HAS_S ? sr : e & 1], 0, 0, 0);
+                for (int e = 0; e < 4; e++) {
+                    Acc &to = acc[HAS_S ? sr : e & 1];
+                    if constexpr (P64) to = __builtin_amdgcn_mfma_f64_16x16x4f64((double)a[sr][j][e], (double)r.b[sr][j][e], to, 0, 0, 0);
+                    else to = __builtin_amdgcn_mfma_f32_16x16x4f32(a[sr][j][e], r.b[sr][j][e], to, 0, 0, 0);
+                }
         request(r, i + 2);
         float *Xw = X[(i + 1) & 1][dst] + rw * LDX + col;
         const size_t slot = REV ? (size_t)(nc - 1 - i) * DD : (size_t)(i + 1) * sstep * DD;
 #pragma unroll
         for (int e = 0; e < 4; e++) {
-            x[e] = acc[0][e] + acc[1][e];
+            x[e] = (float)(acc[0][e] + acc[1][e]);
             Xw[e * LDX] = x[e];
             st[slot + e * D] = x[e];
         }
@@ -408,7 +437,7 @@ __global__ __launch_bounds__((HAS_S ? 2 : 1) * D * 4) void ex_scan_kernel(
 // ── pass 3: gradients of one chunk ──────────────────────────────────────────
 //   pvec [chain][token][4] = <M0, J_t>, <S0, J_t>, -theta_t u_t^T dMo k_t, -theta_t u_t^T dSo k_t
 //   xs [chain][chunk][s][t] as above     scal [chunk][4] = <M0, dMo>, <S0, dMo>, <S0, dSo>
-template <int D, bool FROZEN>
+template <int D, bool FROZEN, bool P64>
 __global__ __launch_bounds__(kThr) void ex_grads_kernel(
     const float *__restrict__ k, const float *__restrict__ q, const float *__restrict__ d_y, const float *__restrict__ alpha,
     const float *__restrict__ theta, const float *__restrict__ eta, const float *__restrict__ m_ckpt,
@@ -422,7 +451,7 @@ __global__ __launch_bounds__(kThr) void ex_grads_kernel(
           *Cc = A2 + MAT, *B9 = Cc + MAT;
     __shared__ Coef cf;
     __shared__ ChunkVecs cv;
-    __shared__ float part[6][2][CW];   // row sums per column half: p0, ps, g1, g2, dam, dbm
+    __shared__ float part[7][2][CW];   // row sums per column half: p0, ps, g1, g2, dam, dbm, u.dR
     __shared__ float part_th[4][CW];   // column sums of dW.c per 16-row block
     __shared__ float dots[3][8];
     // Persistent over a contiguous range of chunks, as ex_local_kernel: the next chunk's nine tiles are requested at the
@@ -460,16 +489,17 @@ __global__ __launch_bounds__(kThr) void ex_grads_kernel(
     int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     asm volatile("" : "+s"(w));
     NLH_STRIP_ORIGIN_OF(w);
-    auto MMA = [&](Strip &acc, auto fa, auto fb) { mma(acc, fa, fb, l); };
-    auto MMAR = [&](Strip &acc, auto fa, auto fb, int p0, int p1) { mma_range(acc, fa, fb, p0, p1, l); };
+    auto MMA = [&](Strip &acc, auto fa, auto fb) { product<P64>(acc, fa, fb, l); };
+    auto MMAR = [&](Strip &acc, auto fa, auto fb, int p0, int p1) { product_range<P64>(acc, fa, fb, p0, p1, l); };
     auto FORC = [&](Strip &acc, auto f) { for_c(acc, f, l); };
-    auto MMD = [&](Strip &acc, auto fa, auto fb) { if constexpr (D == 64) mma(acc, fa, fb, l); else mma_range(acc, fa, fb, 0, D / 32, l); };
+    auto MMD = [&](Strip &acc, auto fa, auto fb) { if constexpr (D == 64) MMA(acc, fa, fb); else MMAR(acc, fa, fb, 0, D / 32); };
+    auto MMD32 = [&](Strip &acc, auto fa, auto fb) { if constexpr (D == 64) mma(acc, fa, fb, l); else mma_range(acc, fa, fb, 0, D / 32, l); };
     const bool dcol = D == 64 || nh == 0;   // this wave's strip lies inside a token x head-size product
     const int chain = itask / nc, ci = itask % nc, t0 = ci * C, L = min(C, s - t0);
     const size_t tok = (size_t)chain * s + t0, task = (size_t)itask;
     fetch_b(itask, tid);
     load_gates(cf, gt);
-    coefficients(cf, gt, L, Cc, nullptr, nullptr);
+    coefficients<real<P64>>(cf, gt, L, Cc, nullptr, nullptr);
     commit(Ks, tk, tid);
     commit(Qs, tq, tid);
     commit(Ds, td, tid);
@@ -478,7 +508,7 @@ __global__ __launch_bounds__(kThr) void ex_grads_kernel(
     auto aK = [&](int m, int kk) { return Ks[(m0 + m) * LDM + kk]; };
     Strip p = zero_strip(), g = zero_strip();   // Q K^T and K K^T while the other tiles are in flight
     MMD(p, [&](int m, int kk) { return Qs[(m0 + m) * LDM + kk]; }, [&](int kk, int n) { return Ks[(n0 + n) * LDM + kk]; });
-    if (!FROZEN) MMD(g, aK, [&](int kk, int n) { return Ks[(n0 + n) * LDM + kk]; });
+    if (!FROZEN) MMD32(g, aK, [&](int kk, int n) { return Ks[(n0 + n) * LDM + kk]; });
     {
         if (!FROZEN) commit(Ts, tt, tid);
         commit(Us, tu, tid);
@@ -505,13 +535,14 @@ __global__ __launch_bounds__(kThr) void ex_grads_kernel(
     Strip udm = zero_strip(), uds = zero_strip();
     if (dcol) {
         Strip kdm = zero_strip(), kds = zero_strip();
-        MMD(kdm, aK, [&](int kk, int n) { return A1[(n0 + n) * LDM + kk]; });
-        MMD(udm, aU, [&](int kk, int n) { return A1[kk * LDM + n0 + n]; });
+        MMD32(kdm, aK, [&](int kk, int n) { return A1[(n0 + n) * LDM + kk]; });
+        MMD32(udm, aU, [&](int kk, int n) { return A1[kk * LDM + n0 + n]; });
         if (has_s) {
-            MMD(kds, aK, [&](int kk, int n) { return A2[(n0 + n) * LDM + kk]; });
-            MMD(uds, aU, [&](int kk, int n) { return A2[kk * LDM + n0 + n]; });
+            MMD32(kds, aK, [&](int kk, int n) { return A2[(n0 + n) * LDM + kk]; });
+            MMD32(uds, aU, [&](int kk, int n) { return A2[kk * LDM + n0 + n]; });
         }
         const float *gi = dUg + task * kDD;
+        Strip ud;
 #pragma unroll
         for (int tl = 0; tl < 2; tl++)
 #pragma unroll
@@ -522,8 +553,10 @@ __global__ __launch_bounds__(kThr) void ex_grads_kernel(
                 if constexpr (FROZEN) {     // dR = dU
                     Ts[row * LDM + col] = du;
                     if (row < L) d_v[(tok + row) * D + col] = -du;
+                    ud.t[tl][i] = du * Us[row * LDM + col];
                 }
             }
+        if constexpr (FROZEN) publish(6, ud);
     }
     __syncthreads();   // dU complete; dMo, dSo no longer needed
     if constexpr (!FROZEN) {
@@ -535,6 +568,9 @@ __global__ __launch_bounds__(kThr) void ex_grads_kernel(
             FORC(dr, [&](int r, int c, float &x) {
                 if (m0 + r < L) d_v[(tok + m0 + r) * D + n0 + c] = -x;
             });
+            Strip ud = dr;
+            FORC(ud, [&](int r, int c, float &x) { x *= Us[(m0 + r) * LDM + n0 + c]; });
+            publish(6, ud);
         }
         __syncthreads();   // T no longer needed
         if (dcol) FORC(dr, [&](int r, int c, float &x) { Ts[(m0 + r) * LDM + n0 + c] = x; });   // dR
@@ -659,7 +695,11 @@ __global__ __launch_bounds__(kThr) void ex_grads_kernel(
         auto sum = [&](int which, int row) { return D == 64 ? part[which][0][row] + part[which][1][row] : part[which][0][row]; };
         const float g1 = sum(2, t), g2 = sum(3, t);
         const float dam = !FROZEN && t + 1 < CW ? sum(4, t + 1) : 0.f, dbm = !FROZEN && t + 1 < CW ? sum(5, t + 1) : 0.f;
-        d_theta[tok + t] = -(((part_th[0][t] + part_th[1][t]) + (part_th[2][t] + part_th[3][t])) + cf.cl[t] * g1 + cf.bl[t] * g2);
+        // theta_t enters the rule as theta_t u_t, so that d_theta_t = u_t . dR_t / theta_t: one dot where the sum over the
+        // tokens behind t adds up to 64 rounded products; that sum is left for a theta that dR vanishes with
+        const float th = cf.th[t];
+        d_theta[tok + t] = th > 1e-18f ? sum(6, t) / th
+            : -(((part_th[0][t] + part_th[1][t]) + (part_th[2][t] + part_th[3][t])) + cf.cl[t] * g1 + cf.bl[t] * g2);
         float *pv = pvec + (tok + t) * 4;
         pv[0] = sum(0, t) + dam;
         pv[1] = sum(1, t) + dbm;
@@ -697,7 +737,7 @@ __global__ __launch_bounds__(kThr) void ex_fwd_local_kernel(
         fetch(tv, v + tok * D, L, tid);
         const Gates gt = fetch_gates(alpha + tok, theta + tok, eta + tok, L, has_s != 0);
         load_gates(cf, gt);
-        coefficients(cf, gt, L, Cc, nullptr, nullptr);
+        coefficients<double>(cf, gt, L, Cc, nullptr, nullptr);
         commit(Ks, tk, tid);
         commit(Vs, tv, tid);
     }
@@ -726,9 +766,9 @@ __global__ __launch_bounds__(kThr) void ex_fwd_local_kernel(
         Strip tv = zero_strip(), z1 = zero_strip(), z2 = zero_strip();
         auto aT = [&](int m, int kk) { return Nn[(m0 + m) * LDM + kk]; };
         const int pe = (ib >> 1) + 1;
-        mma_range(tv, aT, [&](int kk, int n) { return Vs[kk * LDM + n0 + n]; }, 0, pe, l);
-        mma_range(z1, aT, [&](int kk, int n) { return cv.am[kk] * Ks[kk * LDM + n0 + n]; }, 0, pe, l);
-        if (has_s) mma_range(z2, aT, [&](int kk, int n) { return cv.bm[kk] * Ks[kk * LDM + n0 + n]; }, 0, pe, l);
+        mma_range_f64(tv, aT, [&](int kk, int n) { return Vs[kk * LDM + n0 + n]; }, 0, pe, l);
+        mma_range_f64(z1, aT, [&](int kk, int n) { return cv.am[kk] * Ks[kk * LDM + n0 + n]; }, 0, pe, l);
+        if (has_s) mma_range_f64(z2, aT, [&](int kk, int n) { return cv.bm[kk] * Ks[kk * LDM + n0 + n]; }, 0, pe, l);
         for_c(tv, [&](int r, int c, float &x) { Cc[(m0 + r) * LDM + n0 + c] = x; }, l);
         for_c(z1, [&](int r, int c, float &x) { B8[(m0 + r) * LDM + n0 + c] = x; }, l);
         if (has_s) for_c(z2, [&](int r, int c, float &x) { Dg[(m0 + r) * LDM + n0 + c] = x; }, l);
@@ -745,7 +785,9 @@ __global__ __launch_bounds__(kThr) void ex_fwd_local_kernel(
         const float *wv = (o == 2 || o == 3 || o == 5) ? cv.wS : cv.wM;
         const float *Z = FROZEN ? (o >= 4 ? Vs : Ks) : o >= 4 ? Cc : (o & 1) ? Dg : B8;   // FROZEN: Z1 = K, Z2 = 0, T V = V
         Strip x = zero_strip();
-        if (!(FROZEN && (o == 1 || o == 3))) mma(x, [&](int m, int kk) { return Z[kk * LDM + sm0 + m]; }, [&](int kk, int n) { return wv[kk] * Ks[kk * LDM + sn0 + n]; }, l);
+        auto zt = [&](int m, int kk) { return Z[kk * LDM + sm0 + m]; };
+        auto wk = [&](int kk, int n) { return (double)wv[kk] * Ks[kk * LDM + sn0 + n]; };
+        if (!(FROZEN && (o == 1 || o == 3))) mma_f64(x, zt, wk, l);
         const float dg = o == 0 ? aL : o == 1 ? bL : o == 3 ? hL : 0.f;
         for_c(x, [&](int r, int c, float &y) { y = o >= 4 ? -y : sm0 + r == sn0 + c ? y + dg : y; }, l);
         float *mat = out + (size_t)o * DD;
@@ -773,28 +815,34 @@ bool exact_mm_applies(int d, int C) { return (d == 64 || d == 32) && C >= 1 && C
 static int chunk_of(int C) { return C * (CW / C); }
 
 // Cost models from measurements on one MI355X (us).  A chunk costs the two chunk-parallel kernels of the backward about
-// 65 us of a compute unit (42 at head size 32) whatever its length, a scan step 2.0 (0.5); the fused sequential kernel walks a
-// chain's tokens at 0.6 each on a quarter of a compute unit's worth of workgroups (four per chain, one at head size 32),
-// the kernel that reads a whole trajectory at 1.1.  Under a clip or a bound the test on the errors adds two launches to the
-// matrix form where the fused kernel's only adds one on its maxima.
+// 65 us of a compute unit whatever its length (95 with float64 sums, 54 at head size 32), a scan step 2.0 (2.9, 0.65); the
+// fused sequential kernel walks a chain's tokens at 0.6 each on a quarter of a compute unit's worth of workgroups (four per
+// chain, one at head size 32), the kernel that reads a whole trajectory at 1.1.  Under a clip or a bound the test on the
+// errors adds two launches to the matrix form where the fused kernel's only adds one on its maxima.
 bool exact_backward_mm_pays(int seq_len, int batch, int d, int C, bool tested, bool frozen) {
     const int nc = ceil_div(seq_len, frozen ? C : chunk_of(C)), cus = compute_units();
-    const double t_mm = (double)ceil_div(batch * nc, cus) * (d == 64 ? 65.0 : 42.0) + nc * (d == 64 ? 2.0 : 0.5) + (tested ? 20.0 : 10.0);
+    const bool wide = C == 1;
+    const double chunk = d == 32 ? 54.0 : wide ? 95.0 : 65.0, step = d == 32 ? 0.65 : wide ? 2.9 : 2.0;
+    const double t_mm = (double)ceil_div(batch * nc, cus) * chunk + nc * step + (tested ? 20.0 : 10.0);
     const double t_seq = (double)seq_len * (C == 1 ? 1.1 : 0.6) * ceil_div(batch * (d == 64 ? 4 : 1), cus);
     return t_mm < t_seq;
 }
 
-// The sequential forward takes 0.15 a token (0.19 where it keeps a trajectory) as long as its workgroups (four per chain,
-// one at head size 32) fit the chip.  The chunk maps cost 26 of a compute unit per chunk (17 at head size 32), a scan
-// step 2.0 (0.5), and, unless only the final states are wanted, the walk of the chunks' tokens again 0.15 a token for
-// whatever does not run at the same time.
-bool exact_forward_mm_pays(int seq_len, int batch, int d, bool final_only, int run) {
+// The sequential forward takes 0.15 a token as long as its workgroups (four per chain, one at head size 32) fit the chip,
+// and writes the states it keeps at 4.2 TB/s (32 chains of 512 tokens with their trajectory, 537 MB: 128 us).  The chunk
+// maps cost 35 of a compute unit per chunk (20 at head size 32), a scan step 2.6 (0.65), and, unless only the final states
+// are wanted, the walk of the chunks' tokens again 0.15 a token for whatever does not run at the same time, and the same
+// writes.
+bool exact_forward_mm_pays(int seq_len, int batch, int d, bool final_only, int run, long long kept_bytes) {
     const int nc = ceil_div(seq_len, run), cus = compute_units(), parts = d == 64 ? 4 : 1;
     if (nc < 2) return false;
-    double t_mm = (double)ceil_div(batch * (final_only ? nc : nc - 1), cus) * (d == 64 ? 26.0 : 17.0) + nc * (d == 64 ? 2.0 : 0.5) + 8.0;
-    if (!final_only) t_mm += 0.15 * run * ceil_div((long long)batch * nc * parts, cus);
-    const double t_seq = 0.15 * seq_len * ceil_div(batch * parts, cus);
-    return t_mm < t_seq;
+    auto walk = [&](double tokens, long long groups) {
+        const double t = 0.15 * tokens * ceil_div(groups, cus), w = (double)kept_bytes / 4.2e6;
+        return t > w ? t : w;
+    };
+    double t_mm = (double)ceil_div(batch * (final_only ? nc : nc - 1), cus) * (d == 64 ? 35.0 : 20.0) + nc * (d == 64 ? 2.6 : 0.65) + 8.0;
+    if (!final_only) t_mm += walk(run, (long long)batch * nc * parts);
+    return t_mm < walk(seq_len, (long long)batch * parts);
 }
 
 template <int D, bool FROZEN>
@@ -820,10 +868,10 @@ static void forward_states_t(bool has_s, const float *k, const float *v, const f
     KernelTimer kt("ex_scan_kernel");
     const dim3 grid((unsigned)batch * (D / 16));
     if (has_s)
-        hipLaunchKernelGGL((ex_scan_kernel<D, true, false>), grid, dim3(8 * D), 0, stream(), loc, m_initial, s_initial, m_stride,
+        hipLaunchKernelGGL((ex_scan_kernel<D, true, false, true>), grid, dim3(8 * D), 0, stream(), loc, m_initial, s_initial, m_stride,
                            m_states, s_states, state_stride, sstep, nullptr, nullptr, nc, maps);
     else
-        hipLaunchKernelGGL((ex_scan_kernel<D, false, false>), grid, dim3(4 * D), 0, stream(), loc, m_initial, nullptr, m_stride,
+        hipLaunchKernelGGL((ex_scan_kernel<D, false, false, true>), grid, dim3(4 * D), 0, stream(), loc, m_initial, nullptr, m_stride,
                            m_states, nullptr, state_stride, sstep, nullptr, nullptr, nc, maps);
     check_launch("ex_scan_kernel");
 }
@@ -836,7 +884,7 @@ void exact_forward_states(bool has_s, bool frozen, int d, int run, const float *
        batch, run);
 }
 
-template <int D, bool FROZEN>
+template <int D, bool FROZEN, bool P64>
 static bool backward_mm_t(const char *fn, bool has_s, const float *k, const float *v, const float *q, const float *alpha,
                           const float *theta, const float *eta, const float *m_ckpt, const float *s_ckpt, const float *d_y,
                           float *d_k, float *d_v, float *d_q, float *d_alpha, float *d_theta, float *d_eta, float *d_m_initial,
@@ -865,9 +913,9 @@ static bool backward_mm_t(const char *fn, bool has_s, const float *k, const floa
     float *first_m = first, *first_s = first + (size_t)batch * DD;
     static bool attr_set = false;
     if (!attr_set) {
-        set_lds(ex_local_kernel<D, FROZEN, false>, kExLocalLds);
-        set_lds(ex_local_kernel<D, FROZEN, true>, kExLocalLds);
-        set_lds(ex_grads_kernel<D, FROZEN>, kExGradsLds);
+        set_lds(ex_local_kernel<D, FROZEN, false, P64>, kExLocalLds);
+        set_lds(ex_local_kernel<D, FROZEN, true, P64>, kExLocalLds);
+        set_lds(ex_grads_kernel<D, FROZEN, P64>, kExGradsLds);
         attr_set = true;
     }
     if (es.failed()) return true;
@@ -875,7 +923,7 @@ static bool backward_mm_t(const char *fn, bool has_s, const float *k, const floa
     const float *et = has_s ? eta : alpha;
     {
         KernelTimer kt("ex_local_kernel");
-        auto kernel = guard ? ex_local_kernel<D, FROZEN, true> : ex_local_kernel<D, FROZEN, false>;
+        auto kernel = guard ? ex_local_kernel<D, FROZEN, true, P64> : ex_local_kernel<D, FROZEN, false, P64>;
         hipLaunchKernelGGL(kernel, dim3((unsigned)pgrid), dim3(kThr), kExLocalLds, stream(), k, v, q, d_y, alpha, theta, et,
                            m_ckpt, s_ckpt, loc, Tg, Ug, dUg, seq_len, C, nc, nck, cstep, (int)has_s, (int)nchunks, tracks);
         check_launch("ex_local_kernel");
@@ -885,22 +933,22 @@ static bool backward_mm_t(const char *fn, bool has_s, const float *k, const floa
         const dim3 grid((unsigned)batch * (D / 16));
         const long long stride = (long long)(nc + 1) * DD;
         if (has_s)
-            hipLaunchKernelGGL((ex_scan_kernel<D, true, true>), grid, dim3(8 * D), 0, stream(), loc, nullptr, nullptr, 0LL, em, esn,
+            hipLaunchKernelGGL((ex_scan_kernel<D, true, true, P64>), grid, dim3(8 * D), 0, stream(), loc, nullptr, nullptr, 0LL, em, esn,
                                stride, 1, first_m, first_s, nc, nc);
         else
-            hipLaunchKernelGGL((ex_scan_kernel<D, false, true>), grid, dim3(4 * D), 0, stream(), loc, nullptr, nullptr, 0LL, em, nullptr,
+            hipLaunchKernelGGL((ex_scan_kernel<D, false, true, P64>), grid, dim3(4 * D), 0, stream(), loc, nullptr, nullptr, 0LL, em, nullptr,
                                stride, 1, first_m, nullptr, nc, nc);
         check_launch("ex_scan_kernel");
     }
     {
         KernelTimer kt("ex_grads_kernel");
-        hipLaunchKernelGGL((ex_grads_kernel<D, FROZEN>), dim3((unsigned)pgrid), dim3(kThr), kExGradsLds, stream(), k, q, d_y, alpha, theta,
+        hipLaunchKernelGGL((ex_grads_kernel<D, FROZEN, P64>), dim3((unsigned)pgrid), dim3(kThr), kExGradsLds, stream(), k, q, d_y, alpha, theta,
                            et, m_ckpt, s_ckpt, Tg, Ug, dUg, em, esn, d_k, d_v, d_q, d_theta, pvec, xs, scal, seq_len, C, nc, nck, cstep,
                            (int)has_s, (int)nchunks);
         check_launch("ex_grads_kernel");
     }
     chunkwise_gate_gradients(alpha, eta, pvec, xs, scal, d_alpha, d_eta, seq_len, batch, C, has_s, first_m, first_s, DD, per,
-                             nsum, tmp, (int)DD);
+                             nsum, tmp, (int)DD, P64);
     if (es.failed()) return true;
     if (guard && couplings_may_fire_tracked(k, alpha, theta, eta, tracks, has_s, seq_len, batch, C, error_clip, m_norm_guard, D))
         return false;
@@ -917,7 +965,9 @@ bool exact_backward_mm(const char *fn, bool has_s, bool frozen, int d, const flo
              fn, seq_len, batch, d, C, CW);
         return true;
     }
-    auto run = frozen ? backward_mm_t<32, true> : d == 64 ? backward_mm_t<64, false> : backward_mm_t<32, false>;
+    auto run = frozen ? backward_mm_t<32, true, true>
+               : d == 32 ? backward_mm_t<32, false, true>
+               : C == 1 ? backward_mm_t<64, false, true> : backward_mm_t<64, false, false>;
     return run(fn, has_s, k, v, q, alpha, theta, eta, m_ckpt, s_ckpt, d_y, d_k, d_v, d_q, d_alpha, d_theta, d_eta, d_m_initial,
                d_s_initial, seq_len, batch, C, error_clip, m_norm_guard);
 }

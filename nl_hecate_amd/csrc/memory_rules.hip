@@ -679,7 +679,9 @@ static bool launch_fwd_uncoupled(FwdArgs a, int d, int batch, int *tracked_rows)
         const int run = FROZEN ? a.ckpt_interval : kExactChunk;
         const bool kept = FROZEN || STORE == STORE_TRAJ || kExactChunk % a.ckpt_interval == 0;   // the slots of all run starts exist
         if (kept && exact_mm_applies(d, FROZEN ? run : 1) && !(FROZEN && d == 64) && g_exact_form != 2 &&
-            (g_exact_form == 1 ? a.seq_len > run : exact_forward_mm_pays(a.seq_len, batch, d, false, run))) {
+            (g_exact_form == 1 ? a.seq_len > run
+                                : exact_forward_mm_pays(a.seq_len, batch, d, false, run,
+                                                        STORE == STORE_TRAJ ? 4LL * (HAS_S ? 2 : 1) * batch * a.seq_len * d * d : 0))) {
             const int sstep = FROZEN ? 1 : STORE == STORE_TRAJ ? run : run / a.ckpt_interval;
             exact_forward_states(HAS_S, FROZEN, d, run, a.k, a.v, a.alpha, a.theta, a.eta, a.m_initial, a.s_initial, a.m_stride, a.m_out,
                                  a.s_out, a.state_stride, sstep, a.seq_len, a.input_stride, batch);
@@ -962,7 +964,7 @@ static void final_states(const char *fn, const float *k, const float *v, const f
     if (seq_len == 0) { fail("%s: seq_len=0.", fn); return; }
     const size_t dd = (size_t)d * d;
     // three launches of the matrix form against one walk at 0.15 us a token (see exact_forward_mm_pays)
-    if (exact_mm_applies(d, 1) && g_exact_form != 2 && (g_exact_form == 1 || exact_forward_mm_pays(seq_len, batch, d, true, kExactChunk))) {
+    if (exact_mm_applies(d, 1) && g_exact_form != 2 && (g_exact_form == 1 || exact_forward_mm_pays(seq_len, batch, d, true, kExactChunk, 0))) {
         float *sf = HAS_S ? scratch(9, (size_t)batch * dd * sizeof(float)) : nullptr;
         if (es.failed()) return;
         exact_forward_states(HAS_S, false, d, kExactChunk, k, v, alpha, theta, eta, m_initial, s_initial, (long long)dd, m_final, sf, (long long)dd, 0, seq_len,

@@ -39,37 +39,45 @@ __device__ __forceinline__ float lane_bcast(float x, int lane) {
 // (stride LDM; entries outside j <= t < L are zero), plus the vectors (wave 1).  The gates
 // are read from global memory into one register per lane and broadcast per step, so the
 // sequential loops carry no memory latency.  Needs a barrier afterwards.
+// T: type of the recurrences.  In float they round at each of up to 64 steps; float64 leaves the rounding of what is kept.
+template <class T = float>
 __device__ __forceinline__ void coefficients(Coef &cf, const Gates &g, int L, float *Cc, float *Bb, float *Rr) {
     const int j = threadIdx.x & 63, w = threadIdx.x >> 6;
     if (w >= 4) return;
     const float keep_j = 1.f - g.al;   // 1 beyond L
     const float eta_j = g.et;          // 0 beyond L
     const bool jv = j < L;
+    auto keep_at = [&](int t) -> T {
+        if constexpr (sizeof(T) == 8) return 1.0 - (double)lane_bcast(g.al, t);
+        else return lane_bcast(keep_j, t);
+    };
     if (w == 0) {
         // branch-free: tokens after j update the running products; lanes t >= L broadcast
         // keep = 1, eta = 0, which leaves cc unchanged
-        float b = 1.f, cc = 1.f, blv = 0.f;
+        T b = 1, cc = 1;
+        float blv = 0.f;
 #pragma unroll 16
         for (int t = 0; t < CW; t++) {
-            const float keep = lane_bcast(keep_j, t), et = lane_bcast(eta_j, t);
+            const T keep = keep_at(t), et = lane_bcast(eta_j, t);
             const bool after = t > j;
-            b *= after ? et : 1.f;
-            cc = after ? fmaf(keep, cc, b) : cc;
-            blv = (t == L - 1) ? b : blv;
-            if (Cc) Cc[t * LDM + j] = (jv && t >= j && t < L) ? cc : 0.f;
+            b *= after ? et : T(1);
+            cc = after ? fma(keep, cc, b) : cc;
+            blv = (t == L - 1) ? (float)b : blv;
+            if (Cc) Cc[t * LDM + j] = (jv && t >= j && t < L) ? (float)cc : 0.f;
         }
-        cf.cl[j] = jv ? cc : 0.f;
+        cf.cl[j] = jv ? (float)cc : 0.f;
         cf.bl[j] = jv ? blv : 0.f;
     } else if (w == 1) {
         // a_t, beta_t, h_t: every lane runs the same scalar recurrence, lane t keeps step t
-        float a = 1.f, h = 1.f, beta = 0.f, ka = 0.f, kb = 0.f, kh = 0.f;
+        T a = 1, h = 1, beta = 0;
+        float ka = 0.f, kb = 0.f, kh = 0.f;
 #pragma unroll 8
         for (int t = 0; t < CW; t++) {
-            const float keep = lane_bcast(keep_j, t), et = lane_bcast(eta_j, t);
+            const T keep = keep_at(t), et = lane_bcast(eta_j, t);
             a *= keep;
             h *= et;
             beta = keep * beta + h;
-            if (t == j) { ka = a; kb = beta; kh = h; }
+            if (t == j) { ka = (float)a; kb = (float)beta; kh = (float)h; }
         }
         cf.a[j] = j < L ? ka : 0.f;
         cf.beta[j] = j < L ? kb : 0.f;

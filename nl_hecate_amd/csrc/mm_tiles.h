@@ -158,6 +158,67 @@ __device__ __forceinline__ void mma_tile16(f32x4 &acc, FA a, FB b, int k0, int l
 #pragma unroll
     for (int i = 0; i < 4; i++) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(av[i], bv[i], acc, 0, 0, 0);
 }
+// The same three products summed in float64 (v_mfma_f64_16x16x4_f64) and rounded once.  The fp32 instruction rounds after
+// every term of its running sum: a product of unit normals over 64 terms comes out 2.3e-7 wide of the exact one, where a
+// sum over the lanes of a row (sixteen partial sums of four, added in a tree) gives 1.0e-7; summed in float64 it is the
+// final rounding, 0.3e-7.  Half the rate of the fp32 instruction.  Its result rows are dealt out differently, element i of
+// lane l is row 4 i + l/16, so the first operand's rows are exchanged to land where the fp32 strip has them.
+using f64x4 = __attribute__((ext_vector_type(4))) double;
+__device__ __forceinline__ int f64_row(int l) { return 4 * (l & 3) + ((l & 15) >> 2); }
+__device__ __forceinline__ f64x4 widen(const f32x4 &x) { return f64x4{(double)x[0], (double)x[1], (double)x[2], (double)x[3]}; }
+__device__ __forceinline__ f32x4 narrow(const f64x4 &x) { return f32x4{(float)x[0], (float)x[1], (float)x[2], (float)x[3]}; }
+
+template <class FA, class FB>
+__device__ __forceinline__ void mma_f64(Strip &acc, FA a, FB b, int l = threadIdx.x & 63) {
+    const int r = l & 15, ra = f64_row(l), kb = 16 * (l >> 4);
+    f64x4 c0 = widen(acc.t[0]), c1 = widen(acc.t[1]);
+    decltype(a(0, 0)) av[2][4];   // an operand may come as float or, scaled without rounding, as double
+    decltype(b(0, 0)) b0[2][4], b1[2][4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) { av[0][i] = a(ra, kb + i); b0[0][i] = b(kb + i, r); b1[0][i] = b(kb + i, 16 + r); }
+#pragma unroll
+    for (int g = 0; g < 4; g++) {
+        if (g < 3) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int kk = kb + 4 * (g + 1) + i;
+                av[(g + 1) & 1][i] = a(ra, kk); b0[(g + 1) & 1][i] = b(kk, r); b1[(g + 1) & 1][i] = b(kk, 16 + r);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const double x = (double)av[g & 1][i];
+            c0 = __builtin_amdgcn_mfma_f64_16x16x4f64(x, (double)b0[g & 1][i], c0, 0, 0, 0);
+            c1 = __builtin_amdgcn_mfma_f64_16x16x4f64(x, (double)b1[g & 1][i], c1, 0, 0, 0);
+        }
+    }
+    acc.t[0] = narrow(c0);
+    acc.t[1] = narrow(c1);
+}
+template <class FA, class FB>
+__device__ __forceinline__ void mma_range_f64(Strip &acc, FA a, FB b, int p0, int p1, int l = threadIdx.x & 63) {
+    const int r = l & 15, ra = f64_row(l), kq = l >> 4, kb = 16 * (kq & 1) + 8 * (kq >> 1);
+    f64x4 c0 = widen(acc.t[0]), c1 = widen(acc.t[1]);
+    for (int p = p0; p < p1; p++) {
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            float av[4], b0[4], b1[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int kk = 32 * p + kb + 4 * h + i;
+                av[i] = a(ra, kk); b0[i] = b(kk, r); b1[i] = b(kk, 16 + r);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const double x = (double)av[i];
+                c0 = __builtin_amdgcn_mfma_f64_16x16x4f64(x, (double)b0[i], c0, 0, 0, 0);
+                c1 = __builtin_amdgcn_mfma_f64_16x16x4f64(x, (double)b1[i], c1, 0, 0, 0);
+            }
+        }
+    }
+    acc.t[0] = narrow(c0);
+    acc.t[1] = narrow(c1);
+}
 // Element i of tile tl of lane l is C[4*(l/16) + i][16*tl + l%16] of the strip.
 template <class F>
 __device__ __forceinline__ void for_c(Strip &acc, F f, int l = threadIdx.x & 63) {
