@@ -47,10 +47,17 @@ __device__ __forceinline__ void while_true(Fn &f, std::integer_sequence<int, I..
 }
 
 // ── the recurrence ───────────────────────────────────────────────────────────────────────────────────────────────
-// Tiles of 16 tokens.  At a tile's start P_c = M_c X^T for the whole tile comes off the matrix cores; inside the tile
-// token t adds its outer product to the later columns only, P_c[t'] = (1-a_t) P_c[t'] + th_t w_c,t (k_t . x_t'), so a
-// token needs k_t in all waves (one LDS exchange), the products F_k k_t, F_v k_t and the dots of k_t with the tile's x
-// and with the row means; at the tile's end M_c takes the 16 outer products on the matrix cores.
+// Tiles of 16 tokens.  At a tile's start P0_c = M_c X^T for the whole tile comes off the matrix cores; inside the tile
+// token t adds its outer product to the later columns only, P_c[t'] = (1-a_t) P_c[t'] + th_t w_c,t (k_t . x_t') from
+// zero, and the value of column t' is A_t' P0_c[t'] + P_c[t'] with A the retentions so far, so a token needs k_t in all
+// waves (one LDS exchange), the products F_k k_t, F_v k_t and the dots of k_t with the tile's x and with the row means;
+// at the tile's end M_c takes the sum of the 16 outer products on the matrix cores.
+//
+// Rounding feeds back (k into the gates, the gates into every later state), and a saturated gate is the rounding of its
+// mean, whose terms are large and of one sign.  So what the tile starts with and what its tokens add are kept apart, each
+// sum is formed by itself and joined once, the retentions are a float64 product, and the means' P0 is summed and kept in
+// float64.  With one running fp32 value per column y was 1.25 times as far from float64 as with token by token products,
+// the gates 1.4 to 2 times; so it is 0.65 and 0.4 times, for 0.08 ms of the 1.26 below.
 //
 // Two lane layouts, one a permutation of the other's lanes: the matrix cores' (ml, kg) = (lane % 16, lane / 16) and the
 // quads' (r, cq) = (lane / 4, lane % 4).  Lane (ml, kg) holds row ml of the wave's 16 rows, columns 16 kt + 4 kg + v,
@@ -60,11 +67,10 @@ __device__ __forceinline__ void while_true(Fn &f, std::integer_sequence<int, I..
 // lane cq then owns the columns t' = 4 j + cq of P, and column group j is finished with token 4 j + 3.
 // The row means are rows 0 (alpha), 1 (eta) and 2 (v) of a third matrix that every wave carries.
 //
-// Bound by the issue rate of one wave per SIMD (155 instructions a token at 5.3 clocks, 990 clocks a token with the
-// exchange, 6 % of the time at tile starts and ends each).  64 chains of 2048 tokens, head size 64, chunks of 64: 1.18 ms,
-// with the two kernels below 1.41 ms; one kernel that formed all products of a token with all six memories in sequence
-// (it serves longer chunks, selfref.hip) takes 2.30 ms.  Chunks of 1, 4, 8, 16 tokens at 64 chains of 512: 6.65, 2.05,
-// 1.28, 0.88 ms there, 3.47, 1.07, 0.67, 0.46 ms here.
+// Bound by the issue rate of one wave per SIMD (1050 clocks a token with the exchange, tile starts and ends).  64 chains of
+// 2048 tokens, head size 64, chunks of 64: 1.26 ms, with the two kernels below 1.47 ms; one kernel that formed all products of a token with all six memories in sequence
+// (it serves longer chunks, selfref.hip) takes 2.29 ms.  Chunks of 1, 4, 8, 16 tokens at 64 chains of 512: 6.64, 2.04,
+// 1.27, 0.88 ms there, 3.84, 1.15, 0.70, 0.47 ms here.
 
 template <int D, bool SG>
 __global__ __launch_bounds__(4 * D) void selfref_chain_kernel(
@@ -146,31 +152,47 @@ __global__ __launch_bounds__(4 * D) void selfref_chain_kernel(
             const int t2 = tile_end(te);
             if (t2 < s) xnext = load_x(t2, tile_end(t2) - t2);
         }
-        float P[3][4], X[4 * KT];
+        float P0[2][4], P[3][4], X[4 * KT];   // M_c X^T as the tile starts, and what its tokens add
+        double P2[4];
         {
-            f32x4 acc[3] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+            f32x4 acc[2][KT];   // a sum per 16 columns, added up in a tree
+            f64x4 mean_acc = {0., 0., 0., 0.};
 #pragma unroll
             for (int kt = 0; kt < KT; kt++) {
                 const f32x4 xa = *reinterpret_cast<const f32x4 *>(&xt[buf][sigma(ml) * LD + 16 * kt + 4 * kg]);
+                const f32x4 xm = *reinterpret_cast<const f32x4 *>(&xt[buf][ml * LD + 16 * kt + 4 * kg]);
                 const f32x4 xq = *reinterpret_cast<const f32x4 *>(&xt[buf][sigma(r) * LD + 16 * kt + 4 * cq]);
+#pragma unroll
+                for (int c = 0; c < 2; c++) acc[c][kt] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                 for (int v = 0; v < 4; v++) {
                     X[4 * kt + v] = xq[v];
 #pragma unroll
-                    for (int c = 0; c < 3; c++) acc[c] = mfma4(xa[v], M[c][kt][v], acc[c]);
+                    for (int c = 0; c < 2; c++) acc[c][kt] = mfma4(xa[v], M[c][kt][v], acc[c][kt]);
+                    // result rows 4 v + kg: the first operand's rows are the tokens as they stand
+                    mean_acc = __builtin_amdgcn_mfma_f64_16x16x4f64((double)xm[v], (double)M[2][kt][v], mean_acc, 0, 0, 0);
                 }
             }
 #pragma unroll
-            for (int c = 0; c < 3; c++) {
+            for (int c = 0; c < 2; c++) {
+                f32x4 t = acc[c][0];
+                if constexpr (KT == 2) t += acc[c][1];
+                if constexpr (KT == 4) t = (t + acc[c][1]) + (acc[c][2] + acc[c][3]);
 #pragma unroll
-                for (int v = 0; v < 4; v++) P[c][v] = lane_from(to_quad, acc[c][v]);
+                for (int v = 0; v < 4; v++) P0[c][v] = lane_from(to_quad, t[v]);
+            }
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                P2[v] = lane_from64(to_quad, mean_acc[v]);
+                P[0][v] = P[1][v] = P[2][v] = 0.f;
             }
         }
-        float W[3][4], cs[4], keep_tile = 1.f;  // w_c of token 4 j + cq, th times the retention since, of the whole tile
+        float W[3][4], cs[4];
+        double kept = 1.;  // w_c of token 4 j + cq, th times the retention since, of the whole tile
 #pragma unroll
         for (int j = 0; j < 4; j++) W[0][j] = W[1][j] = W[2][j] = cs[j] = 0.f;
-        float k = quad_lane<0>(P[0][0]), v = quad_lane<0>(P[1][0]);
-        float am = lane_value(P[2][0], 0), em = lane_value(P[2][0], 4), vm = lane_value(P[2][0], 8);
+        float k = quad_lane<0>(P0[0][0]), v = quad_lane<0>(P0[1][0]);
+        float am = lane_value((float)P2[0], 0), em = lane_value((float)P2[0], 4), vm = lane_value((float)P2[0], 8);
         // lane t keeps token t's gate means for the caches; what token t - 1 adds to the columns behind t is added while
         // token t's exchange is under way
         float s_am = 0.f, s_em = 0.f;
@@ -225,7 +247,7 @@ __global__ __launch_bounds__(4 * D) void selfref_chain_kernel(
             const float th = SG ? -theta : theta;
 #pragma unroll
             for (int j = 0; j <= J; j++) cs[j] *= keep;
-            keep_tile *= keep;
+            kept *= 1. - (double)alpha;
             cs[J] = cq == Q ? th : cs[J];
 #pragma unroll
             for (int c = 0; c < 3; c++) W[c][J] = cq == Q ? w[c] : W[c][J];
@@ -235,9 +257,10 @@ __global__ __launch_bounds__(4 * D) void selfref_chain_kernel(
 #pragma unroll
                 for (int c = 0; c < 3; c++) pw[c] = th * w[c];
                 pkeep = keep;
-                k = fmaf(pw[0], s1, keep * quad_lane<Q1>(P[0][J1]));
-                v = fmaf(pw[1], s1, keep * quad_lane<Q1>(P[1][J1]));
-                const float m = fmaf(pw[2], s1, keep * P[2][J1]);
+                const float kept1 = (float)kept;
+                k = fmaf(kept1, quad_lane<Q1>(P0[0][J1]), fmaf(pw[0], s1, keep * quad_lane<Q1>(P[0][J1])));
+                v = fmaf(kept1, quad_lane<Q1>(P0[1][J1]), fmaf(pw[1], s1, keep * quad_lane<Q1>(P[1][J1])));
+                const float m = (float)fma(kept, P2[J1], (double)fmaf(pw[2], s1, keep * P[2][J1]));
                 am = lane_value(m, Q1);
                 em = lane_value(m, 4 + Q1);
                 vm = lane_value(m, 8 + Q1);
@@ -247,11 +270,14 @@ __global__ __launch_bounds__(4 * D) void selfref_chain_kernel(
         };
         while_true(step, std::make_integer_sequence<int, kTB>{});
 
-        // M_c <- keep M_c + sum_t cs_t w_c,t k_t^T; every wave has written its part of Kb, Vb
+        // M_c <- keep M_c + sum_t cs_t w_c,t k_t^T; every wave has written its part of Kb, Vb.  The tile's sum is formed by
+        // itself, so that M_c rounds once a tile and not once a token
+        const float keep_tile = (float)kept;
+        f32x4 add[3][KT];
 #pragma unroll
         for (int c = 0; c < 3; c++) {
 #pragma unroll
-            for (int kt = 0; kt < KT; kt++) M[c][kt] *= keep_tile;
+            for (int kt = 0; kt < KT; kt++) add[c][kt] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int j = 0; j < 4; j++) W[c][j] = lane_from(to_mm, W[c][j] * cs[j]);
         }
@@ -262,8 +288,16 @@ __global__ __launch_bounds__(4 * D) void selfref_chain_kernel(
                 for (int kt = 0; kt < KT; kt++) {
                     const float a = Kb[(4 * j + kg) * LD + 16 * kt + ml];
 #pragma unroll
-                    for (int c = 0; c < 3; c++) M[c][kt] = mfma4(a, W[c][j], M[c][kt]);
+                    for (int c = 0; c < 3; c++) add[c][kt] = mfma4(a, W[c][j], add[c][kt]);
                 }
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+#pragma unroll
+            for (int kt = 0; kt < KT; kt++) {
+#pragma unroll
+                for (int v = 0; v < 4; v++) M[c][kt][v] = fmaf(keep_tile, M[c][kt][v], add[c][kt][v]);
             }
         }
         if (stt < nt) {
@@ -371,7 +405,7 @@ __global__ __launch_bounds__(4 * D) void selfref_scan_kernel(
         for (int st = 0; st < ST; st++) w[st] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int kt = 0; kt < KT; kt++) {
-            N[kt] = F[kt] * keep;
+            N[kt] = f32x4{0.f, 0.f, 0.f, 0.f};   // the chunk's sum by itself: F rounds once a chunk
             if (kt + 1 < KT) read_w(kt + 1, (kt + 1) & 1);
             else read_n(0, 0);
             __builtin_amdgcn_sched_barrier(0);
@@ -400,7 +434,10 @@ __global__ __launch_bounds__(4 * D) void selfref_scan_kernel(
             __builtin_amdgcn_sched_barrier(0);
         }
 #pragma unroll
-        for (int kt = 0; kt < KT; kt++) F[kt] = N[kt];
+        for (int kt = 0; kt < KT; kt++) {
+#pragma unroll
+            for (int v = 0; v < 4; v++) F[kt][v] = fmaf(keep, F[kt][v], N[kt][v]);
+        }
         if (ci + 1 < nc) stage(buf ^ 1);
         __syncthreads();
     }

@@ -40,3 +40,27 @@ def test_tiles_of_one_token(C, d):
     want = oracle_run(mems[:2], x[:2], dy[:2], C, True, np.float32)
     for n in ("y", "k", "v", "alpha", "theta"):
         assert_close(n, got[n].reshape(B, -1)[:2].reshape(want[n].shape), want[n])
+
+
+@pytest.mark.parametrize("sg", [True, False])
+@pytest.mark.parametrize("C", [32, 64])
+def test_no_further_from_float64_than_the_token_loop(C, sg):
+    """Gates that saturate low carry every rounding on over the sequence: the sums that feed back are formed so that the
+    result stays at least as close to float64 as the fp32 oracle's token by token loop."""
+    d, s, B = 64, 500, 3
+    err = {n: [] for n in ("y", "alpha", "d_emb", "d_mems")}
+    for seed in range(4):
+        r = np.random.default_rng(60 + seed)
+        u = np.full(d, d ** -0.5, np.float32)
+        mems = ((r.random((B, 6, d, d)) * 2 - 1) * (6.0 / (2 * d)) ** 0.5).astype(np.float32)
+        mems[:, 4] -= 13 * u
+        mems[:, 3] -= 6 * u
+        x = (r.standard_normal((B, s, d)) * (8 * d) ** -0.5 + 0.5 * u).astype(np.float32)
+        dy = r.standard_normal((B, s, d)).astype(np.float32)
+        got, loop, ref = gpu_run(mems, x, dy, C, sg), oracle_run(mems, x, dy, C, sg, np.float32), oracle_run(mems, x, dy, C, sg, np.float64)
+        for n in err:
+            off = lambda a: [np.linalg.norm(a[n].reshape(B, -1)[b].astype(np.float64) - ref[n].reshape(B, -1)[b]) for b in range(B)]
+            err[n] += [np.log(p / q) for p, q in zip(off(got), off(loop))]
+    print(sg, C, {n: round(float(np.exp(np.mean(e))), 2) for n, e in err.items()})
+    for n, e in err.items():
+        assert np.mean(e) <= 0, (n, np.exp(np.mean(e)))
