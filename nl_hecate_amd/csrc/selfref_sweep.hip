@@ -12,7 +12,7 @@
 // so that a token takes one exchange (dg_t), one product with a matrix and the dots of dg_t with the tile's u_s.
 //
 // 64 chains of 2048 tokens, head size 64, chunks of 64: preparation 0.36 ms (one workgroup per compute unit for its LDS;
-// 0.10 are matrix instructions), sweep 1.56 ms: 760 clocks a token (115 instructions of one wave per SIMD and the
+// 0.10 are matrix instructions), sweep 1.60 ms: 760 clocks a token (115 instructions of one wave per SIMD and the
 // exchange), 9.5 k clocks a tile and 34 k a chunk boundary, half of each matrix instructions.  The sweep that formed w, z,
 // dk, dv and the update of dG token by token took 3.16 ms behind 0.23 ms of preparation; without self-generated values it
 // is still the one (selfref.hip), since there dh_t comes back as a second vector.
@@ -317,18 +317,19 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_prepare_kernel(
         request(0, 0);
 #pragma unroll
         for (int jt = 0; jt < KT; jt++) {
-            f32x4 dg2 = kZero;
-            dg[jt] = fx[jt] = kZero;
+            f32x4 dgk[2] = {kZero, kZero}, dgv[2] = {kZero, kZero}, dgq[2] = {kZero, kZero}, fxk[2] = {kZero, kZero};
             if (jt + 1 < KT) request(jt + 1, (jt + 1) & 1);
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int i = 0; i < 4 * KT; i++) {
-                dg[jt] = mfma4(ak[i >> 2][i & 3], f[jt & 1][0][i], dg[jt]);
-                fx[jt] = mfma4(in[0][tile_i][i >> 2][i & 3], f[jt & 1][0][i], fx[jt]);
-                dg2 = mfma4(av[i >> 2][i & 3], f[jt & 1][1][i], dg2);
-                dg[jt] = mfma4(aq[i >> 2][i & 3], f[jt & 1][2][i], dg[jt]);
+                const int h = i >= 2 * KT;
+                dgk[h] = mfma4(ak[i >> 2][i & 3], f[jt & 1][0][i], dgk[h]);
+                fxk[h] = mfma4(in[0][tile_i][i >> 2][i & 3], f[jt & 1][0][i], fxk[h]);
+                dgv[h] = mfma4(av[i >> 2][i & 3], f[jt & 1][1][i], dgv[h]);
+                dgq[h] = mfma4(aq[i >> 2][i & 3], f[jt & 1][2][i], dgq[h]);
             }
-            dg[jt] += dg2;
+            dg[jt] = ((dgk[0] + dgk[1]) + (dgv[0] + dgv[1])) + (dgq[0] + dgq[1]);
+            fx[jt] = fxk[0] + fxk[1];
 #pragma unroll
             for (int v = 0; v < 4; v++) {
                 if (4 * kg + v < nt) {
@@ -670,9 +671,18 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_sweep_kernel(
             lds_barrier();
             if (tile > 0) request(tb - kTB, kTB);
 
-            // W = dG K, Z = dG^T U, Y = F_k^T Z + (F_k - F_v)^T W of the whole tile; T_s = u_s . W_s
-            f32x4 W = kZero, Z = kZero, Y = kZero, Y2 = kZero;
+            // W = dG K, Z = dG^T U, Y = F_k^T Z + (F_k - F_v)^T W of the whole tile; T_s = u_s . W_s.  A sum per 16 terms,
+            // added up in a tree: one running sum rounds at every term (d_x 1.1 to 1.2 times as far from float64)
+            constexpr int NQ = CP / 4;
+            f32x4 Wq[NQ], Zq[NQ], Yq[NQ], Y2q[NQ];
             float U[CP], T = 0.f;
+#pragma unroll
+            for (int q = 0; q < NQ; q++) Wq[q] = Zq[q] = Yq[q] = Y2q[q] = kZero;
+            auto tree = [](const f32x4(&a)[NQ]) {
+                if constexpr (NQ == 4) return (a[0] + a[1]) + (a[2] + a[3]);
+                else if constexpr (NQ == 2) return a[0] + a[1];
+                else return a[0];
+            };
 #pragma unroll
             for (int i = 0; i < CP; i += 4) {
                 const f32x4 k4 = *reinterpret_cast<const f32x4 *>(&T_(A_K, my_s, CP * kg + i));
@@ -680,10 +690,11 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_sweep_kernel(
 #pragma unroll
                 for (int v = 0; v < 4; v++) {
                     U[i + v] = u4[v];
-                    W = mfma4(k4[v], dG[i + v], W);
-                    Z = mfma4(u4[v], dGT[i + v], Z);
+                    Wq[i / 4] = mfma4(k4[v], dG[i + v], Wq[i / 4]);
+                    Zq[i / 4] = mfma4(u4[v], dGT[i + v], Zq[i / 4]);
                 }
             }
+            f32x4 W = tree(Wq), Z = tree(Zq);
 #pragma unroll
             for (int v = 0; v < 4; v++) {
                 T_(A_W, 4 * v + kg, wr + ml) = W[v];
@@ -697,11 +708,11 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_sweep_kernel(
 #pragma unroll
                 for (int v = 0; v < 4; v++) {
                     T = fmaf(U[i + v], w4[v], T);
-                    Y = mfma4(z4[v], FTk[i + v], Y);
-                    Y2 = mfma4(w4[v], FTu[i + v], Y2);
+                    Yq[i / 4] = mfma4(z4[v], FTk[i + v], Yq[i / 4]);
+                    Y2q[i / 4] = mfma4(w4[v], FTu[i + v], Y2q[i / 4]);
                 }
             }
-            Y += Y2;
+            f32x4 Y = tree(Yq) + tree(Y2q);
             T = swapadd32(T, T);
             T = swapadd16(T, T);
 
