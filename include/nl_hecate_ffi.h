@@ -75,7 +75,10 @@ int nlh_selftest_chunk_coef_prepass(const float *alpha, const float *theta, cons
  * b*input_stride*d (gates at b*input_stride) and initial states at b*m_stride;
  * outputs use the local seq_len: y [batch, seq_len, d],
  * m_states / s_states [batch, seq_len+1, d*d].
- * error_clip <= 0 and m_norm_max <= 0 or >= 1e30 disable clip / projection. */
+ * error_clip <= 0 and m_norm_max <= 0 or >= 1e30 disable clip / projection.
+ * The forwards of the exact and frozen rules need no scratch memory.  Head sizes 32 and 64 take up to 256 MiB of it for
+ * few long chains, where it is free to take: not while the launch stream is being captured, and on the first stream that
+ * took it only (until nlh_release_workspace); otherwise they walk the tokens.  So does *_final_states_f32_rocm. */
 /* core/src/cuda_ffi.rs:134 */
 void titans_forward_f32_cuda(const float *k_mem, const float *v_mem, const float *q_mem,
                              const float *alpha, const float *theta, const float *eta,
@@ -268,8 +271,8 @@ void delta_forward_ckpt_batched_f32_rocm(const float *k_mem, const float *v_mem,
 
 
 /* The states after the last token, without outputs or trajectory (no clip, no projection): what a prompt leaves in a
- * memory.  k, v [batch, seq_len, d], gates [batch, seq_len], m_initial / m_final [batch, d*d]; s_initial may be null
- * (zero momentum). */
+ * memory.  k, v [batch, seq_len, d], gates [batch, seq_len], m_initial / m_final [batch, d*d], which may be the same; s_initial
+ * may be null (zero momentum). */
 void titans_final_states_f32_rocm(const float *k_mem, const float *v_mem, const float *alpha, const float *theta,
                                   const float *eta, const float *m_initial, const float *s_initial, float *m_final,
                                   int seq_len, int d, int batch_size);
@@ -696,13 +699,16 @@ void saxpy_multi_rocm(float alpha, const float *const *x, float *const *y, const
 /* One whole decode step (core/src/gpu_forward.rs:3377-3492 gpu_single_token_forward) in four launches: projections of
  * the embedded token, K and V rounded into row `pos` of the bf16 caches [max_len, d], attention over the cache, every
  * level's one-token step on its carried memory, combine, gate, output projection and unembedding.  Blocks until the
- * logits are on the host.  Head size 32, 64 or 128, d <= 4096, at most 8 levels.  Returns 0 on success.
+ * logits are on the host.  Head size 32, 64 or 128, d <= 4096, at most 8 levels, d + heads * (slices of 128 visible keys)
+ * <= 16384.  Returns 0 on success.
  *   embedding_row [d]; w_* [d, d]; w_unembed [d, vocab]
  *   level_ptrs    host array, 8 device pointers per level: w_k, w_v, w_q, w_alpha, b_alpha, w_theta, b_theta,
  *                 memory [heads, hd*hd] (updated in place for an active level)
  *   level_rule    host array: -1 frozen (y = M q with the raw projection), 0 Hebbian, 1 Delta or Titans (zero
- *                 momentum at the start of a call), 2 DGD
- *   level_bounds  host array, 6 per level: alpha floor / ceil, theta floor / ceil, error_clip, m_norm_max
+ *                 momentum at the start of a call; its momentum gate is not read), 2 DGD, 3 as -1 with the normalised
+ *                 projection (the last position of a prompt whose memories stand at their final states)
+ *   level_bounds  host array, 6 per level: alpha floor / ceil (0 and 1: none), theta floor / ceil (0 and FLT_MAX: none),
+ *                 error_clip, m_norm_max
  *   work          device floats, decode_work_floats_rocm(...) of them
  *   workspace     host array of 7 device buffers that receive the step's intermediates: embedded [d] f32, q [d] bf16,
  *                 attention output [d] bf16 and [d] f32, y_combined, gate, gated [d] f32

@@ -22,10 +22,12 @@ bool exact_backward_mm(const char *fn, bool has_s, bool frozen, int d, const flo
 // element offset c * sstep * d*d of its chain's m_states / s_states (chain stride state_stride), from the initial states
 // (chain stride m_stride; s_initial null: zero).  No clip, no projection.  The runs' tokens are then independent walks
 // (FwdArgs::sub_chunks).  sstep 0: the states after the last token instead.
+// false, and nothing launched: there is no scratch for it (scratch_if_free: under capture, on a second stream), the caller
+// walks the tokens.  The runs go through that scratch in stretches that fit it.
 constexpr int kExactChunk = 64;
 // kept_bytes: states that the walk of the tokens writes
 bool exact_forward_mm_pays(int seq_len, int batch, int d, bool final_only, int run, long long kept_bytes);
-void exact_forward_states(bool has_s, bool frozen, int d, int run, const float *k, const float *v, const float *alpha, const float *theta,
+bool exact_forward_states(bool has_s, bool frozen, int d, int run, const float *k, const float *v, const float *alpha, const float *theta,
                           const float *eta, const float *m_initial, const float *s_initial, long long m_stride, float *m_states,
                           float *s_states, long long state_stride, int sstep, int seq_len, int input_stride, int batch);
 

@@ -846,42 +846,57 @@ bool exact_forward_mm_pays(int seq_len, int batch, int d, bool final_only, int r
 }
 
 template <int D, bool FROZEN>
-static void forward_states_t(bool has_s, const float *k, const float *v, const float *alpha, const float *theta, const float *eta,
+static bool forward_states_t(bool has_s, const float *k, const float *v, const float *alpha, const float *theta, const float *eta,
                              const float *m_initial, const float *s_initial, long long m_stride, float *m_states, float *s_states,
                              long long state_stride, int sstep, int seq_len, int input_stride, int batch, int C) {
     const ErrorScope es;
-    // to the starts of all chunks, or (sstep 0) through the last one to the end
+    constexpr size_t DD = (size_t)D * D;
+    // to the starts of all chunks, or (sstep 0) through the last one to the end; in stretches whose maps fit the scratch,
+    // each from the states that the one before it left
     const int nc = ceil_div(seq_len, C), maps = sstep ? nc - 1 : nc;
-    float *loc = scratch(32, (size_t)batch * nc * kExLocMats * D * D * sizeof(float));
+    const size_t per_chunk = (size_t)batch * kExLocMats * DD * sizeof(float);
+    const long long fit = (long long)(kOptionalScratch / per_chunk);
+    const int stretch = fit < maps ? (int)fit : maps;
+    if (stretch < 1) return false;
+    float *loc = scratch_if_free(40, stretch * per_chunk);
+    if (!loc) return false;
     static bool attr_set = false;
     if (!attr_set) {
         set_lds(ex_fwd_local_kernel<D, FROZEN>, kExFwdLds);
         attr_set = true;
     }
-    if (es.failed()) return;
-    {
-        KernelTimer kt("ex_fwd_local_kernel");
-        hipLaunchKernelGGL((ex_fwd_local_kernel<D, FROZEN>), dim3((unsigned)batch * maps), dim3(kThr), kExFwdLds, stream(), k, v, alpha, theta,
-                           has_s ? eta : alpha, loc, seq_len, input_stride, C, nc, maps, (int)has_s);
-        check_launch("ex_fwd_local_kernel");
+    for (int c0 = 0; c0 < maps && !es.failed(); c0 += stretch) {
+        const int n = c0 + stretch < maps ? stretch : maps - c0;
+        const size_t t0 = (size_t)c0 * C;
+        {
+            KernelTimer kt("ex_fwd_local_kernel");
+            hipLaunchKernelGGL((ex_fwd_local_kernel<D, FROZEN>), dim3((unsigned)batch * n), dim3(kThr), kExFwdLds, stream(), k + t0 * D,
+                               v + t0 * D, alpha + t0, theta + t0, (has_s ? eta : alpha) + t0, loc, seq_len - (int)t0, input_stride, C, n, n,
+                               (int)has_s);
+            check_launch("ex_fwd_local_kernel");
+        }
+        KernelTimer kt("ex_scan_kernel");
+        const dim3 grid((unsigned)batch * (D / 16));
+        float *ms = m_states + (size_t)c0 * sstep * DD, *ss = has_s ? s_states + (size_t)c0 * sstep * DD : nullptr;
+        const float *mi = c0 ? ms : m_initial, *si = c0 ? ss : s_initial;
+        const long long stride = c0 ? state_stride : m_stride;
+        if (has_s)
+            hipLaunchKernelGGL((ex_scan_kernel<D, true, false, true>), grid, dim3(8 * D), 0, stream(), loc, mi, si, stride, ms, ss,
+                               state_stride, sstep, nullptr, nullptr, n, n);
+        else
+            hipLaunchKernelGGL((ex_scan_kernel<D, false, false, true>), grid, dim3(4 * D), 0, stream(), loc, mi, nullptr, stride, ms, nullptr,
+                               state_stride, sstep, nullptr, nullptr, n, n);
+        check_launch("ex_scan_kernel");
     }
-    KernelTimer kt("ex_scan_kernel");
-    const dim3 grid((unsigned)batch * (D / 16));
-    if (has_s)
-        hipLaunchKernelGGL((ex_scan_kernel<D, true, false, true>), grid, dim3(8 * D), 0, stream(), loc, m_initial, s_initial, m_stride,
-                           m_states, s_states, state_stride, sstep, nullptr, nullptr, nc, maps);
-    else
-        hipLaunchKernelGGL((ex_scan_kernel<D, false, false, true>), grid, dim3(4 * D), 0, stream(), loc, m_initial, nullptr, m_stride,
-                           m_states, nullptr, state_stride, sstep, nullptr, nullptr, nc, maps);
-    check_launch("ex_scan_kernel");
+    return true;
 }
 
-void exact_forward_states(bool has_s, bool frozen, int d, int run, const float *k, const float *v, const float *alpha, const float *theta,
+bool exact_forward_states(bool has_s, bool frozen, int d, int run, const float *k, const float *v, const float *alpha, const float *theta,
                           const float *eta, const float *m_initial, const float *s_initial, long long m_stride, float *m_states,
                           float *s_states, long long state_stride, int sstep, int seq_len, int input_stride, int batch) {
     auto fn = frozen ? forward_states_t<32, true> : d == 64 ? forward_states_t<64, false> : forward_states_t<32, false>;
-    fn(has_s, k, v, alpha, theta, eta, m_initial, s_initial, m_stride, m_states, s_states, state_stride, sstep, seq_len, input_stride,
-       batch, run);
+    return fn(has_s, k, v, alpha, theta, eta, m_initial, s_initial, m_stride, m_states, s_states, state_stride, sstep, seq_len,
+              input_stride, batch, run);
 }
 
 template <int D, bool FROZEN, bool P64>

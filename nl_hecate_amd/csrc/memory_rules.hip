@@ -105,9 +105,9 @@ __global__ __launch_bounds__(kThreads) void rule_fwd_kernel(FwdArgs a) {
             M[r] = *reinterpret_cast<const float4 *>(mi + off);
             if (HAS_S) {
                 const float *si = sub ? so : a.s_initial + (size_t)chain * a.m_stride;
-                S[r] = *reinterpret_cast<const float4 *>(si + off);
+                if (STORE != STORE_LAST || a.s_initial) S[r] = *reinterpret_cast<const float4 *>(si + off);
             }
-            if (STORE != STORE_NONE && !sub) {
+            if (STORE != STORE_NONE && STORE != STORE_LAST && !sub) {
                 *reinterpret_cast<float4 *>(mo + off) = M[r];
                 if (HAS_S) *reinterpret_cast<float4 *>(so + off) = S[r];
             }
@@ -127,7 +127,7 @@ __global__ __launch_bounds__(kThreads) void rule_fwd_kernel(FwdArgs a) {
     TileRegs<D, TB> rk, rq, rv;
     GateRegs<TB> rg;
     rk.load(kb, 0, 0, seq_len, tid);
-    rq.load(qb, 0, 0, seq_len, tid);
+    if (STORE != STORE_LAST) rq.load(qb, 0, 0, seq_len, tid);
     rv.load(vb, 0, 0, seq_len, tid);
     rg.load(ab, tb, eb, 0, 0, seq_len, tid);
 
@@ -144,14 +144,14 @@ __global__ __launch_bounds__(kThreads) void rule_fwd_kernel(FwdArgs a) {
     for (int ti = 0; ti < ntiles; ti++) {
         const int buf = ti & 1, t0 = ti * TB;
         rk.store_lds(sk[buf], tid);
-        rq.store_lds(sq[buf], tid);
+        if (STORE != STORE_LAST) rq.store_lds(sq[buf], tid);
         rv.store_lds(sv[buf], tid);
         rg.store_lds(sg[buf], tid);
         __syncthreads();
-        if (ti > 0) flush_y(ti - 1);
+        if (STORE != STORE_LAST && ti > 0) flush_y(ti - 1);
         if (ti + 1 < ntiles) {
             rk.load(kb, t0 + TB, 0, seq_len, tid);
-            rq.load(qb, t0 + TB, 0, seq_len, tid);
+            if (STORE != STORE_LAST) rq.load(qb, t0 + TB, 0, seq_len, tid);
             rv.load(vb, t0 + TB, 0, seq_len, tid);
             rg.load(ab, tb, eb, t0 + TB, 0, seq_len, tid);
         }
@@ -166,7 +166,7 @@ __global__ __launch_bounds__(kThreads) void rule_fwd_kernel(FwdArgs a) {
                 if (!FAST && tl >= tn) break;
                 const int t = t0 + tl;
                 const float4 kk = *reinterpret_cast<const float4 *>(&sk[buf][tl * D + cb * 4]);
-                const float4 qq = *reinterpret_cast<const float4 *>(&sq[buf][tl * D + cb * 4]);
+                const float4 qq = STORE != STORE_LAST ? *reinterpret_cast<const float4 *>(&sq[buf][tl * D + cb * 4]) : f4_zero();
                 const float al = sg[buf][tl], th = sg[buf][TB + tl], et = sg[buf][2 * TB + tl];
                 const float ret = 1.f - al;
                 float e[RPL];
@@ -245,7 +245,7 @@ __global__ __launch_bounds__(kThreads) void rule_fwd_kernel(FwdArgs a) {
                     }
                 }
 #pragma unroll
-                for (int r = 0; r < RPL; r++) {
+                for (int r = 0; r < (STORE != STORE_LAST ? RPL : 0); r++) {
                     float yy = group_allreduce<LPR>(dot4(M[r], qq));
                     // all LPR lanes of the row hold yy: same-value store, no divergence
                     sy[buf][tl * ROWS_WG + row_local + r] = yy;
@@ -258,6 +258,12 @@ __global__ __launch_bounds__(kThreads) void rule_fwd_kernel(FwdArgs a) {
         else run_tile(std::false_type{});
     }
     __syncthreads();
+    if constexpr (STORE == STORE_LAST) {
+#pragma unroll
+        for (int r = 0; r < RPL; r++)
+            if (valid[r]) *reinterpret_cast<float4 *>(mo + (size_t)(row0 + r) * D + cb * 4) = M[r];
+        return;
+    }
     if (ntiles > 0) flush_y(ntiles - 1);
     if (TRACK) {
         const float tot = block_allreduce(nmax, sred[0], tid);
@@ -618,6 +624,11 @@ template <int D, int RPL, bool HAS_S, int STORE, bool FROZEN>
 static void launch_fwd_c(const FwdArgs &a, int batch, bool coupled) {
     dim3 grid(batch * a.parts), block(kThreads);
     KernelTimer kt("rule_fwd_kernel");
+    if constexpr (STORE == STORE_LAST) {   // no clip, no projection, no runs
+        hipLaunchKernelGGL((rule_fwd_kernel<D, RPL, HAS_S, STORE, 0, FROZEN>), grid, block, 0, stream(), a);
+        check_launch("rule_fwd_kernel");
+        return;
+    }
     if constexpr (STORE != STORE_NONE && (D == 64 || D == 32)) {
         if (a.sub_chunks > 1) {
             if (a.msq_part) hipLaunchKernelGGL((rule_fwd_kernel<D, RPL, HAS_S, STORE, 4, FROZEN>), grid, block, 0, stream(), a);
@@ -683,11 +694,12 @@ static bool launch_fwd_uncoupled(FwdArgs a, int d, int batch, int *tracked_rows)
                                 : exact_forward_mm_pays(a.seq_len, batch, d, false, run,
                                                         STORE == STORE_TRAJ ? 4LL * (HAS_S ? 2 : 1) * batch * a.seq_len * d * d : 0))) {
             const int sstep = FROZEN ? 1 : STORE == STORE_TRAJ ? run : run / a.ckpt_interval;
-            exact_forward_states(HAS_S, FROZEN, d, run, a.k, a.v, a.alpha, a.theta, a.eta, a.m_initial, a.s_initial, a.m_stride, a.m_out,
-                                 a.s_out, a.state_stride, sstep, a.seq_len, a.input_stride, batch);
-            a.sub_chunks = ceil_div(a.seq_len, run);
-            a.run_len = run;
-            rows *= a.sub_chunks;
+            if (exact_forward_states(HAS_S, FROZEN, d, run, a.k, a.v, a.alpha, a.theta, a.eta, a.m_initial, a.s_initial, a.m_stride,
+                                     a.m_out, a.s_out, a.state_stride, sstep, a.seq_len, a.input_stride, batch)) {
+                a.sub_chunks = ceil_div(a.seq_len, run);
+                a.run_len = run;
+                rows *= a.sub_chunks;
+            }
         }
     }
     if (tracked_rows) {
@@ -963,28 +975,18 @@ static void final_states(const char *fn, const float *k, const float *v, const f
     if (!check_dims(fn, seq_len, d, batch) || batch == 0) return;
     if (seq_len == 0) { fail("%s: seq_len=0.", fn); return; }
     const size_t dd = (size_t)d * d;
-    // three launches of the matrix form against one walk at 0.15 us a token (see exact_forward_mm_pays)
+    // two launches of the matrix form against one walk at 0.15 us a token (see exact_forward_mm_pays)
     if (exact_mm_applies(d, 1) && g_exact_form != 2 && (g_exact_form == 1 || exact_forward_mm_pays(seq_len, batch, d, true, kExactChunk, 0))) {
-        float *sf = HAS_S ? scratch(9, (size_t)batch * dd * sizeof(float)) : nullptr;
+        float *sf = HAS_S ? scratch_if_free(41, (size_t)batch * dd * sizeof(float)) : nullptr;
+        if ((sf || !HAS_S) &&
+            exact_forward_states(HAS_S, false, d, kExactChunk, k, v, alpha, theta, eta, m_initial, s_initial, (long long)dd, m_final, sf,
+                                 (long long)dd, 0, seq_len, seq_len, batch))
+            return;
         if (es.failed()) return;
-        exact_forward_states(HAS_S, false, d, kExactChunk, k, v, alpha, theta, eta, m_initial, s_initial, (long long)dd, m_final, sf, (long long)dd, 0, seq_len,
-                             seq_len, batch);
-        return;
     }
-    float *m2 = scratch(5, 2 * batch * dd * sizeof(float)), *s2 = HAS_S ? scratch(6, 3 * batch * dd * sizeof(float)) : nullptr;
-    float *y = scratch(7, (size_t)batch * seq_len * d * sizeof(float));
-    if (es.failed()) return;
-    if (HAS_S && !s_initial) {
-        float *z = s2 + 2 * batch * dd;
-        hipLaunchKernelGGL(zero_fill_kernel, dim3(ceil_div(batch * dd, 256)), dim3(256), 0, stream(), z, (size_t)batch * dd);
-        check_launch("zero_fill_kernel");
-        s_initial = z;
-    }
-    FwdArgs a{k, v, k, alpha, theta, eta, m_initial, s_initial, m2, s2, y, seq_len, seq_len, seq_len, 1, (long long)dd,
-              (long long)(2 * dd), 0.f, 0.f};
-    if (!launch_fwd<HAS_S, STORE_CKPT>(a, d, batch)) { unsupported(fn, d, false); return; }
-    check_hip(hipMemcpy2DAsync(m_final, dd * sizeof(float), m2 + dd, 2 * dd * sizeof(float), dd * sizeof(float), batch,
-                               hipMemcpyDeviceToDevice, stream()), fn);
+    const FwdArgs a{k, v, k, alpha, theta, eta, m_initial, s_initial, m_final, nullptr, nullptr, seq_len, seq_len, seq_len, 1, (long long)dd,
+                    (long long)dd, 0.f, 0.f};
+    if (!launch_fwd_as<HAS_S, STORE_LAST, false>(a, d, batch, false)) unsupported(fn, d, false);
 }
 
 // ───────────────────────────── C ABI ───────────────────────────────────────

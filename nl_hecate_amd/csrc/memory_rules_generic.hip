@@ -61,9 +61,9 @@ __global__ __launch_bounds__(kGThr) void rule_fwd_generic_kernel(FwdArgs a, int 
     float *mo = a.m_out + (size_t)chain * a.state_stride;
     float *so = HAS_S ? a.s_out + (size_t)chain * a.state_stride : nullptr;
     const float *mi = a.m_initial + (size_t)chain * a.m_stride;
-    const float *si = HAS_S ? a.s_initial + (size_t)chain * a.m_stride : nullptr;
-    // current state: slot t of the trajectory, or the work buffers
-    float *cm = STORE == STORE_TRAJ ? mo : work_m + (size_t)chain * dd;
+    const float *si = HAS_S && (STORE != STORE_LAST || a.s_initial) ? a.s_initial + (size_t)chain * a.m_stride : nullptr;
+    // current state: slot t of the trajectory, the final state's place, or the work buffers
+    float *cm = STORE == STORE_TRAJ || STORE == STORE_LAST ? mo : work_m + (size_t)chain * dd;
     float *cs = HAS_S ? (STORE == STORE_TRAJ ? so : work_s + (size_t)chain * dd) : nullptr;
     float *m0 = FROZEN ? work_m0 + (size_t)chain * dd : nullptr;
     for (size_t e = tid; e < dd; e += kGThr) {
@@ -72,7 +72,7 @@ __global__ __launch_bounds__(kGThr) void rule_fwd_generic_kernel(FwdArgs a, int 
         if (STORE == STORE_CKPT) mo[e] = mv;
         if (FROZEN) m0[e] = mv;
         if (HAS_S) {
-            const float svv = si[e];
+            const float svv = STORE != STORE_LAST || si ? si[e] : 0.f;
             cs[e] = svv;
             if (STORE == STORE_CKPT) so[e] = svv;
         }
@@ -136,7 +136,7 @@ __global__ __launch_bounds__(kGThr) void rule_fwd_generic_kernel(FwdArgs a, int 
             }
             ckpt_slot++;
         }
-        row_products(cm, sq, nullptr, yb + (size_t)t * d, d);   // y = M_{t+1} q
+        if (STORE != STORE_LAST) row_products(cm, sq, nullptr, yb + (size_t)t * d, d);   // y = M_{t+1} q
         __syncthreads();   // the vectors and (frozen) M0 are rewritten next
     }
 }
@@ -253,7 +253,7 @@ void launch_fwd_generic(const FwdArgs &a, int d, int batch, bool has_s, int stor
     const ErrorScope es;
     const size_t dd = (size_t)d * d, lds = (4 * (size_t)d + kGWaves) * sizeof(float);
     if (lds > 64 * 1024) { fail("memory rule: d=%d is beyond the general kernels' LDS vectors (d <= 4000).", d); return; }
-    float *wm = store != STORE_TRAJ ? scratch(16, (size_t)batch * dd * sizeof(float)) : nullptr;
+    float *wm = store != STORE_TRAJ && store != STORE_LAST ? scratch(16, (size_t)batch * dd * sizeof(float)) : nullptr;
     float *ws = (store != STORE_TRAJ && has_s) ? scratch(17, (size_t)batch * dd * sizeof(float)) : nullptr;
     float *w0 = frozen ? scratch(18, (size_t)batch * dd * sizeof(float)) : nullptr;
     if (es.failed()) return;
@@ -265,6 +265,7 @@ void launch_fwd_generic(const FwdArgs &a, int d, int batch, bool has_s, int stor
     do {                                                       \
         if (store == STORE_TRAJ) NLH_GF(HS, STORE_TRAJ, FZ);   \
         else if (store == STORE_CKPT) NLH_GF(HS, STORE_CKPT, FZ); \
+        else if (store == STORE_LAST) NLH_GF(HS, STORE_LAST, FZ); \
         else NLH_GF(HS, STORE_NONE, FZ);                       \
     } while (0)
     if (has_s) { if (frozen) NLH_GF_ST(true, true); else NLH_GF_ST(true, false); }

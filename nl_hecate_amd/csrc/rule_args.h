@@ -21,7 +21,9 @@ struct FwdArgs {
     int sub_chunks, run_len;
 };
 
-enum { STORE_NONE = 0, STORE_TRAJ = 1, STORE_CKPT = 2 };
+// STORE_LAST: M after the last token only (m_out one matrix a chain, may be m_initial; s_initial null: zero), no outputs,
+// q not read
+enum { STORE_NONE = 0, STORE_TRAJ = 1, STORE_CKPT = 2, STORE_LAST = 3 };
 
 // Reverse sweep over [t_start, t_end) of every chain, reading the trajectory
 // M_{t_start..t_end}, S_{t_start..t_end-1} from memory (the reference's

@@ -30,6 +30,8 @@ struct Slot {
     void *ptr = nullptr;
     size_t bytes = 0;
     int device = -1;
+    bool owned = false;            // scratch_if_free: by the stream that took it first
+    hipStream_t owner = nullptr;
 };
 static Slot g_slots[kScratchSlots];
 
@@ -103,6 +105,38 @@ float *scratch(int slot, size_t bytes) {
     if (!s.ptr) return nullptr;
     s.bytes = want;
     s.device = dev;
+    return (float *)s.ptr;
+}
+
+float *scratch_if_free(int slot, size_t bytes) {
+    if (slot < 0 || slot >= kScratchSlots || bytes > kOptionalScratch) return nullptr;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(g_stream, &cap) != hipSuccess) {
+        (void)hipGetLastError();   // a legacy stream while another one is being captured: not ours to use either
+        return nullptr;
+    }
+    if (cap != hipStreamCaptureStatusNone) return nullptr;
+    Slot &s = g_slots[slot];
+    if (s.owned && s.owner != g_stream) return nullptr;
+    int dev = 0;
+    check_hip(hipGetDevice(&dev), "hipGetDevice");
+    if (s.ptr && s.device != dev) return nullptr;
+    if (s.bytes < bytes) {
+        if (s.ptr) {   // no captured graph holds this address: the generation stays
+            check_hip(hipStreamSynchronize(g_stream), "scratch: hipStreamSynchronize");
+            check_hip(hipFree(s.ptr), "scratch: hipFree");
+            s = Slot();
+        }
+        if (hipMalloc(&s.ptr, bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            s.ptr = nullptr;
+            return nullptr;
+        }
+        s.bytes = bytes;
+        s.device = dev;
+    }
+    s.owned = true;
+    s.owner = g_stream;
     return (float *)s.ptr;
 }
 
