@@ -336,18 +336,15 @@ def linear_group(op, a, b, c, m, n, k, bf16_mask=0):
                                   (bf16_mask >> i) & 0xffffffff, m, n, k)
 
 
-def forward_group(params, cfgs, embedded, contexts, s, d, bs, extra=()):
-    """gpu_memory_forward of a group of levels.  extra: (weight, output) pairs of further projections of `embedded` (a bf16
-    output is rounded at the store).  Returns (y [levels, bs*s, d], [cache per level])."""
+def forward_group(params, cfgs, embedded, contexts, s, d, bs):
+    """gpu_memory_forward of a group of levels.  Returns (y [levels, bs*s, d], [cache per level])."""
     cfg, L = cfgs[0], len(cfgs)
     nh, hd = cfg.num_heads, cfg.head_dim
     n, B, dd = bs * s, bs * nh, hd * hd
     titans = cfg.memory_rule == "titans"
     proj = _new(3 * L, n, d)
     mem = list(proj.unbind(0))
-    linear_group(0, [embedded] * (3 * L + len(extra)),
-                 [w for lp in params for w in (lp.w_k, lp.w_v, lp.w_q)] + [w for w, _ in extra], mem + [o for _, o in extra],
-                 n, d, d, sum(1 << (3 * L + i) for i, (_, o) in enumerate(extra) if o.dtype == torch.bfloat16))
+    linear_group(0, [embedded] * (3 * L), [w for lp in params for w in (lp.w_k, lp.w_v, lp.w_q)], mem, n, d, d)
     gate = _new(5 * L, n)
     rows = list(gate.unbind(0))   # per level: k_norms, q_norms, alpha, theta, eta
     heads, gates = _new(3, L * B, s, hd), _new(3 if titans else 2, L * B, s)
