@@ -49,11 +49,6 @@ struct DecArgs {
 };
 
 __device__ __forceinline__ float bf2f(uint16_t u) { return __uint_as_float((uint32_t)u << 16); }
-__device__ __forceinline__ uint16_t f2bf(float x) {   // round to nearest even; NaN stays NaN
-    uint32_t u = __float_as_uint(x);
-    if ((u & 0x7fffffffu) > 0x7f800000u) return (uint16_t)((u >> 16) | 0x40);
-    return (uint16_t)((u + 0x7fffu + ((u >> 16) & 1u)) >> 16);
-}
 __device__ __forceinline__ float dot4(const float4 &a, const float4 &b) { return a.x * b.x + a.y * b.y + a.z * b.z + a.w * b.w; }
 
 __host__ __device__ inline bool reads_only(int rule) { return rule < 0 || rule == 3; }
@@ -102,7 +97,7 @@ __global__ __launch_bounds__(kDecThr) void decode_project_kernel(DecArgs a) {
     if (lane < 4) {
         const float y = lane == 0 ? acc[0] : lane == 1 ? acc[1] : lane == 2 ? acc[2] : acc[3];
         if (out) out[r + lane] = y;
-        else out16[r + lane] = f2bf(y);
+        else out16[r + lane] = f32_to_bf16_rne(y);
     }
     if (blockIdx.x == 0)
         for (int i = threadIdx.x; i < n4; i += kDecThr) reinterpret_cast<float4 *>(a.embedded)[i] = x[i];
@@ -336,7 +331,7 @@ __global__ __launch_bounds__(kDecThr) void decode_output_kernel(DecArgs a) {
 #pragma unroll
             for (int j = 0; j < 4; j++) o += s + j < a.slices ? wgt[(s + j) * a.nh + h] * t[j] : 0.f;
         }
-        const uint16_t o16 = f2bf(o);
+        const uint16_t o16 = f32_to_bf16_rne(o);
         y *= scale;
         const float g = 1.f / (1.f + expf(-y)), at = bf2f(o16);
         gated[i] = at * g;

@@ -15,6 +15,7 @@
 #include <stdint.h>
 
 #include "../../include/nl_hecate_ffi.h"
+#include "lane_ops.h"
 #include "runtime.h"
 
 namespace nlh {
@@ -30,12 +31,6 @@ struct GroupArgs {
     int count, m, n, k, tiles_n, steps, splits;
     float *part;            // splits > 1: [split][m][n]
 };
-
-__device__ __forceinline__ uint16_t to_bf16(float x) {   // round to nearest even; NaN stays NaN
-    uint32_t u = __float_as_uint(x);
-    if ((u & 0x7fffffffu) > 0x7f800000u) return (uint16_t)((u >> 16) | 0x40);
-    return (uint16_t)((u + 0x7fffu + ((u >> 16) & 1u)) >> 16);
-}
 
 // A [ROWS x BK] tile of a row-major operand, contraction contiguous (KC) or rows contiguous.
 template <bool KC, int ROWS, int NTHR>
@@ -157,7 +152,7 @@ __global__ __launch_bounds__(64 * WM * WN) void group_gemm_kernel(GroupArgs g) {
             for (int e = 0; e < 4; e++) {
                 const int row = m0 + wm + 16 * i + 4 * (l >> 4) + e;
                 if (row < g.m && col < g.n) {
-                    if (b16) reinterpret_cast<uint16_t *>(c)[(size_t)row * g.n + col] = to_bf16(acc[i][j][e]);
+                    if (b16) reinterpret_cast<uint16_t *>(c)[(size_t)row * g.n + col] = f32_to_bf16_rne(acc[i][j][e]);
                     else c[(size_t)row * g.n + col] = acc[i][j][e];
                 }
             }

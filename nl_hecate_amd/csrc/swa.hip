@@ -27,12 +27,6 @@ namespace nlh {
 constexpr int kSwaWaves = 4;
 
 __device__ __forceinline__ float bf2f(unsigned short h) { return __uint_as_float(((unsigned)h) << 16); }
-__device__ __forceinline__ unsigned short f2bf(float f) {
-    unsigned u = __float_as_uint(f);
-    if ((u & 0x7fffffffu) > 0x7f800000u) return (unsigned short)((u >> 16) | 0x40);
-    u += 0x7fffu + ((u >> 16) & 1u);
-    return (unsigned short)(u >> 16);
-}
 
 // Orders one wave's LDS writes before reads by its other lanes.
 __device__ __forceinline__ void wave_sync() {
@@ -126,7 +120,7 @@ __global__ __launch_bounds__(kSwaWaves * 64) void swa_forward_kernel(
     for (int s = lane; s < aw; s += 64) {
         const float w = sc[s] * inv;
         sc[s] = w;
-        wr[s] = f2bf(w);
+        wr[s] = f32_to_bf16_rne(w);
     }
     wave_sync();
     // out[d] = sum_s w_s v[key_s][d]  (unrounded weights, as the reference)
@@ -134,7 +128,7 @@ __global__ __launch_bounds__(kSwaWaves * 64) void swa_forward_kernel(
         float acc = 0.f;
         for (int s = 0; s < g.n_p; s++) acc += sc[s] * bf2f(vb[(size_t)s * td + d]);
         for (int w = 0; w < g.ll; w++) acc += sc[n_persistent + w] * bf2f(vb[(size_t)(g.ls + w) * td + d]);
-        out[(b * seq_len + t) * td + h * head_dim + d] = f2bf(acc);
+        out[(b * seq_len + t) * td + h * head_dim + d] = f32_to_bf16_rne(acc);
     }
 }
 
@@ -302,7 +296,7 @@ __global__ __launch_bounds__(kDecThreads) void swa_single_token_kernel(
     __syncthreads();
     if (grp == 0) {
         for (int gg = 1; gg < ngrp; gg++) acc += red[gg * head_dim + d];
-        out[hoff + d] = f2bf(acc);
+        out[hoff + d] = f32_to_bf16_rne(acc);
     }
 }
 
