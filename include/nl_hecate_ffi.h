@@ -76,9 +76,10 @@ int nlh_selftest_chunk_coef_prepass(const float *alpha, const float *theta, cons
  * outputs use the local seq_len: y [batch, seq_len, d],
  * m_states / s_states [batch, seq_len+1, d*d].
  * error_clip <= 0 and m_norm_max <= 0 or >= 1e30 disable clip / projection.
- * The forwards of the exact and frozen rules need no scratch memory.  Head sizes 32 and 64 take up to 256 MiB of it for
- * few long chains, where it is free to take: not while the launch stream is being captured, and on the first stream that
- * took it only (until nlh_release_workspace); otherwise they walk the tokens.  So does *_final_states_f32_rocm. */
+ * The forwards of the exact rule, and of the frozen rule at head size 32, need no scratch memory.  At head sizes 32 and 64
+ * they take up to 256 MiB of it for few long chains, where it is free to take: not while the launch stream is being
+ * captured, and on the first stream that took it only (until nlh_release_workspace); otherwise they walk the tokens.  So do
+ * the *_final_states_f32_rocm. */
 /* core/src/cuda_ffi.rs:134 */
 void titans_forward_f32_cuda(const float *k_mem, const float *v_mem, const float *q_mem,
                              const float *alpha, const float *theta, const float *eta,
