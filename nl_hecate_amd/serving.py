@@ -150,6 +150,15 @@ class DecodeWorkspace:
         self.plans = {}
         self.logits_host = torch.empty(v, dtype=torch.float32, pin_memory=True)
 
+    def __getstate__(self):
+        """Copied and saved without what holds addresses."""
+        return {n: t for n, t in self.__dict__.items() if n not in ("work", "plans")}
+
+    def __setstate__(self, state):
+        host = state.get("logits_host")   # absent from what was saved before the one-call step
+        self.__dict__.update(state, work=_new(0), plans={}, logits_host=(
+            torch.empty(state["logits_gpu"].shape[-1]) if host is None else host).pin_memory())
+
     def written(self):
         """What the one-call step writes besides the logits on the host, in the order of its argument block."""
         return (self.embedded, self.q_bf16, self.attn_out_bf16, self.attn_out, self.y_combined, self.gate, self.gated_out,

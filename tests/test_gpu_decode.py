@@ -257,3 +257,49 @@ def test_windows_past_what_one_call_merges():
         want = np.einsum("ht,thc->hc", w, host(kv.v_cache_bf16[:start + 1].float()).reshape(-1, nh, hd))
         assert np.abs(host(ws.attn_out).reshape(nh, hd) - want).max() <= 2e-2 * np.abs(want).max()
     assert np.isfinite(out).all()
+
+
+@pytest.mark.parametrize("how", ["deepcopy", "pickle"])
+def test_a_used_workspace_can_be_copied_and_saved(how):
+    import copy
+    import pickle
+    gp, cfg, pulse, ctx, kv, ws = small()
+    first = ctx.memory[0].clone()
+    want = SG.gpu_single_token_forward(gp, cfg, 3, pulse, ctx, kv, ws)
+    other = copy.deepcopy(ws) if how == "deepcopy" else pickle.loads(pickle.dumps(ws))
+    assert np.array_equal(host(other.logits_gpu)[0], want) and np.array_equal(other.logits_host.numpy(), want)
+    ws.logits_gpu.zero_()
+    ctx.memory[0].copy_(first)
+    kv.len -= 1
+    assert np.array_equal(SG.gpu_single_token_forward(gp, cfg, 3, pulse, ctx, kv, other), want)
+    assert not host(ws.logits_gpu).any() and np.array_equal(host(other.logits_gpu)[0], want)
+    assert list(other.plans.values())[0][1] is not None
+    old = object.__new__(SG.DecodeWorkspace)
+    old.__setstate__({n: t for n, t in ws.__getstate__().items() if n != "logits_host"})
+    kv.len -= 1
+    ctx.memory[0].copy_(first)
+    assert np.array_equal(SG.gpu_single_token_forward(gp, cfg, 3, pulse, ctx, kv, old), want)
+
+
+def test_non_finite_cache_entries(monkeypatch):
+    """NaN and infinities among the cached keys and values end up where the step by operations has them."""
+    gp, cfg, pulse, ctx, kv, ws = small()
+    first = ctx.memory[0].clone()
+    k0, v0 = kv.k_cache_bf16.clone(), kv.v_cache_bf16.clone()
+    in_one = SG._decode_in_one_call
+    for place in ("k nan", "k inf", "k -inf", "all k -inf", "v nan", "v inf"):
+        kv.k_cache_bf16.copy_(k0)
+        kv.v_cache_bf16.copy_(v0)
+        cache = kv.k_cache_bf16 if "k" in place else kv.v_cache_bf16
+        cache[slice(None) if "all" in place else slice(4, 5), 3 if "k" in place else 40] = float(place.split()[-1])
+        out = []
+        for one in (True, False):
+            monkeypatch.setattr(SG, "_decode_in_one_call", in_one if one else lambda *a: None)
+            ctx.memory[0].copy_(first)
+            kv.len = cfg.seq_len
+            SG.gpu_single_token_forward(gp, cfg, 3, pulse, ctx, kv, ws)
+            out.append(host(ws.attn_out)[0].copy())
+        a, b = out
+        assert np.array_equal(np.isfinite(a), np.isfinite(b)), place
+        ok = np.isfinite(b)
+        assert np.abs(a[ok] - b[ok]).max(initial=0) <= 2e-2 * np.abs(b[ok]).max(initial=1), place
