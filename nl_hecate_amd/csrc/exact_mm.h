@@ -5,7 +5,7 @@
 namespace nlh {
 
 // Backward from states kept every C <= 64 tokens, m_ckpt / s_ckpt [batch][n_ckpt_count(seq_len, C)][d*d] (C = 1: the full
-// trajectory).  Sums in float64 at head size 32 and from full trajectories, in fp32 otherwise.
+// trajectory).  Sums in float64 at head size 32 and below 32 tokens an interval, in fp32 otherwise.
 bool exact_mm_applies(int d, int C);
 // faster than the sequential kernel at this shape (tested: under a clip or a bound)
 bool exact_backward_mm_pays(int seq_len, int batch, int d, int C, bool tested, bool frozen);

@@ -35,14 +35,14 @@
 //
 // P64: which sums are float64 (mm_tiles.h).  The walks that this form stands in for add a row's product up in a tree and
 // are 0.6 to 1.2e-7 off the exact gradients (gates spread over (0, 1); 2 to 4e-7 where the states live for 150 tokens); with
-// fp32 sums throughout the form is at 1.5 to 2.6e-7.  So wherever a walk was replaced, head size 32, full trajectories
-// and the forward's chunk maps, the coefficients' recurrences, the gate sweeps and every product whose rounding reaches a
-// result are float64 sums rounded once: 0.6 to 1.0e-7, each output at or below its walk over spread gates, gates at a
-// model's start and long-lived states.  Left in fp32 are the products that do not show: the inverse, K K^T, K M^T, the maps
+// fp32 sums throughout the form is at 1.5 to 2.6e-7.  So wherever a walk was replaced (wide_sums, and the forward's chunk
+// maps), the coefficients' recurrences, the gate sweeps and every product whose rounding reaches a result are float64 sums
+// rounded once: 0.6 to 1.0e-7, each output at or below its walk over spread gates, gates at a model's start and long-lived
+// states.  Left in fp32 are the products that do not show: the inverse, K K^T, K M^T, the maps
 // of the adjoint scan and the products with the adjoint at the chunk's end.  512 tokens of 32 chains, head size 64: first
 // kernel 38 -> 46 us, gradients 38 -> 65, scan 16 -> 23, gates 10 -> 15; head size 32, 777 tokens of 16: 21 -> 25, 24 -> 32,
-// 5 -> 8, 7 -> 9.  Checkpointed head size 64 keeps fp32 sums: it never replaced a more exact path at these entry points, and
-// its two kernels are bound by their products.
+// 5 -> 8, 7 -> 9.  Head size 64 with checkpoints every 32 tokens and more keeps fp32 sums: there the form is the path that
+// there was, and its two kernels are bound by their products.
 //
 // Under a finite m_norm_max / error clip the pass also leaves the ChainTracks of chunkwise_chain.h behind (|u_t|^2 per
 // token, sums of squares of the checkpoints); the caller tests on them whether a coupling could have fired.
@@ -814,6 +814,10 @@ bool exact_mm_applies(int d, int C) { return (d == 64 || d == 32) && C >= 1 && C
 // whatever its length, and only the states at chunk starts are read.
 static int chunk_of(int C) { return C * (CW / C); }
 
+// Float64 sums (above) for what the walks served: head size 32, full trajectories, and intervals below 32, which pay since
+// a chunk spans several of them.
+static bool wide_sums(int d, int C) { return d == 32 || C < 32; }
+
 // Cost models from measurements on one MI355X (us).  A chunk costs the two chunk-parallel kernels of the backward about
 // 65 us of a compute unit whatever its length (95 with float64 sums, 54 at head size 32), a scan step 2.0 (2.9, 0.65); the
 // fused sequential kernel walks a chain's tokens at 0.6 each on a quarter of a compute unit's worth of workgroups (four per
@@ -821,7 +825,7 @@ static int chunk_of(int C) { return C * (CW / C); }
 // errors adds two launches to the matrix form where the fused kernel's only adds one on its maxima.
 bool exact_backward_mm_pays(int seq_len, int batch, int d, int C, bool tested, bool frozen) {
     const int nc = ceil_div(seq_len, frozen ? C : chunk_of(C)), cus = compute_units();
-    const bool wide = C == 1;
+    const bool wide = wide_sums(d, C);
     const double chunk = d == 32 ? 54.0 : wide ? 95.0 : 65.0, step = d == 32 ? 0.65 : wide ? 2.9 : 2.0;
     const double t_mm = (double)ceil_div(batch * nc, cus) * chunk + nc * step + (tested ? 20.0 : 10.0);
     const double t_seq = (double)seq_len * (C == 1 ? 1.1 : 0.6) * ceil_div(batch * (d == 64 ? 4 : 1), cus);
@@ -982,7 +986,7 @@ bool exact_backward_mm(const char *fn, bool has_s, bool frozen, int d, const flo
     }
     auto run = frozen ? backward_mm_t<32, true, true>
                : d == 32 ? backward_mm_t<32, false, true>
-               : C == 1 ? backward_mm_t<64, false, true> : backward_mm_t<64, false, false>;
+               : wide_sums(d, C) ? backward_mm_t<64, false, true> : backward_mm_t<64, false, false>;
     return run(fn, has_s, k, v, q, alpha, theta, eta, m_ckpt, s_ckpt, d_y, d_k, d_v, d_q, d_alpha, d_theta, d_eta, d_m_initial,
                d_s_initial, seq_len, batch, C, error_clip, m_norm_guard);
 }
