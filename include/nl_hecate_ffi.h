@@ -674,6 +674,8 @@ void swa_single_token_cuda(const uint16_t *q, const uint16_t *k_cache, const uin
  *   Pointer arrays are host arrays of `count` <= 32 device pointers; row lengths multiples of 4. */
 void linear_group_f32_rocm(int op, int count, const float *const *a, const float *const *b, void *const *c,
                            unsigned bf16_mask, int m, int n, int k);
+/* One product of any size, operands as for op of linear_group (op 1: count = 1). */
+void product_f32_rocm(int op, const float *a, const float *b, float *c, int m, int n, int k);
 /* ptrs: host array of 14 device pointers per level: k, v, q [bs*s, d] (k, q normalised in place), w_alpha, b_alpha,
  * w_theta, b_theta, w_eta, b_eta, then written: k_norms, q_norms, alpha, theta, eta [bs*s].  bounds: 4 per level: alpha
  * floor / ceil, theta floor / ceil.  *_heads [levels*bs*nh, s, hd], [levels*bs*nh, s].  q_heads null: no q (its pointers

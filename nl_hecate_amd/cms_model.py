@@ -25,7 +25,7 @@ from . import dispatch as D
 from .cms import ContextState, Pulse
 from .ffi import lib
 from .memory_level import (LevelConfig, LevelGrads, _plain, _ptrs, backward_group, forward_group, gpu_memory_backward,
-                           gpu_memory_forward, group_key, linear_group)
+                           gpu_memory_forward, group_key, linear_group, product)
 from .serving import GpuMAGParams, frozen_level_output, host_ids
 from .tnt import ParallelConfig, gpu_tnt_backward, gpu_tnt_forward
 
@@ -186,7 +186,11 @@ def gpu_cms_forward(params: GpuMAGParams, cfg: ModelConfig, input_ids, target_id
         lib.cms_combine_gate_rocm(ptrs, len(ys), c["attn_out"].data_ptr(), c["y_combined"].data_ptr(),
                                   c["gate"].data_ptr(), c["gated_out"].data_ptr(), n * d)
         c["projected"] = c["gated_out"] @ params.w_o.t()
-    c["logits"] = c["projected"] @ params.w_unembed
+    if _plain(params.w_unembed, d, v):
+        c["logits"] = _new(n, v)
+        product(1, c["projected"], params.w_unembed, c["logits"], n, v, d)
+    else:
+        c["logits"] = c["projected"] @ params.w_unembed
     loss_gpu = _new(1)
     D.call("cross_entropy_forward_cuda", c["logits"], tgt, loss_gpu, n, v)
     valid = c["valid"] = int(((tgt_host >= 0) & (tgt_host < v)).sum())
@@ -212,12 +216,12 @@ def gpu_cms_backward(params: GpuMAGParams, cfg: ModelConfig, cache, collect_outp
     valid = c["valid"]
     d_logits = _new(n, v)
     D.call("cross_entropy_backward_cuda", c["logits"], c["target_ids"], d_logits, n, v, 1.0 / (valid if valid > 0 else 1))
-    if v % 4 == 0 and d % 4 == 0 and _plain(params.w_unembed, d, v):   # a contraction over the vocabulary for few output tiles
+    if _plain(params.w_unembed, d, v):   # a contraction over the vocabulary for few output tiles
         d_projected = _new(n, d)
-        linear_group(0, [d_logits], [params.w_unembed], [d_projected], n, d, v)
+        product(0, d_logits, params.w_unembed, d_projected, n, d, v)
     else:
         d_projected = d_logits @ params.w_unembed.t()
-    torch.mm(c["projected"].t(), d_logits, out=g.d_w_unembed)
+    product(2, c["projected"], d_logits, g.d_w_unembed, d, v, n)
     d_gated_out = d_projected @ params.w_o
     torch.mm(d_projected.t(), c["residual_final"] if cfg.residual else c["gated_out"], out=g.d_w_o)
     if cfg.residual:

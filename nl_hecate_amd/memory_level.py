@@ -336,6 +336,11 @@ def linear_group(op, a, b, c, m, n, k, bf16_mask=0):
                                   (bf16_mask >> i) & 0xffffffff, m, n, k)
 
 
+def product(op, a, b, c, m, n, k):
+    """One product of any size (product_f32_rocm); operands as for op of linear_group, contiguous float32."""
+    lib.product_f32_rocm(op, a.data_ptr(), b.data_ptr(), c.data_ptr(), m, n, k)
+
+
 def forward_group(params, cfgs, embedded, contexts, s, d, bs):
     """gpu_memory_forward of a group of levels.  Returns (y [levels, bs*s, d], [cache per level])."""
     cfg, L = cfgs[0], len(cfgs)

@@ -45,6 +45,47 @@ def test_grouped_products(op, count, m, n, k):
             assert (h.float() - got).abs().max().item() <= 2 ** -7 * got.abs().max().item()
 
 
+@pytest.mark.parametrize("op,m,n,k", [(0, 1, 1, 1), (0, 257, 129, 31), (0, 300, 130, 33), (0, 512, 510, 4097), (0, 2100, 2060, 64),
+                                      (1, 3, 2, 5), (1, 255, 127, 65), (1, 513, 8001, 96), (1, 130, 70, 2000), (2, 1, 3, 7),
+                                      (2, 129, 1003, 50), (2, 512, 8193, 97), (2, 65, 65, 1)])
+def test_single_products_of_any_size(op, m, n, k):
+    print(op, m, n, k, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    shp_a, shp_b = {0: ((m, k), (n, k)), 1: ((m, k), (k, n)), 2: ((k, m), (k, n))}[op]
+    a, b = [torch.randn(*s, generator=g, device="cuda") for s in (shp_a, shp_b)]
+    c = torch.full((m * n + 4,), 7.5, device="cuda")
+    ML.product(op, a, b, c, m, n, k)
+    assert (c[m * n:] == 7.5).all()
+    fit = {0: lambda a, b: a @ b.t(), 1: lambda a, b: a @ b, 2: lambda a, b: a.t() @ b}[op]
+    want, got = fit(a.double(), b.double()), c[:m * n].view(m, n).double()
+    # every product of two floats is kept to 2^-24 of it, every sum of 32 rounds; fp32 products added one by one: as above
+    assert (got - want).abs().max().item() <= 8 * 2 ** -24 * k + 1e-6
+    if k >= 64:   # no further from float64 than sums term by term
+        assert (got - want).norm().item() <= (fit(a, b).double() - want).norm().item()
+    # magnitudes: the pieces of a float follow it down to the last of a bf16's range, 2^-133
+    for scale_a, scale_b in ((2. ** -90, 2. ** 80), (2. ** 100, 2. ** -60), (2. ** -112, 1.)):
+        ML.product(op, a * scale_a, b * scale_b, c, m, n, k)
+        assert (c[:m * n].view(m, n).double() / (scale_a * scale_b) - want).abs().max().item() <= 8 * 2 ** -24 * k + 1e-6
+
+
+@pytest.mark.parametrize("op", [0, 1, 2])
+@pytest.mark.parametrize("m,n,k", [(600, 1300, 64), (72, 67, 35)])
+def test_single_products_keep_non_finite_values_in_their_place(op, m, n, k):
+    g = torch.Generator(device="cuda").manual_seed(5)
+    shp_a, shp_b = {0: ((m, k), (n, k)), 1: ((m, k), (k, n)), 2: ((k, m), (k, n))}[op]
+    a, b = [torch.randn(*s, generator=g, device="cuda") for s in (shp_a, shp_b)]
+    a[3, 5], a[-1, 1], b[2, 7], b[-1, -1] = float("nan"), float("inf"), -float("inf"), 3.4e38
+    c = torch.zeros(m, n, device="cuda")
+    ML.product(op, a, b, c, m, n, k)
+    x, y = {0: (a, b.t()), 1: (a, b), 2: (a.t(), b)}[op]
+    want = sum(x[:, i, None].double() * y[None, i].double() for i in range(k))
+    want = torch.where(want.abs() > 3.5e38, want.sign() * float("inf"), want)
+    near = (want.abs() > 3.3e38) & want.isfinite()   # a sum on either side of the largest float
+    assert torch.equal(c.isnan() | near, want.isnan() | near) and torch.equal(c.isinf() | near, want.isinf() | near)
+    ok = want.isfinite() & ~near
+    assert ((c.double() - want)[ok].abs() <= 8 * 2 ** -24 * k * want[ok].abs().clamp(min=1)).all()
+
+
 @pytest.mark.parametrize("count,m,n,k", [(7, 1000, 1024, 1024), (6, 2000, 512, 512), (12, 512, 512, 512)])
 def test_sum_over_products_rounds_like_products_added_up(count, m, n, k):
     g = torch.Generator(device="cuda").manual_seed(1)
