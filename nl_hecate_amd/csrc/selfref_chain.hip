@@ -22,23 +22,28 @@
 namespace nlh {
 namespace {
 
-template <int LANE>
-__device__ __forceinline__ void set_lane(float &x, float uniform) {
-    asm("v_writelane_b32 %0, %1, %2" : "+v"(x) : "s"(uniform), "n"(LANE));
-}
 template <int Q>
 __device__ __forceinline__ float quad_lane(float x) { return dpp_mov<Q * 0x55>(x); }
-// The gates without a branch: the argument is uniform and the value is needed at once.
-__device__ __forceinline__ float sr_sigmoid_select(float x) {
-    const float y = __builtin_amdgcn_rcpf(1.f + __expf(-x));
+// The gates of x without a branch, from e = 1 + exp(-x) and e = 1 + exp(x).
+__device__ __forceinline__ float sigmoid_of(float x, float e) {
+    const float y = __builtin_amdgcn_rcpf(e);
     return x >= 15.f ? 1.f : x <= -15.f ? 0.f : y;
 }
-__device__ __forceinline__ float sr_softplus_select(float x) {
+__device__ __forceinline__ float softplus_of(float x, float e) {
     constexpr float ln2 = 0x1.62e43p-1f, ln2_rest = -0x1.05c61p-29f;  // ln 2 in two parts
-    const float l = __builtin_amdgcn_logf(1.f + __expf(x)), p = l * ln2;
+    const float l = __builtin_amdgcn_logf(e), p = l * ln2;
     const float y = p + fmaf(l, ln2_rest, fmaf(l, ln2, -p));
     return x >= 15.f ? x : x <= -15.f ? 0.f : y;
 }
+
+__device__ __forceinline__ double lane_value64(double x, int lane) {
+    const long long u = __builtin_bit_cast(long long, x);
+    const unsigned lo = __builtin_amdgcn_readlane((int)u, lane), hi = __builtin_amdgcn_readlane((int)(u >> 32), lane);
+    return __builtin_bit_cast(double, (long long)(((unsigned long long)hi << 32) | lo));
+}
+
+// What lanes of a wave hand to each other through LDS: the hardware keeps a wave's LDS accesses in order, this the compiler.
+__device__ __forceinline__ void wave_lds_fence() { asm volatile("" ::: "memory"); }
 
 // f(0), f(1), ... with the argument as a type, until one returns false
 template <class Fn, int... I>
@@ -57,7 +62,7 @@ __device__ __forceinline__ void while_true(Fn &f, std::integer_sequence<int, I..
 // mean, whose terms are large and of one sign.  So what the tile starts with and what its tokens add are kept apart, each
 // sum is formed by itself and joined once, the retentions are a float64 product, and the means' P0 is summed and kept in
 // float64.  With one running fp32 value per column y was 1.25 times as far from float64 as with token by token products,
-// the gates 1.4 to 2 times; so it is 0.65 and 0.4 times, for 0.08 ms of the 1.26 below.
+// the gates 1.4 to 2 times; so it is 0.65 and 0.4 times, for 0.08 ms.
 //
 // Two lane layouts, one a permutation of the other's lanes: the matrix cores' (ml, kg) = (lane % 16, lane / 16) and the
 // quads' (r, cq) = (lane / 4, lane % 4).  Lane (ml, kg) holds row ml of the wave's 16 rows, columns 16 kt + 4 kg + v,
@@ -65,15 +70,19 @@ __device__ __forceinline__ void while_true(Fn &f, std::integer_sequence<int, I..
 // lane (r, cq) holds row r, columns 16 kt + 4 cq + v of F, so that a product with a vector is 16 fused
 // multiply-adds and two DPP adds.  Tokens of a tile go to the matrix cores in the order sigma(4 a + b) = 4 b + a:
 // lane cq then owns the columns t' = 4 j + cq of P, and column group j is finished with token 4 j + 3.
-// The row means are rows 0 (alpha), 1 (eta) and 2 (v) of a third matrix that every wave carries.
+// The row means (alpha, eta, v) and the gates are one more wave's: a token's gates are wanted only at the end of its step, so
+// the wave hands them over with the token's exchange and works a token ahead in the others' shadow.  It keeps the means and
+// the next token's x as four rows of 16 lanes (four multiply-adds and four DPP adds give the means' products and k . x of the
+// next token at once), its own columns' values a lane each, and goes first on the SIMD that it shares.
 //
-// Bound by the issue rate of one wave per SIMD (1050 clocks a token with the exchange, tile starts and ends).  64 chains of
-// 2048 tokens, head size 64, chunks of 64: 1.26 ms, with the two kernels below 1.47 ms; one kernel that formed all products of a token with all six memories in sequence
-// (it serves longer chunks, selfref.hip) takes 2.29 ms.  Chunks of 1, 4, 8, 16 tokens at 64 chains of 512: 6.64, 2.04,
-// 1.27, 0.88 ms there, 3.84, 1.15, 0.70, 0.47 ms here.
+// Bound by the issue rate of one wave per SIMD: 820 clocks a token (120 vector and LDS instructions of the first four waves,
+// the exchange), 4000 for a tile's start and end.  64 chains of 2048 tokens, head size 64, chunks of 64: 0.92 ms, 1.26 with the
+// means in every wave; with the two kernels below 1.14 ms; one kernel that formed all products of a token with all six
+// memories in sequence (it serves longer chunks, selfref.hip) takes 2.29 ms.  Chunks of 1, 4, 8, 16 tokens at 64 chains of
+// 512: 6.64, 2.04, 1.27, 0.88 ms there, 3.84, 1.15, 0.70, 0.47 ms with the means in every wave.
 
 template <int D, bool SG>
-__global__ __launch_bounds__(4 * D) void selfref_chain_kernel(
+__global__ __launch_bounds__(4 * D + 64) void selfref_chain_kernel(
     float *__restrict__ mems, const float *__restrict__ emb, float *__restrict__ k_cache, float *__restrict__ v_cache,
     float *__restrict__ alpha_cache, float *__restrict__ theta_cache, float *__restrict__ amean_cache,
     float *__restrict__ emean_cache, float *__restrict__ frozen, int s, int C, int nc) {
@@ -83,8 +92,11 @@ __global__ __launch_bounds__(4 * D) void selfref_chain_kernel(
     // k - v, exchange only; two as well: a tile of one token has a single barrier, behind which a slow wave still reads its
     // row while a fast one writes the next tile's first
     __shared__ __align__(16) float Ut[2][SG ? kTB * LD : 4];
-    __shared__ __align__(16) float Sx[NW][kTB];
-    __shared__ __align__(16) float mean[3][D];
+    // k_t . x_t' of the tile's later tokens: a wave's own, two of them because the gates' wave reads the first wave's a step later
+    __shared__ __align__(16) float Sx[2][NW][kTB];
+    __shared__ __align__(16) float mean[4][D];         // row means of M_alpha, M_eta, M_v, as the tile starts; a row of zeros
+    __shared__ __align__(16) float mean_c[3][D];       // the same as the chunk starts
+    __shared__ __align__(16) float gate[2][kTB][4];    // a token's 1 - alpha, the retentions of the tile up to it, theta twice
 
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, wr = 16 * wave;
     const int ml = lane & 15, kg = lane >> 4, r = lane >> 2, cq = lane & 3;
@@ -92,41 +104,137 @@ __global__ __launch_bounds__(4 * D) void selfref_chain_kernel(
     const size_t b = blockIdx.x, tok0 = b * (size_t)s;
     float *mb = mems + b * 6 * DD;
 
-    // M_k, M_v and the row means in the matrix cores' layout; row means of M_alpha, M_eta, M_v
-    f32x4 M[3][KT];
+    for (int e = tid; e < 4 * D; e += 4 * D + 64) {
+        const int which = e / D;
+        float a = 0.f;
+        if (which < 3) {
+            const float *src = mb + (which == 0 ? 4 : which == 1 ? 3 : 1) * DD + e % D;
+#pragma unroll 8
+            for (int c = 0; c < D; c++) a += src[c * D];
+        }
+        mean[which][e % D] = a * (1.f / D);
+    }
+    // the rows of a partial tile behind its last token enter the end-of-tile product times zero
+    for (int e = tid; e < kTB * LD; e += 4 * D + 64) Kt[0][e] = Kt[1][e] = 0.f;
+    // first token behind the tile that starts at t
+    auto tile_end = [&](int t) { return min(min(t + kTB, (t / C + 1) * C), s); };
+
+    if (wave == NW) {  // the gates
+        __builtin_amdgcn_s_setprio(3);   // every token waits for them, and another wave issues on the same SIMD
+        // lane (row, col): row of the means, or token t + 1's x as a fourth; columns 4 col .. 4 col + 3 of it, or the tile's token col
+        constexpr int LR = D / 4;   // lanes of a row that hold columns
+        const int row = lane >> 4, col = lane & 15, c4 = 4 * (col & (LR - 1));
+        const bool writer = row < 3 && (D == 64 || col < LR);
+        const float scale = row == 0 ? -1.4426950408889634f : 1.4426950408889634f;   // exp(-x) of alpha's mean, exp(x) of eta's
+        __syncthreads();
+        f32x4 M = *reinterpret_cast<const f32x4 *>(&mean[row][c4]);
+        int chunk_t = 0;
+        for (int tb = 0, te, buf = 0; tb < s; tb = te, buf ^= 1) {
+            te = tile_end(tb);
+            const int nt = te - tb;
+            const float *Kb = Kt[buf], *Ub = Ut[buf];
+            if (writer) *reinterpret_cast<f32x4 *>(&mean[row][c4]) = M;
+            if (tb == chunk_t) {
+                if (writer) *reinterpret_cast<f32x4 *>(&mean_c[row][c4]) = M;
+                chunk_t += C;
+            }
+            wave_lds_fence();
+            // Means times the tile's x in float64: a block of the instruction is the means' four rows by four tokens, its
+            // result row lane / 16, token lane % 16.
+            double P0 = 0.;
+#pragma unroll
+            for (int kt = 0; kt < KT; kt++) {
+                const f32x4 m4 = *reinterpret_cast<const f32x4 *>(&mean[lane & 3][16 * kt + 4 * row]);
+                const f32x4 x4 = *reinterpret_cast<const f32x4 *>(&xt[buf][col * LD + 16 * kt + 4 * row]);
+#pragma unroll
+                for (int v = 0; v < 4; v++) P0 = __builtin_amdgcn_mfma_f64_4x4x4f64((double)m4[v], (double)x4[v], P0, 0, 0, 0);
+            }
+            // Value of column t' = col before token t': retentions times P0, as two floats, plus what the tile's tokens added.
+            float P = 0.f, pw = 0.f, pkeep = 1.f, mine = 0.f;
+            float high = (float)P0, low = (float)(P0 - (double)high), now = high;
+            double kept = 1.;
+            float W[kTB], th[kTB], keep[kTB];
+#pragma unroll
+            for (int t = 0; t < kTB; t++) { W[t] = th[t] = 0.f; keep[t] = 1.f; }
+            const float *other = row == 3 ? &xt[buf][LD + c4] : &mean_c[row][c4];
+            auto step = [&](auto T) __attribute__((always_inline)) -> bool {
+                constexpr int t = decltype(T)::value;
+                // lane (0, t): alpha's mean, lane (1, t): eta's; both gates in every lane
+                const float e = 1.f + __builtin_amdgcn_exp2f(now * scale);
+                const float sig = sigmoid_of(now, e), soft = softplus_of(now, e);
+                const float mean_v = now;
+                mine = col == t ? now : mine;
+                const float keep_l = 1.f - sig;
+                const double kept_l = kept * (1. - (double)sig);
+                if (col == t && row < 2)
+                    *reinterpret_cast<float2 *>(&gate[buf][t][2 * row]) = row == 0 ? make_float2(keep_l, (float)kept_l) : make_float2(soft, soft);
+                const f32x4 m = *reinterpret_cast<const f32x4 *>(other);
+                if (t + 2 < kTB) other += row == 3 ? LD : 0;
+                lds_barrier();
+                // row 3: x of the next token against k, the other rows the means against u
+                const f32x4 u = *reinterpret_cast<const f32x4 *>((SG && row < 3 ? Ub : Kb) + t * LD + c4);
+                float ps = 0.f;
+                if (t > 0 && t + 1 < kTB) ps = Sx[(t - 1) & 1][0][sigma(col)];
+                __builtin_amdgcn_sched_barrier(0);
+                keep[t] = lane_value(keep_l, t);
+                th[t] = SG ? -lane_value(soft, 16 + t) : lane_value(soft, 16 + t);
+                const float vm = SG ? 0.f : lane_value(mean_v, 32 + t);
+                kept = lane_value64(kept_l, t);
+                const double P1 = kept * P0;
+                high = (float)P1;
+                low = (float)(P1 - (double)high);
+                if (t > 0 && t + 1 < kTB) P = fmaf(pw, ps, pkeep * P);
+                const float rest = fmaf(keep[t], P, low);
+                const float dot = group_allreduce<LR>((m[0] * u[0] + m[1] * u[1]) + (m[2] * u[2] + m[3] * u[3]));
+                W[t] = SG ? dot : vm - dot;
+                if constexpr (t + 1 < kTB) {
+                    pw = th[t] * W[t];
+                    pkeep = keep[t];
+                    now = high + fmaf(pw, lane_value(dot, 48), rest);
+                }
+                return t + 1 < nt;
+            };
+            while_true(step, std::make_integer_sequence<int, kTB>{});
+            // as the other memories: the tile's sum by itself, joined once
+            f32x4 add = f32x4{0.f, 0.f, 0.f, 0.f};
+            float behind = 1.f;
+#pragma unroll
+            for (int t = kTB - 1; t >= 0; t--) {
+                const f32x4 k4 = *reinterpret_cast<const f32x4 *>(Kb + t * LD + c4);
+                const float c = W[t] * (th[t] * behind);
+                behind *= keep[t];
+#pragma unroll
+                for (int v = 0; v < 4; v++) add[v] = fmaf(c, k4[v], add[v]);
+            }
+#pragma unroll
+            for (int v = 0; v < 4; v++) M[v] = fmaf((float)kept, M[v], add[v]);
+            if (col < nt) {
+                const size_t o = tok0 + tb + col;
+                const float e = 1.f + __builtin_amdgcn_exp2f(mine * scale);
+                if (row == 0) { alpha_cache[o] = sigmoid_of(mine, e); amean_cache[o] = mine; }
+                if (row == 1) { theta_cache[o] = softplus_of(mine, e); emean_cache[o] = mine; }
+            }
+        }
+        return;
+    }
+    const int stt = tid / V4, sj = (tid % V4) * 4;  // staging slot: token, column
+    auto load_x = [&](int t, int n) -> float4 {
+        return stt < n ? *reinterpret_cast<const float4 *>(emb + (tok0 + t + stt) * D + sj) : make_float4(0, 0, 0, 0);
+    };
+    int te = tile_end(0);
+    *reinterpret_cast<float4 *>(&xt[0][stt * LD + sj]) = load_x(0, te);
+    float4 xnext = te < s ? load_x(te, tile_end(te) - te) : make_float4(0, 0, 0, 0);
+    // M_k, M_v in the matrix cores' layout
+    f32x4 M[2][KT];
 #pragma unroll
     for (int c = 0; c < 2; c++) {
 #pragma unroll
         for (int kt = 0; kt < KT; kt++)
             M[c][kt] = *reinterpret_cast<const f32x4 *>(mb + c * DD + (wr + ml) * D + 16 * kt + 4 * kg);
     }
-    for (int e = tid; e < 3 * D; e += 4 * D) {
-        const int which = e / D;
-        const float *src = mb + (which == 0 ? 4 : which == 1 ? 3 : 1) * DD + e % D;
-        float a = 0.f;
-#pragma unroll 8
-        for (int c = 0; c < D; c++) a += src[c * D];
-        mean[which][e % D] = a * (1.f / D);
-    }
-    // the rows of a partial tile behind its last token enter the end-of-tile product times zero
-    for (int e = tid; e < kTB * LD; e += 4 * D) Kt[0][e] = Kt[1][e] = 0.f;
-
-    const int stt = tid / V4, sj = (tid % V4) * 4;  // staging slot: token, column
-    auto load_x = [&](int t, int n) -> float4 {
-        return stt < n ? *reinterpret_cast<const float4 *>(emb + (tok0 + t + stt) * D + sj) : make_float4(0, 0, 0, 0);
-    };
-    // first token behind the tile that starts at t
-    auto tile_end = [&](int t) { return min(min(t + kTB, (t / C + 1) * C), s); };
-    int te = tile_end(0);
-    *reinterpret_cast<float4 *>(&xt[0][stt * LD + sj]) = load_x(0, te);
-    float4 xnext = te < s ? load_x(te, tile_end(te) - te) : make_float4(0, 0, 0, 0);
     __syncthreads();
-#pragma unroll
-    for (int kt = 0; kt < KT; kt++)
-        M[2][kt] = ml < 3 ? *reinterpret_cast<const f32x4 *>(&mean[ml < 3 ? ml : 0][16 * kt + 4 * kg])
-                          : f32x4{0.f, 0.f, 0.f, 0.f};
 
-    float F[3][4 * KT];
+    float F[2][4 * KT];
     int chunk_t = 0, ci = 0;
     for (int tb = 0, buf = 0; tb < s; tb = te, buf ^= 1) {
         te = tile_end(tb);
@@ -135,10 +243,10 @@ __global__ __launch_bounds__(4 * D) void selfref_chain_kernel(
         if (tb == chunk_t) {  // snapshot
             float *fb = frozen + (b * nc + ci) * (size_t)6 * DD;
 #pragma unroll
-            for (int c = 0; c < 3; c++) {
+            for (int c = 0; c < 2; c++) {
 #pragma unroll
                 for (int kt = 0; kt < KT; kt++) {
-                    if (c < 2) *reinterpret_cast<f32x4 *>(fb + c * DD + (wr + ml) * D + 16 * kt + 4 * kg) = M[c][kt];
+                    *reinterpret_cast<f32x4 *>(fb + c * DD + (wr + ml) * D + 16 * kt + 4 * kg) = M[c][kt];
 #pragma unroll
                     for (int v = 0; v < 4; v++) F[c][4 * kt + v] = lane_from(to_quad, M[c][kt][v]);
                 }
@@ -152,15 +260,12 @@ __global__ __launch_bounds__(4 * D) void selfref_chain_kernel(
             const int t2 = tile_end(te);
             if (t2 < s) xnext = load_x(t2, tile_end(t2) - t2);
         }
-        float P0[2][4], P[3][4], X[4 * KT];   // M_c X^T as the tile starts, and what its tokens add
-        double P2[4];
+        float P0[2][4], P[2][4], X[4 * KT];   // M_c X^T as the tile starts, and what its tokens add
         {
             f32x4 acc[2][KT];   // a sum per 16 columns, added up in a tree
-            f64x4 mean_acc = {0., 0., 0., 0.};
 #pragma unroll
             for (int kt = 0; kt < KT; kt++) {
                 const f32x4 xa = *reinterpret_cast<const f32x4 *>(&xt[buf][sigma(ml) * LD + 16 * kt + 4 * kg]);
-                const f32x4 xm = *reinterpret_cast<const f32x4 *>(&xt[buf][ml * LD + 16 * kt + 4 * kg]);
                 const f32x4 xq = *reinterpret_cast<const f32x4 *>(&xt[buf][sigma(r) * LD + 16 * kt + 4 * cq]);
 #pragma unroll
                 for (int c = 0; c < 2; c++) acc[c][kt] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -169,8 +274,6 @@ __global__ __launch_bounds__(4 * D) void selfref_chain_kernel(
                     X[4 * kt + v] = xq[v];
 #pragma unroll
                     for (int c = 0; c < 2; c++) acc[c][kt] = mfma4(xa[v], M[c][kt][v], acc[c][kt]);
-                    // result rows 4 v + kg: the first operand's rows are the tokens as they stand
-                    mean_acc = __builtin_amdgcn_mfma_f64_16x16x4f64((double)xm[v], (double)M[2][kt][v], mean_acc, 0, 0, 0);
                 }
             }
 #pragma unroll
@@ -183,20 +286,15 @@ __global__ __launch_bounds__(4 * D) void selfref_chain_kernel(
             }
 #pragma unroll
             for (int v = 0; v < 4; v++) {
-                P2[v] = lane_from64(to_quad, mean_acc[v]);
-                P[0][v] = P[1][v] = P[2][v] = 0.f;
+                P[0][v] = P[1][v] = 0.f;
             }
         }
-        float W[3][4], cs[4];
-        double kept = 1.;  // w_c of token 4 j + cq, th times the retention since, of the whole tile
+        float W[2][4], cs[4], kept = 1.f;  // w_c of token 4 j + cq, th times the retention since, of the whole tile
 #pragma unroll
-        for (int j = 0; j < 4; j++) W[0][j] = W[1][j] = W[2][j] = cs[j] = 0.f;
+        for (int j = 0; j < 4; j++) W[0][j] = W[1][j] = cs[j] = 0.f;
         float k = quad_lane<0>(P0[0][0]), v = quad_lane<0>(P0[1][0]);
-        float am = lane_value((float)P2[0], 0), em = lane_value((float)P2[0], 4), vm = lane_value((float)P2[0], 8);
-        // lane t keeps token t's gate means for the caches; what token t - 1 adds to the columns behind t is added while
-        // token t's exchange is under way
-        float s_am = 0.f, s_em = 0.f;
-        float pw[3] = {0.f, 0.f, 0.f}, pkeep = 1.f;
+        // what token t - 1 adds to the columns behind t is added while token t's exchange is under way
+        float pw[2] = {0.f, 0.f}, pkeep = 1.f;
         float *const out = (SG ? (cq == 0 ? Kb : cq == 1 ? Vb : Ub) : (cq & 1) ? Vb : Kb) + wr + r;
 
         auto step = [&](auto T) __attribute__((always_inline)) -> bool {
@@ -214,7 +312,8 @@ __global__ __launch_bounds__(4 * D) void selfref_chain_kernel(
             lds_barrier();
             float kc[4 * KT], uc[4 * KT];
             f32x4 ps = f32x4{0.f, 0.f, 0.f, 0.f};
-            if (t > 0 && t + 1 < kTB) ps = *reinterpret_cast<const f32x4 *>(&Sx[wave][4 * cq]);
+            if (t > 0 && t + 1 < kTB) ps = *reinterpret_cast<const f32x4 *>(&Sx[(t - 1) & 1][wave][4 * cq]);
+            const f32x4 g = *reinterpret_cast<const f32x4 *>(gate[buf][t]);
 #pragma unroll
             for (int kt = 0; kt < KT; kt++) {
                 const f32x4 k4 = *reinterpret_cast<const f32x4 *>(Kb + t * LD + 16 * kt + 4 * cq);
@@ -228,43 +327,35 @@ __global__ __launch_bounds__(4 * D) void selfref_chain_kernel(
 #pragma unroll
                 for (int j = (t + 1) / 4; j < 4; j++) {
 #pragma unroll
-                    for (int c = 0; c < 3; c++) {
+                    for (int c = 0; c < 2; c++) {
                         P[c][j] = fmaf(pw[c], ps[j], pkeep * P[c][j]);
                         asm volatile("" : "+v"(P[c][j]));  // here, not when the column is needed
                     }
                 }
             }
-            set_lane<t>(s_am, am);
-            set_lane<t>(s_em, em);
-            const float alpha = sr_sigmoid_select(am), theta = sr_softplus_select(em), keep = 1.f - alpha;
             const float S = quad_allreduce(dotn<4 * KT>(X, kc));  // row r: k_t . x of token sigma(r)
-            float w[3];  // w_c,t (self-generated values: its negative)
+            float w[2];  // w_c,t (self-generated values: its negative)
 #pragma unroll
-            for (int c = 0; c < 3; c++) {
+            for (int c = 0; c < 2; c++) {
                 w[c] = quad_allreduce(dotn<4 * KT>(F[c], uc));
-                if (!SG) w[c] = (c == 2 ? vm : v) - w[c];
+                if (!SG) w[c] = v - w[c];
             }
-            const float th = SG ? -theta : theta;
+            const float th = SG ? -g[2] : g[2], keep = g[0];
 #pragma unroll
             for (int j = 0; j <= J; j++) cs[j] *= keep;
-            kept *= 1. - (double)alpha;
+            kept = g[1];
             cs[J] = cq == Q ? th : cs[J];
 #pragma unroll
-            for (int c = 0; c < 3; c++) W[c][J] = cq == Q ? w[c] : W[c][J];
+            for (int c = 0; c < 2; c++) W[c][J] = cq == Q ? w[c] : W[c][J];
             if constexpr (t + 1 < kTB) {
                 constexpr int J1 = (t + 1) / 4, Q1 = (t + 1) % 4;
                 const float s1 = lane_value(S, 4 * sigma(t + 1));
 #pragma unroll
-                for (int c = 0; c < 3; c++) pw[c] = th * w[c];
+                for (int c = 0; c < 2; c++) pw[c] = th * w[c];
                 pkeep = keep;
-                const float kept1 = (float)kept;
-                k = fmaf(kept1, quad_lane<Q1>(P0[0][J1]), fmaf(pw[0], s1, keep * quad_lane<Q1>(P[0][J1])));
-                v = fmaf(kept1, quad_lane<Q1>(P0[1][J1]), fmaf(pw[1], s1, keep * quad_lane<Q1>(P[1][J1])));
-                const float m = (float)fma(kept, P2[J1], (double)fmaf(pw[2], s1, keep * P[2][J1]));
-                am = lane_value(m, Q1);
-                em = lane_value(m, 4 + Q1);
-                vm = lane_value(m, 8 + Q1);
-                if (t + 2 < kTB) Sx[wave][r] = S;  // the wave's own; read back behind the next exchange
+                k = fmaf(kept, quad_lane<Q1>(P0[0][J1]), fmaf(pw[0], s1, keep * quad_lane<Q1>(P[0][J1])));
+                v = fmaf(kept, quad_lane<Q1>(P0[1][J1]), fmaf(pw[1], s1, keep * quad_lane<Q1>(P[1][J1])));
+                if (t + 2 < kTB) Sx[t & 1][wave][r] = S;  // read behind the next exchange
             }
             return t + 1 < nt;
         };
@@ -272,10 +363,9 @@ __global__ __launch_bounds__(4 * D) void selfref_chain_kernel(
 
         // M_c <- keep M_c + sum_t cs_t w_c,t k_t^T; every wave has written its part of Kb, Vb.  The tile's sum is formed by
         // itself, so that M_c rounds once a tile and not once a token
-        const float keep_tile = (float)kept;
-        f32x4 add[3][KT];
+        f32x4 add[2][KT];
 #pragma unroll
-        for (int c = 0; c < 3; c++) {
+        for (int c = 0; c < 2; c++) {
 #pragma unroll
             for (int kt = 0; kt < KT; kt++) add[c][kt] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -288,27 +378,22 @@ __global__ __launch_bounds__(4 * D) void selfref_chain_kernel(
                 for (int kt = 0; kt < KT; kt++) {
                     const float a = Kb[(4 * j + kg) * LD + 16 * kt + ml];
 #pragma unroll
-                    for (int c = 0; c < 3; c++) add[c][kt] = mfma4(a, W[c][j], add[c][kt]);
+                    for (int c = 0; c < 2; c++) add[c][kt] = mfma4(a, W[c][j], add[c][kt]);
                 }
             }
         }
 #pragma unroll
-        for (int c = 0; c < 3; c++) {
+        for (int c = 0; c < 2; c++) {
 #pragma unroll
             for (int kt = 0; kt < KT; kt++) {
 #pragma unroll
-                for (int v = 0; v < 4; v++) M[c][kt][v] = fmaf(keep_tile, M[c][kt][v], add[c][kt][v]);
+                for (int v = 0; v < 4; v++) M[c][kt][v] = fmaf(kept, M[c][kt][v], add[c][kt][v]);
             }
         }
         if (stt < nt) {
             const size_t o = (tok0 + tb + stt) * D + sj;
             *reinterpret_cast<float4 *>(k_cache + o) = *reinterpret_cast<const float4 *>(Kb + stt * LD + sj);
             *reinterpret_cast<float4 *>(v_cache + o) = *reinterpret_cast<const float4 *>(Vb + stt * LD + sj);
-        }
-        if (tid < nt) {
-            const size_t o = tok0 + tb + tid;
-            alpha_cache[o] = sr_sigmoid_select(s_am); theta_cache[o] = sr_softplus_select(s_em);
-            amean_cache[o] = s_am; emean_cache[o] = s_em;
         }
     }
 #pragma unroll
@@ -572,7 +657,7 @@ __global__ __launch_bounds__(4 * D) void selfref_read_kernel(
 template <int D, bool SG>
 void launch(const SelfrefForward &a) {
     const dim3 block(4 * D);
-    hipLaunchKernelGGL((selfref_chain_kernel<D, SG>), dim3(a.batch), block, 0, stream(), a.mems, a.emb, a.k, a.v, a.alpha,
+    hipLaunchKernelGGL((selfref_chain_kernel<D, SG>), dim3(a.batch), dim3(4 * D + 64), 0, stream(), a.mems, a.emb, a.k, a.v, a.alpha,
                        a.theta, a.amean, a.emean, a.frozen, a.s, a.C, a.nc);
     check_launch("selfref_chain_kernel");
     hipLaunchKernelGGL((selfref_scan_kernel<D, SG>), dim3(4 * a.batch), block, 0, stream(), a.mems, a.k, a.v, a.alpha,
