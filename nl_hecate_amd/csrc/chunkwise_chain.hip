@@ -48,7 +48,6 @@ constexpr int kChainThr = 512;     // 8 waves
 constexpr int kTableFloats = CW * CW;
 constexpr int kVecFloats = 4 * CW + 16;
 constexpr int kStageLd = CW + 4;   // row stride (floats) of the table while it is assembled in LDS
-constexpr int kCoefChunksPerWave = 4;
 __device__ __forceinline__ bool tile_live(int bi, int rt, int ct) { return 2 * (bi & 1) + ct >= 2 * (bi >> 1) + rt; }
 
 // Coefficients of one chunk from its gates: one wave per chunk, lane = token.  The vectors come from two scans
@@ -58,10 +57,10 @@ template <bool HAS_S>
 __global__ __launch_bounds__(64) void cw_coef_kernel(const float *__restrict__ alpha,
                                                      const float *__restrict__ theta,
                                                      const float *__restrict__ eta, float *__restrict__ table,
-                                                     float *__restrict__ vecs, int s, int C, int nc, int nchunks) {
+                                                     float *__restrict__ vecs, int s, int C, int nc, int nchunks, int per_wave) {
     __shared__ __align__(16) float stage[(CW + 1) * kStageLd];
     __shared__ float gk[2 * CW], ge[2 * CW];
-    const int j = threadIdx.x, first = blockIdx.x * kCoefChunksPerWave, last = min(nchunks, first + kCoefChunksPerWave);
+    const int j = threadIdx.x, first = blockIdx.x * per_wave, last = min(nchunks, first + per_wave);
     auto gates_of = [&](int chunk) {
         const int chain = chunk / nc, t0 = (chunk % nc) * C;
         return fetch_gates<HAS_S>(alpha, theta, eta, (size_t)chain * s + t0, min(C, s - t0));
@@ -417,8 +416,9 @@ void launch_forward(const char *fn, const u16 *k, const u16 *v, const u16 *q, co
     if (es.failed()) return;
     {
         KernelTimer kt("cw_coef_kernel");
-        hipLaunchKernelGGL(cw_coef_kernel<HAS_S>, dim3(ceil_div(nchunks, kCoefChunksPerWave)), dim3(64), 0, stream(), alpha, theta, eta,
-                           table, vecs, seq_len, chunk_size, nc, nchunks);
+        hipLaunchKernelGGL(cw_coef_kernel<HAS_S>, dim3(ceil_div(nchunks, coef_chunks_per_wave(nchunks))), dim3(64), 0, stream(), alpha, theta, eta,
+                           table, vecs, seq_len, chunk_size, nc, nchunks,
+                           coef_chunks_per_wave(nchunks));
     }
     check_launch("cw_coef_kernel");
     {

@@ -47,7 +47,6 @@ namespace {
 constexpr int kTab = CW * CW;
 constexpr int kVecB = 5 * CW + 16;
 constexpr int kCtLd = CW + 4;   // row stride (floats) of the coefficient copy in LDS
-constexpr int kCoefChunksPerWave = 4;
 __device__ __forceinline__ bool live_b(int bi, int rt, int ct) { return 2 * (bi >> 1) + rt >= 2 * (bi & 1) + ct; }
 
 // One wave per chunk, lane = token: the vectors from two scans of composed maps, the table from
@@ -58,10 +57,10 @@ __global__ __launch_bounds__(64) void cw_coef_bwd_kernel(const float *__restrict
                                                          const float *__restrict__ theta,
                                                          const float *__restrict__ eta,
                                                          float *__restrict__ tab_b, float *__restrict__ vecs,
-                                                         int s, int C, int nc, int nchunks) {
+                                                         int s, int C, int nc, int nchunks, int per_wave) {
     __shared__ __align__(16) float stage[(CW + 1) * kCtLd];
     __shared__ float gk[2 * CW], ge[2 * CW];
-    const int j = threadIdx.x, first = blockIdx.x * kCoefChunksPerWave, last = min(nchunks, first + kCoefChunksPerWave);
+    const int j = threadIdx.x, first = blockIdx.x * per_wave, last = min(nchunks, first + per_wave);
     auto gates_of = [&](int chunk) {
         const int chain = chunk / nc, t0 = (chunk % nc) * C;
         return fetch_gates<HAS_S>(alpha, theta, eta, (size_t)chain * s + t0, min(C, s - t0));
@@ -592,11 +591,13 @@ void chunkwise_backward_coefficients(const float *alpha, const float *theta, con
     const int nc = ceil_div(seq_len, chunk_size), ntask = batch * nc;
     KernelTimer kt("cw_coef_bwd_kernel");
     if (has_s)
-        hipLaunchKernelGGL(cw_coef_bwd_kernel<true>, dim3(ceil_div(ntask, kCoefChunksPerWave)), dim3(64), 0, stream(), alpha, theta,
-                           eta, tab_b, vecs, seq_len, chunk_size, nc, ntask);
+        hipLaunchKernelGGL(cw_coef_bwd_kernel<true>, dim3(ceil_div(ntask, coef_chunks_per_wave(ntask))), dim3(64), 0, stream(), alpha, theta,
+                           eta, tab_b, vecs, seq_len, chunk_size, nc, ntask,
+                           coef_chunks_per_wave(ntask));
     else
-        hipLaunchKernelGGL(cw_coef_bwd_kernel<false>, dim3(ceil_div(ntask, kCoefChunksPerWave)), dim3(64), 0, stream(), alpha, theta,
-                           nullptr, tab_b, vecs, seq_len, chunk_size, nc, ntask);
+        hipLaunchKernelGGL(cw_coef_bwd_kernel<false>, dim3(ceil_div(ntask, coef_chunks_per_wave(ntask))), dim3(64), 0, stream(), alpha, theta,
+                           nullptr, tab_b, vecs, seq_len, chunk_size, nc, ntask,
+                           coef_chunks_per_wave(ntask));
     check_launch("cw_coef_bwd_kernel");
 }
 

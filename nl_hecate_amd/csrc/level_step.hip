@@ -23,6 +23,7 @@
 #include "../../include/nl_hecate_ffi.h"
 #include "bf16_tiles.h"
 #include "chunkwise_grads.h"
+#include "gemm_bf16.h"
 #include "lane_ops.h"
 #include "runtime.h"
 
@@ -122,21 +123,21 @@ __global__ __launch_bounds__(64) void gate_fold_partial_kernel(const float *__re
 #pragma unroll
     for (int q = 0; q < 6; q++) part[(((size_t)lvl * kFoldSlices + sl) * 6 + q) * D + j] = u[q];
 }
-__global__ __launch_bounds__(64) void gate_fold_finish_kernel(const float *__restrict__ part, u16 *__restrict__ ufrag, int D) {
-    const int lvl = blockIdx.y, j = blockIdx.x * 64 + threadIdx.x;
+// a wave per quantity: its sixteen slices are loads without a chain between them (one wave for all six took 10 us)
+__global__ __launch_bounds__(6 * 64) void gate_fold_finish_kernel(const float *__restrict__ part, u16 *__restrict__ ufrag, int D) {
+    const int lvl = blockIdx.y, j = blockIdx.x * 64 + (threadIdx.x & 63), q = threadIdx.x >> 6;
     if (j >= D) return;
     u16 *base = ufrag + ((size_t)lvl * (D / 32) + j / 32) * 512 + (size_t)16 * ((j % 32) / 8) * 8 + j % 8;
     __bf16 *out = reinterpret_cast<__bf16 *>(base);
+    float x[kFoldSlices], u = 0.f;
 #pragma unroll
-    for (int q = 0; q < 6; q++) {
-        float u = 0.f;
-        for (int sl = 0; sl < kFoldSlices; sl++) u += part[(((size_t)lvl * kFoldSlices + sl) * 6 + q) * D + j];
-        const __bf16 hi = (__bf16)u;
-        out[(2 * q) * 8] = hi;
-        out[(2 * q + 1) * 8] = (__bf16)(u - (float)hi);
-    }
+    for (int sl = 0; sl < kFoldSlices; sl++) x[sl] = part[(((size_t)lvl * kFoldSlices + sl) * 6 + q) * D + j];
 #pragma unroll
-    for (int r = 12; r < 16; r++) out[r * 8] = (__bf16)0.f;
+    for (int sl = 0; sl < kFoldSlices; sl++) u += x[sl];
+    const __bf16 hi = (__bf16)u;
+    out[(2 * q) * 8] = hi;
+    out[(2 * q + 1) * 8] = (__bf16)(u - (float)hi);
+    if (q < 4) out[(12 + q) * 8] = (__bf16)0.f;
 }
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
@@ -235,8 +236,7 @@ __global__ __launch_bounds__(kPThr) void level_project_kernel(ProjArgs a) {
     u16 *Xs = reinterpret_cast<u16 *>(smem);                                   // [PT][XS]
     float *red = reinterpret_cast<float *>(smem + (size_t)PT * XS * 2);         // [2][8][PT]: per-wave sums of squares
     float *gdot = red + 2 * 8 * PT;                                             // [2][PT][8]: x . u_q (6 used)
-    float *tot = gdot + 2 * PT * 8;                                             // [PT]: 1 / max(|k|, eps)
-    int *rowoff = reinterpret_cast<int *>(tot + PT);                            // [PT]: b * nh * s + t of the token
+    int *rowoff = reinterpret_cast<int *>(gdot + 2 * PT * 8);                            // [PT]: b * nh * s + t of the token
     u16 *tb = reinterpret_cast<u16 *>(rowoff + PT) + (threadIdx.x >> 6) * 8 * 72;  // per wave: [8][72], see store_tile_rows
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, g = lane >> 4;
     const long long tok0 = (long long)blockIdx.x * PT, n = a.n;
@@ -257,7 +257,7 @@ __global__ __launch_bounds__(kPThr) void level_project_kernel(ProjArgs a) {
             if (e >= PT * D4) continue;
             const bf16x4 h = f4_to_bf4(v[j]);
             *reinterpret_cast<bf16x4 *>(Xs + row * XS + 4 * c4) = h;
-            if (a.x_bf16 && tok0 + row < n) *reinterpret_cast<bf16x4 *>(a.x_bf16 + (tok0 + row) * D + 4 * c4) = h;
+            if (a.x_bf16 && blockIdx.y == 0 && tok0 + row < n) *reinterpret_cast<bf16x4 *>(a.x_bf16 + (tok0 + row) * D + 4 * c4) = h;
         }
     }
     if (tid < PT) {
@@ -270,9 +270,10 @@ __global__ __launch_bounds__(kPThr) void level_project_kernel(ProjArgs a) {
     const size_t wave_frag = (size_t)wave * 64 * D;
     const int l32 = lane & 31, hf = lane >> 5;
 
+    const int jobs = a.n_extra + 3 * a.levels, j0 = jobs * blockIdx.y / gridDim.y, j1 = jobs * (blockIdx.y + 1) / gridDim.y;
     // plain projections: rounded once, token-major
     if (wave_on)
-        for (int e = 0; e < a.n_extra; e++) {
+        for (int e = j0; e < min(j1, a.n_extra); e++) {
             project_block<D>(Xs, a.wfrag + (size_t)e * D * D + wave_frag, acc);
             u16 *out = a.extra_out[e];
 #pragma unroll
@@ -283,11 +284,12 @@ __global__ __launch_bounds__(kPThr) void level_project_kernel(ProjArgs a) {
                 });
         }
 
-    for (int lvl = 0; lvl < a.levels; lvl++) {
-        const size_t pbase = (size_t)(a.n_extra + 3 * lvl) * D * D;
+#pragma unroll 1
+    for (int job = max(j0, a.n_extra); job < j1; job++) {   // k, v, q of the levels
+        const int lvl = (job - a.n_extra) / 3, p = (job - a.n_extra) % 3;
         const size_t chain0 = (size_t)lvl * a.bs * a.nh;
         float *gd = gdot + (lvl & 1) * PT * 8;
-        {   // the six gate dot products of the wave's 16 tokens (token tile `wave`): one tile of 16 columns
+        if (p == 0) {   // the six gate dot products of the wave's 16 tokens (token tile `wave`): one tile of 16 columns
             const bf16x8 *up = reinterpret_cast<const bf16x8 *>(a.ufrag) + (size_t)lvl * KS * 64 + lane;
             const u16 *xb = Xs + (16 * wave + l16) * XS + 8 * g;
             f32x4 ga = zero4();
@@ -297,19 +299,16 @@ __global__ __launch_bounds__(kPThr) void level_project_kernel(ProjArgs a) {
             // lane group g holds rows 4g .. 4g + 3 = (hi, lo) of quantities 2g and 2g + 1
             if (g < 3) *reinterpret_cast<float2 *>(gd + (16 * wave + l16) * 8 + 2 * g) = make_float2(ga[0] + ga[1], ga[2] + ga[3]);
         }
-#pragma unroll 1
-        for (int p = 0; p < 3; p++) {   // k, v, q
-            if (wave_on) project_block<D>(Xs, a.wfrag + pbase + (size_t)p * D * D + wave_frag, acc);
-            if (p == 1) {   // v leaves as it is
-                if (wave_on) {
+        if (wave_on) project_block<D>(Xs, a.wfrag + (size_t)job * D * D + wave_frag, acc);
+        if (p == 1) {   // v leaves as it is
+            if (wave_on) {
 #pragma unroll
-                    for (int tt = 0; tt < T32; tt++)
-                        store_tile_rows(acc[tt], 1.0f, tb, [&](int r) -> u16 * {
-                            return tok0 + 32 * tt + r < n ? a.vh + (chain0 * a.s + rowoff[32 * tt + r] + (size_t)wave * a.s) * 64 : nullptr;
-                        });
-                }
-                continue;
+                for (int tt = 0; tt < T32; tt++)
+                    store_tile_rows(acc[tt], 1.0f, tb, [&](int r) -> u16 * {
+                        return tok0 + 32 * tt + r < n ? a.vh + (chain0 * a.s + rowoff[32 * tt + r] + (size_t)wave * a.s) * 64 : nullptr;
+                    });
             }
+        } else {
             // k, q: the row norm over all D columns = over the eight waves.  The two half-waves hold different columns
             // of the same 32 tokens: one exchange per pair of token tiles leaves tile t32's totals in half t32 % 2, which
             // parks them as red[token][wave]; behind the barrier every lane reads the eight waves' sums of its own four
@@ -351,7 +350,6 @@ __global__ __launch_bounds__(kPThr) void level_project_kernel(ProjArgs a) {
                     inv[tt] = 1.0f / fmaxf(nrm, a.eps);
                     if (wave == 0 && hf == 0) {
                         const long long tok = tok0 + 32 * tt + l32;
-                        if (p == 0) tot[32 * tt + l32] = inv[tt];
                         if (tok < n) (p == 0 ? a.k_norms : a.q_norms)[lvl * n + tok] = nrm;
                     }
                 }
@@ -364,12 +362,14 @@ __global__ __launch_bounds__(kPThr) void level_project_kernel(ProjArgs a) {
                         return tok0 + 32 * tt + r < n ? dst + (chain0 * a.s + rowoff[32 * tt + r] + (size_t)wave * a.s) * 64 : nullptr;
                     });
             }
-            if (p == 2 && tid < 3 * PT) {
-                // the gates: one (token, gate) per thread; the q phase's barrier lies between wave 0's write of the
-                // k norms' inverses, every wave's write of the gate dot products, and this read
+            if (p == 0 && tid < 3 * PT) {
+                // the gates: one (token, gate) per thread; the barrier above lies behind every wave's sums and dot products
                 const int token = tid & (PT - 1), q = tid >> 7;   // PT = 128
                 const long long tok = tok0 + token;
-                const float pre = gd[token * 8 + q] * tot[token] + gd[token * 8 + 3 + q] + a.bias[lvl][q][0];
+                float ssum = rd[token * 8];
+#pragma unroll
+                for (int c = 1; c < CB; c++) ssum += rd[token * 8 + c];
+                const float pre = gd[token * 8 + q] * (1.0f / fmaxf(sqrtf(ssum), a.eps)) + gd[token * 8 + 3 + q] + a.bias[lvl][q][0];
                 const float val = gate_act(q, pre);
                 if (tok < n) {
                     float *tm = q == 0 ? a.alpha : (q == 1 ? a.theta : a.eta), *hm = q == 0 ? a.ah : (q == 1 ? a.th : a.eh);
@@ -642,6 +642,13 @@ __global__ void sum_parts_kernel(const float *__restrict__ part, float *__restri
 // run as one batched GEMM into partial outputs, added in a fixed order.
 bool gemm_weight_grad(const char *what, long long m, long long rows, long long tokens, const u16 *a, long long lda, const u16 *G,
                       long long ldb, float *C) {
+    const ProductBf16 p{G, a, nullptr, C, ldb, lda, (int)rows, (int)m, (int)tokens, 0, true, true};
+    if (product_bf16_serves(p, 2)) {
+        const ErrorScope es;
+        KernelTimer kt(what);
+        product_bf16(p, 2);
+        return !es.failed();
+    }
     const long long tiles = ((m + 127) / 128) * ((rows + 127) / 128);
     int parts = 1;
     while (parts < 16 && tiles * parts < 384 && tokens % (2 * parts) == 0 && tokens / (2 * parts) >= 1024) parts *= 2;
@@ -749,10 +756,10 @@ void level_project_forward_bf16_rocm(const float *x, const float *w_extra, int n
         KernelTimer kt("gate_fold_kernel");
         hipLaunchKernelGGL(gate_fold_partial_kernel, dim3(ceil_div(d, 64), levels, kFoldSlices), dim3(64), 0, stream(), w_levels,
                            fa, fold_part, d);
-        hipLaunchKernelGGL(gate_fold_finish_kernel, dim3(ceil_div(d, 64), levels), dim3(64), 0, stream(), fold_part, ufrag, d);
+        hipLaunchKernelGGL(gate_fold_finish_kernel, dim3(ceil_div(d, 64), levels), dim3(6 * 64), 0, stream(), fold_part, ufrag, d);
         check_launch("gate_fold_kernel");
     }
-    const size_t lds = (size_t)PT * (d + 8) * 2 + (2 * 8 * PT + 2 * PT * 8 + PT + PT) * sizeof(float) + 8 * 8 * 72 * 2;
+    const size_t lds = (size_t)PT * (d + 8) * 2 + (2 * 8 * PT + 2 * PT * 8 + PT) * sizeof(float) + 8 * 8 * 72 * 2;
     static bool attr_set = false;
     if (!attr_set) {
         check_hip(hipFuncSetAttribute(reinterpret_cast<const void *>(level_project_kernel<512>),
@@ -763,7 +770,17 @@ void level_project_forward_bf16_rocm(const float *x, const float *w_extra, int n
     }
     if (es.failed()) return;
     KernelTimer kt("level_project_kernel");
-    const dim3 grid(ceil_div(n, PT));
+    // One workgroup per 128 tokens takes all projections, which reads x once; where that leaves compute units idle or the
+    // last round nearly empty the projections are shared out, at about half a projection's time for another staging of x
+    // (500 tokens, nine projections of 256: 62 us on four workgroups, 18 on 36).
+    const int tiles = ceil_div(n, PT), cus = compute_units();
+    int parts = 1;
+    double best = 0;
+    for (int p = 1; p <= P; p++) {
+        const double time = ceil_div((long long)tiles * p, cus) * (ceil_div(P, p) + 0.5);
+        if (p == 1 || time < 0.95 * best) { best = time; parts = p; }
+    }
+    const dim3 grid((unsigned)tiles, (unsigned)parts);
     if (d == 512) hipLaunchKernelGGL(level_project_kernel<512>, grid, dim3(kPThr), lds, stream(), a);
     else hipLaunchKernelGGL(level_project_kernel<256>, grid, dim3(kPThr), lds, stream(), a);
     check_launch("level_project_kernel");
@@ -878,12 +895,20 @@ void titans_levels_backward_bf16_rocm(const uint16_t *x_bf16, const float *w_ext
                                n_extra, n, d, G, R);
             check_launch("cols_to_bf16_kernel");
         }
-        to_bf16(w_extra, wb, (long long)n_extra * d * d);
     }
-    if (levels) to_bf16(w_levels, wb + (size_t)n_extra * d * d, 3LL * levels * d * d);
     if (es.failed()) return;
     // d_x [n, d] = G [n, R] Wb [R, d];  d_W [R, d] = G^T x  (row-major buffers as column-major operands)
-    if (!gemm_bf16("gemm d_x", rocblas_operation_none, rocblas_operation_none, d, n, R, wb, d, G, R, 0.f, d_x, d)) return;
+    const ProductBf16 px{G, n_extra ? w_extra : w_levels, n_extra && levels ? w_levels : nullptr, d_x, R, d, (int)n, d, (int)R,
+                         n_extra * d, true, false};
+    if (product_bf16_serves(px, 1)) {
+        KernelTimer kt("gemm d_x");
+        product_bf16(px, 1);
+        if (es.failed()) return;
+    } else {
+        if (n_extra) to_bf16(w_extra, wb, (long long)n_extra * d * d);
+        if (levels) to_bf16(w_levels, wb + (size_t)n_extra * d * d, 3LL * levels * d * d);
+        if (es.failed() || !gemm_bf16("gemm d_x", rocblas_operation_none, rocblas_operation_none, d, n, R, wb, d, G, R, 0.f, d_x, d)) return;
+    }
     // the weight gradients: one product when the two outputs are one buffer (a layer's packed gradients)
     if (n_extra && levels && d_w_levels == d_w_extra + (size_t)n_extra * d * d) {
         gemm_weight_grad("gemm d_w", d, R, n, x_bf16, d, G, R, d_w_extra);
@@ -919,6 +944,12 @@ void linear_forward_bf16_rocm(const uint16_t *a_bf16, const float *w, float *out
         fail("linear_forward_bf16_rocm: invalid dims n=%d d_in=%d d_out=%d (d_in * d_out must be a multiple of 4).", n, d_in, d_out);
         return;
     }
+    const ProductBf16 p{a_bf16, w, nullptr, out, d_in, d_in, n, d_out, d_in, 0, true, false};
+    if (product_bf16_serves(p, 0)) {
+        KernelTimer kt("gemm linear");
+        product_bf16(p, 0);
+        return;
+    }
     u16 *wb = reinterpret_cast<u16 *>(scratch(27, (size_t)d_in * d_out * sizeof(u16)));
     if (es.failed()) return;
     to_bf16(w, wb, (long long)d_in * d_out);
@@ -932,6 +963,14 @@ void linear_backward_bf16_rocm(const float *d_out_f32, const uint16_t *a_bf16, c
     const ErrorScope es;
     if (n <= 0 || d_in <= 0 || d_out <= 0 || (d_in * (long long)d_out) % 4 || ((long long)n * d_out) % 4) {
         fail("linear_backward_bf16_rocm: invalid dims n=%d d_in=%d d_out=%d (products must be multiples of 4).", n, d_in, d_out);
+        return;
+    }
+    const ProductBf16 pa{d_out_f32, w, nullptr, d_a, d_out, d_in, n, d_in, d_out, 0, false, false};
+    const ProductBf16 pw{d_out_f32, a_bf16, nullptr, d_w, d_out, d_in, d_out, d_in, n, 0, false, true};
+    if ((!d_a || product_bf16_serves(pa, 1)) && (!d_w || product_bf16_serves(pw, 2))) {
+        KernelTimer kt("gemm linear backward");
+        if (d_a) product_bf16(pa, 1);
+        if (d_w && !es.failed()) product_bf16(pw, 2);
         return;
     }
     u16 *wb = reinterpret_cast<u16 *>(scratch(27, (size_t)d_in * d_out * sizeof(u16)));

@@ -248,6 +248,51 @@ def test_linear_pair_and_combine_gate():
     assert rel_err(host(gated.float()), bf16_round(attn) * want_gate) <= 2.0 ** -8
 
 
+@pytest.mark.parametrize("n,d_in,d_out", [(1, 8, 8), (63, 72, 64), (65, 64, 136), (129, 256, 72), (500, 520, 256), (1000, 256, 1040),
+                                          (4100, 256, 256), (7, 20, 12), (9000, 512, 512)])
+def test_linear_pair_at_the_edges_of_its_tiles(n, d_in, d_out):
+    """Row and contraction remainders, split contractions, sizes that the small kernels leave to the library (20 x 12, 9000
+    rows): fp32 sums of bf16 products, each within 2^-24 a term of the sum of magnitudes."""
+    r = np.random.default_rng(n + d_in + d_out)
+    a, w, g = (r.standard_normal(sh).astype(np.float32) for sh in ((n, d_in), (d_out, d_in), (n, d_out)))
+    ta, tw, tg = torch.from_numpy(a).to(BF).cuda(), dev(w), dev(g)
+    out, d_a, d_w = (torch.full(sh, 7.5, device="cuda") for sh in ((n, d_out), (n, d_in), (d_out, d_in)))
+    lib.linear_forward_bf16_rocm(ta.data_ptr(), tw.data_ptr(), out.data_ptr(), n, d_in, d_out)
+    lib.linear_backward_bf16_rocm(tg.data_ptr(), ta.data_ptr(), tw.data_ptr(), d_a.data_ptr(), d_w.data_ptr(), n, d_in, d_out)
+    a, w, g = bf16_round(a), bf16_round(w), bf16_round(g)
+    for got, x, y in ((out, a, w.T), (d_a, g, w), (d_w, g.T, a)):
+        k = x.shape[1]
+        assert (np.abs(host(got) - x @ y) <= 2 ** -24 * (k + 4) * (np.abs(x) @ np.abs(y)) + 1e-30).all(), (n, d_in, d_out, k)
+
+
+@pytest.mark.parametrize("n_extra,levels", [(3, 2), (1, 1), (2, 0), (0, 3)])
+def test_projections_shared_out_are_those_of_one_workgroup(n_extra, levels):
+    """128 tokens share out the projections over workgroups, the same tokens repeated until they fill the chip do not: the
+    same numbers."""
+    nh, s = 4, 128
+    d, many = nh * 64, 300
+    x, w_extra, w_levels, gates = make_inputs(1, s, nh, levels, n_extra, 5)
+    params = [dev(g[k]) for g in gates for k in GATE_NAMES]
+    res = []
+    for bs in (1, many):
+        n = bs * s
+        xd = dev(np.tile(x, (bs, 1)))
+        we, wl = dev(w_extra if n_extra else np.zeros(4, np.float32)), dev(w_levels if levels else np.zeros(4, np.float32))
+        extra = [torch.zeros(n, d, dtype=BF, device="cuda") for _ in range(n_extra)]
+        xb = torch.zeros(n, d, dtype=BF, device="cuda")
+        L = max(levels, 1)
+        heads = [torch.zeros(L * bs * nh, s, 64, dtype=BF, device="cuda") for _ in range(3)]
+        hg = [torch.zeros(L * bs * nh, s, device="cuda") for _ in range(3)]
+        tm = [torch.zeros(L, n, device="cuda") for _ in range(5)]
+        lib.level_project_forward_bf16_rocm(xd.data_ptr(), we.data_ptr(), n_extra, ptr_array(extra), wl.data_ptr(), ptr_array(params),
+                                            xb.data_ptr(), *[t.data_ptr() for t in (*heads, *hg, *tm)], bs, s, nh, 64, levels, 1e-8)
+        torch.cuda.synchronize()
+        one = [t[:s] for t in extra] + [xb[:s]] + [t.view(L, bs, nh, s, -1)[:, -1] for t in (*heads, *hg)] + [t.view(L, bs, s)[:, -1] for t in tm]
+        res.append([t.clone() for t in one])
+    for i, (p, q) in enumerate(zip(*res)):
+        assert torch.equal(p, q), i
+
+
 def test_layer_with_single_bf16_projections_matches_autograd():
     """The whole layer on the path that issues no GEMM from Python, against the float64 autograd restatement:
     all levels active, then with a frozen level (sequence shorter than its period)."""
