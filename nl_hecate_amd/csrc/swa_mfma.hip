@@ -31,24 +31,37 @@ namespace nlh {
 namespace {
 
 typedef __bf16 bh8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bh2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 // The kernels are templates on the head size HDV (64 or 32): NKS = HDV / 32 contraction steps over the dims, NDT = HDV / 16
 // output tiles of dims; the LDS stages keep 64-wide rows either way.
 constexpr int KS = 64;        // keys per LDS stage
-constexpr int LDH = 72;       // LDS row stride in bf16 elements (144 B: 16-byte rows, conflict-free operand reads)
+constexpr int LDH = 80;       // LDS row stride in bf16 elements (160 B: both kinds of operand reads fall on different banks)
 
 __device__ __forceinline__ f32x4 mfma32(uint4 a, uint4 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bh8, a), __builtin_bit_cast(bh8, b), c, 0, 0, 0);
 }
-// two floats -> two bf16 (round to nearest even) in one dword, x in the low half
+// two floats -> two bf16 (round to nearest even) in one dword, x in the low half.  By hand: where a half is widened again
+// the compiler rounds that element a second time.
 __device__ __forceinline__ unsigned pack2(float x, float y) {
-    const bh2 p = {(__bf16)x, (__bf16)y};
-    return __builtin_bit_cast(unsigned, p);
+    unsigned p;
+    asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(p) : "v"(x), "v"(y));
+    return p;
 }
 __device__ __forceinline__ float bf_lo(unsigned w) { return __uint_as_float(w << 16); }
 __device__ __forceinline__ float bf_hi(unsigned w) { return __uint_as_float(w & 0xffff0000u); }
+// Largest of the four lanes that share l % 16, without LDS: the row exchanges of lane_ops.h.
+__device__ __forceinline__ float groups_max(float x) {
+    float a = x, b = x;
+    asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(a), "+v"(b));
+    a = b = fmaxf(a, b);
+    asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(a), "+v"(b));
+    return fmaxf(a, b);
+}
+// mask of elements e (low half) and e + 1 of those numbered first .. last
+__device__ __forceinline__ unsigned own_pair(int e, int first, int last) {
+    return (e >= first && e <= last ? 0xffffu : 0u) | (e + 1 >= first && e + 1 <= last ? 0xffff0000u : 0u);
+}
 // x, y = hi + lo with hi, lo bf16: the pair carries 16 mantissa bits through a bf16 product
 __device__ __forceinline__ void split2(float x, float y, unsigned &hi, unsigned &lo) {
     hi = pack2(x, y);
@@ -204,8 +217,7 @@ __global__ __launch_bounds__(256, 3) void swa_fwd_stats_kernel(const unsigned sh
             for (int kt = 0; kt < 4; kt++)
 #pragma unroll
                 for (int i = 0; i < 4; i++) mx = fmaxf(mx, sc[kt][qt][i]);
-            mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-            mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+            mx = groups_max(mx);
             const float mnew = fmaxf(mrun[qt], mx * c2);
             const float mref = mnew == -INFINITY ? 0.f : mnew;
             const float alpha = __builtin_amdgcn_exp2f(mrun[qt] - mref);
@@ -259,9 +271,13 @@ __global__ __launch_bounds__(256, 3) void swa_fwd_stats_kernel(const unsigned sh
 
 // Forward of the contract (normalised weights stored) in the same blocks: the weights need the final maximum
 // and sum, so the window is swept twice — scores and running statistics first, then scores again, the weights
-// w = bf16(exp2(s c - m) / sum) to their slot rows (four consecutive slots per lane and tile: 8-byte stores at
+// w = bf16(exp2(s c - m) / sum) to their slot rows (eight consecutive slots per lane and pair of tiles: 16-byte stores at
 // 2-byte alignment) and O^T += V^T w^T.  Slots behind an early query's own key (t < window - 1) are zeroed at
-// the end.
+// the end.  8 x 4096 tokens, 8 heads, window 512: 0.21 ms, 0.14 of them without the stores, 0.18 with stores at 8-byte alignment.
+// Where a stage's key (0..63) goes, so that two tiles leave a lane group g eight consecutive keys, 32 hf + 8 g + 4 c + i in row
+// 4 g + i of tile 2 hf + c: the weights of a query then move 16 bytes a lane, 64 side by side.
+__device__ __forceinline__ int stage_row(int key) { return (key & 32) + 16 * ((key >> 2) & 1) + 4 * ((key >> 3) & 3) + (key & 3); }
+
 template <int HDV>
 __global__ __launch_bounds__(256, 3) void swa_fwd_blocked_kernel(const unsigned short *__restrict__ q,
                                                               const unsigned short *__restrict__ k,
@@ -311,14 +327,14 @@ __global__ __launch_bounds__(256, 3) void swa_fwd_blocked_kernel(const unsigned 
                 for (int qt = 0; qt < 2; qt++)
 #pragma unroll
                     for (int i = 0; i < 4; i++) {
-                        const int key = k0 + 16 * kt + 4 * g + i, tq = qlo + 16 * qt + r;
+                        const int key = k0 + 32 * (kt >> 1) + 8 * g + 4 * (kt & 1) + i, tq = qlo + 16 * qt + r;
                         const bool ok = key <= tq && key >= tq + 1 - ws && tq < s;
                         sc[kt][qt][i] = ok ? sc[kt][qt][i] : -INFINITY;
                     }
         }
     };
 
-    // ---- sweep 1: running maximum and sum ----
+    // ---- sweep 1: running maximum and sum, each lane over its own keys; the four lanes of a query meet at the end ----
     float mrun[2] = {-INFINITY, -INFINITY}, lsum[2] = {0.f, 0.f};
     uint4 kreg[2], vreg[2];
     load_rows<HDV>(km, KS * st_lo, kreg);
@@ -327,7 +343,7 @@ __global__ __launch_bounds__(256, 3) void swa_fwd_blocked_kernel(const unsigned 
 #pragma unroll
         for (int c = 0; c < 2; c++) {
             const int chunk = tid + 256 * c;
-            *reinterpret_cast<uint4 *>(&Ks[buf][chunk >> 3][8 * (chunk & 7)]) = kreg[c];
+            *reinterpret_cast<uint4 *>(&Ks[buf][stage_row(chunk >> 3)][8 * (chunk & 7)]) = kreg[c];
         }
         __syncthreads();
         if (st < st_hi) load_rows<HDV>(km, k0 + KS, kreg);
@@ -341,8 +357,6 @@ __global__ __launch_bounds__(256, 3) void swa_fwd_blocked_kernel(const unsigned 
             for (int kt = 0; kt < 4; kt++)
 #pragma unroll
                 for (int i = 0; i < 4; i++) mx = fmaxf(mx, sc[kt][qt][i]);
-            mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-            mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
             const float mnew = fmaxf(mrun[qt], mx * c2);
             const float mref = mnew == -INFINITY ? 0.f : mnew;
             const float alpha = __builtin_amdgcn_exp2f(mrun[qt] - mref);
@@ -358,11 +372,12 @@ __global__ __launch_bounds__(256, 3) void swa_fwd_blocked_kernel(const unsigned 
     float mc[2], inv[2];
 #pragma unroll
     for (int qt = 0; qt < 2; qt++) {
-        float sum = lsum[qt];
+        const float m = groups_max(mrun[qt]);
+        mc[qt] = m == -INFINITY ? 0.f : m;
+        float sum = lsum[qt] * __builtin_amdgcn_exp2f(mrun[qt] - mc[qt]);
         sum += __shfl_xor(sum, 16, 64);
         sum += __shfl_xor(sum, 32, 64);
         inv[qt] = sum > 0.f ? 1.0f / sum : 0.f;
-        mc[qt] = mrun[qt] == -INFINITY ? 0.f : mrun[qt];
     }
 
     // ---- sweep 2: weights out, O^T = V^T w^T ----
@@ -387,8 +402,8 @@ __global__ __launch_bounds__(256, 3) void swa_fwd_blocked_kernel(const unsigned 
 #pragma unroll
         for (int c = 0; c < 2; c++) {
             const int chunk = tid + 256 * c;
-            *reinterpret_cast<uint4 *>(&Ks[buf][chunk >> 3][8 * (chunk & 7)]) = kreg[c];
-            *reinterpret_cast<uint4 *>(&Vs[buf][chunk >> 3][8 * (chunk & 7)]) = vreg[c];
+            *reinterpret_cast<uint4 *>(&Ks[buf][stage_row(chunk >> 3)][8 * (chunk & 7)]) = kreg[c];
+            *reinterpret_cast<uint4 *>(&Vs[buf][stage_row(chunk >> 3)][8 * (chunk & 7)]) = vreg[c];
         }
         __syncthreads();
         if (st < st_hi) {
@@ -413,21 +428,20 @@ __global__ __launch_bounds__(256, 3) void swa_fwd_blocked_kernel(const unsigned 
                     for (int i = 0; i < 4; i++) w[i] = __builtin_amdgcn_exp2f(fmaf(x[i], c2, -mc[qt])) * inv[qt];
                     wp[c][0] = pack2(w[0], w[1]);
                     wp[c][1] = pack2(w[2], w[3]);
-                    // keys key0 .. key0 + 3 of query tq sit in slots key0 - lsq ..; only keys of the window have one
-                    const int key0 = k0 + 16 * (2 * hf + c) + 4 * g;
-                    if (tq < s) {
-                        if (key0 >= lsq[qt] && key0 + 3 <= tq) {
-                            const uint2 pr = make_uint2(wp[c][0], wp[c][1]);
-                            __builtin_memcpy(wrow[qt] + (key0 - lsq[qt]), &pr, 8);
-                        } else if (key0 + 3 >= lsq[qt] && key0 <= tq) {
-#pragma unroll
-                            for (int i = 0; i < 4; i++)
-                                if (key0 + i >= lsq[qt] && key0 + i <= tq)
-                                    wrow[qt][key0 + i - lsq[qt]] = (unsigned short)(wp[c][i >> 1] >> (16 * (i & 1)));
-                        }
-                    }
                 }
                 pb[qt] = make_uint4(wp[0][0], wp[0][1], wp[1][0], wp[1][1]);
+                // keys key0 .. key0 + 7 of query tq sit in slots key0 - lsq ..; only keys of the window have one
+                const int key0 = k0 + 32 * hf + 8 * g;
+                if (tq < s) {
+                    if (key0 >= lsq[qt] && key0 + 7 <= tq) {
+                        __builtin_memcpy(wrow[qt] + (key0 - lsq[qt]), &pb[qt], 16);
+                    } else if (key0 + 7 >= lsq[qt] && key0 <= tq) {
+#pragma unroll
+                        for (int i = 0; i < 8; i++)
+                            if (key0 + i >= lsq[qt] && key0 + i <= tq)
+                                wrow[qt][key0 + i - lsq[qt]] = (unsigned short)(wp[i >> 2][(i >> 1) & 1] >> (16 * (i & 1)));
+                    }
+                }
             }
 #pragma unroll
             for (int dt = 0; dt < NDT; dt++) {
@@ -612,8 +626,10 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_q_stats_kernel(const unsigned 
 
 // Query pass of the contract (weights read back from the tensor) in the same blocks and the same single sweep as
 // swa_bwd_q_stats_kernel: A = sum_j (w dW) k_j, B = sum_j w k_j and D = sum_j w dW together, d_q = (A - D B)/sqrt(hd).
-// A lane's four keys of a tile are four consecutive slots of its query's row: one 8-byte load (2-byte aligned),
-// requested a stage ahead; only the stages at the two ends of the window go slot by slot.
+// A lane's eight keys of two tiles are eight consecutive slots of its query's row: one 16-byte load (2-byte aligned),
+// requested a stage ahead.  Bound by the latency of a stage's chain of LDS reads, products and element work on two waves a
+// SIMD (matrix cores 0.16, vector units 0.26, LDS 0.11 of their time).  8 x 4096 tokens, 8 heads, window 512: 210 us (247
+// with 8-byte loads, slot by slot with a wait in every stage at the window's ends); 192 without any loads of weights.
 template <int HDV>
 __global__ __launch_bounds__(256, 2) void swa_bwd_q_blocked_kernel(const unsigned short *__restrict__ k,
                                                                    const unsigned short *__restrict__ v,
@@ -661,30 +677,39 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_q_blocked_kernel(const unsigne
 #pragma unroll
         for (int dt = 0; dt < NDT; dt++) { aq[qt][dt] = f32x4{0.f, 0.f, 0.f, 0.f}; bq[qt][dt] = f32x4{0.f, 0.f, 0.f, 0.f}; }
 
-    // weights of a stage for this lane: wreg[kt][qt] = keys k0 + 16 kt + 4 g .. + 3 of query qt, zero outside the window
-    uint2 wreg[4][2];
+    // Weights of a stage for this lane: wreg[hf][qt] = keys k0 + 32 hf + 8 g .. + 7 of query qt (stage_row).  At the window's ends
+    // a piece is read whole as well, out of the rows next to it, and what is not the query's own is taken off where the piece
+    // is used: not here, where that would wait for the read.
+    uint4 wreg[2][2];
+    const size_t all = (size_t)gridDim.y * gridDim.z * s * ws;
+    auto whole = [&](int k0) { return k0 + KS - 1 <= qlo && k0 >= qhi + 1 - ws && qhi < s; };
     auto fetch_weights = [&](int k0) {
-        const bool skip = k0 > qhi || k0 + KS - 1 < qlo + 1 - ws;
-        const bool full = k0 + KS - 1 <= qlo && k0 >= qhi + 1 - ws && qhi < s;
+        const bool skip = k0 > qhi || k0 + KS - 1 < qlo + 1 - ws, full = whole(k0);
 #pragma unroll
-        for (int kt = 0; kt < 4; kt++)
+        for (int hf = 0; hf < 2; hf++)
 #pragma unroll
             for (int qt = 0; qt < 2; qt++) {
-                const int key0 = k0 + 16 * kt + 4 * g;
-                wreg[kt][qt] = make_uint2(0u, 0u);
+                const int key0 = k0 + 32 * hf + 8 * g;
+                wreg[hf][qt] = make_uint4(0u, 0u, 0u, 0u);
                 if (skip) continue;
-                if (full || (key0 >= lsq[qt] && key0 + 3 <= tqs[qt])) {
-                    __builtin_memcpy(&wreg[kt][qt], wrow[qt] + (key0 - lsq[qt]), 8);
-                } else {
-                    unsigned d[2] = {0u, 0u};
+                const unsigned short *p = wrow[qt] + (key0 - lsq[qt]);
+                if (full) {
+                    __builtin_memcpy(&wreg[hf][qt], p, 16);
+                } else if (key0 + 7 >= lsq[qt] && key0 <= tqs[qt]) {
+                    const long long at = p - attn_w;
+                    if (at >= 0 && (size_t)at + 8 <= all) {
+                        __builtin_memcpy(&wreg[hf][qt], p, 16);
+                    } else {   // the first or the last row of all
+                        unsigned d[4] = {0u, 0u, 0u, 0u};
 #pragma unroll
-                    for (int e = 0; e < 4; e++) {
-                        const int key = key0 + e;
-                        unsigned x = 0;
-                        if (key >= lsq[qt] && key <= tqs[qt]) x = wrow[qt][key - lsq[qt]];
-                        d[e >> 1] |= x << (16 * (e & 1));
+                        for (int e = 0; e < 8; e++) {
+                            const int key = key0 + e;
+                            unsigned x = 0;
+                            if (key >= lsq[qt] && key <= tqs[qt]) x = wrow[qt][key - lsq[qt]];
+                            d[e >> 1] |= x << (16 * (e & 1));
+                        }
+                        wreg[hf][qt] = make_uint4(d[0], d[1], d[2], d[3]);
                     }
-                    wreg[kt][qt] = make_uint2(d[0], d[1]);
                 }
             }
     };
@@ -698,14 +723,24 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_q_blocked_kernel(const unsigne
 #pragma unroll
         for (int c = 0; c < 2; c++) {
             const int chunk = tid + 256 * c;
-            *reinterpret_cast<uint4 *>(&Ks[buf][chunk >> 3][8 * (chunk & 7)]) = kreg[c];
-            *reinterpret_cast<uint4 *>(&Vs[buf][chunk >> 3][8 * (chunk & 7)]) = vreg[c];
+            *reinterpret_cast<uint4 *>(&Ks[buf][stage_row(chunk >> 3)][8 * (chunk & 7)]) = kreg[c];
+            *reinterpret_cast<uint4 *>(&Vs[buf][stage_row(chunk >> 3)][8 * (chunk & 7)]) = vreg[c];
         }
-        uint2 wcur[4][2];
+        uint4 wcur[2][2];
+        const bool full = whole(k0);
 #pragma unroll
-        for (int kt = 0; kt < 4; kt++)
+        for (int hf = 0; hf < 2; hf++)
 #pragma unroll
-            for (int qt = 0; qt < 2; qt++) wcur[kt][qt] = wreg[kt][qt];
+            for (int qt = 0; qt < 2; qt++) {
+                wcur[hf][qt] = wreg[hf][qt];
+                if (!full) {
+                    const int key0 = k0 + 32 * hf + 8 * g, first = lsq[qt] - key0, last = tqs[qt] - key0;
+                    wcur[hf][qt].x &= own_pair(0, first, last);
+                    wcur[hf][qt].y &= own_pair(2, first, last);
+                    wcur[hf][qt].z &= own_pair(4, first, last);
+                    wcur[hf][qt].w &= own_pair(6, first, last);
+                }
+            }
         __syncthreads();
         if (st < st_hi) {
             load_rows<HDV>(km, k0 + KS, kreg);
@@ -727,7 +762,7 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_q_blocked_kernel(const unsigne
                     dw = mfma32(av0, dol[qt][0], dw);
                     if constexpr (NKS == 2) dw = mfma32(av1, doh[qt][1], dw);
                     if constexpr (NKS == 2) dw = mfma32(av1, dol[qt][1], dw);
-                    const uint2 wp = wcur[kt][qt];
+                    const uint2 wp = c ? make_uint2(wcur[hf][qt].z, wcur[hf][qt].w) : make_uint2(wcur[hf][qt].x, wcur[hf][qt].y);
                     x[c][0] = bf_lo(wp.x) * dw[0];
                     x[c][1] = bf_hi(wp.x) * dw[1];
                     x[c][2] = bf_lo(wp.y) * dw[2];
@@ -735,7 +770,7 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_q_blocked_kernel(const unsigne
                     dpart[qt] += (x[c][0] + x[c][1]) + (x[c][2] + x[c][3]);
                 }
                 split8(x[0], x[1], xh[qt], xl[qt]);
-                wb[qt] = make_uint4(wcur[2 * hf][qt].x, wcur[2 * hf][qt].y, wcur[2 * hf + 1][qt].x, wcur[2 * hf + 1][qt].y);
+                wb[qt] = wcur[hf][qt];
             }
 #pragma unroll
             for (int dt = 0; dt < NDT; dt++) {
@@ -869,7 +904,7 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_k_stats_kernel(const unsigned 
                 for (int jt = 0; jt < 2; jt++) {
                     f32x4 sc = mfma32(aq0, kf[jt][0], f32x4{0.f, 0.f, 0.f, 0.f});
                     if constexpr (NKS == 2) sc = mfma32(aq1, kf[jt][1], sc);
-                    f32x4 dw = mfma32(ah0, vf[jt][0], f32x4{0.f, 0.f, 0.f, 0.f});
+                    f32x4 dw = mfma32(ah0, vf[jt][0], -d4);   // dW - D
                     dw = mfma32(al0, vf[jt][0], dw);
                     if constexpr (NKS == 2) dw = mfma32(ah1, vf[jt][1], dw);
                     if constexpr (NKS == 2) dw = mfma32(al1, vf[jt][1], dw);
@@ -882,10 +917,10 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_k_stats_kernel(const unsigned 
                     }
                     wp[jt][c][0] = pack2(w[0], w[1]);   // as the weight tensor holds them
                     wp[jt][c][1] = pack2(w[2], w[3]);
-                    ds[jt][c][0] = bf_lo(wp[jt][c][0]) * (dw[0] - d4[0]) * scale;
-                    ds[jt][c][1] = bf_hi(wp[jt][c][0]) * (dw[1] - d4[1]) * scale;
-                    ds[jt][c][2] = bf_lo(wp[jt][c][1]) * (dw[2] - d4[2]) * scale;
-                    ds[jt][c][3] = bf_hi(wp[jt][c][1]) * (dw[3] - d4[3]) * scale;
+                    ds[jt][c][0] = bf_lo(wp[jt][c][0]) * dw[0];
+                    ds[jt][c][1] = bf_hi(wp[jt][c][0]) * dw[1];
+                    ds[jt][c][2] = bf_lo(wp[jt][c][1]) * dw[2];
+                    ds[jt][c][3] = bf_hi(wp[jt][c][1]) * dw[3];
                 }
             }
 #pragma unroll
@@ -918,7 +953,7 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_k_stats_kernel(const unsigned 
             unsigned short *pk = o16.k + (row0 + key) * o16.ld + hoff, *pv = o16.v + (row0 + key) * o16.ld + hoff;
 #pragma unroll
             for (int dt = 0; dt < NDT; dt++) {
-                const f32x4 a = dk[jt][dt], c = dv[jt][dt];
+                const f32x4 a = dk[jt][dt] * scale, c = dv[jt][dt];
                 *reinterpret_cast<uint2 *>(pk + 16 * dt + 4 * g) = make_uint2(pack2(a[0], a[1]), pack2(a[2], a[3]));
                 *reinterpret_cast<uint2 *>(pv + 16 * dt + 4 * g) = make_uint2(pack2(c[0], c[1]), pack2(c[2], c[3]));
             }
@@ -928,7 +963,7 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_k_stats_kernel(const unsigned 
 #pragma unroll
         for (int dt = 0; dt < NDT; dt++) {
             f32x4 *ck = reinterpret_cast<f32x4 *>(pk + 16 * dt + 4 * g), *cv = reinterpret_cast<f32x4 *>(pv + 16 * dt + 4 * g);
-            *ck = *ck + dk[jt][dt];
+            *ck = *ck + dk[jt][dt] * scale;
             *cv = *cv + dv[jt][dt];
         }
     }
@@ -937,7 +972,9 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_k_stats_kernel(const unsigned 
 // Key pass of the contract in query blocks, like swa_bwd_k_stats_kernel, with the weights read back from the tensor:
 // the stage's 64 query rows x the block's 128 keys are 256 contiguous bytes per query where the window covers them;
 // they are staged in LDS as [query][key] and a lane takes its two tiles (rows = queries, column = its key) with one
-// transposing read, which is both the B operand of d_v^T += dO^T w and the w of dS = w (dW - D_t) / sqrt(hd).
+// transposing read, which is both the B operand of d_v^T += dO^T w and the w of dS = w (dW - D_t); -D_t is what the sum of
+// dW starts from, 1 / sqrt(hd) is applied to the sum.  Same size as above: 232 us (266 with a wait for slots read one by one
+// in the stages at the window's ends and two more vector instructions an element).
 constexpr int LDW = 144;   // row stride of the weight stage (288 B: the transposing reads of a group fall on 32 banks)
 
 template <int HDV>
@@ -961,9 +998,9 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_k_blocked_kernel(const unsigne
     const int jlo = j0 + 32 * wave, jhi = jlo + 31;
     const int st_lo = j0 / KS, st_hi = min(s - 1, j0 + FQ - 1 + ws - 1) / KS;
     const float *dvb = dvec + (size_t)(b * H + h) * s;
-    const unsigned short *awb = attn_w + ((size_t)(b * H + h) * s) * ws;
-    const StageSrc qm{q, row0, total, hoff, s};
     const float scale = kInvSqrt;
+    const long long row_first = (long long)(b * H + h) * s * ws, all = (long long)gridDim.y * gridDim.z * s * ws;
+    const StageSrc qm{q, row0, total, hoff, s};
 
     uint4 vf[2][2];
 #pragma unroll
@@ -993,30 +1030,35 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_k_blocked_kernel(const unsigne
             if (t < s && dcol < HDV) dreg[c] = *reinterpret_cast<const f32x4 *>(d_out + (row0 + t) * total + hoff + dcol + 4 * c);
         }
         ddreg = (tid < KS && t_lo + tid < s) ? dvb[t_lo + tid] : 0.f;
-        // weights of query t for keys j0 + 32 (tid % 4) .. + 31: four pieces of 8 keys
+        // weights of query t for keys j0 + 32 (tid % 4) .. + 31: four pieces of 8 keys, read whole at the window's ends too
+        // (out of the rows next to it) and freed of what is not the query's own where they go to LDS
         const int lsq = max(t + 1 - ws, 0), thi = t < s ? t : -1;
 #pragma unroll
         for (int c = 0; c < 4; c++) {
             const int key0 = j0 + 32 * (tid & 3) + 8 * c;
             wreg[c] = make_uint4(0, 0, 0, 0);
-            if (key0 >= lsq && key0 + 7 <= thi) {
-                __builtin_memcpy(&wreg[c], awb + (size_t)t * ws + (key0 - lsq), 16);
-            } else if (key0 + 7 >= lsq && key0 <= thi) {
-                unsigned d[4] = {0u, 0u, 0u, 0u};
+            if (key0 + 7 >= lsq && key0 <= thi) {
+                const long long at = row_first + (long long)t * ws + (key0 - lsq);
+                if (at >= 0 && at + 8 <= all) {
+                    __builtin_memcpy(&wreg[c], attn_w + at, 16);
+                } else {   // the first or the last row of all
+                    unsigned d[4] = {0u, 0u, 0u, 0u};
 #pragma unroll
-                for (int e = 0; e < 8; e++) {
-                    const int key = key0 + e;
-                    unsigned x = 0;
-                    if (key >= lsq && key <= thi) x = awb[(size_t)t * ws + (key - lsq)];
-                    d[e >> 1] |= x << (16 * (e & 1));
+                    for (int e = 0; e < 8; e++) {
+                        const int key = key0 + e;
+                        unsigned x = 0;
+                        if (key >= lsq && key <= thi) x = attn_w[row_first + (long long)t * ws + (key - lsq)];
+                        d[e >> 1] |= x << (16 * (e & 1));
+                    }
+                    wreg[c] = make_uint4(d[0], d[1], d[2], d[3]);
                 }
-                wreg[c] = make_uint4(d[0], d[1], d[2], d[3]);
             }
         }
     };
     fetch_stage(KS * st_lo);
     for (int st = st_lo; st <= st_hi; st++) {
         const int buf = (st - st_lo) & 1, t_lo = KS * st;
+        const bool inner = t_lo >= j0 + FQ - 1 && t_lo + KS - 1 <= j0 + ws - 1 && t_lo + KS - 1 < s;   // every query sees every key
 #pragma unroll
         for (int c = 0; c < 2; c++) {
             const int chunk = tid + 256 * c;
@@ -1027,7 +1069,17 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_k_blocked_kernel(const unsigne
             *reinterpret_cast<uint4 *>(&Dl[buf][drow][dcol + 8 * c]) = lo;
         }
 #pragma unroll
-        for (int c = 0; c < 4; c++) *reinterpret_cast<uint4 *>(&Wt[drow][32 * (tid & 3) + 8 * c]) = wreg[c];
+        for (int c = 0; c < 4; c++) {
+            if (!inner) {
+                const int t = t_lo + drow, key0 = j0 + 32 * (tid & 3) + 8 * c;
+                const int first = max(t + 1 - ws, 0) - key0, last = (t < s ? t : -1) - key0;
+                wreg[c].x &= own_pair(0, first, last);
+                wreg[c].y &= own_pair(2, first, last);
+                wreg[c].z &= own_pair(4, first, last);
+                wreg[c].w &= own_pair(6, first, last);
+            }
+            *reinterpret_cast<uint4 *>(&Wt[drow][32 * (tid & 3) + 8 * c]) = wreg[c];
+        }
         if (tid < KS) Dd[buf][tid] = ddreg;
         __syncthreads();
         if (st < st_hi) fetch_stage(t_lo + KS);
@@ -1047,15 +1099,15 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_k_blocked_kernel(const unsigne
                     const f32x4 d4 = *reinterpret_cast<const f32x4 *>(&Dd[buf][16 * qt + 4 * g]);
 #pragma unroll
                     for (int jt = 0; jt < 2; jt++) {
-                        f32x4 dw = mfma32(ah0, vf[jt][0], f32x4{0.f, 0.f, 0.f, 0.f});
+                        f32x4 dw = mfma32(ah0, vf[jt][0], -d4);   // dW - D
                         dw = mfma32(al0, vf[jt][0], dw);
                         if constexpr (NKS == 2) dw = mfma32(ah1, vf[jt][1], dw);
                         if constexpr (NKS == 2) dw = mfma32(al1, vf[jt][1], dw);
                         const unsigned w01 = c ? wpk[jt].z : wpk[jt].x, w23 = c ? wpk[jt].w : wpk[jt].y;
-                        ds[jt][c][0] = bf_lo(w01) * (dw[0] - d4[0]) * scale;
-                        ds[jt][c][1] = bf_hi(w01) * (dw[1] - d4[1]) * scale;
-                        ds[jt][c][2] = bf_lo(w23) * (dw[2] - d4[2]) * scale;
-                        ds[jt][c][3] = bf_hi(w23) * (dw[3] - d4[3]) * scale;
+                        ds[jt][c][0] = bf_lo(w01) * dw[0];
+                        ds[jt][c][1] = bf_hi(w01) * dw[1];
+                        ds[jt][c][2] = bf_lo(w23) * dw[2];
+                        ds[jt][c][3] = bf_hi(w23) * dw[3];
                     }
                 }
 #pragma unroll
@@ -1085,7 +1137,7 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_k_blocked_kernel(const unsigne
 #pragma unroll
         for (int dt = 0; dt < NDT; dt++) {
             f32x4 *ck = reinterpret_cast<f32x4 *>(pk + 16 * dt + 4 * g), *cv = reinterpret_cast<f32x4 *>(pv + 16 * dt + 4 * g);
-            *ck = *ck + dk[jt][dt];
+            *ck = *ck + dk[jt][dt] * scale;
             *cv = *cv + dv[jt][dt];
         }
     }

@@ -70,6 +70,30 @@ def test_swa_forward_backward_parity(B, s, H, hd, ws, npers):
     assert_close("d_v e2e", dv2, ov, REL_TOL_BF16)
 
 
+@pytest.mark.parametrize("s,ws", [(1, 1), (2, 1), (9, 3), (64, 5), (65, 9), (127, 63), (129, 64), (130, 65), (257, 130), (700, 511)])
+@pytest.mark.parametrize("hd", [32, 64])
+def test_weights_at_the_ends_of_the_window_and_of_the_tensor(s, ws, hd):
+    """Pieces of eight weights that hang over a query's row: what lies next to it is another query's, and before the first row
+    and behind the last one there is nothing to read.  Not-a-number weights of one head stay with that head."""
+    B, H = 2, 2
+    q, k, v, go = _case(B, s, H, hd, s + ws + hd)
+    out, aw = gpu_forward(q, k, v, ws, H, 0)
+    oo, awo = orc.swa_forward(q, k, v, ws, H, 0)
+    assert np.abs(orc.bf16_to_f32(aw) - orc.bf16_to_f32(awo)).max() < 1e-2
+    assert_close("out", orc.bf16_to_f32(out), orc.bf16_to_f32(oo), REL_TOL_BF16)
+    want = orc.swa_backward(q, k, v, awo, go, ws, H, 0)
+    # a window of one key: dS = w (dW - D) is zero up to the 16 bits that w dW keeps, and the fp32 sum of dW
+    zero = 2 ** -16 * hd * np.abs(go).max() * max(np.abs(orc.bf16_to_f32(x)).max() for x in (q, k, v)) ** 2
+    close = lambda n, g, w: assert_close(n, g, w, 1e-4) if ws > 1 or n == "d_v" else np.testing.assert_allclose(g, w, atol=zero)
+    for n, g, w in zip(("d_q", "d_k", "d_v"), gpu_backward(q, k, v, awo, go, ws, H, 0), want):
+        close(n, g, w)
+    bad = awo.copy()
+    bad[0, 1], bad[1, 0] = 0x7fc0, 0x7fc0
+    for n, g, w in zip(("d_q", "d_k", "d_v"), gpu_backward(q, k, v, bad, go, ws, H, 0), want):
+        for b, h in ((0, 0), (1, 1)):
+            close(n, g[b, :, h * hd:(h + 1) * hd], w[b, :, h * hd:(h + 1) * hd])
+
+
 def test_swa_known_answers_on_gpu():
     """core/src/swa.rs:286-344: window 1 copies V; identical keys average V."""
     bf = lambda x: orc.f32_to_bf16(np.asarray(x, np.float32))
