@@ -62,6 +62,10 @@ __device__ __forceinline__ float groups_max(float x) {
 __device__ __forceinline__ unsigned own_pair(int e, int first, int last) {
     return (e >= first && e <= last ? 0xffffu : 0u) | (e + 1 >= first && e + 1 <= last ? 0xffff0000u : 0u);
 }
+// Whether eight slots from `slot` on of query t's row, some of them the row's own, lie inside a head of s rows of ws slots.
+__device__ __forceinline__ bool piece_inside(int t, int s, int ws, int slot) {
+    return min(t, 8) * ws + slot >= 0 && (min(s - 1 - t, 8) + 1) * ws - slot >= 8;
+}
 // x, y = hi + lo with hi, lo bf16: the pair carries 16 mantissa bits through a bf16 product
 __device__ __forceinline__ void split2(float x, float y, unsigned &hi, unsigned &lo) {
     hi = pack2(x, y);
@@ -681,7 +685,7 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_q_blocked_kernel(const unsigne
     // a piece is read whole as well, out of the rows next to it, and what is not the query's own is taken off where the piece
     // is used: not here, where that would wait for the read.
     uint4 wreg[2][2];
-    const size_t all = (size_t)gridDim.y * gridDim.z * s * ws;
+    const bool outer_head = b * H + h == 0 || b * H + h == (int)(gridDim.y * gridDim.z) - 1;
     auto whole = [&](int k0) { return k0 + KS - 1 <= qlo && k0 >= qhi + 1 - ws && qhi < s; };
     auto fetch_weights = [&](int k0) {
         const bool skip = k0 > qhi || k0 + KS - 1 < qlo + 1 - ws, full = whole(k0);
@@ -696,8 +700,7 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_q_blocked_kernel(const unsigne
                 if (full) {
                     __builtin_memcpy(&wreg[hf][qt], p, 16);
                 } else if (key0 + 7 >= lsq[qt] && key0 <= tqs[qt]) {
-                    const long long at = p - attn_w;
-                    if (at >= 0 && (size_t)at + 8 <= all) {
+                    if (!outer_head || piece_inside(tqs[qt], s, ws, key0 - lsq[qt])) {
                         __builtin_memcpy(&wreg[hf][qt], p, 16);
                     } else {   // the first or the last row of all
                         unsigned d[4] = {0u, 0u, 0u, 0u};
@@ -999,7 +1002,8 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_k_blocked_kernel(const unsigne
     const int st_lo = j0 / KS, st_hi = min(s - 1, j0 + FQ - 1 + ws - 1) / KS;
     const float *dvb = dvec + (size_t)(b * H + h) * s;
     const float scale = kInvSqrt;
-    const long long row_first = (long long)(b * H + h) * s * ws, all = (long long)gridDim.y * gridDim.z * s * ws;
+    const unsigned short *awb = attn_w + (size_t)(b * H + h) * s * ws;
+    const bool outer_head = b * H + h == 0 || b * H + h == (int)(gridDim.y * gridDim.z) - 1;
     const StageSrc qm{q, row0, total, hoff, s};
 
     uint4 vf[2][2];
@@ -1033,21 +1037,21 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_k_blocked_kernel(const unsigne
         // weights of query t for keys j0 + 32 (tid % 4) .. + 31: four pieces of 8 keys, read whole at the window's ends too
         // (out of the rows next to it) and freed of what is not the query's own where they go to LDS
         const int lsq = max(t + 1 - ws, 0), thi = t < s ? t : -1;
+        const unsigned short *wrow = awb + (size_t)t * ws;
 #pragma unroll
         for (int c = 0; c < 4; c++) {
             const int key0 = j0 + 32 * (tid & 3) + 8 * c;
             wreg[c] = make_uint4(0, 0, 0, 0);
             if (key0 + 7 >= lsq && key0 <= thi) {
-                const long long at = row_first + (long long)t * ws + (key0 - lsq);
-                if (at >= 0 && at + 8 <= all) {
-                    __builtin_memcpy(&wreg[c], attn_w + at, 16);
+                if (!outer_head || piece_inside(t, s, ws, key0 - lsq)) {
+                    __builtin_memcpy(&wreg[c], wrow + (key0 - lsq), 16);
                 } else {   // the first or the last row of all
                     unsigned d[4] = {0u, 0u, 0u, 0u};
 #pragma unroll
                     for (int e = 0; e < 8; e++) {
                         const int key = key0 + e;
                         unsigned x = 0;
-                        if (key >= lsq && key <= thi) x = attn_w[row_first + (long long)t * ws + (key - lsq)];
+                        if (key >= lsq && key <= thi) x = wrow[key - lsq];
                         d[e >> 1] |= x << (16 * (e & 1));
                     }
                     wreg[c] = make_uint4(d[0], d[1], d[2], d[3]);
@@ -1073,10 +1077,12 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_k_blocked_kernel(const unsigne
             if (!inner) {
                 const int t = t_lo + drow, key0 = j0 + 32 * (tid & 3) + 8 * c;
                 const int first = max(t + 1 - ws, 0) - key0, last = (t < s ? t : -1) - key0;
-                wreg[c].x &= own_pair(0, first, last);
-                wreg[c].y &= own_pair(2, first, last);
-                wreg[c].z &= own_pair(4, first, last);
-                wreg[c].w &= own_pair(6, first, last);
+                if (__any(first > 0 || last < 7)) {
+                    wreg[c].x &= own_pair(0, first, last);
+                    wreg[c].y &= own_pair(2, first, last);
+                    wreg[c].z &= own_pair(4, first, last);
+                    wreg[c].w &= own_pair(6, first, last);
+                }
             }
             *reinterpret_cast<uint4 *>(&Wt[drow][32 * (tid & 3) + 8 * c]) = wreg[c];
         }
