@@ -47,17 +47,22 @@ __device__ __forceinline__ bf16x8 ld_op_tr(const u16 *X, int row0, int ks) {
     const s16x8 ab = __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7);
     return __builtin_bit_cast(bf16x8, ab);
 }
+// Two floats rounded to bf16 (nearest, even) in one dword, x in the low half.  By hand: where a half is widened again the
+// compiler rounds that element a second time.
+__device__ __forceinline__ unsigned bf16_pair(float x, float y) {
+    unsigned p;
+    asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(p) : "v"(x), "v"(y));
+    return p;
+}
 // x = hi + lo with hi, lo bf16; both stored as four consecutive elements at off.
 __device__ __forceinline__ void split_store(u16 *H, u16 *Lo, int off, f32x4 x) {
-    bf16x4 h, lo;
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const __bf16 hb = (__bf16)x[i];
-        h[i] = hb;
-        lo[i] = (__bf16)(x[i] - (float)hb);
-    }
-    *reinterpret_cast<bf16x4 *>(H + off) = h;
-    *reinterpret_cast<bf16x4 *>(Lo + off) = lo;
+    uint2 h, lo;
+    h.x = bf16_pair(x[0], x[1]);
+    h.y = bf16_pair(x[2], x[3]);
+    lo.x = bf16_pair(x[0] - __uint_as_float(h.x << 16), x[1] - __uint_as_float(h.x & 0xffff0000u));
+    lo.y = bf16_pair(x[2] - __uint_as_float(h.y << 16), x[3] - __uint_as_float(h.y & 0xffff0000u));
+    *reinterpret_cast<uint2 *>(H + off) = h;
+    *reinterpret_cast<uint2 *>(Lo + off) = lo;
 }
 __device__ __forceinline__ float lane_bcast(float x, int lane) {
     return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), lane));
