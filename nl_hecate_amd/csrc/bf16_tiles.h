@@ -47,11 +47,13 @@ __device__ __forceinline__ bf16x8 ld_op_tr(const u16 *X, int row0, int ks) {
     const s16x8 ab = __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7);
     return __builtin_bit_cast(bf16x8, ab);
 }
-// Two floats rounded to bf16 (nearest, even) in one dword, x in the low half.  By hand: where a half is widened again the
-// compiler rounds that element a second time.
+// Two floats rounded to bf16 (nearest, even) in one dword, x in the low half, opaque to the compiler: where it sees a half
+// widened again it rounds that element a second time.  (The rounding itself stays the compiler's: it knows how long a product's
+// result takes to arrive, which it does not look for inside an asm statement.)
 __device__ __forceinline__ unsigned bf16_pair(float x, float y) {
-    unsigned p;
-    asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(p) : "v"(x), "v"(y));
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    unsigned p = __builtin_bit_cast(unsigned, bf16x2{(__bf16)x, (__bf16)y});
+    asm("" : "+v"(p));
     return p;
 }
 // x = hi + lo with hi, lo bf16; both stored as four consecutive elements at off.

@@ -45,10 +45,10 @@ struct GroupArgs {
 };
 
 // x = hi + mid + lo, three bf16 whose 24 bits hold all of x's.  Two elements at a time, packed as the matrix cores read them;
-// the instruction by hand, because the compiler rounds each element once more to take it off.
+// opaque, because where the compiler sees a piece taken off it rounds that element a second time.
 __device__ __forceinline__ uint32_t bf16_pair(float x, float y) {
-    uint32_t p;
-    asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(p) : "v"(x), "v"(y));
+    uint32_t p = __builtin_bit_cast(uint32_t, bf16x2{(__bf16)x, (__bf16)y});
+    asm("" : "+v"(p));
     return p;
 }
 __device__ __forceinline__ void take_off(float &x, float &y, uint32_t p) {

@@ -31,6 +31,7 @@ namespace nlh {
 namespace {
 
 typedef __bf16 bh8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bh2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 // The kernels are templates on the head size HDV (64 or 32): NKS = HDV / 32 contraction steps over the dims, NDT = HDV / 16
@@ -41,11 +42,11 @@ constexpr int LDH = 80;       // LDS row stride in bf16 elements (160 B: both ki
 __device__ __forceinline__ f32x4 mfma32(uint4 a, uint4 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bh8, a), __builtin_bit_cast(bh8, b), c, 0, 0, 0);
 }
-// two floats -> two bf16 (round to nearest even) in one dword, x in the low half.  By hand: where a half is widened again
-// the compiler rounds that element a second time.
+// two floats -> two bf16 (round to nearest even) in one dword, x in the low half; opaque, because where the compiler sees a half
+// widened again it rounds that element a second time
 __device__ __forceinline__ unsigned pack2(float x, float y) {
-    unsigned p;
-    asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(p) : "v"(x), "v"(y));
+    unsigned p = __builtin_bit_cast(unsigned, bh2{(__bf16)x, (__bf16)y});
+    asm("" : "+v"(p));
     return p;
 }
 __device__ __forceinline__ float bf_lo(unsigned w) { return __uint_as_float(w << 16); }
