@@ -16,8 +16,19 @@ constexpr int HD = 64;             // head size
 constexpr int CW = 64;             // tokens per chunk tile
 constexpr int LDB = 72;            // LDS row stride of a bf16 matrix (144 B: 16-byte rows, conflict-free operand reads)
 constexpr int BMAT = 64 * LDB;     // elements per bf16 matrix
+constexpr int kPerm = 64 * 64;     // elements of a matrix in the permuted layout below
 constexpr int kTileThr = 512;      // 8 waves
 
+// The other layout of a bf16 matrix, of kPerm = 64 x 64 elements, element (row, col): rows of 64, their eight 16-byte blocks permuted by the row's bits 1 to 3 so that
+// what one access takes together falls on different banks.  That is, of a 64-bank LDS: for ld_op rows 0..3 and 12..15 of a
+// block with rows 4..11 of the next; for ld_op_tr rows 0..3 and 8..11 of two blocks; for the 8-byte writes of an accumulator
+// tile sixteen rows of one block.  A row stride that is odd in 16-byte units serves the last but not the first two, an even one
+// the other way round: with either, half of the LDS time of the chain kernels was conflicts (adjoint scan at 128 chains of 4096
+// tokens 191 us so, 168 permuted; forward scan 221, 218).
+__device__ __forceinline__ int bf_at(int row, int col) {
+    const int e = (row >> 1) & 7, f = ((e & 3) << 1) ^ (e >> 2) * 5;
+    return row * 64 + (((col >> 3) ^ f) << 3) + (col & 7);
+}
 __device__ __forceinline__ f32x4 zero4() { return f32x4{0.f, 0.f, 0.f, 0.f}; }
 __device__ __forceinline__ float bf2f(u16 h) { return __uint_as_float(((unsigned)h) << 16); }
 __device__ __forceinline__ f32x4 mfma32(bf16x8 a, bf16x8 b, f32x4 c) {
@@ -30,6 +41,15 @@ __device__ __forceinline__ bf16x8 ld_op(const u16 *X, int row0, int ks) {
     const int l = threadIdx.x & 63;
     return *reinterpret_cast<const bf16x8 *>(X + (row0 + (l & 15)) * LDB + 32 * ks + 8 * (l >> 4));
 }
+__device__ __forceinline__ bf16x8 tr_pair(const u16 *p, const u16 *p4) {
+    typedef short s16x4 __attribute__((ext_vector_type(4)));
+    typedef short s16x8 __attribute__((ext_vector_type(8)));
+    typedef __attribute__((address_space(3))) s16x4 *lds_ptr;
+    const s16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)p);
+    const s16x4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)p4);
+    const s16x8 ab = __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7);
+    return __builtin_bit_cast(bf16x8, ab);
+}
 // The same operand from a matrix stored the other way round (element (contraction index k, row n) at
 // X[k * STRIDE + n]), with no transposed copy: ds_read_b64_tr_b16 works on groups of 16 lanes; when lane s of
 // a group addresses the four elements X[k0 + s/4][n0 + 4 (s%4) .. + 3], lane i receives X[k0 .. k0 + 3][n0 + i].
@@ -37,15 +57,18 @@ __device__ __forceinline__ bf16x8 ld_op(const u16 *X, int row0, int ks) {
 // elements, a multiple of 4; conflict-free inside a group when STRIDE / 2 is 8 modulo 16 (48, 80, ..).
 template <int STRIDE>
 __device__ __forceinline__ bf16x8 ld_op_tr(const u16 *X, int row0, int ks) {
-    typedef short s16x4 __attribute__((ext_vector_type(4)));
-    typedef short s16x8 __attribute__((ext_vector_type(8)));
-    typedef __attribute__((address_space(3))) s16x4 *lds_ptr;
     const int l = threadIdx.x & 63, sl = l & 15;
     const u16 *p = X + (32 * ks + 8 * (l >> 4) + (sl >> 2)) * STRIDE + row0 + 4 * (sl & 3);
-    const s16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)p);
-    const s16x4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(p + 4 * STRIDE));
-    const s16x8 ab = __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7);
-    return __builtin_bit_cast(bf16x8, ab);
+    return tr_pair(p, p + 4 * STRIDE);
+}
+// ld_op and ld_op_tr of a matrix in the permuted layout
+__device__ __forceinline__ bf16x8 ld_perm(const u16 *X, int row0, int ks) {
+    const int l = threadIdx.x & 63;
+    return *reinterpret_cast<const bf16x8 *>(X + bf_at(row0 + (l & 15), 32 * ks + 8 * (l >> 4)));
+}
+__device__ __forceinline__ bf16x8 ld_perm_tr(const u16 *X, int row0, int ks) {   // row0 a multiple of 16
+    const int l = threadIdx.x & 63, sl = l & 15, k = 32 * ks + 8 * (l >> 4) + (sl >> 2), n = row0 + 4 * (sl & 3);
+    return tr_pair(X + bf_at(k, n), X + bf_at(k + 4, n));
 }
 // Two floats rounded to bf16 (nearest, even) in one dword, x in the low half, opaque to the compiler: where it sees a half
 // widened again it rounds that element a second time.  (The rounding itself stays the compiler's: it knows how long a product's

@@ -24,10 +24,16 @@
 namespace nlh {
 namespace {
 
-constexpr int HMAT = 32 * LDB;   // elements of a 32-row bf16 matrix
-constexpr int DYS = 48;          // row stride of a [token][32 rows] bf16 matrix (read through ld_op_tr)
-constexpr int DYM = 64 * DYS;
-constexpr int kLate = 2 * BMAT + 6 * DYM;   // elements of one copy of a chunk's staged inputs
+constexpr int HMAT = 32 * 64;   // elements of a 32-row bf16 matrix
+constexpr int DYM = 64 * 32;     // elements of a [token][32 rows] bf16 matrix
+// Element (token, row) of it: rows of 64 bytes, the halves of a row exchanged with the token's bit 3, so that the tokens
+// 0..3 and 8..11 that a transposing read takes together fall on different banks.
+__device__ __forceinline__ int dy_at(int t, int i) { return t * 32 + ((((i >> 3) ^ ((t >> 2) & 2))) << 3) + (i & 7); }
+__device__ __forceinline__ bf16x8 ld_dy_tr(const u16 *X, int row0, int ks) {   // as ld_op_tr
+    const int l = threadIdx.x & 63, sl = l & 15, k = 32 * ks + 8 * (l >> 4) + (sl >> 2), n = row0 + 4 * (sl & 3);
+    return tr_pair(X + dy_at(k, n), X + dy_at(k + 4, n));
+}
+constexpr int kLate = 2 * kPerm + 6 * DYM;   // elements of one copy of a chunk's staged inputs
 constexpr int kCvec = 5 * CW + 8;
 
 template <bool HAS_S>
@@ -36,8 +42,8 @@ __global__ __launch_bounds__(kTileThr) void cw_adjoint_chain_kernel(
     const float *__restrict__ tab_b, const float *__restrict__ vecs, u16 *__restrict__ dm_snap,
     u16 *__restrict__ ds_snap, float *__restrict__ dm_first, float *__restrict__ ds_first, int s, int C, int nc, int batch, int tab_floats, int vec_floats, HeadRows dyr) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    u16 *WPh = reinterpret_cast<u16 *>(smem_raw), *WPl = WPh + BMAT;   // (W.P)^T [j][t]
-    u16 *dMh = WPl + BMAT, *dMl = dMh + HMAT;                          // dMo [i][c]
+    u16 *WPh = reinterpret_cast<u16 *>(smem_raw), *WPl = WPh + kPerm;   // (W.P)^T [j][t]
+    u16 *dMh = WPl + kPerm, *dMl = dMh + HMAT;                          // dMo [i][c]
     u16 *dSh = dMl + HMAT, *dSl = dSh + HMAT;                          // dSo [i][c]
     u16 *dEh = dSl + HMAT, *dEl = dEh + HMAT;                          // dE^T [i][j]
     // The staged inputs of a chunk exist twice, so that the next step's copy is written while this step's is
@@ -55,7 +61,7 @@ __global__ __launch_bounds__(kTileThr) void cw_adjoint_chain_kernel(
     const int yt = tid >> 3, yg = tid & 7;                                        // dY tile: row t, 4-element block
 
     // zero what is never written again: tiles of (W.P)^T above the diagonal
-    for (int e = tid; e < BMAT / 2; e += kTileThr) {
+    for (int e = tid; e < kPerm / 2; e += kTileThr) {
         reinterpret_cast<unsigned *>(WPh)[e] = 0u;
         reinterpret_cast<unsigned *>(WPl)[e] = 0u;
     }
@@ -98,13 +104,13 @@ __global__ __launch_bounds__(kTileThr) void cw_adjoint_chain_kernel(
     // does not use.
     auto commit = [&](int c, int par) {
         const int L = min(C, s - c * C);
-        u16 *Kr = late + par * kLate, *Qr = Kr + BMAT;
-        u16 *dYh = Qr + BMAT, *dYl = dYh + DYM, *dYah = dYl + DYM, *dYal = dYah + DYM, *dYbh = dYal + DYM, *dYbl = dYbh + DYM;
+        u16 *Kr = late + par * kLate, *Qr = Kr + kPerm;
+        u16 *dYh = Qr + kPerm, *dYl = dYh + DYM, *dYah = dYl + DYM, *dYal = dYah + DYM, *dYbh = dYal + DYM, *dYbl = dYbh + DYM;
         if (st_t >= L) { nK = make_uint4(0, 0, 0, 0); nQ = nK; }
         if (yt >= L) ndY = zero4();
-        *reinterpret_cast<uint4 *>(Kr + st_t * LDB + st_cb * 8) = nK;
-        *reinterpret_cast<uint4 *>(Qr + st_t * LDB + st_cb * 8) = nQ;
-        const int off = yt * DYS + yg * 4;
+        *reinterpret_cast<uint4 *>(Kr + bf_at(st_t, st_cb * 8)) = nK;
+        *reinterpret_cast<uint4 *>(Qr + bf_at(st_t, st_cb * 8)) = nQ;
+        const int off = dy_at(yt, yg * 4);
         split_store(dYh, dYl, off, ndY);
         split_store(dYah, dYal, off, na * ndY);
         if (HAS_S) split_store(dYbh, dYbl, off, nb * ndY);
@@ -118,7 +124,7 @@ __global__ __launch_bounds__(kTileThr) void cw_adjoint_chain_kernel(
     // from the LDS copy at the top of the next step, as whole 128-byte rows (from the accumulator layout a wave
     // would store 32-byte pieces of 16 different lines).  The gradient of the initial state (slot 0) leaves in fp32.
     auto publish = [&](int slot) {
-        const int e = (i0 + 16 * ct + r16) * HD + 16 * rt + 4 * g, off = (16 * ct + r16) * LDB + 16 * rt + 4 * g;
+        const int e = (i0 + 16 * ct + r16) * HD + 16 * rt + 4 * g, off = bf_at(16 * ct + r16, 16 * rt + 4 * g);
         split_store(dMh, dMl, off, dM);
         if (HAS_S) split_store(dSh, dSl, off, dS);
         if (slot == 0) {
@@ -129,7 +135,7 @@ __global__ __launch_bounds__(kTileThr) void cw_adjoint_chain_kernel(
     auto store_snapshot = [&](int slot) {   // threads 0..255: a row piece of dMo, 256..511: of dSo
         const int which = tid >> 8, row = (tid & 255) >> 3, c8 = (tid & 7) * 8;
         if (which && !HAS_S) return;
-        const uint4 x = *reinterpret_cast<const uint4 *>((which ? dSh : dMh) + row * LDB + c8);
+        const uint4 x = *reinterpret_cast<const uint4 *>((which ? dSh : dMh) + bf_at(row, c8));
         *reinterpret_cast<uint4 *>((which ? ds_snap : dm_snap) + state0 + (size_t)slot * HD * HD + (i0 + row) * HD + c8) = x;
     };
 
@@ -137,17 +143,17 @@ __global__ __launch_bounds__(kTileThr) void cw_adjoint_chain_kernel(
     // on the scan, so it is computed a step ahead, in the shadow of the step's last phase.
     auto weights = [&](int par) {
         const float *cvec = cvecs + par * kCvec;
-        const u16 *Kr = late + par * kLate, *Qr = Kr + BMAT;
-        const bf16x8 aq[2] = {ld_op(Qr, 16 * tt, 0), ld_op(Qr, 16 * tt, 1)};
+        const u16 *Kr = late + par * kLate, *Qr = Kr + kPerm;
+        const bf16x8 aq[2] = {ld_perm(Qr, 16 * tt, 0), ld_perm(Qr, 16 * tt, 1)};
 #pragma unroll
         for (int x = 0; x < 2; x++) {
             const int jt = jt0 + x;
             if (jt <= tt) {
                 f32x4 p = zero4();
 #pragma unroll
-                for (int ks = 0; ks < 2; ks++) p = mfma32(aq[ks], ld_op(Kr, 16 * jt, ks), p);
+                for (int ks = 0; ks < 2; ks++) p = mfma32(aq[ks], ld_perm(Kr, 16 * jt, ks), p);
                 const float nth = -cvec[4 * CW + 16 * jt + r16];
-                split_store(WPh, WPl, (16 * jt + r16) * LDB + 16 * tt + 4 * g, nth * ctab[x] * p);   // [j][t .. t+3]
+                split_store(WPh, WPl, bf_at(16 * jt + r16, 16 * tt + 4 * g), nth * ctab[x] * p);   // [j][t .. t+3]
             }
         }
     };
@@ -166,8 +172,8 @@ __global__ __launch_bounds__(kTileThr) void cw_adjoint_chain_kernel(
     for (int c = nc - 1; c >= 0; c--) {
         const int L = min(C, s - c * C), par = c & 1;
         const float *cvec = cvecs + par * kCvec;
-        const u16 *Kr = late + par * kLate, *Qr = Kr + BMAT;
-        const u16 *dYh = Qr + BMAT, *dYl = dYh + DYM, *dYah = dYl + DYM, *dYal = dYah + DYM, *dYbh = dYal + DYM, *dYbl = dYbh + DYM;
+        const u16 *Kr = late + par * kLate, *Qr = Kr + kPerm;
+        const u16 *dYh = Qr + kPerm, *dYl = dYh + DYM, *dYah = dYl + DYM, *dYal = dYah + DYM, *dYbh = dYal + DYM, *dYbl = dYbh + DYM;
         store_snapshot(c + 1);
         commit(max(c - 1, 0), par ^ 1);
         fetch(max(c - 2, 0));
@@ -176,23 +182,23 @@ __global__ __launch_bounds__(kTileThr) void cw_adjoint_chain_kernel(
             f32x4 e1 = zero4(), e2 = zero4(), e3 = zero4();
 #pragma unroll
             for (int ks = 0; ks < 2; ks++) {
-                const bf16x8 wh = ld_op(WPh, 16 * rt, ks), wl = ld_op(WPl, 16 * rt, ks), ak = ld_op(Kr, 16 * rt, ks);
-                const bf16x8 yh = ld_op_tr<DYS>(dYh, 16 * ct, ks), yl = ld_op_tr<DYS>(dYl, 16 * ct, ks);
+                const bf16x8 wh = ld_perm(WPh, 16 * rt, ks), wl = ld_perm(WPl, 16 * rt, ks), ak = ld_perm(Kr, 16 * rt, ks);
+                const bf16x8 yh = ld_dy_tr(dYh, 16 * ct, ks), yl = ld_dy_tr(dYl, 16 * ct, ks);
                 e1 = mfma32(wh, yh, e1);
                 e1 = mfma32(wl, yh, e1);
                 e1 = mfma32(wh, yl, e1);
-                e2 = mfma32(ak, ld_op(dMh, 16 * ct, ks), e2);
-                e2 = mfma32(ak, ld_op(dMl, 16 * ct, ks), e2);
+                e2 = mfma32(ak, ld_perm(dMh, 16 * ct, ks), e2);
+                e2 = mfma32(ak, ld_perm(dMl, 16 * ct, ks), e2);
                 if (HAS_S) {
-                    e3 = mfma32(ak, ld_op(dSh, 16 * ct, ks), e3);
-                    e3 = mfma32(ak, ld_op(dSl, 16 * ct, ks), e3);
+                    e3 = mfma32(ak, ld_perm(dSh, 16 * ct, ks), e3);
+                    e3 = mfma32(ak, ld_perm(dSl, 16 * ct, ks), e3);
                 }
             }
             const int j4 = 16 * rt + 4 * g;
             const f32x4 th = *reinterpret_cast<const f32x4 *>(cvec + 4 * CW + j4);
             const f32x4 cl = *reinterpret_cast<const f32x4 *>(cvec + 2 * CW + j4);
             const f32x4 bl = *reinterpret_cast<const f32x4 *>(cvec + 3 * CW + j4);
-            split_store(dEh, dEl, (16 * ct + r16) * LDB + j4, e1 - th * (cl * e2 + bl * e3));   // [i][j .. j+3]
+            split_store(dEh, dEl, bf_at(16 * ct + r16, j4), e1 - th * (cl * e2 + bl * e3));   // [i][j .. j+3]
         }
         __syncthreads();
         // ── dM0^T, dS0^T: tile rows c = 16 rt.., columns i = 16 ct.. ──
@@ -200,14 +206,14 @@ __global__ __launch_bounds__(kTileThr) void cw_adjoint_chain_kernel(
             f32x4 am = zero4(), as = zero4();
 #pragma unroll
             for (int ks = 0; ks < 2; ks++) {
-                const bf16x8 aq = ld_op_tr<LDB>(Qr, 16 * rt, ks), ak = ld_op_tr<LDB>(Kr, 16 * rt, ks);   // Q^T, K^T
-                am = mfma32(aq, ld_op_tr<DYS>(dYah, 16 * ct, ks), am);
-                am = mfma32(aq, ld_op_tr<DYS>(dYal, 16 * ct, ks), am);
-                am = mfma32(ak, ld_op(dEh, 16 * ct, ks), am);
-                am = mfma32(ak, ld_op(dEl, 16 * ct, ks), am);
+                const bf16x8 aq = ld_perm_tr(Qr, 16 * rt, ks), ak = ld_perm_tr(Kr, 16 * rt, ks);   // Q^T, K^T
+                am = mfma32(aq, ld_dy_tr(dYah, 16 * ct, ks), am);
+                am = mfma32(aq, ld_dy_tr(dYal, 16 * ct, ks), am);
+                am = mfma32(ak, ld_perm(dEh, 16 * ct, ks), am);
+                am = mfma32(ak, ld_perm(dEl, 16 * ct, ks), am);
                 if (HAS_S) {
-                    as = mfma32(aq, ld_op_tr<DYS>(dYbh, 16 * ct, ks), as);
-                    as = mfma32(aq, ld_op_tr<DYS>(dYbl, 16 * ct, ks), as);
+                    as = mfma32(aq, ld_dy_tr(dYbh, 16 * ct, ks), as);
+                    as = mfma32(aq, ld_dy_tr(dYbl, 16 * ct, ks), as);
                 }
             }
             const float aL = cvec[L - 1], betaL = cvec[CW + L - 1], hL = cvec[5 * CW + 4];
@@ -223,7 +229,7 @@ __global__ __launch_bounds__(kTileThr) void cw_adjoint_chain_kernel(
     }
 }
 
-constexpr size_t kAdjointLds = (2 * BMAT + 6 * HMAT + 2 * kLate) * sizeof(u16) + 2 * kCvec * sizeof(float);
+constexpr size_t kAdjointLds = (2 * kPerm + 6 * HMAT + 2 * kLate) * sizeof(u16) + 2 * kCvec * sizeof(float);
 
 }  // namespace
 

@@ -114,13 +114,13 @@ __global__ __launch_bounds__(kChainThr) void cw_chain_fwd_kernel(
     const float *__restrict__ table, const float *__restrict__ vecs, const float *__restrict__ m_initial,
     const float *__restrict__ s_initial, float *__restrict__ m_states, float *__restrict__ s_states,
     float *__restrict__ y, int s, int C, int nc, int batch, HeadRows yr, ChainTracks tr) {
-    constexpr int HMAT = 32 * LDB;   // a 32-row matrix
+    constexpr int HMAT = 32 * 64;   // a 32-row matrix
     extern __shared__ __align__(16) unsigned char smem_raw[];
     u16 *Kr = reinterpret_cast<u16 *>(smem_raw);   // K [t][c]
-    u16 *Kt0 = Kr + BMAT, *Kt1 = Kt0 + BMAT;       // K^T [c][t] of this chunk / V [t][i] until K^T of the next lands
-    u16 *Qr0 = Kt1 + BMAT, *Qr1 = Qr0 + BMAT;      // Q [t][c], alternating between chunks
-    u16 *WPh = Qr1 + BMAT, *WPl = WPh + BMAT;      // W.P [t][j]
-    u16 *Mh = WPl + BMAT, *Ml = Mh + HMAT;         // chunk-start M [i][c], this workgroup's 32 rows, hi / lo
+    u16 *Kt0 = Kr + kPerm, *Kt1 = Kt0 + kPerm;       // K^T [c][t] of this chunk / V [t][i] until K^T of the next lands
+    u16 *Qr0 = Kt1 + kPerm, *Qr1 = Qr0 + kPerm;      // Q [t][c], alternating between chunks
+    u16 *WPh = Qr1 + kPerm, *WPl = WPh + kPerm;      // W.P [t][j]
+    u16 *Mh = WPl + kPerm, *Ml = Mh + HMAT;         // chunk-start M [i][c], this workgroup's 32 rows, hi / lo
     u16 *Sh = Ml + HMAT, *Sl = Sh + HMAT;          // chunk-start S
     u16 *Eh = Sl + HMAT, *El = Eh + HMAT;          // E^T [i][t]
     u16 *EMh = El + HMAT, *EMl = EMh + HMAT;       // (E.wM)^T
@@ -188,17 +188,17 @@ __global__ __launch_bounds__(kChainThr) void cw_chain_fwd_kernel(
         // arrival to this point
         asm volatile("" : "+v"(sv.x), "+v"(sv.y), "+v"(sv.z), "+v"(sv.w), "+v"(vn));
     };
-    auto commit_rows = [&](u16 *dst, const uint4 &x) { *reinterpret_cast<uint4 *>(dst + st_t * LDB + st_cb * 8) = x; };
+    auto commit_rows = [&](u16 *dst, const uint4 &x) { *reinterpret_cast<uint4 *>(dst + bf_at(st_t, st_cb * 8)) = x; };
     auto commit_kt = [&](u16 *Kt) {
         const unsigned kw[4] = {sk.x, sk.y, sk.z, sk.w};
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            Kt[(st_cb * 8 + 2 * i) * LDB + st_t] = (u16)(kw[i] & 0xffffu);
-            Kt[(st_cb * 8 + 2 * i + 1) * LDB + st_t] = (u16)(kw[i] >> 16);
+            Kt[bf_at(st_cb * 8 + 2 * i, st_t)] = (u16)(kw[i] & 0xffffu);
+            Kt[bf_at(st_cb * 8 + 2 * i + 1, st_t)] = (u16)(kw[i] >> 16);
         }
     };
     auto commit_v = [&](u16 *dst) {
-        if (tid < 256) *reinterpret_cast<uint4 *>(dst + vt * LDB + vcb * 8) = sv;
+        if (tid < 256) *reinterpret_cast<uint4 *>(dst + bf_at(vt, vcb * 8)) = sv;
     };
     auto commit_vecs = [&]() {
         if (tid < 4 * CW + 4) cvec[tid] = vn;
@@ -219,7 +219,7 @@ __global__ __launch_bounds__(kChainThr) void cw_chain_fwd_kernel(
     auto stage_state = [&]() {             // -> LDS operands of the next chunk
 #pragma unroll
         for (int ct = 0; ct < 2; ct++) {
-            const int off = (16 * ct + r16) * LDB + 16 * bi + 4 * g;
+            const int off = bf_at(16 * ct + r16, 16 * bi + 4 * g);
             split_store(Mh, Ml, off, Mm[ct]);
             if (HAS_S) split_store(Sh, Sl, off, Sm[ct]);
         }
@@ -268,8 +268,8 @@ __global__ __launch_bounds__(kChainThr) void cw_chain_fwd_kernel(
         // ── first half: E^T, (E.wM)^T, (E.wS)^T (group X) and W.P (group Y) ──
         if (grpX) {
             // E[t][i]: rows t = 16 bi .., columns i = 16 ct ..
-            const bf16x8 aK[2] = {ld_op(Kr, 16 * bi, 0), ld_op(Kr, 16 * bi, 1)};
-            const bf16x8 aV = ld_op(Kn, 16 * bi, 0);
+            const bf16x8 aK[2] = {ld_perm(Kr, 16 * bi, 0), ld_perm(Kr, 16 * bi, 1)};
+            const bf16x8 aV = ld_perm(Kn, 16 * bi, 0);
             const f32x4 wm = *reinterpret_cast<const f32x4 *>(cvec + 2 * CW + 16 * bi + 4 * g);
             const f32x4 wsv = *reinterpret_cast<const f32x4 *>(cvec + 3 * CW + 16 * bi + 4 * g);
             f32x4 esq = zero4();
@@ -278,12 +278,12 @@ __global__ __launch_bounds__(kChainThr) void cw_chain_fwd_kernel(
                 f32x4 e = zero4();
 #pragma unroll
                 for (int ks = 0; ks < 2; ks++) {
-                    e = mfma32(aK[ks], ld_op(Mh, 16 * ct, ks), e);
-                    e = mfma32(aK[ks], ld_op(Ml, 16 * ct, ks), e);
+                    e = mfma32(aK[ks], ld_perm(Mh, 16 * ct, ks), e);
+                    e = mfma32(aK[ks], ld_perm(Ml, 16 * ct, ks), e);
                 }
                 e = mfma32(aV, negI[ct], e);
                 if (TRACK) esq += e * e;
-                const int off = (16 * ct + r16) * LDB + 16 * bi + 4 * g;   // [i][t .. t+3]
+                const int off = bf_at(16 * ct + r16, 16 * bi + 4 * g);   // [i][t .. t+3]
                 split_store(Eh, El, off, e);
                 split_store(EMh, EMl, off, e * wm);
                 if (HAS_S) split_store(ESh, ESl, off, e * wsv);
@@ -299,13 +299,13 @@ __global__ __launch_bounds__(kChainThr) void cw_chain_fwd_kernel(
 #pragma unroll
             for (int rt = 0; rt < 2; rt++)
 #pragma unroll
-                for (int ks = 0; ks < 2; ks++) aK[rt][ks] = ld_op(Kr, bm + 16 * rt, ks);
+                for (int ks = 0; ks < 2; ks++) aK[rt][ks] = ld_perm(Kr, bm + 16 * rt, ks);
             f32x4 acc[2][2] = {{zero4(), zero4()}, {zero4(), zero4()}};
 #pragma unroll
             for (int ks = 0; ks < 2; ks++)
 #pragma unroll
                 for (int ct = 0; ct < 2; ct++) {
-                    const bf16x8 bq = ld_op(Qc, bn + 16 * ct, ks);
+                    const bf16x8 bq = ld_perm(Qc, bn + 16 * ct, ks);
 #pragma unroll
                     for (int rt = 0; rt < 2; rt++)     // P^T[j][t]: rows j, columns t
                         acc[rt][ct] = mfma32(aK[rt][ks], bq, acc[rt][ct]);
@@ -314,7 +314,7 @@ __global__ __launch_bounds__(kChainThr) void cw_chain_fwd_kernel(
             for (int rt = 0; rt < 2; rt++)
 #pragma unroll
                 for (int ct = 0; ct < 2; ct++)         // [t][j .. j+3]
-                    split_store(WPh, WPl, (bn + 16 * ct + r16) * LDB + bm + 16 * rt + 4 * g,
+                    split_store(WPh, WPl, bf_at(bn + 16 * ct + r16, bm + 16 * rt + 4 * g),
                                 wc[rt][ct] * acc[rt][ct]);
         }
         __syncthreads();
@@ -327,18 +327,18 @@ __global__ __launch_bounds__(kChainThr) void cw_chain_fwd_kernel(
             y0[0] = y0[1] = y1[0] = y1[1] = zero4();
 #pragma unroll
             for (int ks = 0; ks < 2; ks++) {
-                const bf16x8 bQ = ld_op(Qc, 16 * bi, ks), bWh = ld_op(WPh, 16 * bi, ks), bWl = ld_op(WPl, 16 * bi, ks);
+                const bf16x8 bQ = ld_perm(Qc, 16 * bi, ks), bWh = ld_perm(WPh, 16 * bi, ks), bWl = ld_perm(WPl, 16 * bi, ks);
 #pragma unroll
                 for (int rt = 0; rt < 2; rt++) {
-                    const bf16x8 eh = ld_op(Eh, 16 * rt, ks);
-                    y0[rt] = mfma32(ld_op(Mh, 16 * rt, ks), bQ, y0[rt]);
-                    y0[rt] = mfma32(ld_op(Ml, 16 * rt, ks), bQ, y0[rt]);
+                    const bf16x8 eh = ld_perm(Eh, 16 * rt, ks);
+                    y0[rt] = mfma32(ld_perm(Mh, 16 * rt, ks), bQ, y0[rt]);
+                    y0[rt] = mfma32(ld_perm(Ml, 16 * rt, ks), bQ, y0[rt]);
                     y2[rt] = mfma32(eh, bWh, y2[rt]);
                     y2[rt] = mfma32(eh, bWl, y2[rt]);
-                    y2[rt] = mfma32(ld_op(El, 16 * rt, ks), bWh, y2[rt]);
+                    y2[rt] = mfma32(ld_perm(El, 16 * rt, ks), bWh, y2[rt]);
                     if (HAS_S) {
-                        y1[rt] = mfma32(ld_op(Sh, 16 * rt, ks), bQ, y1[rt]);
-                        y1[rt] = mfma32(ld_op(Sl, 16 * rt, ks), bQ, y1[rt]);
+                        y1[rt] = mfma32(ld_perm(Sh, 16 * rt, ks), bQ, y1[rt]);
+                        y1[rt] = mfma32(ld_perm(Sl, 16 * rt, ks), bQ, y1[rt]);
                     }
                 }
             }
@@ -350,14 +350,14 @@ __global__ __launch_bounds__(kChainThr) void cw_chain_fwd_kernel(
             f32x4 am[2] = {zero4(), zero4()}, as[2] = {zero4(), zero4()};
 #pragma unroll
             for (int ks = 0; ks < 2; ks++) {
-                const bf16x8 aKt = ld_op(Kc, 16 * bi, ks);
+                const bf16x8 aKt = ld_perm(Kc, 16 * bi, ks);
 #pragma unroll
                 for (int ct = 0; ct < 2; ct++) {
-                    am[ct] = mfma32(aKt, ld_op(EMh, 16 * ct, ks), am[ct]);
-                    am[ct] = mfma32(aKt, ld_op(EMl, 16 * ct, ks), am[ct]);
+                    am[ct] = mfma32(aKt, ld_perm(EMh, 16 * ct, ks), am[ct]);
+                    am[ct] = mfma32(aKt, ld_perm(EMl, 16 * ct, ks), am[ct]);
                     if (HAS_S) {
-                        as[ct] = mfma32(aKt, ld_op(ESh, 16 * ct, ks), as[ct]);
-                        as[ct] = mfma32(aKt, ld_op(ESl, 16 * ct, ks), as[ct]);
+                        as[ct] = mfma32(aKt, ld_perm(ESh, 16 * ct, ks), as[ct]);
+                        as[ct] = mfma32(aKt, ld_perm(ESl, 16 * ct, ks), as[ct]);
                     }
                 }
             }
@@ -392,7 +392,7 @@ __global__ __launch_bounds__(kChainThr) void cw_chain_fwd_kernel(
     }
 }
 
-constexpr size_t kChainFwdLds = (7 * BMAT + 10 * 32 * LDB) * sizeof(u16) + (4 * CW + 4) * sizeof(float);
+constexpr size_t kChainFwdLds = (7 * kPerm + 10 * 32 * 64) * sizeof(u16) + (4 * CW + 4) * sizeof(float);
 
 template <bool HAS_S>
 void launch_forward(const char *fn, const u16 *k, const u16 *v, const u16 *q, const float *alpha, const float *theta,
