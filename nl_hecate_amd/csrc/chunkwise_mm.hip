@@ -34,6 +34,7 @@
 #include "chunkwise_guard.h"
 #include "mm_coef.h"
 #include "mm_tiles.h"
+#include "quad_rows.h"
 #include "rule_common.h"
 #include "runtime.h"
 
@@ -45,6 +46,15 @@ using namespace mmt;
 // Per-chunk scratch written by the local passes and read by the scans:
 //   loc  [chain][chunk][4][64*64]: T_a, T_b, C_1, C_2      locs [chain][chunk][4]: a_L, beta_L, h_L
 constexpr size_t kLocMats = 4;
+// in the order in which the scan's waves take them, 1 KB of consecutive memory a load: T_a, T_b [column tile][piece of four
+// contraction indices][lane], C_1, C_2 [row block][column tile][lane].  A lane of an accumulator tile (rows 16 ib + 4 (l / 16)
+// + i, column 16 ct + l % 16) holds one piece of either.
+__device__ __forceinline__ void store_operand_tile(float *mat, const f32x4 &t, int ib, int ct, int l) {
+    *reinterpret_cast<f32x4 *>(mat + ((ct * 4 + (l >> 4)) * 64 + 16 * ib + (l & 15)) * 4) = t;
+}
+__device__ __forceinline__ void store_acc_tile(float *mat, const f32x4 &t, int ib, int ct, int l) {
+    *reinterpret_cast<f32x4 *>(mat + ((ib * 4 + ct) * 64 + l) * 4) = t;
+}
 
 // ── pass 1 (forward) / shared with the backward: chunk-local matrices ───────
 // T_a = a_L I + K^T diag(wM) K,  T_b = K^T diag(wS) K  (both symmetric);
@@ -96,102 +106,110 @@ __global__ __launch_bounds__(kThr) void cw_local_fwd_kernel(const TIn *__restric
         Strip acc = zero_strip();
         mma(acc, [&](int m, int kk) { return Am[kk * LDM + m0 + m] * wv[kk]; }, bK);
         for_c(acc, [&](int r, int c, float &x) {
-            const int row = m0 + r, col = n0 + c;
-            float y = o < 2 ? x : -x;
-            if (o == 0 && row == col) y += aL;
-            out[(size_t)o * HD * HD + row * HD + col] = y;
+            if (o >= 2) x = -x;
+            if (o == 0 && m0 + r == n0 + c) x += aL;
         });
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+            if (o < 2) store_operand_tile(out + (size_t)o * HD * HD, acc.t[t], m0 / 16, n0 / 16 + t, threadIdx.x & 63);
+            else store_acc_tile(out + (size_t)o * HD * HD, acc.t[t], m0 / 16, n0 / 16 + t, threadIdx.x & 63);
+        }
     }
 }
 
-// ── pass 2: scan over chunks, one workgroup per (chain, 32-row block) ────────
+// ── pass 2: scan over chunks, one workgroup per (chain, 16-row block) ────────
 // FWD:  X1' = X1 T_a + s1 X2 + C_1,  X2' = X1 T_b + s2 X2 + C_2,  (s1, s2) = (beta_L, h_L)
 //       states[chain][c+1] = f(states[chain][c]), slot 0 = initial state
 // BWD:  X1' = X1 T_a + X2 T_b + C_1, X2' = s1 X1 + s2 X2 + C_2
 //       states[chain][c] = g(states[chain][c+1]), slot nc = 0
-// Eight strips per step: (product 0/1) x (16-row half) x (32-column half).
-template <bool FWD>
-__global__ __launch_bounds__(kThr) void cw_scan_kernel(const float *__restrict__ init1,
-                                                       const float *__restrict__ init2,
-                                                       const float *__restrict__ loc,
-                                                       const float *__restrict__ locs, float *__restrict__ st1,
-                                                       float *__restrict__ st2, int nc, int has_s) {
-    __shared__ float X1[32 * LDM], X2[32 * LDM], Ta[MAT], Tb[MAT], part[4][16 * 33];
-    const int chain = blockIdx.x >> 1, r0 = 32 * (blockIdx.x & 1);
-    const int w = threadIdx.x >> 6, which = w >> 2, m0 = 16 * ((w >> 1) & 1), n0 = 32 * (w & 1), pidx = w & 3;
-    float *s1p = st1 + (size_t)chain * (nc + 1) * HD * HD, *s2p = st2 ? st2 + (size_t)chain * (nc + 1) * HD * HD : nullptr;
-    for (int e = threadIdx.x; e < 32 * 64; e += kThr) {
-        const int rr = e >> 6, cc = e & 63;
-        float x1 = 0.f, x2 = 0.f;
-        if (FWD) {
-            x1 = init1[(size_t)chain * HD * HD + (r0 + rr) * HD + cc];
-            if (has_s) x2 = init2[(size_t)chain * HD * HD + (r0 + rr) * HD + cc];
+// The rows of X never mix: 16 of them are a workgroup's, 16 columns a wave's (four waves).  A wave keeps its columns of X1, X2
+// in registers and takes both products for them, T_a and T_b straight from memory as operands, two steps ahead; only X as an
+// operand goes through LDS, in two buffers with one barrier a step.  Bound by the 32 fp32 matrix instructions of a step (1024
+// clocks of 2500) and the exchange around them: 32 chains x 24 chunks 25 us forward, 26 backward (54 and 59 with 32 rows a
+// workgroup, T staged in LDS and three barriers a step).
+template <bool FWD, bool HAS_S>   // HAS_S at compile time: only a fixed number of stores and loads in flight can be waited past
+__global__ __launch_bounds__(256) void cw_scan_kernel(const float *__restrict__ init1, const float *__restrict__ init2,
+                                                      const float *__restrict__ loc, const float *__restrict__ locs,
+                                                      float *__restrict__ st1, float *__restrict__ st2, int nc, int batch) {
+    constexpr int LX = 68;   // row stride: 16-byte rows
+    __shared__ __align__(16) float X[2][2][16 * LX];
+    // the four workgroups of a chain read the same T: ids 8 apart share an XCD's L2
+    const int id = blockIdx.x, chain = batch & 7 ? id >> 2 : (id >> 5) * 8 + (id & 7), r0 = 16 * (batch & 7 ? id & 3 : (id >> 3) & 3);
+    const int l = threadIdx.x & 63, r = l & 15, kb = 16 * (l >> 4), m = 4 * (l >> 4), ct = threadIdx.x >> 6, col = 16 * ct + r;
+    float *s1p = st1 + (size_t)chain * (nc + 1) * HD * HD, *s2p = HAS_S ? st2 + (size_t)chain * (nc + 1) * HD * HD : nullptr;
+    const size_t own = (size_t)(r0 + m) * HD + col;   // this lane's rows m .. m + 3 of the block, column col
+    f32x4 x1 = {0.f, 0.f, 0.f, 0.f}, x2 = x1;
+    auto leave = [&](int buf, size_t slot) {   // for the next step's operands, and as a state
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            X[buf][0][(m + i) * LX + col] = x1[i];
+            X[buf][1][(m + i) * LX + col] = x2[i];
+            s1p[slot * HD * HD + own + i * HD] = x1[i];
+            if (HAS_S) s2p[slot * HD * HD + own + i * HD] = x2[i];
         }
-        X1[rr * LDM + cc] = x1; X2[rr * LDM + cc] = x2;
-        const size_t slot = FWD ? 0 : nc;
-        s1p[slot * HD * HD + (r0 + rr) * HD + cc] = x1;
-        if (s2p) s2p[slot * HD * HD + (r0 + rr) * HD + cc] = x2;
+    };
+    if (FWD) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            x1[i] = init1[(size_t)chain * HD * HD + own + i * HD];
+            if (HAS_S) x2[i] = init2[(size_t)chain * HD * HD + own + i * HD];
+        }
     }
-    // Operands of step+1 (two 64x64 matrices, this wave's strip of the additive term, the two
-    // scalars) are fetched into registers while step runs, so a step costs no HBM round trip.
-    Tile<float> ta, tb;
-    Strip cnext = zero_strip(), cadd;
-    float scn = 0.f, s1, s2;   // lanes 4 j + 1, 2 of scn: the two scalars of the next step
-    auto prefetch = [&](int step) {
+    leave(0, FWD ? 0 : nc);
+    struct Inputs { f32x4 ta[4], tb[4], c1, c2; float scalars; } in[2];
+    auto prefetch = [&](int step, Inputs &n) __attribute__((always_inline)) {
         const int ci = FWD ? step : nc - 1 - step;
         const float *lc = loc + ((size_t)chain * nc + ci) * kLocMats * HD * HD;
-        const float *sc = locs + ((size_t)chain * nc + ci) * 4;
-        fetch(ta, lc, 64);
-        fetch(tb, lc + HD * HD, 64);
-        // a vector load (lane-dependent address) on purpose: a scalar load would share a counter with the LDS reads of
-        // the step's product, which would then wait for it to come back from memory
-        scn = sc[threadIdx.x & 3];
-        const float *Cm = lc + (FWD ? 2 + which : (which ? 3 : 2)) * HD * HD;
-        for_c(cnext, [&](int r, int c, float &x) { x = Cm[(r0 + m0 + r) * HD + n0 + c]; });
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+            n.ta[g] = *reinterpret_cast<const f32x4 *>(lc + ((ct * 4 + g) * 64 + l) * 4);
+            n.tb[g] = *reinterpret_cast<const f32x4 *>(lc + HD * HD + ((ct * 4 + g) * 64 + l) * 4);
+        }
+        n.c1 = *reinterpret_cast<const f32x4 *>(lc + 2 * HD * HD + ((r0 / 16 * 4 + ct) * 64 + l) * 4);
+        n.c2 = *reinterpret_cast<const f32x4 *>(lc + 3 * HD * HD + ((r0 / 16 * 4 + ct) * 64 + l) * 4);
+        // a vector load (lane-dependent address) on purpose: a scalar load would share a counter with the LDS reads
+        n.scalars = locs[((size_t)chain * nc + ci) * 4 + (threadIdx.x & 3)];
     };
-    prefetch(0);
-    for (int step = 0; step < nc; step++) {
-        const int ci = FWD ? step : nc - 1 - step;
-        __syncthreads();  // previous step's readers of Ta/Tb and writers of X1/X2 are done
-        commit(Ta, ta);
-        commit(Tb, tb);
-        s1 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, scn), 1));
-        s2 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, scn), 2));
-        cadd = cnext;
-        __syncthreads();
-        if (step + 1 < nc) prefetch(step + 1);
-        Strip acc = zero_strip(), out = zero_strip();
-        const float *T = which ? Tb : Ta;
-        const float *Xs = (FWD || !which) ? X1 : X2;
-        mma(acc, [&](int m, int kk) { return Xs[(m0 + m) * LDM + kk]; },
-            [&](int kk, int n) { return T[kk * LDM + n0 + n]; });
+    auto take = [&](int step, Inputs &n, int buf) __attribute__((always_inline)) {
+        lds_barrier();   // the buffer is complete; the other one's readers are past their products
+        f32x4 a1[4], a2[4], p1 = {0.f, 0.f, 0.f, 0.f}, p2 = p1;
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+            a1[g] = *reinterpret_cast<const f32x4 *>(&X[buf][0][r * LX + kb + 4 * g]);
+            a2[g] = FWD ? a1[g] : *reinterpret_cast<const f32x4 *>(&X[buf][1][r * LX + kb + 4 * g]);
+        }
+#pragma unroll
+        for (int k = 0; k < 16; k++) {
+            p1 = __builtin_amdgcn_mfma_f32_16x16x4f32(a1[k >> 2][k & 3], n.ta[k >> 2][k & 3], p1, 0, 0, 0);
+            p2 = __builtin_amdgcn_mfma_f32_16x16x4f32(a2[k >> 2][k & 3], n.tb[k >> 2][k & 3], p2, 0, 0, 0);
+        }
+        const float s1 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, n.scalars), 1));
+        const float s2 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, n.scalars), 2));
         if (FWD) {
-            const float sx = which ? s2 : s1;
-            for_c(out, [&](int r, int c, float &x) { x = sx * X2[(m0 + r) * LDM + n0 + c]; });
 #pragma unroll
-            for (int i = 0; i < 4; i++) { out.t[0][i] += acc.t[0][i] + cadd.t[0][i]; out.t[1][i] += acc.t[1][i] + cadd.t[1][i]; }
-        } else if (which) {
-            for_c(acc, [&](int r, int c, float &x) { part[pidx][r * 33 + c] = x; });
-            for_c(out, [&](int r, int c, float &x) {
-                x = s1 * X1[(m0 + r) * LDM + n0 + c] + s2 * X2[(m0 + r) * LDM + n0 + c];
-            });
+            for (int i = 0; i < 4; i++) {
+                x1[i] = s1 * x2[i] + (p1[i] + n.c1[i]);
+                x2[i] = s2 * x2[i] + (p2[i] + n.c2[i]);
+            }
+        } else {
 #pragma unroll
-            for (int i = 0; i < 4; i++) { out.t[0][i] += cadd.t[0][i]; out.t[1][i] += cadd.t[1][i]; }
+            for (int i = 0; i < 4; i++) {
+                const float y = s1 * x1[i] + s2 * x2[i] + n.c2[i];
+                x1[i] = p2[i] + (p1[i] + n.c1[i]);
+                x2[i] = y;
+            }
         }
-        __syncthreads();  // all reads of the old X1/X2 are done; partial products are in LDS
-        if (!FWD && !which) {
-            for_c(out, [&](int r, int c, float &x) { x = part[pidx][r * 33 + c]; });
-#pragma unroll
-            for (int i = 0; i < 4; i++) { out.t[0][i] += acc.t[0][i] + cadd.t[0][i]; out.t[1][i] += acc.t[1][i] + cadd.t[1][i]; }
-        }
-        float *Xd = which ? X2 : X1;
-        float *gd = which ? s2p : s1p;
-        const size_t slot = FWD ? ci + 1 : ci;
-        for_c(out, [&](int r, int c, float &x) {
-            Xd[(m0 + r) * LDM + n0 + c] = x;
-            if (gd) gd[slot * HD * HD + (r0 + m0 + r) * HD + n0 + c] = x;
-        });
+        leave(buf ^ 1, FWD ? step + 1 : nc - 1 - step);
+        prefetch(min(step + 2, nc - 1), n);
+    };
+    prefetch(0, in[0]);
+    prefetch(min(1, nc - 1), in[1]);
+    int step = 0;
+    for (; step + 2 <= nc; step += 2) {
+        take(step, in[0], 0);
+        take(step + 1, in[1], 1);
     }
+    if (step < nc) take(step, in[0], 0);
 }
 
 // ── pass 3 (forward): outputs of one chunk ──────────────────────────────────
@@ -354,10 +372,9 @@ __global__ __launch_bounds__(kThr) void cw_local_bwd_kernel(const TIn *__restric
         const float *wv = o ? wS : wM;
         Strip acc = zero_strip();
         mma(acc, [&](int m, int kk) { return Ks[kk * LDM + m0 + m] * wv[kk]; }, bK);
-        for_c(acc, [&](int r, int c, float &x) {
-            const int row = m0 + r, col = n0 + c;
-            out[(size_t)o * HD * HD + row * HD + col] = x + ((o == 0 && row == col) ? aL : 0.f);
-        });
+        for_c(acc, [&](int r, int c, float &x) { x += (o == 0 && m0 + r == n0 + c) ? aL : 0.f; });
+#pragma unroll
+        for (int t = 0; t < 2; t++) store_operand_tile(out + (size_t)o * HD * HD, acc.t[t], m0 / 16, n0 / 16 + t, threadIdx.x & 63);
     }
     {   // Cc <- c[t][j] * (q_t . k_j), in place (own strip only)
         Strip p = zero_strip();
@@ -380,8 +397,11 @@ __global__ __launch_bounds__(kThr) void cw_local_bwd_kernel(const TIn *__restric
     if (has_s)
         mma(gs, [&](int m, int kk) { return cf.beta[kk] * Ds[kk * LDM + m0 + m]; },
             [&](int kk, int n) { return Qs[kk * LDM + n0 + n]; });
-    for_c(g0, [&](int r, int c, float &x) { out[(size_t)2 * HD * HD + (m0 + r) * HD + n0 + c] = x; });
-    for_c(gs, [&](int r, int c, float &x) { out[(size_t)3 * HD * HD + (m0 + r) * HD + n0 + c] = x; });
+#pragma unroll
+    for (int t = 0; t < 2; t++) {
+        store_acc_tile(out + (size_t)2 * HD * HD, g0.t[t], m0 / 16, n0 / 16 + t, threadIdx.x & 63);
+        store_acc_tile(out + (size_t)3 * HD * HD, gs.t[t], m0 / 16, n0 / 16 + t, threadIdx.x & 63);
+    }
     __syncthreads();   // LDS is rewritten by the next task
     }
 }
@@ -667,8 +687,8 @@ void forward_mm(const char *fn, const TIn *k, const TIn *v, const TIn *q, const 
     hipLaunchKernelGGL((cw_local_fwd_kernel<TIn>), dim3(batch * nc), dim3(kThr), 0, stream(), k, v, alpha, theta,
                        eta, sc.loc, sc.locs, seq_len, chunk_size, nc, (int)has_s);
     check_launch("cw_local_fwd_kernel");
-    hipLaunchKernelGGL((cw_scan_kernel<true>), dim3(batch * 2), dim3(kThr), 0, stream(), m_initial, s_initial,
-                       sc.loc, sc.locs, m_states, has_s ? s_states : nullptr, nc, (int)has_s);
+    hipLaunchKernelGGL((has_s ? cw_scan_kernel<true, true> : cw_scan_kernel<true, false>), dim3(batch * 4), dim3(256), 0, stream(),
+                       m_initial, s_initial, sc.loc, sc.locs, m_states, s_states, nc, batch);
     check_launch("cw_scan_kernel");
     if (tracks)
         hipLaunchKernelGGL((cw_out_fwd_kernel<TIn, true>), dim3(persistent_grid(batch * nc)), dim3(kThr), kOutFwdLds,
@@ -744,8 +764,8 @@ bool backward_mm(const char *fn, const TIn *k, const TIn *v, const TIn *q, const
                            stream(), k, q, d_y, alpha, theta, eta, sc.loc, sc.locs, seq_len, chunk_size, nc,
                            (int)has_s, batch * nc);
         check_launch("cw_local_bwd_kernel");
-        hipLaunchKernelGGL((cw_scan_kernel<false>), dim3(batch * 2), dim3(kThr), 0, stream(), nullptr, nullptr,
-                           sc.loc, sc.locs, dm_states, ds_states, nc, (int)has_s);
+        hipLaunchKernelGGL((has_s ? cw_scan_kernel<false, true> : cw_scan_kernel<false, false>), dim3(batch * 4), dim3(256), 0, stream(),
+                           nullptr, nullptr, sc.loc, sc.locs, dm_states, ds_states, nc, batch);
         check_launch("cw_scan_kernel");
         KernelTimer kt("cw_grads_bwd_kernel");
         if (guard)
