@@ -102,6 +102,17 @@ __device__ __forceinline__ float group_allreduce(float x) {
     return x;
 }
 
+// Two such sums, step by step side by side: each fills the other's wait states.
+template <int G>
+__device__ __forceinline__ void group_allreduce2(float &x, float &y) {
+    if constexpr (G >= 2) { x += dpp_mov<DPP_XOR1>(x); y += dpp_mov<DPP_XOR1>(y); }
+    if constexpr (G >= 4) { x += dpp_mov<DPP_XOR2>(x); y += dpp_mov<DPP_XOR2>(y); }
+    if constexpr (G >= 8) { x += dpp_mov<DPP_HALF_MIRROR>(x); y += dpp_mov<DPP_HALF_MIRROR>(y); }
+    if constexpr (G >= 16) { x += dpp_mov<DPP_MIRROR>(x); y += dpp_mov<DPP_MIRROR>(y); }
+    if constexpr (G >= 32) { x = swapadd16(x, x); y = swapadd16(y, y); }
+    if constexpr (G >= 64) { x = swapadd32(x, x); y = swapadd32(y, y); }
+}
+
 // x + (value of x in lane ^ MASK), for values that differ between lanes.
 template <int MASK>
 __device__ __forceinline__ float xor_add(float x) {

@@ -161,20 +161,26 @@ __global__ __launch_bounds__(kThreads) void rule_fwd_kernel(FwdArgs a) {
         // of later tokens overlap the dependent chain of earlier ones.
         auto run_tile = [&](auto fast_c) {
             constexpr bool FAST = decltype(fast_c)::value;
+            // p = M k of the token at hand.  The next token's is summed over the row's lanes together with this token's y: both
+            // wait on M, and a sum by itself spends half of its time on the wait states between its DPP adds (64 chains x 2048
+            // tokens of 64 with momentum 270 -> 251 us).  Bound by the instructions of a token, about 45 at 4 clocks and more
+            // each: two columns a lane and twice the waves took 381 us.
+            float4 kk = *reinterpret_cast<const float4 *>(&sk[buf][cb * 4]);
+            float p[RPL];
+#pragma unroll
+            for (int r = 0; r < RPL; r++) p[r] = group_allreduce<LPR>(dot4(FROZEN ? M0[r] : M[r], kk));
 #pragma unroll
             for (int tl = 0; tl < TB; tl++) {
                 if (!FAST && tl >= tn) break;
                 const int t = t0 + tl;
-                const float4 kk = *reinterpret_cast<const float4 *>(&sk[buf][tl * D + cb * 4]);
                 const float4 qq = STORE != STORE_LAST ? *reinterpret_cast<const float4 *>(&sq[buf][tl * D + cb * 4]) : f4_zero();
                 const float al = sg[buf][tl], th = sg[buf][TB + tl], et = sg[buf][2 * TB + tl];
                 const float ret = 1.f - al;
                 float e[RPL];
 #pragma unroll
                 for (int r = 0; r < RPL; r++) {
-                    float p = group_allreduce<LPR>(dot4(FROZEN ? M0[r] : M[r], kk));
                     float vv = sv[buf][tl * D + (valid[r] ? row0 + r : 0)];
-                    e[r] = valid[r] ? p - vv : 0.f;
+                    e[r] = valid[r] ? p[r] - vv : 0.f;
                 }
                 if (COUPLED && clip_on) {
                     float sq_sum = 0.f;
@@ -244,11 +250,19 @@ __global__ __launch_bounds__(kThreads) void rule_fwd_kernel(FwdArgs a) {
                         }
                     }
                 }
+                if (tl + 1 < TB) kk = *reinterpret_cast<const float4 *>(&sk[buf][(tl + 1) * D + cb * 4]);
 #pragma unroll
-                for (int r = 0; r < (STORE != STORE_LAST ? RPL : 0); r++) {
-                    float yy = group_allreduce<LPR>(dot4(M[r], qq));
+                for (int r = 0; r < RPL; r++) {
+                    float yy = STORE != STORE_LAST ? dot4(M[r], qq) : 0.f;
+                    if (tl + 1 < TB) {
+                        p[r] = dot4(FROZEN ? M0[r] : M[r], kk);
+                        if constexpr (STORE != STORE_LAST) group_allreduce2<LPR>(p[r], yy);
+                        else p[r] = group_allreduce<LPR>(p[r]);
+                    } else if constexpr (STORE != STORE_LAST) {
+                        yy = group_allreduce<LPR>(yy);
+                    }
                     // all LPR lanes of the row hold yy: same-value store, no divergence
-                    sy[buf][tl * ROWS_WG + row_local + r] = yy;
+                    if constexpr (STORE != STORE_LAST) sy[buf][tl * ROWS_WG + row_local + r] = yy;
                 }
             }
         };
