@@ -12,7 +12,7 @@
 //   3. decode_output_kernel    attention slices merged, levels combined, sigmoid gate, output projection
 //   4. decode_logits_kernel    the unembedding, written to the workspace and to host-visible memory
 // Measured on one MI355X at d = 512, four levels of which one is active, window 512, vocabulary 32 000: 0.50 -> 0.058 ms
-// a token with the host side, of which 5.2 + 4.6 + 7.0 + 12.1 us in the four kernels (the last one moves 65 MB at
+// a token with the host side, of which 4.9 + 4.4 + 5.3 + 12.1 us in the four kernels (the last one moves 65 MB at
 // 5.4 TB/s) and about 11 us before the first one starts and after the last one has ended.
 #include <float.h>
 #include <hip/hip_runtime.h>
@@ -285,8 +285,8 @@ __global__ __launch_bounds__(kDecThr) void decode_heads_kernel(DecArgs a) {
 
 // Eight rows of the output projection per workgroup; every workgroup forms the whole gated vector for itself.  The
 // chain of loads is what takes the time, so nothing is loaded behind a value it does not need: the weights of the first
-// 1024 columns are requested at the top, the slices' statistics go through LDS, a thread's slices and levels are read
-// in batches of four (10.0 -> 7.0 us at d = 512, 5 slices, 4 levels).
+// 1024 columns, the slices' statistics (one thread each, then shared in LDS) and the levels and slices of a thread's first
+// two columns are all requested at the top (10.0 -> 7.0 -> 5.3 us at d = 512, 5 slices, 4 levels).
 __global__ __launch_bounds__(kDecThr) void decode_output_kernel(DecArgs a) {
     extern __shared__ float smem[];
     float *gated = smem, *wgt = smem + a.d;   // [d], [slices][heads]: a slice's weight in the merged softmax
@@ -301,8 +301,36 @@ __global__ __launch_bounds__(kDecThr) void decode_output_kernel(DecArgs a) {
         p0[j] = w0[i];
         p1[j] = w1[i];
     }
+    constexpr int NL = 4, NS = 8;
+    float ty[2][NL], to[2][NS];
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
+        const int i = min(tid + c * kDecThr, d - 1);
+#pragma unroll
+        for (int j = 0; j < NL; j++) ty[c][j] = a.lv[min(j, a.levels - 1)].y[i];
+#pragma unroll
+        for (int j = 0; j < NS; j++) to[c][j] = a.part_o[(size_t)min(j, a.slices - 1) * d + i];
+    }
     const float scale = a.levels > 2 ? 1.f / sqrtf((float)a.levels) : 1.f;
-    for (int h = tid; h < a.nh; h += kDecThr) {
+    const int stats = a.slices * a.nh;
+    if (stats <= min(kDecThr, d)) {   // one of them a thread; their sums wait where gated will stand
+        float2 ml = make_float2(0.f, 0.f);
+        if (tid < stats) {
+            ml = *reinterpret_cast<const float2 *>(a.part_ml + (size_t)tid * 2);
+            wgt[tid] = ml.x;
+            gated[tid] = ml.y;
+        }
+        __syncthreads();
+        float weight = 0.f;
+        if (tid < stats) {
+            float mx = -FLT_MAX, sum = 0.f;
+            for (int i = tid % a.nh; i < stats; i += a.nh) mx = fmaxf(mx, wgt[i]);
+            for (int i = tid % a.nh; i < stats; i += a.nh) sum += expf(wgt[i] - mx) * gated[i];
+            weight = expf(ml.x - mx) * (1.f / sum);
+        }
+        __syncthreads();
+        if (tid < stats) wgt[tid] = weight;
+    } else for (int h = tid; h < a.nh; h += kDecThr) {
         float mx = -FLT_MAX, sum = 0.f;
         for (int s = 0; s < a.slices; s++) mx = fmaxf(mx, a.part_ml[((size_t)s * a.nh + h) * 2]);
         for (int s = 0; s < a.slices; s++) {
@@ -315,21 +343,21 @@ __global__ __launch_bounds__(kDecThr) void decode_output_kernel(DecArgs a) {
         for (int s = 0; s < a.slices; s++) wgt[s * a.nh + h] *= inv;
     }
     __syncthreads();
-    for (int i = tid; i < d; i += kDecThr) {
+    auto column = [&](int i, const float(&t0)[NL], const float(&o0)[NS]) {
         const int h = i / a.hd;
         float o = 0.f, y = 0.f;
-        for (int l = 0; l < a.levels; l += 4) {
-            float t[4];
+        for (int l = 0; l < a.levels; l += NL) {
+            float t[NL];
 #pragma unroll
-            for (int j = 0; j < 4; j++) t[j] = l + j < a.levels ? a.lv[l + j].y[i] : 0.f;
+            for (int j = 0; j < NL; j++) t[j] = l + j < a.levels ? l ? a.lv[l + j].y[i] : t0[j] : 0.f;
             y += (t[0] + t[1]) + (t[2] + t[3]);
         }
-        for (int s = 0; s < a.slices; s += 4) {
-            float t[4];
+        for (int s = 0; s < a.slices; s += NS) {
+            float t[NS];
 #pragma unroll
-            for (int j = 0; j < 4; j++) t[j] = a.part_o[(size_t)min(s + j, a.slices - 1) * d + i];
+            for (int j = 0; j < NS; j++) t[j] = s ? a.part_o[(size_t)min(s + j, a.slices - 1) * d + i] : o0[j];
 #pragma unroll
-            for (int j = 0; j < 4; j++) o += s + j < a.slices ? wgt[(s + j) * a.nh + h] * t[j] : 0.f;
+            for (int j = 0; j < NS; j++) o += s + j < a.slices ? wgt[(s + j) * a.nh + h] * t[j] : 0.f;
         }
         const uint16_t o16 = f32_to_bf16_rne(o);
         y *= scale;
@@ -342,6 +370,17 @@ __global__ __launch_bounds__(kDecThr) void decode_output_kernel(DecArgs a) {
             a.gate[i] = g;
             a.gated[i] = at * g;
         }
+    };
+#pragma unroll
+    for (int c = 0; c < 2; c++)
+        if (tid + c * kDecThr < d) column(tid + c * kDecThr, ty[c], to[c]);
+    for (int i = tid + 2 * kDecThr; i < d; i += kDecThr) {
+        float t[NL], o[NS];
+#pragma unroll
+        for (int j = 0; j < NL; j++) t[j] = a.lv[min(j, a.levels - 1)].y[i];
+#pragma unroll
+        for (int j = 0; j < NS; j++) o[j] = a.part_o[(size_t)min(j, a.slices - 1) * d + i];
+        column(i, t, o);
     }
     __syncthreads();
     float acc0 = 0.f, acc1 = 0.f;

@@ -303,3 +303,39 @@ def test_non_finite_cache_entries(monkeypatch):
         assert np.array_equal(np.isfinite(a), np.isfinite(b)), place
         ok = np.isfinite(b)
         assert np.abs(a[ok] - b[ok]).max(initial=0) <= 2e-2 * np.abs(b[ok]).max(initial=1), place
+
+
+@pytest.mark.parametrize("nh,hd,levels,keys", [
+    (2, 32, 5, 9 * 128 - 3),     # more levels and slices than the first batch of loads holds
+    (16, 32, 1, 17 * 128 + 1),   # more statistics than threads
+    (1, 32, 4, 33 * 128),        # more statistics than columns
+    (10, 64, 8, 100)])           # more columns than two a thread
+def test_output_merge_at_its_edges(nh, hd, levels, keys):
+    d, v = nh * hd, 20
+    g = torch.Generator(device="cuda").manual_seed(keys)
+    r = lambda *sh: torch.randn(*sh, generator=g, device="cuda") * 0.1
+    lp = [MemoryLevelParams(r(d, d), r(d, d), r(d, d), r(2 * d), r(1), r(2 * d), r(1), r(2 * d), r(1)) for _ in range(levels)]
+    gp = SG.GpuMAGParams(r(v, d), r(d, d), r(d, d), r(d, d), r(d, d), r(d, v), lp)
+    cfg = SG.ServeConfig(d, v, nh, hd, keys, keys - 1, [LevelConfig("delta", nh, hd) for _ in range(levels)], decode_tokens=2)
+    kv, ws = SG.GpuKVCache(keys + 1, d, 1), SG.DecodeWorkspace(d, v)
+    kv.k_cache_bf16.copy_(r(keys + 1, d) * 30)
+    kv.v_cache_bf16.copy_(r(keys + 1, d) * 10)
+    kv.len = keys - 1
+    ctx = ContextState([r(nh, hd * hd) for _ in range(levels)])
+    out = SG.gpu_single_token_forward(gp, cfg, 3, Pulse(0, [False] * levels), ctx, kv, ws)
+    assert list(ws.plans.values())[0][1] is not None
+    f64 = lambda t: host(t.float()).astype(np.float64)
+    q, kc, vc = (f64(t).reshape(-1, nh, hd) for t in (ws.q_bf16, kv.k_cache_bf16[:keys], kv.v_cache_bf16[:keys]))
+    w = np.einsum("hc,thc->ht", q[0], kc) / np.sqrt(hd)
+    w = np.exp(w - w.max(1, keepdims=True))
+    attn = np.einsum("ht,thc->hc", w / w.sum(1, keepdims=True), vc).reshape(-1)
+    got = f64(ws.attn_out)[0]
+    assert np.abs(got - attn).max() <= 2 ** -8 * np.abs(attn).max()   # rounded to bf16 once
+    x = f64(gp.w_embed)[3]
+    y = sum(np.einsum("hij,hj->hi", f64(m).reshape(nh, hd, hd), (f64(p.w_q) @ x).reshape(nh, hd))
+            for m, p in zip(ctx.memory, lp)).reshape(-1) * (levels ** -0.5 if levels > 2 else 1.0)
+    scale = sum(np.abs(f64(m)).max() for m in ctx.memory) * np.abs(x).max() * d * hd * 0.4
+    assert np.abs(f64(ws.y_combined)[0] - y).max() <= 2e-7 * scale   # float sums of d and of hd products
+    gated = got / (1 + np.exp(-f64(ws.y_combined)[0]))
+    assert_close("gated", f64(ws.gated_out)[0], gated, 1e-6)
+    assert_close("logits", out, (f64(gp.w_o) @ gated) @ f64(gp.w_unembed), 1e-5)
