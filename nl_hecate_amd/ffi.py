@@ -6,12 +6,14 @@ a Rust/C caller would bind.  There is no CPU fallback: if the HIP library has
 not been built, loading raises.
 """
 import ctypes
+import importlib.util
 import os
 import re
 
 _PKG = os.path.dirname(os.path.abspath(__file__))
 HEADER = os.path.join(os.path.dirname(_PKG), "include", "nl_hecate_ffi.h")
 LIB_PATH = os.path.join(_PKG, "lib", "libnl_hecate_rocm.so")
+KEY_PATH = os.path.join(_PKG, "lib", "plan_key.so")
 
 _CTYPES = {
     "int": ctypes.c_int,
@@ -79,3 +81,16 @@ class _Lib:
 
 
 lib = _Lib()
+
+
+def tensor_key(tensors):
+    """Address, type, device, sizes and strides of every tensor as one bytes object (csrc/plan_key.cpp).  The first call
+    puts the compiled function in this one's place."""
+    global tensor_key
+    if not os.path.exists(KEY_PATH):
+        raise RuntimeError(f"{KEY_PATH} is missing: build it with `make -C nl_hecate_amd/csrc`.")
+    spec = importlib.util.spec_from_file_location("plan_key", KEY_PATH)
+    module = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(module)
+    tensor_key = module.tensor_key
+    return tensor_key(tensors)

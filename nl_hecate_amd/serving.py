@@ -19,6 +19,7 @@ import numpy as np
 import torch
 
 from . import dispatch as D
+from . import ffi
 from .cms import ContextState, Pulse
 from .ffi import lib
 from .mag_layer import MemoryLevelParams
@@ -178,7 +179,9 @@ def _keys_fit(cfg, pos):
 
 
 # level_rule of decode_token_rocm; a Titans level starts every call with zero momentum, so its one-token step is Delta's
-_DTYPE = operator.attrgetter("dtype")
+_LEVEL_TENSORS = operator.attrgetter("w_k", "w_v", "w_q", "w_alpha", "b_alpha", "w_theta", "b_theta")
+_LEVEL_OPTIONS = operator.attrgetter("memory_rule", "memory_layers", "num_heads", "head_dim", "alpha_floor", "alpha_ceil",
+                                     "theta_floor", "theta_ceil", "error_clip", "m_norm_max")
 _DECODE_RULE = {"hebbian": 0, "delta": 1, "titans": 1, "dgd": 2}
 
 
@@ -227,7 +230,7 @@ def _decode_plan(params, cfg, active, context, kv_cache, ws, tensors):
     written = [t.data_ptr() for t in ws.written()]
     tail = (kv_cache.k_cache_bf16.data_ptr(), kv_cache.v_cache_bf16.data_ptr(), work.data_ptr(), (ctypes.c_void_p * 7)(*written[:7]),
             written[7], ws.logits_host.data_ptr())
-    return weights, level_args, tail
+    return ptrs[0], weights, level_args, tail
 
 
 def _decode_in_one_call(params, cfg, token_id, pulse, context, kv_cache, ws):
@@ -240,23 +243,18 @@ def _decode_in_one_call(params, cfg, token_id, pulse, context, kv_cache, ws):
     levels, lcfgs = params.levels, cfg.levels
     tensors = [params.w_embed, params.w_q, params.w_k, params.w_v, params.w_o, params.w_unembed, kv_cache.k_cache_bf16,
                kv_cache.v_cache_bf16]
-    key = [cfg.d_model, cfg.num_heads, cfg.head_dim, cfg.vocab_size, cfg.window_size, cfg.n_persistent]
+    active = tuple(map(bool, pulse.active_levels[:k]))
+    options = [cfg.d_model, cfg.num_heads, cfg.head_dim, cfg.vocab_size, cfg.window_size, cfg.n_persistent, kv_cache.d,
+               kv_cache.max_len]
     for lv in range(k):
-        lp, lc = levels[lv], lcfgs[lv]
+        lp = levels[lv]
         if not hasattr(lp, "w_alpha"):
             return None
-        tensors += (lp.w_k, lp.w_v, lp.w_q, lp.w_alpha, lp.b_alpha, lp.w_theta, lp.b_theta, context.memory[lv])
-        key += (lc.memory_rule, lc.memory_layers, lc.num_heads, lc.head_dim, lc.alpha_floor, lc.alpha_ceil, lc.theta_floor,
-                lc.theta_ceil, lc.error_clip, lc.m_norm_max)
-    active = tuple(map(bool, pulse.active_levels[:k]))
-    key += map(torch.Tensor.data_ptr, tensors)
-    key += map(torch.Tensor.stride, tensors)   # a tensor can be transposed or resized where it stands
-    key += map(torch.Tensor.size, tensors)
-    key += map(_DTYPE, tensors)
-    written = ws.written()
-    key += map(torch.Tensor.data_ptr, written)
-    key += map(torch.Tensor.numel, written)
-    key += (kv_cache.d, kv_cache.max_len, kv_cache._scratch_k.numel(), ws.logits_host.numel(), ws.logits_host.data_ptr())
+        tensors += _LEVEL_TENSORS(lp)
+        tensors.append(context.memory[lv])
+        options += _LEVEL_OPTIONS(lcfgs[lv])
+    # a tensor can be transposed or resized where it stands: sizes and strides are read anew as well as the address
+    key = (options, ffi.tensor_key([*tensors, *ws.written(), kv_cache._scratch_k, ws.logits_host]))
     made_for, plan = ws.plans.get(active, (None, None))
     if made_for != key:
         plan = _decode_plan(params, cfg, active, context, kv_cache, ws, tensors)
@@ -265,8 +263,8 @@ def _decode_in_one_call(params, cfg, token_id, pulse, context, kv_cache, ws):
         ws.plans[active] = (key, plan)
     if plan is None:
         return None
-    weights, level_args, tail = plan
-    rc = lib.decode_token_rocm(key[6 + 10 * k] + 4 * cfg.d_model * token_id, *weights, *level_args, k, cfg.d_model,
+    rows, weights, level_args, tail = plan
+    rc = lib.decode_token_rocm(rows + 4 * cfg.d_model * token_id, *weights, *level_args, k, cfg.d_model,
                                cfg.num_heads, cfg.vocab_size, cfg.window_size, cfg.n_persistent, kv_cache.len, *tail)
     if rc:
         raise RuntimeError(f"decode_token_rocm failed ({rc})")

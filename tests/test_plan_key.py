@@ -1,0 +1,39 @@
+"""The key that an argument block of tensor addresses is kept under: whatever a tensor can change where it stands shows."""
+import pytest
+import torch
+
+from nl_hecate_amd import ffi
+
+
+@pytest.mark.parametrize("change", ["nothing", "values", "transpose", "shape", "resize", "data", "type", "view"])
+def test_key_of_a_tensor_that_changed_where_it_stands(change):
+    t, other = torch.zeros(6, 6), torch.zeros(2, 3, dtype=torch.bfloat16)
+    before = ffi.tensor_key([t, other])
+    assert isinstance(before, bytes) and before == ffi.tensor_key((t, other))
+    keep = t.data
+    if change == "values":
+        t.add_(1)
+    elif change == "transpose":
+        t.t_()
+    elif change == "shape":
+        t.data = keep.view(36)
+    elif change == "resize":
+        t.resize_(6, 5)
+    elif change == "data":
+        t.data = torch.zeros(6, 6)
+    elif change == "type":
+        t.data = keep.view(torch.int32)
+    elif change == "view":
+        t = t[1:]
+    assert (before == ffi.tensor_key([t, other])) == (change in ("nothing", "values"))
+
+
+def test_key_of_what_has_no_address():
+    assert ffi.tensor_key([]) == b""
+    for bad, error in (([None], TypeError), ([1.0], TypeError), (3, TypeError),
+                       ([torch.zeros(2, device="meta"), "w"], TypeError)):
+        with pytest.raises(error):
+            ffi.tensor_key(bad)
+    sparse = torch.eye(3).to_sparse()
+    with pytest.raises(RuntimeError):
+        ffi.tensor_key([sparse])
