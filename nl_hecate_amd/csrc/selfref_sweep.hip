@@ -12,10 +12,16 @@
 // so that a token takes one exchange (dg_t), one product with a matrix and the dots of dg_t with the tile's u_s.
 //
 // 64 chains of 2048 tokens, head size 64, chunks of 64: preparation 0.36 ms (one workgroup per compute unit for its LDS;
-// 0.10 are matrix instructions), sweep 1.60 ms: 760 clocks a token (115 instructions of one wave per SIMD and the
-// exchange), 9.5 k clocks a tile and 34 k a chunk boundary, half of each matrix instructions.  The sweep that formed w, z,
-// dk, dv and the update of dG token by token took 3.16 ms behind 0.23 ms of preparation; without self-generated values it
-// is still the one (selfref.hip), since there dh_t comes back as a second vector.
+// 0.10 are matrix instructions), sweep 1.45 ms: 850 clocks a token (115 instructions of one wave per SIMD and the exchange),
+// 7 k clocks a tile and 26 k a chunk boundary, most of those matrix instructions.  The sweep that formed w, z, dk, dv and the
+// update of dG token by token took 3.16 ms behind 0.23 ms of preparation; without self-generated values it is still the one
+// (selfref.hip), since there dh_t comes back as a second vector.
+//
+// The sweep has two waves for each 16 rows.  The first half does what the tokens wait for, and across a chunk boundary the
+// gradients of F_q and F_mem; the second half those of F_k and F_v, at the boundary and from every tile's dk and dv, stores
+// dg, and brings the next boundary's matrices into LDS while the first is among the tokens.  One wave a SIMD did all of it
+// in 1.60 ms (9.5 k clocks a tile, 34 k a boundary, half of either with the matrix cores idle; 774 a token: the second wave
+// costs the tokens some issue slots and the registers beyond 256).
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
@@ -439,13 +445,78 @@ __device__ __forceinline__ void across_rows3(float &a, float &b, float &c) {
     a += a1; b += b1; c += c1;
 }
 
-// One workgroup per chain, a wave per 16 rows.  Lane (ml, kg) = (lane % 16, lane / 16) holds of every matrix row ml of
+// dynamic LDS of the sweep: a tile's arrays; G_L^T, two F, dF' of the second half; dF of the first half; dk and dv
+constexpr int sweep_tile_floats(int d) { return 8 * kTB * (d + 4); }
+constexpr int sweep_lds_floats(int d) { return sweep_tile_floats(d) + 6 * d * (d + 4) + d / 16 * 8 * 64; }
+
+// What a chunk's tokens add to dF whatever the sweep finds: the lane's part of a wave's 16 rows.
+template <int D>
+__device__ __forceinline__ void token_sums(f32x4 (&sums)[D / 16], const float *outer, int tid) {
+    constexpr int JT = D / 16;
+#pragma unroll
+    for (int jt = 0; jt < JT; jt++)
+        sums[jt] = *reinterpret_cast<const f32x4 *>(outer + ((size_t)((tid >> 6) * JT + jt) * 64 + (tid & 63)) * 4);
+}
+
+// A wave's 16 rows of a matrix in LDS from its accumulators.
+template <int D>
+__device__ __forceinline__ void put_rows(float *m, const f32x4 (&x)[D / 16], int tid) {
+    const int lane = tid & 63, row = 16 * (tid >> 6) + 4 * (lane >> 4);
+#pragma unroll
+    for (int jt = 0; jt < D / 16; jt++) {
+#pragma unroll
+        for (int v = 0; v < 4; v++) m[(row + v) * (D + 4) + 16 * jt + (lane & 15)] = x[jt][v];
+    }
+}
+
+// F_c of a chunk boundary, a workgroup half's part of each thread.
+template <int D>
+__device__ __forceinline__ void request_matrix(f32x4 (&m)[D / 16], const float *f, int tid) {
+#pragma unroll
+    for (int i = 0; i < D / 16; i++) m[i] = *reinterpret_cast<const f32x4 *>(f + (tid + i * 4 * D) * 4);
+}
+template <int D>
+__device__ __forceinline__ void stage_matrix(float *Fs, const f32x4 (&m)[D / 16], int tid) {
+#pragma unroll
+    for (int i = 0; i < D / 16; i++) {
+        const int e = tid + i * 4 * D;
+        *reinterpret_cast<f32x4 *>(Fs + (e / (D / 4)) * (D + 4) + (e % (D / 4)) * 4) = m[i];
+    }
+}
+
+// One memory across a chunk boundary: accG += F_c^T dF'_c, accN = dF'_c G_L^T.
+template <int D>
+__device__ __forceinline__ void boundary_products(const float *Fs, const float *Bm, const float *GLT, f32x4 (&accG)[D / 16],
+                                                  f32x4 (&accN)[D / 16], int tid) {
+    constexpr int KT = D / 16, JT = D / 16, LD = D + 4;
+    asm volatile("" : "+v"(tid));   // addresses made of it are not to live across the sweep
+    const int wave = tid >> 6, lane = tid & 63, ml = lane & 15, kg = lane >> 4, wr = 16 * wave;
+#pragma unroll
+    for (int jt = 0; jt < JT; jt++) accN[jt] = kZero;
+    // contraction in the order 16 c + 4 kg + v: rows 4 apart put the four kg of a read on different banks
+#pragma unroll
+    for (int c = 0; c < KT; c++) {
+        const f32x4 a2 = *reinterpret_cast<const f32x4 *>(Bm + (wr + ml) * LD + 16 * c + 4 * kg);  // dF'_c
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            const int k = 16 * c + 4 * kg + v;
+            const float a1 = Fs[k * LD + wr + ml];  // F_c^T
+#pragma unroll
+            for (int jt = 0; jt < JT; jt++) {
+                accG[jt] = mfma4(a1, Bm[k * LD + 16 * jt + ml], accG[jt]);
+                accN[jt] = mfma4(a2[v], GLT[k * LD + 16 * jt + ml], accN[jt]);
+            }
+        }
+    }
+}
+
+// One workgroup per chain, two waves per 16 rows (above).  Lane (ml, kg) = (lane % 16, lane / 16) holds of every matrix row ml of
 // the wave's rows, columns CP kg + i (CP = D / 4): operand and result of the tile products (the contraction index runs
 // over (i, kg)), and the coefficients of a product with a vector whose element CP kg + i is broadcast from lane i of
 // DPP row kg.  dG is kept a second time by columns (dGT).  Tokens of a tile are result rows in the order sigma, so that
 // lane kg owns the columns s = 4 v + kg of Y.
 template <int D>
-__global__ __launch_bounds__(4 * D) void selfref_bwd_sweep_kernel(
+__global__ __launch_bounds__(8 * D) void selfref_bwd_sweep_kernel(
     const float *__restrict__ emb, const float *__restrict__ k_cache, const float *__restrict__ v_cache,
     const float *__restrict__ frozen, const float *__restrict__ gl, const float *__restrict__ tok,
     const float *__restrict__ outer, const float *__restrict__ csv, float *__restrict__ d_emb,
@@ -453,8 +524,11 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_sweep_kernel(
     constexpr int CP = D / 4, KT = D / 16, JT = D / 16, NT = 4 * D, NW = D / 16, DD = D * D, V4 = D / 4, LD = D + 4;
     constexpr int TF = sweep_token_floats(D), TILE = kTB * LD;
     enum { A_K, A_U, A_X, A_DG0, A_FX, A_DG, A_W, A_Z, A_COUNT };
-    constexpr int RAW = A_COUNT * TILE > 3 * D * LD ? A_COUNT * TILE : 3 * D * LD;
-    __shared__ __align__(16) float raw[RAW];
+    static_assert(A_COUNT == 8);
+    extern __shared__ __align__(16) float raw[];
+    float *const GLT = raw + sweep_tile_floats(D), *const Fa = GLT + D * LD, *const Fb = Fa + D * LD, *const Bm = Fb + D * LD;
+    float *const kept = Bm + D * LD;                 // the gradients of F_q and F_mem between the boundaries
+    float *const dkv = kept + 2 * D * LD;            // dk, dv of a tile's tokens: [wave][v][2][lane]
     constexpr int LG = D + 16;                       // rows 4 v + kg of g fall on different banks for the four kg
     __shared__ __align__(16) float tg[kTB * LG];     // g
     __shared__ __align__(16) float gam[kTB * kTB];   // x_t . k_s, s in the order sigma
@@ -464,20 +538,121 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_sweep_kernel(
     __shared__ float sp[NW];
 #define T_(a, t, i) raw[(a) * TILE + (t) * LD + (i)]
 
-    const int tid = threadIdx.x, r = tid >> 2, cq = tid & 3, wave = tid >> 6, lane = tid & 63;
+    const bool second = __builtin_amdgcn_readfirstlane(threadIdx.x) >= NT;
+    const int tid = second ? threadIdx.x - NT : threadIdx.x, r = tid >> 2, cq = tid & 3, wave = tid >> 6, lane = tid & 63;
     const int ml = lane & 15, kg = lane >> 4, wr = 16 * wave, c0 = cq * CP;
+    const int s_of = sigma(lane & 15), kg_of = lane >> 4;   // as my_s and kg, for masks that stay in scalar registers
     const size_t b = blockIdx.x, tok0 = b * (size_t)s;
-    const int stt = tid / V4, sj = (tid % V4) * 4;      // staging slot: token, column
-    const int ve = CP * kg + ml % CP;                   // the vector element a lane holds
-    const int tcol = CP * (ml >> 2) + (ml & 3);         // column of result row ml of block 0; block kt: + 4 kt
-    const int my_s = sigma(ml);                         // token of operand row ml
 
-    f32x4 dFm[4][JT], accEA = kZero;
+    f32x4 accEA = kZero;
     float dG[CP], dGT[CP], sig = 0.f;
+    float *dmb = d_mems + b * 6 * DD;
+    if (second) {   // the gradients of F_k and F_v, and as many barriers as the first half meets
+        f32x4 dFm[2][JT];
+        for (int ci = nc - 1; ci >= 0; ci--) {
+            const int t0 = ci * C, L = min(C, s - t0), ntile = (L + kTB - 1) / kTB;
+            const size_t chunk = b * nc + ci;
+            const float *fz = frozen + chunk * 6 * DD;
+            int me = tid;
+            asm volatile("" : "+v"(me));
+            const int wave = me >> 6, lane = me & 63, ml = lane & 15, kg = lane >> 4;
+            if (ci < nc - 1) put_rows<D>(Bm, dFm[0], me);
+            lds_barrier();
+            if (ci < nc - 1) {
+                f32x4 accG[JT], accN[JT], sums[2][JT], Fv[JT], Fm[JT];
+                request_matrix<D>(Fv, fz + DD, me);
+                request_matrix<D>(Fm, fz + 5 * DD, me);
+                token_sums<D>(sums[0], outer + chunk * 4 * DD, me);
+                token_sums<D>(sums[1], outer + (chunk * 4 + 1) * DD, me);
 #pragma unroll
-    for (int c = 0; c < 4; c++) {
+                for (int i = 0; i < JT; i++) accG[i] = kZero;
 #pragma unroll
-        for (int jt = 0; jt < JT; jt++) dFm[c][jt] = kZero;
+                for (int c = 0; c < 2; c++) {
+                    if (c) {
+                        stage_matrix<D>(Fa, Fv, me);
+                        stage_matrix<D>(Fb, Fm, me);
+                        put_rows<D>(Bm, dFm[1], me);
+                        lds_barrier();
+                    }
+                    boundary_products<D>(Fa, Bm, GLT, accG, accN, me);
+#pragma unroll
+                    for (int jt = 0; jt < JT; jt++) dFm[c][jt] = accN[jt] + sums[c][jt];
+                    lds_barrier();   // every wave has read its matrices
+                }
+                put_rows<D>(Bm, accG, me);
+                lds_barrier();   // the first half adds them up
+                lds_barrier();
+            } else {
+                token_sums<D>(dFm[0], outer + chunk * 4 * DD, me);
+                token_sums<D>(dFm[1], outer + (chunk * 4 + 1) * DD, me);
+            }
+            f32x4 Fk[JT], Fq[JT];
+            float G[CP];
+            // A tile's share of dF, its dg and the next boundary's matrices wait in registers until the other half is among the
+            // tokens of the tile after it, which leave the matrix cores alone; a part of them behind each of four barriers, so
+            // that no token waits for this half.
+            const int stt = me / V4, sj = (me % V4) * 4;
+            float op[4][2], gt[4][JT];
+            f32x4 dg;
+            auto pending = [&](int tile, auto part) {
+                constexpr int v = decltype(part)::value;
+#pragma unroll
+                for (int jt = 0; jt < JT; jt++) {
+                    dFm[0][jt] = mfma4(op[v][0], gt[v][jt], dFm[0][jt]);
+                    dFm[1][jt] = mfma4(op[v][1], gt[v][jt], dFm[1][jt]);
+                }
+                if (v == 0 && tile * kTB + stt < L) *reinterpret_cast<f32x4 *>(d_emb + (tok0 + t0 + tile * kTB + stt) * D + sj) = dg;
+                if (v == 0 || ci == 0 || tile != ntile - 1) return;
+                if (v == 1) stage_matrix<D>(Fa, Fk, me);
+                if (v == 2) stage_matrix<D>(Fb, Fq, me);
+                if (v == 3) {
+#pragma unroll
+                    for (int i = 0; i < CP; i++) GLT[((me & 3) * CP + i) * LD + (me >> 2)] = G[i];
+                }
+            };
+            using std::integral_constant;
+            for (int tile = ntile - 1; tile >= 0; tile--) {
+                const int nt = min(kTB, L - tile * kTB);
+                for (int i = 0; i < 4; i++) lds_barrier();   // top, tile staged, W and Z, the first token
+                if (tile < ntile - 1) pending(tile + 1, integral_constant<int, 0>{});
+                lds_barrier();
+                if (tile < ntile - 1) pending(tile + 1, integral_constant<int, 1>{});
+                lds_barrier();
+                if (tile < ntile - 1) pending(tile + 1, integral_constant<int, 2>{});
+                lds_barrier();
+                if (tile < ntile - 1) pending(tile + 1, integral_constant<int, 3>{});
+                else if (ci > 0) {   // the next boundary's matrices
+                    const float *f = fz - 6 * DD;
+                    lds_read<CP>(G, gl + (chunk - 1) * DD + (me >> 2) * D + (me & 3) * CP);
+                    request_matrix<D>(Fk, f, me);
+                    request_matrix<D>(Fq, f + 2 * DD, me);
+                }
+                for (int i = 3; i < 4 * ((nt + 3) / 4); i++) lds_barrier();   // the other tokens in whole groups of four; dk, dv
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    op[v][0] = dkv[((wave * 4 + v) * 2) * 64 + lane];
+                    op[v][1] = dkv[((wave * 4 + v) * 2 + 1) * 64 + lane];
+#pragma unroll
+                    for (int jt = 0; jt < JT; jt++) gt[v][jt] = tg[(4 * v + kg) * LG + 16 * jt + ml];
+                }
+                dg = *reinterpret_cast<const f32x4 *>(&T_(A_DG, stt, sj));
+            }
+            pending(0, integral_constant<int, 0>{});
+            pending(0, integral_constant<int, 1>{});
+            pending(0, integral_constant<int, 2>{});
+            pending(0, integral_constant<int, 3>{});
+        }
+#pragma unroll
+        for (int c = 0; c < 2; c++) {   // gradients of the initial memories
+#pragma unroll
+            for (int jt = 0; jt < JT; jt++) {
+#pragma unroll
+                for (int v = 0; v < 4; v++) dmb[(size_t)c * DD + (wr + 4 * kg + v) * D + 16 * jt + ml] = dFm[c][jt][v];
+            }
+        }
+        __syncthreads();
+        __syncthreads();
+        return;
     }
 #pragma unroll
     for (int i = 0; i < CP; i++) dG[i] = dGT[i] = 0.f;
@@ -488,128 +663,78 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_sweep_kernel(
     pf_k = pf_v = pf_x = pf_g = pf_dg = pf_fx = pf_gam = make_float4(0, 0, 0, 0);
 #pragma unroll
     for (int i = 0; i < 6; i++) pf_s[i] = 0.f;
-    // Inputs of a tile, requested one tile ahead; rows behind the chunk's last token are zeros.
-    auto request = [&](int first, int nt) {
-        const float4 z = make_float4(0, 0, 0, 0);
-        const size_t o = (tok0 + first + stt) * D + sj;
-        const float *tp = tok + (tok0 + first + stt) * TF;
-        const bool on = stt < nt;
-        auto two = [&](const float *q) {  // rows of tok are 8 bytes aligned
-            const float2 lo = *reinterpret_cast<const float2 *>(q), hi = *reinterpret_cast<const float2 *>(q + 2);
-            return make_float4(lo.x, lo.y, hi.x, hi.y);
-        };
-        pf_k = on ? *reinterpret_cast<const float4 *>(k_cache + o) : z;
-        pf_v = on ? *reinterpret_cast<const float4 *>(v_cache + o) : z;
-        pf_x = on ? *reinterpret_cast<const float4 *>(emb + o) : z;
-        pf_g = on ? two(tp + sj) : z;
-        pf_dg = on ? two(tp + D + sj) : z;
-        pf_fx = on ? two(tp + 2 * D + sj) : z;
-        if (tid < 64) pf_gam = tid / 4 < nt ? two(tok + (tok0 + first + tid / 4) * TF + 3 * D + 4 * (tid % 4)) : z;
-        if (tid < kTB) {  // zeros behind the last token: it passes everything on as it is
-            const float *e = tok + (tok0 + first + min(tid, nt - 1)) * TF + 3 * D + 16;
-#pragma unroll
-            for (int i = 0; i < 6; i++) pf_s[i] = tid < nt ? e[i] : 0.f;
-        }
-    };
-
     for (int ci = nc - 1; ci >= 0; ci--) {
         const int t0 = ci * C, L = min(C, s - t0), ntile = (L + kTB - 1) / kTB;
         const size_t chunk = b * nc + ci;
         const float *fz = frozen + chunk * 6 * DD;
-        // in the order of their use: G_L and F_k for the boundary, then what the tiles read
-        float G[CP];
-        f32x4 fnext[JT];
-        if (ci < nc - 1) {
-            lds_read<CP>(G, gl + chunk * DD + r * D + c0);
-#pragma unroll
-            for (int i = 0; i < JT; i++) {
-                const int e = tid + i * NT;
-                fnext[i] = *reinterpret_cast<const f32x4 *>(fz + (e / V4) * D + (e % V4) * 4);
+        // the thread's place through an opaque copy, once per chunk: addresses made of it are not to live across the sweep
+        int me = tid;
+        asm volatile("" : "+v"(me));
+        const int r = me >> 2, cq = me & 3, wave = me >> 6, lane = me & 63, ml = lane & 15, kg = lane >> 4, wr = 16 * wave,
+                  c0 = cq * CP, stt = me / V4, sj = (me % V4) * 4;
+        // Inputs of a tile, requested one tile ahead; rows behind the chunk's last token are zeros.
+        auto request = [&](int first, int nt) {
+            const size_t o = (tok0 + first + stt) * D + sj;
+            const float *tp = tok + (tok0 + first + stt) * TF;
+            auto two = [&](const float *q) {  // rows of tok are 8 bytes aligned
+                const float2 lo = *reinterpret_cast<const float2 *>(q), hi = *reinterpret_cast<const float2 *>(q + 2);
+                return make_float4(lo.x, lo.y, hi.x, hi.y);
+            };
+            // branches: a choice of values is one of addresses to the compiler, and so a flat load, which the LDS barriers of
+            // the tokens would wait for
+            pf_k = pf_v = pf_x = pf_g = pf_dg = pf_fx = make_float4(0, 0, 0, 0);
+            if (stt < nt) {
+                pf_k = *reinterpret_cast<const float4 *>(k_cache + o);
+                pf_v = *reinterpret_cast<const float4 *>(v_cache + o);
+                pf_x = *reinterpret_cast<const float4 *>(emb + o);
+                pf_g = two(tp + sj);
+                pf_dg = two(tp + D + sj);
+                pf_fx = two(tp + 2 * D + sj);
             }
-        }
-        request(t0 + (ntile - 1) * kTB, L - (ntile - 1) * kTB);
-        // rows of F_k^T and (F_k - F_v)^T, column sums of F_eta, F_alpha
-        float FTk[CP], FTu[CP];
+            if (tid < 64) {
+                pf_gam = make_float4(0, 0, 0, 0);
+                if (tid / 4 < nt) pf_gam = two(tok + (tok0 + first + tid / 4) * TF + 3 * D + 4 * (tid % 4));
+            }
+            if (tid < kTB) {  // zeros behind the last token: it passes everything on as it is
 #pragma unroll
-        for (int i = 0; i < CP; i++) {
-            const float *f = fz + (CP * kg + i) * D + wr + ml;
-            FTk[i] = f[0];
-            FTu[i] = f[DD];
-        }
-        const float csE = csv[chunk * 2 * D + wr + ml], csA = csv[chunk * 2 * D + D + wr + ml];
-        f32x4 sums[4][JT];  // what the chunk's tokens add to dF whatever the sweep finds
+                for (int i = 0; i < 6; i++) pf_s[i] = 0.f;
+                if (tid < nt) {
+                    const float *e = tok + (tok0 + first + tid) * TF + 3 * D + 16;
 #pragma unroll
-        for (int c = 0; c < 4; c++) {
-#pragma unroll
-            for (int jt = 0; jt < JT; jt++)
-                sums[c][jt] = *reinterpret_cast<const f32x4 *>(outer + (chunk * 4 + c) * DD +
-                                                               ((size_t)(wave * JT + jt) * 64 + lane) * 4);
-        }
+                    for (int i = 0; i < 6; i++) pf_s[i] = e[i];
+                }
+            }
+        };
+        float FTk[CP], FTu[CP];   // rows of F_k^T and (F_k - F_v)^T
+        // column sums of F_eta, F_alpha
+        float csE = csv[chunk * 2 * D + wr + ml], csA = csv[chunk * 2 * D + D + wr + ml];
         // LDS-only barriers from here on: the requests above and the stores of dg stay under way across them
+        if (ci < nc - 1 && kg == 0) { av[0][wr + ml] = accEA[0]; av[1][wr + ml] = accEA[1]; }
         lds_barrier();
         sig = 0.f;
         if (ci < nc - 1) {
             // Chunk boundary: gradients of F'_c = F_c G_L flow into dG_L = sum_c F_c^T dF'_c and dF_c = dF'_c G_L^T, on
             // the matrix cores; the rows of dF_eta, dF_alpha are all equal (rank-1 terms of dG_L).
-            float *Fs = raw, *Bm = raw + D * LD, *GLT = raw + 2 * D * LD;
-            float q[CP];
-#pragma unroll
-            for (int i = 0; i < CP; i++) GLT[(c0 + i) * LD + r] = G[i];
-            if (kg == 0) { av[0][wr + ml] = accEA[0]; av[1][wr + ml] = accEA[1]; }
-            lds_barrier();
-            {
-                float eE[CP], eA[CP];
-                lds_read<CP>(eE, &av[0][c0]);
-                lds_read<CP>(eA, &av[1][c0]);
-                const float e = csv[chunk * 2 * D + r], a = csv[chunk * 2 * D + D + r];
-#pragma unroll
-                for (int i = 0; i < CP; i++) q[i] = e * eE[i] + a * eA[i];
-            }
+            float q[CP], G[CP];
+            const float e = csv[chunk * 2 * D + r], a = csv[chunk * 2 * D + D + r];
             f32x4 accG[JT];
 #pragma unroll
             for (int i = 0; i < JT; i++) accG[i] = kZero;
+            f32x4 dF[JT], sums[JT];
 #pragma unroll
-            for (int comp = 0; comp < 4; comp++) {
-                lds_barrier();
-#pragma unroll
-                for (int i = 0; i < JT; i++) {
-                    const int e = tid + i * NT;
-                    *reinterpret_cast<f32x4 *>(Fs + (e / V4) * LD + (e % V4) * 4) = fnext[i];
+            for (int c = 0; c < 2; c++) {
+                if (c) {
+                    put_rows<D>(kept, dF, me);
+                    lds_barrier();
                 }
-                if (comp < 3) {
-                    const float *nf = fz + (size_t)(comp < 2 ? comp + 1 : 5) * DD;
+                token_sums<D>(sums, outer + (chunk * 4 + 2 + c) * DD, me);
 #pragma unroll
-                    for (int i = 0; i < JT; i++) {
-                        const int e = tid + i * NT;
-                        fnext[i] = *reinterpret_cast<const f32x4 *>(nf + (e / V4) * D + (e % V4) * 4);
-                    }
-                }
+                for (int i = 0; i < CP; i++) (c ? FTu : FTk)[i] = Fa[(CP * kg + i) * LD + wr + ml];
+                boundary_products<D>(Fb, kept + c * D * LD, GLT, accG, dF, me);
 #pragma unroll
-                for (int jt = 0; jt < JT; jt++) {
-#pragma unroll
-                    for (int v = 0; v < 4; v++) Bm[(wr + 4 * kg + v) * LD + 16 * jt + ml] = dFm[comp][jt][v];
-                }
-                f32x4 accN[JT];
-#pragma unroll
-                for (int jt = 0; jt < JT; jt++) accN[jt] = kZero;
-                lds_barrier();
-                // contraction in the order 16 c + 4 kg + v: rows 4 apart put the four kg of a read on different banks
-#pragma unroll
-                for (int c = 0; c < KT; c++) {
-                    const f32x4 a2 = *reinterpret_cast<const f32x4 *>(Bm + (wr + ml) * LD + 16 * c + 4 * kg);  // dF'_c
-#pragma unroll
-                    for (int v = 0; v < 4; v++) {
-                        const int k = 16 * c + 4 * kg + v;
-                        const float a1 = Fs[k * LD + wr + ml];  // F_c^T
-#pragma unroll
-                        for (int jt = 0; jt < JT; jt++) {
-                            accG[jt] = mfma4(a1, Bm[k * LD + 16 * jt + ml], accG[jt]);
-                            accN[jt] = mfma4(a2[v], GLT[k * LD + 16 * jt + ml], accN[jt]);
-                        }
-                    }
-                }
-#pragma unroll
-                for (int jt = 0; jt < JT; jt++) dFm[comp][jt] = accN[jt];
+                for (int jt = 0; jt < JT; jt++) dF[jt] += sums[jt];
+                if (c) request(t0 + (ntile - 1) * kTB, L - (ntile - 1) * kTB);
+                lds_barrier();  // every wave has read its matrices
             }
             {   // accE <- G_L accE, accA <- G_L accA: rows 0 and 1 of one more product
                 f32x4 accV = kZero;
@@ -621,39 +746,62 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_sweep_kernel(
                 }
                 accEA = accV;
             }
-            lds_barrier();  // every wave has read Bm
+            put_rows<D>(kept + D * LD, dF, me);
+            put_rows<D>(Fb, accG, me);
+            {
+                float eE[CP], eA[CP];
+                lds_read<CP>(eE, &av[0][c0]);
+                lds_read<CP>(eA, &av[1][c0]);
 #pragma unroll
-            for (int jt = 0; jt < JT; jt++) {
-#pragma unroll
-                for (int v = 0; v < 4; v++) Bm[(wr + 4 * kg + v) * LD + 16 * jt + ml] = accG[jt][v];
+                for (int i = 0; i < CP; i++) q[i] = e * eE[i] + a * eA[i];
             }
-            __builtin_amdgcn_wave_barrier();
-            float t[CP];
-            lds_read<CP>(t, Bm + r * LD + c0);
+            lds_barrier();  // both halves' sums are there
+            float t[CP], h[CP];
+            lds_read<CP>(t, Fb + r * LD + c0);
+            lds_read<CP>(h, Bm + r * LD + c0);
 #pragma unroll
-            for (int i = 0; i < CP; i++) t[i] += q[i];
-            vec_store<CP>(Bm + r * LD + c0, t);
+            for (int i = 0; i < CP; i++) t[i] += h[i] + q[i];
+            vec_store<CP>(Fb + r * LD + c0, t);
             // sigma_L = <G_L, dG_L>; then (1-a_t) <G_t, dG_{t+1}> = sigma_{t+1} + th_t u.W_t and
             // sigma_t = that + dg.g + dp.p carry the inner product the gradient of alpha needs
+#pragma unroll
+            for (int i = 0; i < CP; i++) G[i] = GLT[(c0 + i) * LD + r];
             const float part = wave_allreduce(dotn<CP>(G, t));
             if (lane == 0) sp[wave] = part;
             lds_barrier();
 #pragma unroll
             for (int w = 0; w < NW; w++) sig += sp[w];
-            lds_read<CP>(dG, Bm + (wr + ml) * LD + CP * kg);
+            lds_read<CP>(dG, Fb + (wr + ml) * LD + CP * kg);
 #pragma unroll
-            for (int i = 0; i < CP; i++) dGT[i] = Bm[(CP * kg + i) * LD + wr + ml];
-        }
+            for (int i = 0; i < CP; i++) dGT[i] = Fb[(CP * kg + i) * LD + wr + ml];
+        } else {
+            request(t0 + (ntile - 1) * kTB, L - (ntile - 1) * kTB);
 #pragma unroll
-        for (int c = 0; c < 4; c++) {
-#pragma unroll
-            for (int jt = 0; jt < JT; jt++) dFm[c][jt] += sums[c][jt];
+            for (int i = 0; i < CP; i++) {
+                const float *f = fz + (CP * kg + i) * D + wr + ml;
+                FTk[i] = f[0];
+                FTu[i] = f[DD];
+            }
+            f32x4 sums[2][JT];
+            token_sums<D>(sums[0], outer + (chunk * 4 + 2) * DD, me);
+            token_sums<D>(sums[1], outer + (chunk * 4 + 3) * DD, me);
+            put_rows<D>(kept, sums[0], me);
+            put_rows<D>(kept + D * LD, sums[1], me);
         }
 #pragma unroll
         for (int i = 0; i < CP; i++) FTu[i] = FTk[i] - FTu[i];
+        // arrived here: a wait for them inside the tile loop would be one for the next tile's requests as well
+        asm volatile("" : "+v"(csE), "+v"(csA));
 
         for (int tile = ntile - 1; tile >= 0; tile--) {
             const int tb = t0 + tile * kTB, nt = min(kTB, t0 + L - tb);
+            int me = tid;   // and once per tile
+            asm volatile("" : "+v"(me));
+            const int tid = me, wave = tid >> 6, lane = tid & 63, ml = lane & 15, kg = lane >> 4, wr = 16 * wave,
+                      stt = tid / V4, sj = (tid % V4) * 4,      // staging slot: token, column
+                      ve = CP * kg + ml % CP,                   // the vector element a lane holds
+                      tcol = CP * (ml >> 2) + (ml & 3),         // column of result row ml of block 0; block kt: + 4 kt
+                      my_s = sigma(ml);                         // token of operand row ml
             lds_barrier();
             *reinterpret_cast<float4 *>(&T_(A_K, stt, sj)) = pf_k;
             *reinterpret_cast<float4 *>(&T_(A_U, stt, sj)) =
@@ -669,7 +817,6 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_sweep_kernel(
                 *reinterpret_cast<float2 *>(&sc[tid][4]) = make_float2(pf_s[4], pf_s[5]);
             }
             lds_barrier();
-            if (tile > 0) request(tb - kTB, kTB);
 
             // W = dG K, Z = dG^T U, Y = F_k^T Z + (F_k - F_v)^T W of the whole tile; T_s = u_s . W_s.  A sum per 16 terms,
             // added up in a tree: one running sum rounds at every term (d_x 1.1 to 1.2 times as far from float64)
@@ -715,6 +862,7 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_sweep_kernel(
             f32x4 Y = tree(Yq) + tree(Y2q);
             T = swapadd32(T, T);
             T = swapadd16(T, T);
+            if (tile > 0) request(tb - kTB, kTB);
 
             // a_ts = dg_t . u_s for t = 4 j + kg, and prod_{s<r<t} (1-a_r); the same product over the whole tile above s;
             // prod_{r<t} (1-a_r) for t = 4 j + kg
@@ -737,6 +885,7 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_sweep_kernel(
                 T_(A_DG, t, wr + ml) = fmaf(da, csA, fmaf(de, csE, fmaf(-th, ybc, dg0)));
                 lds_barrier();
                 const float dgv = T_(A_DG, t, ve), gv = tg[t * LG + ve];
+                __builtin_amdgcn_sched_barrier(0);  // first in the queue: the step's chain starts with them
                 const f32x4 ps = *reinterpret_cast<const f32x4 *>(&Sx[wave][4 * kg]);
                 const float gml = gam[t * kTB + ml], fx = T_(A_FX, t, wr + ml);
                 const f32x4 g4 = *reinterpret_cast<const f32x4 *>(&gam[t * kTB + 4 * kg]);
@@ -747,14 +896,14 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_sweep_kernel(
                 }
                 __builtin_amdgcn_sched_barrier(0);  // what follows runs while the reads are under way
                 // tables of the tile's end: the retention of token t counts for the pairs around it
-                const float km = my_s < t ? keep : 1.f;
+                const float km = s_of < t ? keep : 1.f;
                 above *= km;
 #pragma unroll
                 for (int j = J; j < 4; j++) { ct[j] *= km; below[j] *= keep; }
                 keep_tile *= keep;
-                const bool mine = kg == Q;
+                const bool mine = kg_of == Q;
                 below[J] = mine ? 1.f : below[J];
-                ct[J] = mine ? (my_s < t ? 1.f : 0.f) : ct[J];
+                ct[J] = mine ? (s_of < t ? 1.f : 0.f) : ct[J];
                 et[J] = mine ? (ml == 0 ? de : da) : et[J];
                 float yold = 0.f;
                 if constexpr (t > 0) {
@@ -808,16 +957,13 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_sweep_kernel(
 #pragma unroll
             for (int v = 0; v < 4; v++) {
                 const int t = 4 * v + kg;
-                const float th = sc[t][1], dv = th * W[v], dk = -th * (Z[v] + W[v]);
-                const float ea = ml < 2 ? et[v] : 0.f;
-#pragma unroll
-                for (int jt = 0; jt < JT; jt++) {
-                    const float g = tg[t * LG + 16 * jt + ml];
-                    dFm[0][jt] = mfma4(dk, g, dFm[0][jt]);
-                    dFm[1][jt] = mfma4(dv, g, dFm[1][jt]);
-                }
-                accEA = mfma4(ea, tg[t * LG + wr + ml], accEA);
+                const float th = sc[t][1];
+                dkv[((wave * 4 + v) * 2) * 64 + lane] = -th * (Z[v] + W[v]);
+                dkv[((wave * 4 + v) * 2 + 1) * 64 + lane] = th * W[v];
             }
+            lds_barrier();
+#pragma unroll
+            for (int v = 0; v < 4; v++) accEA = mfma4(ml < 2 ? et[v] : 0.f, tg[(4 * v + kg) * LG + wr + ml], accEA);
             if (tile > 0) {  // the chunk's first tile has no use for its dG: G_0 = I
                 f32x4 n[KT], nT[KT];
 #pragma unroll
@@ -844,21 +990,14 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_sweep_kernel(
                     for (int v = 0; v < 4; v++) { dG[4 * kt + v] = n[kt][v]; dGT[4 * kt + v] = nT[kt][v]; }
                 }
             }
-            if (stt < nt)
-                *reinterpret_cast<float4 *>(d_emb + (tok0 + tb + stt) * D + sj) =
-                    *reinterpret_cast<const float4 *>(&T_(A_DG, stt, sj));
         }
     }
-    // gradients of the initial memories
-    float *dmb = d_mems + b * 6 * DD;
 #pragma unroll
-    for (int comp = 0; comp < 4; comp++) {
-        float *dst = dmb + (comp < 3 ? comp : 5) * DD;
-#pragma unroll
-        for (int jt = 0; jt < JT; jt++) {
-#pragma unroll
-            for (int v = 0; v < 4; v++) dst[(wr + 4 * kg + v) * D + 16 * jt + ml] = dFm[comp][jt][v];
-        }
+    for (int i = 0; i < JT; i++) {   // gradients of the initial memories, rows of every wave's own
+        const int row = wr + 16 * i / JT + lane / (4 * JT), at = lane % (4 * JT) * 4;
+        *reinterpret_cast<f32x4 *>(dmb + (size_t)2 * DD + row * D + at) = *reinterpret_cast<const f32x4 *>(kept + row * LD + at);
+        *reinterpret_cast<f32x4 *>(dmb + (size_t)5 * DD + row * D + at) =
+            *reinterpret_cast<const f32x4 *>(kept + (D + row) * LD + at);
     }
     __syncthreads();
     if (kg == 0) { av[0][wr + ml] = accEA[0]; av[1][wr + ml] = accEA[1]; }
@@ -883,8 +1022,11 @@ void launch(const SelfrefSweep &a) {
     hipLaunchKernelGGL((selfref_bwd_prepare_kernel<D>), dim3(a.batch * a.nc), dim3(4 * D), lds, stream(), a.emb, a.d_y, a.k,
                        a.v, a.q, a.alpha, a.theta, a.amean, a.emean, a.frozen, a.gl, a.tok, a.outer, a.csv, a.s, a.C, a.nc);
     check_launch("selfref_bwd_prepare_kernel");
+    constexpr size_t sweep_lds = sweep_lds_floats(D) * sizeof(float);
+    check_hip(hipFuncSetAttribute(reinterpret_cast<const void *>(selfref_bwd_sweep_kernel<D>),
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)sweep_lds), "dynamic LDS size");
     KernelTimer kt("selfref_bwd_kernel");
-    hipLaunchKernelGGL((selfref_bwd_sweep_kernel<D>), dim3(a.batch), dim3(4 * D), 0, stream(), a.emb, a.k, a.v, a.frozen,
+    hipLaunchKernelGGL((selfref_bwd_sweep_kernel<D>), dim3(a.batch), dim3(8 * D), sweep_lds, stream(), a.emb, a.k, a.v, a.frozen,
                        a.gl, a.tok, a.outer, a.csv, a.d_emb, a.d_mems, a.s, a.C, a.nc);
     check_launch("selfref_bwd_sweep_kernel");
 }

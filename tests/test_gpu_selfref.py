@@ -151,3 +151,13 @@ def test_saturated_decay_gate(sg, d, C, early):                                 
         e_gpu = float(np.abs(got[n].reshape(r.shape) - r).max()) / scale
         e_f32 = float(np.abs(want[n].reshape(r.shape) - r).max()) / scale
         assert e_gpu <= max(1e-4, 4.0 * e_f32), f"{n}: {e_gpu:.2e} against float64, float32 oracle {e_f32:.2e}"
+
+
+@pytest.mark.parametrize("B,s,d,C", [
+    (2, 208, 64, 64),    # boundaries into and out of chunks of four tiles
+    (2, 80, 64, 16),     # chunks of one tile: nothing of a tile waits for the next
+    (3, 99, 32, 48),
+    (2, 35, 16, 16),     # a wave a half
+    (1, 77, 64, 19)])    # tiles of sixteen and of three tokens
+def test_sweep_in_two_halves(B, s, d, C):
+    test_forward_backward_match_oracle(B, s, d, C, True)
