@@ -14,13 +14,13 @@ typedef unsigned short u16;
 
 constexpr int HD = 64;             // head size
 constexpr int CW = 64;             // tokens per chunk tile
-constexpr int LDB = 72;            // LDS row stride of a bf16 matrix (144 B: 16-byte rows, conflict-free operand reads)
+constexpr int LDB = 72;            // LDS row stride of a bf16 matrix: 144 B, 16-byte rows (the permuted layout below has fewer bank conflicts)
 constexpr int BMAT = 64 * LDB;     // elements per bf16 matrix
 constexpr int kPerm = 64 * 64;     // elements of a matrix in the permuted layout below
 constexpr int kTileThr = 512;      // 8 waves
 
-// The other layout of a bf16 matrix, of kPerm = 64 x 64 elements, element (row, col): rows of 64, their eight 16-byte blocks permuted by the row's bits 1 to 3 so that
-// what one access takes together falls on different banks.  That is, of a 64-bank LDS: for ld_op rows 0..3 and 12..15 of a
+// The other layout of a bf16 matrix, of kPerm = 64 x 64 elements, element (row, col): rows of 64, their eight 16-byte blocks
+// permuted by the row's bits 1 to 3 so that what one access takes together falls on different banks.  That is, of a 64-bank LDS: for ld_op rows 0..3 and 12..15 of a
 // block with rows 4..11 of the next; for ld_op_tr rows 0..3 and 8..11 of two blocks; for the 8-byte writes of an accumulator
 // tile sixteen rows of one block.  A row stride that is odd in 16-byte units serves the last but not the first two, an even one
 // the other way round: with either, half of the LDS time of the chain kernels was conflicts (adjoint scan at 128 chains of 4096

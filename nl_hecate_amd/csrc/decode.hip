@@ -11,8 +11,8 @@
 //                              window): attention scores and the slice's share of the output.  All independent.
 //   3. decode_output_kernel    attention slices merged, levels combined, sigmoid gate, output projection
 //   4. decode_logits_kernel    the unembedding, written to the workspace and to host-visible memory
-// Measured on one MI355X at d = 512, four levels of which one is active, window 512, vocabulary 32 000: 0.50 -> 0.058 ms
-// a token with the host side, of which 4.9 + 4.4 + 5.3 + 12.1 us in the four kernels (the last one moves 65 MB at
+// Measured on one MI355X at d = 512, four levels of which one is active, window 512, vocabulary 32 000: 0.50 -> 0.048 ms
+// a token with the host side, of which 4.9 + 4.4 + 5.3 + 12.0 us in the four kernels (the last one moves 65 MB at
 // 5.4 TB/s) and about 11 us before the first one starts and after the last one has ended.
 #include <float.h>
 #include <hip/hip_runtime.h>
