@@ -12,7 +12,7 @@
 //   3. decode_output_kernel    attention slices merged, levels combined, sigmoid gate, output projection
 //   4. decode_logits_kernel    the unembedding, written to the workspace and to host-visible memory
 // Measured on one MI355X at d = 512, four levels of which one is active, window 512, vocabulary 32 000: 0.50 -> 0.048 ms
-// a token with the host side, of which 4.9 + 4.4 + 5.3 + 12.0 us in the four kernels (the last one moves 65 MB at
+// a token with the host side, of which 4.1 + 4.4 + 4.9 + 12.2 us in the four kernels (the last one moves 65 MB at
 // 5.4 TB/s) and about 11 us before the first one starts and after the last one has ended.
 #include <float.h>
 #include <hip/hip_runtime.h>
@@ -30,7 +30,7 @@ constexpr int kMaxLevels = 8;
 constexpr int kSliceKeys = 128;   // keys of the window per attention workgroup: 4 passes of 32 (head size 64)
 
 struct DecLevel {
-    const float *w_k, *w_v, *w_q, *w_alpha, *b_alpha, *w_theta, *b_theta;
+    const float *w_alpha, *b_alpha, *w_theta, *b_theta;
     float *memory;               // [heads, hd*hd]
     float *k, *v, *q, *y;        // [d] each, in the work buffer
     float alpha_floor, alpha_ceil, theta_floor, theta_ceil, clip, m_norm;
@@ -38,14 +38,17 @@ struct DecLevel {
 };
 struct DecArgs {
     const float *x;              // the token's embedding row
-    const float *w_q, *w_k, *w_v, *w_o;
-    uint16_t *q_bf16, *k_row, *v_row;
+    const float *w_o;
+    uint16_t *q_bf16;
     const uint16_t *k_cache, *v_cache;
     float *part_o, *part_ml;     // attention slices: [slice][d], [slice][heads][2]
     float *embedded, *attn_out, *y_combined, *gate, *gated, *projected;
     uint16_t *attn_bf16;
-    int d, nh, hd, levels, pos, window, n_persistent, slices;
+    int d, nh, hd_log2, levels, pos, window, n_persistent, slices;
     DecLevel lv[kMaxLevels];
+    // the products with the embedded token: d rows each, outputs q, k, v of the attention (rounded) or floats
+    const float *seg_w[3 + 3 * kMaxLevels];
+    void *seg_out[3 + 3 * kMaxLevels];
 };
 
 __device__ __forceinline__ float bf2f(uint16_t u) { return __uint_as_float((uint32_t)u << 16); }
@@ -53,28 +56,15 @@ __device__ __forceinline__ float dot4(const float4 &a, const float4 &b) { return
 
 __host__ __device__ inline bool reads_only(int rule) { return rule < 0 || rule == 3; }
 
-// Segments of d rows in the order: attention q, k, v, then per active level k, v, q, per frozen level q.
+// Segments of d rows in the order: attention q, k, v, then per active level k, v, q, per frozen level q; their addresses come
+// by number (a search over the levels' rules, one scalar load after the other, stood ahead of every other load: 4.85 -> 4.05 us
+// at d = 512, four levels of which one is active).
 __global__ __launch_bounds__(kDecThr) void decode_project_kernel(DecArgs a) {
-    const int lane = threadIdx.x & 63, wave = (blockIdx.x * kDecThr + threadIdx.x) >> 6;
-    const int row0 = wave * 4, seg = row0 / a.d, r = row0 - seg * a.d, n4 = a.d >> 2;
-    const float *w;
-    float *out = nullptr;
-    uint16_t *out16 = nullptr;
-    if (seg == 0) { w = a.w_q; out16 = a.q_bf16; }
-    else if (seg == 1) { w = a.w_k; out16 = a.k_row; }
-    else if (seg == 2) { w = a.w_v; out16 = a.v_row; }
-    else {
-        int s = seg - 3, l = 0;
-        for (; l < a.levels; l++) {
-            const int n = reads_only(a.lv[l].rule) ? 1 : 3;
-            if (s < n) break;
-            s -= n;
-        }
-        if (l == a.levels) return;
-        if (reads_only(a.lv[l].rule)) s = 2;
-        w = s == 0 ? a.lv[l].w_k : s == 1 ? a.lv[l].w_v : a.lv[l].w_q;
-        out = s == 0 ? a.lv[l].k : s == 1 ? a.lv[l].v : a.lv[l].q;
-    }
+    const int lane = threadIdx.x & 63, seg = blockIdx.y, n4 = a.d >> 2;   // d is a multiple of 32: whole workgroups of 16 rows
+    const int r = 16 * blockIdx.x + 4 * __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const float *w = a.seg_w[seg];
+    float *out = seg < 3 ? nullptr : (float *)a.seg_out[seg];
+    uint16_t *out16 = (uint16_t *)a.seg_out[seg];
     const float4 *x = reinterpret_cast<const float4 *>(a.x);
     const float4 *w0 = reinterpret_cast<const float4 *>(w + (size_t)r * a.d);
     float acc[4] = {0.f, 0.f, 0.f, 0.f};
@@ -99,7 +89,7 @@ __global__ __launch_bounds__(kDecThr) void decode_project_kernel(DecArgs a) {
         if (out) out[r + lane] = y;
         else out16[r + lane] = f32_to_bf16_rne(y);
     }
-    if (blockIdx.x == 0)
+    if (blockIdx.x == 0 && seg == 0)
         for (int i = threadIdx.x; i < n4; i += kDecThr) reinterpret_cast<float4 *>(a.embedded)[i] = x[i];
 }
 
@@ -278,15 +268,15 @@ __device__ __forceinline__ void attention_slice(const DecArgs &a, int h, int sli
 template <int HD>
 __global__ __launch_bounds__(kDecThr) void decode_heads_kernel(DecArgs a) {
     __shared__ float red[16 + 4 * HD];
-    const int n_attn = a.nh * a.slices, b = blockIdx.x;
-    if (b < n_attn) attention_slice<HD>(a, b % a.nh, b / a.nh, red);
-    else level_head<HD>(a, (b - n_attn) / a.nh, (b - n_attn) % a.nh, red);
+    const int h = blockIdx.x, part = blockIdx.y;
+    if (part < a.slices) attention_slice<HD>(a, h, part, red);
+    else level_head<HD>(a, part - a.slices, h, red);
 }
 
 // Eight rows of the output projection per workgroup; every workgroup forms the whole gated vector for itself.  The
 // chain of loads is what takes the time, so nothing is loaded behind a value it does not need: the weights of the first
 // 1024 columns, the slices' statistics (one thread each, then shared in LDS) and the levels and slices of a thread's first
-// two columns are all requested at the top (10.0 -> 7.0 -> 5.3 us at d = 512, 5 slices, 4 levels).
+// two columns are all requested at the top (10.0 -> 7.0 -> 4.9 us at d = 512, 5 slices, 4 levels).
 __global__ __launch_bounds__(kDecThr) void decode_output_kernel(DecArgs a) {
     extern __shared__ float smem[];
     float *gated = smem, *wgt = smem + a.d;   // [d], [slices][heads]: a slice's weight in the merged softmax
@@ -344,7 +334,7 @@ __global__ __launch_bounds__(kDecThr) void decode_output_kernel(DecArgs a) {
     }
     __syncthreads();
     auto column = [&](int i, const float(&t0)[NL], const float(&o0)[NS]) {
-        const int h = i / a.hd;
+        const int h = i >> a.hd_log2;
         float o = 0.f, y = 0.f;
         for (int l = 0; l < a.levels; l += NL) {
             float t[NL];
@@ -477,9 +467,8 @@ int decode_token_rocm(const float *embedding_row, const float *w_q, const float 
     }
     DecArgs a;
     a.x = embedding_row;
-    a.w_q = w_q; a.w_k = w_k; a.w_v = w_v; a.w_o = w_o;
+    a.w_o = w_o;
     a.k_cache = k_cache; a.v_cache = v_cache;
-    a.k_row = k_cache + (size_t)pos * d; a.v_row = v_cache + (size_t)pos * d;
     a.embedded = (float *)workspace[0];
     a.q_bf16 = (uint16_t *)workspace[1];
     a.attn_bf16 = (uint16_t *)workspace[2];
@@ -487,7 +476,7 @@ int decode_token_rocm(const float *embedding_row, const float *w_q, const float 
     a.y_combined = (float *)workspace[4];
     a.gate = (float *)workspace[5];
     a.gated = (float *)workspace[6];
-    a.d = d; a.nh = heads; a.hd = hd; a.levels = levels; a.pos = pos; a.window = window; a.n_persistent = n_persistent;
+    a.d = d; a.nh = heads; a.hd_log2 = hd == 32 ? 5 : hd == 64 ? 6 : 7; a.levels = levels; a.pos = pos; a.window = window; a.n_persistent = n_persistent;
     const int n_pre = pos + 1 < n_persistent ? pos + 1 : n_persistent;
     const int ls = pos + 1 - window > n_persistent ? pos + 1 - window : n_persistent;
     const int n_keys = n_pre + (pos + 1 > ls ? pos + 1 - ls : 0);
@@ -497,12 +486,14 @@ int decode_token_rocm(const float *embedding_row, const float *w_q, const float 
         return 1;
     }
     float *p = work;
-    int segs = 3;
+    int segs = 0;
+    a.seg_w[segs] = w_q; a.seg_out[segs++] = a.q_bf16;
+    a.seg_w[segs] = w_k; a.seg_out[segs++] = k_cache + (size_t)pos * d;
+    a.seg_w[segs] = w_v; a.seg_out[segs++] = v_cache + (size_t)pos * d;
     for (int l = 0; l < levels; l++) {
         const void *const *lp = level_ptrs + 8 * l;
         const float *b = level_bounds + 6 * l;
         DecLevel &lv = a.lv[l];
-        lv.w_k = (const float *)lp[0]; lv.w_v = (const float *)lp[1]; lv.w_q = (const float *)lp[2];
         lv.w_alpha = (const float *)lp[3]; lv.b_alpha = (const float *)lp[4];
         lv.w_theta = (const float *)lp[5]; lv.b_theta = (const float *)lp[6];
         lv.memory = (float *)const_cast<void *>(lp[7]);
@@ -510,7 +501,11 @@ int decode_token_rocm(const float *embedding_row, const float *w_q, const float 
         p += 4 * d;
         lv.alpha_floor = b[0]; lv.alpha_ceil = b[1]; lv.theta_floor = b[2]; lv.theta_ceil = b[3]; lv.clip = b[4]; lv.m_norm = b[5];
         lv.rule = level_rule[l];
-        segs += reads_only(lv.rule) ? 1 : 3;
+        if (!reads_only(lv.rule)) {
+            a.seg_w[segs] = (const float *)lp[0]; a.seg_out[segs++] = lv.k;
+            a.seg_w[segs] = (const float *)lp[1]; a.seg_out[segs++] = lv.v;
+        }
+        a.seg_w[segs] = (const float *)lp[2]; a.seg_out[segs++] = lv.q;
     }
     a.part_o = p; p += (size_t)a.slices * d;
     a.part_ml = p; p += (size_t)a.slices * heads * 2;
@@ -518,12 +513,12 @@ int decode_token_rocm(const float *embedding_row, const float *w_q, const float 
     const hipStream_t st = stream();
     {
         KernelTimer kt("decode_project_kernel");
-        hipLaunchKernelGGL(decode_project_kernel, dim3(ceil_div((long long)segs * d, 16)), dim3(kDecThr), 0, st, a);
+        hipLaunchKernelGGL(decode_project_kernel, dim3(d / 16, segs), dim3(kDecThr), 0, st, a);
         check_launch("decode_project_kernel");
     }
     {
         KernelTimer kt("decode_heads_kernel");
-        const dim3 grid(heads * (a.slices + levels));
+        const dim3 grid(heads, a.slices + levels);
         if (hd == 32) hipLaunchKernelGGL(decode_heads_kernel<32>, grid, dim3(kDecThr), 0, st, a);
         else if (hd == 64) hipLaunchKernelGGL(decode_heads_kernel<64>, grid, dim3(kDecThr), 0, st, a);
         else hipLaunchKernelGGL(decode_heads_kernel<128>, grid, dim3(kDecThr), 0, st, a);
