@@ -1,8 +1,14 @@
 """The key that an argument block of tensor addresses is kept under: whatever a tensor can change where it stands shows."""
+import os
+import subprocess
+
 import pytest
 import torch
 
 from nl_hecate_amd import ffi
+
+if not os.path.exists(ffi.KEY_PATH):   # host code: builds without the library
+    subprocess.check_call(["make", "-s", "-C", os.path.join(os.path.dirname(os.path.abspath(ffi.__file__)), "csrc"), "plan_key"])
 
 
 @pytest.mark.parametrize("change", ["nothing", "values", "transpose", "shape", "resize", "data", "type", "view"])
