@@ -15,6 +15,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <atomic>
+
 #include "../../include/nl_hecate_ffi.h"
 #include "chunkwise_chain.h"
 #include "chunkwise_guard.h"
@@ -23,6 +25,10 @@
 #include "runtime.h"
 
 namespace nlh {
+
+bool force_sequential = false;
+bool last_test_fired = false;
+
 namespace {
 
 using namespace mmt;
@@ -171,14 +177,28 @@ __global__ __launch_bounds__(256) void cw_guard_tracks_kernel(const TOK *__restr
     if (bad) *flag = 1;
 }
 
-__global__ void guard_clear_kernel(int *flag) { *flag = 0; }
+// The flag of a test stands in pinned host memory, where a kernel stores to it only if the test fires: a flag on the device
+// took a launch to clear and a copy to read (32 chains x 1500 tokens, float, bounded, forward and backward 333 -> 320 us).
+constexpr int kFlags = 64;   // in turn: tests of several threads do not share one
+int *g_host_flags = nullptr;
+std::atomic<unsigned> g_next_flag{0};
 
-int *g_host_flag = nullptr;
+int *lowered_flag() {
+    if (!g_host_flags)
+        check_hip(hipHostMalloc(reinterpret_cast<void **>(&g_host_flags), kFlags * sizeof(int), hipHostMallocDefault), "hipHostMalloc");
+    if (!g_host_flags) return nullptr;
+    int *flag = g_host_flags + g_next_flag++ % kFlags;
+    *(volatile int *)flag = 0;
+    return flag;
+}
+
+bool test_fired(const ErrorScope &es, const int *flag) {
+    check_hip(hipStreamSynchronize(stream()), "guard flag sync");
+    last_test_fired = es.failed() || *(const volatile int *)flag != 0;
+    return last_test_fired;
+}
 
 }  // namespace
-
-bool force_sequential = false;
-bool last_test_fired = false;
 
 bool guard_possible() {
     if (force_sequential) return false;
@@ -191,13 +211,11 @@ static bool couplings_may_fire_t(const TOK *k, const TOK *v, const float *alpha,
                                  const float *m_states, const float *s_states, int seq_len, int batch, int chunk_size,
                                  float error_clip, float m_norm_max) {
     const ErrorScope es;
-    int *flag = reinterpret_cast<int *>(scratch(31, 256));
-    if (!g_host_flag) check_hip(hipHostMalloc(reinterpret_cast<void **>(&g_host_flag), 256, hipHostMallocDefault), "hipHostMalloc");
-    if (es.failed() || !g_host_flag) return true;
+    int *flag = lowered_flag();
+    if (es.failed() || !flag) return true;
     const int nc = (seq_len + chunk_size - 1) / chunk_size;
     {
         KernelTimer kt("cw_guard_kernel");
-        hipLaunchKernelGGL(guard_clear_kernel, dim3(1), dim3(1), 0, stream(), flag);
         const dim3 grid((unsigned)batch * nc);
         if (s_states)
             hipLaunchKernelGGL((cw_guard_kernel<TOK, true>), grid, dim3(kThr), 0, stream(), k, v, alpha, theta, eta, m_states,
@@ -207,11 +225,7 @@ static bool couplings_may_fire_t(const TOK *k, const TOK *v, const float *alpha,
                                s_states, seq_len, chunk_size, nc, error_clip, m_norm_max, flag);
         check_launch("cw_guard_kernel");
     }
-    *g_host_flag = 1;
-    check_hip(hipMemcpyAsync(g_host_flag, flag, sizeof(int), hipMemcpyDeviceToHost, stream()), "guard flag copy");
-    check_hip(hipStreamSynchronize(stream()), "guard flag sync");
-    last_test_fired = es.failed() || *g_host_flag != 0;
-    return last_test_fired;
+    return test_fired(es, flag);
 }
 
 namespace {
@@ -226,21 +240,15 @@ __global__ void norm_bound_kernel(const float *__restrict__ msq_part, int batch,
 
 bool norm_bound_exceeded(const float *msq_part, int batch, int parts, float m_norm_max) {
     const ErrorScope es;
-    int *flag = reinterpret_cast<int *>(scratch(31, 256));
-    if (!g_host_flag) check_hip(hipHostMalloc(reinterpret_cast<void **>(&g_host_flag), 256, hipHostMallocDefault), "hipHostMalloc");
-    if (es.failed() || !g_host_flag) return true;
+    int *flag = lowered_flag();
+    if (es.failed() || !flag) return true;
     {
         KernelTimer kt("norm_bound_kernel");
-        hipLaunchKernelGGL(guard_clear_kernel, dim3(1), dim3(1), 0, stream(), flag);
         hipLaunchKernelGGL(norm_bound_kernel, dim3((batch + 255) / 256), dim3(256), 0, stream(), msq_part, batch, parts,
                            m_norm_max * m_norm_max, flag);
         check_launch("norm_bound_kernel");
     }
-    *g_host_flag = 1;
-    check_hip(hipMemcpyAsync(g_host_flag, flag, sizeof(int), hipMemcpyDeviceToHost, stream()), "guard flag copy");
-    check_hip(hipStreamSynchronize(stream()), "guard flag sync");
-    last_test_fired = es.failed() || *g_host_flag != 0;
-    return last_test_fired;
+    return test_fired(es, flag);
 }
 
 template <typename TOK>
@@ -248,13 +256,11 @@ static bool tracked_test(const TOK *k, const float *alpha, const float *theta, c
                          bool has_s, int seq_len, int batch, int chunk_size, float error_clip, float m_norm_max,
                          float split_slack, int hd) {
     const ErrorScope es;
-    int *flag = reinterpret_cast<int *>(scratch(31, 256));
-    if (!g_host_flag) check_hip(hipHostMalloc(reinterpret_cast<void **>(&g_host_flag), 256, hipHostMallocDefault), "hipHostMalloc");
-    if (es.failed() || !g_host_flag) return true;
+    int *flag = lowered_flag();
+    if (es.failed() || !flag) return true;
     const int nc = (seq_len + chunk_size - 1) / chunk_size, nchunks = batch * nc;
     {
         KernelTimer kt("cw_guard_tracks_kernel");
-        hipLaunchKernelGGL(guard_clear_kernel, dim3(1), dim3(1), 0, stream(), flag);
         const dim3 grid((unsigned)((nchunks + 3) / 4));
         if (has_s)
             hipLaunchKernelGGL((cw_guard_tracks_kernel<TOK, true>), grid, dim3(256), 0, stream(), k, alpha, theta, eta, tr.e2,
@@ -264,11 +270,7 @@ static bool tracked_test(const TOK *k, const float *alpha, const float *theta, c
                                tr.nrm, seq_len, chunk_size, nc, nchunks, error_clip, m_norm_max, split_slack, hd, flag);
         check_launch("cw_guard_tracks_kernel");
     }
-    *g_host_flag = 1;
-    check_hip(hipMemcpyAsync(g_host_flag, flag, sizeof(int), hipMemcpyDeviceToHost, stream()), "guard flag copy");
-    check_hip(hipStreamSynchronize(stream()), "guard flag sync");
-    last_test_fired = es.failed() || *g_host_flag != 0;
-    return last_test_fired;
+    return test_fired(es, flag);
 }
 
 ChainTracks chain_tracks(int seq_len, int batch, int chunk_size) {

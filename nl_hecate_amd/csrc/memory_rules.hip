@@ -692,7 +692,7 @@ static bool launch_fwd_as(FwdArgs a, int d, int batch, bool coupled) {
 // The Frobenius projection couples the rows of a chain only at the tokens where it fires.  With a bound and no
 // error clip, the uncoupled kernels run first and keep an upper bound of max_t |M_t|_F^2 per workgroup; when the
 // bound stays below m_norm_max^2 no projection could have fired and their results are the coupled kernels' (one
-// 4-byte read-back and a stream synchronisation decide); otherwise the coupled kernels run and overwrite everything.
+// stream synchronisation and a flag in pinned memory decide); otherwise the coupled kernels run and overwrite everything.
 // Few long chains leave the sequential walk's chip idle: where it pays the uncoupled kernels run over independent runs of
 // every chain, from chunk-start states by the matrix form's scan (exact_mm.h).  tracked_rows: leave the bound's partial
 // maxima in scratch 23, that many rows of them.
