@@ -276,13 +276,10 @@ __global__ __launch_bounds__(256, 3) void swa_fwd_stats_kernel(const unsigned sh
 
 // Forward of the contract (normalised weights stored) in the same blocks: the weights need the final maximum
 // and sum, so the window is swept twice — scores and running statistics first, then scores again, the weights
-// w = bf16(exp2(s c - m) / sum) to their slot rows (eight consecutive slots per lane and pair of tiles: 16-byte stores at
+// w = bf16(exp2(s c - m) / sum) to their slot rows (four consecutive slots per lane and tile: 8-byte stores at
 // 2-byte alignment) and O^T += V^T w^T.  Slots behind an early query's own key (t < window - 1) are zeroed at
-// the end.  8 x 4096 tokens, 8 heads, window 512: 0.21 ms, 0.14 of them without the stores, 0.18 with stores at 8-byte alignment.
-// Where a stage's key (0..63) goes, so that two tiles leave a lane group g eight consecutive keys, 32 hf + 8 g + 4 c + i in row
-// 4 g + i of tile 2 hf + c: the weights of a query then move 16 bytes a lane, 64 side by side.
-__device__ __forceinline__ int stage_row(int key) { return (key & 32) + 16 * ((key >> 2) & 1) + 4 * ((key >> 3) & 3) + (key & 3); }
-
+// the end.  8 x 4096 tokens, 8 heads, window 512: 0.21 ms, 0.14 of them without the stores.  A lane's own maximum and sum,
+// joined at the end, and 16-byte stores from stages permuted by stage_row took the same 0.21 ms and other bf16 neighbours.
 template <int HDV>
 __global__ __launch_bounds__(256, 3) void swa_fwd_blocked_kernel(const unsigned short *__restrict__ q,
                                                               const unsigned short *__restrict__ k,
@@ -332,14 +329,14 @@ __global__ __launch_bounds__(256, 3) void swa_fwd_blocked_kernel(const unsigned 
                 for (int qt = 0; qt < 2; qt++)
 #pragma unroll
                     for (int i = 0; i < 4; i++) {
-                        const int key = k0 + 32 * (kt >> 1) + 8 * g + 4 * (kt & 1) + i, tq = qlo + 16 * qt + r;
+                        const int key = k0 + 16 * kt + 4 * g + i, tq = qlo + 16 * qt + r;
                         const bool ok = key <= tq && key >= tq + 1 - ws && tq < s;
                         sc[kt][qt][i] = ok ? sc[kt][qt][i] : -INFINITY;
                     }
         }
     };
 
-    // ---- sweep 1: running maximum and sum, each lane over its own keys; the four lanes of a query meet at the end ----
+    // ---- sweep 1: running maximum and sum ----
     float mrun[2] = {-INFINITY, -INFINITY}, lsum[2] = {0.f, 0.f};
     uint4 kreg[2], vreg[2];
     load_rows<HDV>(km, KS * st_lo, kreg);
@@ -348,7 +345,7 @@ __global__ __launch_bounds__(256, 3) void swa_fwd_blocked_kernel(const unsigned 
 #pragma unroll
         for (int c = 0; c < 2; c++) {
             const int chunk = tid + 256 * c;
-            *reinterpret_cast<uint4 *>(&Ks[buf][stage_row(chunk >> 3)][8 * (chunk & 7)]) = kreg[c];
+            *reinterpret_cast<uint4 *>(&Ks[buf][chunk >> 3][8 * (chunk & 7)]) = kreg[c];
         }
         __syncthreads();
         if (st < st_hi) load_rows<HDV>(km, k0 + KS, kreg);
@@ -362,6 +359,8 @@ __global__ __launch_bounds__(256, 3) void swa_fwd_blocked_kernel(const unsigned 
             for (int kt = 0; kt < 4; kt++)
 #pragma unroll
                 for (int i = 0; i < 4; i++) mx = fmaxf(mx, sc[kt][qt][i]);
+            mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+            mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
             const float mnew = fmaxf(mrun[qt], mx * c2);
             const float mref = mnew == -INFINITY ? 0.f : mnew;
             const float alpha = __builtin_amdgcn_exp2f(mrun[qt] - mref);
@@ -377,12 +376,11 @@ __global__ __launch_bounds__(256, 3) void swa_fwd_blocked_kernel(const unsigned 
     float mc[2], inv[2];
 #pragma unroll
     for (int qt = 0; qt < 2; qt++) {
-        const float m = groups_max(mrun[qt]);
-        mc[qt] = m == -INFINITY ? 0.f : m;
-        float sum = lsum[qt] * __builtin_amdgcn_exp2f(mrun[qt] - mc[qt]);
+        float sum = lsum[qt];
         sum += __shfl_xor(sum, 16, 64);
         sum += __shfl_xor(sum, 32, 64);
         inv[qt] = sum > 0.f ? 1.0f / sum : 0.f;
+        mc[qt] = mrun[qt] == -INFINITY ? 0.f : mrun[qt];
     }
 
     // ---- sweep 2: weights out, O^T = V^T w^T ----
@@ -407,8 +405,8 @@ __global__ __launch_bounds__(256, 3) void swa_fwd_blocked_kernel(const unsigned 
 #pragma unroll
         for (int c = 0; c < 2; c++) {
             const int chunk = tid + 256 * c;
-            *reinterpret_cast<uint4 *>(&Ks[buf][stage_row(chunk >> 3)][8 * (chunk & 7)]) = kreg[c];
-            *reinterpret_cast<uint4 *>(&Vs[buf][stage_row(chunk >> 3)][8 * (chunk & 7)]) = vreg[c];
+            *reinterpret_cast<uint4 *>(&Ks[buf][chunk >> 3][8 * (chunk & 7)]) = kreg[c];
+            *reinterpret_cast<uint4 *>(&Vs[buf][chunk >> 3][8 * (chunk & 7)]) = vreg[c];
         }
         __syncthreads();
         if (st < st_hi) {
@@ -433,20 +431,21 @@ __global__ __launch_bounds__(256, 3) void swa_fwd_blocked_kernel(const unsigned 
                     for (int i = 0; i < 4; i++) w[i] = __builtin_amdgcn_exp2f(fmaf(x[i], c2, -mc[qt])) * inv[qt];
                     wp[c][0] = pack2(w[0], w[1]);
                     wp[c][1] = pack2(w[2], w[3]);
-                }
-                pb[qt] = make_uint4(wp[0][0], wp[0][1], wp[1][0], wp[1][1]);
-                // keys key0 .. key0 + 7 of query tq sit in slots key0 - lsq ..; only keys of the window have one
-                const int key0 = k0 + 32 * hf + 8 * g;
-                if (tq < s) {
-                    if (key0 >= lsq[qt] && key0 + 7 <= tq) {
-                        __builtin_memcpy(wrow[qt] + (key0 - lsq[qt]), &pb[qt], 16);
-                    } else if (key0 + 7 >= lsq[qt] && key0 <= tq) {
+                    // keys key0 .. key0 + 3 of query tq sit in slots key0 - lsq ..; only keys of the window have one
+                    const int key0 = k0 + 16 * (2 * hf + c) + 4 * g;
+                    if (tq < s) {
+                        if (key0 >= lsq[qt] && key0 + 3 <= tq) {
+                            const uint2 pr = make_uint2(wp[c][0], wp[c][1]);
+                            __builtin_memcpy(wrow[qt] + (key0 - lsq[qt]), &pr, 8);
+                        } else if (key0 + 3 >= lsq[qt] && key0 <= tq) {
 #pragma unroll
-                        for (int i = 0; i < 8; i++)
-                            if (key0 + i >= lsq[qt] && key0 + i <= tq)
-                                wrow[qt][key0 + i - lsq[qt]] = (unsigned short)(wp[i >> 2][(i >> 1) & 1] >> (16 * (i & 1)));
+                            for (int i = 0; i < 4; i++)
+                                if (key0 + i >= lsq[qt] && key0 + i <= tq)
+                                    wrow[qt][key0 + i - lsq[qt]] = (unsigned short)(wp[c][i >> 1] >> (16 * (i & 1)));
+                        }
                     }
                 }
+                pb[qt] = make_uint4(wp[0][0], wp[0][1], wp[1][0], wp[1][1]);
             }
 #pragma unroll
             for (int dt = 0; dt < NDT; dt++) {
@@ -628,6 +627,10 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_q_stats_kernel(const unsigned 
         }
     }
 }
+
+// Where a stage's key (0..63) goes, so that two tiles leave a lane group g eight consecutive keys, 32 hf + 8 g + 4 c + i in row
+// 4 g + i of tile 2 hf + c: the weights of a query are then read 16 bytes a lane, 64 side by side.
+__device__ __forceinline__ int stage_row(int key) { return (key & 32) + 16 * ((key >> 2) & 1) + 4 * ((key >> 3) & 3) + (key & 3); }
 
 // Query pass of the contract (weights read back from the tensor) in the same blocks and the same single sweep as
 // swa_bwd_q_stats_kernel: A = sum_j (w dW) k_j, B = sum_j w k_j and D = sum_j w dW together, d_q = (A - D B)/sqrt(hd).

@@ -2,6 +2,8 @@
 CPU oracle.  bf16 path: relative 2e-2; with identical stored weights the
 backward agrees to fp32 round-off (1e-4).  The reference's own bounds are
 absolute 1e-2 forward / 5e-2 backward (core/tests/test_cuda_swa.rs:100,325)."""
+import hashlib
+
 import numpy as np
 import pytest
 import torch
@@ -92,6 +94,17 @@ def test_weights_at_the_ends_of_the_window_and_of_the_tensor(s, ws, hd):
     for n, g, w in zip(("d_q", "d_k", "d_v"), gpu_backward(q, k, v, bad, go, ws, H, 0), want):
         for b, h in ((0, 0), (1, 1)):
             close(n, g[b, :, h * hd:(h + 1) * hd], w[b, :, h * hd:(h + 1) * hd])
+
+
+@pytest.mark.parametrize("B,s,H,hd,ws,out_sha,weights_sha", [
+    (2, 200, 2, 64, 101, "39254ebcd0a0b1f8", "dcebf74d717c1b4a"), (1, 130, 4, 32, 64, "648ca9851ced95a6", "6e7b503d0744f92d"),
+    (1, 600, 2, 32, 512, "e8ca654e090d2dec", "0835120c6c18c666"), (1, 1100, 1, 64, 300, "8e4477cb35da8df1", "9bb869c3df3355f5")])
+def test_forward_keeps_its_order_of_sums(B, s, H, hd, ws, out_sha, weights_sha):
+    """Weights and output bit for bit.  Another order of the sums rounds some of them to the neighbouring bf16 value, and the
+    gradient of a single bias of the whole model, a sum that can cancel to 1e-6 of its terms, then moves by a fifth."""
+    q, k, v, _ = _case(B, s, H, hd, s)
+    out, aw = gpu_forward(q, k, v, ws, H, 0)
+    assert [hashlib.sha256(x.tobytes()).hexdigest()[:16] for x in (out, aw)] == [out_sha, weights_sha]
 
 
 def test_swa_known_answers_on_gpu():
