@@ -26,6 +26,7 @@
 #include "lane_ops.h"
 #include "runtime.h"
 #include "swa_mfma.h"
+#include "swa_pieces.h"
 
 namespace nlh {
 namespace {
@@ -62,10 +63,6 @@ __device__ __forceinline__ float groups_max(float x) {
 // mask of elements e (low half) and e + 1 of those numbered first .. last
 __device__ __forceinline__ unsigned own_pair(int e, int first, int last) {
     return (e >= first && e <= last ? 0xffffu : 0u) | (e + 1 >= first && e + 1 <= last ? 0xffff0000u : 0u);
-}
-// Whether eight slots from `slot` on of query t's row, some of them the row's own, lie inside a head of s rows of ws slots.
-__device__ __forceinline__ bool piece_inside(int t, int s, int ws, int slot) {
-    return min(t, 8) * ws + slot >= 0 && (min(s - 1 - t, 8) + 1) * ws - slot >= 8;
 }
 // x, y = hi + lo with hi, lo bf16: the pair carries 16 mantissa bits through a bf16 product
 __device__ __forceinline__ void split2(float x, float y, unsigned &hi, unsigned &lo) {
@@ -689,7 +686,7 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_q_blocked_kernel(const unsigne
     // a piece is read whole as well, out of the rows next to it, and what is not the query's own is taken off where the piece
     // is used: not here, where that would wait for the read.
     uint4 wreg[2][2];
-    const bool outer_head = b * H + h == 0 || b * H + h == (int)(gridDim.y * gridDim.z) - 1;
+    const bool at_edge = edge_head(b * H + h, (int)(gridDim.y * gridDim.z), s, ws);
     auto whole = [&](int k0) { return k0 + KS - 1 <= qlo && k0 >= qhi + 1 - ws && qhi < s; };
     auto fetch_weights = [&](int k0) {
         const bool skip = k0 > qhi || k0 + KS - 1 < qlo + 1 - ws, full = whole(k0);
@@ -704,9 +701,9 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_q_blocked_kernel(const unsigne
                 if (full) {
                     __builtin_memcpy(&wreg[hf][qt], p, 16);
                 } else if (key0 + 7 >= lsq[qt] && key0 <= tqs[qt]) {
-                    if (!outer_head || piece_inside(tqs[qt], s, ws, key0 - lsq[qt])) {
+                    if (!at_edge || piece_inside(tqs[qt], s, ws, key0 - lsq[qt])) {
                         __builtin_memcpy(&wreg[hf][qt], p, 16);
-                    } else {   // the first or the last row of all
+                    } else {   // at the tensor's own ends
                         unsigned d[4] = {0u, 0u, 0u, 0u};
 #pragma unroll
                         for (int e = 0; e < 8; e++) {
@@ -1007,7 +1004,7 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_k_blocked_kernel(const unsigne
     const float *dvb = dvec + (size_t)(b * H + h) * s;
     const float scale = kInvSqrt;
     const unsigned short *awb = attn_w + (size_t)(b * H + h) * s * ws;
-    const bool outer_head = b * H + h == 0 || b * H + h == (int)(gridDim.y * gridDim.z) - 1;
+    const bool at_edge = edge_head(b * H + h, (int)(gridDim.y * gridDim.z), s, ws);
     const StageSrc qm{q, row0, total, hoff, s};
 
     uint4 vf[2][2];
@@ -1047,9 +1044,9 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_k_blocked_kernel(const unsigne
             const int key0 = j0 + 32 * (tid & 3) + 8 * c;
             wreg[c] = make_uint4(0, 0, 0, 0);
             if (key0 + 7 >= lsq && key0 <= thi) {
-                if (!outer_head || piece_inside(t, s, ws, key0 - lsq)) {
+                if (!at_edge || piece_inside(t, s, ws, key0 - lsq)) {
                     __builtin_memcpy(&wreg[c], wrow + (key0 - lsq), 16);
-                } else {   // the first or the last row of all
+                } else {   // at the tensor's own ends
                     unsigned d[4] = {0u, 0u, 0u, 0u};
 #pragma unroll
                     for (int e = 0; e < 8; e++) {
