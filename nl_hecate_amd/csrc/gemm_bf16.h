@@ -12,7 +12,8 @@ struct ProductBf16 {
     int m, n, k, k_first;
     bool a_bf16, b_bf16;
 };
-// Sizes and alignments that these kernels take, and take faster than the library.
+// Sizes, alignments and places (c apart from the operands) that these kernels take, and sizes that they take faster than the
+// library.
 bool product_bf16_serves(const ProductBf16 &p, int op);
 void product_bf16(const ProductBf16 &p, int op);   // scratch slot 30 where the contraction is split
 

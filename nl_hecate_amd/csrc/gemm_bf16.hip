@@ -147,6 +147,17 @@ bool product_bf16_serves(const ProductBf16 &p, int op) {
     // rows along the contiguous dimension and contraction indices along it come eight at a time
     if (p.n % 8 || (op == 2 ? p.m : p.k) % 8 || p.lda % 8 || p.ldb % 8 || (p.b2 && p.k_first % TB)) return false;
     if (!al16(p.a) || !al16(p.b) || !al16(p.b2) || !al16(p.c)) return false;
+    // A result in the place of an operand: the operands are read while the first tiles are stored.  The callers' other path
+    // has its fp32 operands converted into scratch before anything is written.
+    const auto meets = [&](const void *x, long long rows, long long cols, long long ld, bool bf16) {
+        const uintptr_t x0 = (uintptr_t)x, x1 = x0 + ((rows - 1) * ld + cols) * (bf16 ? 2 : 4);
+        const uintptr_t c0 = (uintptr_t)p.c, c1 = c0 + (size_t)p.m * p.n * sizeof(float);
+        return x && x0 < c1 && c0 < x1;
+    };
+    const int kb = p.b2 ? p.k_first : p.k;
+    if (meets(p.a, op == 2 ? p.k : p.m, op == 2 ? p.m : p.k, p.lda, p.a_bf16) ||
+        meets(p.b, op == 0 ? p.n : kb, op == 0 ? p.k : p.n, p.ldb, p.b_bf16) || meets(p.b2, p.k - kb, p.n, p.ldb, p.b_bf16))
+        return false;
     // In a captured graph, us here / library kernel with its conversions (and the library's slabs for op 2):
     //   op 0  d 512 x 512: 2000 rows 8.7 / 10.0, 4000 12.8 / 11.5; 256 x 2304: 1000 8.5 / 12.3, 2000 13 / 13
     //   op 1  256 x 2304: 500 rows 11 / 17, 2000 17 / 24, 4000 35 / 28; 512 x 7680: 500 32 / 39

@@ -265,6 +265,31 @@ def test_linear_pair_at_the_edges_of_its_tiles(n, d_in, d_out):
         assert (np.abs(host(got) - x @ y) <= 2 ** -24 * (k + 4) * (np.abs(x) @ np.abs(y)) + 1e-30).all(), (n, d_in, d_out, k)
 
 
+@pytest.mark.parametrize("place", ["d_a over d_out", "d_w over w", "d_w over d_out", "d_a over w", "out over w", "d_a behind the start of d_out"])
+def test_linear_pair_in_place(place):
+    """A result in the place of an fp32 operand is the one in a place of its own: operands are rounded before it is written."""
+    n = d = 512
+    r = np.random.default_rng(8)
+    ta = torch.from_numpy(r.standard_normal((n, d)).astype(np.float32)).to(BF).cuda()
+    room = torch.zeros(2 * n * d, device="cuda")
+    tg, tw = room[:n * d].view(n, d), dev(r.standard_normal((d, d)).astype(np.float32))
+    tg.copy_(torch.from_numpy(r.standard_normal((n, d)).astype(np.float32)))
+    a, w, g = host(ta.float()), bf16_round(host(tw)), bf16_round(host(tg))
+    new = lambda: torch.full((n, d), 7.5, device="cuda")
+    out, d_a, d_w = new(), new(), new()
+    if place == "out over w":
+        out = tw
+        lib.linear_forward_bf16_rocm(ta.data_ptr(), tw.data_ptr(), out.data_ptr(), n, d, d)
+        got = [(out, a, w.T)]
+    else:
+        d_a = dict([("d_a over d_out", tg), ("d_a over w", tw), ("d_a behind the start of d_out", room[8 * d:8 * d + n * d].view(n, d))]).get(place, d_a)
+        d_w = {"d_w over w": tw, "d_w over d_out": tg}.get(place, d_w)
+        lib.linear_backward_bf16_rocm(tg.data_ptr(), ta.data_ptr(), tw.data_ptr(), d_a.data_ptr(), d_w.data_ptr(), n, d, d)
+        got = [(d_a, g, w), (d_w, g.T, a)]
+    for t, x, y in got:
+        assert (np.abs(host(t) - x @ y) <= 2 ** -24 * (n + 4) * (np.abs(x) @ np.abs(y))).all()
+
+
 @pytest.mark.parametrize("n_extra,levels", [(3, 2), (1, 1), (2, 0), (0, 3)])
 def test_projections_shared_out_are_those_of_one_workgroup(n_extra, levels):
     """128 tokens share out the projections over workgroups, the same tokens repeated until they fill the chip do not: the
