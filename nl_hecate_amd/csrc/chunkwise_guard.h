@@ -1,7 +1,7 @@
 // Device-side test of whether the error clip or the Frobenius projection of the reference's chunkwise kernels
-// can fire for a call, given the chunk-start states (chunkwise_guard.hip).  Costs one chunk-parallel kernel, a
-// 4-byte copy to the host and a synchronisation of the launch stream (the reference's chunkwise wrappers
-// synchronise the device themselves); not available while the launch stream is being captured.
+// can fire for a call, given the chunk-start states (chunkwise_guard.hip).  Costs one chunk-parallel kernel and a
+// synchronisation of the launch stream (the reference's chunkwise wrappers synchronise the device themselves);
+// not available while the launch stream is being captured.
 #pragma once
 #include <stdint.h>
 

@@ -15,11 +15,10 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-#include <atomic>
-
 #include "../../include/nl_hecate_ffi.h"
 #include "chunkwise_chain.h"
 #include "chunkwise_guard.h"
+#include "guard_flags.h"
 #include "lane_ops.h"
 #include "mm_tiles.h"
 #include "runtime.h"
@@ -57,7 +56,7 @@ __global__ __launch_bounds__(kThr) void cw_guard_kernel(const TOK *__restrict__ 
                                                         const float *__restrict__ alpha, const float *__restrict__ theta,
                                                         const float *__restrict__ eta, const float *__restrict__ m_states,
                                                         const float *__restrict__ s_states, int seq_len, int C, int nc,
-                                                        float clip, float mmax, int *__restrict__ flag) {
+                                                        float clip, float mmax, GuardFlag *__restrict__ flag) {
     __shared__ float Ks[MAT], Ms[MAT];
     __shared__ float en2[2][CW], kn2[CW], red[2][8];
     const int tid = threadIdx.x, chunk = blockIdx.x % nc, chain = blockIdx.x / nc;
@@ -126,7 +125,8 @@ __global__ __launch_bounds__(kThr) void cw_guard_kernel(const TOK *__restrict__ 
             worst = t < L ? fmaxf(worst, nM) : worst;
         }
         if (proj_on && worst * kSlack > mmax) bad = true;
-        if (bad) *flag = 1;
+        if (blockIdx.x == 0 && tid == 0) flag->reached = 1;
+        if (bad) flag->fired = 1;
     }
 }
 
@@ -139,7 +139,7 @@ __global__ __launch_bounds__(256) void cw_guard_tracks_kernel(const TOK *__restr
                                                               const float *__restrict__ theta, const float *__restrict__ eta,
                                                               const float *__restrict__ e2, const float *__restrict__ nrm,
                                                               int seq_len, int C, int nc, int nchunks, float clip, float mmax,
-                                                              float split_slack, int hd, int *__restrict__ flag) {
+                                                              float split_slack, int hd, GuardFlag *__restrict__ flag) {
     const int lane = threadIdx.x & 63, task = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (task >= nchunks) return;   // waves are independent: no barrier below
     const int chain = task / nc, c = task % nc, t0 = c * C, L = min(C, seq_len - t0);
@@ -174,27 +174,24 @@ __global__ __launch_bounds__(256) void cw_guard_tracks_kernel(const TOK *__restr
         worst = t < L ? fmaxf(worst, nM) : worst;
     }
     if (proj_on && worst * kSlack > mmax) bad = true;
-    if (bad) *flag = 1;
+    if (blockIdx.x == 0 && threadIdx.x == 0) flag->reached = 1;
+    if (bad) flag->fired = 1;
 }
 
-// The flag of a test stands in pinned host memory, where a kernel stores to it only if the test fires: a flag on the device
-// took a launch to clear and a copy to read (32 chains x 1500 tokens, float, bounded, forward and backward 333 -> 320 us).
-constexpr int kFlags = 64;   // in turn: tests of several threads do not share one
-int *g_host_flags = nullptr;
-std::atomic<unsigned> g_next_flag{0};
-
-int *lowered_flag() {
-    if (!g_host_flags)
-        check_hip(hipHostMalloc(reinterpret_cast<void **>(&g_host_flags), kFlags * sizeof(int), hipHostMallocDefault), "hipHostMalloc");
-    if (!g_host_flags) return nullptr;
-    int *flag = g_host_flags + g_next_flag++ % kFlags;
-    *(volatile int *)flag = 0;
-    return flag;
+// The flag of a test stands in pinned host memory, where a kernel stores a word, and another if the test fires: a flag on the
+// device took a launch to clear and a copy to read (32 chains x 1500 tokens, float, bounded, forward and backward 333 -> 320 us).
+GuardFlag *lowered_flag() {
+    static GuardFlags<64> flags;
+    return flags.lowered([](size_t bytes) {
+        void *p = nullptr;
+        check_hip(hipHostMalloc(&p, bytes, hipHostMallocDefault), "hipHostMalloc");
+        return p;
+    });
 }
 
-bool test_fired(const ErrorScope &es, const int *flag) {
+bool test_fired(const ErrorScope &es, const GuardFlag *flag) {
     check_hip(hipStreamSynchronize(stream()), "guard flag sync");
-    last_test_fired = es.failed() || *(const volatile int *)flag != 0;
+    last_test_fired = es.failed() || !guard_clear(flag);
     return last_test_fired;
 }
 
@@ -211,7 +208,7 @@ static bool couplings_may_fire_t(const TOK *k, const TOK *v, const float *alpha,
                                  const float *m_states, const float *s_states, int seq_len, int batch, int chunk_size,
                                  float error_clip, float m_norm_max) {
     const ErrorScope es;
-    int *flag = lowered_flag();
+    GuardFlag *flag = lowered_flag();
     if (es.failed() || !flag) return true;
     const int nc = (seq_len + chunk_size - 1) / chunk_size;
     {
@@ -229,18 +226,19 @@ static bool couplings_may_fire_t(const TOK *k, const TOK *v, const float *alpha,
 }
 
 namespace {
-__global__ void norm_bound_kernel(const float *__restrict__ msq_part, int batch, int parts, float limit_sq, int *flag) {
+__global__ void norm_bound_kernel(const float *__restrict__ msq_part, int batch, int parts, float limit_sq, GuardFlag *flag) {
     const int b = blockIdx.x * blockDim.x + threadIdx.x;
     if (b >= batch) return;
     float tot = 0.f;
     for (int p = 0; p < parts; p++) tot += msq_part[b * parts + p];
-    if (!(tot * (1.0f + 1e-3f) <= limit_sq)) *flag = 1;   // also raised by a NaN
+    if (b == 0) flag->reached = 1;
+    if (!(tot * (1.0f + 1e-3f) <= limit_sq)) flag->fired = 1;   // also raised by a NaN
 }
 }  // namespace
 
 bool norm_bound_exceeded(const float *msq_part, int batch, int parts, float m_norm_max) {
     const ErrorScope es;
-    int *flag = lowered_flag();
+    GuardFlag *flag = lowered_flag();
     if (es.failed() || !flag) return true;
     {
         KernelTimer kt("norm_bound_kernel");
@@ -256,7 +254,7 @@ static bool tracked_test(const TOK *k, const float *alpha, const float *theta, c
                          bool has_s, int seq_len, int batch, int chunk_size, float error_clip, float m_norm_max,
                          float split_slack, int hd) {
     const ErrorScope es;
-    int *flag = lowered_flag();
+    GuardFlag *flag = lowered_flag();
     if (es.failed() || !flag) return true;
     const int nc = (seq_len + chunk_size - 1) / chunk_size, nchunks = batch * nc;
     {
