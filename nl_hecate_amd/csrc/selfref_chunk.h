@@ -7,7 +7,6 @@ namespace nlh {
 
 constexpr int kTB = 16;  // tokens staged in LDS at a time
 using f32x4 = float __attribute__((ext_vector_type(4)));
-using f64x4 = double __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
@@ -15,16 +14,11 @@ __device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) {
 __device__ __forceinline__ float lane_from(int byte_addr, float x) {
     return __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(byte_addr, __builtin_bit_cast(int, x)));
 }
-__device__ __forceinline__ double lane_from64(int byte_addr, double x) {
-    const long long u = __builtin_bit_cast(long long, x);
-    const unsigned lo = __builtin_amdgcn_ds_bpermute(byte_addr, (int)u), hi = __builtin_amdgcn_ds_bpermute(byte_addr, (int)(u >> 32));
-    return __builtin_bit_cast(double, (long long)(((unsigned long long)hi << 32) | lo));
-}
 __device__ __forceinline__ float lane_value(float x, int lane) {
     return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), lane));
 }
 // The order in which a tile's 16 tokens are rows of a matrix product: result row 4 kg + v is token 4 v + kg.  Its own
-// inverse, and the order in which the float64 instruction deals out its result rows.
+// inverse.
 __host__ __device__ constexpr int sigma(int t) { return 4 * (t & 3) + (t >> 2); }
 
 // core/src/tensor.rs:202-207, 221-227.  The gates sit on the per-token critical path of the forward,
