@@ -27,7 +27,8 @@ PyObject *tensor_key(PyObject *, PyObject *tensors) {
             }
             const at::Tensor &t = THPVariable_Unpack(item);
             key.push_back((int64_t)(intptr_t)t.data_ptr());
-            key.push_back((int64_t)t.scalar_type() | (int64_t)t.device().type() << 8 | (int64_t)t.device().index() << 16 |
+            // a tensor without a device index has -1
+            key.push_back((int64_t)t.scalar_type() | (int64_t)t.device().type() << 8 | (int64_t)(uint8_t)t.device().index() << 16 |
                           t.dim() << 32);
             for (const int64_t v : t.sizes()) key.push_back(v);
             for (const int64_t v : t.strides()) key.push_back(v);

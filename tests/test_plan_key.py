@@ -2,6 +2,7 @@
 import os
 import subprocess
 
+import numpy as np
 import pytest
 import torch
 
@@ -32,6 +33,13 @@ def test_key_of_a_tensor_that_changed_where_it_stands(change):
     elif change == "view":
         t = t[1:]
     assert (before == ffi.tensor_key([t, other])) == (change in ("nothing", "values"))
+
+
+@pytest.mark.parametrize("shape", [(), (4,), (2, 3), (2, 0, 5)])
+def test_key_says_how_many_sizes_follow(shape):
+    """Type, device and rank share a word; the -1 that stands for the device index of a CPU tensor is not to cover the rank."""
+    words = np.frombuffer(ffi.tensor_key([torch.zeros(shape)]), np.int64)
+    assert len(words) == 2 + 2 * len(shape) and words[1] >> 32 == len(shape)
 
 
 def test_key_of_what_has_no_address():
