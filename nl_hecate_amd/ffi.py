@@ -9,6 +9,7 @@ import ctypes
 import importlib.util
 import os
 import re
+import warnings
 
 _PKG = os.path.dirname(os.path.abspath(__file__))
 HEADER = os.path.join(os.path.dirname(_PKG), "include", "nl_hecate_ffi.h")
@@ -83,14 +84,24 @@ class _Lib:
 lib = _Lib()
 
 
+def _python_key(tensors):
+    """tensor_key without the extension: what it reads, by Python calls, four a tensor."""
+    import torch
+    return repr([(torch.Tensor.data_ptr(t), t.dtype, t.device, torch.Tensor.size(t), torch.Tensor.stride(t))
+                 for t in tensors]).encode() if tensors else b""
+
+
 def tensor_key(tensors):
     """Address, type, device, sizes and strides of every tensor as one bytes object (csrc/plan_key.cpp).  The first call
-    puts the compiled function in this one's place."""
+    puts the compiled function in this one's place, or where only the library was built, or the extension for another torch,
+    one that takes 15 us more a decode step."""
     global tensor_key
-    if not os.path.exists(KEY_PATH):
-        raise RuntimeError(f"{KEY_PATH} is missing: build it with `make -C nl_hecate_amd/csrc`.")
-    spec = importlib.util.spec_from_file_location("plan_key", KEY_PATH)
-    module = importlib.util.module_from_spec(spec)
-    spec.loader.exec_module(module)
-    tensor_key = module.tensor_key
+    try:
+        spec = importlib.util.spec_from_file_location("plan_key", KEY_PATH)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        tensor_key = module.tensor_key
+    except ImportError as e:
+        warnings.warn(f"{KEY_PATH} cannot be loaded ({e}): decode steps are slower. Build it with `make -C nl_hecate_amd/csrc`.")
+        tensor_key = _python_key
     return tensor_key(tensors)
