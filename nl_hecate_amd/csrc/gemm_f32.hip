@@ -288,17 +288,21 @@ __global__ __launch_bounds__(64 * WM * WN) void group_gemm_kernel(GroupArgs g) {
             for (int j = 0; j < TN; j++) acc[i][j] += sum[i][j];
     }
     const int row0 = m0 + wm + 4 * (l >> 4), col0 = n0 + wn + (l & 15);
-    // Pieces of an infinity, and of what rounds to one, are not numbers: a wave whose results are not all finite forms them
-    // again from the operands as they are.
-    bool finite = true;
+    // Pieces of an infinity, and of what rounds to one, are not numbers, and pieces of a float below 2^-110 end at the last of a
+    // bf16's range, 2^-133, short of its 24 bits: a wave whose results are not all finite, or in part too small to tell that
+    // their operands were not (2^-80, as much as 2^30 above), forms them again from the operands as they are.
+    constexpr uint32_t kSmall = (127 - 80) << 23;
+    bool sound = true;
 #pragma unroll
     for (int i = 0; i < TM; i++)
 #pragma unroll
         for (int j = 0; j < TN; j++)
 #pragma unroll
-            for (int e = 0; e < 4; e++)
-                finite &= (__float_as_uint(acc[i][j][e]) & 0x7f800000u) != 0x7f800000u || row0 + 16 * i + e >= g.m || col0 + 16 * j >= g.n;
-    if (__any(!finite)) {
+            for (int e = 0; e < 4; e++) {
+                const uint32_t u = __float_as_uint(acc[i][j][e]) & 0x7fffffffu;
+                sound &= u - kSmall < 0x7f800000u - kSmall || u == 0 || row0 + 16 * i + e >= g.m || col0 + 16 * j >= g.n;
+            }
+    if (__any(!sound)) {
 #pragma unroll
         for (int i = 0; i < TM; i++)
 #pragma unroll

@@ -86,6 +86,28 @@ def test_single_products_keep_non_finite_values_in_their_place(op, m, n, k):
     assert ((c.double() - want)[ok].abs() <= 8 * 2 ** -24 * k * want[ok].abs().clamp(min=1)).all()
 
 
+@pytest.mark.parametrize("op", [0, 1, 2])
+@pytest.mark.parametrize("m,n,k", [(600, 1300, 128), (130, 70, 2000)])
+def test_single_products_of_the_smallest_floats(op, m, n, k):
+    """Operands whose three pieces do not hold all of their bits any more, alone and as one row among others; zeros stay."""
+    g = torch.Generator(device="cuda").manual_seed(6)
+    shp_a, shp_b = {0: ((m, k), (n, k)), 1: ((m, k), (k, n)), 2: ((k, m), (k, n))}[op]
+    a, b = [torch.randn(*s, generator=g, device="cuda") for s in (shp_a, shp_b)]
+    fit = {0: lambda a, b: a @ b.t(), 1: lambda a, b: a @ b, 2: lambda a, b: a.t() @ b}[op]
+    c = torch.zeros(m, n, device="cuda")
+    for scale, scale_b, row in ((2. ** -113, 1., None), (2. ** -120, 1., 5), (2. ** -122, 2. ** 20, None), (2. ** -125, 2. ** 5, m - 1)):
+        x, y = a.clone(), b * scale_b
+        rows = x.t() if op == 2 else x
+        rows[...] = rows * scale if row is None else rows.index_copy(0, torch.tensor([row], device="cuda"), rows[row:row + 1] * scale)
+        rows[7] = 0
+        ML.product(op, x, y, c, m, n, k)
+        want, by_terms = fit(x.double(), y.double()), fit(x, y).double()
+        at = slice(None) if row is None else slice(row, row + 1)
+        # sums term by term like the library's, in another order: as many roundings of sums of the same size, within twice
+        assert (c.double() - want)[at].norm().item() <= 2 * (by_terms - want)[at].norm().item(), (scale, scale_b, row)
+        assert (c[7] == 0).all()
+
+
 @pytest.mark.parametrize("count,m,n,k", [(7, 1000, 1024, 1024), (6, 2000, 512, 512), (12, 512, 512, 512)])
 def test_sum_over_products_rounds_like_products_added_up(count, m, n, k):
     g = torch.Generator(device="cuda").manual_seed(1)
