@@ -292,10 +292,11 @@ def test_linear_pair_in_place(place):
 
 @pytest.mark.parametrize("n_extra,levels", [(3, 2), (1, 1), (2, 0), (0, 3)])
 def test_projections_shared_out_are_those_of_one_workgroup(n_extra, levels):
-    """128 tokens share out the projections over workgroups, the same tokens repeated until they fill the chip do not: the
-    same numbers."""
+    """128 tokens share out the projections over workgroups, the same tokens repeated until there is a tile of 128 for every
+    compute unit do not (two parts would be two rounds of at least half the projections and another staging): the same
+    numbers."""
     nh, s = 4, 128
-    d, many = nh * 64, 300
+    d, many = nh * 64, torch.cuda.get_device_properties(0).multi_processor_count
     x, w_extra, w_levels, gates = make_inputs(1, s, nh, levels, n_extra, 5)
     params = [dev(g[k]) for g in gates for k in GATE_NAMES]
     res = []
