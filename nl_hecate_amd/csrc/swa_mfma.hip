@@ -23,6 +23,8 @@
 #include <math.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "lane_ops.h"
 #include "runtime.h"
 #include "swa_mfma.h"
@@ -474,6 +476,58 @@ __global__ __launch_bounds__(256, 3) void swa_fwd_blocked_kernel(const unsigned 
     }
 }
 
+// The backward passes of a call that leaves the chip idle (SPLIT): bound by one wave's chain of stages, so a workgroup has 32
+// queries (keys) instead of 128, its four waves share out the window instead of the rows (two stages at a time, half a stage
+// each), and their sums are joined at the end.  What a workgroup stages then serves a quarter of the rows: taken while
+// the four times as many workgroups still fit the chip at once, two a compute unit.  Both passes, contract / statistics, us
+// before and after, head size 64, window 512: 32 blocks of 128 rows 46 -> 21 / 60 -> 28, 112 blocks 58 -> 35 / 73 -> 42;
+// where they do not fit, 192 blocks 63 -> 62 or 75, 256 blocks (window 256) 46 -> 52, 512 blocks 92 -> 131.
+constexpr int SQ = 32;     // queries (keys) per workgroup of these
+// tile (t, dt) of the joined sums stays with one wave
+template <int NDT, bool SPLIT>
+__device__ __forceinline__ bool own_tile(int t, int dt, int wave) { return !SPLIT || wave == 2 * t + dt / (NDT / 2); }
+// x, y: sums of the four waves over their own keys; afterwards a wave has the whole sums of its own tiles.  buf: the stages,
+// room for 16 KB a wave.
+template <int NDT>
+__device__ __forceinline__ void join_waves(f32x4 (&x)[2][4], f32x4 (&y)[2][4], float *buf, int wave, int l) {
+    f32x4 *m = reinterpret_cast<f32x4 *>(buf) + l;
+    constexpr int N = NDT / 2;   // tiles of x (and of y) that a wave ends up with
+    __syncthreads();             // the stages are read
+#pragma unroll
+    for (int o = 0; o < 4; o++) {
+        if (o == wave) continue;
+        const int from = (wave - o - 1) & 3;   // 0 .. 2
+#pragma unroll
+        for (int e = 0; e < N; e++) {
+            m[((o * 3 + from) * 2 * N + 2 * e) * 64] = x[o >> 1][(o & 1) * N + e];
+            m[((o * 3 + from) * 2 * N + 2 * e + 1) * 64] = y[o >> 1][(o & 1) * N + e];
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int o = 0; o < 4; o++) {
+        if (o != wave) continue;
+#pragma unroll
+        for (int e = 0; e < N; e++) {
+            f32x4 &a = x[o >> 1][(o & 1) * N + e], &c = y[o >> 1][(o & 1) * N + e];
+            const f32x4 *p = m + (o * 3 * 2 * N + 2 * e) * 64, *q = p + 64;
+            a = (a + p[0]) + (p[2 * N * 64] + p[4 * N * 64]);
+            c = (c + q[0]) + (q[2 * N * 64] + q[4 * N * 64]);
+        }
+    }
+}
+__device__ __forceinline__ void join_waves(float (&x)[2], float *buf, int wave, int l) {
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < 2; e++) buf[(e * 4 + wave) * 64 + l] = x[e];
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < 2; e++) {
+        const float *p = buf + e * 256 + l;
+        x[e] = (p[0] + p[64]) + (p[128] + p[192]);
+    }
+}
+
 // Query pass on statistics, in key blocks like swa_fwd_stats_kernel (one workgroup per 128 queries, one wave per
 // 32), in ONE sweep over the window.  dS = w (dW - D) needs D_t = sum_j w dW of the whole window, so the sweep
 // accumulates the two sums that do not:  A^T = K^T (w dW)^T and B^T = K^T w^T, and D itself, and ends with
@@ -483,7 +537,7 @@ __global__ __launch_bounds__(256, 3) void swa_fwd_blocked_kernel(const unsigned 
 // Per stage a wave forms S^T = K Q^T, the weights w = bf16(exp2(s c - m) / sum) as the weight tensor would hold
 // them, dW^T = V dO^T; dO and w dW enter as hi + lo pairs, w is exact in bf16.  K^T is read from the K rows
 // through ds_read_b64_tr_b16 in the key order that the score tiles leave in the lanes.  D goes to dvec.
-template <int HDV, bool OUT16>
+template <int HDV, bool OUT16, bool SPLIT>
 __global__ __launch_bounds__(256, 2) void swa_bwd_q_stats_kernel(const unsigned short *__restrict__ q,
                                                                  const unsigned short *__restrict__ k,
                                                                  const unsigned short *__restrict__ v,
@@ -491,16 +545,17 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_q_stats_kernel(const unsigned 
                                                                  const float *__restrict__ d_out,
                                                                  float *__restrict__ d_q, float *__restrict__ dvec,
                                                                  int s, int H, int ws, Out16 o16) {
-    __shared__ __align__(16) unsigned short Ks[2][KS][LDH], Vs[2][KS][LDH];   // stages [key][dim]
+    __shared__ __align__(16) unsigned short KV[SPLIT ? 5 : 4][KS][LDH];   // two stages [key][dim] of K, then of V
+    unsigned short (*const Ks)[KS][LDH] = KV, (*const Vs)[KS][LDH] = KV + 2;
     const int tid = threadIdx.x, wave = tid >> 6, l = tid & 63, r = l & 15, g = l >> 4;
     const BlockCoord bc = xcd_block_coord(H);
-    const int t0 = bc.x * FQ, h = bc.h, b = bc.b;
+    const int t0 = bc.x * (SPLIT ? SQ : FQ), h = bc.h, b = bc.b;
     constexpr int NKS = HDV / 32, NDT = HDV / 16;
     constexpr float kInvSqrt = HDV == 64 ? 0.125f : 0.17677669529663687f;   // 1 / sqrt(head size)
     const int total = H * HDV, hoff = h * HDV;
     const size_t row0 = (size_t)b * s;
-    const int qlo = t0 + 32 * wave, qhi = qlo + 31;
-    const int st_lo = max(t0 + 1 - ws, 0) / KS, st_hi = min(t0 + FQ - 1, s - 1) / KS;
+    const int qlo = SPLIT ? t0 : t0 + 32 * wave, qhi = qlo + 31;
+    const int st_lo = max(t0 + 1 - ws, 0) / KS, st_hi = min(t0 + (SPLIT ? SQ : FQ) - 1, s - 1) / KS;
     const StageSrc km{k, row0, total, hoff, s}, vm{v, row0, total, hoff, s};
     const float c2 = kInvSqrt * 1.44269504088896340736f, scale = kInvSqrt;
 
@@ -534,26 +589,33 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_q_stats_kernel(const unsigned 
 #pragma unroll
         for (int dt = 0; dt < NDT; dt++) { aq[qt][dt] = f32x4{0.f, 0.f, 0.f, 0.f}; bq[qt][dt] = f32x4{0.f, 0.f, 0.f, 0.f}; }
 
-    uint4 kreg[2], vreg[2];
-    load_rows<HDV>(km, KS * st_lo, kreg);
-    load_rows<HDV>(vm, KS * st_lo, vreg);
-    for (int st = st_lo; st <= st_hi; st++) {
-        const int buf = (st - st_lo) & 1, k0 = KS * st;
+    uint4 kreg[SPLIT ? 2 : 1][2], vreg[SPLIT ? 2 : 1][2];
+    auto fetch_stages = [&](int first) {
 #pragma unroll
-        for (int c = 0; c < 2; c++) {
-            const int chunk = tid + 256 * c;
-            *reinterpret_cast<uint4 *>(&Ks[buf][chunk >> 3][8 * (chunk & 7)]) = kreg[c];
-            *reinterpret_cast<uint4 *>(&Vs[buf][chunk >> 3][8 * (chunk & 7)]) = vreg[c];
+        for (int p = 0; p < (SPLIT ? 2 : 1); p++) {
+            load_rows<HDV>(km, first + KS * p, kreg[p]);
+            load_rows<HDV>(vm, first + KS * p, vreg[p]);
         }
+    };
+    fetch_stages(KS * st_lo);
+    for (int st = st_lo; st <= st_hi; st += SPLIT ? 2 : 1) {
+        const int buf = SPLIT ? wave >> 1 : (st - st_lo) & 1, k0 = KS * (SPLIT ? st + buf : st);
+        if (SPLIT && st > st_lo) __syncthreads();   // both stages are read
+#pragma unroll
+        for (int p = 0; p < (SPLIT ? 2 : 1); p++)
+#pragma unroll
+            for (int c = 0; c < 2; c++) {
+                const int chunk = tid + 256 * c, to = SPLIT ? p : buf;
+                *reinterpret_cast<uint4 *>(&Ks[to][chunk >> 3][8 * (chunk & 7)]) = kreg[p][c];
+                *reinterpret_cast<uint4 *>(&Vs[to][chunk >> 3][8 * (chunk & 7)]) = vreg[p][c];
+            }
         __syncthreads();
-        if (st < st_hi) {
-            load_rows<HDV>(km, k0 + KS, kreg);
-            load_rows<HDV>(vm, k0 + KS, vreg);
-        }
+        if (st + (SPLIT ? 1 : 0) < st_hi) fetch_stages(KS * (st + (SPLIT ? 2 : 1)));
         if (k0 > qhi || k0 + KS - 1 < qlo + 1 - ws) continue;
         const bool full = k0 + KS - 1 <= qlo && k0 >= qhi + 1 - ws && qhi < s;
 #pragma unroll
-        for (int hf = 0; hf < 2; hf++) {
+        for (int half = 0; half < (SPLIT ? 1 : 2); half++) {
+            const int hf = SPLIT ? wave & 1 : half;
             uint4 xh[2], xl[2], wb[2];
 #pragma unroll
             for (int qt = 0; qt < 2; qt++) {
@@ -600,18 +662,25 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_q_stats_kernel(const unsigned 
             }
         }
     }
+    if constexpr (SPLIT) {
+        float *buf = reinterpret_cast<float *>(&Ks[0][0][0]);
+        join_waves<NDT>(aq, bq, buf, wave, l);
+        join_waves(dpart, buf, wave, l);
+    }
 #pragma unroll
     for (int qt = 0; qt < 2; qt++) {
         const int tq = qlo + 16 * qt + r;
+        if (SPLIT && qt != wave >> 1) continue;
         float dsum = dpart[qt];
         dsum += __shfl_xor(dsum, 16, 64);
         dsum += __shfl_xor(dsum, 32, 64);
         if (tq < s) {
-            if (g == 0) dvec[(size_t)(b * H + h) * s + tq] = dsum;
+            if (g == 0 && !(SPLIT && (wave & 1))) dvec[(size_t)(b * H + h) * s + tq] = dsum;
             if (OUT16) {
                 unsigned short *ob = o16.q + (row0 + tq) * o16.ld + hoff;
 #pragma unroll
                 for (int dt = 0; dt < NDT; dt++) {
+                    if (!own_tile<NDT, SPLIT>(qt, dt, wave)) continue;
                     const f32x4 x = (aq[qt][dt] - dsum * bq[qt][dt]) * scale;
                     *reinterpret_cast<uint2 *>(ob + 16 * dt + 4 * g) = make_uint2(pack2(x[0], x[1]), pack2(x[2], x[3]));
                 }
@@ -619,7 +688,8 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_q_stats_kernel(const unsigned 
                 float *ob = d_q + (row0 + tq) * total + hoff;
 #pragma unroll
                 for (int dt = 0; dt < NDT; dt++)
-                    *reinterpret_cast<f32x4 *>(ob + 16 * dt + 4 * g) = (aq[qt][dt] - dsum * bq[qt][dt]) * scale;
+                    if (own_tile<NDT, SPLIT>(qt, dt, wave))
+                        *reinterpret_cast<f32x4 *>(ob + 16 * dt + 4 * g) = (aq[qt][dt] - dsum * bq[qt][dt]) * scale;
             }
         }
     }
@@ -635,23 +705,24 @@ __device__ __forceinline__ int stage_row(int key) { return (key & 32) + 16 * ((k
 // requested a stage ahead.  Bound by the latency of a stage's chain of LDS reads, products and element work on two waves a
 // SIMD (matrix cores 0.16, vector units 0.26, LDS 0.11 of their time).  8 x 4096 tokens, 8 heads, window 512: 210 us (247
 // with 8-byte loads, slot by slot with a wait in every stage at the window's ends); 192 without any loads of weights.
-template <int HDV>
+template <int HDV, bool SPLIT>
 __global__ __launch_bounds__(256, 2) void swa_bwd_q_blocked_kernel(const unsigned short *__restrict__ k,
                                                                    const unsigned short *__restrict__ v,
                                                                    const unsigned short *__restrict__ attn_w,
                                                                    const float *__restrict__ d_out,
                                                                    float *__restrict__ d_q, float *__restrict__ dvec,
                                                                    int s, int H, int ws) {
-    __shared__ __align__(16) unsigned short Ks[2][KS][LDH], Vs[2][KS][LDH];   // stages [key][dim]
+    __shared__ __align__(16) unsigned short KV[SPLIT ? 5 : 4][KS][LDH];   // two stages [key][dim] of K, then of V
+    unsigned short (*const Ks)[KS][LDH] = KV, (*const Vs)[KS][LDH] = KV + 2;
     const int tid = threadIdx.x, wave = tid >> 6, l = tid & 63, r = l & 15, g = l >> 4;
     const BlockCoord bc = xcd_block_coord(H);
-    const int t0 = bc.x * FQ, h = bc.h, b = bc.b;
+    const int t0 = bc.x * (SPLIT ? SQ : FQ), h = bc.h, b = bc.b;
     constexpr int NKS = HDV / 32, NDT = HDV / 16;
     constexpr float kInvSqrt = HDV == 64 ? 0.125f : 0.17677669529663687f;   // 1 / sqrt(head size)
     const int total = H * HDV, hoff = h * HDV;
     const size_t row0 = (size_t)b * s;
-    const int qlo = t0 + 32 * wave, qhi = qlo + 31;
-    const int st_lo = max(t0 + 1 - ws, 0) / KS, st_hi = min(t0 + FQ - 1, s - 1) / KS;
+    const int qlo = SPLIT ? t0 : t0 + 32 * wave, qhi = qlo + 31;
+    const int st_lo = max(t0 + 1 - ws, 0) / KS, st_hi = min(t0 + (SPLIT ? SQ : FQ) - 1, s - 1) / KS;
     const StageSrc km{k, row0, total, hoff, s}, vm{v, row0, total, hoff, s};
     const float scale = kInvSqrt;
 
@@ -685,24 +756,25 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_q_blocked_kernel(const unsigne
     // Weights of a stage for this lane: wreg[hf][qt] = keys k0 + 32 hf + 8 g .. + 7 of query qt (stage_row).  At the window's ends
     // a piece is read whole as well, out of the rows next to it, and what is not the query's own is taken off where the piece
     // is used: not here, where that would wait for the read.
-    uint4 wreg[2][2];
+    constexpr int NH = SPLIT ? 1 : 2;
+    uint4 wreg[NH][2];
     const bool at_edge = edge_head(b * H + h, (int)(gridDim.y * gridDim.z), s, ws);
     auto whole = [&](int k0) { return k0 + KS - 1 <= qlo && k0 >= qhi + 1 - ws && qhi < s; };
     auto fetch_weights = [&](int k0) {
         const bool skip = k0 > qhi || k0 + KS - 1 < qlo + 1 - ws, full = whole(k0);
 #pragma unroll
-        for (int hf = 0; hf < 2; hf++)
+        for (int half = 0; half < NH; half++)
 #pragma unroll
             for (int qt = 0; qt < 2; qt++) {
-                const int key0 = k0 + 32 * hf + 8 * g;
-                wreg[hf][qt] = make_uint4(0u, 0u, 0u, 0u);
+                const int key0 = k0 + 32 * (SPLIT ? wave & 1 : half) + 8 * g;
+                wreg[half][qt] = make_uint4(0u, 0u, 0u, 0u);
                 if (skip) continue;
                 const unsigned short *p = wrow[qt] + (key0 - lsq[qt]);
                 if (full) {
-                    __builtin_memcpy(&wreg[hf][qt], p, 16);
+                    __builtin_memcpy(&wreg[half][qt], p, 16);
                 } else if (key0 + 7 >= lsq[qt] && key0 <= tqs[qt]) {
                     if (!at_edge || piece_inside(tqs[qt], s, ws, key0 - lsq[qt])) {
-                        __builtin_memcpy(&wreg[hf][qt], p, 16);
+                        __builtin_memcpy(&wreg[half][qt], p, 16);
                     } else {   // at the tensor's own ends
                         unsigned d[4] = {0u, 0u, 0u, 0u};
 #pragma unroll
@@ -712,48 +784,55 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_q_blocked_kernel(const unsigne
                             if (key >= lsq[qt] && key <= tqs[qt]) x = wrow[qt][key - lsq[qt]];
                             d[e >> 1] |= x << (16 * (e & 1));
                         }
-                        wreg[hf][qt] = make_uint4(d[0], d[1], d[2], d[3]);
+                        wreg[half][qt] = make_uint4(d[0], d[1], d[2], d[3]);
                     }
                 }
             }
     };
 
-    uint4 kreg[2], vreg[2];
-    load_rows<HDV>(km, KS * st_lo, kreg);
-    load_rows<HDV>(vm, KS * st_lo, vreg);
-    fetch_weights(KS * st_lo);
-    for (int st = st_lo; st <= st_hi; st++) {
-        const int buf = (st - st_lo) & 1, k0 = KS * st;
+    const int sub = SPLIT ? wave >> 1 : 0;   // which stage of a pair is this wave's
+    uint4 kreg[SPLIT ? 2 : 1][2], vreg[SPLIT ? 2 : 1][2];
+    auto fetch_stages = [&](int first) {
 #pragma unroll
-        for (int c = 0; c < 2; c++) {
-            const int chunk = tid + 256 * c;
-            *reinterpret_cast<uint4 *>(&Ks[buf][stage_row(chunk >> 3)][8 * (chunk & 7)]) = kreg[c];
-            *reinterpret_cast<uint4 *>(&Vs[buf][stage_row(chunk >> 3)][8 * (chunk & 7)]) = vreg[c];
+        for (int p = 0; p < (SPLIT ? 2 : 1); p++) {
+            load_rows<HDV>(km, first + KS * p, kreg[p]);
+            load_rows<HDV>(vm, first + KS * p, vreg[p]);
         }
-        uint4 wcur[2][2];
+        fetch_weights(first + KS * sub);
+    };
+    fetch_stages(KS * st_lo);
+    for (int st = st_lo; st <= st_hi; st += SPLIT ? 2 : 1) {
+        const int buf = SPLIT ? sub : (st - st_lo) & 1, k0 = KS * (st + sub);
+        if (SPLIT && st > st_lo) __syncthreads();   // both stages are read
+#pragma unroll
+        for (int p = 0; p < (SPLIT ? 2 : 1); p++)
+#pragma unroll
+            for (int c = 0; c < 2; c++) {
+                const int chunk = tid + 256 * c, to = SPLIT ? p : buf;
+                *reinterpret_cast<uint4 *>(&Ks[to][stage_row(chunk >> 3)][8 * (chunk & 7)]) = kreg[p][c];
+                *reinterpret_cast<uint4 *>(&Vs[to][stage_row(chunk >> 3)][8 * (chunk & 7)]) = vreg[p][c];
+            }
+        uint4 wcur[NH][2];
         const bool full = whole(k0);
 #pragma unroll
-        for (int hf = 0; hf < 2; hf++)
+        for (int half = 0; half < NH; half++)
 #pragma unroll
             for (int qt = 0; qt < 2; qt++) {
-                wcur[hf][qt] = wreg[hf][qt];
+                wcur[half][qt] = wreg[half][qt];
                 if (!full) {
-                    const int key0 = k0 + 32 * hf + 8 * g, first = lsq[qt] - key0, last = tqs[qt] - key0;
-                    wcur[hf][qt].x &= own_pair(0, first, last);
-                    wcur[hf][qt].y &= own_pair(2, first, last);
-                    wcur[hf][qt].z &= own_pair(4, first, last);
-                    wcur[hf][qt].w &= own_pair(6, first, last);
+                    const int key0 = k0 + 32 * (SPLIT ? wave & 1 : half) + 8 * g, first = lsq[qt] - key0, last = tqs[qt] - key0;
+                    wcur[half][qt].x &= own_pair(0, first, last);
+                    wcur[half][qt].y &= own_pair(2, first, last);
+                    wcur[half][qt].z &= own_pair(4, first, last);
+                    wcur[half][qt].w &= own_pair(6, first, last);
                 }
             }
         __syncthreads();
-        if (st < st_hi) {
-            load_rows<HDV>(km, k0 + KS, kreg);
-            load_rows<HDV>(vm, k0 + KS, vreg);
-            fetch_weights(k0 + KS);
-        }
+        if (st + (SPLIT ? 1 : 0) < st_hi) fetch_stages(KS * (st + (SPLIT ? 2 : 1)));
         if (k0 > qhi || k0 + KS - 1 < qlo + 1 - ws) continue;
 #pragma unroll
-        for (int hf = 0; hf < 2; hf++) {
+        for (int half = 0; half < NH; half++) {
+            const int hf = SPLIT ? wave & 1 : half;
             uint4 xh[2], xl[2], wb[2];
 #pragma unroll
             for (int qt = 0; qt < 2; qt++) {
@@ -766,7 +845,7 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_q_blocked_kernel(const unsigne
                     dw = mfma32(av0, dol[qt][0], dw);
                     if constexpr (NKS == 2) dw = mfma32(av1, doh[qt][1], dw);
                     if constexpr (NKS == 2) dw = mfma32(av1, dol[qt][1], dw);
-                    const uint2 wp = c ? make_uint2(wcur[hf][qt].z, wcur[hf][qt].w) : make_uint2(wcur[hf][qt].x, wcur[hf][qt].y);
+                    const uint2 wp = c ? make_uint2(wcur[half][qt].z, wcur[half][qt].w) : make_uint2(wcur[half][qt].x, wcur[half][qt].y);
                     x[c][0] = bf_lo(wp.x) * dw[0];
                     x[c][1] = bf_hi(wp.x) * dw[1];
                     x[c][2] = bf_lo(wp.y) * dw[2];
@@ -774,7 +853,7 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_q_blocked_kernel(const unsigne
                     dpart[qt] += (x[c][0] + x[c][1]) + (x[c][2] + x[c][3]);
                 }
                 split8(x[0], x[1], xh[qt], xl[qt]);
-                wb[qt] = wcur[hf][qt];
+                wb[qt] = wcur[half][qt];
             }
 #pragma unroll
             for (int dt = 0; dt < NDT; dt++) {
@@ -788,18 +867,25 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_q_blocked_kernel(const unsigne
             }
         }
     }
+    if constexpr (SPLIT) {
+        float *buf = reinterpret_cast<float *>(&Ks[0][0][0]);
+        join_waves<NDT>(aq, bq, buf, wave, l);
+        join_waves(dpart, buf, wave, l);
+    }
 #pragma unroll
     for (int qt = 0; qt < 2; qt++) {
         const int tq = qlo + 16 * qt + r;
+        if (SPLIT && qt != wave >> 1) continue;
         float dsum = dpart[qt];
         dsum += __shfl_xor(dsum, 16, 64);
         dsum += __shfl_xor(dsum, 32, 64);
         if (tq < s) {
-            if (g == 0) dvec[(size_t)(b * H + h) * s + tq] = dsum;
+            if (g == 0 && !(SPLIT && (wave & 1))) dvec[(size_t)(b * H + h) * s + tq] = dsum;
             float *ob = d_q + (row0 + tq) * total + hoff;
 #pragma unroll
             for (int dt = 0; dt < NDT; dt++)
-                *reinterpret_cast<f32x4 *>(ob + 16 * dt + 4 * g) = (aq[qt][dt] - dsum * bq[qt][dt]) * scale;
+                if (own_tile<NDT, SPLIT>(qt, dt, wave))
+                    *reinterpret_cast<f32x4 *>(ob + 16 * dt + 4 * g) = (aq[qt][dt] - dsum * bq[qt][dt]) * scale;
         }
     }
 }
@@ -810,7 +896,7 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_q_blocked_kernel(const unsigne
 // accumulates d_v^T += dO^T w and d_k^T += Q^T dS.  The Q and dO rows of a stage are staged as they arrive (dO as
 // hi + lo); the products that contract over queries read them through ds_read_b64_tr_b16 in the query order
 // that the score tiles leave in the lanes.  K and V of the wave's keys sit in registers.
-template <int HDV, bool OUT16>
+template <int HDV, bool OUT16, bool SPLIT>
 __global__ __launch_bounds__(256, 2) void swa_bwd_k_stats_kernel(const unsigned short *__restrict__ q,
                                                                  const unsigned short *__restrict__ k,
                                                                  const unsigned short *__restrict__ v,
@@ -819,17 +905,18 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_k_stats_kernel(const unsigned 
                                                                  const float *__restrict__ dvec,
                                                                  float *__restrict__ d_k, float *__restrict__ d_v,
                                                                  int s, int H, int ws, Out16 o16) {
-    __shared__ __align__(16) unsigned short Qs[2][KS][LDH], Dh[2][KS][LDH], Dl[2][KS][LDH];   // [query][dim]
+    __shared__ __align__(16) unsigned short QD[6][KS][LDH];   // two stages [query][dim] of Q, then of dO's hi, then lo
+    unsigned short (*const Qs)[KS][LDH] = QD, (*const Dh)[KS][LDH] = QD + 2, (*const Dl)[KS][LDH] = QD + 4;
     __shared__ __align__(16) float Mc[2][KS], Iv[2][KS], Dd[2][KS];   // the stage's queries: maximum, 1 / sum, D
     const int tid = threadIdx.x, wave = tid >> 6, l = tid & 63, r = l & 15, g = l >> 4;
     const BlockCoord bc = xcd_block_coord(H);
-    const int j0 = bc.x * FQ, h = bc.h, b = bc.b;
+    const int j0 = bc.x * (SPLIT ? SQ : FQ), h = bc.h, b = bc.b;
     constexpr int NKS = HDV / 32, NDT = HDV / 16;
     constexpr float kInvSqrt = HDV == 64 ? 0.125f : 0.17677669529663687f;   // 1 / sqrt(head size)
     const int total = H * HDV, hoff = h * HDV;
     const size_t row0 = (size_t)b * s;
-    const int jlo = j0 + 32 * wave, jhi = jlo + 31;            // this wave's keys
-    const int st_lo = j0 / KS, st_hi = min(s - 1, j0 + FQ - 1 + ws - 1) / KS;
+    const int jlo = SPLIT ? j0 : j0 + 32 * wave, jhi = jlo + 31;            // this wave's keys
+    const int st_lo = j0 / KS, st_hi = min(s - 1, j0 + (SPLIT ? SQ : FQ) - 1 + ws - 1) / KS;
     const float *dvb = dvec + (size_t)(b * H + h) * s;
     const float2 *stb = stats + (size_t)(b * H + h) * s;
     const StageSrc qm{q, row0, total, hoff, s};
@@ -856,42 +943,53 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_k_stats_kernel(const unsigned 
         for (int dt = 0; dt < NDT; dt++) { dk[jt][dt] = f32x4{0.f, 0.f, 0.f, 0.f}; dv[jt][dt] = f32x4{0.f, 0.f, 0.f, 0.f}; }
 
     // one stage ahead in registers: Q rows (two 16-byte pieces per thread), dO rows (thread = quarter row)
-    uint4 qreg[2];
-    f32x4 dreg[4];
+    constexpr int NP = SPLIT ? 2 : 1;
+    uint4 qreg[NP][2];
+    f32x4 dreg[NP][4];
     float2 streg = make_float2(0.f, 0.f);
     float ddreg = 0.f;
     const int drow = tid >> 2, dcol = 16 * (tid & 3);
-    auto fetch_stage = [&](int t_lo) {
-        load_rows<HDV>(qm, t_lo, qreg);
-        const int t = t_lo + drow;
+    auto fetch_stages = [&](int t_lo) {
 #pragma unroll
-        for (int c = 0; c < 4; c++) {
-            dreg[c] = f32x4{0.f, 0.f, 0.f, 0.f};
-            if (t < s && dcol < HDV) dreg[c] = *reinterpret_cast<const f32x4 *>(d_out + (row0 + t) * total + hoff + dcol + 4 * c);
+        for (int p = 0; p < NP; p++) {
+            load_rows<HDV>(qm, t_lo + KS * p, qreg[p]);
+            const int t = t_lo + KS * p + drow;
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                dreg[p][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+                if (t < s && dcol < HDV) dreg[p][c] = *reinterpret_cast<const f32x4 *>(d_out + (row0 + t) * total + hoff + dcol + 4 * c);
+            }
         }
         streg = make_float2(0.f, 0.f);
         ddreg = 0.f;
-        if (tid < KS && t_lo + tid < s) { streg = stb[t_lo + tid]; ddreg = dvb[t_lo + tid]; }
+        if (tid < NP * KS && t_lo + tid < s) { streg = stb[t_lo + tid]; ddreg = dvb[t_lo + tid]; }
     };
-    fetch_stage(KS * st_lo);
-    for (int st = st_lo; st <= st_hi; st++) {
-        const int buf = (st - st_lo) & 1, t_lo = KS * st;
+    fetch_stages(KS * st_lo);
+    for (int st = st_lo; st <= st_hi; st += NP) {
+        const int buf = SPLIT ? wave >> 1 : (st - st_lo) & 1, t_lo = KS * (SPLIT ? st + buf : st);
+        if (SPLIT && st > st_lo) __syncthreads();   // both stages are read
 #pragma unroll
-        for (int c = 0; c < 2; c++) {
-            const int chunk = tid + 256 * c;
-            *reinterpret_cast<uint4 *>(&Qs[buf][chunk >> 3][8 * (chunk & 7)]) = qreg[c];
-            uint4 hi, lo;
-            split8(dreg[2 * c], dreg[2 * c + 1], hi, lo);
-            *reinterpret_cast<uint4 *>(&Dh[buf][drow][dcol + 8 * c]) = hi;
-            *reinterpret_cast<uint4 *>(&Dl[buf][drow][dcol + 8 * c]) = lo;
+        for (int p = 0; p < NP; p++)
+#pragma unroll
+            for (int c = 0; c < 2; c++) {
+                const int chunk = tid + 256 * c, to = SPLIT ? p : buf;
+                *reinterpret_cast<uint4 *>(&Qs[to][chunk >> 3][8 * (chunk & 7)]) = qreg[p][c];
+                uint4 hi, lo;
+                split8(dreg[p][2 * c], dreg[p][2 * c + 1], hi, lo);
+                *reinterpret_cast<uint4 *>(&Dh[to][drow][dcol + 8 * c]) = hi;
+                *reinterpret_cast<uint4 *>(&Dl[to][drow][dcol + 8 * c]) = lo;
+            }
+        if (tid < NP * KS) {
+            const int to = SPLIT ? tid / KS : buf;
+            Mc[to][tid % KS] = streg.x; Iv[to][tid % KS] = streg.y; Dd[to][tid % KS] = ddreg;
         }
-        if (tid < KS) { Mc[buf][tid] = streg.x; Iv[buf][tid] = streg.y; Dd[buf][tid] = ddreg; }
         __syncthreads();
-        if (st < st_hi) fetch_stage(t_lo + KS);
+        if (st + NP - 1 < st_hi) fetch_stages(KS * (st + NP));
         if (t_lo + KS - 1 < jlo || t_lo > jhi + ws - 1) continue;   // no query of this stage sees a key of this wave
         const bool full = t_lo >= jhi && t_lo + KS - 1 <= jlo + ws - 1 && t_lo + KS - 1 < s && jhi < s;
 #pragma unroll
-        for (int hq = 0; hq < 2; hq++) {
+        for (int half = 0; half < 3 - NP; half++) {
+            const int hq = SPLIT ? wave & 1 : half;
             uint4 wpk[2], dsh[2], dsl[2];
             f32x4 ds[2][2];
             unsigned wp[2][2][2];
@@ -948,6 +1046,7 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_k_stats_kernel(const unsigned 
             }
         }
     }
+    if constexpr (SPLIT) join_waves<NDT>(dk, dv, reinterpret_cast<float *>(&QD[0][0][0]), wave, l);
     // accumulate: column = key jlo + 16 jt + r, rows = dims 16 dt + 4 g ..
 #pragma unroll
     for (int jt = 0; jt < 2; jt++) {
@@ -957,6 +1056,7 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_k_stats_kernel(const unsigned 
             unsigned short *pk = o16.k + (row0 + key) * o16.ld + hoff, *pv = o16.v + (row0 + key) * o16.ld + hoff;
 #pragma unroll
             for (int dt = 0; dt < NDT; dt++) {
+                if (!own_tile<NDT, SPLIT>(jt, dt, wave)) continue;
                 const f32x4 a = dk[jt][dt] * scale, c = dv[jt][dt];
                 *reinterpret_cast<uint2 *>(pk + 16 * dt + 4 * g) = make_uint2(pack2(a[0], a[1]), pack2(a[2], a[3]));
                 *reinterpret_cast<uint2 *>(pv + 16 * dt + 4 * g) = make_uint2(pack2(c[0], c[1]), pack2(c[2], c[3]));
@@ -966,6 +1066,7 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_k_stats_kernel(const unsigned 
         float *pk = d_k + (row0 + key) * total + hoff, *pv = d_v + (row0 + key) * total + hoff;
 #pragma unroll
         for (int dt = 0; dt < NDT; dt++) {
+            if (!own_tile<NDT, SPLIT>(jt, dt, wave)) continue;
             f32x4 *ck = reinterpret_cast<f32x4 *>(pk + 16 * dt + 4 * g), *cv = reinterpret_cast<f32x4 *>(pv + 16 * dt + 4 * g);
             *ck = *ck + dk[jt][dt] * scale;
             *cv = *cv + dv[jt][dt];
@@ -981,7 +1082,7 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_k_stats_kernel(const unsigned 
 // in the stages at the window's ends and two more vector instructions an element).
 constexpr int LDW = 144;   // row stride of the weight stage (288 B: the transposing reads of a group fall on 32 banks)
 
-template <int HDV>
+template <int HDV, bool SPLIT>
 __global__ __launch_bounds__(256, 2) void swa_bwd_k_blocked_kernel(const unsigned short *__restrict__ q,
                                                                    const unsigned short *__restrict__ v,
                                                                    const unsigned short *__restrict__ attn_w,
@@ -989,18 +1090,20 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_k_blocked_kernel(const unsigne
                                                                    const float *__restrict__ dvec,
                                                                    float *__restrict__ d_k, float *__restrict__ d_v,
                                                                    int s, int H, int ws) {
-    __shared__ __align__(16) unsigned short Qs[2][KS][LDH], Dh[2][KS][LDH], Dl[2][KS][LDH];   // [query][dim]
-    __shared__ __align__(16) unsigned short Wt[KS][LDW];                                       // [query][key of the block]
+    constexpr int NP = SPLIT ? 2 : 1, LDK = SPLIT ? 48 : LDW;
+    __shared__ __align__(16) unsigned short QD[6][KS][LDH];    // two stages [query][dim] of Q, then of dO's hi, then lo
+    __shared__ __align__(16) unsigned short Wt[NP * KS][LDK];  // [query][key of the block]
+    unsigned short (*const Qs)[KS][LDH] = QD, (*const Dh)[KS][LDH] = QD + 2, (*const Dl)[KS][LDH] = QD + 4;
     __shared__ __align__(16) float Dd[2][KS];
     const int tid = threadIdx.x, wave = tid >> 6, l = tid & 63, r = l & 15, g = l >> 4;
     const BlockCoord bc = xcd_block_coord(H);
-    const int j0 = bc.x * FQ, h = bc.h, b = bc.b;
+    const int j0 = bc.x * (SPLIT ? SQ : FQ), h = bc.h, b = bc.b;
     constexpr int NKS = HDV / 32, NDT = HDV / 16;
     constexpr float kInvSqrt = HDV == 64 ? 0.125f : 0.17677669529663687f;   // 1 / sqrt(head size)
     const int total = H * HDV, hoff = h * HDV;
     const size_t row0 = (size_t)b * s;
-    const int jlo = j0 + 32 * wave, jhi = jlo + 31;
-    const int st_lo = j0 / KS, st_hi = min(s - 1, j0 + FQ - 1 + ws - 1) / KS;
+    const int jlo = SPLIT ? j0 : j0 + 32 * wave, jhi = jlo + 31;
+    const int st_lo = j0 / KS, st_hi = min(s - 1, j0 + (SPLIT ? SQ : FQ) - 1 + ws - 1) / KS;
     const float *dvb = dvec + (size_t)(b * H + h) * s;
     const float scale = kInvSqrt;
     const unsigned short *awb = attn_w + (size_t)(b * H + h) * s * ws;
@@ -1022,82 +1125,93 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_k_blocked_kernel(const unsigne
 #pragma unroll
         for (int dt = 0; dt < NDT; dt++) { dk[jt][dt] = f32x4{0.f, 0.f, 0.f, 0.f}; dv[jt][dt] = f32x4{0.f, 0.f, 0.f, 0.f}; }
 
-    uint4 qreg[2], wreg[4];
-    f32x4 dreg[4];
+    // Weights: thread (query drow, quarter) reads the quarter's pieces of eight keys of the query's row
+    constexpr int NW = SPLIT ? 1 : 4, QK = 8 * NW;
+    uint4 qreg[NP][2], wreg[NP][NW];
+    f32x4 dreg[NP][4];
     float ddreg = 0.f;
     const int drow = tid >> 2, dcol = 16 * (tid & 3);
-    auto fetch_stage = [&](int t_lo) {
-        load_rows<HDV>(qm, t_lo, qreg);
-        const int t = t_lo + drow;
+    auto fetch_stages = [&](int t_lo) {
+        ddreg = (tid < NP * KS && t_lo + tid < s) ? dvb[t_lo + tid] : 0.f;
 #pragma unroll
-        for (int c = 0; c < 4; c++) {
-            dreg[c] = f32x4{0.f, 0.f, 0.f, 0.f};
-            if (t < s && dcol < HDV) dreg[c] = *reinterpret_cast<const f32x4 *>(d_out + (row0 + t) * total + hoff + dcol + 4 * c);
-        }
-        ddreg = (tid < KS && t_lo + tid < s) ? dvb[t_lo + tid] : 0.f;
-        // weights of query t for keys j0 + 32 (tid % 4) .. + 31: four pieces of 8 keys, read whole at the window's ends too
-        // (out of the rows next to it) and freed of what is not the query's own where they go to LDS
-        const int lsq = max(t + 1 - ws, 0), thi = t < s ? t : -1;
-        const unsigned short *wrow = awb + (size_t)t * ws;
+        for (int p = 0; p < NP; p++) {
+            load_rows<HDV>(qm, t_lo + KS * p, qreg[p]);
+            const int t = t_lo + KS * p + drow;
 #pragma unroll
-        for (int c = 0; c < 4; c++) {
-            const int key0 = j0 + 32 * (tid & 3) + 8 * c;
-            wreg[c] = make_uint4(0, 0, 0, 0);
-            if (key0 + 7 >= lsq && key0 <= thi) {
-                if (!at_edge || piece_inside(t, s, ws, key0 - lsq)) {
-                    __builtin_memcpy(&wreg[c], wrow + (key0 - lsq), 16);
-                } else {   // at the tensor's own ends
-                    unsigned d[4] = {0u, 0u, 0u, 0u};
+            for (int c = 0; c < 4; c++) {
+                dreg[p][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+                if (t < s && dcol < HDV) dreg[p][c] = *reinterpret_cast<const f32x4 *>(d_out + (row0 + t) * total + hoff + dcol + 4 * c);
+            }
+            // pieces are read whole at the window's ends too (out of the rows next to it) and freed of what is not the
+            // query's own where they go to LDS
+            const int lsq = max(t + 1 - ws, 0), thi = t < s ? t : -1;
+            const unsigned short *wrow = awb + (size_t)t * ws;
 #pragma unroll
-                    for (int e = 0; e < 8; e++) {
-                        const int key = key0 + e;
-                        unsigned x = 0;
-                        if (key >= lsq && key <= thi) x = wrow[key - lsq];
-                        d[e >> 1] |= x << (16 * (e & 1));
+            for (int c = 0; c < NW; c++) {
+                const int key0 = j0 + QK * (tid & 3) + 8 * c;
+                wreg[p][c] = make_uint4(0, 0, 0, 0);
+                if (key0 + 7 >= lsq && key0 <= thi) {
+                    if (!at_edge || piece_inside(t, s, ws, key0 - lsq)) {
+                        __builtin_memcpy(&wreg[p][c], wrow + (key0 - lsq), 16);
+                    } else {   // at the tensor's own ends
+                        unsigned d[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+                        for (int e = 0; e < 8; e++) {
+                            const int key = key0 + e;
+                            unsigned x = 0;
+                            if (key >= lsq && key <= thi) x = wrow[key - lsq];
+                            d[e >> 1] |= x << (16 * (e & 1));
+                        }
+                        wreg[p][c] = make_uint4(d[0], d[1], d[2], d[3]);
                     }
-                    wreg[c] = make_uint4(d[0], d[1], d[2], d[3]);
                 }
             }
         }
     };
-    fetch_stage(KS * st_lo);
-    for (int st = st_lo; st <= st_hi; st++) {
-        const int buf = (st - st_lo) & 1, t_lo = KS * st;
-        const bool inner = t_lo >= j0 + FQ - 1 && t_lo + KS - 1 <= j0 + ws - 1 && t_lo + KS - 1 < s;   // every query sees every key
+    fetch_stages(KS * st_lo);
+    for (int st = st_lo; st <= st_hi; st += NP) {
+        const int buf = SPLIT ? wave >> 1 : (st - st_lo) & 1, t_lo = KS * (SPLIT ? st + buf : st);
 #pragma unroll
-        for (int c = 0; c < 2; c++) {
-            const int chunk = tid + 256 * c;
-            *reinterpret_cast<uint4 *>(&Qs[buf][chunk >> 3][8 * (chunk & 7)]) = qreg[c];
-            uint4 hi, lo;
-            split8(dreg[2 * c], dreg[2 * c + 1], hi, lo);
-            *reinterpret_cast<uint4 *>(&Dh[buf][drow][dcol + 8 * c]) = hi;
-            *reinterpret_cast<uint4 *>(&Dl[buf][drow][dcol + 8 * c]) = lo;
-        }
+        for (int p = 0; p < NP; p++) {
+            const int to = SPLIT ? p : buf, t_p = KS * (st + p);
+            const bool inner = t_p >= j0 + (SPLIT ? SQ : FQ) - 1 && t_p + KS - 1 <= j0 + ws - 1 && t_p + KS - 1 < s;   // every query sees every key
 #pragma unroll
-        for (int c = 0; c < 4; c++) {
-            if (!inner) {
-                const int t = t_lo + drow, key0 = j0 + 32 * (tid & 3) + 8 * c;
-                const int first = max(t + 1 - ws, 0) - key0, last = (t < s ? t : -1) - key0;
-                if (__any(first > 0 || last < 7)) {
-                    wreg[c].x &= own_pair(0, first, last);
-                    wreg[c].y &= own_pair(2, first, last);
-                    wreg[c].z &= own_pair(4, first, last);
-                    wreg[c].w &= own_pair(6, first, last);
-                }
+            for (int c = 0; c < 2; c++) {
+                const int chunk = tid + 256 * c;
+                *reinterpret_cast<uint4 *>(&Qs[to][chunk >> 3][8 * (chunk & 7)]) = qreg[p][c];
+                uint4 hi, lo;
+                split8(dreg[p][2 * c], dreg[p][2 * c + 1], hi, lo);
+                *reinterpret_cast<uint4 *>(&Dh[to][drow][dcol + 8 * c]) = hi;
+                *reinterpret_cast<uint4 *>(&Dl[to][drow][dcol + 8 * c]) = lo;
             }
-            *reinterpret_cast<uint4 *>(&Wt[drow][32 * (tid & 3) + 8 * c]) = wreg[c];
+#pragma unroll
+            for (int c = 0; c < NW; c++) {
+                uint4 &w = wreg[p][c];
+                if (!inner) {
+                    const int t = t_p + drow, key0 = j0 + QK * (tid & 3) + 8 * c;
+                    const int first = max(t + 1 - ws, 0) - key0, last = (t < s ? t : -1) - key0;
+                    if (__any(first > 0 || last < 7)) {
+                        w.x &= own_pair(0, first, last);
+                        w.y &= own_pair(2, first, last);
+                        w.z &= own_pair(4, first, last);
+                        w.w &= own_pair(6, first, last);
+                    }
+                }
+                *reinterpret_cast<uint4 *>(&Wt[KS * (SPLIT ? p : 0) + drow][QK * (tid & 3) + 8 * c]) = w;
+            }
         }
-        if (tid < KS) Dd[buf][tid] = ddreg;
+        if (tid < NP * KS) Dd[SPLIT ? tid / KS : buf][tid % KS] = ddreg;
         __syncthreads();
-        if (st < st_hi) fetch_stage(t_lo + KS);
+        if (st + NP - 1 < st_hi) fetch_stages(KS * (st + NP));
         if (!(t_lo + KS - 1 < jlo || t_lo > jhi + ws - 1)) {   // a query of this stage sees a key of this wave
 #pragma unroll
-            for (int hq = 0; hq < 2; hq++) {
+            for (int half = 0; half < 3 - NP; half++) {
+                const int hq = SPLIT ? wave & 1 : half;
                 const int ra = 32 * hq + 4 * g, rb = ra + 16;
                 uint4 wpk[2], dsh[2], dsl[2];
                 f32x4 ds[2][2];
 #pragma unroll
-                for (int jt = 0; jt < 2; jt++) wpk[jt] = ld_tr2<LDW>(Wt, ra, rb, 32 * wave + 16 * jt);
+                for (int jt = 0; jt < 2; jt++) wpk[jt] = ld_tr2<LDK>(Wt + (SPLIT ? KS * buf : 0), ra, rb, (SPLIT ? 0 : 32 * wave) + 16 * jt);
 #pragma unroll
                 for (int c = 0; c < 2; c++) {
                     const int qt = 2 * hq + c;
@@ -1136,6 +1250,7 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_k_blocked_kernel(const unsigne
         }
         __syncthreads();   // the weight stage has one buffer: every wave is done with it before the next one lands
     }
+    if constexpr (SPLIT) join_waves<NDT>(dk, dv, reinterpret_cast<float *>(&QD[0][0][0]), wave, l);
 #pragma unroll
     for (int jt = 0; jt < 2; jt++) {
         const int key = jlo + 16 * jt + r;
@@ -1143,6 +1258,7 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_k_blocked_kernel(const unsigne
         float *pk = d_k + (row0 + key) * total + hoff, *pv = d_v + (row0 + key) * total + hoff;
 #pragma unroll
         for (int dt = 0; dt < NDT; dt++) {
+            if (!own_tile<NDT, SPLIT>(jt, dt, wave)) continue;
             f32x4 *ck = reinterpret_cast<f32x4 *>(pk + 16 * dt + 4 * g), *cv = reinterpret_cast<f32x4 *>(pv + 16 * dt + 4 * g);
             *ck = *ck + dk[jt][dt] * scale;
             *cv = *cv + dv[jt][dt];
@@ -1173,6 +1289,14 @@ bool swa_forward_mfma(const uint16_t *q, const uint16_t *k, const uint16_t *v, u
     return true;
 }
 
+// f with the head size, the kind of output and SPLIT as types
+template <class F>
+static void choose(bool wide, bool out16, bool split, F f) {
+    auto third = [&](auto hd, auto o) { if (split) f(hd, o, std::true_type{}); else f(hd, o, std::false_type{}); };
+    auto second = [&](auto hd) { if (out16) third(hd, std::true_type{}); else third(hd, std::false_type{}); };
+    if (wide) second(std::integral_constant<int, 64>{}); else second(std::integral_constant<int, 32>{});
+}
+
 bool swa_backward_mfma(const uint16_t *q, const uint16_t *k, const uint16_t *v, const uint16_t *attn_weights,
                        const float *d_attn_out, float *d_q, float *d_k, float *d_v, int seq_len, int num_heads,
                        int head_dim, int window, int batch, int n_persistent, const float *stats, const SwaGradCols *cols) {
@@ -1180,43 +1304,45 @@ bool swa_backward_mfma(const uint16_t *q, const uint16_t *k, const uint16_t *v, 
     if ((head_dim != 64 && head_dim != 32) || n_persistent != 0 || window > 512 || window < 1) return false;
     float *dvec = scratch(1, (size_t)batch * num_heads * seq_len * sizeof(float));
     if (es.failed()) return true;
+    // 32 rows a workgroup while those fit the chip at once, two to a compute unit (both sides above join_waves)
+    const bool split = 2ll * ceil_div(seq_len, FQ) * num_heads * batch <= compute_units();
+    const dim3 grid(ceil_div(seq_len, split ? SQ : FQ), num_heads, batch);
+    const bool wide = head_dim == 64;
     if (stats) {
         const float2 *st2 = reinterpret_cast<const float2 *>(stats);
-        const dim3 grid((seq_len + FQ - 1) / FQ, num_heads, batch);
         const Out16 o16 = cols ? Out16{cols->q, cols->k, cols->v, cols->ld} : Out16{nullptr, nullptr, nullptr, 0};
-#define NLH_SWA_BWD_STATS(HDV, O16)                                                                                       \
-    {                                                                                                                     \
-        {                                                                                                                 \
-            KernelTimer kt("swa_bwd_q_stats_kernel");                                                                     \
-            hipLaunchKernelGGL((swa_bwd_q_stats_kernel<HDV, O16>), grid, dim3(256), 0, stream(), q, k, v, st2, d_attn_out, d_q, \
-                               dvec, seq_len, num_heads, window, o16);                                                    \
-            check_launch("swa_bwd_q_stats_kernel");                                                                       \
-        }                                                                                                                 \
-        KernelTimer kt("swa_bwd_k_stats_kernel");                                                                         \
-        hipLaunchKernelGGL((swa_bwd_k_stats_kernel<HDV, O16>), grid, dim3(256), 0, stream(), q, k, v, st2, d_attn_out, dvec,   \
-                           d_k, d_v, seq_len, num_heads, window, o16);                                                    \
-        check_launch("swa_bwd_k_stats_kernel");                                                                           \
-    }
-        if (head_dim == 64) { if (cols) NLH_SWA_BWD_STATS(64, true) else NLH_SWA_BWD_STATS(64, false) }
-        else { if (cols) NLH_SWA_BWD_STATS(32, true) else NLH_SWA_BWD_STATS(32, false) }
-#undef NLH_SWA_BWD_STATS
+        auto both = [&](auto hd, auto out16, auto halves) {
+            constexpr int HDV = decltype(hd)::value;
+            constexpr bool O16 = decltype(out16)::value, SPLIT = decltype(halves)::value;
+            {
+                KernelTimer kt("swa_bwd_q_stats_kernel");
+                hipLaunchKernelGGL((swa_bwd_q_stats_kernel<HDV, O16, SPLIT>), grid, dim3(256), 0, stream(), q, k, v, st2, d_attn_out,
+                                   d_q, dvec, seq_len, num_heads, window, o16);
+                check_launch("swa_bwd_q_stats_kernel");
+            }
+            KernelTimer kt("swa_bwd_k_stats_kernel");
+            hipLaunchKernelGGL((swa_bwd_k_stats_kernel<HDV, O16, SPLIT>), grid, dim3(256), 0, stream(), q, k, v, st2, d_attn_out,
+                               dvec, d_k, d_v, seq_len, num_heads, window, o16);
+            check_launch("swa_bwd_k_stats_kernel");
+        };
+        choose(wide, cols != nullptr, split, both);
         return true;
     }
     if (cols) return false;   // bf16 column output exists for the statistics pair only
-    {
-        KernelTimer kt("swa_bwd_q_blocked_kernel");
-        if (head_dim == 64) hipLaunchKernelGGL(swa_bwd_q_blocked_kernel<64>, dim3((seq_len + FQ - 1) / FQ, num_heads, batch), dim3(256), 0,
-                           stream(), k, v, attn_weights, d_attn_out, d_q, dvec, seq_len, num_heads, window);
-        else hipLaunchKernelGGL(swa_bwd_q_blocked_kernel<32>, dim3((seq_len + FQ - 1) / FQ, num_heads, batch), dim3(256), 0,
-                           stream(), k, v, attn_weights, d_attn_out, d_q, dvec, seq_len, num_heads, window);
-        check_launch("swa_bwd_q_blocked_kernel");
-    }
-    KernelTimer kt("swa_bwd_k_blocked_kernel");
-    if (head_dim == 64) hipLaunchKernelGGL(swa_bwd_k_blocked_kernel<64>, dim3((seq_len + FQ - 1) / FQ, num_heads, batch), dim3(256), 0, stream(), q,
-                       v, attn_weights, d_attn_out, dvec, d_k, d_v, seq_len, num_heads, window);
-    else hipLaunchKernelGGL(swa_bwd_k_blocked_kernel<32>, dim3((seq_len + FQ - 1) / FQ, num_heads, batch), dim3(256), 0, stream(), q,
-                       v, attn_weights, d_attn_out, dvec, d_k, d_v, seq_len, num_heads, window);
-    check_launch("swa_bwd_k_blocked_kernel");
+    choose(wide, false, split, [&](auto hd, auto, auto halves) {
+        constexpr int HDV = decltype(hd)::value;
+        constexpr bool SPLIT = decltype(halves)::value;
+        {
+            KernelTimer kt("swa_bwd_q_blocked_kernel");
+            hipLaunchKernelGGL((swa_bwd_q_blocked_kernel<HDV, SPLIT>), grid, dim3(256), 0, stream(), k, v, attn_weights, d_attn_out,
+                               d_q, dvec, seq_len, num_heads, window);
+            check_launch("swa_bwd_q_blocked_kernel");
+        }
+        KernelTimer kt("swa_bwd_k_blocked_kernel");
+        hipLaunchKernelGGL((swa_bwd_k_blocked_kernel<HDV, SPLIT>), grid, dim3(256), 0, stream(), q, v, attn_weights, d_attn_out, dvec,
+                           d_k, d_v, seq_len, num_heads, window);
+        check_launch("swa_bwd_k_blocked_kernel");
+    });
     return true;
 }
 

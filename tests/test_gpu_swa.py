@@ -107,6 +107,36 @@ def test_forward_keeps_its_order_of_sums(B, s, H, hd, ws, out_sha, weights_sha):
     assert [hashlib.sha256(x.tobytes()).hexdigest()[:16] for x in (out, aw)] == [out_sha, weights_sha]
 
 
+@pytest.mark.parametrize("s,ws,hd", [(1, 4, 64), (31, 32, 32), (33, 2, 64), (128, 128, 32), (161, 64, 64), (200, 101, 32),
+                                     (353, 130, 64), (600, 512, 64), (600, 511, 32)])
+def test_backward_in_blocks_of_32_rows_and_of_128(s, ws, hd):
+    """The same sequences alone (few blocks: 32 rows a workgroup, the window shared out over its waves) and as one of many
+    (128 rows).  The two differ in the order of fp32 sums; a D that moves by that can take an element of dS to the other neighbour
+    in the 16 bits that its pair keeps, 2^-17 of it."""
+    H, blocks = 2, -(-s // 128) * 2
+    n = torch.cuda.get_device_properties(0).multi_processor_count // (2 * blocks) + 1
+    q, k, v, go = _case(1, s, H, hd, s + ws)
+    many = lambda a: np.repeat(a, n, 0)
+    _, aw = gpu_forward(q, k, v, ws, H, 0)
+    few, lots = gpu_backward(q, k, v, aw, go, ws, H, 0), gpu_backward(many(q), many(k), many(v), many(aw), many(go), ws, H, 0)
+
+    def stats_pair(q, k, v, go):
+        B, td = len(q), H * hd
+        out, st = torch.zeros(B, s, td, dtype=torch.uint16, device="cuda"), zeros(B, H, s, 2)
+        g = [zeros(B, s, td) for _ in range(3)]
+        D.call("swa_forward_lse_bf16_rocm", _u16(q), _u16(k), _u16(v), out, st, s, H, hd, ws, B)
+        D.call("swa_backward_lse_bf16_rocm", _u16(q), _u16(k), _u16(v), st, dev(go), *g, s, H, hd, ws, B)
+        torch.cuda.synchronize()
+        return [host(x) for x in g]
+
+    few += tuple(stats_pair(q, k, v, go))
+    lots += tuple(stats_pair(many(q), many(k), many(v), many(go)))
+    size = max(np.linalg.norm(x) for x in few)
+    for a, b in zip(few, lots):
+        assert np.array_equal(b, many(b[:1]))
+        assert np.linalg.norm(a[0] - b[0]) <= 1e-5 * np.linalg.norm(a[0]) + 1e-6 * size
+
+
 def test_swa_known_answers_on_gpu():
     """core/src/swa.rs:286-344: window 1 copies V; identical keys average V."""
     bf = lambda x: orc.f32_to_bf16(np.asarray(x, np.float32))
