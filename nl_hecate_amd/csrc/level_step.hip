@@ -30,7 +30,6 @@
 namespace nlh {
 namespace {
 
-constexpr int PT = 128;       // tokens per workgroup of the projection kernel
 constexpr int kPThr = 512;    // 8 waves
 constexpr int kMaxLevels = 8;
 constexpr int kMaxExtra = 4;
@@ -141,18 +140,19 @@ __global__ __launch_bounds__(6 * 64) void gate_fold_finish_kernel(const float *_
 }
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
-constexpr int T32 = PT / 32;   // token tiles of 32 per workgroup
-
-// acc[t32][c32][i] = sum_k W[col][k] x[token][k] with token = 32 t32 + lane % 32 of the workgroup's 128 and
+// Token tiles of 32 per workgroup: T32 = 4, or 1 for few tokens (project_launch).
+// acc[t32][c32][i] = sum_k W[col][k] x[token][k] with token = 32 t32 + lane % 32 of the workgroup's and
 // col = 32 c32 + 8 (i / 4) + 4 (lane / 32) + i % 4 of the wave's 64 columns, on v_mfma_f32_32x32x16_bf16 (measured
 // on this part: 98 % of the data-sheet rate, where the 16 x 16 x 32 shape issues at 54 %).  The weights are the A
-// operand straight from global memory (a ring of four 32-wide steps, requested three steps ahead), x the B operand
+// operand straight from global memory (a ring of four 32-wide steps, requested three steps ahead; eight where one token
+// tile's products are too short to cover a load), x the B operand
 // from LDS (two token tiles per unit of four products, the next unit's pair requested before this unit's products
 // are issued).  Fully unrolled, with the order of requests and products pinned: left to itself the scheduler sinks
 // every load to its first use and the wave then waits a full memory latency per step.
-template <int D>
+template <int D, int T32>
 __device__ __forceinline__ void project_block(const u16 *Xs, const u16 *wf, f32x16 (&acc)[T32][2]) {
-    constexpr int XS = D + 8, KS = D / 32, RING = 4, UPK = 2 * (T32 / 2), UNITS = KS * UPK;   // units per 32-wide step
+    constexpr int PAIR = T32 > 1 ? 2 : 1, NP = T32 / PAIR;   // token tiles of a unit, units of a 16-wide half step
+    constexpr int XS = D + 8, KS = D / 32, RING = T32 > 1 ? 4 : 8, UPK = 2 * NP, UNITS = KS * UPK;   // units per 32-wide step
     const int lane = threadIdx.x & 63;
     const bf16x8 *wp = reinterpret_cast<const bf16x8 *>(wf) + lane;   // step ks: [2 k halves][2 column tiles][64 lanes]
     const u16 *xb = Xs + (lane & 31) * XS + 8 * (lane >> 5);
@@ -162,29 +162,30 @@ __device__ __forceinline__ void project_block(const u16 *Xs, const u16 *wf, f32x
         for (int c = 0; c < 2; c++)
 #pragma unroll
             for (int i = 0; i < 16; i++) acc[t][c][i] = 0.f;
-    bf16x8 w[RING][4], b[2][2];
+    bf16x8 w[RING][4], b[2][PAIR];
 #pragma unroll
     for (int p = 0; p < RING - 1 && p < KS; p++)
 #pragma unroll
         for (int f = 0; f < 4; f++) w[p][f] = wp[(p * 4 + f) * 64];
-    b[0][0] = *reinterpret_cast<const bf16x8 *>(xb);
-    b[0][1] = *reinterpret_cast<const bf16x8 *>(xb + 32 * XS);
+#pragma unroll
+    for (int h = 0; h < PAIR; h++) b[0][h] = *reinterpret_cast<const bf16x8 *>(xb + 32 * h * XS);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int u = 0; u < UNITS; u++) {
         // unit u: k half kh of step ks, token tiles 2 pr and 2 pr + 1
-        const int ks = u / UPK, kh = (u % UPK) / (T32 / 2), pr = u % (T32 / 2);
+        const int ks = u / UPK, kh = (u % UPK) / NP, pr = u % NP;
         if (u % UPK == 0 && ks + RING - 1 < KS) {
 #pragma unroll
             for (int f = 0; f < 4; f++) w[(ks + RING - 1) % RING][f] = wp[((ks + RING - 1) * 4 + f) * 64];
         }
         if (u + 1 < UNITS) {
-            const int nks = (u + 1) / UPK, nkh = ((u + 1) % UPK) / (T32 / 2), npr = (u + 1) % (T32 / 2);
-            b[(u + 1) & 1][0] = *reinterpret_cast<const bf16x8 *>(xb + 64 * npr * XS + 32 * nks + 16 * nkh);
-            b[(u + 1) & 1][1] = *reinterpret_cast<const bf16x8 *>(xb + (64 * npr + 32) * XS + 32 * nks + 16 * nkh);
+            const int nks = (u + 1) / UPK, nkh = ((u + 1) % UPK) / NP, npr = (u + 1) % NP;
+#pragma unroll
+            for (int h = 0; h < PAIR; h++)
+                b[(u + 1) & 1][h] = *reinterpret_cast<const bf16x8 *>(xb + (64 * npr + 32 * h) * XS + 32 * nks + 16 * nkh);
         }
 #pragma unroll
-        for (int h = 0; h < 2; h++)
+        for (int h = 0; h < PAIR; h++)
 #pragma unroll
             for (int c = 0; c < 2; c++)
                 acc[2 * pr + h][c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[ks % RING][2 * kh + c], b[u & 1][h], acc[2 * pr + h][c], 0, 0, 0);
@@ -229,8 +230,15 @@ __device__ __forceinline__ void store_tile_rows(const f32x16 (&t)[2], float scal
 
 __device__ __forceinline__ float gate_act(int q, float pre) { return q == 1 ? softplus_(pre) : sigmoid_(pre); }
 
-template <int D>
+template <int D, int T32>
+constexpr size_t project_lds() {
+    constexpr int PT = 32 * T32;
+    return (size_t)PT * (D + 8) * 2 + (2 * 8 * PT + 2 * PT * 8 + PT) * sizeof(float) + 8 * 8 * 72 * 2;
+}
+
+template <int D, int T32>
 __global__ __launch_bounds__(kPThr) void level_project_kernel(ProjArgs a) {
+    constexpr int PT = 32 * T32;   // tokens per workgroup
     constexpr int XS = D + 8, CB = D / 64, D4 = D / 4, KS = D / 32;
     extern __shared__ __align__(16) unsigned char smem[];
     u16 *Xs = reinterpret_cast<u16 *>(smem);                                   // [PT][XS]
@@ -274,7 +282,7 @@ __global__ __launch_bounds__(kPThr) void level_project_kernel(ProjArgs a) {
     // plain projections: rounded once, token-major
     if (wave_on)
         for (int e = j0; e < min(j1, a.n_extra); e++) {
-            project_block<D>(Xs, a.wfrag + (size_t)e * D * D + wave_frag, acc);
+            project_block<D, T32>(Xs, a.wfrag + (size_t)e * D * D + wave_frag, acc);
             u16 *out = a.extra_out[e];
 #pragma unroll
             for (int tt = 0; tt < T32; tt++)
@@ -289,7 +297,7 @@ __global__ __launch_bounds__(kPThr) void level_project_kernel(ProjArgs a) {
         const int lvl = (job - a.n_extra) / 3, p = (job - a.n_extra) % 3;
         const size_t chain0 = (size_t)lvl * a.bs * a.nh;
         float *gd = gdot + (lvl & 1) * PT * 8;
-        if (p == 0) {   // the six gate dot products of the wave's 16 tokens (token tile `wave`): one tile of 16 columns
+        if (p == 0 && 16 * wave < PT) {   // the six gate dot products of the wave's 16 tokens (token tile `wave`): one tile of 16 columns
             const bf16x8 *up = reinterpret_cast<const bf16x8 *>(a.ufrag) + (size_t)lvl * KS * 64 + lane;
             const u16 *xb = Xs + (16 * wave + l16) * XS + 8 * g;
             f32x4 ga = zero4();
@@ -299,7 +307,7 @@ __global__ __launch_bounds__(kPThr) void level_project_kernel(ProjArgs a) {
             // lane group g holds rows 4g .. 4g + 3 = (hi, lo) of quantities 2g and 2g + 1
             if (g < 3) *reinterpret_cast<float2 *>(gd + (16 * wave + l16) * 8 + 2 * g) = make_float2(ga[0] + ga[1], ga[2] + ga[3]);
         }
-        if (wave_on) project_block<D>(Xs, a.wfrag + (size_t)job * D * D + wave_frag, acc);
+        if (wave_on) project_block<D, T32>(Xs, a.wfrag + (size_t)job * D * D + wave_frag, acc);
         if (p == 1) {   // v leaves as it is
             if (wave_on) {
 #pragma unroll
@@ -324,8 +332,13 @@ __global__ __launch_bounds__(kPThr) void level_project_kernel(ProjArgs a) {
 #pragma unroll
                         for (int i = 0; i < 16; i++) ss[tt] += acc[tt][c][i] * acc[tt][c][i];
                 }
-                rd[(32 * hf + l32) * 8 + wave] = swapadd32(ss[0], ss[1]);          // lower half: tile 0, upper half: tile 1
-                rd[(32 * (2 + hf) + l32) * 8 + wave] = swapadd32(ss[2], ss[3]);
+                if constexpr (T32 == 4) {
+                    rd[(32 * hf + l32) * 8 + wave] = swapadd32(ss[0], ss[1]);          // lower half: tile 0, upper half: tile 1
+                    rd[(32 * (2 + hf) + l32) * 8 + wave] = swapadd32(ss[2], ss[3]);
+                } else {
+                    const float sum = swapadd32(ss[0], ss[0]);
+                    if (hf == 0) rd[l32 * 8 + wave] = sum;
+                }
             }
             __syncthreads();
             float inv[T32];
@@ -364,7 +377,7 @@ __global__ __launch_bounds__(kPThr) void level_project_kernel(ProjArgs a) {
             }
             if (p == 0 && tid < 3 * PT) {
                 // the gates: one (token, gate) per thread; the barrier above lies behind every wave's sums and dot products
-                const int token = tid & (PT - 1), q = tid >> 7;   // PT = 128
+                const int token = tid % PT, q = tid / PT;
                 const long long tok = tok0 + token;
                 float ssum = rd[token * 8];
 #pragma unroll
@@ -684,6 +697,36 @@ void to_bf16(const float *x, u16 *out, long long count) {
     check_launch("f32_to_bf16_vec_kernel");
 }
 
+// One workgroup per 128 tokens takes all projections, which reads x once; where that leaves compute units idle or the last
+// round nearly empty the projections are shared out, at about half a projection's time for another staging of x (500
+// tokens, nine projections of 256: 62 us on four workgroups, 18 on 36).  Where 128 tokens by one projection still leave a third
+// of the compute units without any, what counts is how long one workgroup takes: 32 tokens by one projection.  Whole
+// call, us, 128 / 32 tokens: 500 tokens, nine projections of 256 24 / 17, of 512 44 / 29; at 144 pairs of (128 tokens,
+// projection) 26 / 24 to 26 and 48 / 45, at 180 31 / 29 and 52 / 50, at 216 29 / 31 and 50 / 55.
+template <int D>
+void project_launch(const ProjArgs &a, long long n, int P) {
+    static bool attr_set = false;
+    if (!attr_set) {
+        check_hip(hipFuncSetAttribute(reinterpret_cast<const void *>(level_project_kernel<D, 4>),
+                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)project_lds<D, 4>()), "dynamic LDS size");
+        check_hip(hipFuncSetAttribute(reinterpret_cast<const void *>(level_project_kernel<D, 1>),
+                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)project_lds<D, 1>()), "dynamic LDS size");
+        attr_set = true;
+    }
+    const int tiles = ceil_div(n, 128), cus = compute_units();
+    if (3ll * tiles * P <= 2 * cus) {
+        hipLaunchKernelGGL((level_project_kernel<D, 1>), dim3(ceil_div(n, 32), P), dim3(kPThr), (project_lds<D, 1>()), stream(), a);
+        return;
+    }
+    int parts = 1;
+    double best = 0;
+    for (int p = 1; p <= P; p++) {
+        const double time = ceil_div((long long)tiles * p, cus) * (ceil_div(P, p) + 0.5);
+        if (p == 1 || time < 0.95 * best) { best = time; parts = p; }
+    }
+    hipLaunchKernelGGL((level_project_kernel<D, 4>), dim3((unsigned)tiles, (unsigned)parts), dim3(kPThr), (project_lds<D, 4>()), stream(), a);
+}
+
 bool step_dims_ok(const char *fn, int bs, int s, int nh, int hd, int levels, int n_extra, int chunk) {
     const int d = nh * hd;
     if (bs <= 0 || s <= 0 || nh <= 0 || hd != 64 || levels < 0 || levels > kMaxLevels || n_extra < 0 ||
@@ -759,30 +802,8 @@ void level_project_forward_bf16_rocm(const float *x, const float *w_extra, int n
         hipLaunchKernelGGL(gate_fold_finish_kernel, dim3(ceil_div(d, 64), levels), dim3(6 * 64), 0, stream(), fold_part, ufrag, d);
         check_launch("gate_fold_kernel");
     }
-    const size_t lds = (size_t)PT * (d + 8) * 2 + (2 * 8 * PT + 2 * PT * 8 + PT) * sizeof(float) + 8 * 8 * 72 * 2;
-    static bool attr_set = false;
-    if (!attr_set) {
-        check_hip(hipFuncSetAttribute(reinterpret_cast<const void *>(level_project_kernel<512>),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)((size_t)PT * 520 * 2 + 17408 + 9216)), "dynamic LDS size");
-        check_hip(hipFuncSetAttribute(reinterpret_cast<const void *>(level_project_kernel<256>),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)((size_t)PT * 264 * 2 + 17408 + 9216)), "dynamic LDS size");
-        attr_set = true;
-    }
-    if (es.failed()) return;
     KernelTimer kt("level_project_kernel");
-    // One workgroup per 128 tokens takes all projections, which reads x once; where that leaves compute units idle or the
-    // last round nearly empty the projections are shared out, at about half a projection's time for another staging of x
-    // (500 tokens, nine projections of 256: 62 us on four workgroups, 18 on 36).
-    const int tiles = ceil_div(n, PT), cus = compute_units();
-    int parts = 1;
-    double best = 0;
-    for (int p = 1; p <= P; p++) {
-        const double time = ceil_div((long long)tiles * p, cus) * (ceil_div(P, p) + 0.5);
-        if (p == 1 || time < 0.95 * best) { best = time; parts = p; }
-    }
-    const dim3 grid((unsigned)tiles, (unsigned)parts);
-    if (d == 512) hipLaunchKernelGGL(level_project_kernel<512>, grid, dim3(kPThr), lds, stream(), a);
-    else hipLaunchKernelGGL(level_project_kernel<256>, grid, dim3(kPThr), lds, stream(), a);
+    if (d == 512) project_launch<512>(a, n, P); else project_launch<256>(a, n, P);
     check_launch("level_project_kernel");
 }
 

@@ -319,6 +319,34 @@ def test_projections_shared_out_are_those_of_one_workgroup(n_extra, levels):
         assert torch.equal(p, q), i
 
 
+@pytest.mark.parametrize("s,nh", [(1, 4), (31, 8), (33, 4), (97, 8), (129, 4), (161, 8)])
+def test_projections_of_few_tokens_are_those_of_many(s, nh):
+    """32 tokens by one projection a workgroup while those are few, 128 tokens by one or several, and by all: the same sums
+    in the same order."""
+    levels, n_extra = 2, 3
+    P, d, cus = n_extra + 3 * levels, nh * 64, torch.cuda.get_device_properties(0).multi_processor_count
+    x, w_extra, w_levels, gates = make_inputs(1, s, nh, levels, n_extra, s + nh)
+    params = [dev(g[k]) for g in gates for k in GATE_NAMES]
+    middle = (2 * cus // (3 * P) + 1) * 128 // s + 1
+    res = []
+    for bs in (1, middle, cus * 128 // s + 1):
+        n = bs * s
+        xd, we, wl = dev(np.tile(x, (bs, 1))), dev(w_extra), dev(w_levels)
+        extra = [torch.zeros(n, d, dtype=BF, device="cuda") for _ in range(n_extra)]
+        xb = torch.zeros(n, d, dtype=BF, device="cuda")
+        heads = [torch.zeros(levels * bs * nh, s, 64, dtype=BF, device="cuda") for _ in range(3)]
+        hg = [torch.zeros(levels * bs * nh, s, device="cuda") for _ in range(3)]
+        tm = [torch.zeros(levels, n, device="cuda") for _ in range(5)]
+        lib.level_project_forward_bf16_rocm(xd.data_ptr(), we.data_ptr(), n_extra, ptr_array(extra), wl.data_ptr(), ptr_array(params),
+                                            xb.data_ptr(), *[t.data_ptr() for t in (*heads, *hg, *tm)], bs, s, nh, 64, levels, 1e-8)
+        torch.cuda.synchronize()
+        res.append([t.view(bs, s, -1)[b].clone() for t in (*extra, xb) for b in (0, bs - 1)]
+                   + [t.view(levels, bs, nh, s, -1)[:, b].clone() for t in (*heads, *hg) for b in (0, bs - 1)]
+                   + [t.view(levels, bs, s)[:, b].clone() for t in tm for b in (0, bs - 1)])
+    for i, (p, q, r) in enumerate(zip(*res)):
+        assert torch.equal(p, q) and torch.equal(q, r), i
+
+
 def test_layer_with_single_bf16_projections_matches_autograd():
     """The whole layer on the path that issues no GEMM from Python, against the float64 autograd restatement:
     all levels active, then with a frozen level (sequence shorter than its period)."""
