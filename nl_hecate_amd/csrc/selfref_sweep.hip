@@ -5,26 +5,31 @@
 //     dg_t = F_k^T dk_t + F_v^T dv_t + F_q^T dq_t + de_t csE + da_t csA,   dG_t = (1-a_t) dG_{t+1} + dg_t x_t^T + dp_t q_t^T.
 // The part of dG that dp q^T drives depends on nothing the sweep produces, so its W, Z, and with them a first part of
 // dk, dv, dth and dg, come from selfref_bwd_prepare_kernel (one workgroup per chunk, the whole chip), as do the outer
-// products of those parts that make up dF.  What is left for selfref_bwd_sweep_kernel (one workgroup per chain) is the
+// products of those parts that make up dF.  The gradients of F_q and F_mem and their share of dG at the boundaries need nothing
+// else: selfref_bwd_scan_kernel, selfref_bwd_share_kernel.  What is left for selfref_bwd_sweep_kernel (one workgroup per chain) is the
 // part that dg x^T and the chunk boundary drive, carried as Y_s = F_k^T Z_s + (F_k - F_v)^T W_s:
 //     Y_s <- (1-a_t) Y_s + (F_k^T x_t) (dg_t . u_s) + ((F_k - F_v)^T dg_t) (x_t . k_s)      for the earlier tokens s of a tile
 //     dg_s = dg0_s - th_s Y_s + de_s csE + da_s csA
 // so that a token takes one exchange (dg_t), one product with a matrix and the dots of dg_t with the tile's u_s.
 //
 // 64 chains of 2048 tokens, head size 64, chunks of 64: preparation 0.36 ms (one workgroup per compute unit for its LDS;
-// 0.10 are matrix instructions), sweep 1.45 ms: 850 clocks a token (115 instructions of one wave per SIMD and the exchange),
-// 7 k clocks a tile and 26 k a chunk boundary, most of those matrix instructions.  The sweep that formed w, z, dk, dv and the
+// 0.10 are matrix instructions), scan 0.06 and share 0.03, sweep 1.30 ms: 870 clocks a token (115 instructions of one wave per
+// SIMD and the exchange), 6.7 k clocks a tile and 15 k a chunk boundary, most of those matrix instructions.  The sweep that formed w, z, dk, dv and the
 // update of dG token by token took 3.16 ms behind 0.23 ms of preparation; without self-generated values it is still the one
 // (selfref.hip), since there dh_t comes back as a second vector.
 //
-// The sweep has two waves for each 16 rows.  The first half does what the tokens wait for, and across a chunk boundary the
-// gradients of F_q and F_mem; the second half those of F_k and F_v, at the boundary and from every tile's dk and dv, stores
-// dg, and brings the next boundary's matrices into LDS while the first is among the tokens.  One wave a SIMD did all of it
+// The sweep has two waves for each 16 rows.  The first half does what the tokens wait for; the second half the gradients of F_k
+// and F_v, from every tile's dk and dv and across the boundaries, stores dg, and brings the next tile's inputs and the next
+// boundary's matrices into LDS while the first is among the tokens.  One wave a SIMD did all of it
 // in 1.60 ms (9.5 k clocks a tile, 34 k a boundary, half of either with the matrix cores idle; 774 a token: the second wave
-// costs the tokens some issue slots and the registers beyond 256).
+// costs the tokens some issue slots and the registers beyond 256).  With F_q and F_mem in the sweep, each half two
+// memories at a boundary and the first half its own inputs, it was 1.45 ms (7.7 k a tile, 26 k a boundary).  A matrix instruction of
+// the second half keeps the first from issuing for as long: forming dF across the boundary among the tokens hides its
+// latencies, not its instructions.
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
+#include <utility>
 
 #include "../../include/nl_hecate_ffi.h"
 #include "lane_ops.h"
@@ -57,7 +62,7 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_prepare_kernel(
     const float *__restrict__ v_cache, const float *__restrict__ q_cache, const float *__restrict__ alpha_cache,
     const float *__restrict__ theta_cache, const float *__restrict__ amean_cache,
     const float *__restrict__ emean_cache, const float *__restrict__ frozen, float *__restrict__ gl,
-    float *__restrict__ tok, float *__restrict__ outer, float *__restrict__ csv, int s, int C, int nc) {
+    float *__restrict__ tok, float *__restrict__ outer, float *__restrict__ csv, float *__restrict__ d_mems, int s, int C, int nc) {
     constexpr int KT = D / 16, NW = D / 16, NT = 4 * D, DD = D * D, KL = D + 4, V4 = D / 4, TPW = 4 / NW;
     constexpr int TF = sweep_token_floats(D);
     using P = PrepareLds<D>;
@@ -346,7 +351,8 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_prepare_kernel(
             }
         }
     }
-    // outer products: dF_k, dF_v, dF_q with g, dF_mem with p; stored as the sweep's lanes hold them
+    // outer products: dF_k, dF_v, dF_q with g, dF_mem with p; the first two stored as the sweep's lanes hold them, the others
+    // as matrices
     float dy[kLrC / 4];
 #pragma unroll
     for (int i = 0; i < kLrC / 4; i++) {
@@ -392,20 +398,193 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_prepare_kernel(
                 const float bg = e[3 * kLrC * KL + 16 * jt + ml], bp = e[4 * kLrC * KL + 16 * jt + ml];
                 o[0][jt] = mfma4(ak, bg, o[0][jt]);
                 o[1][jt] = mfma4(av, bg, o[1][jt]);
-                o[2][jt] = mfma4(aq, bg, o[2][jt]);
-                o[3][jt] = mfma4(ay, bp, o[3][jt]);
+                o[2][jt] = mfma4(bg, aq, o[2][jt]);
+                o[3][jt] = mfma4(bp, ay, o[3][jt]);
             }
         }
     }
 #pragma unroll
-    for (int c = 0; c < 4; c++) {
+    for (int jt = 0; jt < KT; jt++) {
 #pragma unroll
-        for (int jt = 0; jt < KT; jt++)
+        for (int c = 0; c < 2; c++)
             *reinterpret_cast<f32x4 *>(outer + (chunk * 4 + c) * DD + ((size_t)(wave * KT + jt) * 64 + lane) * 4) = o[c][jt];
+#pragma unroll
+        for (int c = 2; c < 4; c++) {
+            const int at = (wr + ml) * D + 16 * jt + 4 * kg;
+            if (nc > 1) *reinterpret_cast<f32x4 *>(outer + (chunk * 4 + c) * DD + at) = o[c][jt];
+            else *reinterpret_cast<f32x4 *>(d_mems + (b * 6 + (c == 2 ? 2 : 5)) * DD + at) = o[c][jt];   // no chunk passes them on
+        }
     }
 }
 
+// ── matrices ─────────────────────────────────────────────────────────────────────────────────────────────────────
+// What a chunk's tokens add to dF whatever the sweep finds: the lane's part of a wave's 16 rows.
+template <int D>
+__device__ __forceinline__ void token_sums(f32x4 (&sums)[D / 16], const float *outer, int tid) {
+    constexpr int JT = D / 16;
+#pragma unroll
+    for (int jt = 0; jt < JT; jt++)
+        sums[jt] = *reinterpret_cast<const f32x4 *>(outer + ((size_t)((tid >> 6) * JT + jt) * 64 + (tid & 63)) * 4);
+}
+
+// A wave's 16 rows of a matrix in LDS from its accumulators.
+template <int D>
+__device__ __forceinline__ void put_rows(float *m, const f32x4 (&x)[D / 16], int tid) {
+    const int lane = tid & 63, row = 16 * (tid >> 6) + 4 * (lane >> 4);
+#pragma unroll
+    for (int jt = 0; jt < D / 16; jt++) {
+#pragma unroll
+        for (int v = 0; v < 4; v++) m[(row + v) * (D + 4) + 16 * jt + (lane & 15)] = x[jt][v];
+    }
+}
+
+// A matrix by way of registers to LDS, 4 D threads.
+template <int D>
+__device__ __forceinline__ void request_matrix(f32x4 (&m)[D / 16], const float *f, int tid) {
+#pragma unroll
+    for (int i = 0; i < D / 16; i++) m[i] = *reinterpret_cast<const f32x4 *>(f + (tid + i * 4 * D) * 4);
+}
+template <int D>
+__device__ __forceinline__ void stage_matrix(float *Fs, const f32x4 (&m)[D / 16], int tid) {
+#pragma unroll
+    for (int i = 0; i < D / 16; i++) {
+        const int e = tid + i * 4 * D;
+        *reinterpret_cast<f32x4 *>(Fs + (e / (D / 4)) * (D + 4) + (e % (D / 4)) * 4) = m[i];
+    }
+}
+
+// acc += F_0^T B_0 + .. + F_(N-1)^T B_(N-1), the wave's 16 rows: contraction in the order 16 c + 4 kg + v, since rows 4 apart put
+// the four kg of a read on different banks.  Operands are read two steps ahead: left to the compiler, a read stands right
+// before its use.
+template <int D, int N>
+__device__ __forceinline__ void share_products(const float *const (&F)[N], const float *const (&B)[N], f32x4 (&acc)[D / 16], int wr,
+                                               int ml, int kg) {
+    constexpr int JT = D / 16, LD = D + 4, STEPS = D / 4;
+    float a[3], b[3][JT];
+    auto read = [&](int i) __attribute__((always_inline)) {
+        const int k = 16 * (i % STEPS >> 2) + 4 * kg + (i & 3);
+        a[i % 3] = F[i / STEPS][k * LD + wr + ml];
+#pragma unroll
+        for (int jt = 0; jt < JT; jt++) b[i % 3][jt] = B[i / STEPS][k * LD + 16 * jt + ml];
+    };
+    read(0);
+    read(1);
+#pragma unroll
+    for (int i = 0; i < N * STEPS; i++) {
+        if (i + 2 < N * STEPS) read(i + 2);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int jt = 0; jt < JT; jt++) acc[jt] = mfma4(a[i % 3], b[i % 3][jt], acc[jt]);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+// Part c < KT of acc += B G_L^T, the wave's 16 rows, which are all it needs of B.
+template <int D>
+__device__ __forceinline__ void pass_part(const float *Bm, const float *GLT, f32x4 (&acc)[D / 16], int c, int wr, int ml, int kg) {
+    constexpr int JT = D / 16, LD = D + 4;
+    const f32x4 a = *reinterpret_cast<const f32x4 *>(Bm + (wr + ml) * LD + 16 * c + 4 * kg);
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+        const int k = 16 * c + 4 * kg + v;
+#pragma unroll
+        for (int jt = 0; jt < JT; jt++) acc[jt] = mfma4(a[v], GLT[k * LD + 16 * jt + ml], acc[jt]);
+    }
+}
+
+// ── the gradients of F_q and F_mem ───────────────────────────────────────────────────────────────────────────────
+// Nothing of the sweep reaches them: dF_c <- dF'_c G_L^T + what the chunk's tokens add, chunk by chunk backwards, a row by
+// itself.  A wave takes 16 rows of one of the two through a chain; its lane (ml, kg) holds row ml, columns 16 kt + 4 kg + v, operand and
+// result of the product at once, and G_L comes straight from memory, two chunks ahead.  The matrices of `outer` become dF_c in place.
+// 64 chains of 32 chunks, head size 64: 62 us, matrix instructions 27 of them.
+template <int D>
+__global__ __launch_bounds__(64) void selfref_bwd_scan_kernel(const float *__restrict__ gl, float *__restrict__ outer,
+                                                              float *__restrict__ d_mems, int nc, int batch) {
+    constexpr int KT = D / 16, DD = D * D;
+    const int lane = threadIdx.x, ml = lane & 15, kg = lane >> 4;
+    const size_t b = blockIdx.x % batch;   // the waves of a chain share an XCD's L2
+    const int c = blockIdx.x / batch & 1, row0 = 16 * (blockIdx.x / batch >> 1);
+    float *rows = outer + (b * nc * 4 + 2 + c) * DD + (row0 + ml) * D + 4 * kg;
+    const float *g = gl + b * nc * DD + ml * D + 4 * kg;
+    f32x4 f[KT], G[2][KT][KT], sums[2][KT];
+    auto request = [&](int ci, int set) __attribute__((always_inline)) {
+#pragma unroll
+        for (int kt = 0; kt < KT; kt++) {
+            sums[set][kt] = *reinterpret_cast<const f32x4 *>(rows + (size_t)ci * 4 * DD + 16 * kt);
+#pragma unroll
+            for (int jt = 0; jt < KT; jt++) G[set][kt][jt] = *reinterpret_cast<const f32x4 *>(g + (size_t)ci * DD + 16 * jt * D + 16 * kt);
+        }
+    };
+    // Loads and stores stand on every path: the memory counter is in order, and behind a branch a wait would be for all of them.
+    auto step = [&](int ci, int set) __attribute__((always_inline)) {
+        f32x4 acc[KT];
+#pragma unroll
+        for (int jt = 0; jt < KT; jt++) acc[jt] = kZero;
+#pragma unroll
+        for (int kt = 0; kt < KT; kt++) {
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+#pragma unroll
+                for (int jt = 0; jt < KT; jt++) acc[jt] = mfma4(G[set][kt][jt][v], f[kt][v], acc[jt]);
+            }
+        }
+#pragma unroll
+        for (int jt = 0; jt < KT; jt++) f[jt] = acc[jt] + sums[set][jt];
+        __builtin_amdgcn_sched_barrier(0);
+        request(max(ci - 2, 0), set);
+#pragma unroll
+        for (int jt = 0; jt < KT; jt++) *reinterpret_cast<f32x4 *>(rows + (size_t)ci * 4 * DD + 16 * jt) = f[jt];
+        __builtin_amdgcn_sched_barrier(0);
+    };
+#pragma unroll
+    for (int kt = 0; kt < KT; kt++) f[kt] = *reinterpret_cast<const f32x4 *>(rows + (size_t)(nc - 1) * 4 * DD + 16 * kt);
+    request(max(nc - 2, 0), 0);
+    request(max(nc - 3, 0), 1);
+    int ci = nc - 2;
+    for (; ci >= 1; ci -= 2) {
+        step(ci, 0);
+        step(ci - 1, 1);
+    }
+    if (ci == 0) step(0, 0);
+    float *out = d_mems + (b * 6 + (c ? 5 : 2)) * DD + (row0 + ml) * D + 4 * kg;
+#pragma unroll
+    for (int jt = 0; jt < KT; jt++) *reinterpret_cast<f32x4 *>(out + 16 * jt) = f[jt];
+}
+
+// Their share of dG_L at the end of every chunk but a chain's last: F_q^T dF'_q + F_mem^T dF'_mem, in place of the next chunk's
+// dF_q and in the order of the sweep's lanes.  A workgroup per chunk, one memory after the other.  26 us for 1984 chunks at
+// head size 64: 80 KB a chunk, 14 us of matrix instructions.
+template <int D>
+__global__ __launch_bounds__(4 * D) void selfref_bwd_share_kernel(const float *__restrict__ frozen, float *__restrict__ outer, int nc) {
+    constexpr int JT = D / 16, DD = D * D, LD = D + 4;
+    __shared__ __align__(16) float Fs[D * LD], Bm[D * LD];
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, ml = lane & 15, kg = lane >> 4, wr = 16 * wave;
+    const size_t chunk = blockIdx.x / (nc - 1) * nc + blockIdx.x % (nc - 1);
+    const float *fz = frozen + chunk * 6 * DD;
+    float *df = outer + ((chunk + 1) * 4 + 2) * DD;
+    f32x4 acc[JT], f[2][JT], d[2][JT];
+    request_matrix<D>(f[0], fz + 2 * DD, tid);
+    request_matrix<D>(d[0], df, tid);
+    request_matrix<D>(f[1], fz + 5 * DD, tid);
+    request_matrix<D>(d[1], df + DD, tid);
+#pragma unroll
+    for (int jt = 0; jt < JT; jt++) acc[jt] = kZero;
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
+        if (c) __syncthreads();
+        stage_matrix<D>(Fs, f[c], tid);
+        stage_matrix<D>(Bm, d[c], tid);
+        __syncthreads();
+        share_products<D, 1>({Fs}, {Bm}, acc, wr, ml, kg);
+    }
+#pragma unroll
+    for (int jt = 0; jt < JT; jt++) *reinterpret_cast<f32x4 *>(df + ((size_t)(wave * JT + jt) * 64 + lane) * 4) = acc[jt];
+}
+
 // ── the sweep ────────────────────────────────────────────────────────────────────────────────────────────────────
+template <class Fn, int... I>
+__device__ __forceinline__ void for_each(Fn &f, std::integer_sequence<int, I...>) {
+    (f(std::integral_constant<int, I>{}), ...);
+}
 // f(4 J + 3) ... f(4 J) with the argument as a type, if the tile has tokens there
 template <int J, class Fn>
 __device__ __forceinline__ void four_down(Fn &f, int nt) {
@@ -445,70 +624,9 @@ __device__ __forceinline__ void across_rows3(float &a, float &b, float &c) {
     a += a1; b += b1; c += c1;
 }
 
-// dynamic LDS of the sweep: a tile's arrays; G_L^T, two F, dF' of the second half; dF of the first half; dk and dv
-constexpr int sweep_tile_floats(int d) { return 8 * kTB * (d + 4); }
-constexpr int sweep_lds_floats(int d) { return sweep_tile_floats(d) + 6 * d * (d + 4) + d / 16 * 8 * 64; }
-
-// What a chunk's tokens add to dF whatever the sweep finds: the lane's part of a wave's 16 rows.
-template <int D>
-__device__ __forceinline__ void token_sums(f32x4 (&sums)[D / 16], const float *outer, int tid) {
-    constexpr int JT = D / 16;
-#pragma unroll
-    for (int jt = 0; jt < JT; jt++)
-        sums[jt] = *reinterpret_cast<const f32x4 *>(outer + ((size_t)((tid >> 6) * JT + jt) * 64 + (tid & 63)) * 4);
-}
-
-// A wave's 16 rows of a matrix in LDS from its accumulators.
-template <int D>
-__device__ __forceinline__ void put_rows(float *m, const f32x4 (&x)[D / 16], int tid) {
-    const int lane = tid & 63, row = 16 * (tid >> 6) + 4 * (lane >> 4);
-#pragma unroll
-    for (int jt = 0; jt < D / 16; jt++) {
-#pragma unroll
-        for (int v = 0; v < 4; v++) m[(row + v) * (D + 4) + 16 * jt + (lane & 15)] = x[jt][v];
-    }
-}
-
-// F_c of a chunk boundary, a workgroup half's part of each thread.
-template <int D>
-__device__ __forceinline__ void request_matrix(f32x4 (&m)[D / 16], const float *f, int tid) {
-#pragma unroll
-    for (int i = 0; i < D / 16; i++) m[i] = *reinterpret_cast<const f32x4 *>(f + (tid + i * 4 * D) * 4);
-}
-template <int D>
-__device__ __forceinline__ void stage_matrix(float *Fs, const f32x4 (&m)[D / 16], int tid) {
-#pragma unroll
-    for (int i = 0; i < D / 16; i++) {
-        const int e = tid + i * 4 * D;
-        *reinterpret_cast<f32x4 *>(Fs + (e / (D / 4)) * (D + 4) + (e % (D / 4)) * 4) = m[i];
-    }
-}
-
-// One memory across a chunk boundary: accG += F_c^T dF'_c, accN = dF'_c G_L^T.
-template <int D>
-__device__ __forceinline__ void boundary_products(const float *Fs, const float *Bm, const float *GLT, f32x4 (&accG)[D / 16],
-                                                  f32x4 (&accN)[D / 16], int tid) {
-    constexpr int KT = D / 16, JT = D / 16, LD = D + 4;
-    asm volatile("" : "+v"(tid));   // addresses made of it are not to live across the sweep
-    const int wave = tid >> 6, lane = tid & 63, ml = lane & 15, kg = lane >> 4, wr = 16 * wave;
-#pragma unroll
-    for (int jt = 0; jt < JT; jt++) accN[jt] = kZero;
-    // contraction in the order 16 c + 4 kg + v: rows 4 apart put the four kg of a read on different banks
-#pragma unroll
-    for (int c = 0; c < KT; c++) {
-        const f32x4 a2 = *reinterpret_cast<const f32x4 *>(Bm + (wr + ml) * LD + 16 * c + 4 * kg);  // dF'_c
-#pragma unroll
-        for (int v = 0; v < 4; v++) {
-            const int k = 16 * c + 4 * kg + v;
-            const float a1 = Fs[k * LD + wr + ml];  // F_c^T
-#pragma unroll
-            for (int jt = 0; jt < JT; jt++) {
-                accG[jt] = mfma4(a1, Bm[k * LD + 16 * jt + ml], accG[jt]);
-                accN[jt] = mfma4(a2[v], GLT[k * LD + 16 * jt + ml], accN[jt]);
-            }
-        }
-    }
-}
+// dynamic LDS of the sweep: a tile's inputs, twice; dg; G_L^T; F and dF' of k and v; dk and dv
+constexpr int sweep_tile_floats(int d) { return kTB * (5 * (d + 4) + d + 16); }
+constexpr int sweep_lds_floats(int d) { return 2 * sweep_tile_floats(d) + kTB * (d + 4) + 5 * d * (d + 4) + d / 16 * 8 * 64; }
 
 // One workgroup per chain, two waves per 16 rows (above).  Lane (ml, kg) = (lane % 16, lane / 16) holds of every matrix row ml of
 // the wave's rows, columns CP kg + i (CP = D / 4): operand and result of the tile products (the contraction index runs
@@ -523,20 +641,21 @@ __global__ __launch_bounds__(8 * D) void selfref_bwd_sweep_kernel(
     float *__restrict__ d_mems, int s, int C, int nc) {
     constexpr int CP = D / 4, KT = D / 16, JT = D / 16, NT = 4 * D, NW = D / 16, DD = D * D, V4 = D / 4, LD = D + 4;
     constexpr int TF = sweep_token_floats(D), TILE = kTB * LD;
-    enum { A_K, A_U, A_X, A_DG0, A_FX, A_DG, A_W, A_Z, A_COUNT };
-    static_assert(A_COUNT == 8);
-    extern __shared__ __align__(16) float raw[];
-    float *const GLT = raw + sweep_tile_floats(D), *const Fa = GLT + D * LD, *const Fb = Fa + D * LD, *const Bm = Fb + D * LD;
-    float *const kept = Bm + D * LD;                 // the gradients of F_q and F_mem between the boundaries
-    float *const dkv = kept + 2 * D * LD;            // dk, dv of a tile's tokens: [wave][v][2][lane]
     constexpr int LG = D + 16;                       // rows 4 v + kg of g fall on different banks for the four kg
-    __shared__ __align__(16) float tg[kTB * LG];     // g
-    __shared__ __align__(16) float gam[kTB * kTB];   // x_t . k_s, s in the order sigma
-    __shared__ __align__(16) float sc[kTB][8];       // alpha, theta, sigmoid' / (d keep), softplus' / d, dth0, dp . p
+    enum { A_K, A_U, A_X, A_DG0, A_FX };             // and g behind them
+    extern __shared__ __align__(16) float raw[];
+    constexpr int SET = sweep_tile_floats(D);
+    static_assert(SET >= D * LD, "dG_L in the place of a tile's inputs");
+    float *const DG = raw + 2 * SET, *const GLT = DG + TILE, *const Fa = GLT + D * LD, *const Fb = Fa + D * LD;   // G_L^T, F_k, F_v
+    float *const Ba = Fb + D * LD, *const Bb = Ba + D * LD;   // dF'_k, dF'_v
+    float *const dkv = Bb + D * LD;                  // dk, dv of a tile's tokens: [wave][v][2][lane]
+    __shared__ __align__(16) float gams[2][kTB * kTB];   // x_t . k_s, s in the order sigma
+    __shared__ __align__(16) float scs[2][kTB][8];       // alpha, theta, sigmoid' / (d keep), softplus' / d, dth0, dp . p
     __shared__ __align__(16) float Sx[NW][kTB], Cx[NW][kTB];
-    __shared__ __align__(16) float av[2][D];
+    __shared__ __align__(16) float av[2][D], av1[2][D];   // accE, accA at a boundary, before and behind it
     __shared__ float sp[NW];
-#define T_(a, t, i) raw[(a) * TILE + (t) * LD + (i)]
+#define T_(a, t, i) set[(a) * TILE + (t) * LD + (i)]
+#define DG_(t, i) DG[(t) * LD + (i)]
 
     const bool second = __builtin_amdgcn_readfirstlane(threadIdx.x) >= NT;
     const int tid = second ? threadIdx.x - NT : threadIdx.x, r = tid >> 2, cq = tid & 3, wave = tid >> 6, lane = tid & 63;
@@ -549,44 +668,104 @@ __global__ __launch_bounds__(8 * D) void selfref_bwd_sweep_kernel(
     float *dmb = d_mems + b * 6 * DD;
     if (second) {   // the gradients of F_k and F_v, and as many barriers as the first half meets
         f32x4 dFm[2][JT];
-        for (int ci = nc - 1; ci >= 0; ci--) {
+        // Inputs of a tile: requested while the tile two before it is worked on, and in LDS while the tile before it is, in the
+        // set that that one does not use.  Rows behind a chunk's last token are zeros.
+        float4 pf_k, pf_v, pf_x, pf_g, pf_dg, pf_fx, pf_gam;
+        float pf_s[6];
+        int pf_ci = nc - 1, pf_tile = (s - (nc - 1) * C - 1) / kTB, pf_nt = 0;   // the tile to request; tokens of the one requested
+        // No branch around the loads: the memory counter is in order, and behind a branch a wait would be for all of them.
+        auto request = [&](int me) __attribute__((always_inline)) {
+            const int first = pf_ci * C + pf_tile * kTB, last = min(pf_ci * C + C, s) - 1, stt = me / V4, sj = (me % V4) * 4;
+            pf_nt = min(kTB, last + 1 - first);
+            const size_t at = tok0 + min(first + stt, last), o = at * D + sj;
+            const float *tp = tok + at * TF;
+            auto two = [&](const float *q) {  // rows of tok are 8 bytes aligned
+                const float2 lo = *reinterpret_cast<const float2 *>(q), hi = *reinterpret_cast<const float2 *>(q + 2);
+                return make_float4(lo.x, lo.y, hi.x, hi.y);
+            };
+            pf_k = *reinterpret_cast<const float4 *>(k_cache + o);
+            pf_v = *reinterpret_cast<const float4 *>(v_cache + o);
+            pf_x = *reinterpret_cast<const float4 *>(emb + o);
+            pf_g = two(tp + sj);
+            pf_dg = two(tp + D + sj);
+            pf_fx = two(tp + 2 * D + sj);
+            pf_gam = two(tok + (tok0 + min(first + (me >> 2 & 15), last)) * TF + 3 * D + 4 * (me & 3));
+            const float *e = tok + (tok0 + min(first + (me & 15), last)) * TF + 3 * D + 16;
+#pragma unroll
+            for (int i = 0; i < 6; i++) pf_s[i] = e[i];
+            if (pf_tile > 0) pf_tile--;
+            else if (pf_ci > 0) { pf_ci--; pf_tile = (C - 1) / kTB; }   // behind the last tile: it again, not used
+        };
+        auto stage = [&](int buf, int me) __attribute__((always_inline)) {
+            float *set = raw + buf * SET;
+            const int stt = me / V4, sj = (me % V4) * 4;
+            auto in = [&](const float4 &x, int t) { return t < pf_nt ? x : make_float4(0, 0, 0, 0); };
+            const float4 k = in(pf_k, stt), v = in(pf_v, stt);
+            *reinterpret_cast<float4 *>(&T_(A_K, stt, sj)) = k;
+            *reinterpret_cast<float4 *>(&T_(A_U, stt, sj)) = make_float4(k.x - v.x, k.y - v.y, k.z - v.z, k.w - v.w);
+            *reinterpret_cast<float4 *>(&T_(A_X, stt, sj)) = in(pf_x, stt);
+            *reinterpret_cast<float4 *>(&T_(A_DG0, stt, sj)) = in(pf_dg, stt);
+            *reinterpret_cast<float4 *>(&T_(A_FX, stt, sj)) = in(pf_fx, stt);
+            *reinterpret_cast<float4 *>(set + 5 * TILE + stt * LG + sj) = in(pf_g, stt);
+            if (me < 64) *reinterpret_cast<float4 *>(&gams[buf][4 * me]) = in(pf_gam, me >> 2);
+            if (me < kTB) {   // zeros behind the last token: it passes everything on as it is
+                float x[6];
+#pragma unroll
+                for (int i = 0; i < 6; i++) x[i] = me < pf_nt ? pf_s[i] : 0.f;
+                *reinterpret_cast<f32x4 *>(&scs[buf][me][0]) = f32x4{x[0], x[1], x[2], x[3]};
+                *reinterpret_cast<float2 *>(&scs[buf][me][4]) = make_float2(x[4], x[5]);
+            }
+        };
+        request(tid);
+        stage(0, tid);
+        request(tid);
+        for (int ci = nc - 1, buf = 0; ci >= 0; ci--) {
             const int t0 = ci * C, L = min(C, s - t0), ntile = (L + kTB - 1) / kTB;
             const size_t chunk = b * nc + ci;
             const float *fz = frozen + chunk * 6 * DD;
             int me = tid;
             asm volatile("" : "+v"(me));
             const int wave = me >> 6, lane = me & 63, ml = lane & 15, kg = lane >> 4;
-            if (ci < nc - 1) put_rows<D>(Bm, dFm[0], me);
+            if (ci < nc - 1) {
+                put_rows<D>(Ba, dFm[0], me);
+                put_rows<D>(Bb, dFm[1], me);
+            }
             lds_barrier();
             if (ci < nc - 1) {
-                f32x4 accG[JT], accN[JT], sums[2][JT], Fv[JT], Fm[JT];
-                request_matrix<D>(Fv, fz + DD, me);
-                request_matrix<D>(Fm, fz + 5 * DD, me);
-                token_sums<D>(sums[0], outer + chunk * 4 * DD, me);
-                token_sums<D>(sums[1], outer + (chunk * 4 + 1) * DD, me);
+                // accE <- G_L accE, accA <- G_L accA: rows 0 and 1 of one more product
+                f32x4 accV[KT];
 #pragma unroll
-                for (int i = 0; i < JT; i++) accG[i] = kZero;
+                for (int c = 0; c < KT; c++) {
+                    const f32x4 a = ml < 2 ? *reinterpret_cast<const f32x4 *>(&av[ml][16 * c + 4 * kg]) : kZero;
+                    accV[c] = kZero;
 #pragma unroll
-                for (int c = 0; c < 2; c++) {
-                    if (c) {
-                        stage_matrix<D>(Fa, Fv, me);
-                        stage_matrix<D>(Fb, Fm, me);
-                        put_rows<D>(Bm, dFm[1], me);
-                        lds_barrier();
-                    }
-                    boundary_products<D>(Fa, Bm, GLT, accG, accN, me);
-#pragma unroll
-                    for (int jt = 0; jt < JT; jt++) dFm[c][jt] = accN[jt] + sums[c][jt];
-                    lds_barrier();   // every wave has read its matrices
+                    for (int v = 0; v < 4; v++) accV[c] = mfma4(a[v], GLT[(16 * c + 4 * kg + v) * LD + 16 * wave + ml], accV[c]);
                 }
-                put_rows<D>(Bm, accG, me);
-                lds_barrier();   // the first half adds them up
-                lds_barrier();
+#pragma unroll
+                for (int c = 1; c < KT; c++) accV[0] += accV[c];
+                if (kg == 0) { av1[0][16 * wave + ml] = accV[0][0]; av1[1][16 * wave + ml] = accV[0][1]; }
+                lds_barrier();   // dG_L is there
             } else {
                 token_sums<D>(dFm[0], outer + chunk * 4 * DD, me);
                 token_sums<D>(dFm[1], outer + (chunk * 4 + 1) * DD, me);
             }
-            f32x4 Fk[JT], Fq[JT];
+            // Across the boundary dF_c = dF'_c G_L^T + what the tokens add: nobody waits for it, so it is formed while the other
+            // half is among the tokens of the chunk's last tile, a part behind a barrier.
+            f32x4 across[JT], sums[JT];
+            auto pass = [&](auto part) {
+                constexpr int c = decltype(part)::value / KT, q = decltype(part)::value % KT;
+                if (q == 0) {
+                    token_sums<D>(sums, outer + (chunk * 4 + c) * DD, me);
+#pragma unroll
+                    for (int jt = 0; jt < JT; jt++) across[jt] = kZero;
+                }
+                pass_part<D>(c ? Bb : Ba, GLT, across, q, 16 * wave, ml, kg);
+                if (q == KT - 1) {
+#pragma unroll
+                    for (int jt = 0; jt < JT; jt++) dFm[c][jt] = across[jt] + sums[jt];
+                }
+            };
+            f32x4 Fk[JT], Fv[JT];
             float G[CP];
             // A tile's share of dF, its dg and the next boundary's matrices wait in registers until the other half is among the
             // tokens of the tile after it, which leave the matrix cores alone; a part of them behind each of four barriers, so
@@ -604,16 +783,19 @@ __global__ __launch_bounds__(8 * D) void selfref_bwd_sweep_kernel(
                 if (v == 0 && tile * kTB + stt < L) *reinterpret_cast<f32x4 *>(d_emb + (tok0 + t0 + tile * kTB + stt) * D + sj) = dg;
                 if (v == 0 || ci == 0 || tile != ntile - 1) return;
                 if (v == 1) stage_matrix<D>(Fa, Fk, me);
-                if (v == 2) stage_matrix<D>(Fb, Fq, me);
+                if (v == 2) stage_matrix<D>(Fb, Fv, me);
                 if (v == 3) {
 #pragma unroll
                     for (int i = 0; i < CP; i++) GLT[((me & 3) * CP + i) * LD + (me >> 2)] = G[i];
                 }
             };
             using std::integral_constant;
-            for (int tile = ntile - 1; tile >= 0; tile--) {
+            for (int tile = ntile - 1; tile >= 0; tile--, buf ^= 1) {
                 const int nt = min(kTB, L - tile * kTB);
-                for (int i = 0; i < 4; i++) lds_barrier();   // top, tile staged, W and Z, the first token
+                const float *set = raw + buf * SET, *tg = set + 5 * TILE;
+                for (int i = 0; i < 3; i++) lds_barrier();   // top, W and Z, the first token
+                stage(buf ^ 1, me);
+                request(me);
                 if (tile < ntile - 1) pending(tile + 1, integral_constant<int, 0>{});
                 lds_barrier();
                 if (tile < ntile - 1) pending(tile + 1, integral_constant<int, 1>{});
@@ -625,9 +807,19 @@ __global__ __launch_bounds__(8 * D) void selfref_bwd_sweep_kernel(
                     const float *f = fz - 6 * DD;
                     lds_read<CP>(G, gl + (chunk - 1) * DD + (me >> 2) * D + (me & 3) * CP);
                     request_matrix<D>(Fk, f, me);
-                    request_matrix<D>(Fq, f + 2 * DD, me);
+                    request_matrix<D>(Fv, f + DD, me);
                 }
-                for (int i = 3; i < 4 * ((nt + 3) / 4); i++) lds_barrier();   // the other tokens in whole groups of four; dk, dv
+                int left = 4 * ((nt + 3) / 4) - 3;   // the other tokens in whole groups of four; dk, dv
+                if (tile == ntile - 1 && ci < nc - 1) {
+                    const bool spread = left > 2 * KT;
+                    auto next = [&](auto part) __attribute__((always_inline)) {
+                        if (spread) lds_barrier();
+                        pass(part);
+                    };
+                    for_each(next, std::make_integer_sequence<int, 2 * KT>{});
+                    left -= spread ? 2 * KT : 0;
+                }
+                for (int i = 0; i < left; i++) lds_barrier();
 #pragma unroll
                 for (int v = 0; v < 4; v++) {
                     op[v][0] = dkv[((wave * 4 + v) * 2) * 64 + lane];
@@ -635,7 +827,7 @@ __global__ __launch_bounds__(8 * D) void selfref_bwd_sweep_kernel(
 #pragma unroll
                     for (int jt = 0; jt < JT; jt++) gt[v][jt] = tg[(4 * v + kg) * LG + 16 * jt + ml];
                 }
-                dg = *reinterpret_cast<const f32x4 *>(&T_(A_DG, stt, sj));
+                dg = *reinterpret_cast<const f32x4 *>(DG + stt * LD + sj);
             }
             pending(0, integral_constant<int, 0>{});
             pending(0, integral_constant<int, 1>{});
@@ -658,143 +850,88 @@ __global__ __launch_bounds__(8 * D) void selfref_bwd_sweep_kernel(
     for (int i = 0; i < CP; i++) dG[i] = dGT[i] = 0.f;
     if (tid < NW * kTB) (&Sx[0][0])[tid] = 0.f;
 
-    float4 pf_k, pf_v, pf_x, pf_g, pf_dg, pf_fx, pf_gam;
-    float pf_s[6];
-    pf_k = pf_v = pf_x = pf_g = pf_dg = pf_fx = pf_gam = make_float4(0, 0, 0, 0);
+    // A chunk's share of dG_L and column sums of F_eta, F_alpha, requested in the last tile of the chunk behind it.
+    f32x4 share[JT], csr[2];
+    float cs1[2];
+    auto ahead = [&](size_t chunk, int me, bool behind) __attribute__((always_inline)) {
+        const int row = 16 * (me >> 6);
+        if (behind) token_sums<D>(share, outer + ((chunk + 1) * 4 + 2) * DD, me);   // of F_q and F_mem
+        const float *c = csv + chunk * 2 * D + row;
 #pragma unroll
-    for (int i = 0; i < 6; i++) pf_s[i] = 0.f;
-    for (int ci = nc - 1; ci >= 0; ci--) {
+        for (int i = 0; i < 2; i++) csr[i] = *reinterpret_cast<const f32x4 *>(c + i * D + 4 * (me >> 4 & 3));
+        cs1[0] = c[me & 15];
+        cs1[1] = c[D + (me & 15)];
+    };
+    ahead(b * nc + nc - 1, tid, false);
+    for (int ci = nc - 1, buf = 0; ci >= 0; ci--) {
         const int t0 = ci * C, L = min(C, s - t0), ntile = (L + kTB - 1) / kTB;
         const size_t chunk = b * nc + ci;
         const float *fz = frozen + chunk * 6 * DD;
         // the thread's place through an opaque copy, once per chunk: addresses made of it are not to live across the sweep
         int me = tid;
         asm volatile("" : "+v"(me));
-        const int r = me >> 2, cq = me & 3, wave = me >> 6, lane = me & 63, ml = lane & 15, kg = lane >> 4, wr = 16 * wave,
-                  c0 = cq * CP, stt = me / V4, sj = (me % V4) * 4;
-        // Inputs of a tile, requested one tile ahead; rows behind the chunk's last token are zeros.
-        auto request = [&](int first, int nt) {
-            const size_t o = (tok0 + first + stt) * D + sj;
-            const float *tp = tok + (tok0 + first + stt) * TF;
-            auto two = [&](const float *q) {  // rows of tok are 8 bytes aligned
-                const float2 lo = *reinterpret_cast<const float2 *>(q), hi = *reinterpret_cast<const float2 *>(q + 2);
-                return make_float4(lo.x, lo.y, hi.x, hi.y);
-            };
-            // branches: a choice of values is one of addresses to the compiler, and so a flat load, which the LDS barriers of
-            // the tokens would wait for
-            pf_k = pf_v = pf_x = pf_g = pf_dg = pf_fx = make_float4(0, 0, 0, 0);
-            if (stt < nt) {
-                pf_k = *reinterpret_cast<const float4 *>(k_cache + o);
-                pf_v = *reinterpret_cast<const float4 *>(v_cache + o);
-                pf_x = *reinterpret_cast<const float4 *>(emb + o);
-                pf_g = two(tp + sj);
-                pf_dg = two(tp + D + sj);
-                pf_fx = two(tp + 2 * D + sj);
-            }
-            if (tid < 64) {
-                pf_gam = make_float4(0, 0, 0, 0);
-                if (tid / 4 < nt) pf_gam = two(tok + (tok0 + first + tid / 4) * TF + 3 * D + 4 * (tid % 4));
-            }
-            if (tid < kTB) {  // zeros behind the last token: it passes everything on as it is
-#pragma unroll
-                for (int i = 0; i < 6; i++) pf_s[i] = 0.f;
-                if (tid < nt) {
-                    const float *e = tok + (tok0 + first + tid) * TF + 3 * D + 16;
-#pragma unroll
-                    for (int i = 0; i < 6; i++) pf_s[i] = e[i];
-                }
-            }
-        };
+        const int wave = me >> 6, lane = me & 63, ml = lane & 15, kg = lane >> 4, wr = 16 * wave;
         float FTk[CP], FTu[CP];   // rows of F_k^T and (F_k - F_v)^T
-        // column sums of F_eta, F_alpha
-        float csE = csv[chunk * 2 * D + wr + ml], csA = csv[chunk * 2 * D + D + wr + ml];
-        // LDS-only barriers from here on: the requests above and the stores of dg stay under way across them
+        float csE = cs1[0], csA = cs1[1];
+        // LDS-only barriers from here on: requests and the stores of dg stay under way across them
         if (ci < nc - 1 && kg == 0) { av[0][wr + ml] = accEA[0]; av[1][wr + ml] = accEA[1]; }
         lds_barrier();
         sig = 0.f;
         if (ci < nc - 1) {
             // Chunk boundary: gradients of F'_c = F_c G_L flow into dG_L = sum_c F_c^T dF'_c and dF_c = dF'_c G_L^T, on
             // the matrix cores; the rows of dF_eta, dF_alpha are all equal (rank-1 terms of dG_L).
-            float q[CP], G[CP];
-            const float e = csv[chunk * 2 * D + r], a = csv[chunk * 2 * D + D + r];
             f32x4 accG[JT];
 #pragma unroll
             for (int i = 0; i < JT; i++) accG[i] = kZero;
-            f32x4 dF[JT], sums[JT];
+            share_products<D, 2>({Fa, Fb}, {Ba, Bb}, accG, wr, ml, kg);
 #pragma unroll
-            for (int c = 0; c < 2; c++) {
-                if (c) {
-                    put_rows<D>(kept, dF, me);
-                    lds_barrier();
-                }
-                token_sums<D>(sums, outer + (chunk * 4 + 2 + c) * DD, me);
-#pragma unroll
-                for (int i = 0; i < CP; i++) (c ? FTu : FTk)[i] = Fa[(CP * kg + i) * LD + wr + ml];
-                boundary_products<D>(Fb, kept + c * D * LD, GLT, accG, dF, me);
-#pragma unroll
-                for (int jt = 0; jt < JT; jt++) dF[jt] += sums[jt];
-                if (c) request(t0 + (ntile - 1) * kTB, L - (ntile - 1) * kTB);
-                lds_barrier();  // every wave has read its matrices
+            for (int i = 0; i < CP; i++) {
+                FTk[i] = Fa[(CP * kg + i) * LD + wr + ml];
+                FTu[i] = Fb[(CP * kg + i) * LD + wr + ml];
             }
-            {   // accE <- G_L accE, accA <- G_L accA: rows 0 and 1 of one more product
-                f32x4 accV = kZero;
-#pragma unroll
-                for (int c = 0; c < KT; c++) {
-                    const f32x4 a = ml < 2 ? *reinterpret_cast<const f32x4 *>(&av[ml][16 * c + 4 * kg]) : kZero;
-#pragma unroll
-                    for (int v = 0; v < 4; v++) accV = mfma4(a[v], GLT[(16 * c + 4 * kg + v) * LD + wr + ml], accV);
-                }
-                accEA = accV;
-            }
-            put_rows<D>(kept + D * LD, dF, me);
-            put_rows<D>(Fb, accG, me);
-            {
-                float eE[CP], eA[CP];
-                lds_read<CP>(eE, &av[0][c0]);
-                lds_read<CP>(eA, &av[1][c0]);
-#pragma unroll
-                for (int i = 0; i < CP; i++) q[i] = e * eE[i] + a * eA[i];
-            }
-            lds_barrier();  // both halves' sums are there
-            float t[CP], h[CP];
-            lds_read<CP>(t, Fb + r * LD + c0);
-            lds_read<CP>(h, Bm + r * LD + c0);
-#pragma unroll
-            for (int i = 0; i < CP; i++) t[i] += h[i] + q[i];
-            vec_store<CP>(Fb + r * LD + c0, t);
             // sigma_L = <G_L, dG_L>; then (1-a_t) <G_t, dG_{t+1}> = sigma_{t+1} + th_t u.W_t and
             // sigma_t = that + dg.g + dp.p carry the inner product the gradient of alpha needs
+            float part[JT];
 #pragma unroll
-            for (int i = 0; i < CP; i++) G[i] = GLT[(c0 + i) * LD + r];
-            const float part = wave_allreduce(dotn<CP>(G, t));
-            if (lane == 0) sp[wave] = part;
+            for (int jt = 0; jt < JT; jt++) {
+                const float eE = av[0][16 * jt + ml], eA = av[1][16 * jt + ml];
+                const f32x4 G = *reinterpret_cast<const f32x4 *>(GLT + (16 * jt + ml) * LD + wr + 4 * kg);
+#pragma unroll
+                for (int v = 0; v < 4; v++) share[jt][v] += accG[jt][v] + (csr[0][v] * eE + csr[1][v] * eA);
+                part[jt] = (G[0] * share[jt][0] + G[1] * share[jt][1]) + (G[2] * share[jt][2] + G[3] * share[jt][3]);
+            }
+#pragma unroll
+            for (int jt = 1; jt < JT; jt++) part[0] += part[jt];
+            float *const dGL = raw + (buf ^ 1) * SET;   // the set of the tile before is idle here
+            put_rows<D>(dGL, share, me);
+            const float whole = wave_allreduce(part[0]);
+            if (lane == 0) sp[wave] = whole;
             lds_barrier();
+            accEA = kZero;   // rows 0 and 1 count
+            if (kg == 0) { accEA[0] = av1[0][wr + ml]; accEA[1] = av1[1][wr + ml]; }
 #pragma unroll
             for (int w = 0; w < NW; w++) sig += sp[w];
-            lds_read<CP>(dG, Fb + (wr + ml) * LD + CP * kg);
+            lds_read<CP>(dG, dGL + (wr + ml) * LD + CP * kg);
 #pragma unroll
-            for (int i = 0; i < CP; i++) dGT[i] = Fb[(CP * kg + i) * LD + wr + ml];
+            for (int i = 0; i < CP; i++) dGT[i] = dGL[(CP * kg + i) * LD + wr + ml];
         } else {
-            request(t0 + (ntile - 1) * kTB, L - (ntile - 1) * kTB);
 #pragma unroll
             for (int i = 0; i < CP; i++) {
                 const float *f = fz + (CP * kg + i) * D + wr + ml;
                 FTk[i] = f[0];
                 FTu[i] = f[DD];
             }
-            f32x4 sums[2][JT];
-            token_sums<D>(sums[0], outer + (chunk * 4 + 2) * DD, me);
-            token_sums<D>(sums[1], outer + (chunk * 4 + 3) * DD, me);
-            put_rows<D>(kept, sums[0], me);
-            put_rows<D>(kept + D * LD, sums[1], me);
         }
 #pragma unroll
         for (int i = 0; i < CP; i++) FTu[i] = FTk[i] - FTu[i];
         // arrived here: a wait for them inside the tile loop would be one for the next tile's requests as well
         asm volatile("" : "+v"(csE), "+v"(csA));
 
-        for (int tile = ntile - 1; tile >= 0; tile--) {
-            const int tb = t0 + tile * kTB, nt = min(kTB, t0 + L - tb);
+        for (int tile = ntile - 1; tile >= 0; tile--, buf ^= 1) {
+            const int nt = min(kTB, L - tile * kTB);
+            float *const set = raw + buf * SET, *const tg = set + 5 * TILE;
+            const float *const gam = gams[buf], (*const sc)[8] = scs[buf];
+            float *const Ws = raw + (buf ^ 1) * SET, *const Zs = Ws + TILE;   // until the next tile's inputs come
             int me = tid;   // and once per tile
             asm volatile("" : "+v"(me));
             const int tid = me, wave = tid >> 6, lane = tid & 63, ml = lane & 15, kg = lane >> 4, wr = 16 * wave,
@@ -803,20 +940,7 @@ __global__ __launch_bounds__(8 * D) void selfref_bwd_sweep_kernel(
                       tcol = CP * (ml >> 2) + (ml & 3),         // column of result row ml of block 0; block kt: + 4 kt
                       my_s = sigma(ml);                         // token of operand row ml
             lds_barrier();
-            *reinterpret_cast<float4 *>(&T_(A_K, stt, sj)) = pf_k;
-            *reinterpret_cast<float4 *>(&T_(A_U, stt, sj)) =
-                make_float4(pf_k.x - pf_v.x, pf_k.y - pf_v.y, pf_k.z - pf_v.z, pf_k.w - pf_v.w);
-            *reinterpret_cast<float4 *>(&T_(A_X, stt, sj)) = pf_x;
-            *reinterpret_cast<float4 *>(&tg[stt * LG + sj]) = pf_g;
-            *reinterpret_cast<float4 *>(&T_(A_DG0, stt, sj)) = pf_dg;
-            *reinterpret_cast<float4 *>(&T_(A_FX, stt, sj)) = pf_fx;
-            *reinterpret_cast<float4 *>(&T_(A_DG, stt, sj)) = make_float4(0, 0, 0, 0);
-            if (tid < 64) *reinterpret_cast<float4 *>(&gam[4 * tid]) = pf_gam;
-            if (tid < kTB) {
-                *reinterpret_cast<f32x4 *>(&sc[tid][0]) = f32x4{pf_s[0], pf_s[1], pf_s[2], pf_s[3]};
-                *reinterpret_cast<float2 *>(&sc[tid][4]) = make_float2(pf_s[4], pf_s[5]);
-            }
-            lds_barrier();
+            if (nt < kTB) *reinterpret_cast<float4 *>(DG + stt * LD + sj) = make_float4(0, 0, 0, 0);   // dg behind the last token
 
             // W = dG K, Z = dG^T U, Y = F_k^T Z + (F_k - F_v)^T W of the whole tile; T_s = u_s . W_s.  A sum per 16 terms,
             // added up in a tree: one running sum rounds at every term (d_x 1.1 to 1.2 times as far from float64)
@@ -844,14 +968,14 @@ __global__ __launch_bounds__(8 * D) void selfref_bwd_sweep_kernel(
             f32x4 W = tree(Wq), Z = tree(Zq);
 #pragma unroll
             for (int v = 0; v < 4; v++) {
-                T_(A_W, 4 * v + kg, wr + ml) = W[v];
-                T_(A_Z, 4 * v + kg, wr + ml) = Z[v];
+                Ws[(4 * v + kg) * LD + wr + ml] = W[v];
+                Zs[(4 * v + kg) * LD + wr + ml] = Z[v];
             }
             lds_barrier();
 #pragma unroll
             for (int i = 0; i < CP; i += 4) {
-                const f32x4 w4 = *reinterpret_cast<const f32x4 *>(&T_(A_W, my_s, CP * kg + i));
-                const f32x4 z4 = *reinterpret_cast<const f32x4 *>(&T_(A_Z, my_s, CP * kg + i));
+                const f32x4 w4 = *reinterpret_cast<const f32x4 *>(Ws + my_s * LD + CP * kg + i);
+                const f32x4 z4 = *reinterpret_cast<const f32x4 *>(Zs + my_s * LD + CP * kg + i);
 #pragma unroll
                 for (int v = 0; v < 4; v++) {
                     T = fmaf(U[i + v], w4[v], T);
@@ -862,7 +986,7 @@ __global__ __launch_bounds__(8 * D) void selfref_bwd_sweep_kernel(
             f32x4 Y = tree(Yq) + tree(Y2q);
             T = swapadd32(T, T);
             T = swapadd16(T, T);
-            if (tile > 0) request(tb - kTB, kTB);
+            if (tile == 0 && ci > 0) ahead(chunk - 1, me, true);
 
             // a_ts = dg_t . u_s for t = 4 j + kg, and prod_{s<r<t} (1-a_r); the same product over the whole tile above s;
             // prod_{r<t} (1-a_r) for t = 4 j + kg
@@ -882,9 +1006,9 @@ __global__ __launch_bounds__(8 * D) void selfref_bwd_sweep_kernel(
                 const float th = s0[1], keep = 1.f - s0[0], sig0 = s1.y;
                 const float dth = s1.x - uw, keepalp = fmaf(-th, dth, sig);
                 const float da = -keepalp * s0[2], de = dth * s0[3];
-                T_(A_DG, t, wr + ml) = fmaf(da, csA, fmaf(de, csE, fmaf(-th, ybc, dg0)));
+                DG_(t, wr + ml) = fmaf(da, csA, fmaf(de, csE, fmaf(-th, ybc, dg0)));
                 lds_barrier();
-                const float dgv = T_(A_DG, t, ve), gv = tg[t * LG + ve];
+                const float dgv = DG_(t, ve), gv = tg[t * LG + ve];
                 __builtin_amdgcn_sched_barrier(0);  // first in the queue: the step's chain starts with them
                 const f32x4 ps = *reinterpret_cast<const f32x4 *>(&Sx[wave][4 * kg]);
                 const float gml = gam[t * kTB + ml], fx = T_(A_FX, t, wr + ml);
@@ -951,7 +1075,7 @@ __global__ __launch_bounds__(8 * D) void selfref_bwd_sweep_kernel(
 #pragma unroll
             for (int j = 0; j < 4; j++) {
                 const int t = 4 * j + kg;
-                W = mfma4(ct[j] * gam[t * kTB + ml], T_(A_DG, t, wr + ml), W);
+                W = mfma4(ct[j] * gam[t * kTB + ml], DG_(t, wr + ml), W);
                 Z = mfma4(ct[j] * at[j], T_(A_X, t, wr + ml), Z);
             }
 #pragma unroll
@@ -977,11 +1101,11 @@ __global__ __launch_bounds__(8 * D) void selfref_bwd_sweep_kernel(
 #pragma unroll
                 for (int j = 0; j < 4; j++) {
                     const int t = 4 * j + kg;
-                    const float bg = below[j] * T_(A_DG, t, wr + ml), bx = below[j] * T_(A_X, t, wr + ml);
+                    const float bg = below[j] * DG_(t, wr + ml), bx = below[j] * T_(A_X, t, wr + ml);
 #pragma unroll
                     for (int kt = 0; kt < KT; kt++) {
                         n[kt] = mfma4(T_(A_X, t, tcol + 4 * kt), bg, n[kt]);
-                        nT[kt] = mfma4(T_(A_DG, t, tcol + 4 * kt), bx, nT[kt]);
+                        nT[kt] = mfma4(DG_(t, tcol + 4 * kt), bx, nT[kt]);
                     }
                 }
 #pragma unroll
@@ -991,13 +1115,6 @@ __global__ __launch_bounds__(8 * D) void selfref_bwd_sweep_kernel(
                 }
             }
         }
-    }
-#pragma unroll
-    for (int i = 0; i < JT; i++) {   // gradients of the initial memories, rows of every wave's own
-        const int row = wr + 16 * i / JT + lane / (4 * JT), at = lane % (4 * JT) * 4;
-        *reinterpret_cast<f32x4 *>(dmb + (size_t)2 * DD + row * D + at) = *reinterpret_cast<const f32x4 *>(kept + row * LD + at);
-        *reinterpret_cast<f32x4 *>(dmb + (size_t)5 * DD + row * D + at) =
-            *reinterpret_cast<const f32x4 *>(kept + (D + row) * LD + at);
     }
     __syncthreads();
     if (kg == 0) { av[0][wr + ml] = accEA[0]; av[1][wr + ml] = accEA[1]; }
@@ -1010,6 +1127,7 @@ __global__ __launch_bounds__(8 * D) void selfref_bwd_sweep_kernel(
         vec_store<CP>(dmb + 4 * DD + r * D + c0, eA);
     }
 #undef T_
+#undef DG_
 }
 
 template <int D>
@@ -1020,8 +1138,16 @@ void launch(const SelfrefSweep &a) {
     check_hip(hipFuncSetAttribute(reinterpret_cast<const void *>(selfref_bwd_prepare_kernel<D>),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds), "dynamic LDS size");
     hipLaunchKernelGGL((selfref_bwd_prepare_kernel<D>), dim3(a.batch * a.nc), dim3(4 * D), lds, stream(), a.emb, a.d_y, a.k,
-                       a.v, a.q, a.alpha, a.theta, a.amean, a.emean, a.frozen, a.gl, a.tok, a.outer, a.csv, a.s, a.C, a.nc);
+                       a.v, a.q, a.alpha, a.theta, a.amean, a.emean, a.frozen, a.gl, a.tok, a.outer, a.csv, a.d_mems, a.s, a.C, a.nc);
     check_launch("selfref_bwd_prepare_kernel");
+    if (a.nc > 1) {
+        hipLaunchKernelGGL((selfref_bwd_scan_kernel<D>), dim3(2 * (D / 16) * a.batch), dim3(64), 0, stream(), a.gl, a.outer, a.d_mems,
+                           a.nc, a.batch);
+        check_launch("selfref_bwd_scan_kernel");
+        hipLaunchKernelGGL((selfref_bwd_share_kernel<D>), dim3(a.batch * (a.nc - 1)), dim3(4 * D), 0, stream(), a.frozen, a.outer,
+                           a.nc);
+        check_launch("selfref_bwd_share_kernel");
+    }
     constexpr size_t sweep_lds = sweep_lds_floats(D) * sizeof(float);
     check_hip(hipFuncSetAttribute(reinterpret_cast<const void *>(selfref_bwd_sweep_kernel<D>),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)sweep_lds), "dynamic LDS size");

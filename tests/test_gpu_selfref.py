@@ -83,6 +83,20 @@ def test_forward_backward_match_oracle(B, s, d, C, sg):
         assert_close(n, got[n].reshape(ref[n].shape), ref[n])
 
 
+@pytest.mark.parametrize("B,s,d,C", [
+    # gradients across chunk boundaries: 2 to 5 chunks (the scan over chunks takes two a turn), a chunk's last tile with 1, 4, 5,
+    # 8, 9, 12, 13 or 16 tokens (what crosses the boundary is spread over its tokens where there are enough of them)
+    (1, 34, 64, 17), (2, 60, 64, 20), (1, 84, 64, 21), (1, 120, 64, 24), (2, 75, 64, 25), (1, 112, 64, 28), (1, 145, 64, 29),
+    (1, 160, 64, 32), (2, 99, 32, 33), (1, 80, 32, 20), (1, 105, 32, 21), (2, 46, 16, 23), (1, 85, 16, 17), (3, 5, 64, 2)])
+def test_gradients_across_chunk_boundaries(B, s, d, C):
+    mems, x, dy = inputs(B, s, d, seed=B * 1000 + s + d + C + 7)
+    print(f"selfref boundaries B={B} s={s} d={d} C={C}", flush=True)
+    got = gpu_run(mems, x, dy, C, True)
+    ref = oracle_run(mems, x, dy, C, True, np.float64)
+    for n in ("d_emb", "d_mems"):
+        assert_close(n, got[n].reshape(ref[n].shape), ref[n])
+
+
 def test_chunk_size_one_equals_sequential_semantics():
     """chunkwise_self_ref.rs:661-716: at C=1 the result does not depend on the snapshots
     being stale, so C=1 and the oracle's per-token rule agree (covered above); here the
