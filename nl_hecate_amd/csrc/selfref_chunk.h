@@ -58,9 +58,29 @@ struct ChunkLds {
     }
 };
 
-// Stages the chunk [t0, t0 + L) and builds its tables; ends with a barrier.  Without THETA the table holds
-// prod_{s<r<t} (1-a_r) alone.
-template <int D, bool SG, bool THETA = true>
+// A chunk's tables from its keys and gates, one wave.  Without THETA the table holds prod_{s<r<t} (1-a_r) alone.
+template <int D, bool THETA>
+__device__ __forceinline__ void chunk_tables(const ChunkLds<D> &m, int L, int lane) {
+    // Lane s builds column s of c downwards, c_{t,s} = th_s prod_{s<r<t} (1-a_r), so that a row's writes fall on 64
+    // banks; the retentions come from the lanes that hold them, and A_t is their running product.
+    const bool on = lane < L;
+    const float th = on ? m.cth[lane] : 0.f, keep = on ? 1.f - m.cal[lane] : 1.f, head = THETA ? th : 1.f;
+    float P = 1.f, A = 1.f, mine = 1.f;
+#pragma unroll
+    for (int t = 0; t < kLrC; t++) {  // retention 1 behind the last token: P and A stay as they are
+        const float k = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, keep), t));
+        const bool behind = lane < t;
+        m.CT[t * kLrC + lane] = behind ? head * P : 0.f;
+        P *= behind ? k : 1.f;
+        mine = lane == t ? A : mine;
+        A *= k;
+    }
+    m.cL[lane] = on ? th * P : 0.f;
+    if (on) m.cA[lane] = mine;
+    if (lane == 0) m.cA[L] = A;
+}
+// Stages the chunk [t0, t0 + L) and builds its tables; ends with a barrier.
+template <int D, bool SG>
 __device__ __forceinline__ void chunk_setup(const ChunkLds<D> &m, const float *__restrict__ k_cache,
                                             const float *__restrict__ v_cache, const float *__restrict__ alpha_cache,
                                             const float *__restrict__ theta_cache, size_t tok0, int t0, int L, int tid) {
@@ -78,25 +98,7 @@ __device__ __forceinline__ void chunk_setup(const ChunkLds<D> &m, const float *_
     for (int e = L * KL + tid; e < kLrC * KL; e += NT) { m.KC[e] = 0.f; m.XC[e] = 0.f; }
     for (int e = tid; e < L; e += NT) { m.cal[e] = alpha_cache[tok0 + t0 + e]; m.cth[e] = theta_cache[tok0 + t0 + e]; }
     __syncthreads();
-    if (tid < 64) {
-        // Lane s builds column s of c downwards, c_{t,s} = th_s prod_{s<r<t} (1-a_r), so that a row's writes fall on 64
-        // banks; the retentions come from the lanes that hold them, and A_t is their running product.
-        const bool on = tid < L;
-        const float th = on ? m.cth[tid] : 0.f, keep = on ? 1.f - m.cal[tid] : 1.f, head = THETA ? th : 1.f;
-        float P = 1.f, A = 1.f, mine = 1.f;
-#pragma unroll
-        for (int t = 0; t < kLrC; t++) {  // retention 1 behind the last token: P and A stay as they are
-            const float k = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, keep), t));
-            const bool behind = tid < t;
-            m.CT[t * kLrC + tid] = behind ? head * P : 0.f;
-            P *= behind ? k : 1.f;
-            mine = tid == t ? A : mine;
-            A *= k;
-        }
-        m.cL[tid] = on ? th * P : 0.f;
-        if (on) m.cA[tid] = mine;
-        if (tid == 0) m.cA[L] = A;
-    }
+    if (tid < 64) chunk_tables<D, true>(m, L, tid);
     __syncthreads();
 }
 

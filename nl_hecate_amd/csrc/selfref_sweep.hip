@@ -12,7 +12,7 @@
 //     dg_s = dg0_s - th_s Y_s + de_s csE + da_s csA
 // so that a token takes one exchange (dg_t), one product with a matrix and the dots of dg_t with the tile's u_s.
 //
-// 64 chains of 2048 tokens, head size 64, chunks of 64: preparation 0.36 ms (one workgroup per compute unit for its LDS;
+// 64 chains of 2048 tokens, head size 64, chunks of 64: preparation 0.29 ms (one workgroup per compute unit for its LDS;
 // 0.10 are matrix instructions), scan 0.06 and share 0.03, sweep 1.30 ms: 870 clocks a token (115 instructions of one wave per
 // SIMD and the exchange), 6.7 k clocks a tile and 15 k a chunk boundary, most of those matrix instructions.  The sweep that formed w, z, dk, dv and the
 // update of dG token by token took 3.16 ms behind 0.23 ms of preparation; without self-generated values it is still the one
@@ -46,343 +46,423 @@ constexpr f32x4 kZero = {0.f, 0.f, 0.f, 0.f};
 __device__ __forceinline__ float row_sum(float x) { return group_allreduce<16>(x); }
 
 // ── what does not depend on the sweep ────────────────────────────────────────────────────────────────────────────
-// LDS: the chunk's k and u, the table of retentions, the masked scores of q with the earlier k and of dp with the
-// earlier u (negative), dp, and 16 rows of every wave's own for changes of layout.  The first five make room for
-// q, then for dk0, dv0, dq, g, p as the operands of the outer products.
+// LDS: the chunk's k and u, the table of retentions, the masked scores of x and of q with the earlier k and of dp with the
+// earlier u (negative), dp, and what the two waves of a tile add up; then q in the place of k, and dk0, dv0, dq, g, p as
+// operands in front of the sums.
 template <int D>
 struct PrepareLds {
-    static constexpr int KL = D + 4, NW = D / 16;
-    static constexpr int wq = 0, wd = wq + kLrC * kWL, dp = wd + kLrC * kWL, rows = dp + kLrC * KL,
-                         floats = rows + NW * kTB * kWL;
+    static constexpr int KL = D + 4;
+    static constexpr int wx = 0, wq = wx + kLrC * kWL, wd = wq + kLrC * kWL, dp = wd + kLrC * kWL, sums = dp + kLrC * KL,
+                         floats = sums + 4 * kLrC;
 };
+constexpr int kPrepThr = 512;
+// N neighbouring columns, one for each of a wave's column tiles
+template <int N>
+__device__ __forceinline__ void load_columns(float (&x)[N], const float *p) {
+    if constexpr (N == 2) {
+        const float2 t = *reinterpret_cast<const float2 *>(p);
+        x[0] = t.x; x[1] = t.y;
+    } else {
+        x[0] = p[0];
+    }
+}
+template <int N>
+__device__ __forceinline__ void store_columns(float *p, const float (&x)[N]) {
+    if constexpr (N == 2) *reinterpret_cast<float2 *>(p) = make_float2(x[0], x[1]);
+    else p[0] = x[0];
+}
 
+// A workgroup per chunk, eight waves: two for each tile of 16 tokens, which share its scores by tiles of earlier tokens and its
+// results by columns, and for each 16 rows of a D x D result, by columns.  Waves w and w + 4 share a SIMD and take tiles w and
+// 3 - w, whose numbers of earlier tokens add up to the same.  One workgroup fills a compute unit's LDS, so its own latencies are
+// what bounds it: 82 k clocks a chunk, 31 k of them matrix instructions, 19 k until the chunk is in LDS, 19 k where the
+// low-rank products wait and F_k, F_v, F_q are on their way.  2048 chunks at head size 64: 293 us; four waves, one for each tile, whose
+// column sums of F_eta and F_alpha were 64 loads one after the other, took 363.
 template <int D>
-__global__ __launch_bounds__(4 * D) void selfref_bwd_prepare_kernel(
+__global__ __launch_bounds__(kPrepThr) void selfref_bwd_prepare_kernel(
     const float *__restrict__ emb, const float *__restrict__ d_y, const float *__restrict__ k_cache,
     const float *__restrict__ v_cache, const float *__restrict__ q_cache, const float *__restrict__ alpha_cache,
     const float *__restrict__ theta_cache, const float *__restrict__ amean_cache,
     const float *__restrict__ emean_cache, const float *__restrict__ frozen, float *__restrict__ gl,
     float *__restrict__ tok, float *__restrict__ outer, float *__restrict__ csv, float *__restrict__ d_mems, int s, int C, int nc) {
-    constexpr int KT = D / 16, NW = D / 16, NT = 4 * D, DD = D * D, KL = D + 4, V4 = D / 4, TPW = 4 / NW;
+    constexpr int KT = D / 16, DD = D * D, KL = D + 4, V4 = D / 4;
+    constexpr int JH = KT > 1 ? KT / 2 : 1, CG = KT / JH;   // a wave's column tiles; groups of columns
     constexpr int TF = sweep_token_floats(D);
     using P = PrepareLds<D>;
     extern __shared__ __align__(16) float lds[];
     const ChunkLds<D> m(lds);
-    float *Wq = m.tiles + P::wq, *Wd = m.tiles + P::wd, *DP = m.tiles + P::dp;
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, ml = lane & 15, kg = lane >> 4, wr = 16 * wave;
-    float *row = m.tiles + P::rows + wave * kTB * kWL;
+    float *Wx = m.tiles + P::wx, *Wq = m.tiles + P::wq, *Wd = m.tiles + P::wd, *DP = m.tiles + P::dp, *sums = m.tiles + P::sums;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, ml = lane & 15, kg = lane >> 4;
     const int ci = blockIdx.x % nc;
     const size_t b = blockIdx.x / nc, chunk = blockIdx.x, tok0 = b * (size_t)s;
     const int t0 = ci * C, L = min(C, s - t0), ntile = (L + kTB - 1) / kTB;
     const float *fz = frozen + chunk * 6 * DD;
+    const int half = wave >> 2, tile = half ? 7 - wave : wave, li0 = tile * kTB, nt = min(kTB, L - li0);
+    const bool live = tile < ntile, columns = live && half < CG;   // tokens there; columns as well
+    // Column ml of this wave's column tile j is column JH ml + j of its share: one load serves both tiles.
+    const int cw = 16 * JH * (half < CG ? half : 0) + JH * ml;
+    const size_t tk = tok0 + t0 + li0;
+    float *out = tok + tk * TF;
 
-    for (int e = tid; e < 2 * D; e += NT) {  // column sums of F_eta, F_alpha
-        const float *src = fz + (size_t)(3 + e / D) * DD + (e % D);
-        float a = 0.f;
+    // Requested in the order in which they are waited for.  First the chunk's k and v: row e / V4, columns 4 (e % V4) ..
+    constexpr int LOADS = kLrC * V4 / kPrepThr > 0 ? kLrC * V4 / kPrepThr : 1;
+    f32x4 k4[LOADS], v4[LOADS];
 #pragma unroll
-        for (int c = 0; c < D; c++) a += src[c * D];
-        csv[chunk * 2 * D + e] = a;
+    for (int i = 0; i < LOADS; i++) {
+        const int e = tid + i * kPrepThr;
+        const size_t o = (tok0 + t0 + min(e / V4, L - 1)) * D + (e % V4) * 4;
+        k4[i] = *reinterpret_cast<const f32x4 *>(k_cache + o);
+        v4[i] = *reinterpret_cast<const f32x4 *>(v_cache + o);
     }
-    for (int e = tid; e < L; e += NT) {  // the sweep's scalars of a token
-        const size_t i = tok0 + t0 + e;
-        const float al = alpha_cache[i], keep = 1.f - al, sa = sr_sigmoid(amean_cache[i]);
-        float *o = tok + i * TF + 3 * D + 16;
-        o[0] = al;
-        o[1] = theta_cache[i];
-        // sigmoid' of the mean over d keep (the sweep forms keep <G_t, dG_{t+1}>): a saturated gate has no gradient
-        o[2] = keep > 0.f ? sa * (1.f - sa) * (1.f / D) / keep : 0.f;
-        o[3] = sr_sigmoid(emean_cache[i]) * (1.f / D);  // softplus' of the mean over d
+    float al = 0.f, th = 0.f;
+    float amean = 0.f, emean = 0.f;
+    if (tid < L) {
+        const size_t i = tok0 + t0 + tid;
+        al = alpha_cache[i]; th = theta_cache[i]; amean = amean_cache[i]; emean = emean_cache[i];
     }
-    f32x4 in[3][TPW][KT];  // x, q, dy of the wave's tokens, requested ahead of the tables
-#pragma unroll
-    for (int i = 0; i < TPW; i++) {
-        const int li = (wave + i * NW) * kTB + ml;
-        const size_t o = (tok0 + t0 + min(li, L - 1)) * D + 4 * kg;
+    f32x4 in[3][KT];   // x, q, dy of the tile's tokens as operands
+    float xr[2][4][JH];   // x, q as results: token 4 kg + v, column cw + j
+    float fm[4 * KT][JH];   // F_mem, this wave's columns
+    if (live) {
+        const size_t o = (tk + min(ml, nt - 1)) * D + 4 * kg;
 #pragma unroll
         for (int kt = 0; kt < KT; kt++) {
-            in[0][i][kt] = li < L ? *reinterpret_cast<const f32x4 *>(emb + o + 16 * kt) : kZero;
-            in[1][i][kt] = li < L ? *reinterpret_cast<const f32x4 *>(q_cache + o + 16 * kt) : kZero;
-            in[2][i][kt] = li < L ? *reinterpret_cast<const f32x4 *>(d_y + o + 16 * kt) : kZero;
+            in[0][kt] = *reinterpret_cast<const f32x4 *>(emb + o + 16 * kt);
+            in[1][kt] = *reinterpret_cast<const f32x4 *>(q_cache + o + 16 * kt);
+            in[2][kt] = *reinterpret_cast<const f32x4 *>(d_y + o + 16 * kt);
         }
-    }
-    // scores that no token of the chunk has, and rows behind its last token, enter products times zero
-    for (int e = tid; e < 2 * kLrC * kWL + kLrC * KL; e += NT) Wq[e] = 0.f;
-    chunk_setup<D, true, false>(m, k_cache, v_cache, alpha_cache, theta_cache, tok0, t0, L, tid);
-    for (int e = L + tid; e < kLrC; e += NT) m.cth[e] = 0.f;
-    __syncthreads();
-
-    // a wave's rows: 16 tokens as operand rows (token ml, dims 16 kt + 4 kg + v) or as results (token 4 kg + v, dim
-    // 16 jt + ml)
-    auto put = [&](const f32x4(&x)[KT]) {
-        __builtin_amdgcn_wave_barrier();
 #pragma unroll
-        for (int jt = 0; jt < KT; jt++) {
-#pragma unroll
-            for (int v = 0; v < 4; v++) row[(4 * kg + v) * kWL + 16 * jt + ml] = x[jt][v];
-        }
-        __builtin_amdgcn_wave_barrier();
-    };
-    auto as_operand = [&](f32x4(&a)[KT]) {
-#pragma unroll
-        for (int kt = 0; kt < KT; kt++) a[kt] = *reinterpret_cast<const f32x4 *>(row + ml * kWL + 16 * kt + 4 * kg);
-    };
-
-    f32x4 g[TPW][KT], p[TPW][KT], dq[TPW][KT];
-#pragma unroll
-    for (int i = 0; i < TPW; i++) {
-        const int tile = wave + i * NW, li0 = tile * kTB, nt = min(kTB, L - li0), tile_i = i;
-#pragma unroll
-        for (int jt = 0; jt < KT; jt++) g[i][jt] = p[i][jt] = dq[i][jt] = kZero;
-        if (tile >= ntile) continue;
-        const size_t tk = tok0 + t0 + li0;
-        // out = A x - sum_s th_s c_ts (x_t . L_s) R_s; the scores without th go to sc (negative with NEG)
-        auto low_rank = [&](const f32x4(&a)[KT], const float *Lr, const float *R, float *sc, float sign, float *gam,
-                            f32x4(&out)[KT]) {
-            for (int st = 0; st <= tile; st++) {
-                f32x4 acc = kZero;
-#pragma unroll
-                for (int kt = 0; kt < KT; kt++) {
-                    const f32x4 l = *reinterpret_cast<const f32x4 *>(Lr + (16 * st + ml) * KL + 16 * kt + 4 * kg);
-#pragma unroll
-                    for (int v = 0; v < 4; v++) acc = mfma4(a[kt][v], l[v], acc);
-                }
-#pragma unroll
-                for (int v = 0; v < 4; v++) {
-                    const int tt = 4 * kg + v, li = li0 + tt, s1 = 16 * st + ml;
-                    const bool on = tt < nt && s1 < li;
-                    sc[tt * kWL + s1] = on ? sign * m.CT[li * kLrC + s1] * acc[v] : 0.f;
-                    // x_t . k_s of the tile's own tokens, in the order sigma
-                    if (gam && st == tile && tt < nt) gam[(size_t)tt * TF + sigma(ml)] = on ? acc[v] : 0.f;
-                }
-            }
-            __builtin_amdgcn_wave_barrier();
-            f32x4 acc[KT];
-#pragma unroll
-            for (int jt = 0; jt < KT; jt++) acc[jt] = kZero;
-            for (int st = 0; st <= tile; st++) {
-                const f32x4 w = *reinterpret_cast<const f32x4 *>(sc + ml * kWL + 16 * st + 4 * kg);
-                const f32x4 th = *reinterpret_cast<const f32x4 *>(m.cth + 16 * st + 4 * kg);
-#pragma unroll
-                for (int v = 0; v < 4; v++) {
-#pragma unroll
-                    for (int jt = 0; jt < KT; jt++)
-                        acc[jt] = mfma4(sign * w[v] * th[v], R[(16 * st + 4 * kg + v) * KL + 16 * jt + ml], acc[jt]);
-                }
-            }
-#pragma unroll
-            for (int jt = 0; jt < KT; jt++) {
-#pragma unroll
-                for (int v = 0; v < 4; v++) {
-                    const int tt = 4 * kg + v;
-                    out[jt][v] = tt < nt ? fmaf(m.cA[li0 + tt], out[jt][v], -acc[jt][v]) : 0.f;
-                }
-            }
-            __builtin_amdgcn_wave_barrier();
-        };
-        auto as_result = [&](const f32x4(&a)[KT], f32x4(&x)[KT]) {
-            __builtin_amdgcn_wave_barrier();
-#pragma unroll
-            for (int kt = 0; kt < KT; kt++) *reinterpret_cast<f32x4 *>(row + ml * kWL + 16 * kt + 4 * kg) = a[kt];
-            __builtin_amdgcn_wave_barrier();
-#pragma unroll
-            for (int jt = 0; jt < KT; jt++) {
-#pragma unroll
-                for (int v = 0; v < 4; v++) x[jt][v] = row[(4 * kg + v) * kWL + 16 * jt + ml];
-            }
-            __builtin_amdgcn_wave_barrier();
-        };
-        f32x4 a[KT];
-        float *out = tok + tk * TF;
-        as_result(in[0][i], g[i]);  // g = G x
-        low_rank(in[0][i], m.KC, m.XC, row, 1.f, out + 3 * D, g[i]);
-        as_result(in[1][i], p[i]);  // p = G q
-        low_rank(in[1][i], m.KC, m.XC, Wq + li0 * kWL, 1.f, nullptr, p[i]);
-        f32x4 dp[KT];  // dp = F_mem^T dy, dq = G^T dp
-        {
-            float f[2][4 * KT];  // the next 16 columns are requested before the products of the current ones
-            auto request = [&](int jt, int w) __attribute__((always_inline)) {
-#pragma unroll
-                for (int i = 0; i < 4 * KT; i++)
-                    f[w][i] = fz[5 * DD + (16 * (i >> 2) + 4 * kg + (i & 3)) * D + 16 * jt + ml];
-            };
-            request(0, 0);
-#pragma unroll
-            for (int jt = 0; jt < KT; jt++) {
-                dp[jt] = kZero;
-                if (jt + 1 < KT) request(jt + 1, (jt + 1) & 1);
-                __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for (int i = 0; i < 4 * KT; i++) dp[jt] = mfma4(in[2][tile_i][i >> 2][i & 3], f[jt & 1][i], dp[jt]);
-            }
-        }
-        float pp[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int jt = 0; jt < KT; jt++) {
-#pragma unroll
-            for (int v = 0; v < 4; v++) {
-                DP[(li0 + 4 * kg + v) * KL + 16 * jt + ml] = dp[jt][v];
-                pp[v] = fmaf(dp[jt][v], p[i][jt][v], pp[v]);
-            }
-        }
+        for (int i = 0; i < 4 * KT; i++) load_columns(fm[i], fz + 5 * DD + (16 * (i >> 2) + 4 * kg + (i & 3)) * D + cw);
 #pragma unroll
         for (int v = 0; v < 4; v++) {
-            pp[v] = row_sum(pp[v]);
-            if (ml == 0 && 4 * kg + v < nt) out[(size_t)(4 * kg + v) * TF + 3 * D + 21] = pp[v];
-        }
-        put(dp);
-        as_operand(a);
-#pragma unroll
-        for (int jt = 0; jt < KT; jt++) dq[i][jt] = dp[jt];
-        low_rank(a, m.XC, m.KC, Wd + li0 * kWL, -1.f, nullptr, dq[i]);
-#pragma unroll
-        for (int jt = 0; jt < KT; jt++) {
-#pragma unroll
-            for (int v = 0; v < 4; v++)
-                if (4 * kg + v < nt) out[(size_t)(4 * kg + v) * TF + 16 * jt + ml] = g[i][jt][v];
+            const size_t e = (tk + min(4 * kg + v, nt - 1)) * D + cw;
+            load_columns(xr[0][v], emb + e);
+            load_columns(xr[1][v], q_cache + e);
         }
     }
-    if (ci < nc - 1) {  // G_L = A_L I - sum_s c_Ls u_s k_s^T; wave w takes rows 16 w ..
-        f32x4 acc[KT];
+    // column sums of F_eta, F_alpha: a column's share of the rows per thread
+    constexpr int PARTS = kPrepThr / (2 * D), ROWS = D / PARTS;
+    float cs[ROWS];
+    {
+        const int e = tid % (2 * D);
+        const float *src = fz + (size_t)(3 + e / D) * DD + tid / (2 * D) * ROWS * D + e % D;
 #pragma unroll
-        for (int jt = 0; jt < KT; jt++) acc[jt] = kZero;
-        const int kend = (L + 3) & ~3;
-        for (int k0 = 0; k0 < kend; k0 += 4) {
-            const float au = m.XC[(k0 + kg) * KL + wr + ml] * m.cL[k0 + kg];
+        for (int c = 0; c < ROWS; c++) cs[c] = src[c * D];
+    }
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int jt = 0; jt < KT; jt++) acc[jt] = mfma4(au, m.KC[(k0 + kg) * KL + 16 * jt + ml], acc[jt]);
+    for (int i = 0; i < LOADS; i++) {   // rows behind a short chunk's last token enter products times zero
+        const int e = tid + i * kPrepThr, li = e / V4, j = (e % V4) * 4;
+        if (li < kLrC) {
+            *reinterpret_cast<f32x4 *>(m.KC + li * KL + j) = li < L ? k4[i] : kZero;
+            *reinterpret_cast<f32x4 *>(m.XC + li * KL + j) = li < L ? k4[i] - v4[i] : kZero;
+        }
+    }
+    if (tid < kLrC) { m.cal[tid] = al; m.cth[tid] = th; }
+    if (tid < 4 * kLrC) sums[tid] = 0.f;
+    lds_barrier();   // of LDS only: the other requests stay under way
+
+    // rows that no token has are zeros in every operand
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+#pragma unroll
+        for (int kt = 0; kt < KT; kt++) in[i][kt] = live && ml < nt ? in[i][kt] : kZero;
+    }
+    // products of 16 rows with those of the tile's earlier tokens, a tile's two waves in turn; c: which of the wave's
+    auto score = [&](const f32x4(&a)[KT], const float *Lr, f32x4(&acc)[2]) {
+#pragma unroll
+        for (int c = 0; c < 2; c++) {
+            acc[c] = kZero;
+            const int st = 2 * c + half;
+            if (st > tile) continue;
+#pragma unroll
+            for (int kt = 0; kt < KT; kt++) {
+                const f32x4 l = *reinterpret_cast<const f32x4 *>(Lr + (16 * st + ml) * KL + 16 * kt + 4 * kg);
+#pragma unroll
+                for (int v = 0; v < 4; v++) acc[c] = mfma4(a[kt][v], l[v], acc[c]);
+            }
+        }
+    };
+    // masked, with the retentions in between, to W (negative with sign -1); x_t . k_s of the tile's own tokens to gam as well, in
+    // the order sigma
+    auto put_scores = [&](const f32x4(&acc)[2], float *W, float sign, float *gam) {
+#pragma unroll
+        for (int c = 0; c < 2; c++) {
+            const int st = 2 * c + half;
+            if (st > tile) continue;
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int tt = 4 * kg + v, li = li0 + tt, s1 = 16 * st + ml;
+                const bool on = tt < nt && s1 < li;
+                W[li * kWL + s1] = on ? sign * m.CT[li * kLrC + s1] * acc[c][v] : 0.f;
+                if (gam && st == tile && tt < nt) gam[(size_t)tt * TF + sigma(ml)] = on ? acc[c][v] : 0.f;
+            }
+        }
+    };
+    // sum over this wave's columns of a product of two results, to the half's 64 sums
+    auto add_up = [&](float (&x)[4], float *to) {
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            x[v] = row_sum(x[v]);
+            if (ml == 0) to[half * kLrC + li0 + 4 * kg + v] = x[v];
+        }
+    };
+
+    f32x4 sx[2], sq[2];
+    float dp[4][JH];
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+#pragma unroll
+        for (int j = 0; j < JH; j++) dp[v][j] = 0.f;
+    }
+    if (live) {
+        score(in[0], m.KC, sx);
+        score(in[1], m.KC, sq);
+    }
+    if (columns) {   // dp = F_mem^T dy
+#pragma unroll
+        for (int j = 0; j < JH; j++) {
+            f32x4 acc = kZero;
+#pragma unroll
+            for (int i = 0; i < 4 * KT; i++) acc = mfma4(in[2][i >> 2][i & 3], fm[i][j], acc);
+#pragma unroll
+            for (int v = 0; v < 4; v++) dp[v][j] = acc[v];
+        }
+#pragma unroll
+        for (int v = 0; v < 4; v++) store_columns(DP + (li0 + 4 * kg + v) * KL + cw, dp[v]);
+    }
+#pragma unroll
+    for (int n = ROWS / 2; n > 0; n /= 2) {
+#pragma unroll
+        for (int c = 0; c < n; c++) cs[c] += cs[c + n];
+    }
+    m.Wt[tid] = cs[0];
+    if (wave == 7) chunk_tables<D, false>(m, L, lane);   // the wave with the fewest scores
+    lds_barrier();
+    f32x4 sd[2];
+    if (live) {
+        put_scores(sx, Wx, 1.f, out + 3 * D);
+        put_scores(sq, Wq, 1.f, nullptr);
+        f32x4 a[KT];
+#pragma unroll
+        for (int kt = 0; kt < KT; kt++) a[kt] = *reinterpret_cast<const f32x4 *>(DP + (li0 + ml) * KL + 16 * kt + 4 * kg);
+        score(a, m.XC, sd);
+        put_scores(sd, Wd, -1.f, nullptr);
+    }
+    if (tid < 2 * D) {
+        float a = 0.f;
+#pragma unroll
+        for (int i = 0; i < PARTS; i++) a += m.Wt[i * 2 * D + tid];
+        csv[chunk * 2 * D + tid] = a;
+    }
+    lds_barrier();
+    // g = G x, p = G q, dq = G^T dp
+    if (columns) {   // A x - sum_s th_s c_ts (scores) R_s for this wave's columns, the three side by side
+        f32x4 acc[3][JH];
+#pragma unroll
+        for (int j = 0; j < JH; j++) acc[0][j] = acc[1][j] = acc[2][j] = kZero;
+        for (int st = 0; st <= tile; st++) {
+            const int at = (li0 + ml) * kWL + 16 * st + 4 * kg;
+            const f32x4 wx = *reinterpret_cast<const f32x4 *>(Wx + at), wq = *reinterpret_cast<const f32x4 *>(Wq + at),
+                        wd = *reinterpret_cast<const f32x4 *>(Wd + at), th = *reinterpret_cast<const f32x4 *>(m.cth + 16 * st + 4 * kg);
+            float u[4][JH], kk[4][JH];
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                load_columns(u[v], m.XC + (16 * st + 4 * kg + v) * KL + cw);
+                load_columns(kk[v], m.KC + (16 * st + 4 * kg + v) * KL + cw);
+            }
+            __builtin_amdgcn_sched_barrier(0);   // all reads ahead of the products
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+#pragma unroll
+                for (int j = 0; j < JH; j++) {
+                    acc[0][j] = mfma4(wx[v] * th[v], u[v][j], acc[0][j]);
+                    acc[1][j] = mfma4(wq[v] * th[v], u[v][j], acc[1][j]);
+                    acc[2][j] = mfma4(-wd[v] * th[v], kk[v][j], acc[2][j]);
+                }
+            }
+        }
+        float pp[4];
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            const int tt = 4 * kg + v;
+            const float A = m.cA[li0 + tt];
+            pp[v] = 0.f;
+#pragma unroll
+            for (int j = 0; j < JH; j++) {
+                xr[0][v][j] = tt < nt ? fmaf(A, xr[0][v][j], -acc[0][j][v]) : 0.f;
+                xr[1][v][j] = tt < nt ? fmaf(A, xr[1][v][j], -acc[1][j][v]) : 0.f;
+                pp[v] = fmaf(dp[v][j], xr[1][v][j], pp[v]);
+                dp[v][j] = tt < nt ? fmaf(A, dp[v][j], -acc[2][j][v]) : 0.f;   // dq from here on
+            }
+            if (tt < nt) store_columns(out + (size_t)tt * TF + cw, xr[0][v]);
+        }
+        add_up(pp, sums);
+    }
+    const int rb = wave % KT, wr = 16 * rb, c0 = JH * (wave / KT < CG ? wave / KT : 0);   // D x D results: rows, column tiles
+    const bool rows = wave < KT * CG;
+    if (ci < nc - 1 && rows) {  // G_L = A_L I - sum_s c_Ls u_s k_s^T
+        f32x4 acc[JH];
+#pragma unroll
+        for (int j = 0; j < JH; j++) acc[j] = kZero;
+        for (int k0 = 0; k0 < L; k0 += 16) {   // rows behind the last token are zeros
+            float au[4], bk[4][JH];
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int k = k0 + 4 * i + kg;
+                au[i] = m.XC[k * KL + wr + ml] * m.cL[k];
+#pragma unroll
+                for (int j = 0; j < JH; j++) bk[i][j] = m.KC[k * KL + 16 * (c0 + j) + ml];
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+#pragma unroll
+                for (int j = 0; j < JH; j++) acc[j] = mfma4(au[i], bk[i][j], acc[j]);
+            }
         }
         const float aL = m.cA[L];
 #pragma unroll
-        for (int jt = 0; jt < KT; jt++) {
+        for (int j = 0; j < JH; j++) {
 #pragma unroll
             for (int v = 0; v < 4; v++) {
-                const int r = wr + 4 * kg + v, c = 16 * jt + ml;
-                gl[chunk * DD + r * D + c] = (r == c ? aL : 0.f) - acc[jt][v];
+                const int r = wr + 4 * kg + v, c = 16 * (c0 + j) + ml;
+                gl[chunk * DD + r * D + c] = (r == c ? aL : 0.f) - acc[j][v];
             }
         }
     }
-    __syncthreads();
-    float *Q = m.KC;
-    for (int e = tid; e < L * V4; e += NT) {
-        const int li = e / V4, j = (e % V4) * 4;
-        *reinterpret_cast<float4 *>(Q + li * KL + j) =
-            *reinterpret_cast<const float4 *>(q_cache + (tok0 + t0 + li) * D + j);
+    f32x4 q4[LOADS];   // q in the layout of the first loads
+#pragma unroll
+    for (int i = 0; i < LOADS; i++) {
+        const int e = tid + i * kPrepThr;
+        q4[i] = *reinterpret_cast<const f32x4 *>(q_cache + (tok0 + t0 + min(e / V4, L - 1)) * D + (e % V4) * 4);
     }
-    __syncthreads();
-    f32x4 dk[TPW][KT], dv[TPW][KT];
+    // F_k, F_v, F_q, this wave's columns, ahead of their products
+    float f[3][4 * KT][JH];
+    if (columns) {
 #pragma unroll
-    for (int i = 0; i < TPW; i++) {
-        const int tile = wave + i * NW, li0 = tile * kTB, nt = min(kTB, L - li0), tile_i = i;
+        for (int c = 0; c < 3; c++) {
 #pragma unroll
-        for (int jt = 0; jt < KT; jt++) dk[i][jt] = dv[i][jt] = kZero;
-        if (tile >= ntile) continue;
-        const size_t tk = tok0 + t0 + li0;
-        float *out = tok + tk * TF;
+            for (int i = 0; i < 4 * KT; i++) load_columns(f[c][i], fz + c * DD + (16 * (i >> 2) + 4 * kg + (i & 3)) * D + cw);
+        }
+    }
+    lds_barrier();
+    float *Q = m.KC;
+#pragma unroll
+    for (int i = 0; i < LOADS; i++) {
+        const int e = tid + i * kPrepThr, li = e / V4, j = (e % V4) * 4;
+        if (li < L) *reinterpret_cast<f32x4 *>(Q + li * KL + j) = q4[i];
+    }
+    lds_barrier();
+    f32x4 dk[JH], dv[JH];
+#pragma unroll
+    for (int j = 0; j < JH; j++) dk[j] = dv[j] = kZero;
+    if (columns) {
         // W_s = sum_t c_ts (q_t . k_s) dp_t, -Z_s = -sum_t c_ts (dp_t . u_s) q_t over the later tokens
         for (int st = tile; st < ntile; st++) {
 #pragma unroll
             for (int v = 0; v < 4; v++) {
                 const int t = 16 * st + 4 * kg + v;
                 const float wq = Wq[t * kWL + li0 + ml], wd = Wd[t * kWL + li0 + ml];
+                float p[JH], q[JH];
+                load_columns(p, DP + t * KL + cw);
+                load_columns(q, Q + t * KL + cw);
 #pragma unroll
-                for (int jt = 0; jt < KT; jt++) {
-                    dv[i][jt] = mfma4(wq, DP[t * KL + 16 * jt + ml], dv[i][jt]);
-                    dk[i][jt] = mfma4(wd, Q[t * KL + 16 * jt + ml], dk[i][jt]);
+                for (int j = 0; j < JH; j++) {
+                    dv[j] = mfma4(wq, p[j], dv[j]);
+                    dk[j] = mfma4(wd, q[j], dk[j]);
                 }
             }
         }
         float uw[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int jt = 0; jt < KT; jt++) {
+        for (int v = 0; v < 4; v++) {
+            const int li = li0 + 4 * kg + v;
+            const float th = m.cth[li];
+            float u[JH];
+            load_columns(u, m.XC + li * KL + cw);
 #pragma unroll
-            for (int v = 0; v < 4; v++) {
-                const int li = li0 + 4 * kg + v;
-                uw[v] = fmaf(m.XC[li * KL + 16 * jt + ml], dv[i][jt][v], uw[v]);
-                const float th = m.cth[li];
-                dk[i][jt][v] = th * (dk[i][jt][v] - dv[i][jt][v]);
-                dv[i][jt][v] *= th;
+            for (int j = 0; j < JH; j++) {
+                uw[v] = fmaf(u[j], dv[j][v], uw[v]);
+                dk[j][v] = th * (dk[j][v] - dv[j][v]);
+                dv[j][v] *= th;
             }
         }
+        add_up(uw, sums + 2 * kLrC);
+    }
+    lds_barrier();
+    if (tid < L) {   // the sweep's scalars of a token
+        float *o = tok + (tok0 + t0 + tid) * TF + 3 * D + 16;
+        const float keep = 1.f - al, sa = sr_sigmoid(amean);
+        o[0] = al;
+        o[1] = th;
+        // sigmoid' of the mean over d keep (the sweep forms keep <G_t, dG_{t+1}>): a saturated gate has no gradient
+        o[2] = keep > 0.f ? sa * (1.f - sa) * (1.f / D) / keep : 0.f;
+        o[3] = sr_sigmoid(emean) * (1.f / D);  // softplus' of the mean over d
+        o[4] = -(sums[2 * kLrC + tid] + sums[3 * kLrC + tid]);
+        o[5] = sums[tid] + sums[kLrC + tid];
+    }
+    float *Es = lds;  // dk, dv, dq, g, p: rows of stride KL, in front of the sums
+    if (columns) {
 #pragma unroll
         for (int v = 0; v < 4; v++) {
-            uw[v] = row_sum(uw[v]);
-            if (ml == 0 && 4 * kg + v < nt) out[(size_t)(4 * kg + v) * TF + 3 * D + 20] = -uw[v];
-        }
-        // dg0 = F_k^T dk + F_v^T dv + F_q^T dq, and F_k^T x
-        f32x4 dg[KT], fx[KT], ak[KT], av[KT], aq[KT];
-        put(dk[i]);
-        as_operand(ak);
-        put(dv[i]);
-        as_operand(av);
-        put(dq[i]);
-        as_operand(aq);
-        float f[2][3][4 * KT];  // the next 16 columns of F_k, F_v, F_q ahead of the products of the current ones
-        auto request = [&](int jt, int w) __attribute__((always_inline)) {
+            float *e = Es + (li0 + 4 * kg + v) * KL + cw, k1[JH], v1[JH];
 #pragma unroll
-            for (int c = 0; c < 3; c++) {
-#pragma unroll
-                for (int i = 0; i < 4 * KT; i++)
-                    f[w][c][i] = fz[c * DD + (16 * (i >> 2) + 4 * kg + (i & 3)) * D + 16 * jt + ml];
-            }
-        };
-        request(0, 0);
-#pragma unroll
-        for (int jt = 0; jt < KT; jt++) {
-            f32x4 dgk[2] = {kZero, kZero}, dgv[2] = {kZero, kZero}, dgq[2] = {kZero, kZero}, fxk[2] = {kZero, kZero};
-            if (jt + 1 < KT) request(jt + 1, (jt + 1) & 1);
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int i = 0; i < 4 * KT; i++) {
-                const int h = i >= 2 * KT;
-                dgk[h] = mfma4(ak[i >> 2][i & 3], f[jt & 1][0][i], dgk[h]);
-                fxk[h] = mfma4(in[0][tile_i][i >> 2][i & 3], f[jt & 1][0][i], fxk[h]);
-                dgv[h] = mfma4(av[i >> 2][i & 3], f[jt & 1][1][i], dgv[h]);
-                dgq[h] = mfma4(aq[i >> 2][i & 3], f[jt & 1][2][i], dgq[h]);
-            }
-            dg[jt] = ((dgk[0] + dgk[1]) + (dgv[0] + dgv[1])) + (dgq[0] + dgq[1]);
-            fx[jt] = fxk[0] + fxk[1];
-#pragma unroll
-            for (int v = 0; v < 4; v++) {
-                if (4 * kg + v < nt) {
-                    float *o = out + (size_t)(4 * kg + v) * TF + 16 * jt + ml;
-                    o[D] = dg[jt][v];
-                    o[2 * D] = fx[jt][v];
-                }
-            }
+            for (int j = 0; j < JH; j++) { k1[j] = dk[j][v]; v1[j] = dv[j][v]; }
+            store_columns(e, k1);
+            store_columns(e + kLrC * KL, v1);
+            store_columns(e + 2 * kLrC * KL, dp[v]);
+            store_columns(e + 3 * kLrC * KL, xr[0][v]);
+            store_columns(e + 4 * kLrC * KL, xr[1][v]);
         }
     }
-    // outer products: dF_k, dF_v, dF_q with g, dF_mem with p; the first two stored as the sweep's lanes hold them, the others
-    // as matrices
     float dy[kLrC / 4];
 #pragma unroll
     for (int i = 0; i < kLrC / 4; i++) {
         const int li = 16 * (i >> 2) + 4 * kg + (i & 3);
         dy[i] = li < L ? d_y[(tok0 + t0 + li) * D + wr + ml] : 0.f;
     }
-    __syncthreads();
-    float *Es = lds;  // dk, dv, dq, g, p: rows of stride KL, in front of the waves' own rows
+    lds_barrier();
+    if (columns) {   // dg0 = F_k^T dk + F_v^T dv + F_q^T dq, and F_k^T x
+        f32x4 a[3][KT];
 #pragma unroll
-    for (int i = 0; i < TPW; i++) {
-        const int li0 = (wave + i * NW) * kTB;
+        for (int c = 0; c < 3; c++) {
 #pragma unroll
-        for (int jt = 0; jt < KT; jt++) {
+            for (int kt = 0; kt < KT; kt++) a[c][kt] = *reinterpret_cast<const f32x4 *>(Es + (c * kLrC + li0 + ml) * KL + 16 * kt + 4 * kg);
+        }
+        float dg[4][JH], fx[4][JH];
 #pragma unroll
-            for (int v = 0; v < 4; v++) {
-                float *e = Es + (li0 + 4 * kg + v) * KL + 16 * jt + ml;
-                e[0] = dk[i][jt][v];
-                e[kLrC * KL] = dv[i][jt][v];
-                e[2 * kLrC * KL] = dq[i][jt][v];
-                e[3 * kLrC * KL] = g[i][jt][v];
-                e[4 * kLrC * KL] = p[i][jt][v];
+        for (int j = 0; j < JH; j++) {
+            f32x4 dgk[2] = {kZero, kZero}, dgv[2] = {kZero, kZero}, dgq[2] = {kZero, kZero}, fxk[2] = {kZero, kZero};
+#pragma unroll
+            for (int i = 0; i < 4 * KT; i++) {
+                const int h = i >= 2 * KT;
+                dgk[h] = mfma4(a[0][i >> 2][i & 3], f[0][i][j], dgk[h]);
+                fxk[h] = mfma4(in[0][i >> 2][i & 3], f[0][i][j], fxk[h]);
+                dgv[h] = mfma4(a[1][i >> 2][i & 3], f[1][i][j], dgv[h]);
+                dgq[h] = mfma4(a[2][i >> 2][i & 3], f[2][i][j], dgq[h]);
+            }
+            const f32x4 dg4 = ((dgk[0] + dgk[1]) + (dgv[0] + dgv[1])) + (dgq[0] + dgq[1]), fx4 = fxk[0] + fxk[1];
+#pragma unroll
+            for (int v = 0; v < 4; v++) { dg[v][j] = dg4[v]; fx[v][j] = fx4[v]; }
+        }
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            if (4 * kg + v < nt) {
+                float *o = out + (size_t)(4 * kg + v) * TF + cw;
+                store_columns(o + D, dg[v]);
+                store_columns(o + 2 * D, fx[v]);
             }
         }
     }
-    __syncthreads();
-    f32x4 o[4][KT];
+    if (!rows) return;
+    // outer products: dF_k, dF_v, dF_q with g, dF_mem with p; the first two stored as the sweep's lanes hold them, the others
+    // as matrices
+    f32x4 o[4][JH];
 #pragma unroll
     for (int c = 0; c < 4; c++) {
 #pragma unroll
-        for (int jt = 0; jt < KT; jt++) o[c][jt] = kZero;
+        for (int j = 0; j < JH; j++) o[c][j] = kZero;
     }
 #pragma unroll
     for (int st = 0; st < kLrC / 16; st++) {
@@ -394,25 +474,26 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_prepare_kernel(
             const float ak = e[wr + ml], av = e[kLrC * KL + wr + ml], aq = e[2 * kLrC * KL + wr + ml];
             const float ay = dy[4 * st + v];
 #pragma unroll
-            for (int jt = 0; jt < KT; jt++) {
-                const float bg = e[3 * kLrC * KL + 16 * jt + ml], bp = e[4 * kLrC * KL + 16 * jt + ml];
-                o[0][jt] = mfma4(ak, bg, o[0][jt]);
-                o[1][jt] = mfma4(av, bg, o[1][jt]);
-                o[2][jt] = mfma4(bg, aq, o[2][jt]);
-                o[3][jt] = mfma4(bp, ay, o[3][jt]);
+            for (int j = 0; j < JH; j++) {
+                const float bg = e[3 * kLrC * KL + 16 * (c0 + j) + ml], bp = e[4 * kLrC * KL + 16 * (c0 + j) + ml];
+                o[0][j] = mfma4(ak, bg, o[0][j]);
+                o[1][j] = mfma4(av, bg, o[1][j]);
+                o[2][j] = mfma4(bg, aq, o[2][j]);
+                o[3][j] = mfma4(bp, ay, o[3][j]);
             }
         }
     }
 #pragma unroll
-    for (int jt = 0; jt < KT; jt++) {
+    for (int j = 0; j < JH; j++) {
+        const int jt = c0 + j;
 #pragma unroll
         for (int c = 0; c < 2; c++)
-            *reinterpret_cast<f32x4 *>(outer + (chunk * 4 + c) * DD + ((size_t)(wave * KT + jt) * 64 + lane) * 4) = o[c][jt];
+            *reinterpret_cast<f32x4 *>(outer + (chunk * 4 + c) * DD + ((size_t)(rb * KT + jt) * 64 + lane) * 4) = o[c][j];
 #pragma unroll
         for (int c = 2; c < 4; c++) {
             const int at = (wr + ml) * D + 16 * jt + 4 * kg;
-            if (nc > 1) *reinterpret_cast<f32x4 *>(outer + (chunk * 4 + c) * DD + at) = o[c][jt];
-            else *reinterpret_cast<f32x4 *>(d_mems + (b * 6 + (c == 2 ? 2 : 5)) * DD + at) = o[c][jt];   // no chunk passes them on
+            if (nc > 1) *reinterpret_cast<f32x4 *>(outer + (chunk * 4 + c) * DD + at) = o[c][j];
+            else *reinterpret_cast<f32x4 *>(d_mems + (b * 6 + (c == 2 ? 2 : 5)) * DD + at) = o[c][j];   // no chunk passes them on
         }
     }
 }
@@ -1133,11 +1214,11 @@ __global__ __launch_bounds__(8 * D) void selfref_bwd_sweep_kernel(
 template <int D>
 void launch(const SelfrefSweep &a) {
     constexpr size_t lds = (chunk_lds_floats<D>(0) + PrepareLds<D>::floats) * sizeof(float);
-    static_assert(5 * kLrC * (D + 4) <= chunk_lds_floats<D>(0) + PrepareLds<D>::rows, "operands of the outer products");
+    static_assert(5 * kLrC * (D + 4) <= chunk_lds_floats<D>(0) + PrepareLds<D>::sums, "operands of the outer products");
     static_assert(lds <= 160 * 1024, "LDS");
     check_hip(hipFuncSetAttribute(reinterpret_cast<const void *>(selfref_bwd_prepare_kernel<D>),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds), "dynamic LDS size");
-    hipLaunchKernelGGL((selfref_bwd_prepare_kernel<D>), dim3(a.batch * a.nc), dim3(4 * D), lds, stream(), a.emb, a.d_y, a.k,
+    hipLaunchKernelGGL((selfref_bwd_prepare_kernel<D>), dim3(a.batch * a.nc), dim3(kPrepThr), lds, stream(), a.emb, a.d_y, a.k,
                        a.v, a.q, a.alpha, a.theta, a.amean, a.emean, a.frozen, a.gl, a.tok, a.outer, a.csv, a.d_mems, a.s, a.C, a.nc);
     check_launch("selfref_bwd_prepare_kernel");
     if (a.nc > 1) {
