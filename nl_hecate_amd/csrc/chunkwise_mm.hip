@@ -81,7 +81,7 @@ __global__ __launch_bounds__(kThr) void cw_local_fwd_kernel(const TIn *__restric
         fetch(tv, v + tok * HD, L);
         const Gates gt = fetch_gates(alpha + tok, theta + tok, eta + tok, L, has_s != 0);
         load_gates(cf, gt);
-        coefficients(cf, gt, L, nullptr, nullptr, nullptr);
+        coefficients(cf, gt, L, nullptr);
         commit(Ks, tk);
         commit(Vs, tv);
     }
@@ -252,7 +252,7 @@ __global__ __launch_bounds__(kThr) void cw_out_fwd_kernel(const TIn *__restrict_
     const int chain = task / nc, ci = task % nc, t0 = ci * C, L = min(C, s - t0);
     const size_t tok = (size_t)chain * s + t0;
     load_gates(cf, gt);
-    coefficients(cf, gt, L, Cc, nullptr, nullptr);
+    coefficients(cf, gt, L, Cc);
     commit(Ks, tk);
     commit(Qs, tq);
     commit(Es, tv);
@@ -349,7 +349,7 @@ __global__ __launch_bounds__(kThr) void cw_local_bwd_kernel(const TIn *__restric
     for (int task = task_lo; task < task_hi; task++) {
     const int chain = task / nc, ci = task % nc, t0 = ci * C, L = min(C, s - t0);
     load_gates(cf, gt);
-    coefficients(cf, gt, L, Cc, nullptr, nullptr);
+    coefficients(cf, gt, L, Cc);
     commit(Ks, tk);
     commit(Qs, tq);
     commit(Ds, td);
@@ -451,7 +451,7 @@ __global__ __launch_bounds__(kThr) void cw_grads_bwd_kernel(
     const size_t st1 = ((size_t)chain * (nc + 1) + ci + 1) * HD * HD;
     fetch_task(task);
     load_gates(cf, gt);
-    coefficients(cf, gt, L, Cc, nullptr, nullptr);
+    coefficients(cf, gt, L, Cc);
     commit(Ks, tk);
     commit(Qs, tq);
     commit(Es, tv);

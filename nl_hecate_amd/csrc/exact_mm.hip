@@ -207,7 +207,7 @@ __global__ __launch_bounds__(kThr) void ex_local_kernel(
     (void)t0;
     {
         load_gates(cf, gt);
-        coefficients<real<P64>>(cf, gt, L, Cc, nullptr, nullptr);
+        coefficients<real<P64>>(cf, gt, L, Cc);
         commit(Ks, tk, tid);
         commit(Vs, tv, tid);
         commit(Qs, tq, tid);
@@ -499,7 +499,7 @@ __global__ __launch_bounds__(kThr) void ex_grads_kernel(
     const size_t tok = (size_t)chain * s + t0, task = (size_t)itask;
     fetch_b(itask, tid);
     load_gates(cf, gt);
-    coefficients<real<P64>>(cf, gt, L, Cc, nullptr, nullptr);
+    coefficients<real<P64>>(cf, gt, L, Cc);
     commit(Ks, tk, tid);
     commit(Qs, tq, tid);
     commit(Ds, td, tid);
@@ -737,7 +737,7 @@ __global__ __launch_bounds__(kThr) void ex_fwd_local_kernel(
         fetch(tv, v + tok * D, L, tid);
         const Gates gt = fetch_gates(alpha + tok, theta + tok, eta + tok, L, has_s != 0);
         load_gates(cf, gt);
-        coefficients<double>(cf, gt, L, Cc, nullptr, nullptr);
+        coefficients<double>(cf, gt, L, Cc);
         commit(Ks, tk, tid);
         commit(Vs, tv, tid);
     }

@@ -102,6 +102,30 @@ def test_backward_matches_oracle(B, s, C, bf16):
         assert_close(n, host(g[n]), want[n], tol)
 
 
+@pytest.mark.parametrize("C", [15, 16, 17, 32, 33, 47, 49, 63])
+def test_coefficients_at_the_edges_of_their_blocks(C):
+    """The coefficients come from four waves, 16 tokens each, that meet in composed maps: chunks that end one token before, at and
+    behind a block's end, the last chunk of five tokens, retentions and etas of zero at the blocks' edges."""
+    B, d = 2, 64
+    s = 2 * C + 5
+    x = make(B, s, d, seed=900 + C, bf16=False)
+    for t in {t for t in (0, 15, 16, 31, C - 1) if t < C}:
+        x["alpha"][:, t] = 1.0 if t % 2 else 0.0
+        x["eta"][:, C + t] = 0.0
+    print(f"chunkwise_mm coefficients C={C}", flush=True)
+    want, want_g = oracle_chunkwise(x, C)
+    f = gpu_forward(x, C, False)
+    assert_close("y", host(f["y"]), want["y"], 1e-4)
+    g = dict(d_k=zeros(B, s, d), d_v=zeros(B, s, d), d_q=zeros(B, s, d), d_alpha=zeros(B, s),
+             d_theta=zeros(B, s), d_eta=zeros(B, s), d_m_initial=zeros(d, d), d_s_initial=zeros(d, d))
+    D.call("titans_chunkwise_backward_mm_f32_rocm", f["k"], f["v"], f["q"], f["al"], f["th"], f["et"], f["mc"], f["sc"],
+           dev(x["dy"]), g["d_k"], g["d_v"], g["d_q"], g["d_alpha"], g["d_theta"], g["d_eta"], g["d_m_initial"],
+           g["d_s_initial"], s, d, B, C)
+    torch.cuda.synchronize()
+    for n in g:
+        assert_close(n, host(g[n]), want_g[n], 1e-4)
+
+
 @pytest.mark.parametrize("bf16", [True, False])
 def test_saturated_gates(bf16):
     """alpha exactly 0 and 1 (retention 1 and 0: the memory is wiped), eta exactly 0 and 1, theta 0, at
