@@ -258,6 +258,7 @@ unsigned nlh_adamw_step(nlh_adamw *o, const int *active_levels, float lr, float 
     std::vector<float *> w, g, m, v;
     std::vector<int> n;
     std::vector<float> bc1, bc2;
+    std::vector<nlh::UpdateBounds> bounds;
     const bool clip = max_grad_norm > 0.0f;
     if (clip) {
         // the clip factor stays on the device; the update below applies it to the gradients it reads (and writes
@@ -291,15 +292,12 @@ unsigned nlh_adamw_step(nlh_adamw *o, const int *active_levels, float lr, float 
         w.push_back(t.w); g.push_back(t.g); m.push_back(t.m); v.push_back(t.v); n.push_back(t.n);
         bc1.push_back(t.group < 0 ? sbc1 : lbc1[t.group]);
         bc2.push_back(t.group < 0 ? sbc2 : lbc2[t.group]);
+        bounds.push_back({t.clamp, t.lo, t.hi});
     }
     unsigned rc = nlh::adamw_update_multi_scaled(w.data(), (const float *const *)g.data(), m.data(), v.data(),
                                                  n.data(), bc1.data(), bc2.data(), (int)w.size(), lr, o->beta1,
-                                                 o->beta2, o->eps, o->weight_decay, clip ? norm_scale + 1 : nullptr);
-    if (rc) return rc;
-    for (auto &t : o->tensors)
-        if (t.clamp && (t.group < 0 || (active_levels && active_levels[t.group])))
-            clamp_f32_cuda(t.w, t.n, t.lo, t.hi);
-    return 0;
+                                                 o->beta2, o->eps, o->weight_decay, clip ? norm_scale + 1 : nullptr, bounds.data());
+    return rc;
 }
 
 // ── level combine + MAG gate ────────────────────────────────────────────────

@@ -29,6 +29,12 @@ __device__ __forceinline__ void adamw_one(float &w, float g, float &m, float &v,
     const float m_hat = mi * bc1_inv, v_hat = vi * bc2_inv;
     w -= lr * (m_hat / (sqrtf(v_hat) + eps) + wd * w);
 }
+// Bounds of a tensor after its update, in the update itself: a launch of its own took 4.5 us for the one float of a b_theta.
+struct Bounds {
+    bool on;
+    float lo, hi;
+    __device__ __forceinline__ float operator()(float w) const { return on ? fmaxf(lo, fminf(hi, w)) : w; }
+};
 
 struct AdamwHyper { float lr, b1, b2, eps, wd; };
 
@@ -37,7 +43,7 @@ struct AdamwHyper { float lr, b1, b2, eps, wd; };
 template <bool SCALE>
 __device__ __forceinline__ void adamw_span(float *w, const float *g, float *m, float *v, int n,
                                            int start, int stride, const AdamwHyper &h, float bc1, float bc2,
-                                           const float *scale_ptr = nullptr) {
+                                           const Bounds &in, const float *scale_ptr = nullptr) {
     const bool vec = ((((uintptr_t)w) | ((uintptr_t)g) | ((uintptr_t)m) | ((uintptr_t)v)) & 15) == 0;
     float sc = 1.0f;
     if (SCALE) sc = *scale_ptr;
@@ -57,7 +63,7 @@ __device__ __forceinline__ void adamw_span(float *w, const float *g, float *m, f
             adamw_one(W.y, G.y, M.y, V.y, h.lr, h.b1, h.b2, h.eps, bc1, bc2, h.wd);
             adamw_one(W.z, G.z, M.z, V.z, h.lr, h.b1, h.b2, h.eps, bc1, bc2, h.wd);
             adamw_one(W.w, G.w, M.w, V.w, h.lr, h.b1, h.b2, h.eps, bc1, bc2, h.wd);
-            reinterpret_cast<float4 *>(w)[j] = W;
+            reinterpret_cast<float4 *>(w)[j] = make_float4(in(W.x), in(W.y), in(W.z), in(W.w));
             reinterpret_cast<float4 *>(m)[j] = M;
             reinterpret_cast<float4 *>(v)[j] = V;
         }
@@ -65,19 +71,22 @@ __device__ __forceinline__ void adamw_span(float *w, const float *g, float *m, f
             float gi = g[i];
             if (scaled) { gi *= sc; gw[i] = gi; }
             adamw_one(w[i], gi, m[i], v[i], h.lr, h.b1, h.b2, h.eps, bc1, bc2, h.wd);
+            w[i] = in(w[i]);
         }
     } else {
         for (int i = start; i < n; i += stride) {
             float gi = g[i];
             if (scaled) { gi *= sc; gw[i] = gi; }
             adamw_one(w[i], gi, m[i], v[i], h.lr, h.b1, h.b2, h.eps, bc1, bc2, h.wd);
+            w[i] = in(w[i]);
         }
     }
 }
 
 __global__ void adamw_kernel(float *w, const float *g, float *m, float *v, int n, AdamwHyper h,
                              float bc1, float bc2) {
-    adamw_span<false>(w, g, m, v, n, blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x, h, bc1, bc2);
+    adamw_span<false>(w, g, m, v, n, blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x, h, bc1, bc2,
+                      Bounds{false, 0.f, 0.f});
 }
 
 // Up to kMaxTensors tensors per launch, passed by value in the kernel argument.
@@ -89,6 +98,7 @@ struct AdamwBatch {
     float *v[kMaxTensors];
     int n[kMaxTensors];
     float bc1[kMaxTensors], bc2[kMaxTensors];
+    Bounds in[kMaxTensors];
     int blk_begin[kMaxTensors + 1];  // first workgroup of each tensor
     int count;
 };
@@ -100,7 +110,7 @@ __global__ void adamw_multi_kernel(AdamwBatch b, AdamwHyper h, const float *scal
     const int nblk = b.blk_begin[t + 1] - b.blk_begin[t];
     const int lb = blockIdx.x - b.blk_begin[t];
     adamw_span<SCALE>(b.w[t], b.g[t], b.m[t], b.v[t], b.n[t], lb * blockDim.x + threadIdx.x, nblk * blockDim.x, h,
-                      b.bc1[t], b.bc2[t], scale_ptr);
+                      b.bc1[t], b.bc2[t], b.in[t], scale_ptr);
 }
 
 // One partial per 256 elements (the reference's layout, core/kernels/adamw.cu:86-127):
@@ -287,7 +297,7 @@ unsigned adamw_update_multi_rocm(float *const *w, const float *const *g, float *
                                  const int *n, const float *bc1_inv, const float *bc2_inv, int count,
                                  float lr, float beta1, float beta2, float eps, float weight_decay) {
     return nlh::adamw_update_multi_scaled(w, g, m, v, n, bc1_inv, bc2_inv, count, lr, beta1, beta2, eps, weight_decay,
-                                          nullptr);
+                                          nullptr, nullptr);
 }
 
 }  // extern "C"
@@ -295,7 +305,7 @@ unsigned adamw_update_multi_rocm(float *const *w, const float *const *g, float *
 unsigned nlh::adamw_update_multi_scaled(float *const *w, const float *const *g, float *const *m, float *const *v,
                                         const int *n, const float *bc1_inv, const float *bc2_inv, int count, float lr,
                                         float beta1, float beta2, float eps, float weight_decay,
-                                        const float *scale_ptr) {
+                                        const float *scale_ptr, const UpdateBounds *bounds) {
     const AdamwHyper h{lr, beta1, beta2, eps, weight_decay};
     // a batch is the next kMaxTensors input slots (empty ones skipped), so no tensor is seen twice
     for (int first = 0; first < count; first += kMaxTensors) {
@@ -307,6 +317,7 @@ unsigned nlh::adamw_update_multi_scaled(float *const *w, const float *const *g, 
             const int c = b.count++;
             b.w[c] = w[i]; b.g[c] = g[i]; b.m[c] = m[i]; b.v[c] = v[i]; b.n[c] = n[i];
             b.bc1[c] = bc1_inv[i]; b.bc2[c] = bc2_inv[i];
+            b.in[c] = bounds ? Bounds{bounds[i].on, bounds[i].lo, bounds[i].hi} : Bounds{false, 0.f, 0.f};
             b.blk_begin[c] = blocks;
             int nb = (n[i] / 4 + kOptThreads - 1) / kOptThreads;
             blocks += nb < 1 ? 1 : (nb > 256 ? 256 : nb);
