@@ -1012,7 +1012,7 @@ void titans_levels_forward_bf16_rocm(const float *x, const float *w_extra, int n
  * gradients [n, d] of the plain projections' outputs, or n_extra null pointers when the caller has already
  * written them as bf16 into columns e * d .. of the operand that level_grad_operand_rocm returns; d_gate_params:
  * host array of 6 * levels device pointers (overwritten).  As on the reference's GPU path nothing flows from the gates into k and v.
- * d_m_initial, d_s_initial [head_dim^2] are accumulated (+=, summed over all chains). */
+ * d_m_initial, d_s_initial [head_dim^2] are accumulated (+=, summed over all chains); both null: not wanted. */
 void titans_levels_backward_bf16_rocm(const uint16_t *x_bf16, const float *w_extra, int n_extra, const float *const *d_extra,
                                       const float *w_levels, const uint16_t *k_heads, const uint16_t *v_heads,
                                       const uint16_t *q_heads, const float *alpha_heads, const float *theta_heads,

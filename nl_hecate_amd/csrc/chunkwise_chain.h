@@ -15,11 +15,15 @@ namespace nlh {
 // of squares of the chunk-start M and S (eight partials per chunk and matrix).  Null: not wanted.
 struct ChainTracks { float *e2, *nrm; };
 
+// Where the states behind the last token go besides (null: nowhere): [batch, d, d] each, m_initial and s_initial themselves
+// where a caller carries them on.
+struct ChainFinal { float *m, *s; };
+
 bool chunkwise_chain_forward_bf16(const char *fn, const uint16_t *k, const uint16_t *v, const uint16_t *q,
                                   const float *alpha, const float *theta, const float *eta, const float *m_initial,
                                   const float *s_initial, float *m_states, float *s_states, float *y, int seq_len,
                                   int d, int batch, int chunk_size, bool has_s, const HeadRows *y_rows = nullptr,
-                                  const ChainTracks *tracks = nullptr);
+                                  const ChainTracks *tracks = nullptr, const ChainFinal *final_states = nullptr);
 
 // The float-token matrix form (chunkwise_mm.hip) with the same side outputs; eta / s_initial / s_states null without
 // momentum.

@@ -111,9 +111,9 @@ __global__ __launch_bounds__(64) void cw_coef_kernel(const float *__restrict__ a
 template <bool HAS_S, bool TRACK>
 __global__ __launch_bounds__(kChainThr) void cw_chain_fwd_kernel(
     const u16 *__restrict__ k, const u16 *__restrict__ v, const u16 *__restrict__ q,
-    const float *__restrict__ table, const float *__restrict__ vecs, const float *__restrict__ m_initial,
-    const float *__restrict__ s_initial, float *__restrict__ m_states, float *__restrict__ s_states,
-    float *__restrict__ y, int s, int C, int nc, int batch, HeadRows yr, ChainTracks tr) {
+    const float *__restrict__ table, const float *__restrict__ vecs, const float *m_initial, const float *s_initial,
+    float *__restrict__ m_states, float *__restrict__ s_states,
+    float *__restrict__ y, int s, int C, int nc, int batch, HeadRows yr, ChainTracks tr, ChainFinal fin) {
     constexpr int HMAT = 32 * 64;   // a 32-row matrix
     extern __shared__ __align__(16) unsigned char smem_raw[];
     u16 *Kr = reinterpret_cast<u16 *>(smem_raw);   // K [t][c]
@@ -390,6 +390,14 @@ __global__ __launch_bounds__(kChainThr) void cw_chain_fwd_kernel(
         commit_vecs();
         __syncthreads();
     }
+    if (!grpX && fin.m) {   // may be the initial states: this thread has read its part of those
+#pragma unroll
+        for (int ct = 0; ct < 2; ct++) {
+            const size_t o = (size_t)chain * HD * HD + (i0 + 16 * ct + r16) * HD + 16 * bi + 4 * g;
+            *reinterpret_cast<f32x4 *>(fin.m + o) = Mm[ct];
+            if (HAS_S) *reinterpret_cast<f32x4 *>(fin.s + o) = Sm[ct];
+        }
+    }
 }
 
 constexpr size_t kChainFwdLds = (7 * kPerm + 10 * 32 * 64) * sizeof(u16) + (4 * CW + 4) * sizeof(float);
@@ -398,7 +406,7 @@ template <bool HAS_S>
 void launch_forward(const char *fn, const u16 *k, const u16 *v, const u16 *q, const float *alpha, const float *theta,
                     const float *eta, const float *m_initial, const float *s_initial, float *m_states,
                     float *s_states, float *y, int seq_len, int batch, int chunk_size, const HeadRows &yr,
-                    const ChainTracks *tracks) {
+                    const ChainTracks *tracks, const ChainFinal &fin) {
     const ErrorScope es;
     const int nc = ceil_div(seq_len, chunk_size), nchunks = batch * nc;
     float *table = scratch(3, (size_t)nchunks * kTableFloats * sizeof(float));
@@ -426,11 +434,11 @@ void launch_forward(const char *fn, const u16 *k, const u16 *v, const u16 *q, co
         if (tracks)
             hipLaunchKernelGGL((cw_chain_fwd_kernel<HAS_S, true>), dim3(2 * batch), dim3(kChainThr), kChainFwdLds, stream(), k,
                                v, q, table, vecs, m_initial, s_initial, m_states, s_states, y, seq_len, chunk_size, nc, batch,
-                               yr, *tracks);
+                               yr, *tracks, fin);
         else
             hipLaunchKernelGGL((cw_chain_fwd_kernel<HAS_S, false>), dim3(2 * batch), dim3(kChainThr), kChainFwdLds, stream(), k,
                                v, q, table, vecs, m_initial, s_initial, m_states, s_states, y, seq_len, chunk_size, nc, batch,
-                               yr, ChainTracks{nullptr, nullptr});
+                               yr, ChainTracks{nullptr, nullptr}, fin);
     }
     check_launch(fn);
 }
@@ -441,15 +449,16 @@ bool chunkwise_chain_forward_bf16(const char *fn, const uint16_t *k, const uint1
                                   const float *alpha, const float *theta, const float *eta, const float *m_initial,
                                   const float *s_initial, float *m_states, float *s_states, float *y, int seq_len,
                                   int d, int batch, int chunk_size, bool has_s, const HeadRows *y_rows,
-                                  const ChainTracks *tracks) {
+                                  const ChainTracks *tracks, const ChainFinal *final_states) {
     if (d != HD || chunk_size < 1 || chunk_size > CW || seq_len <= 0 || batch <= 0) return false;
     const HeadRows yr = y_rows ? *y_rows : head_major_rows(seq_len, HD);
+    const ChainFinal fin = final_states ? *final_states : ChainFinal{nullptr, nullptr};
     if (has_s)
         launch_forward<true>(fn, k, v, q, alpha, theta, eta, m_initial, s_initial, m_states, s_states, y, seq_len,
-                             batch, chunk_size, yr, tracks);
+                             batch, chunk_size, yr, tracks, fin);
     else
         launch_forward<false>(fn, k, v, q, alpha, theta, nullptr, m_initial, nullptr, m_states, nullptr, y, seq_len,
-                              batch, chunk_size, yr, tracks);
+                              batch, chunk_size, yr, tracks, fin);
     return true;
 }
 

@@ -787,8 +787,8 @@ bool backward_mm(const char *fn, const TIn *k, const TIn *v, const TIn *q, const
     const float *ds_first = packed ? reinterpret_cast<const float *>(reinterpret_cast<const uint16_t *>(ds_states) + n_snap)
                                    : ds_states;
     const int per = 8, rows = ceil_div(batch, per);
-    const int nsum = has_s && d_s_initial ? 2 : 1;
-    float *tmp = scratch(10, (size_t)nsum * rows * HD * HD * sizeof(float));
+    const int nsum = !d_m_initial ? 0 : has_s && d_s_initial ? 2 : 1;   // null: a caller has no use for them
+    float *tmp = nsum ? scratch(10, (size_t)nsum * rows * HD * HD * sizeof(float)) : nullptr;
     if (es.failed()) return true;
     // d_alpha, d_eta, and in the same launch the first stage of the deterministic sum of d_m_initial, d_s_initial
     chunkwise_gate_gradients(alpha, eta, pvec, xs, scal, d_alpha, d_eta, seq_len, batch, chunk_size, has_s, dm_first,
@@ -796,6 +796,7 @@ bool backward_mm(const char *fn, const TIn *k, const TIn *v, const TIn *q, const
     if (guard && couplings_may_fire_tracked(k, alpha, theta, eta, tracks, has_s, seq_len, batch, chunk_size, guard->error_clip,
                                             guard->m_norm_max))
         return false;
+    if (!nsum) return true;
     KernelTimer kt("cw_add_rows_kernel");
     hipLaunchKernelGGL(cw_add_rows_kernel, dim3(HD * HD / 256, 1, nsum), dim3(256), 0, stream(), tmp, d_m_initial,
                        d_s_initial, rows);

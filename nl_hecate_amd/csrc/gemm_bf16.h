@@ -16,5 +16,8 @@ struct ProductBf16 {
 // library.
 bool product_bf16_serves(const ProductBf16 &p, int op);
 void product_bf16(const ProductBf16 &p, int op);   // scratch slot 30 where the contraction is split
+// op 1 of a and op 2 of b, both served: side by side in one launch where neither's result meets what the other reads or writes
+// and the types are those of a projection's gradients, one after the other elsewhere.
+void product_bf16_pair(const ProductBf16 &a, const ProductBf16 &b);
 
 }  // namespace nlh

@@ -68,15 +68,19 @@ struct Operand {
 };
 
 template <int OP, class TA, class TBe>
-__global__ __launch_bounds__(kThr) void product_bf16_kernel(Args g) {
+constexpr int kBufElems = 2 * (Operand<OP != 2, TA>::ELEMS + Operand<OP == 0, TBe>::ELEMS);
+
+// Block tile `tile`, run `split` of the contraction; lds: kBufElems.
+template <int OP, class TA, class TBe>
+__device__ __forceinline__ void product(const Args &g, int tile, int split, u16 *lds) {
     using OA = Operand<OP != 2, TA>;
     using OB = Operand<OP == 0, TBe>;
-    __shared__ __align__(16) u16 sa[2][OA::ELEMS], sb[2][OB::ELEMS];
+    u16 *sa[2] = {lds, lds + OA::ELEMS}, *sb[2] = {lds + 2 * OA::ELEMS, lds + 2 * OA::ELEMS + OB::ELEMS};
     const ProductBf16 &p = g.p;
-    const int m0 = (int)blockIdx.x % g.tiles_m * TB, n0 = (int)blockIdx.x / g.tiles_m * TB;
+    const int m0 = tile % g.tiles_m * TB, n0 = tile / g.tiles_m * TB;
     const int l = threadIdx.x & 63, w = threadIdx.x >> 6, wm = (w >> 1) * 32, wn = (w & 1) * 32;
     const int total = (p.k + TB - 1) / TB, per = (total + g.splits - 1) / g.splits;
-    const int s0 = min(total, (int)blockIdx.y * per), s1 = min(total, s0 + per);
+    const int s0 = min(total, split * per), s1 = min(total, s0 + per);
     OA ra[2];
     OB rb[2];
     auto load = [&](int s, int set) __attribute__((always_inline)) {
@@ -111,7 +115,7 @@ __global__ __launch_bounds__(kThr) void product_bf16_kernel(Args g) {
         step(s, 0);
         if (s + 1 < s1) step(s + 1, 1);
     }
-    float *c = g.splits > 1 ? g.part + (size_t)blockIdx.y * p.m * p.n : p.c;
+    float *c = g.splits > 1 ? g.part + (size_t)split * p.m * p.n : p.c;
 #pragma unroll
     for (int i = 0; i < 2; i++)
 #pragma unroll
@@ -121,6 +125,22 @@ __global__ __launch_bounds__(kThr) void product_bf16_kernel(Args g) {
                 const int row = m0 + wm + 16 * i + 4 * (l >> 4) + e, col = n0 + wn + 16 * j + (l & 15);
                 if (row < p.m && col < p.n) c[(size_t)row * p.n + col] = acc[i][j][e];
             }
+}
+
+template <int OP, class TA, class TBe>
+__global__ __launch_bounds__(kThr) void product_bf16_kernel(Args g) {
+    __shared__ __align__(16) u16 lds[kBufElems<OP, TA, TBe>];
+    product<OP, TA, TBe>(g, blockIdx.x, blockIdx.y, lds);
+}
+// The gradients of a projection: dW (op 2, the longer ones, first) and dx (op 1) are no larger at a few hundred tokens than
+// the launch between them.  Layer step of 500 tokens, d = 256: 6 + 10 and 9 + 10 us one after the other, 11 and 12 together.
+template <class TG, class TW, class TX>
+__global__ __launch_bounds__(kThr) void product_bf16_pair_kernel(Args dw, Args dx, int dw_blocks, int dw_tiles, int dx_tiles) {
+    constexpr int A = kBufElems<2, TG, TX>, B = kBufElems<1, TG, TW>;
+    __shared__ __align__(16) u16 lds[A > B ? A : B];
+    const int i = blockIdx.x;
+    if (i < dw_blocks) product<2, TG, TX>(dw, i % dw_tiles, i / dw_tiles, lds);
+    else product<1, TG, TW>(dx, (i - dw_blocks) % dx_tiles, (i - dw_blocks) / dx_tiles, lds);
 }
 
 __global__ __launch_bounds__(256) void product_sum_kernel(const float *__restrict__ part, float *__restrict__ c, long long n4, int splits) {
@@ -166,27 +186,69 @@ bool product_bf16_serves(const ProductBf16 &p, int op) {
     return 2.0 * p.m * p.n * p.k <= kLargest[op];
 }
 
-void product_bf16(const ProductBf16 &p, int op) {
-    const ErrorScope es;
+namespace {
+Args product_args(const ProductBf16 &p) {
     Args g{};
     g.p = p;
     g.tiles_m = ceil_div(p.m, TB);
-    const int tiles = g.tiles_m * ceil_div(p.n, TB), steps = ceil_div(p.k, TB);
-    g.splits = std::max(1, std::min({4 * compute_units() / tiles, steps / 6, 16}));
+    g.splits = std::max(1, std::min({4 * compute_units() / (g.tiles_m * ceil_div(p.n, TB)), ceil_div(p.k, TB) / 6, 16}));
+    return g;
+}
+size_t part_floats(const Args &g) { return g.splits > 1 ? (size_t)g.splits * g.p.m * g.p.n : 0; }
+void sum_parts(const Args &g) {
+    if (g.splits == 1) return;
+    const long long n4 = (long long)g.p.m * g.p.n / 4;
+    hipLaunchKernelGGL(product_sum_kernel, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, stream(), g.part, g.p.c, n4, g.splits);
+    check_launch("product_sum_kernel");
+}
+}  // namespace
+
+void product_bf16(const ProductBf16 &p, int op) {
+    const ErrorScope es;
+    Args g = product_args(p);
     if (g.splits > 1) {
-        g.part = scratch(30, (size_t)g.splits * p.m * p.n * sizeof(float));
+        g.part = scratch(30, part_floats(g) * sizeof(float));
         if (es.failed()) return;
     }
-    const dim3 grid((unsigned)tiles, (unsigned)g.splits);
+    const dim3 grid((unsigned)(g.tiles_m * ceil_div(p.n, TB)), (unsigned)g.splits);
     if (op == 0) launch<0>(g, grid);
     else if (op == 1) launch<1>(g, grid);
     else launch<2>(g, grid);
     check_launch("product_bf16_kernel");
-    if (g.splits > 1) {
-        const long long n4 = (long long)p.m * p.n / 4;
-        hipLaunchKernelGGL(product_sum_kernel, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, stream(), g.part, p.c, n4, g.splits);
-        check_launch("product_sum_kernel");
+    sum_parts(g);
+}
+
+void product_bf16_pair(const ProductBf16 &a, const ProductBf16 &b) {
+    const ErrorScope es;
+    const auto result_meets = [](const ProductBf16 &p, const void *x, long long rows, long long cols, long long ld, int bytes) {
+        const uintptr_t x0 = (uintptr_t)x, x1 = x0 + ((rows - 1) * ld + cols) * bytes, c0 = (uintptr_t)p.c;
+        return x && x0 < c0 + (size_t)p.m * p.n * sizeof(float) && c0 < x1;
+    };
+    const int kb = a.b2 ? a.k_first : a.k, ab = a.b_bf16 ? 2 : 4, bb = b.b_bf16 ? 2 : 4;
+    const bool apart = !result_meets(b, a.a, a.m, a.k, a.lda, a.a_bf16 ? 2 : 4) && !result_meets(b, a.b, kb, a.n, a.ldb, ab) &&
+                       !result_meets(b, a.b2, a.k - kb, a.n, a.ldb, ab) && !result_meets(a, b.a, b.k, b.m, b.lda, b.a_bf16 ? 2 : 4) &&
+                       !result_meets(a, b.b, b.k, b.n, b.ldb, bb) && !result_meets(a, b.c, b.m, b.n, b.n, 4);
+    if (!apart || a.a_bf16 != b.a_bf16 || a.b_bf16 || !b.b_bf16) {
+        product_bf16(a, 1);
+        if (!es.failed()) product_bf16(b, 2);
+        return;
     }
+    Args dx = product_args(a), dw = product_args(b);
+    if (dx.splits > 1 || dw.splits > 1) {
+        float *part = scratch(30, (part_floats(dx) + part_floats(dw)) * sizeof(float));
+        if (es.failed()) return;
+        dx.part = part;
+        dw.part = part + part_floats(dx);
+    }
+    const int dx_tiles = dx.tiles_m * ceil_div(a.n, TB), dw_tiles = dw.tiles_m * ceil_div(b.n, TB), dw_blocks = dw_tiles * dw.splits;
+    const dim3 grid((unsigned)(dw_blocks + dx_tiles * dx.splits));
+    if (a.a_bf16)
+        hipLaunchKernelGGL((product_bf16_pair_kernel<u16, float, u16>), grid, dim3(kThr), 0, stream(), dw, dx, dw_blocks, dw_tiles, dx_tiles);
+    else
+        hipLaunchKernelGGL((product_bf16_pair_kernel<float, float, u16>), grid, dim3(kThr), 0, stream(), dw, dx, dw_blocks, dw_tiles, dx_tiles);
+    check_launch("product_bf16_pair_kernel");
+    sum_parts(dx);
+    sum_parts(dw);
 }
 
 }  // namespace nlh

@@ -22,6 +22,7 @@
 
 #include "../../include/nl_hecate_ffi.h"
 #include "bf16_tiles.h"
+#include "chunkwise_chain.h"
 #include "chunkwise_grads.h"
 #include "gemm_bf16.h"
 #include "lane_ops.h"
@@ -57,7 +58,7 @@ __device__ __forceinline__ bf16x4 f4_to_bf4(const float4 &x) {
 struct ProjArgs {
     const float *x;            // [n, D]
     u16 *x_bf16;               // [n, D]: x rounded to bf16 (the backward's GEMM operand); may be null
-    const u16 *wfrag;          // packed weights, projection p at p * D * D (wfrag_pack_kernel)
+    const u16 *wfrag;          // packed weights, projection p at p * D * D (wfrag_pack)
     const u16 *ufrag;          // folded gate vectors of every level, [levels][D / 32][64][8] (gate_fold_kernel)
     u16 *extra_out[kMaxExtra]; // plain projections, bf16 [n, D] each
     const float *bias[kMaxLevels][3];   // b_alpha, b_theta, b_eta
@@ -69,23 +70,24 @@ struct ProjArgs {
     float eps;
 };
 
-// Packs P matrices W_p [D, D] (row = output column, contraction index contiguous) into the order in which
+// Packs P matrices W_p [D, D] (row = output column, contraction index contiguous; the first n_extra in w_extra) into the order in which
 // the projection kernel's waves read them, as A operands of v_mfma_f32_32x32x16_bf16:
 // [p][column block of 64][k step of 16][tile of 32 columns][lane][8], lane l holding column 32 * tile + l % 32,
 // contraction indices 16 * step + 8 * (l / 32) .. + 8: one 16-byte load per lane and tile, 2 KB contiguous per
 // wave and step.
-__global__ void wfrag_pack_kernel(const float *__restrict__ W, u16 *__restrict__ out, int P, int D) {
+__device__ __forceinline__ void wfrag_pack(const float *__restrict__ w_extra, int n_extra, const float *__restrict__ w_levels,
+                                           u16 *__restrict__ out, int P, int D, int block, int blocks) {
     const long long total = (long long)P * D * D / 8;
     const int KS = D / 16, CB = D / 64;
-    for (long long o = (long long)blockIdx.x * blockDim.x + threadIdx.x; o < total; o += (long long)gridDim.x * blockDim.x) {
+    for (long long o = (long long)block * kSThr + threadIdx.x; o < total; o += (long long)blocks * kSThr) {
         const int lane = (int)(o & 63), c32 = (int)((o >> 6) & 1);
         long long r = o >> 7;
         const int ks = (int)(r % KS);
         r /= KS;
         const int cb = (int)(r % CB);
-        const long long p = r / CB;
+        const int p = (int)(r / CB);
         const int row = 64 * cb + 32 * c32 + (lane & 31), k0 = 16 * ks + 8 * (lane >> 5);
-        const float *src = W + (p * D + row) * D + k0;
+        const float *src = (p < n_extra ? w_extra + (size_t)p * D * D : w_levels + (size_t)(p - n_extra) * D * D) + (size_t)row * D + k0;
         const float4 a = *reinterpret_cast<const float4 *>(src), b = *reinterpret_cast<const float4 *>(src + 4);
         const bf16x8 v = {(__bf16)a.x, (__bf16)a.y, (__bf16)a.z, (__bf16)a.w, (__bf16)b.x, (__bf16)b.y, (__bf16)b.z, (__bf16)b.w};
         *reinterpret_cast<bf16x8 *>(out + o * 8) = v;
@@ -103,11 +105,9 @@ __global__ void wfrag_pack_kernel(const float *__restrict__ W, u16 *__restrict__
 struct FoldArgs { const float *w[kMaxLevels][3]; };
 constexpr int kFoldSlices = 16;   // the sum over the D columns is cut into slices that run as separate workgroups
 // part [levels][kFoldSlices][6][D]: slice sl's share of u_q[j]
-__global__ __launch_bounds__(64) void gate_fold_partial_kernel(const float *__restrict__ w_levels, FoldArgs g,
-                                                               float *__restrict__ part, int D) {
-    const int lvl = blockIdx.y, sl = blockIdx.z, j = blockIdx.x * 64 + threadIdx.x;
+__device__ __forceinline__ void gate_fold_partial(const float *__restrict__ w_levels, const FoldArgs &g, float *__restrict__ part,
+                                                  int D, int lvl, int sl, int j) {
     const int per = D / kFoldSlices, c0 = sl * per;
-    if (j >= D) return;
     const float *Wk = w_levels + (size_t)lvl * 3 * D * D, *Wv = Wk + (size_t)D * D;
     float u[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll 8
@@ -121,6 +121,19 @@ __global__ __launch_bounds__(64) void gate_fold_partial_kernel(const float *__re
     }
 #pragma unroll
     for (int q = 0; q < 6; q++) part[(((size_t)lvl * kFoldSlices + sl) * 6 + q) * D + j] = u[q];
+}
+// Both in one launch, the fold's waves behind the packing's blocks: what either takes is its launch (4.7 us each of the 231 of a
+// layer step over 500 tokens, when the plain projections, the levels' and the fold were three).
+__global__ __launch_bounds__(kSThr) void weights_prepare_kernel(const float *__restrict__ w_extra, int n_extra,
+                                                                const float *__restrict__ w_levels, int levels, u16 *__restrict__ out,
+                                                                int D, int pack_blocks, FoldArgs g, float *__restrict__ part) {
+    if ((int)blockIdx.x < pack_blocks) {
+        wfrag_pack(w_extra, n_extra, w_levels, out, n_extra + 3 * levels, D, blockIdx.x, pack_blocks);
+        return;
+    }
+    const int u = __builtin_amdgcn_readfirstlane((blockIdx.x - pack_blocks) * (kSThr / 64) + threadIdx.x / 64);   // 64 columns of a slice of a level
+    const int sl = u % kFoldSlices, lvl = u / kFoldSlices % levels, jb = u / kFoldSlices / levels;
+    if (64 * jb < D) gate_fold_partial(w_levels, g, part, D, lvl, sl, 64 * jb + (threadIdx.x & 63));
 }
 // a wave per quantity: its sixteen slices are loads without a chain between them (one wave for all six took 10 us)
 __global__ __launch_bounds__(6 * 64) void gate_fold_finish_kernel(const float *__restrict__ part, u16 *__restrict__ ufrag, int D) {
@@ -567,19 +580,6 @@ __global__ void f32_to_bf16_vec_kernel(const float *__restrict__ x, u16 *__restr
         *reinterpret_cast<bf16x4 *>(out + 4 * i) = f4_to_bf4(*reinterpret_cast<const float4 *>(x + 4 * i));
 }
 
-// last slot of every chain's chunk states -> the carried context memories (copy_final_m_batch, gpu_forward.rs:2824)
-__global__ void final_states_kernel(const float *__restrict__ mc, const float *__restrict__ sc, float *__restrict__ m_ctx,
-                                    float *__restrict__ s_ctx, long long chains, int slots, int dd4) {
-    const long long total = chains * dd4;
-    for (long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x; e < total; e += (long long)gridDim.x * blockDim.x) {
-        const long long c = e / dd4;
-        const int i = (int)(e % dd4);
-        const size_t src = ((size_t)c * slots + slots - 1) * dd4 + i;
-        reinterpret_cast<float4 *>(m_ctx)[e] = reinterpret_cast<const float4 *>(mc)[src];
-        reinterpret_cast<float4 *>(s_ctx)[e] = reinterpret_cast<const float4 *>(sc)[src];
-    }
-}
-
 // gate = sigmoid(scale * sum_l y_l); gated = attn * gate as bf16 (the output projection's operand)
 struct LevelYs { const float *y[kMaxLevels]; };
 __global__ void combine_gate_x1_kernel(LevelYs lv, int k, float scale, const u16 *__restrict__ attn, float *__restrict__ gate,
@@ -786,19 +786,14 @@ void level_project_forward_bf16_rocm(const float *x, const float *w_extra, int n
     a.k_norms = k_norms; a.q_norms = q_norms; a.alpha = alpha; a.theta = theta; a.eta = eta;
     a.n = n; a.bs = bs; a.s = seq_len; a.nh = heads; a.n_extra = n_extra; a.levels = levels; a.eps = eps;
     {
-        KernelTimer kt("wfrag_pack_kernel");
-        if (n_extra)
-            hipLaunchKernelGGL(wfrag_pack_kernel, dim3(stream_blocks((long long)n_extra * d * d / 8, 2048)), dim3(kSThr), 0,
-                               stream(), w_extra, wfrag, n_extra, d);
-        if (levels)
-            hipLaunchKernelGGL(wfrag_pack_kernel, dim3(stream_blocks(3LL * levels * d * d / 8, 2048)), dim3(kSThr), 0, stream(),
-                               w_levels, wfrag + (size_t)n_extra * d * d, 3 * levels, d);
-        check_launch("wfrag_pack_kernel");
+        KernelTimer kt("weights_prepare_kernel");
+        const int pack = stream_blocks((long long)P * d * d / 8, 2048), fold = levels * kFoldSlices * (d / 64) / (kSThr / 64);
+        hipLaunchKernelGGL(weights_prepare_kernel, dim3(pack + fold), dim3(kSThr), 0, stream(), w_extra, n_extra, w_levels, levels, wfrag,
+                           d, pack, fa, fold_part);
+        check_launch("weights_prepare_kernel");
     }
     if (levels) {
         KernelTimer kt("gate_fold_kernel");
-        hipLaunchKernelGGL(gate_fold_partial_kernel, dim3(ceil_div(d, 64), levels, kFoldSlices), dim3(64), 0, stream(), w_levels,
-                           fa, fold_part, d);
         hipLaunchKernelGGL(gate_fold_finish_kernel, dim3(ceil_div(d, 64), levels), dim3(6 * 64), 0, stream(), fold_part, ufrag, d);
         check_launch("gate_fold_kernel");
     }
@@ -820,16 +815,12 @@ void titans_levels_forward_bf16_rocm(const float *x, const float *w_extra, int n
                                     alpha_heads, theta_heads, eta_heads, k_norms, q_norms, alpha, theta, eta, bs, seq_len,
                                     heads, head_dim, levels, eps);
     if (es.failed() || levels == 0) return;
-    const int chains = levels * bs * heads, nc = (seq_len + chunk_size - 1) / chunk_size;
-    titans_chunkwise_forward_bf16_tokens_rocm(k_heads, v_heads, q_heads, alpha_heads, theta_heads, eta_heads, m_context,
-                                              s_context, m_chunk_states, s_chunk_states, y_tokens, seq_len, head_dim, chains,
-                                              chunk_size, heads, levels);
-    if (es.failed()) return;
-    KernelTimer kt("final_states_kernel");
-    const int dd4 = head_dim * head_dim / 4;
-    hipLaunchKernelGGL(final_states_kernel, dim3(stream_blocks((long long)chains * dd4, 2048)), dim3(kSThr), 0, stream(),
-                       m_chunk_states, s_chunk_states, m_context, s_context, (long long)chains, nc + 1, dd4);
-    check_launch("final_states_kernel");
+    const int chains = levels * bs * heads;
+    const HeadRows yr = token_major_rows(seq_len, head_dim, heads, bs * heads, true);
+    const ChainFinal carried{m_context, s_context};
+    chunkwise_chain_forward_bf16("titans_levels_forward_bf16_rocm", k_heads, v_heads, q_heads, alpha_heads, theta_heads,
+                                 eta_heads, m_context, s_context, m_chunk_states, s_chunk_states, y_tokens, seq_len, head_dim,
+                                 chains, chunk_size, true, &yr, nullptr, &carried);
 }
 
 uint16_t *level_grad_operand_rocm(int bs, int seq_len, int heads, int head_dim, int levels, int n_extra, long long *ld) {
@@ -921,7 +912,15 @@ void titans_levels_backward_bf16_rocm(const uint16_t *x_bf16, const float *w_ext
     // d_x [n, d] = G [n, R] Wb [R, d];  d_W [R, d] = G^T x  (row-major buffers as column-major operands)
     const ProductBf16 px{G, n_extra ? w_extra : w_levels, n_extra && levels ? w_levels : nullptr, d_x, R, d, (int)n, d, (int)R,
                          n_extra * d, true, false};
+    // the weight gradients: one product when the two outputs are one buffer (a layer's packed gradients)
+    const bool one_dw = n_extra && levels && d_w_levels == d_w_extra + (size_t)n_extra * d * d;
     if (product_bf16_serves(px, 1)) {
+        const ProductBf16 pw{G, x_bf16, nullptr, d_w_extra, R, d, (int)R, d, (int)n, 0, true, true};
+        if (one_dw && product_bf16_serves(pw, 2)) {
+            KernelTimer kt("gemm d_x and d_w");
+            product_bf16_pair(px, pw);
+            return;
+        }
         KernelTimer kt("gemm d_x");
         product_bf16(px, 1);
         if (es.failed()) return;
@@ -930,8 +929,7 @@ void titans_levels_backward_bf16_rocm(const uint16_t *x_bf16, const float *w_ext
         if (levels) to_bf16(w_levels, wb + (size_t)n_extra * d * d, 3LL * levels * d * d);
         if (es.failed() || !gemm_bf16("gemm d_x", rocblas_operation_none, rocblas_operation_none, d, n, R, wb, d, G, R, 0.f, d_x, d)) return;
     }
-    // the weight gradients: one product when the two outputs are one buffer (a layer's packed gradients)
-    if (n_extra && levels && d_w_levels == d_w_extra + (size_t)n_extra * d * d) {
+    if (one_dw) {
         gemm_weight_grad("gemm d_w", d, R, n, x_bf16, d, G, R, d_w_extra);
         return;
     }
@@ -990,8 +988,9 @@ void linear_backward_bf16_rocm(const float *d_out_f32, const uint16_t *a_bf16, c
     const ProductBf16 pw{d_out_f32, a_bf16, nullptr, d_w, d_out, d_in, d_out, d_in, n, 0, false, true};
     if ((!d_a || product_bf16_serves(pa, 1)) && (!d_w || product_bf16_serves(pw, 2))) {
         KernelTimer kt("gemm linear backward");
-        if (d_a) product_bf16(pa, 1);
-        if (d_w && !es.failed()) product_bf16(pw, 2);
+        if (d_a && d_w) product_bf16_pair(pa, pw);
+        else if (d_a) product_bf16(pa, 1);
+        else if (d_w) product_bf16(pw, 2);
         return;
     }
     u16 *wb = reinterpret_cast<u16 *>(scratch(27, (size_t)d_in * d_out * sizeof(u16)));

@@ -529,7 +529,6 @@ class MagLayer:
                                             d_attn.data_ptr(), g_op, g_op + 2 * d, g_op + 4 * d, ld.value, s, nh, hd,
                                             self.window, bs)
         d_x = _new(bs, s, d)
-        seeds = _zeros(2, hd, hd)
         d_extra = (ctypes.c_void_p * 3)(None, None, None)
         gl = grads.levels[:na]
         gate_out = (ctypes.c_void_p * (6 * na))(*[t.data_ptr() for g in gl for t in
@@ -539,7 +538,7 @@ class MagLayer:
             c["vh"].data_ptr(), c["qh"].data_ptr(), c["ah"].data_ptr(), c["th"].data_ptr(), c["eh"].data_ptr(),
             c["k_norms"].data_ptr(), c["q_norms"].data_ptr(), c["alpha"].data_ptr(), c["theta"].data_ptr(),
             c["eta"].data_ptr(), c["mc"].data_ptr(), c["sc"].data_ptr(), d_ycomb.data_ptr(), d_x.data_ptr(),
-            grads.pack.data_ptr(), grads.pack[3 * d:].data_ptr(), gate_out, seeds[0].data_ptr(), seeds[1].data_ptr(),
+            grads.pack.data_ptr(), grads.pack[3 * d:].data_ptr(), gate_out, None, None,
             bs, s, nh, hd, na, self.chunk, 1e-8)
         for i, lv in enumerate(range(na, k)):
             # read-only level: only the q path carries gradient
@@ -592,7 +591,7 @@ class MagLayer:
         do2 = d_out.reshape(n, d)
         if grads is None:
             grads = self.new_grads()
-        else:
+        elif not (cache.get("bf16") and cache["na"] == self.k):   # with every level active each one is written
             grads.flat.zero_()
         if cache.get("bf16"):
             return self._backward_bf16(cache, d_out, grads), grads

@@ -265,6 +265,23 @@ def test_linear_pair_at_the_edges_of_its_tiles(n, d_in, d_out):
         assert (np.abs(host(got) - x @ y) <= 2 ** -24 * (k + 4) * (np.abs(x) @ np.abs(y)) + 1e-30).all(), (n, d_in, d_out, k)
 
 
+@pytest.mark.parametrize("n,d_in,d_out", [(8, 64, 64), (72, 128, 64), (500, 256, 512), (1504, 256, 256)])
+def test_linear_gradients_side_by_side_are_those_of_single_calls(n, d_in, d_out):
+    """Both gradients of a projection in one launch against one call each: the same tiles, bit for bit, with and without a
+    contraction that is split (the longer ones)."""
+    g = torch.Generator(device="cuda").manual_seed(n)
+    tg, tw = torch.randn(n, d_out, generator=g, device="cuda"), torch.randn(d_out, d_in, generator=g, device="cuda")
+    ta = torch.randn(n, d_in, generator=g, device="cuda").to(BF)
+    out = [[torch.full(shape, float("nan"), device="cuda") for shape in ((n, d_in), (d_out, d_in))] for _ in range(2)]
+    call = lambda d_a, d_w: lib.linear_backward_bf16_rocm(tg.data_ptr(), ta.data_ptr(), tw.data_ptr(), d_a, d_w, n, d_in, d_out)
+    call(out[0][0].data_ptr(), out[0][1].data_ptr())
+    call(out[1][0].data_ptr(), None)
+    call(None, out[1][1].data_ptr())
+    torch.cuda.synchronize()
+    for both, one in zip(*out):
+        assert torch.equal(both, one)
+
+
 @pytest.mark.parametrize("place", ["d_a over d_out", "d_w over w", "d_w over d_out", "d_a over w", "out over w", "d_a behind the start of d_out"])
 def test_linear_pair_in_place(place):
     """A result in the place of an fp32 operand is the one in a place of its own: operands are rounded before it is written."""
