@@ -26,10 +26,10 @@
 namespace nlh {
 namespace {
 
-// Chunks that a wave of the coefficient passes walks over: up to four once there are waves enough for every compute unit's
-// eight places (their loads then run under the chunk before), one where there are fewer (four sequences of eight chunks:
+// Chunks that a wave of the coefficient passes walks over: up to four once there are sixteen waves for every compute unit
+// (their loads then run under the chunk before), one where there are fewer (four sequences of eight chunks:
 // 13 us in eight waves, 5 in 32).
-inline int coef_chunks_per_wave(int chunks) { return std::clamp(chunks / (8 * compute_units()), 1, 4); }
+inline int coef_chunks_per_wave(int chunks) { return std::clamp(chunks / (16 * compute_units()), 1, 4); }
 
 typedef float cf32x4 __attribute__((ext_vector_type(4)));
 
@@ -216,7 +216,11 @@ __device__ __forceinline__ cf32x4 coef_tile_jt(const ChunkCoef &cc, int J, int T
 // ── Coefficient tables written to HBM by a pre-pass (one wave per chunk) ──
 // The vectors of a chunk from two scans of composed maps instead of 64-step loops:
 //   a, beta, h = R, X, H of G(0..t);  cl, bl = R + X, H of G(t+1..63)   (tokens beyond L: identity map)
-struct ChunkVectors { float a, beta, h, cl, bl; };
+// and what its table is formed from: head_t, tail_t, and the maps of the two middle blocks.
+struct ChunkVectors {
+    float a, beta, h, cl, bl;
+    Map3 head, tail, mid1, mid2;
+};
 __device__ __forceinline__ ChunkVectors coef_vectors(float keep, float et, bool in) {
     const int t = threadIdx.x & 63;
     const Map3 g = in ? Map3{keep, et, et} : map_identity();
@@ -241,46 +245,101 @@ __device__ __forceinline__ ChunkVectors coef_vectors(float keep, float et, bool 
     const Map3 pre = T == 0 ? map_identity() : (T == 1 ? pre1 : (T == 2 ? pre2 : pre3));
     const Map3 post = T == 3 ? map_identity() : (T == 2 ? post2 : (T == 1 ? post1 : post0));
     const Map3 pf = compose(hd, pre), sx = compose(post, tl);
-    return ChunkVectors{pf.R, pf.X, pf.H, sx.R + sx.X, sx.H};
+    return ChunkVectors{pf.R, pf.X, pf.H, sx.R + sx.X, sx.H, hd, tl, blk[1], blk[2]};
 }
 
-// stage[t * LD + j] = scale_j c[t][j] for j <= t < L and zero elsewhere (64 rows of LD floats, LD a multiple of 4,
-// and one spare row behind them).
-// One wave, lane = j.  Lane j walks t = j, j + 1, .. on its own: at step i every lane multiplies (no lane waits
-// for its column to start), the gates of token j + i come from LDS (gk, ge: 128 floats each, identity from 64
-// on) at an immediate offset, and the destination is base + i * LD.  A step is two multiply-adds and a store
-// per lane, against a dozen instructions when the lanes advance through t together.
-template <int LD, bool SCALED>
-__device__ __forceinline__ void coef_table_columns(float *stage, float *gk, float *ge, float keep, float et,
-                                                   float scale, int L) {
-    const int j = threadIdx.x & 63;
-    gk[j] = keep; gk[64 + j] = 1.f;   // the caller passes keep = 1, eta = 0 beyond L
-    ge[j] = et;   ge[64 + j] = 0.f;
-    for (int e = j; e < 64 * LD / 4; e += 64) reinterpret_cast<cf32x4 *>(stage)[e] = cf32x4{0.f, 0.f, 0.f, 0.f};
-    // the gates of tokens j + 1 .. j + 63 in registers (requested in one go: no step waits for LDS), and every
-    // lane stores at every step (a lane whose column has ended stores to a spare row): no branch inside the walk
-    float kk[64], ee[64];
-#pragma unroll
-    for (int i = 1; i < 64; i++) { kk[i] = gk[j + i]; ee[i] = ge[j + i]; }
-    float b = 1.f, c = 1.f;
-    float *dst = stage + j * (LD + 1), *spare = stage + 64 * LD + j;
-    const bool jv = j < L;
-    dst[0] = jv ? (SCALED ? scale : 1.f) : 0.f;
-    if (L == 64) {
-#pragma unroll
-        for (int i = 1; i < 64; i++) {
-            b *= ee[i];
-            c = fmaf(kk[i], c, b);
-            *(j < 64 - i ? dst + i * LD : spare) = SCALED ? scale * c : c;
-        }
-    } else {
-#pragma unroll
-        for (int i = 1; i < 64; i++) {
-            b *= ee[i];
-            c = fmaf(kk[i], c, b);
-            *(j < 64 - i ? dst + i * LD : spare) = (jv && j < L - i) ? (SCALED ? scale * c : c) : 0.f;
-        }
+// The table scale_j c[t][j] of one chunk, tile by tile of 16 x 16, without a recurrence over its 64 tokens: tiles below the diagonal are head_t . mid . tail_j, two multiply-adds an entry, and the four tiles on it one
+// recurrence of 16 steps, a lane per column, whose gates come from the neighbouring lanes.  What bounds the pre-passes then is
+// the 10 KB that a chunk's ten tiles take in HBM: 8192 chunks in 19 and 18 us, 5.2 TB/s (27 and 37 when a lane walked down its
+// column, 64 steps, in 18 KB of LDS that let eight waves onto a compute unit), 16384 in 42 and 41 (50 and 64).
+constexpr int kDiagLd = 20;   // row stride (floats) of the diagonal tiles
+struct ChunkTable {
+    float hR[64], hX[64];             // head_t, zero beyond L
+    float zc[64], zh[64];             // tail_j times the column's factor
+    float diag[(64 + 16) * kDiagLd];  // [t][j % 16]; the last 16 rows take what runs past the chunk's end
+};
+// once per wave, before the first chunk: the part above the diagonal of the first tile, which no chunk writes
+__device__ __forceinline__ void chunk_table_clear(ChunkTable &ct) {
+    for (int e = threadIdx.x & 63; e < 16 * kDiagLd; e += 64) ct.diag[e] = 0.f;
+}
+// value of lane (i + N) of the same 16-lane row, zero behind its end
+template <int N>
+__device__ __forceinline__ float row_ahead(float x) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x100 + N, 0xF, 0xF, true));
+}
+template <int I>
+__device__ __forceinline__ void diag_steps(float *dst, float keep, float et, float b, float c) {
+    if constexpr (I < 16) {
+        b *= row_ahead<I>(et);
+        c = fmaf(row_ahead<I>(keep), c, b);
+        dst[I * kDiagLd] = c;
+        diag_steps<I + 1>(dst, keep, et, b, c);
     }
+}
+__device__ __forceinline__ void wave_lds_order() {   // LDS that the lanes of one wave exchange
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+// One wave, lane = token; keep and et are zero or the identity's beyond L, scale zero there.
+// A lane whose block has ended goes on with gates of zero: it writes zeros, and they land in the part of the next tile that is
+// above the diagonal (token j + i of the next block, column j: i < 16 leaves it above), which needs them.
+__device__ __forceinline__ void chunk_table_build(ChunkTable &ct, const ChunkVectors &cv, float keep, float et, float scale, int L) {
+    const int t = threadIdx.x & 63;
+    const bool in = t < L;
+    wave_lds_order();   // the chunk before has been read
+    ct.hR[t] = in ? cv.head.R : 0.f;
+    ct.hX[t] = in ? cv.head.X : 0.f;
+    ct.zc[t] = scale * (cv.tail.R + cv.tail.X);
+    ct.zh[t] = scale * cv.tail.H;
+    float *dst = ct.diag + t * kDiagLd + (t & 15);
+    dst[0] = scale;
+    diag_steps<1>(dst, in ? keep : 0.f, in ? et : 0.f, scale, scale);
+    wave_lds_order();
+}
+// what stands between blocks J and T > J
+template <int T, int J>
+__device__ __forceinline__ Map3 map_between(const ChunkVectors &cv) {
+    if constexpr (T == 2 && J == 0) return cv.mid1;
+    else if constexpr (T == 3 && J == 1) return cv.mid2;
+    else if constexpr (T == 3 && J == 0) return compose(cv.mid2, cv.mid1);
+    else return map_identity();
+}
+// Tile (T, J <= T): element i of lane l at t = 16 T + l % 16, j = 16 J + 4 (l / 16) + i (BY_TOKEN = false), or at
+// t = 16 T + 4 (l / 16) + i, j = 16 J + l % 16 (BY_TOKEN = true).
+template <bool BY_TOKEN, int T, int J>
+__device__ __forceinline__ cf32x4 chunk_table_tile(const ChunkTable &ct, const ChunkVectors &cv) {
+    const int l = threadIdx.x & 63, one = l & 15, four = 4 * (l >> 4);
+    auto four_of = [&](const float *p) { return *reinterpret_cast<const cf32x4 *>(p + four); };
+    if constexpr (T == J) {
+        const float *p = ct.diag + 16 * T * kDiagLd;
+        if constexpr (!BY_TOKEN) return four_of(p + one * kDiagLd);
+        p += four * kDiagLd + one;
+        return cf32x4{p[0], p[kDiagLd], p[2 * kDiagLd], p[3 * kDiagLd]};
+    } else {
+        const Map3 m = map_between<T, J>(cv);
+        cf32x4 out;
+        if constexpr (BY_TOKEN) {
+            const cf32x4 hR = four_of(ct.hR + 16 * T), hX = four_of(ct.hX + 16 * T);
+            const float zc = ct.zc[16 * J + one], zh = ct.zh[16 * J + one];
+            const float pc = fmaf(m.R, zc, m.X * zh), ph = m.H * zh;   // mid . tail: (R + X, H) of it is (pc, ph)
+#pragma unroll
+            for (int i = 0; i < 4; i++) out[i] = fmaf(hR[i], pc, hX[i] * ph);
+        } else {
+            const float hR = ct.hR[16 * T + one], hX = ct.hX[16 * T + one];
+            const float aR = hR * m.R, aX = fmaf(hR, m.X, hX * m.H);
+            const cf32x4 zc = four_of(ct.zc + 16 * J), zh = four_of(ct.zh + 16 * J);
+#pragma unroll
+            for (int i = 0; i < 4; i++) out[i] = fmaf(aR, zc[i], aX * zh[i]);
+        }
+        return out;
+    }
+}
+// f(T, J, tile) for the ten tiles on or below the diagonal
+template <bool BY_TOKEN, int T, int J, class F>
+__device__ __forceinline__ void chunk_table_tiles(const ChunkTable &ct, const ChunkVectors &cv, F &&f) {
+    f(T, J, chunk_table_tile<BY_TOKEN, T, J>(ct, cv));
+    if constexpr (J < T) chunk_table_tiles<BY_TOKEN, T, J + 1>(ct, cv, f);
+    else if constexpr (T < 3) chunk_table_tiles<BY_TOKEN, T + 1, 0>(ct, cv, f);
 }
 
 }  // namespace

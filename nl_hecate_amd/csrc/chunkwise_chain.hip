@@ -47,26 +47,24 @@ constexpr int kChainThr = 512;     // 8 waves
 //         then a_L, beta_L, h_L, one unused float and four zeros
 constexpr int kTableFloats = CW * CW;
 constexpr int kVecFloats = 4 * CW + 16;
-constexpr int kStageLd = CW + 4;   // row stride (floats) of the table while it is assembled in LDS
 __device__ __forceinline__ bool tile_live(int bi, int rt, int ct) { return 2 * (bi & 1) + ct >= 2 * (bi >> 1) + rt; }
 
 // Coefficients of one chunk from its gates: one wave per chunk, lane = token.  The vectors come from two scans
-// of composed maps, the table from coef_table_columns; it is assembled in LDS as W[t][j] and leaves in the
-// consumers' order as 16-byte stores of consecutive lanes.
+// of composed maps, the table tile by tile in the consumers' order (chunk_table_tiles), as 16-byte stores of consecutive lanes.
 template <bool HAS_S>
 __global__ __launch_bounds__(64) void cw_coef_kernel(const float *__restrict__ alpha,
                                                      const float *__restrict__ theta,
                                                      const float *__restrict__ eta, float *__restrict__ table,
                                                      float *__restrict__ vecs, int s, int C, int nc, int nchunks, int per_wave) {
-    __shared__ __align__(16) float stage[(CW + 1) * kStageLd];
-    __shared__ float gk[2 * CW], ge[2 * CW];
+    __shared__ __align__(16) ChunkTable ct;
+    chunk_table_clear(ct);
     const int j = threadIdx.x, first = blockIdx.x * per_wave, last = min(nchunks, first + per_wave);
     auto gates_of = [&](int chunk) {
         const int chain = chunk / nc, t0 = (chunk % nc) * C;
         return fetch_gates<HAS_S>(alpha, theta, eta, (size_t)chain * s + t0, min(C, s - t0));
     };
     // a wave walks over a few chunks with the next chunk's gates in flight: a wave per chunk would spend most of
-    // its life waiting for its three loads, and LDS allows only eight waves per compute unit
+    // its life waiting for its three loads
     Gates gn = gates_of(first);
     for (int chunk = first; chunk < last; chunk++) {
         const int L = min(C, s - (chunk % nc) * C);
@@ -82,17 +80,12 @@ __global__ __launch_bounds__(64) void cw_coef_kernel(const float *__restrict__ a
         vo[3 * CW + j] = nth * cv.bl;
         if (j == 63) { vo[4 * CW] = cv.a; vo[4 * CW + 1] = cv.beta; vo[4 * CW + 2] = cv.h; }   // the values at token L - 1
         if (j < 4) vo[4 * CW + 4 + j] = 0.f;   // zero pad: what tiles of W above the diagonal read
-        coef_table_columns<kStageLd, true>(stage, gk, ge, keep, et, nth, L);
+        chunk_table_build(ct, cv, keep, et, nth, L);
         float *out = table + (size_t)chunk * kTableFloats;
-        // the ten 16 x 16 tiles on or below the diagonal (token tile T >= column tile J), one 16-byte piece per lane each
-#pragma unroll
-        for (int T = 0; T < 4; T++)
-#pragma unroll
-            for (int J = 0; J <= T; J++) {
-                const int tile = ((J >> 1) * 2 + (T >> 1)) * 4 + (J & 1) * 2 + (T & 1);   // (bi, rt, ct) of the layout above
-                *reinterpret_cast<f32x4 *>(out + (tile * 64 + j) * 4) =
-                    *reinterpret_cast<const f32x4 *>(stage + (16 * T + (j & 15)) * kStageLd + 16 * J + 4 * (j >> 4));
-            }
+        chunk_table_tiles<false, 0, 0>(ct, cv, [&](int T, int J, const cf32x4 &w) __attribute__((always_inline)) {
+            const int tile = ((J >> 1) * 2 + (T >> 1)) * 4 + (J & 1) * 2 + (T & 1);   // (bi, rt, ct) of the layout above
+            *reinterpret_cast<cf32x4 *>(out + (tile * 64 + j) * 4) = w;
+        });
     }
 }
 

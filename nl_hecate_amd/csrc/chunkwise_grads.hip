@@ -49,24 +49,23 @@ constexpr int kVecB = 5 * CW + 16;
 constexpr int kCtLd = CW + 4;   // row stride (floats) of the coefficient copy in LDS
 __device__ __forceinline__ bool live_b(int bi, int rt, int ct) { return 2 * (bi >> 1) + rt >= 2 * (bi & 1) + ct; }
 
-// One wave per chunk, lane = token: the vectors from two scans of composed maps, the table from
-// coef_table_columns, assembled in LDS as c[t][j] and gathered in the consumers' order on the way out, as
-// 16-byte stores of consecutive lanes.
+// One wave per chunk, lane = token: the vectors from two scans of composed maps, the table tile by tile in the consumers'
+// order (chunk_table_tiles), as 16-byte stores of consecutive lanes.
 template <bool HAS_S>
 __global__ __launch_bounds__(64) void cw_coef_bwd_kernel(const float *__restrict__ alpha,
                                                          const float *__restrict__ theta,
                                                          const float *__restrict__ eta,
                                                          float *__restrict__ tab_b, float *__restrict__ vecs,
                                                          int s, int C, int nc, int nchunks, int per_wave) {
-    __shared__ __align__(16) float stage[(CW + 1) * kCtLd];
-    __shared__ float gk[2 * CW], ge[2 * CW];
+    __shared__ __align__(16) ChunkTable ct;
+    chunk_table_clear(ct);
     const int j = threadIdx.x, first = blockIdx.x * per_wave, last = min(nchunks, first + per_wave);
     auto gates_of = [&](int chunk) {
         const int chain = chunk / nc, t0 = (chunk % nc) * C;
         return fetch_gates<HAS_S>(alpha, theta, eta, (size_t)chain * s + t0, min(C, s - t0));
     };
     // a wave walks over a few chunks with the next chunk's gates in flight (a wave per chunk would spend most of
-    // its life waiting for its three loads, and LDS allows only eight waves per compute unit)
+    // its life waiting for its three loads)
     Gates gn = gates_of(first);
     for (int chunk = first; chunk < last; chunk++) {
         const int L = min(C, s - (chunk % nc) * C);
@@ -83,17 +82,12 @@ __global__ __launch_bounds__(64) void cw_coef_bwd_kernel(const float *__restrict
         vo[4 * CW + j] = g.th;
         if (j < 4) vo[5 * CW + j] = 0.f;   // what tiles above the diagonal read
         if (j == 63) vo[5 * CW + 4] = cv.h;   // h at token L - 1
-        coef_table_columns<kCtLd, false>(stage, gk, ge, keep, et, 1.f, L);
+        chunk_table_build(ct, cv, keep, et, jv ? 1.f : 0.f, L);
         float *ob = tab_b + (size_t)chunk * kTab;
-        // the ten 16 x 16 tiles on or below the diagonal (token tile T >= column tile J), one 16-byte piece per lane each
-#pragma unroll
-        for (int T = 0; T < 4; T++)
-#pragma unroll
-            for (int J = 0; J <= T; J++) {
-                const int tile = ((T >> 1) * 2 + (J >> 1)) * 4 + (T & 1) * 2 + (J & 1);   // (bi, rt, ct) of the layout above
-                const float *p = stage + (16 * T + 4 * (j >> 4)) * kCtLd + 16 * J + (j & 15);
-                *reinterpret_cast<f32x4 *>(ob + (tile * 64 + j) * 4) = f32x4{p[0], p[kCtLd], p[2 * kCtLd], p[3 * kCtLd]};
-            }
+        chunk_table_tiles<true, 0, 0>(ct, cv, [&](int T, int J, const cf32x4 &c) __attribute__((always_inline)) {
+            const int tile = ((T >> 1) * 2 + (J >> 1)) * 4 + (T & 1) * 2 + (J & 1);   // (bi, rt, ct) of the layout above
+            *reinterpret_cast<cf32x4 *>(ob + (tile * 64 + j) * 4) = c;
+        });
     }
 }
 

@@ -163,9 +163,8 @@ namespace nlh {
 // the forward's W[t][j]; vecs [5][64] = a, beta, h, cl, bl of token (lane).
 __global__ void chunk_coef_prepass_kernel(const float *alpha, const float *theta, const float *eta, int L,
                                           float *table, float *table_scaled, float *vecs) {
-    constexpr int LD = 68;
-    __shared__ __align__(16) float stage[65 * LD];
-    __shared__ float gk[128], ge[128];
+    __shared__ __align__(16) ChunkTable ct;
+    chunk_table_clear(ct);
     const int l = threadIdx.x;
     const bool in = l < L;
     const float keep = in ? 1.f - alpha[l] : 1.f, et = in ? eta[l] : 0.f, nth = in ? -theta[l] : 0.f;
@@ -175,10 +174,17 @@ __global__ void chunk_coef_prepass_kernel(const float *alpha, const float *theta
     vecs[2 * 64 + l] = cv.h;
     vecs[3 * 64 + l] = cv.cl;
     vecs[4 * 64 + l] = cv.bl;
-    coef_table_columns<LD, false>(stage, gk, ge, keep, et, 1.f, L);
-    for (int t = 0; t < 64; t++) table[t * 64 + l] = stage[t * LD + l];
-    coef_table_columns<LD, true>(stage, gk, ge, keep, et, nth, L);
-    for (int t = 0; t < 64; t++) table_scaled[t * 64 + l] = stage[t * LD + l];
+    for (int t = 0; t < 64; t++) table[t * 64 + l] = table_scaled[t * 64 + l] = 0.f;
+    __syncthreads();
+    const int one = l & 15, four = 4 * (l >> 4);
+    chunk_table_build(ct, cv, keep, et, in ? 1.f : 0.f, L);
+    chunk_table_tiles<true, 0, 0>(ct, cv, [&](int T, int J, const cf32x4 &c) {
+        for (int i = 0; i < 4; i++) table[(16 * T + four + i) * 64 + 16 * J + one] = c[i];
+    });
+    chunk_table_build(ct, cv, keep, et, nth, L);
+    chunk_table_tiles<false, 0, 0>(ct, cv, [&](int T, int J, const cf32x4 &w) {
+        for (int i = 0; i < 4; i++) table_scaled[(16 * T + one) * 64 + 16 * J + four + i] = w[i];
+    });
 }
 }  // namespace nlh
 
