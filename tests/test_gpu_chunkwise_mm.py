@@ -267,3 +267,36 @@ def test_delta_matrix_form_matches_oracle(B, s, C, bf16):
     for n in ("d_k", "d_v", "d_q", "d_alpha", "d_theta"):
         assert_close(n, host(g[n]), np.stack([o[n] for o in bw]), tol)
     assert_close("d_m_initial", host(g["d_m"]), sum(o["d_m"] for o in bw), tol)
+
+
+@pytest.mark.parametrize("rule,n,s,C", [("titans", 72, 2000, 64), ("titans", 9, 2049, 8), ("delta", 72, 2000, 32)])
+def test_gate_gradients_of_more_chunks_than_waves(rule, n, s, C):
+    """A wave of the gate sweeps walks over several chunks, the short last ones of chains among them; each chain's gradients are
+    those of a call with too few chunks for that, bit for bit, and the sums over the chains those of the parts."""
+    g = torch.Generator(device="cuda").manual_seed(n + C)
+    rnd = lambda *shape: torch.randn(*shape, generator=g, device="cuda")
+    mats, slots = (2, -(-s // C) + 1) if rule == "titans" else (1, -(-s // C) + 1)
+    kvq = [(rnd(n, s, 64) / 8).to(torch.bfloat16) for _ in range(3)]
+    gates = [torch.sigmoid(rnd(n, s)) for _ in range(mats + 1)]
+    m0, d_y = rnd(n, 64, 64) * 0.1, rnd(n, s, 64)
+
+    def both(a, b):
+        cut = lambda t: t[a:b].contiguous()
+        x, initial = [cut(t) for t in kvq + gates], [cut(m0)] + [zeros(b - a, 64, 64)] * (mats - 1)
+        states = [zeros(b - a, slots, 64, 64) for _ in range(mats)]
+        out = [zeros(b - a, s, 64) for _ in range(3)] + [zeros(b - a, s) for _ in gates]
+        d0 = [zeros(64, 64) for _ in range(mats)]
+        D.call(f"{rule}_chunkwise_forward_bf16_rocm", *x, *initial, *states, zeros(b - a, s, 64), s, 64, b - a, C)
+        D.call(f"{rule}_chunkwise_backward_bf16_rocm", *x, *states, cut(d_y), *out, *d0, s, 64, b - a, C)
+        torch.cuda.synchronize()
+        return out[3:], d0
+
+    whole, d0 = both(0, n)
+    cuts = [i * n // 9 for i in range(10)]
+    parts = [both(a, b) for a, b in zip(cuts, cuts[1:])]
+    for i, t in enumerate(whole):
+        assert torch.equal(t, torch.cat([p[0][i] for p in parts])), i
+    for i, t in enumerate(d0):   # n float terms in another order
+        want = sum(p[1][i].double() for p in parts)
+        size = sum(p[1][i].abs().double() for p in parts)
+        assert ((t.double() - want).abs() <= 2 ** -24 * 2 * n * (size + 8 * size.mean())).all(), i
