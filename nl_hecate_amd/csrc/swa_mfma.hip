@@ -62,6 +62,11 @@ __device__ __forceinline__ float groups_max(float x) {
     asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(a), "+v"(b));
     return fmaxf(a, b);
 }
+// LDS that the lanes of one wave exchange
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
 // mask of elements e (low half) and e + 1 of those numbered first .. last
 __device__ __forceinline__ unsigned own_pair(int e, int first, int last) {
     return (e >= first && e <= last ? 0xffffu : 0u) | (e + 1 >= first && e + 1 <= last ? 0xffff0000u : 0u);
@@ -275,11 +280,15 @@ __global__ __launch_bounds__(256, 3) void swa_fwd_stats_kernel(const unsigned sh
 
 // Forward of the contract (normalised weights stored) in the same blocks: the weights need the final maximum
 // and sum, so the window is swept twice — scores and running statistics first, then scores again, the weights
-// w = bf16(exp2(s c - m) / sum) to their slot rows (four consecutive slots per lane and tile: 8-byte stores at
-// 2-byte alignment) and O^T += V^T w^T.  Slots behind an early query's own key (t < window - 1) are zeroed at
-// the end.  8 x 4096 tokens, 8 heads, window 512: 0.21 ms, 0.14 of them without the stores.  A lane's own maximum and sum,
-// joined at the end, and 16-byte stores from stages permuted by stage_row took the same 0.21 ms and other bf16 neighbours.
-template <int HDV>
+// w = bf16(exp2(s c - m) / sum) to their slot rows and O^T += V^T w^T.  Slots behind an early query's own key (t < window - 1)
+// are zeroed at the end.
+// What bounds it is the weights' way out: a query's row in the tensor starts at its own key, so a lane's four keys are 8 bytes at
+// any even address.  Where rows are whole 16-byte pieces (PIECES) a wave passes the stage's weights of 16 queries through LDS,
+// behind the eight keys before the stage, and stores the pieces that the stage completes: 128 contiguous aligned bytes a query.
+// 8 x 4096 tokens, 8 heads, window 512: 0.21 -> 0.175 ms, 0.14 without any stores; forward and backward 589 -> 556 us.
+// A lane's own maximum and sum, joined at the end, gave other bf16 neighbours.
+constexpr int LDP = 76;    // row stride of the pieces' LDS (8 keys of the stage before, 64 of this one)
+template <int HDV, bool PIECES>
 __global__ __launch_bounds__(256, 3) void swa_fwd_blocked_kernel(const unsigned short *__restrict__ q,
                                                               const unsigned short *__restrict__ k,
                                                               const unsigned short *__restrict__ v,
@@ -288,6 +297,7 @@ __global__ __launch_bounds__(256, 3) void swa_fwd_blocked_kernel(const unsigned 
                                                               int ws) {
     __shared__ __align__(16) unsigned short Ks[2][KS][LDH];   // K stage [key][dim]
     __shared__ __align__(16) unsigned short Vs[2][KS][LDV];   // V stage [key][dim]
+    __shared__ __align__(16) unsigned short Ws[PIECES ? 4 : 1][PIECES ? 16 : 1][LDP];   // a wave each: weights on their way out
     const int tid = threadIdx.x, wave = tid >> 6, l = tid & 63, r = l & 15, g = l >> 4;
     const BlockCoord bc = xcd_block_coord(H);
     const int t0 = bc.x * FQ, h = bc.h, b = bc.b;
@@ -388,14 +398,8 @@ __global__ __launch_bounds__(256, 3) void swa_fwd_blocked_kernel(const unsigned 
     for (int qt = 0; qt < 2; qt++)
 #pragma unroll
         for (int dt = 0; dt < NDT; dt++) o[qt][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
-    unsigned short *wrow[2];
-    int lsq[2];
-#pragma unroll
-    for (int qt = 0; qt < 2; qt++) {
-        const int tq = qlo + 16 * qt + r;
-        lsq[qt] = max(tq + 1 - ws, 0);
-        wrow[qt] = attn_w + ((size_t)(b * H + h) * s + min(tq, s - 1)) * ws;
-    }
+    unsigned short *wblk = attn_w + ((size_t)(b * H + h) * s + qlo) * ws;   // row of the wave's first query
+    uint2 before[2] = {};   // PIECES: the weights of the last tile of the stage before
     __syncthreads();   // every wave is done with the buffers of sweep 1
     load_rows<HDV>(km, KS * st_lo, kreg);
     load_rows<HDV>(vm, KS * st_lo, vreg);
@@ -415,37 +419,72 @@ __global__ __launch_bounds__(256, 3) void swa_fwd_blocked_kernel(const unsigned 
         if (k0 > qhi || k0 + KS - 1 < qlo + 1 - ws) continue;
         f32x4 sc[4][2];
         scores(buf, k0, sc);
+        unsigned wp[2][4][2];
+#pragma unroll
+        for (int qt = 0; qt < 2; qt++)
+#pragma unroll
+            for (int kt = 0; kt < 4; kt++) {
+                const f32x4 x = sc[kt][qt];
+                float w[4];
+#pragma unroll
+                for (int i = 0; i < 4; i++) w[i] = __builtin_amdgcn_exp2f(fmaf(x[i], c2, -mc[qt])) * inv[qt];
+                wp[qt][kt][0] = pack2(w[0], w[1]);
+                wp[qt][kt][1] = pack2(w[2], w[3]);
+            }
+        if constexpr (PIECES) {
+            unsigned short(*W)[LDP] = Ws[wave];
+            const int pr = l >> 3, pj = l & 7;   // the lane's row (of 8) and piece on the way out
+#pragma unroll
+            for (int qt = 0; qt < 2; qt++) {
+                wave_lds_order();
+                if (g >= 2) *reinterpret_cast<uint2 *>(&W[r][4 * (g - 2)]) = before[qt];
+#pragma unroll
+                for (int kt = 0; kt < 4; kt++) *reinterpret_cast<uint2 *>(&W[r][8 + 16 * kt + 4 * g]) = make_uint2(wp[qt][kt][0], wp[qt][kt][1]);
+                before[qt] = make_uint2(wp[qt][3][0], wp[qt][3][1]);
+                wave_lds_order();
+#pragma unroll
+                for (int half = 0; half < 2; half++) {
+                    const int row = 8 * half + pr, tq = qlo + 16 * qt + row, ls = max(tq + 1 - ws, 0);
+                    const int first = k0 - ls, piece = (first >> 3) + pj;   // slots 8 piece .. + 7: keys from k0 - first % 8 + 8 pj on
+                    // the stage completes eight pieces, less those in front of the row and behind the query's own key
+                    const int e = 8 - (first & 7) + 8 * pj, sh = 16 * (e & 1);
+                    const unsigned *src = reinterpret_cast<const unsigned *>(W[row]) + (e >> 1);
+                    const unsigned d0 = src[0], d1 = src[1], d2 = src[2], d3 = src[3], d4 = src[4];   // d4 may lie in the row's pad: unused then
+                    if (tq < s && piece >= 0 && 8 * piece <= tq - ls)
+                        *reinterpret_cast<uint4 *>(wblk + (size_t)(16 * qt + row) * ws + 8 * piece) =
+                            make_uint4(__builtin_amdgcn_alignbit(d1, d0, sh), __builtin_amdgcn_alignbit(d2, d1, sh),
+                                       __builtin_amdgcn_alignbit(d3, d2, sh), __builtin_amdgcn_alignbit(d4, d3, sh));
+                }
+            }
+        } else {
+#pragma unroll
+            for (int qt = 0; qt < 2; qt++) {
+                const int tq = qlo + 16 * qt + r, ls = max(tq + 1 - ws, 0);
+                unsigned short *wrow = wblk + (size_t)(16 * qt + r) * ws;
+#pragma unroll
+                for (int kt = 0; kt < 4; kt++) {
+                    // keys key0 .. key0 + 3 of query tq sit in slots key0 - ls ..; only keys of the window have one
+                    const int key0 = k0 + 16 * kt + 4 * g;
+                    if (tq < s) {
+                        if (key0 >= ls && key0 + 3 <= tq) {
+                            const uint2 pr = make_uint2(wp[qt][kt][0], wp[qt][kt][1]);
+                            __builtin_memcpy(wrow + (key0 - ls), &pr, 8);
+                        } else if (key0 + 3 >= ls && key0 <= tq) {
+#pragma unroll
+                            for (int i = 0; i < 4; i++)
+                                if (key0 + i >= ls && key0 + i <= tq)
+                                    wrow[key0 + i - ls] = (unsigned short)(wp[qt][kt][i >> 1] >> (16 * (i & 1)));
+                        }
+                    }
+                }
+            }
+        }
 #pragma unroll
         for (int hf = 0; hf < 2; hf++) {
             uint4 pb[2];
 #pragma unroll
-            for (int qt = 0; qt < 2; qt++) {
-                const int tq = qlo + 16 * qt + r;
-                unsigned wp[2][2];
-#pragma unroll
-                for (int c = 0; c < 2; c++) {
-                    const f32x4 x = sc[2 * hf + c][qt];
-                    float w[4];
-#pragma unroll
-                    for (int i = 0; i < 4; i++) w[i] = __builtin_amdgcn_exp2f(fmaf(x[i], c2, -mc[qt])) * inv[qt];
-                    wp[c][0] = pack2(w[0], w[1]);
-                    wp[c][1] = pack2(w[2], w[3]);
-                    // keys key0 .. key0 + 3 of query tq sit in slots key0 - lsq ..; only keys of the window have one
-                    const int key0 = k0 + 16 * (2 * hf + c) + 4 * g;
-                    if (tq < s) {
-                        if (key0 >= lsq[qt] && key0 + 3 <= tq) {
-                            const uint2 pr = make_uint2(wp[c][0], wp[c][1]);
-                            __builtin_memcpy(wrow[qt] + (key0 - lsq[qt]), &pr, 8);
-                        } else if (key0 + 3 >= lsq[qt] && key0 <= tq) {
-#pragma unroll
-                            for (int i = 0; i < 4; i++)
-                                if (key0 + i >= lsq[qt] && key0 + i <= tq)
-                                    wrow[qt][key0 + i - lsq[qt]] = (unsigned short)(wp[c][i >> 1] >> (16 * (i & 1)));
-                        }
-                    }
-                }
-                pb[qt] = make_uint4(wp[0][0], wp[0][1], wp[1][0], wp[1][1]);
-            }
+            for (int qt = 0; qt < 2; qt++)
+                pb[qt] = make_uint4(wp[qt][2 * hf][0], wp[qt][2 * hf][1], wp[qt][2 * hf + 1][0], wp[qt][2 * hf + 1][1]);
 #pragma unroll
             for (int dt = 0; dt < NDT; dt++) {
                 const uint4 av = ld_tr2<LDV>(Vs[buf], 32 * hf + 4 * g, 32 * hf + 16 + 4 * g, 16 * dt);
@@ -1281,10 +1320,11 @@ bool swa_forward_mfma(const uint16_t *q, const uint16_t *k, const uint16_t *v, u
         return true;
     }
     KernelTimer kt("swa_fwd_blocked_kernel");
-    if (head_dim == 64) hipLaunchKernelGGL(swa_fwd_blocked_kernel<64>, dim3((seq_len + FQ - 1) / FQ, num_heads, batch), dim3(256), 0, stream(), q,
-                       k, v, out, attn_weights, seq_len, num_heads, window);
-    else hipLaunchKernelGGL(swa_fwd_blocked_kernel<32>, dim3((seq_len + FQ - 1) / FQ, num_heads, batch), dim3(256), 0, stream(), q,
-                       k, v, out, attn_weights, seq_len, num_heads, window);
+    const bool pieces = window % 8 == 0 && ((uintptr_t)attn_weights & 15) == 0;   // rows of whole 16-byte pieces
+    auto kernel = head_dim == 64 ? (pieces ? swa_fwd_blocked_kernel<64, true> : swa_fwd_blocked_kernel<64, false>)
+                                 : (pieces ? swa_fwd_blocked_kernel<32, true> : swa_fwd_blocked_kernel<32, false>);
+    hipLaunchKernelGGL(kernel, dim3((seq_len + FQ - 1) / FQ, num_heads, batch), dim3(256), 0, stream(), q, k, v, out, attn_weights,
+                       seq_len, num_heads, window);
     check_launch("swa_fwd_blocked_kernel");
     return true;
 }

@@ -107,6 +107,26 @@ def test_forward_keeps_its_order_of_sums(B, s, H, hd, ws, out_sha, weights_sha):
     assert [hashlib.sha256(x.tobytes()).hexdigest()[:16] for x in (out, aw)] == [out_sha, weights_sha]
 
 
+@pytest.mark.parametrize("hd", [64, 32])
+@pytest.mark.parametrize("s,ws", [(1, 8), (65, 8), (64, 64), (63, 512), (127, 24), (129, 72), (300, 64), (777, 256), (1100, 512)])
+def test_weights_stored_in_pieces_and_in_fours(s, ws, hd):
+    """Rows of whole 16-byte pieces leave through LDS; the same call on a weight tensor two elements further on, whose rows are not,
+    stores a lane's keys by themselves: weights and output bit for bit the same, and nothing outside the tensor touched."""
+    B, H = 2, 3
+    q, k, v, _ = _case(B, s, H, hd, 900 + s + ws + hd)
+    n, got = B * H * s * ws, []
+    for at in (8, 10):
+        out = torch.zeros(B, s, H * hd, dtype=torch.uint16, device="cuda")
+        room = torch.full((n + 24,), 0x7fc0, dtype=torch.uint16, device="cuda")
+        D.call("swa_forward_f32_cuda", _u16(q), _u16(k), _u16(v), out, room[at:at + n], s, H, hd, ws, B, 0)
+        torch.cuda.synchronize()
+        a = room.cpu().numpy()
+        assert (a[:at] == 0x7fc0).all() and (a[at + n:] == 0x7fc0).all()
+        got.append((a[at:at + n], out.cpu().numpy()))
+    for x, y in zip(*got):
+        assert np.array_equal(x, y)
+
+
 @pytest.mark.parametrize("s,ws,hd", [(1, 4, 64), (31, 32, 32), (33, 2, 64), (128, 128, 32), (161, 64, 64), (200, 101, 32),
                                      (353, 130, 64), (600, 512, 64), (600, 511, 32)])
 def test_backward_in_blocks_of_32_rows_and_of_128(s, ws, hd):
