@@ -203,6 +203,16 @@ def gpu_cms_backward(params: GpuMAGParams, cfg: ModelConfig, cache, collect_outp
     c = cache
     s, d, v, nh, hd, ws, bs = cfg.seq_len, cfg.d_model, cfg.vocab_size, cfg.num_heads, cfg.head_dim, cfg.window_size, c["bs"]
     n = bs * s
+    # the two longest kernels first: the forward ended by waiting for its loss, so nothing runs until they are there, and the
+    # gradients' buffers are made under them
+    valid = c["valid"]
+    d_logits = _new(n, v)
+    D.call("cross_entropy_backward_cuda", c["logits"], c["target_ids"], d_logits, n, v, 1.0 / (valid if valid > 0 else 1))
+    if _plain(params.w_unembed, d, v):   # a contraction over the vocabulary for few output tiles
+        d_projected = _new(n, d)
+        product(0, d_logits, params.w_unembed, d_projected, n, d, v)
+    else:
+        d_projected = d_logits @ params.w_unembed.t()
     inter = lambda lv: cfg.levels[lv].intermediate_size if cfg.levels[lv].memory_rule == "swiglu" else 0
     # what a product or a grouped level writes whole needs no clearing
     lgrads = []
@@ -213,14 +223,6 @@ def gpu_cms_backward(params: GpuMAGParams, cfg: ModelConfig, cache, collect_outp
     wq, wk, wv, wo = _new(4, d, d).unbind(0)
     ln_g = _zeros(4, d).unbind(0)
     g = GpuMAGGrads(_zeros(v, d), wq, wk, wv, wo, _new(d, v), *ln_g, lgrads, [0.0] * cfg.k)
-    valid = c["valid"]
-    d_logits = _new(n, v)
-    D.call("cross_entropy_backward_cuda", c["logits"], c["target_ids"], d_logits, n, v, 1.0 / (valid if valid > 0 else 1))
-    if _plain(params.w_unembed, d, v):   # a contraction over the vocabulary for few output tiles
-        d_projected = _new(n, d)
-        product(0, d_logits, params.w_unembed, d_projected, n, d, v)
-    else:
-        d_projected = d_logits @ params.w_unembed.t()
     product(2, c["projected"], d_logits, g.d_w_unembed, d, v, n)
     d_gated_out = d_projected @ params.w_o
     torch.mm(d_projected.t(), c["residual_final"] if cfg.residual else c["gated_out"], out=g.d_w_o)
