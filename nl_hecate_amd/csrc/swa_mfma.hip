@@ -129,7 +129,11 @@ __device__ __forceinline__ uint4 ld_op(unsigned short (*T)[LDH], int row0, int k
 // unnormalised weights; the division by the sum happens once at the end.  K and V rows are staged as they
 // arrive; V^T is read through ds_read_b64_tr_b16: group g of a wave takes keys 32 hf + 4 g .. + 3 and
 // 32 hf + 16 + 4 g .. + 3, which are exactly the rows that the two score tiles of that half leave in its lanes.
-constexpr int FQ = 128;    // queries per workgroup
+// Queries per workgroup: 32 a wave, or 16 (NQ = 1) below two workgroups of 128 for a compute unit: a call then takes as long as
+// one wave's chain of stages, which is shorter with one query tile.  Every query's sums keep their order.  Workgroups of 128,
+// us with 32 and with 16 (weights stored; statistics): 32 30 / 19; 12.9 / 9.1, 256 32 / 25; 17 / 13.5, 376 28 / 21; 16 / 11.6,
+// 512 41 / 42; 22.7 / 20.8.
+constexpr int FQ = 128;
 constexpr int LDV = 80;    // row stride of the V stage (160 B: the transposing reads of a group fall on 32 banks)
 
 template <int LD>
@@ -143,7 +147,7 @@ __device__ __forceinline__ uint4 ld_tr2(const unsigned short (*T)[LD], int row_a
     return make_uint4(ua.x, ua.y, ub.x, ub.y);
 }
 
-template <int HDV>
+template <int HDV, int NQ>
 __global__ __launch_bounds__(256, 3) void swa_fwd_stats_kernel(const unsigned short *__restrict__ q,
                                                             const unsigned short *__restrict__ k,
                                                             const unsigned short *__restrict__ v,
@@ -152,31 +156,34 @@ __global__ __launch_bounds__(256, 3) void swa_fwd_stats_kernel(const unsigned sh
     __shared__ __align__(16) unsigned short Ks[2][KS][LDH];   // K stage [key][dim]
     __shared__ __align__(16) unsigned short Vs[2][KS][LDV];   // V stage [key][dim]
     const int tid = threadIdx.x, wave = tid >> 6, l = tid & 63, r = l & 15, g = l >> 4;
+    constexpr int kRows = 64 * NQ;
     const BlockCoord bc = xcd_block_coord(H);
-    const int t0 = bc.x * FQ, h = bc.h, b = bc.b;
+    const int t0 = bc.x * kRows, h = bc.h, b = bc.b;
     constexpr int NKS = HDV / 32, NDT = HDV / 16;
     constexpr float kInvSqrt = HDV == 64 ? 0.125f : 0.17677669529663687f;   // 1 / sqrt(head size)
     const int total = H * HDV, hoff = h * HDV;
     const size_t row0 = (size_t)b * s;
-    const int qlo = t0 + 32 * wave, qhi = qlo + 31;           // this wave's queries
-    const int st_lo = max(t0 + 1 - ws, 0) / KS, st_hi = min(t0 + FQ - 1, s - 1) / KS;
+    const int qlo = t0 + 16 * NQ * wave, qhi = qlo + 16 * NQ - 1;           // this wave's queries
+    const int st_lo = max(t0 + 1 - ws, 0) / KS, st_hi = min(t0 + kRows - 1, s - 1) / KS;
     const StageSrc km{k, row0, total, hoff, s}, vm{v, row0, total, hoff, s};
 
-    uint4 qf[2][2];   // B operand: query qlo + 16 qt + r, dims 32 ks + 8 g ..
+    uint4 qf[NQ][2];   // B operand: query qlo + 16 qt + r, dims 32 ks + 8 g ..
 #pragma unroll
-    for (int qt = 0; qt < 2; qt++)
+    for (int qt = 0; qt < NQ; qt++)
 #pragma unroll
         for (int ks = 0; ks < NKS; ks++) {
             const int tq = qlo + 16 * qt + r;
             qf[qt][ks] = make_uint4(0, 0, 0, 0);
             if (tq < s) qf[qt][ks] = *reinterpret_cast<const uint4 *>(q + (row0 + tq) * total + hoff + 32 * ks + 8 * g);
         }
-    f32x4 o[2][4];
+    f32x4 o[NQ][4];
 #pragma unroll
-    for (int qt = 0; qt < 2; qt++)
+    for (int qt = 0; qt < NQ; qt++)
 #pragma unroll
         for (int dt = 0; dt < NDT; dt++) o[qt][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
-    float mrun[2] = {-INFINITY, -INFINITY}, lsum[2] = {0.f, 0.f};   // running maximum (exp2 units), this lane's share of the sum
+    float mrun[NQ], lsum[NQ];   // running maximum (exp2 units), this lane's share of the sum
+#pragma unroll
+    for (int qt = 0; qt < NQ; qt++) { mrun[qt] = -INFINITY; lsum[qt] = 0.f; }
     const float c2 = kInvSqrt * 1.44269504088896340736f;   // log2(e) / sqrt(head size)
 
     uint4 kreg[2], vreg[2];
@@ -196,12 +203,12 @@ __global__ __launch_bounds__(256, 3) void swa_fwd_stats_kernel(const unsigned sh
             load_rows<HDV>(vm, k0 + KS, vreg);
         }
         if (k0 > qhi || k0 + KS - 1 < qlo + 1 - ws) continue;   // no key of this stage is seen by this wave's queries
-        f32x4 sc[4][2];
+        f32x4 sc[4][NQ];
 #pragma unroll
         for (int kt = 0; kt < 4; kt++) {
             const uint4 a0 = ld_op(Ks[buf], 16 * kt, 0), a1 = ld_op(Ks[buf], 16 * kt, 1);
 #pragma unroll
-            for (int qt = 0; qt < 2; qt++) {
+            for (int qt = 0; qt < NQ; qt++) {
                 sc[kt][qt] = mfma32(a0, qf[qt][0], f32x4{0.f, 0.f, 0.f, 0.f});
                 if constexpr (NKS == 2) sc[kt][qt] = mfma32(a1, qf[qt][1], sc[kt][qt]);
             }
@@ -211,7 +218,7 @@ __global__ __launch_bounds__(256, 3) void swa_fwd_stats_kernel(const unsigned sh
 #pragma unroll
             for (int kt = 0; kt < 4; kt++)
 #pragma unroll
-                for (int qt = 0; qt < 2; qt++)
+                for (int qt = 0; qt < NQ; qt++)
 #pragma unroll
                     for (int i = 0; i < 4; i++) {
                         const int key = k0 + 16 * kt + 4 * g + i, tq = qlo + 16 * qt + r;
@@ -220,7 +227,7 @@ __global__ __launch_bounds__(256, 3) void swa_fwd_stats_kernel(const unsigned sh
                     }
         }
 #pragma unroll
-        for (int qt = 0; qt < 2; qt++) {
+        for (int qt = 0; qt < NQ; qt++) {
             float mx = -INFINITY;
 #pragma unroll
             for (int kt = 0; kt < 4; kt++)
@@ -246,9 +253,9 @@ __global__ __launch_bounds__(256, 3) void swa_fwd_stats_kernel(const unsigned sh
         }
 #pragma unroll
         for (int hf = 0; hf < 2; hf++) {
-            uint4 pb[2];
+            uint4 pb[NQ];
 #pragma unroll
-            for (int qt = 0; qt < 2; qt++) {
+            for (int qt = 0; qt < NQ; qt++) {
                 const f32x4 p0 = sc[2 * hf][qt], p1 = sc[2 * hf + 1][qt];
                 pb[qt] = make_uint4(pack2(p0[0], p0[1]), pack2(p0[2], p0[3]), pack2(p1[0], p1[1]), pack2(p1[2], p1[3]));
             }
@@ -256,12 +263,12 @@ __global__ __launch_bounds__(256, 3) void swa_fwd_stats_kernel(const unsigned sh
             for (int dt = 0; dt < NDT; dt++) {
                 const uint4 av = ld_tr2<LDV>(Vs[buf], 32 * hf + 4 * g, 32 * hf + 16 + 4 * g, 16 * dt);
 #pragma unroll
-                for (int qt = 0; qt < 2; qt++) o[qt][dt] = mfma32(av, pb[qt], o[qt][dt]);
+                for (int qt = 0; qt < NQ; qt++) o[qt][dt] = mfma32(av, pb[qt], o[qt][dt]);
             }
         }
     }
 #pragma unroll
-    for (int qt = 0; qt < 2; qt++) {
+    for (int qt = 0; qt < NQ; qt++) {
         const int tq = qlo + 16 * qt + r;
         float sum = lsum[qt];
         sum += __shfl_xor(sum, 16, 64);
@@ -288,7 +295,7 @@ __global__ __launch_bounds__(256, 3) void swa_fwd_stats_kernel(const unsigned sh
 // 8 x 4096 tokens, 8 heads, window 512: 0.21 -> 0.175 ms, 0.14 without any stores; forward and backward 589 -> 556 us.
 // A lane's own maximum and sum, joined at the end, gave other bf16 neighbours.
 constexpr int LDP = 76;    // row stride of the pieces' LDS (8 keys of the stage before, 64 of this one)
-template <int HDV, bool PIECES>
+template <int HDV, bool PIECES, int NQ>
 __global__ __launch_bounds__(256, 3) void swa_fwd_blocked_kernel(const unsigned short *__restrict__ q,
                                                               const unsigned short *__restrict__ k,
                                                               const unsigned short *__restrict__ v,
@@ -299,20 +306,21 @@ __global__ __launch_bounds__(256, 3) void swa_fwd_blocked_kernel(const unsigned 
     __shared__ __align__(16) unsigned short Vs[2][KS][LDV];   // V stage [key][dim]
     __shared__ __align__(16) unsigned short Ws[PIECES ? 4 : 1][PIECES ? 16 : 1][LDP];   // a wave each: weights on their way out
     const int tid = threadIdx.x, wave = tid >> 6, l = tid & 63, r = l & 15, g = l >> 4;
+    constexpr int kRows = 64 * NQ;
     const BlockCoord bc = xcd_block_coord(H);
-    const int t0 = bc.x * FQ, h = bc.h, b = bc.b;
+    const int t0 = bc.x * kRows, h = bc.h, b = bc.b;
     constexpr int NKS = HDV / 32, NDT = HDV / 16;
     constexpr float kInvSqrt = HDV == 64 ? 0.125f : 0.17677669529663687f;   // 1 / sqrt(head size)
     const int total = H * HDV, hoff = h * HDV;
     const size_t row0 = (size_t)b * s;
-    const int qlo = t0 + 32 * wave, qhi = qlo + 31;
-    const int st_lo = max(t0 + 1 - ws, 0) / KS, st_hi = min(t0 + FQ - 1, s - 1) / KS;
+    const int qlo = t0 + 16 * NQ * wave, qhi = qlo + 16 * NQ - 1;
+    const int st_lo = max(t0 + 1 - ws, 0) / KS, st_hi = min(t0 + kRows - 1, s - 1) / KS;
     const StageSrc km{k, row0, total, hoff, s}, vm{v, row0, total, hoff, s};
     const float c2 = kInvSqrt * 1.44269504088896340736f;
 
-    uint4 qf[2][2];
+    uint4 qf[NQ][2];
 #pragma unroll
-    for (int qt = 0; qt < 2; qt++)
+    for (int qt = 0; qt < NQ; qt++)
 #pragma unroll
         for (int ks = 0; ks < NKS; ks++) {
             const int tq = qlo + 16 * qt + r;
@@ -320,12 +328,12 @@ __global__ __launch_bounds__(256, 3) void swa_fwd_blocked_kernel(const unsigned 
             if (tq < s) qf[qt][ks] = *reinterpret_cast<const uint4 *>(q + (row0 + tq) * total + hoff + 32 * ks + 8 * g);
         }
     // scores of one stage for this wave's two query tiles, masked keys at -inf
-    auto scores = [&](int buf, int k0, f32x4 (&sc)[4][2]) {
+    auto scores = [&](int buf, int k0, f32x4 (&sc)[4][NQ]) {
 #pragma unroll
         for (int kt = 0; kt < 4; kt++) {
             const uint4 a0 = ld_op(Ks[buf], 16 * kt, 0), a1 = ld_op(Ks[buf], 16 * kt, 1);
 #pragma unroll
-            for (int qt = 0; qt < 2; qt++) {
+            for (int qt = 0; qt < NQ; qt++) {
                 sc[kt][qt] = mfma32(a0, qf[qt][0], f32x4{0.f, 0.f, 0.f, 0.f});
                 if constexpr (NKS == 2) sc[kt][qt] = mfma32(a1, qf[qt][1], sc[kt][qt]);
             }
@@ -335,7 +343,7 @@ __global__ __launch_bounds__(256, 3) void swa_fwd_blocked_kernel(const unsigned 
 #pragma unroll
             for (int kt = 0; kt < 4; kt++)
 #pragma unroll
-                for (int qt = 0; qt < 2; qt++)
+                for (int qt = 0; qt < NQ; qt++)
 #pragma unroll
                     for (int i = 0; i < 4; i++) {
                         const int key = k0 + 16 * kt + 4 * g + i, tq = qlo + 16 * qt + r;
@@ -346,7 +354,9 @@ __global__ __launch_bounds__(256, 3) void swa_fwd_blocked_kernel(const unsigned 
     };
 
     // ---- sweep 1: running maximum and sum ----
-    float mrun[2] = {-INFINITY, -INFINITY}, lsum[2] = {0.f, 0.f};
+    float mrun[NQ], lsum[NQ];
+#pragma unroll
+    for (int qt = 0; qt < NQ; qt++) { mrun[qt] = -INFINITY; lsum[qt] = 0.f; }
     uint4 kreg[2], vreg[2];
     load_rows<HDV>(km, KS * st_lo, kreg);
     for (int st = st_lo; st <= st_hi; st++) {
@@ -359,10 +369,10 @@ __global__ __launch_bounds__(256, 3) void swa_fwd_blocked_kernel(const unsigned 
         __syncthreads();
         if (st < st_hi) load_rows<HDV>(km, k0 + KS, kreg);
         if (k0 > qhi || k0 + KS - 1 < qlo + 1 - ws) continue;
-        f32x4 sc[4][2];
+        f32x4 sc[4][NQ];
         scores(buf, k0, sc);
 #pragma unroll
-        for (int qt = 0; qt < 2; qt++) {
+        for (int qt = 0; qt < NQ; qt++) {
             float mx = -INFINITY;
 #pragma unroll
             for (int kt = 0; kt < 4; kt++)
@@ -382,9 +392,9 @@ __global__ __launch_bounds__(256, 3) void swa_fwd_blocked_kernel(const unsigned 
             lsum[qt] = fmaf(lsum[qt], alpha, part);
         }
     }
-    float mc[2], inv[2];
+    float mc[NQ], inv[NQ];
 #pragma unroll
-    for (int qt = 0; qt < 2; qt++) {
+    for (int qt = 0; qt < NQ; qt++) {
         float sum = lsum[qt];
         sum += __shfl_xor(sum, 16, 64);
         sum += __shfl_xor(sum, 32, 64);
@@ -393,13 +403,13 @@ __global__ __launch_bounds__(256, 3) void swa_fwd_blocked_kernel(const unsigned 
     }
 
     // ---- sweep 2: weights out, O^T = V^T w^T ----
-    f32x4 o[2][4];
+    f32x4 o[NQ][4];
 #pragma unroll
-    for (int qt = 0; qt < 2; qt++)
+    for (int qt = 0; qt < NQ; qt++)
 #pragma unroll
         for (int dt = 0; dt < NDT; dt++) o[qt][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
     unsigned short *wblk = attn_w + ((size_t)(b * H + h) * s + qlo) * ws;   // row of the wave's first query
-    uint2 before[2] = {};   // PIECES: the weights of the last tile of the stage before
+    uint2 before[NQ] = {};   // PIECES: the weights of the last tile of the stage before
     __syncthreads();   // every wave is done with the buffers of sweep 1
     load_rows<HDV>(km, KS * st_lo, kreg);
     load_rows<HDV>(vm, KS * st_lo, vreg);
@@ -417,11 +427,11 @@ __global__ __launch_bounds__(256, 3) void swa_fwd_blocked_kernel(const unsigned 
             load_rows<HDV>(vm, k0 + KS, vreg);
         }
         if (k0 > qhi || k0 + KS - 1 < qlo + 1 - ws) continue;
-        f32x4 sc[4][2];
+        f32x4 sc[4][NQ];
         scores(buf, k0, sc);
-        unsigned wp[2][4][2];
+        unsigned wp[NQ][4][2];
 #pragma unroll
-        for (int qt = 0; qt < 2; qt++)
+        for (int qt = 0; qt < NQ; qt++)
 #pragma unroll
             for (int kt = 0; kt < 4; kt++) {
                 const f32x4 x = sc[kt][qt];
@@ -435,7 +445,7 @@ __global__ __launch_bounds__(256, 3) void swa_fwd_blocked_kernel(const unsigned 
             unsigned short(*W)[LDP] = Ws[wave];
             const int pr = l >> 3, pj = l & 7;   // the lane's row (of 8) and piece on the way out
 #pragma unroll
-            for (int qt = 0; qt < 2; qt++) {
+            for (int qt = 0; qt < NQ; qt++) {
                 wave_lds_order();
                 if (g >= 2) *reinterpret_cast<uint2 *>(&W[r][4 * (g - 2)]) = before[qt];
 #pragma unroll
@@ -458,7 +468,7 @@ __global__ __launch_bounds__(256, 3) void swa_fwd_blocked_kernel(const unsigned 
             }
         } else {
 #pragma unroll
-            for (int qt = 0; qt < 2; qt++) {
+            for (int qt = 0; qt < NQ; qt++) {
                 const int tq = qlo + 16 * qt + r, ls = max(tq + 1 - ws, 0);
                 unsigned short *wrow = wblk + (size_t)(16 * qt + r) * ws;
 #pragma unroll
@@ -481,29 +491,29 @@ __global__ __launch_bounds__(256, 3) void swa_fwd_blocked_kernel(const unsigned 
         }
 #pragma unroll
         for (int hf = 0; hf < 2; hf++) {
-            uint4 pb[2];
+            uint4 pb[NQ];
 #pragma unroll
-            for (int qt = 0; qt < 2; qt++)
+            for (int qt = 0; qt < NQ; qt++)
                 pb[qt] = make_uint4(wp[qt][2 * hf][0], wp[qt][2 * hf][1], wp[qt][2 * hf + 1][0], wp[qt][2 * hf + 1][1]);
 #pragma unroll
             for (int dt = 0; dt < NDT; dt++) {
                 const uint4 av = ld_tr2<LDV>(Vs[buf], 32 * hf + 4 * g, 32 * hf + 16 + 4 * g, 16 * dt);
 #pragma unroll
-                for (int qt = 0; qt < 2; qt++) o[qt][dt] = mfma32(av, pb[qt], o[qt][dt]);
+                for (int qt = 0; qt < NQ; qt++) o[qt][dt] = mfma32(av, pb[qt], o[qt][dt]);
             }
         }
     }
     // early queries: the slots behind the query's own key hold zeros
     if (qlo < ws - 1) {
         unsigned short *awb = attn_w + ((size_t)(b * H + h) * s) * ws;
-        for (int qi = 0; qi < 32; qi++) {
+        for (int qi = 0; qi < 16 * NQ; qi++) {
             const int tt = qlo + qi;
             if (tt >= s || tt >= ws - 1) break;
             for (int slot = tt + 1 + l; slot < ws; slot += 64) awb[(size_t)tt * ws + slot] = 0;
         }
     }
 #pragma unroll
-    for (int qt = 0; qt < 2; qt++) {
+    for (int qt = 0; qt < NQ; qt++) {
         const int tq = qlo + 16 * qt + r;
         if (tq < s) {
             unsigned short *ob = out + (row0 + tq) * total + hoff;
@@ -1310,21 +1320,24 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_k_blocked_kernel(const unsigne
 bool swa_forward_mfma(const uint16_t *q, const uint16_t *k, const uint16_t *v, uint16_t *out, uint16_t *attn_weights,
                       int seq_len, int num_heads, int head_dim, int window, int batch, int n_persistent, float *stats) {
     if ((head_dim != 64 && head_dim != 32) || n_persistent != 0 || window > 512 || window < 1) return false;
+    const bool few = (long long)ceil_div(seq_len, FQ) * num_heads * batch < 2LL * compute_units();
+    const dim3 grid(ceil_div(seq_len, few ? FQ / 2 : FQ), num_heads, batch);
+    const bool wide = head_dim == 64;
     if (stats) {
         KernelTimer kt("swa_fwd_stats_kernel");
-        if (head_dim == 64) hipLaunchKernelGGL(swa_fwd_stats_kernel<64>, dim3((seq_len + FQ - 1) / FQ, num_heads, batch), dim3(256), 0, stream(), q,
-                           k, v, out, reinterpret_cast<float2 *>(stats), seq_len, num_heads, window);
-        else hipLaunchKernelGGL(swa_fwd_stats_kernel<32>, dim3((seq_len + FQ - 1) / FQ, num_heads, batch), dim3(256), 0, stream(), q,
-                           k, v, out, reinterpret_cast<float2 *>(stats), seq_len, num_heads, window);
+        auto kernel = wide ? (few ? swa_fwd_stats_kernel<64, 1> : swa_fwd_stats_kernel<64, 2>)
+                           : (few ? swa_fwd_stats_kernel<32, 1> : swa_fwd_stats_kernel<32, 2>);
+        hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream(), q, k, v, out, reinterpret_cast<float2 *>(stats), seq_len, num_heads, window);
         check_launch("swa_fwd_stats_kernel");
         return true;
     }
     KernelTimer kt("swa_fwd_blocked_kernel");
     const bool pieces = window % 8 == 0 && ((uintptr_t)attn_weights & 15) == 0;   // rows of whole 16-byte pieces
-    auto kernel = head_dim == 64 ? (pieces ? swa_fwd_blocked_kernel<64, true> : swa_fwd_blocked_kernel<64, false>)
-                                 : (pieces ? swa_fwd_blocked_kernel<32, true> : swa_fwd_blocked_kernel<32, false>);
-    hipLaunchKernelGGL(kernel, dim3((seq_len + FQ - 1) / FQ, num_heads, batch), dim3(256), 0, stream(), q, k, v, out, attn_weights,
-                       seq_len, num_heads, window);
+    auto kernel = few ? (wide ? (pieces ? swa_fwd_blocked_kernel<64, true, 1> : swa_fwd_blocked_kernel<64, false, 1>)
+                              : (pieces ? swa_fwd_blocked_kernel<32, true, 1> : swa_fwd_blocked_kernel<32, false, 1>))
+                      : (wide ? (pieces ? swa_fwd_blocked_kernel<64, true, 2> : swa_fwd_blocked_kernel<64, false, 2>)
+                              : (pieces ? swa_fwd_blocked_kernel<32, true, 2> : swa_fwd_blocked_kernel<32, false, 2>));
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream(), q, k, v, out, attn_weights, seq_len, num_heads, window);
     check_launch("swa_fwd_blocked_kernel");
     return true;
 }

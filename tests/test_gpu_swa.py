@@ -127,6 +127,35 @@ def test_weights_stored_in_pieces_and_in_fours(s, ws, hd):
         assert np.array_equal(x, y)
 
 
+@pytest.mark.parametrize("hd", [64, 32])
+@pytest.mark.parametrize("s,ws", [(129, 64), (300, 72), (300, 101), (515, 512)])
+def test_forward_with_one_query_tile_a_wave_and_with_two(s, ws, hd):
+    """A call that fills the chip takes 32 queries a wave, its batch elements by themselves 16: bit for bit the same, weights stored
+    in pieces, in fours, or not at all."""
+    B, H = 64, 4
+    q, k, v, _ = _case(B, s, H, hd, 950 + s + ws + hd)
+    tq, tk, tv = _u16(q), _u16(k), _u16(v)
+
+    def stored(x, at):
+        n = len(x[0])
+        out = torch.zeros(n, s, H * hd, dtype=torch.uint16, device="cuda")
+        room = torch.full((n * H * s * ws + 16,), 0x7fc0, dtype=torch.uint16, device="cuda")
+        D.call("swa_forward_f32_cuda", *x, out, room[at:], s, H, hd, ws, n, 0)
+        return out, room[at:at + n * H * s * ws].clone().view(n, H, s, ws)
+
+    def statistics(x):
+        n = len(x[0])
+        out, st = torch.zeros(n, s, H * hd, dtype=torch.uint16, device="cuda"), zeros(n, H, s, 2)
+        D.call("swa_forward_lse_bf16_rocm", *x, out, st, s, H, hd, ws, n)
+        return out, st
+
+    for run in (lambda x: stored(x, 8), lambda x: stored(x, 10), statistics):
+        whole = run((tq, tk, tv))
+        for i in (0, 13, B - 1):
+            for a, b in zip(whole, run((tq[i:i + 1], tk[i:i + 1], tv[i:i + 1]))):
+                assert np.array_equal(a[i:i + 1].cpu().numpy(), b.cpu().numpy())
+
+
 @pytest.mark.parametrize("s,ws,hd", [(1, 4, 64), (31, 32, 32), (33, 2, 64), (128, 128, 32), (161, 64, 64), (200, 101, 32),
                                      (353, 130, 64), (600, 512, 64), (600, 511, 32)])
 def test_backward_in_blocks_of_32_rows_and_of_128(s, ws, hd):
