@@ -127,8 +127,7 @@ struct EbBatch {
 // mode 0: dst += src (accumulate); 1: dst -= lr * src, then src <- 0 (apply_and_reset);
 // 2: dst <- 0 (reset); 3: dst <- src (seed)
 __global__ void eb_map_kernel(EbBatch b, int mode, float lr) {
-    int t = 0;
-    while (t + 1 < b.count && (int)blockIdx.x >= b.blk_begin[t + 1]) t++;
+    const int t = batch_entry(b.blk_begin, b.count, blockIdx.x);
     const int nblk = b.blk_begin[t + 1] - b.blk_begin[t], local = blockIdx.x - b.blk_begin[t];
     float *d = b.dst[t];
     float *sp = b.src[t];

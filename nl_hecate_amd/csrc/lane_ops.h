@@ -165,6 +165,13 @@ __device__ __forceinline__ void wave_reduce_scatter(float (&v)[N], float (&out)[
     for (int n = 0; n < N / 4; n++) out[n] = group_allreduce<16>(out[n]);
 }
 
+// Which entry of a batch block blk belongs to: begin[0 .. count), ascending, at most 64; blk is the same for the whole wave and all
+// of its lanes are here.  One load for all entries; a walk over them was a chain of scalar loads.
+__device__ __forceinline__ int batch_entry(const int *begin, int count, int blk) {
+    const int l = threadIdx.x & 63;
+    return __builtin_popcountll(__builtin_amdgcn_ballot_w64(blk >= begin[l < count ? l : 0] && l > 0 && l < count));
+}
+
 __device__ __forceinline__ float dot4(const float4 &a, const float4 &b) {
     return a.x * b.x + a.y * b.y + a.z * b.z + a.w * b.w;
 }

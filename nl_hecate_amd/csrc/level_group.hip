@@ -280,8 +280,7 @@ __global__ __launch_bounds__(kThr) void level_heads_repeat_kernel(const float4 *
 constexpr int kMaxSaxpy = 64, kSaxpyPer = 4096;   // elements per workgroup
 struct SaxpyArgs { const float *x[kMaxSaxpy]; float *y[kMaxSaxpy]; int n[kMaxSaxpy], first[kMaxSaxpy + 1]; int count; float alpha; };
 __global__ __launch_bounds__(kThr) void saxpy_multi_kernel(SaxpyArgs a) {
-    int t = 0;
-    while (t + 1 < a.count && (int)blockIdx.x >= a.first[t + 1]) t++;
+    const int t = batch_entry(a.first, a.count, blockIdx.x);
     const float *x = a.x[t];
     float *y = a.y[t];
     const int i0 = ((int)blockIdx.x - a.first[t]) * kSaxpyPer, i1 = min(a.n[t], i0 + kSaxpyPer);

@@ -105,8 +105,7 @@ struct AdamwBatch {
 
 template <bool SCALE>
 __global__ void adamw_multi_kernel(AdamwBatch b, AdamwHyper h, const float *scale_ptr) {
-    int t = 0;
-    while (t + 1 < b.count && (int)blockIdx.x >= b.blk_begin[t + 1]) t++;
+    const int t = batch_entry(b.blk_begin, b.count, blockIdx.x);
     const int nblk = b.blk_begin[t + 1] - b.blk_begin[t];
     const int lb = blockIdx.x - b.blk_begin[t];
     adamw_span<SCALE>(b.w[t], b.g[t], b.m[t], b.v[t], b.n[t], lb * blockDim.x + threadIdx.x, nblk * blockDim.x, h,
@@ -201,8 +200,7 @@ __global__ void norm_sq_multi_kernel(PtrBatch b, float *__restrict__ partial) {
     const int nwaves = (gridDim.x * blockDim.x) >> 6;
     const int total = b.blk_begin[b.count];
     for (int blk = wave; blk < total; blk += nwaves) {
-        int t = 0;
-        while (t + 1 < b.count && blk >= b.blk_begin[t + 1]) t++;
+        const int t = batch_entry(b.blk_begin, b.count, blk);
         const float *a = b.p[t];
         const int n = b.n[t], base = (blk - b.blk_begin[t]) * kNormBlock;
         float s = 0.f;
@@ -228,8 +226,7 @@ __global__ void norm_sq_multi_kernel(PtrBatch b, float *__restrict__ partial) {
 __global__ void scale_multi_kernel(PtrBatch b, const float *scale_ptr) {
     const float scale = *scale_ptr;
     if (scale >= 1.0f) return;
-    int t = 0;
-    while (t + 1 < b.count && (int)blockIdx.x >= b.blk_begin[t + 1]) t++;
+    const int t = batch_entry(b.blk_begin, b.count, blockIdx.x);
     const int nblk = b.blk_begin[t + 1] - b.blk_begin[t];
     float *g = b.p[t];
     for (int i = (blockIdx.x - b.blk_begin[t]) * blockDim.x + threadIdx.x; i < b.n[t]; i += nblk * blockDim.x)
