@@ -318,43 +318,37 @@ __global__ __launch_bounds__(kThr) void cw_out_fwd_kernel(const TIn *__restrict_
 //   T_a, T_b as in the forward (the chunk map is right-multiplication by symmetric matrices)
 //   C_1 = G0  = (a.dY)^T Q + dE_loc^T K,   dE_loc[j] = -theta_j sum_{t>=j} c[t,j] (q_t.k_j) dy_t
 //   C_2 = GS0 = (beta.dY)^T Q
-template <class TIn>
-__global__ __launch_bounds__(kThr) void cw_local_bwd_kernel(const TIn *__restrict__ k, const TIn *__restrict__ q,
+// A workgroup per chunk.  PAIR: two to a compute unit (four matrices of LDS, 128 registers), so that one's loads run under the
+// other's products, taken where there are more chunks than compute units; a chunk by itself is faster with the registers.
+// Against one persistent workgroup a compute unit that asked for its next chunk ahead, forward and backward of the rule, us: 2048
+// chunks 617 -> 608, 768 296 -> 293 (this kernel 42 -> 38), 8192 2141 -> 2102; as pairs 40 and 252 chunks lose 2.
+template <class TIn, bool PAIR>
+__global__ __launch_bounds__(kThr, PAIR ? 4 : 2) void cw_local_bwd_kernel(const TIn *__restrict__ k, const TIn *__restrict__ q,
                                                             const float *__restrict__ d_y,
                                                             const float *__restrict__ alpha,
                                                             const float *__restrict__ theta,
                                                             const float *__restrict__ eta, float *__restrict__ loc,
                                                             float *__restrict__ locs, int s, int C, int nc,
-                                                            int has_s, int ntask) {
+                                                            int has_s) {
     extern __shared__ float smem[];
-    float *Ks = smem, *Qs = Ks + MAT, *Ds = Qs + MAT, *Cc = Ds + MAT, *El = Cc + MAT;
+    float *Ks = smem, *Qs = Ks + MAT, *Ds = Qs + MAT, *Cc = Ds + MAT, *El = PAIR ? Cc : Cc + MAT;   // a pair: E in the place of what it is formed from
     __shared__ Coef cf;
     __shared__ float wM[CW], wS[CW];
     NLH_STRIP_ORIGIN();
+    const int task = blockIdx.x, chain = task / nc, ci = task % nc, t0 = ci * C, L = min(C, s - t0);
+    const size_t tok = (size_t)chain * s + t0;
     Tile<TIn> tk, tq;
     Tile<float> td;
-    Gates gt;
-    auto fetch_task = [&](int task) {
-        const int chain = task / nc, ci = task % nc, t0 = ci * C, L = min(C, s - t0);
-        const size_t tok = (size_t)chain * s + t0;
-        gt = fetch_gates(alpha + tok, theta + tok, eta + tok, L, has_s != 0);
-        fetch(tk, k + tok * HD, L);
-        fetch(tq, q + tok * HD, L);
-        fetch(td, d_y + tok * HD, L);
-    };
-    // contiguous task range per workgroup: consecutive chunks of a chain share pages and cache lines
-    const int per = (ntask + (int)gridDim.x - 1) / (int)gridDim.x, task_lo = blockIdx.x * per,
-              task_hi = min(ntask, task_lo + per);
-    if (task_lo < task_hi) fetch_task(task_lo);
-    for (int task = task_lo; task < task_hi; task++) {
-    const int chain = task / nc, ci = task % nc, t0 = ci * C, L = min(C, s - t0);
+    const Gates gt = fetch_gates(alpha + tok, theta + tok, eta + tok, L, has_s != 0);
+    fetch(tk, k + tok * HD, L);
+    fetch(tq, q + tok * HD, L);
+    fetch(td, d_y + tok * HD, L);
     load_gates(cf, gt);
     coefficients(cf, gt, L, Cc);
     commit(Ks, tk);
     commit(Qs, tq);
     commit(Ds, td);
     __syncthreads();
-    if (task + 1 < task_hi) fetch_task(task + 1);
     if (threadIdx.x < CW) {
         wM[threadIdx.x] = -cf.th[threadIdx.x] * cf.cl[threadIdx.x];
         wS[threadIdx.x] = -cf.th[threadIdx.x] * cf.bl[threadIdx.x];
@@ -387,6 +381,7 @@ __global__ __launch_bounds__(kThr) void cw_local_bwd_kernel(const TIn *__restric
         Strip e = zero_strip();
         mma(e, [&](int m, int kk) { return Cc[kk * LDM + m0 + m]; },
             [&](int kk, int n) { return Ds[kk * LDM + n0 + n]; });
+        if constexpr (PAIR) __syncthreads();
         for_c(e, [&](int r, int c, float &x) { El[(m0 + r) * LDM + n0 + c] = -cf.th[m0 + r] * x; });
     }
     __syncthreads();
@@ -402,10 +397,8 @@ __global__ __launch_bounds__(kThr) void cw_local_bwd_kernel(const TIn *__restric
         store_acc_tile(out + (size_t)2 * HD * HD, g0.t[t], m0 / 16, n0 / 16 + t, threadIdx.x & 63);
         store_acc_tile(out + (size_t)3 * HD * HD, gs.t[t], m0 / 16, n0 / 16 + t, threadIdx.x & 63);
     }
-    __syncthreads();   // LDS is rewritten by the next task
-    }
 }
-constexpr size_t kLocalBwdLds = 5 * MAT * sizeof(float);
+constexpr size_t kLocalBwdLds = 5 * MAT * sizeof(float), kLocalBwdPairLds = 4 * MAT * sizeof(float);
 
 // ── backward, main per-chunk pass: dQ, dK, dV, dtheta; exports for the gate pass ──
 //   pvec [chain][token][4] = p0, ps, -theta g1, -theta g2   xs [chain][chunk][j][t] = -theta_j (dy_t.e_j)(q_t.k_j)
@@ -739,8 +732,10 @@ bool backward_mm(const char *fn, const TIn *k, const TIn *v, const TIn *q, const
     if (es.failed()) return true;
     static bool attr_set = false;
     if (!attr_set) {
-        set_lds(cw_local_bwd_kernel<float>, kLocalBwdLds);
-        set_lds(cw_local_bwd_kernel<uint16_t>, kLocalBwdLds);
+        set_lds(cw_local_bwd_kernel<float, false>, kLocalBwdLds);
+        set_lds(cw_local_bwd_kernel<uint16_t, false>, kLocalBwdLds);
+        set_lds(cw_local_bwd_kernel<float, true>, kLocalBwdPairLds);
+        set_lds(cw_local_bwd_kernel<uint16_t, true>, kLocalBwdPairLds);
         set_lds(cw_grads_bwd_kernel<float, false>, kGradsBwdLds);
         set_lds(cw_grads_bwd_kernel<float, true>, kGradsBwdLds);
         set_lds(cw_grads_bwd_kernel<uint16_t, false>, kGradsBwdLds);
@@ -760,9 +755,10 @@ bool backward_mm(const char *fn, const TIn *k, const TIn *v, const TIn *q, const
                              scal, tab_b, vecs, seq_len, batch, chunk_size, has_s,
                              persistent_grid(batch * nc), dy_rows, out16, guard ? &tracks : nullptr);
     } else {
-        hipLaunchKernelGGL((cw_local_bwd_kernel<TIn>), dim3(persistent_grid(batch * nc)), dim3(kThr), kLocalBwdLds,
-                           stream(), k, q, d_y, alpha, theta, eta, sc.loc, sc.locs, seq_len, chunk_size, nc,
-                           (int)has_s, batch * nc);
+        const bool pair = batch * nc > compute_units();
+        hipLaunchKernelGGL((pair ? cw_local_bwd_kernel<TIn, true> : cw_local_bwd_kernel<TIn, false>), dim3(batch * nc), dim3(kThr),
+                           pair ? kLocalBwdPairLds : kLocalBwdLds, stream(), k, q, d_y, alpha, theta, eta, sc.loc, sc.locs, seq_len, chunk_size, nc,
+                           (int)has_s);
         check_launch("cw_local_bwd_kernel");
         hipLaunchKernelGGL((has_s ? cw_scan_kernel<false, true> : cw_scan_kernel<false, false>), dim3(batch * 4), dim3(256), 0, stream(),
                            nullptr, nullptr, sc.loc, sc.locs, dm_states, ds_states, nc, batch);
