@@ -8,7 +8,8 @@
 // elements per lane: lane (r = l % 16, g = l / 16) supplies row r, contraction
 // elements 8 g .. 8 g + 7 of a 32-wide step.
 //
-// Every kernel works in blocks: one workgroup per 128 queries (keys in the key passes), one wave per 32, stages
+// Every kernel works in blocks: one workgroup per 128 queries (keys in the key passes), one wave per 32, or, where those leave the
+// chip idle, 64 with 16 a wave (forward) or 32 in all (backward), and stages
 // of 64 keys (queries) whose rows are staged in LDS exactly as they arrive.  A 16x16 result tile leaves rows
 // 4 g + i in a lane; where two such tiles become an operand again with their rows as contraction index (the
 // weights in O^T = V^T w^T, dS in d_q^T = K^T dS^T, ..), the matching operand is read from the row-major stage
@@ -82,6 +83,20 @@ __device__ __forceinline__ void split8(f32x4 a, f32x4 b, uint4 &hi, uint4 &lo) {
     split2(b[0], b[1], hi.z, lo.z);
     split2(b[2], b[3], hi.w, lo.w);
 }
+// x = w dw of four elements, the weights w in two bf16 pairs, and x = hi + lo with lo from the product before it is rounded.  Explicit
+// fma here and in D's terms: which of these the compiler fuses by itself depends on the code around them, and so would bits.
+__device__ __forceinline__ void split_products(unsigned w01, unsigned w23, f32x4 dw, f32x4 &x, uint2 &hi, uint2 &lo) {
+    const float w[4] = {bf_lo(w01), bf_hi(w01), bf_lo(w23), bf_hi(w23)};
+#pragma unroll
+    for (int i = 0; i < 4; i++) x[i] = w[i] * dw[i];
+    hi = make_uint2(pack2(x[0], x[1]), pack2(x[2], x[3]));
+    lo = make_uint2(pack2(fmaf(w[0], dw[0], -bf_lo(hi.x)), fmaf(w[1], dw[1], -bf_hi(hi.x))),
+                    pack2(fmaf(w[2], dw[2], -bf_lo(hi.y)), fmaf(w[3], dw[3], -bf_hi(hi.y))));
+}
+// their sum
+__device__ __forceinline__ float sum_products(unsigned w01, unsigned w23, f32x4 dw, f32x4 x) {
+    return fmaf(bf_lo(w01), dw[0], x[1]) + fmaf(bf_lo(w23), dw[2], x[3]);
+}
 // Workgroup -> (block of the sequence, head * batch) with all blocks of one head on one XCD.
 // Workgroups go to the 8 XCDs round robin in linear order, and each XCD has its own L2; blocks
 // of one head share K and V rows, so they are given linear ids that are equal modulo 8.
@@ -116,7 +131,8 @@ __device__ __forceinline__ void load_rows(const StageSrc &m, int first, uint4 (&
     }
 }
 // operand of a 32-wide step: row r of the tile at row0, contraction elements 32 ks + 8 g .. + 7
-__device__ __forceinline__ uint4 ld_op(unsigned short (*T)[LDH], int row0, int ks) {
+template <int LD>
+__device__ __forceinline__ uint4 ld_op(unsigned short (*T)[LD], int row0, int ks) {
     const int l = threadIdx.x & 63;
     return *reinterpret_cast<const uint4 *>(&T[row0 + (l & 15)][32 * ks + 8 * (l >> 4)]);
 }
@@ -526,56 +542,26 @@ __global__ __launch_bounds__(256, 3) void swa_fwd_blocked_kernel(const unsigned 
 }
 
 // The backward passes of a call that leaves the chip idle (SPLIT): bound by one wave's chain of stages, so a workgroup has 32
-// queries (keys) instead of 128, its four waves share out the window instead of the rows (two stages at a time, half a stage
-// each), and their sums are joined at the end.  What a workgroup stages then serves a quarter of the rows: taken while
-// the four times as many workgroups still fit the chip at once, two a compute unit.  Both passes, contract / statistics, us
-// before and after, head size 64, window 512: 32 blocks of 128 rows 46 -> 21 / 60 -> 28, 112 blocks 58 -> 35 / 73 -> 42;
-// where they do not fit, 192 blocks 63 -> 62 or 75, 256 blocks (window 256) 46 -> 52, 512 blocks 92 -> 131.
+// queries (keys) instead of 128.  Two stages at a time, its four waves form the weights and dS of half a stage each, pass them
+// on through LDS (HalfStage), and add the products of both stages up in the order of the keys (queries), each wave for
+// a quarter of the result's tiles.  Every sum then has the order that it has in a block of 128, so that a sequence's gradients
+// are the same bits alone and in any batch.
+// What a workgroup stages serves a quarter of the rows: taken while the four times as many workgroups still fit the chip at
+// once, two a compute unit.  Both passes, contract / statistics, us as blocks of 128 and so, head size 64, window 512: 32 blocks of 128
+// rows 46 -> 23 / 60 -> 28, 112 blocks 58 -> 38 / 73 -> 43 (21 / 27.5 and 35 / 41 with every wave's sums of its own half stages,
+// joined at the end); where they do not fit, with joined sums, 192 blocks 63 -> 62 or 75, 256 blocks (window 256) 46 -> 52, 512 blocks 92 -> 131.
 constexpr int SQ = 32;     // queries (keys) per workgroup of these
-// tile (t, dt) of the joined sums stays with one wave
+constexpr int LDQ = 72;  // row stride of the key passes' stages there: two workgroups fit a compute unit
+// Operands of the products over half a stage, on their way from the wave that forms them: [tile of rows][operand][lane]
+template <int N>
+using HalfStage = uint4[2][N][64];
+// The tiles of the result that a wave adds up: NT of rows from tile0 on, ND of dims from dt0 on
 template <int NDT, bool SPLIT>
-__device__ __forceinline__ bool own_tile(int t, int dt, int wave) { return !SPLIT || wave == 2 * t + dt / (NDT / 2); }
-// x, y: sums of the four waves over their own keys; afterwards a wave has the whole sums of its own tiles.  buf: the stages,
-// room for 16 KB a wave.
-template <int NDT>
-__device__ __forceinline__ void join_waves(f32x4 (&x)[2][4], f32x4 (&y)[2][4], float *buf, int wave, int l) {
-    f32x4 *m = reinterpret_cast<f32x4 *>(buf) + l;
-    constexpr int N = NDT / 2;   // tiles of x (and of y) that a wave ends up with
-    __syncthreads();             // the stages are read
-#pragma unroll
-    for (int o = 0; o < 4; o++) {
-        if (o == wave) continue;
-        const int from = (wave - o - 1) & 3;   // 0 .. 2
-#pragma unroll
-        for (int e = 0; e < N; e++) {
-            m[((o * 3 + from) * 2 * N + 2 * e) * 64] = x[o >> 1][(o & 1) * N + e];
-            m[((o * 3 + from) * 2 * N + 2 * e + 1) * 64] = y[o >> 1][(o & 1) * N + e];
-        }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int o = 0; o < 4; o++) {
-        if (o != wave) continue;
-#pragma unroll
-        for (int e = 0; e < N; e++) {
-            f32x4 &a = x[o >> 1][(o & 1) * N + e], &c = y[o >> 1][(o & 1) * N + e];
-            const f32x4 *p = m + (o * 3 * 2 * N + 2 * e) * 64, *q = p + 64;
-            a = (a + p[0]) + (p[2 * N * 64] + p[4 * N * 64]);
-            c = (c + q[0]) + (q[2 * N * 64] + q[4 * N * 64]);
-        }
-    }
-}
-__device__ __forceinline__ void join_waves(float (&x)[2], float *buf, int wave, int l) {
-    __syncthreads();
-#pragma unroll
-    for (int e = 0; e < 2; e++) buf[(e * 4 + wave) * 64 + l] = x[e];
-    __syncthreads();
-#pragma unroll
-    for (int e = 0; e < 2; e++) {
-        const float *p = buf + e * 256 + l;
-        x[e] = (p[0] + p[64]) + (p[128] + p[192]);
-    }
-}
+struct OwnTiles {
+    static constexpr int NT = SPLIT ? 1 : 2, ND = SPLIT ? NDT / 2 : NDT;
+    int tile0, dt0;
+    __device__ __forceinline__ explicit OwnTiles(int wave) : tile0(SPLIT ? wave >> 1 : 0), dt0(SPLIT ? (wave & 1) * ND : 0) {}
+};
 
 // Query pass on statistics, in key blocks like swa_fwd_stats_kernel (one workgroup per 128 queries, one wave per
 // 32), in ONE sweep over the window.  dS = w (dW - D) needs D_t = sum_j w dW of the whole window, so the sweep
@@ -594,7 +580,9 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_q_stats_kernel(const unsigned 
                                                                  const float *__restrict__ d_out,
                                                                  float *__restrict__ d_q, float *__restrict__ dvec,
                                                                  int s, int H, int ws, Out16 o16) {
-    __shared__ __align__(16) unsigned short KV[SPLIT ? 5 : 4][KS][LDH];   // two stages [key][dim] of K, then of V
+    __shared__ __align__(16) unsigned short KV[4][KS][LDH];   // two stages [key][dim] of K, then of V
+    __shared__ HalfStage<3> Px[SPLIT ? 4 : 1];                // SPLIT: w dW hi and lo and w of a wave's half stage,
+    __shared__ float Dx[SPLIT ? 4 : 1][2][2][64];             // and its terms of D
     unsigned short (*const Ks)[KS][LDH] = KV, (*const Vs)[KS][LDH] = KV + 2;
     const int tid = threadIdx.x, wave = tid >> 6, l = tid & 63, r = l & 15, g = l >> 4;
     const BlockCoord bc = xcd_block_coord(H);
@@ -609,7 +597,7 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_q_stats_kernel(const unsigned 
     const float c2 = kInvSqrt * 1.44269504088896340736f, scale = kInvSqrt;
 
     uint4 qf[2][2], doh[2][2], dol[2][2];
-    float mc[2], inv[2], dpart[2] = {0.f, 0.f};
+    float mc[2], inv[2];
 #pragma unroll
     for (int qt = 0; qt < 2; qt++) {
         const int tq = qlo + 16 * qt + r;
@@ -632,11 +620,30 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_q_stats_kernel(const unsigned 
             inv[qt] = st2.y;
         }
     }
-    f32x4 aq[2][4], bq[2][4];
+    using Own = OwnTiles<NDT, SPLIT>;
+    const Own own(wave);
+    f32x4 aq[Own::NT][Own::ND], bq[Own::NT][Own::ND];
+    float dpart[Own::NT];
 #pragma unroll
-    for (int qt = 0; qt < 2; qt++)
+    for (int t = 0; t < Own::NT; t++) {
+        dpart[t] = 0.f;
 #pragma unroll
-        for (int dt = 0; dt < NDT; dt++) { aq[qt][dt] = f32x4{0.f, 0.f, 0.f, 0.f}; bq[qt][dt] = f32x4{0.f, 0.f, 0.f, 0.f}; }
+        for (int dt = 0; dt < Own::ND; dt++) { aq[t][dt] = f32x4{0.f, 0.f, 0.f, 0.f}; bq[t][dt] = f32x4{0.f, 0.f, 0.f, 0.f}; }
+    }
+    // half hf of a stage added to the sums of this wave's tiles
+    auto add = [&](unsigned short(*K)[LDH], int hf, const uint4(&xh)[Own::NT], const uint4(&xl)[Own::NT], const uint4(&wb)[Own::NT])
+                   __attribute__((always_inline)) {
+#pragma unroll
+        for (int dt = 0; dt < Own::ND; dt++) {
+            const uint4 a = ld_tr2<LDH>(K, 32 * hf + 4 * g, 32 * hf + 16 + 4 * g, 16 * (own.dt0 + dt));
+#pragma unroll
+            for (int t = 0; t < Own::NT; t++) {
+                aq[t][dt] = mfma32(a, xh[t], aq[t][dt]);
+                aq[t][dt] = mfma32(a, xl[t], aq[t][dt]);
+                bq[t][dt] = mfma32(a, wb[t], bq[t][dt]);
+            }
+        }
+    };
 
     uint4 kreg[SPLIT ? 2 : 1][2], vreg[SPLIT ? 2 : 1][2];
     auto fetch_stages = [&](int first) {
@@ -649,7 +656,7 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_q_stats_kernel(const unsigned 
     fetch_stages(KS * st_lo);
     for (int st = st_lo; st <= st_hi; st += SPLIT ? 2 : 1) {
         const int buf = SPLIT ? wave >> 1 : (st - st_lo) & 1, k0 = KS * (SPLIT ? st + buf : st);
-        if (SPLIT && st > st_lo) __syncthreads();   // both stages are read
+        if (SPLIT && st > st_lo) __syncthreads();   // the stages and half stages before are read
 #pragma unroll
         for (int p = 0; p < (SPLIT ? 2 : 1); p++)
 #pragma unroll
@@ -660,7 +667,7 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_q_stats_kernel(const unsigned 
             }
         __syncthreads();
         if (st + (SPLIT ? 1 : 0) < st_hi) fetch_stages(KS * (st + (SPLIT ? 2 : 1)));
-        if (k0 > qhi || k0 + KS - 1 < qlo + 1 - ws) continue;
+        if (!SPLIT && (k0 > qhi || k0 + KS - 1 < qlo + 1 - ws)) continue;   // SPLIT: a stage of no key of these queries is not added
         const bool full = k0 + KS - 1 <= qlo && k0 >= qhi + 1 - ws && qhi < s;
 #pragma unroll
         for (int half = 0; half < (SPLIT ? 1 : 2); half++) {
@@ -668,8 +675,8 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_q_stats_kernel(const unsigned 
             uint4 xh[2], xl[2], wb[2];
 #pragma unroll
             for (int qt = 0; qt < 2; qt++) {
-                f32x4 x[2];
                 unsigned wp[2][2];
+                uint2 hi[2], lo[2];
 #pragma unroll
                 for (int c = 0; c < 2; c++) {
                     const int kt = 2 * hf + c;
@@ -690,55 +697,59 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_q_stats_kernel(const unsigned 
                     }
                     wp[c][0] = pack2(w[0], w[1]);   // as the weight tensor holds them
                     wp[c][1] = pack2(w[2], w[3]);
-                    x[c][0] = bf_lo(wp[c][0]) * dw[0];
-                    x[c][1] = bf_hi(wp[c][0]) * dw[1];
-                    x[c][2] = bf_lo(wp[c][1]) * dw[2];
-                    x[c][3] = bf_hi(wp[c][1]) * dw[3];
-                    dpart[qt] += (x[c][0] + x[c][1]) + (x[c][2] + x[c][3]);
+                    f32x4 x;
+                    split_products(wp[c][0], wp[c][1], dw, x, hi[c], lo[c]);
+                    const float d4 = sum_products(wp[c][0], wp[c][1], dw, x);
+                    if constexpr (SPLIT) Dx[wave][qt][c][l] = d4;
+                    else dpart[qt] += d4;
                 }
-                split8(x[0], x[1], xh[qt], xl[qt]);
+                xh[qt] = make_uint4(hi[0].x, hi[0].y, hi[1].x, hi[1].y);
+                xl[qt] = make_uint4(lo[0].x, lo[0].y, lo[1].x, lo[1].y);
                 wb[qt] = make_uint4(wp[0][0], wp[0][1], wp[1][0], wp[1][1]);
             }
+            if constexpr (SPLIT) {
 #pragma unroll
-            for (int dt = 0; dt < NDT; dt++) {
-                const uint4 a = ld_tr2<LDH>(Ks[buf], 32 * hf + 4 * g, 32 * hf + 16 + 4 * g, 16 * dt);
+                for (int qt = 0; qt < 2; qt++) { Px[wave][qt][0][l] = xh[qt]; Px[wave][qt][1][l] = xl[qt]; Px[wave][qt][2][l] = wb[qt]; }
+            } else {
+                add(Ks[buf], hf, xh, xl, wb);
+            }
+        }
+        if constexpr (SPLIT) {
+            __syncthreads();   // the four half stages are there
 #pragma unroll
-                for (int qt = 0; qt < 2; qt++) {
-                    aq[qt][dt] = mfma32(a, xh[qt], aq[qt][dt]);
-                    aq[qt][dt] = mfma32(a, xl[qt], aq[qt][dt]);
-                    bq[qt][dt] = mfma32(a, wb[qt], bq[qt][dt]);
+            for (int p = 0; p < 2; p++) {
+                if (st + p > st_hi) break;
+#pragma unroll
+                for (int hf = 0; hf < 2; hf++) {
+                    const int h = 2 * p + hf;
+                    const auto &x = Px[h][own.tile0];
+                    dpart[0] += Dx[h][own.tile0][0][l];
+                    dpart[0] += Dx[h][own.tile0][1][l];
+                    add(Ks[p], hf, {x[0][l]}, {x[1][l]}, {x[2][l]});
                 }
             }
         }
     }
-    if constexpr (SPLIT) {
-        float *buf = reinterpret_cast<float *>(&Ks[0][0][0]);
-        join_waves<NDT>(aq, bq, buf, wave, l);
-        join_waves(dpart, buf, wave, l);
-    }
 #pragma unroll
-    for (int qt = 0; qt < 2; qt++) {
-        const int tq = qlo + 16 * qt + r;
-        if (SPLIT && qt != wave >> 1) continue;
-        float dsum = dpart[qt];
+    for (int t = 0; t < Own::NT; t++) {
+        const int tq = qlo + 16 * (own.tile0 + t) + r;
+        float dsum = dpart[t];
         dsum += __shfl_xor(dsum, 16, 64);
         dsum += __shfl_xor(dsum, 32, 64);
         if (tq < s) {
-            if (g == 0 && !(SPLIT && (wave & 1))) dvec[(size_t)(b * H + h) * s + tq] = dsum;
+            if (g == 0 && own.dt0 == 0) dvec[(size_t)(b * H + h) * s + tq] = dsum;
             if (OUT16) {
                 unsigned short *ob = o16.q + (row0 + tq) * o16.ld + hoff;
 #pragma unroll
-                for (int dt = 0; dt < NDT; dt++) {
-                    if (!own_tile<NDT, SPLIT>(qt, dt, wave)) continue;
-                    const f32x4 x = (aq[qt][dt] - dsum * bq[qt][dt]) * scale;
-                    *reinterpret_cast<uint2 *>(ob + 16 * dt + 4 * g) = make_uint2(pack2(x[0], x[1]), pack2(x[2], x[3]));
+                for (int dt = 0; dt < Own::ND; dt++) {
+                    const f32x4 x = (aq[t][dt] - dsum * bq[t][dt]) * scale;
+                    *reinterpret_cast<uint2 *>(ob + 16 * (own.dt0 + dt) + 4 * g) = make_uint2(pack2(x[0], x[1]), pack2(x[2], x[3]));
                 }
             } else {
                 float *ob = d_q + (row0 + tq) * total + hoff;
 #pragma unroll
-                for (int dt = 0; dt < NDT; dt++)
-                    if (own_tile<NDT, SPLIT>(qt, dt, wave))
-                        *reinterpret_cast<f32x4 *>(ob + 16 * dt + 4 * g) = (aq[qt][dt] - dsum * bq[qt][dt]) * scale;
+                for (int dt = 0; dt < Own::ND; dt++)
+                    *reinterpret_cast<f32x4 *>(ob + 16 * (own.dt0 + dt) + 4 * g) = (aq[t][dt] - dsum * bq[t][dt]) * scale;
             }
         }
     }
@@ -761,7 +772,9 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_q_blocked_kernel(const unsigne
                                                                    const float *__restrict__ d_out,
                                                                    float *__restrict__ d_q, float *__restrict__ dvec,
                                                                    int s, int H, int ws) {
-    __shared__ __align__(16) unsigned short KV[SPLIT ? 5 : 4][KS][LDH];   // two stages [key][dim] of K, then of V
+    __shared__ __align__(16) unsigned short KV[4][KS][LDH];   // two stages [key][dim] of K, then of V
+    __shared__ HalfStage<3> Px[SPLIT ? 4 : 1];                // SPLIT: w dW hi and lo and w of a wave's half stage,
+    __shared__ float Dx[SPLIT ? 4 : 1][2][2][64];             // and its terms of D
     unsigned short (*const Ks)[KS][LDH] = KV, (*const Vs)[KS][LDH] = KV + 2;
     const int tid = threadIdx.x, wave = tid >> 6, l = tid & 63, r = l & 15, g = l >> 4;
     const BlockCoord bc = xcd_block_coord(H);
@@ -778,7 +791,6 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_q_blocked_kernel(const unsigne
     uint4 doh[2][2], dol[2][2];
     const unsigned short *wrow[2];
     int lsq[2], tqs[2];
-    float dpart[2] = {0.f, 0.f};
 #pragma unroll
     for (int qt = 0; qt < 2; qt++) {
         const int tq = qlo + 16 * qt + r;
@@ -796,11 +808,30 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_q_blocked_kernel(const unsigne
             split8(x0, x1, doh[qt][ks], dol[qt][ks]);
         }
     }
-    f32x4 aq[2][4], bq[2][4];
+    using Own = OwnTiles<NDT, SPLIT>;
+    const Own own(wave);
+    f32x4 aq[Own::NT][Own::ND], bq[Own::NT][Own::ND];
+    float dpart[Own::NT];
 #pragma unroll
-    for (int qt = 0; qt < 2; qt++)
+    for (int t = 0; t < Own::NT; t++) {
+        dpart[t] = 0.f;
 #pragma unroll
-        for (int dt = 0; dt < NDT; dt++) { aq[qt][dt] = f32x4{0.f, 0.f, 0.f, 0.f}; bq[qt][dt] = f32x4{0.f, 0.f, 0.f, 0.f}; }
+        for (int dt = 0; dt < Own::ND; dt++) { aq[t][dt] = f32x4{0.f, 0.f, 0.f, 0.f}; bq[t][dt] = f32x4{0.f, 0.f, 0.f, 0.f}; }
+    }
+    // half hf of a stage added to the sums of this wave's tiles
+    auto add = [&](unsigned short(*K)[LDH], int hf, const uint4(&xh)[Own::NT], const uint4(&xl)[Own::NT], const uint4(&wb)[Own::NT])
+                   __attribute__((always_inline)) {
+#pragma unroll
+        for (int dt = 0; dt < Own::ND; dt++) {
+            const uint4 a = ld_tr2<LDH>(K, 32 * hf + 4 * g, 32 * hf + 16 + 4 * g, 16 * (own.dt0 + dt));
+#pragma unroll
+            for (int t = 0; t < Own::NT; t++) {
+                aq[t][dt] = mfma32(a, xh[t], aq[t][dt]);
+                aq[t][dt] = mfma32(a, xl[t], aq[t][dt]);
+                bq[t][dt] = mfma32(a, wb[t], bq[t][dt]);
+            }
+        }
+    };
 
     // Weights of a stage for this lane: wreg[hf][qt] = keys k0 + 32 hf + 8 g .. + 7 of query qt (stage_row).  At the window's ends
     // a piece is read whole as well, out of the rows next to it, and what is not the query's own is taken off where the piece
@@ -852,7 +883,7 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_q_blocked_kernel(const unsigne
     fetch_stages(KS * st_lo);
     for (int st = st_lo; st <= st_hi; st += SPLIT ? 2 : 1) {
         const int buf = SPLIT ? sub : (st - st_lo) & 1, k0 = KS * (st + sub);
-        if (SPLIT && st > st_lo) __syncthreads();   // both stages are read
+        if (SPLIT && st > st_lo) __syncthreads();   // the stages and half stages before are read
 #pragma unroll
         for (int p = 0; p < (SPLIT ? 2 : 1); p++)
 #pragma unroll
@@ -878,14 +909,14 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_q_blocked_kernel(const unsigne
             }
         __syncthreads();
         if (st + (SPLIT ? 1 : 0) < st_hi) fetch_stages(KS * (st + (SPLIT ? 2 : 1)));
-        if (k0 > qhi || k0 + KS - 1 < qlo + 1 - ws) continue;
+        if (!SPLIT && (k0 > qhi || k0 + KS - 1 < qlo + 1 - ws)) continue;   // SPLIT: a stage of no key of these queries is not added
 #pragma unroll
         for (int half = 0; half < NH; half++) {
             const int hf = SPLIT ? wave & 1 : half;
             uint4 xh[2], xl[2], wb[2];
 #pragma unroll
             for (int qt = 0; qt < 2; qt++) {
-                f32x4 x[2];
+                uint2 hi[2], lo[2];
 #pragma unroll
                 for (int c = 0; c < 2; c++) {
                     const int kt = 2 * hf + c;
@@ -895,46 +926,51 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_q_blocked_kernel(const unsigne
                     if constexpr (NKS == 2) dw = mfma32(av1, doh[qt][1], dw);
                     if constexpr (NKS == 2) dw = mfma32(av1, dol[qt][1], dw);
                     const uint2 wp = c ? make_uint2(wcur[half][qt].z, wcur[half][qt].w) : make_uint2(wcur[half][qt].x, wcur[half][qt].y);
-                    x[c][0] = bf_lo(wp.x) * dw[0];
-                    x[c][1] = bf_hi(wp.x) * dw[1];
-                    x[c][2] = bf_lo(wp.y) * dw[2];
-                    x[c][3] = bf_hi(wp.y) * dw[3];
-                    dpart[qt] += (x[c][0] + x[c][1]) + (x[c][2] + x[c][3]);
+                    f32x4 x;
+                    split_products(wp.x, wp.y, dw, x, hi[c], lo[c]);
+                    const float d4 = sum_products(wp.x, wp.y, dw, x);
+                    if constexpr (SPLIT) Dx[wave][qt][c][l] = d4;
+                    else dpart[qt] += d4;
                 }
-                split8(x[0], x[1], xh[qt], xl[qt]);
+                xh[qt] = make_uint4(hi[0].x, hi[0].y, hi[1].x, hi[1].y);
+                xl[qt] = make_uint4(lo[0].x, lo[0].y, lo[1].x, lo[1].y);
                 wb[qt] = wcur[half][qt];
             }
+            if constexpr (SPLIT) {
 #pragma unroll
-            for (int dt = 0; dt < NDT; dt++) {
-                const uint4 a = ld_tr2<LDH>(Ks[buf], 32 * hf + 4 * g, 32 * hf + 16 + 4 * g, 16 * dt);
+                for (int qt = 0; qt < 2; qt++) { Px[wave][qt][0][l] = xh[qt]; Px[wave][qt][1][l] = xl[qt]; Px[wave][qt][2][l] = wb[qt]; }
+            } else {
+                add(Ks[buf], hf, xh, xl, wb);
+            }
+        }
+        if constexpr (SPLIT) {
+            __syncthreads();   // the four half stages are there
 #pragma unroll
-                for (int qt = 0; qt < 2; qt++) {
-                    aq[qt][dt] = mfma32(a, xh[qt], aq[qt][dt]);
-                    aq[qt][dt] = mfma32(a, xl[qt], aq[qt][dt]);
-                    bq[qt][dt] = mfma32(a, wb[qt], bq[qt][dt]);
+            for (int p = 0; p < 2; p++) {
+                if (st + p > st_hi) break;
+#pragma unroll
+                for (int hf = 0; hf < 2; hf++) {
+                    const int h = 2 * p + hf;
+                    const auto &x = Px[h][own.tile0];
+                    dpart[0] += Dx[h][own.tile0][0][l];
+                    dpart[0] += Dx[h][own.tile0][1][l];
+                    add(Ks[p], hf, {x[0][l]}, {x[1][l]}, {x[2][l]});
                 }
             }
         }
     }
-    if constexpr (SPLIT) {
-        float *buf = reinterpret_cast<float *>(&Ks[0][0][0]);
-        join_waves<NDT>(aq, bq, buf, wave, l);
-        join_waves(dpart, buf, wave, l);
-    }
 #pragma unroll
-    for (int qt = 0; qt < 2; qt++) {
-        const int tq = qlo + 16 * qt + r;
-        if (SPLIT && qt != wave >> 1) continue;
-        float dsum = dpart[qt];
+    for (int t = 0; t < Own::NT; t++) {
+        const int tq = qlo + 16 * (own.tile0 + t) + r;
+        float dsum = dpart[t];
         dsum += __shfl_xor(dsum, 16, 64);
         dsum += __shfl_xor(dsum, 32, 64);
         if (tq < s) {
-            if (g == 0 && !(SPLIT && (wave & 1))) dvec[(size_t)(b * H + h) * s + tq] = dsum;
+            if (g == 0 && own.dt0 == 0) dvec[(size_t)(b * H + h) * s + tq] = dsum;
             float *ob = d_q + (row0 + tq) * total + hoff;
 #pragma unroll
-            for (int dt = 0; dt < NDT; dt++)
-                if (own_tile<NDT, SPLIT>(qt, dt, wave))
-                    *reinterpret_cast<f32x4 *>(ob + 16 * dt + 4 * g) = (aq[qt][dt] - dsum * bq[qt][dt]) * scale;
+            for (int dt = 0; dt < Own::ND; dt++)
+                *reinterpret_cast<f32x4 *>(ob + 16 * (own.dt0 + dt) + 4 * g) = (aq[t][dt] - dsum * bq[t][dt]) * scale;
         }
     }
 }
@@ -954,9 +990,11 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_k_stats_kernel(const unsigned 
                                                                  const float *__restrict__ dvec,
                                                                  float *__restrict__ d_k, float *__restrict__ d_v,
                                                                  int s, int H, int ws, Out16 o16) {
-    __shared__ __align__(16) unsigned short QD[6][KS][LDH];   // two stages [query][dim] of Q, then of dO's hi, then lo
-    unsigned short (*const Qs)[KS][LDH] = QD, (*const Dh)[KS][LDH] = QD + 2, (*const Dl)[KS][LDH] = QD + 4;
+    constexpr int LD = SPLIT ? LDQ : LDH;
+    __shared__ __align__(16) unsigned short QD[6][KS][LD];   // two stages [query][dim] of Q, then of dO's hi, then lo
+    unsigned short (*const Qs)[KS][LD] = QD, (*const Dh)[KS][LD] = QD + 2, (*const Dl)[KS][LD] = QD + 4;
     __shared__ __align__(16) float Mc[2][KS], Iv[2][KS], Dd[2][KS];   // the stage's queries: maximum, 1 / sum, D
+    __shared__ HalfStage<3> Px[SPLIT ? 4 : 1];   // SPLIT: dS hi and lo and w of a wave's half stage
     const int tid = threadIdx.x, wave = tid >> 6, l = tid & 63, r = l & 15, g = l >> 4;
     const BlockCoord bc = xcd_block_coord(H);
     const int j0 = bc.x * (SPLIT ? SQ : FQ), h = bc.h, b = bc.b;
@@ -985,11 +1023,31 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_k_stats_kernel(const unsigned 
                 vf[jt][ks] = *reinterpret_cast<const uint4 *>(v + o);
             }
         }
-    f32x4 dk[2][4], dv[2][4];   // d_k^T, d_v^T: rows = dims 16 dt + 4 g + i, column = key
+    using Own = OwnTiles<NDT, SPLIT>;
+    const Own own(wave);
+    f32x4 dk[Own::NT][Own::ND], dv[Own::NT][Own::ND];   // d_k^T, d_v^T: rows = dims 16 dt + 4 g + i, column = key
 #pragma unroll
-    for (int jt = 0; jt < 2; jt++)
+    for (int t = 0; t < Own::NT; t++)
 #pragma unroll
-        for (int dt = 0; dt < NDT; dt++) { dk[jt][dt] = f32x4{0.f, 0.f, 0.f, 0.f}; dv[jt][dt] = f32x4{0.f, 0.f, 0.f, 0.f}; }
+        for (int dt = 0; dt < Own::ND; dt++) { dk[t][dt] = f32x4{0.f, 0.f, 0.f, 0.f}; dv[t][dt] = f32x4{0.f, 0.f, 0.f, 0.f}; }
+    // half hq of the stage in buffer `at` added to the sums of this wave's tiles
+    auto add = [&](int at, int hq, const uint4(&dsh)[Own::NT], const uint4(&dsl)[Own::NT], const uint4(&wpk)[Own::NT])
+                   __attribute__((always_inline)) {
+        const int ra = 32 * hq + 4 * g, rb = ra + 16;
+#pragma unroll
+        for (int dt = 0; dt < Own::ND; dt++) {
+            const uint4 aq = ld_tr2<LD>(Qs[at], ra, rb, 16 * (own.dt0 + dt));    // Q^T [dim][query]
+            const uint4 ah = ld_tr2<LD>(Dh[at], ra, rb, 16 * (own.dt0 + dt));    // dO^T hi / lo
+            const uint4 al = ld_tr2<LD>(Dl[at], ra, rb, 16 * (own.dt0 + dt));
+#pragma unroll
+            for (int t = 0; t < Own::NT; t++) {
+                dk[t][dt] = mfma32(aq, dsh[t], dk[t][dt]);
+                dk[t][dt] = mfma32(aq, dsl[t], dk[t][dt]);
+                dv[t][dt] = mfma32(ah, wpk[t], dv[t][dt]);
+                dv[t][dt] = mfma32(al, wpk[t], dv[t][dt]);
+            }
+        }
+    };
 
     // one stage ahead in registers: Q rows (two 16-byte pieces per thread), dO rows (thread = quarter row)
     constexpr int NP = SPLIT ? 2 : 1;
@@ -1016,7 +1074,7 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_k_stats_kernel(const unsigned 
     fetch_stages(KS * st_lo);
     for (int st = st_lo; st <= st_hi; st += NP) {
         const int buf = SPLIT ? wave >> 1 : (st - st_lo) & 1, t_lo = KS * (SPLIT ? st + buf : st);
-        if (SPLIT && st > st_lo) __syncthreads();   // both stages are read
+        if (SPLIT && st > st_lo) __syncthreads();   // the stages and half stages before are read
 #pragma unroll
         for (int p = 0; p < NP; p++)
 #pragma unroll
@@ -1034,13 +1092,14 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_k_stats_kernel(const unsigned 
         }
         __syncthreads();
         if (st + NP - 1 < st_hi) fetch_stages(KS * (st + NP));
-        if (t_lo + KS - 1 < jlo || t_lo > jhi + ws - 1) continue;   // no query of this stage sees a key of this wave
+        // no query of this stage sees a key of this wave (SPLIT: such a stage is not added)
+        if (!SPLIT && (t_lo + KS - 1 < jlo || t_lo > jhi + ws - 1)) continue;
         const bool full = t_lo >= jhi && t_lo + KS - 1 <= jlo + ws - 1 && t_lo + KS - 1 < s && jhi < s;
 #pragma unroll
         for (int half = 0; half < 3 - NP; half++) {
             const int hq = SPLIT ? wave & 1 : half;
             uint4 wpk[2], dsh[2], dsl[2];
-            f32x4 ds[2][2];
+            uint2 hi[2][2], lo[2][2];
             unsigned wp[2][2][2];
 #pragma unroll
             for (int c = 0; c < 2; c++) {
@@ -1068,57 +1127,59 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_k_stats_kernel(const unsigned 
                     }
                     wp[jt][c][0] = pack2(w[0], w[1]);   // as the weight tensor holds them
                     wp[jt][c][1] = pack2(w[2], w[3]);
-                    ds[jt][c][0] = bf_lo(wp[jt][c][0]) * dw[0];
-                    ds[jt][c][1] = bf_hi(wp[jt][c][0]) * dw[1];
-                    ds[jt][c][2] = bf_lo(wp[jt][c][1]) * dw[2];
-                    ds[jt][c][3] = bf_hi(wp[jt][c][1]) * dw[3];
+                    f32x4 ds;
+                    split_products(wp[jt][c][0], wp[jt][c][1], dw, ds, hi[jt][c], lo[jt][c]);
                 }
             }
 #pragma unroll
             for (int jt = 0; jt < 2; jt++) {
                 wpk[jt] = make_uint4(wp[jt][0][0], wp[jt][0][1], wp[jt][1][0], wp[jt][1][1]);
-                split8(ds[jt][0], ds[jt][1], dsh[jt], dsl[jt]);
+                dsh[jt] = make_uint4(hi[jt][0].x, hi[jt][0].y, hi[jt][1].x, hi[jt][1].y);
+                dsl[jt] = make_uint4(lo[jt][0].x, lo[jt][0].y, lo[jt][1].x, lo[jt][1].y);
             }
+            if constexpr (SPLIT) {
 #pragma unroll
-            for (int dt = 0; dt < NDT; dt++) {
-                const int ra = 32 * hq + 4 * g, rb = ra + 16;
-                const uint4 aq = ld_tr2<LDH>(Qs[buf], ra, rb, 16 * dt);    // Q^T [dim][query]
-                const uint4 ah = ld_tr2<LDH>(Dh[buf], ra, rb, 16 * dt);    // dO^T hi / lo
-                const uint4 al = ld_tr2<LDH>(Dl[buf], ra, rb, 16 * dt);
+                for (int jt = 0; jt < 2; jt++) { Px[wave][jt][0][l] = dsh[jt]; Px[wave][jt][1][l] = dsl[jt]; Px[wave][jt][2][l] = wpk[jt]; }
+            } else {
+                add(buf, hq, dsh, dsl, wpk);
+            }
+        }
+        if constexpr (SPLIT) {
+            __syncthreads();   // the four half stages are there
 #pragma unroll
-                for (int jt = 0; jt < 2; jt++) {
-                    dk[jt][dt] = mfma32(aq, dsh[jt], dk[jt][dt]);
-                    dk[jt][dt] = mfma32(aq, dsl[jt], dk[jt][dt]);
-                    dv[jt][dt] = mfma32(ah, wpk[jt], dv[jt][dt]);
-                    dv[jt][dt] = mfma32(al, wpk[jt], dv[jt][dt]);
+            for (int p = 0; p < 2; p++) {
+                if (st + p > st_hi) break;
+#pragma unroll
+                for (int hq = 0; hq < 2; hq++) {
+                    const auto &x = Px[2 * p + hq][own.tile0];
+                    add(p, hq, {x[0][l]}, {x[1][l]}, {x[2][l]});
                 }
             }
         }
     }
-    if constexpr (SPLIT) join_waves<NDT>(dk, dv, reinterpret_cast<float *>(&QD[0][0][0]), wave, l);
     // accumulate: column = key jlo + 16 jt + r, rows = dims 16 dt + 4 g ..
 #pragma unroll
-    for (int jt = 0; jt < 2; jt++) {
-        const int key = jlo + 16 * jt + r;
+    for (int t = 0; t < Own::NT; t++) {
+        const int key = jlo + 16 * (own.tile0 + t) + r;
         if (key >= s) continue;
         if (OUT16) {
             unsigned short *pk = o16.k + (row0 + key) * o16.ld + hoff, *pv = o16.v + (row0 + key) * o16.ld + hoff;
 #pragma unroll
-            for (int dt = 0; dt < NDT; dt++) {
-                if (!own_tile<NDT, SPLIT>(jt, dt, wave)) continue;
-                const f32x4 a = dk[jt][dt] * scale, c = dv[jt][dt];
-                *reinterpret_cast<uint2 *>(pk + 16 * dt + 4 * g) = make_uint2(pack2(a[0], a[1]), pack2(a[2], a[3]));
-                *reinterpret_cast<uint2 *>(pv + 16 * dt + 4 * g) = make_uint2(pack2(c[0], c[1]), pack2(c[2], c[3]));
+            for (int dt = 0; dt < Own::ND; dt++) {
+                const int at = 16 * (own.dt0 + dt) + 4 * g;
+                const f32x4 a = dk[t][dt] * scale, c = dv[t][dt];
+                *reinterpret_cast<uint2 *>(pk + at) = make_uint2(pack2(a[0], a[1]), pack2(a[2], a[3]));
+                *reinterpret_cast<uint2 *>(pv + at) = make_uint2(pack2(c[0], c[1]), pack2(c[2], c[3]));
             }
             continue;
         }
         float *pk = d_k + (row0 + key) * total + hoff, *pv = d_v + (row0 + key) * total + hoff;
 #pragma unroll
-        for (int dt = 0; dt < NDT; dt++) {
-            if (!own_tile<NDT, SPLIT>(jt, dt, wave)) continue;
-            f32x4 *ck = reinterpret_cast<f32x4 *>(pk + 16 * dt + 4 * g), *cv = reinterpret_cast<f32x4 *>(pv + 16 * dt + 4 * g);
-            *ck = *ck + dk[jt][dt] * scale;
-            *cv = *cv + dv[jt][dt];
+        for (int dt = 0; dt < Own::ND; dt++) {
+            const int at = 16 * (own.dt0 + dt) + 4 * g;
+            f32x4 *ck = reinterpret_cast<f32x4 *>(pk + at), *cv = reinterpret_cast<f32x4 *>(pv + at);
+            *ck = *ck + dk[t][dt] * scale;
+            *cv = *cv + dv[t][dt];
         }
     }
 }
@@ -1139,11 +1200,12 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_k_blocked_kernel(const unsigne
                                                                    const float *__restrict__ dvec,
                                                                    float *__restrict__ d_k, float *__restrict__ d_v,
                                                                    int s, int H, int ws) {
-    constexpr int NP = SPLIT ? 2 : 1, LDK = SPLIT ? 48 : LDW;
-    __shared__ __align__(16) unsigned short QD[6][KS][LDH];    // two stages [query][dim] of Q, then of dO's hi, then lo
+    constexpr int NP = SPLIT ? 2 : 1, LDK = SPLIT ? SQ : LDW, LD = SPLIT ? LDQ : LDH;
+    __shared__ __align__(16) unsigned short QD[6][KS][LD];    // two stages [query][dim] of Q, then of dO's hi, then lo
     __shared__ __align__(16) unsigned short Wt[NP * KS][LDK];  // [query][key of the block]
-    unsigned short (*const Qs)[KS][LDH] = QD, (*const Dh)[KS][LDH] = QD + 2, (*const Dl)[KS][LDH] = QD + 4;
+    unsigned short (*const Qs)[KS][LD] = QD, (*const Dh)[KS][LD] = QD + 2, (*const Dl)[KS][LD] = QD + 4;
     __shared__ __align__(16) float Dd[2][KS];
+    __shared__ HalfStage<2> Px[SPLIT ? 4 : 1];   // SPLIT: dS hi and lo of a wave's half stage
     const int tid = threadIdx.x, wave = tid >> 6, l = tid & 63, r = l & 15, g = l >> 4;
     const BlockCoord bc = xcd_block_coord(H);
     const int j0 = bc.x * (SPLIT ? SQ : FQ), h = bc.h, b = bc.b;
@@ -1168,11 +1230,31 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_k_blocked_kernel(const unsigne
             vf[jt][ks] = make_uint4(0, 0, 0, 0);
             if (key < s) vf[jt][ks] = *reinterpret_cast<const uint4 *>(v + (row0 + key) * total + hoff + 32 * ks + 8 * g);
         }
-    f32x4 dk[2][4], dv[2][4];
+    using Own = OwnTiles<NDT, SPLIT>;
+    const Own own(wave);
+    f32x4 dk[Own::NT][Own::ND], dv[Own::NT][Own::ND];   // d_k^T, d_v^T: rows = dims 16 dt + 4 g + i, column = key
 #pragma unroll
-    for (int jt = 0; jt < 2; jt++)
+    for (int t = 0; t < Own::NT; t++)
 #pragma unroll
-        for (int dt = 0; dt < NDT; dt++) { dk[jt][dt] = f32x4{0.f, 0.f, 0.f, 0.f}; dv[jt][dt] = f32x4{0.f, 0.f, 0.f, 0.f}; }
+        for (int dt = 0; dt < Own::ND; dt++) { dk[t][dt] = f32x4{0.f, 0.f, 0.f, 0.f}; dv[t][dt] = f32x4{0.f, 0.f, 0.f, 0.f}; }
+    // half hq of the stage in buffer `at` added to the sums of this wave's tiles
+    auto add = [&](int at, int hq, const uint4(&dsh)[Own::NT], const uint4(&dsl)[Own::NT], const uint4(&wpk)[Own::NT])
+                   __attribute__((always_inline)) {
+        const int ra = 32 * hq + 4 * g, rb = ra + 16;
+#pragma unroll
+        for (int dt = 0; dt < Own::ND; dt++) {
+            const uint4 aq = ld_tr2<LD>(Qs[at], ra, rb, 16 * (own.dt0 + dt));    // Q^T [dim][query]
+            const uint4 ah = ld_tr2<LD>(Dh[at], ra, rb, 16 * (own.dt0 + dt));    // dO^T hi / lo
+            const uint4 al = ld_tr2<LD>(Dl[at], ra, rb, 16 * (own.dt0 + dt));
+#pragma unroll
+            for (int t = 0; t < Own::NT; t++) {
+                dk[t][dt] = mfma32(aq, dsh[t], dk[t][dt]);
+                dk[t][dt] = mfma32(aq, dsl[t], dk[t][dt]);
+                dv[t][dt] = mfma32(ah, wpk[t], dv[t][dt]);
+                dv[t][dt] = mfma32(al, wpk[t], dv[t][dt]);
+            }
+        }
+    };
 
     // Weights: thread (query drow, quarter) reads the quarter's pieces of eight keys of the query's row
     constexpr int NW = SPLIT ? 1 : 4, QK = 8 * NW;
@@ -1217,6 +1299,11 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_k_blocked_kernel(const unsigne
             }
         }
     };
+    // weights of half hq of the stage in buffer `at` for key tile jt
+    auto weights = [&](int at, int hq, int jt) __attribute__((always_inline)) {
+        const int ra = 32 * hq + 4 * g;
+        return ld_tr2<LDK>(Wt + (SPLIT ? KS * at : 0), ra, ra + 16, (SPLIT ? 0 : 32 * wave) + 16 * jt);
+    };
     fetch_stages(KS * st_lo);
     for (int st = st_lo; st <= st_hi; st += NP) {
         const int buf = SPLIT ? wave >> 1 : (st - st_lo) & 1, t_lo = KS * (SPLIT ? st + buf : st);
@@ -1252,15 +1339,15 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_k_blocked_kernel(const unsigne
         if (tid < NP * KS) Dd[SPLIT ? tid / KS : buf][tid % KS] = ddreg;
         __syncthreads();
         if (st + NP - 1 < st_hi) fetch_stages(KS * (st + NP));
-        if (!(t_lo + KS - 1 < jlo || t_lo > jhi + ws - 1)) {   // a query of this stage sees a key of this wave
+        // a query of this stage sees a key of this wave (SPLIT: a stage without one is not added)
+        if (SPLIT || !(t_lo + KS - 1 < jlo || t_lo > jhi + ws - 1)) {
 #pragma unroll
             for (int half = 0; half < 3 - NP; half++) {
                 const int hq = SPLIT ? wave & 1 : half;
-                const int ra = 32 * hq + 4 * g, rb = ra + 16;
                 uint4 wpk[2], dsh[2], dsl[2];
-                f32x4 ds[2][2];
+                uint2 hi[2][2], lo[2][2];
 #pragma unroll
-                for (int jt = 0; jt < 2; jt++) wpk[jt] = ld_tr2<LDK>(Wt + (SPLIT ? KS * buf : 0), ra, rb, (SPLIT ? 0 : 32 * wave) + 16 * jt);
+                for (int jt = 0; jt < 2; jt++) wpk[jt] = weights(buf, hq, jt);
 #pragma unroll
                 for (int c = 0; c < 2; c++) {
                     const int qt = 2 * hq + c;
@@ -1274,43 +1361,48 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_k_blocked_kernel(const unsigne
                         if constexpr (NKS == 2) dw = mfma32(ah1, vf[jt][1], dw);
                         if constexpr (NKS == 2) dw = mfma32(al1, vf[jt][1], dw);
                         const unsigned w01 = c ? wpk[jt].z : wpk[jt].x, w23 = c ? wpk[jt].w : wpk[jt].y;
-                        ds[jt][c][0] = bf_lo(w01) * dw[0];
-                        ds[jt][c][1] = bf_hi(w01) * dw[1];
-                        ds[jt][c][2] = bf_lo(w23) * dw[2];
-                        ds[jt][c][3] = bf_hi(w23) * dw[3];
+                        f32x4 ds;
+                        split_products(w01, w23, dw, ds, hi[jt][c], lo[jt][c]);
                     }
                 }
 #pragma unroll
-                for (int jt = 0; jt < 2; jt++) split8(ds[jt][0], ds[jt][1], dsh[jt], dsl[jt]);
+                for (int jt = 0; jt < 2; jt++) {
+                    dsh[jt] = make_uint4(hi[jt][0].x, hi[jt][0].y, hi[jt][1].x, hi[jt][1].y);
+                    dsl[jt] = make_uint4(lo[jt][0].x, lo[jt][0].y, lo[jt][1].x, lo[jt][1].y);
+                }
+                if constexpr (SPLIT) {
 #pragma unroll
-                for (int dt = 0; dt < NDT; dt++) {
-                    const uint4 aq = ld_tr2<LDH>(Qs[buf], ra, rb, 16 * dt);    // Q^T [dim][query]
-                    const uint4 ah = ld_tr2<LDH>(Dh[buf], ra, rb, 16 * dt);    // dO^T hi / lo
-                    const uint4 al = ld_tr2<LDH>(Dl[buf], ra, rb, 16 * dt);
+                    for (int jt = 0; jt < 2; jt++) { Px[wave][jt][0][l] = dsh[jt]; Px[wave][jt][1][l] = dsl[jt]; }
+                } else {
+                    add(buf, hq, dsh, dsl, wpk);
+                }
+            }
+        }
+        if constexpr (SPLIT) {
+            __syncthreads();   // the four half stages are there
 #pragma unroll
-                    for (int jt = 0; jt < 2; jt++) {
-                        dk[jt][dt] = mfma32(aq, dsh[jt], dk[jt][dt]);
-                        dk[jt][dt] = mfma32(aq, dsl[jt], dk[jt][dt]);
-                        dv[jt][dt] = mfma32(ah, wpk[jt], dv[jt][dt]);
-                        dv[jt][dt] = mfma32(al, wpk[jt], dv[jt][dt]);
-                    }
+            for (int p = 0; p < 2; p++) {
+                if (st + p > st_hi) break;
+#pragma unroll
+                for (int hq = 0; hq < 2; hq++) {
+                    const auto &x = Px[2 * p + hq][own.tile0];
+                    add(p, hq, {x[0][l]}, {x[1][l]}, {weights(p, hq, own.tile0)});
                 }
             }
         }
         __syncthreads();   // the weight stage has one buffer: every wave is done with it before the next one lands
     }
-    if constexpr (SPLIT) join_waves<NDT>(dk, dv, reinterpret_cast<float *>(&QD[0][0][0]), wave, l);
 #pragma unroll
-    for (int jt = 0; jt < 2; jt++) {
-        const int key = jlo + 16 * jt + r;
+    for (int t = 0; t < Own::NT; t++) {
+        const int key = jlo + 16 * (own.tile0 + t) + r;
         if (key >= s) continue;
         float *pk = d_k + (row0 + key) * total + hoff, *pv = d_v + (row0 + key) * total + hoff;
 #pragma unroll
-        for (int dt = 0; dt < NDT; dt++) {
-            if (!own_tile<NDT, SPLIT>(jt, dt, wave)) continue;
-            f32x4 *ck = reinterpret_cast<f32x4 *>(pk + 16 * dt + 4 * g), *cv = reinterpret_cast<f32x4 *>(pv + 16 * dt + 4 * g);
-            *ck = *ck + dk[jt][dt] * scale;
-            *cv = *cv + dv[jt][dt];
+        for (int dt = 0; dt < Own::ND; dt++) {
+            const int at = 16 * (own.dt0 + dt) + 4 * g;
+            f32x4 *ck = reinterpret_cast<f32x4 *>(pk + at), *cv = reinterpret_cast<f32x4 *>(pv + at);
+            *ck = *ck + dk[t][dt] * scale;
+            *cv = *cv + dv[t][dt];
         }
     }
 }
@@ -1357,7 +1449,7 @@ bool swa_backward_mfma(const uint16_t *q, const uint16_t *k, const uint16_t *v, 
     if ((head_dim != 64 && head_dim != 32) || n_persistent != 0 || window > 512 || window < 1) return false;
     float *dvec = scratch(1, (size_t)batch * num_heads * seq_len * sizeof(float));
     if (es.failed()) return true;
-    // 32 rows a workgroup while those fit the chip at once, two to a compute unit (both sides above join_waves)
+    // 32 rows a workgroup while those fit the chip at once, two to a compute unit (both sides at SQ)
     const bool split = 2ll * ceil_div(seq_len, FQ) * num_heads * batch <= compute_units();
     const dim3 grid(ceil_div(seq_len, split ? SQ : FQ), num_heads, batch);
     const bool wide = head_dim == 64;

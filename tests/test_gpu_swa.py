@@ -160,8 +160,7 @@ def test_forward_with_one_query_tile_a_wave_and_with_two(s, ws, hd):
                                      (353, 130, 64), (600, 512, 64), (600, 511, 32)])
 def test_backward_in_blocks_of_32_rows_and_of_128(s, ws, hd):
     """The same sequences alone (few blocks: 32 rows a workgroup, the window shared out over its waves) and as one of many
-    (128 rows).  The two differ in the order of fp32 sums; a D that moves by that can take an element of dS to the other neighbour
-    in the 16 bits that its pair keeps, 2^-17 of it."""
+    (128 rows): every sum has one order, so a sequence's gradients are the same bits whatever batch it comes in."""
     H, blocks = 2, -(-s // 128) * 2
     n = torch.cuda.get_device_properties(0).multi_processor_count // (2 * blocks) + 1
     q, k, v, go = _case(1, s, H, hd, s + ws)
@@ -180,10 +179,8 @@ def test_backward_in_blocks_of_32_rows_and_of_128(s, ws, hd):
 
     few += tuple(stats_pair(q, k, v, go))
     lots += tuple(stats_pair(many(q), many(k), many(v), many(go)))
-    size = max(np.linalg.norm(x) for x in few)
     for a, b in zip(few, lots):
-        assert np.array_equal(b, many(b[:1]))
-        assert np.linalg.norm(a[0] - b[0]) <= 1e-5 * np.linalg.norm(a[0]) + 1e-6 * size
+        assert np.array_equal(b, many(a))
 
 
 def test_swa_known_answers_on_gpu():
