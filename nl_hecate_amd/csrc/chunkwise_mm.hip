@@ -714,6 +714,8 @@ bool backward_mm(const char *fn, const TIn *k, const TIn *v, const TIn *q, const
     if (!check_mm_args(fn, seq_len, d, batch, chunk_size)) return true;
     if (out16 && sizeof(TIn) != 2) { fail("%s: bf16 gradient slabs are served for bf16 tokens only.", fn); return true; }
     if (dy_rows && sizeof(TIn) != 2) { fail("%s: token-major d_y is served for bf16 tokens only.", fn); return true; }
+    const bool no_first = out16 && !d_m_initial && !d_s_initial;   // the level step may have no use for them
+    if (!d_m_initial && !no_first) { fail("%s: d_m_initial is null.", fn); return true; }
     if (guard && (out16 || dy_rows)) { fail("%s: the in-pass test is served for head-major fp32 gradients only.", fn); return true; }
     ChainTracks tracks{nullptr, nullptr};
     if (guard) tracks = chain_tracks(seq_len, batch, chunk_size);
@@ -783,7 +785,7 @@ bool backward_mm(const char *fn, const TIn *k, const TIn *v, const TIn *q, const
     const float *ds_first = packed ? reinterpret_cast<const float *>(reinterpret_cast<const uint16_t *>(ds_states) + n_snap)
                                    : ds_states;
     const int per = 8, rows = ceil_div(batch, per);
-    const int nsum = !d_m_initial ? 0 : has_s && d_s_initial ? 2 : 1;   // null: a caller has no use for them
+    const int nsum = no_first ? 0 : has_s && d_s_initial ? 2 : 1;
     float *tmp = nsum ? scratch(10, (size_t)nsum * rows * HD * HD * sizeof(float)) : nullptr;
     if (es.failed()) return true;
     // d_alpha, d_eta, and in the same launch the first stage of the deterministic sum of d_m_initial, d_s_initial

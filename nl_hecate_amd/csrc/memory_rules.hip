@@ -926,6 +926,7 @@ static void backward_ckpt_any(bool has_s, bool frozen, bool allow_fused,
                               float error_clip, float m_norm_max, const char *fn) {
     if (!check_dims(fn, seq_len, d, batch) || batch == 0 || seq_len == 0) return;
     if (C <= 0) { fail("%s: interval/chunk size %d must be > 0.", fn, C); return; }
+    if (!d_m_initial || (has_s && !d_s_initial)) { fail("%s: the gradient of an initial state is null.", fn); return; }
     // no clip: the fused kernel replays without the projection; with a bound it checks afterwards that none could
     // have fired (see launch_fwd) and otherwise leaves the call to the replay schedule below
     const bool bound = coupled_needed(0.f, m_norm_max);

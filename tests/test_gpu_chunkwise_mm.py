@@ -10,6 +10,7 @@ import pytest
 import torch
 
 from nl_hecate_amd import dispatch as D
+from nl_hecate_amd.ffi import lib
 from oracle import pyoracle as orc
 from tests.gpu_util import assert_close, dev, host, rule_inputs, zeros
 
@@ -267,6 +268,31 @@ def test_delta_matrix_form_matches_oracle(B, s, C, bf16):
     for n in ("d_k", "d_v", "d_q", "d_alpha", "d_theta"):
         assert_close(n, host(g[n]), np.stack([o[n] for o in bw]), tol)
     assert_close("d_m_initial", host(g["d_m"]), sum(o["d_m"] for o in bw), tol)
+
+
+@pytest.mark.parametrize("entry", ["titans_chunkwise_backward_bf16_rocm", "titans_chunkwise_backward_mm_f32_rocm",
+                                   "titans_chunkwise_backward_bf16_guarded_rocm", "titans_chunkwise_backward_f32_cuda",
+                                   "delta_chunkwise_backward_bf16_rocm", "delta_chunkwise_backward_f32_cuda"])
+def test_gradients_of_the_initial_states_are_not_dropped(entry):
+    """A null d_m_initial is refused by every entry point, with and without a d_s_initial, which is not left unwritten either; with
+    a bound as well, where the sequential kernels may come to write both."""
+    B, s, d, C = 2, 40, 64, 16
+    titans, dt = entry.startswith("titans"), torch.bfloat16 if "bf16" in entry else torch.float32
+    bounds = (0.0, 1e6) if "guarded" in entry or "cuda" in entry else ()
+    kvq = [torch.zeros(B, s, d, dtype=dt, device="cuda") for _ in range(3)]
+    gates = [zeros(B, s) for _ in range(3 if titans else 2)]
+    states = [zeros(B, 4, d, d) for _ in range(2 if titans else 1)]
+    out = [zeros(B, s, d) for _ in range(3)] + [zeros(B, s) for _ in gates]
+    torch.cuda.synchronize()
+    lib.nlh_set_error_mode(1)
+    try:
+        for first in [(None, zeros(d, d)), (None, None)] if titans else [(None,)]:
+            lib.nlh_clear_error()
+            D.call(entry, *kvq, *gates, *states, zeros(B, s, d), *out, *first, s, d, B, C, *bounds)
+            assert b"is null" in lib.nlh_last_error()
+    finally:
+        lib.nlh_clear_error()
+        lib.nlh_set_error_mode(0)
 
 
 @pytest.mark.parametrize("rule,n,s,C", [("titans", 72, 2000, 64), ("titans", 9, 2049, 8), ("delta", 72, 2000, 32)])
