@@ -114,3 +114,37 @@ def test_frozen_rule_at_head_size_32(has_s, B, s, C, bound):
         assert_close(n, got[0][n], fo[n], 1e-4)
     for n in go:
         assert_close(n, got[1][n], go[n], 1e-4)
+
+
+@pytest.mark.parametrize("rule,d", [("titans", 32), ("delta", 32), ("titans", 64)])
+def test_gate_gradients_of_more_chunks_than_waves(rule, d):
+    """The gate sweeps in float64 where a wave walks over several chunks (sixteen waves a compute unit are there at most), the short
+    last ones of chains among them: the gate gradients of every chain are those of a call with too few chunks for that, bit for
+    bit."""
+    C, per_chain, titans = 64, 65, rule == "titans"
+    n, s = 16 * torch.cuda.get_device_properties(0).multi_processor_count // per_chain + 2, 64 * (per_chain - 1) + 5
+    print(rule, d, n, s, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(d + titans)
+    rnd = lambda *shape: torch.randn(*shape, generator=g, device="cuda")
+    k, q = (x / x.norm(dim=-1, keepdim=True) for x in (rnd(n, s, d), rnd(n, s, d)))
+    gates = [torch.sigmoid(rnd(n, s)) for _ in range(3 if titans else 2)]
+    x, m0, d_y = [k, rnd(n, s, d), q] + gates, rnd(n, d * d) * 0.02, rnd(n, s, d)
+    slots = orc.checkpoint_count(s, C)
+
+    def both(a, b):
+        cut = lambda t: t[a:b].contiguous()
+        args, states = [cut(t) for t in x], [zeros(b - a, slots, d * d) for _ in range(2 if titans else 1)]
+        initial = [cut(m0)] + [zeros(b - a, d * d)] * (len(states) - 1)
+        out = [zeros(b - a, s, d) for _ in range(3)] + [zeros(b - a, s) for _ in gates]
+        first = [zeros(d, d) for _ in states]
+        D.call(f"{rule}_forward_ckpt_batched_f32_rocm", *args, *initial, *states, zeros(b - a, s, d), s, d, b - a, C, 0.0, F32_MAX)
+        ran = kernels_run(lambda: D.call(f"{rule}_backward_ckpt_f32_rocm", *args, *states, cut(d_y), *out, *first, s, d, b - a, C,
+                                         0.0, F32_MAX))
+        assert "cw_gates_sweep_kernel" in ran, ran
+        return [out[3]] + out[5:]
+
+    whole = both(0, n)
+    cuts = [i * n // 9 for i in range(10)]
+    parts = [both(a, b) for a, b in zip(cuts, cuts[1:])]
+    for i, t in enumerate(whole):
+        assert t.isfinite().all() and torch.equal(t, torch.cat([p[i] for p in parts])), i
