@@ -160,7 +160,8 @@ extern "C" int nlh_selftest_chunk_coef(const float *alpha, const float *theta, c
 
 namespace nlh {
 // The helpers of the coefficient pre-passes on one chunk: table[t][j] = theta-free c[t][j] and, with scale = -theta_j,
-// the forward's W[t][j]; vecs [5][64] = a, beta, h, cl, bl of token (lane).
+// the forward's W[t][j]; vecs [5][64] = a, beta, h, cl, bl of token (lane).  Every table follows one of another length and other
+// gates in the same LDS, as in a wave that walks over chunks.
 __global__ void chunk_coef_prepass_kernel(const float *alpha, const float *theta, const float *eta, int L,
                                           float *table, float *table_scaled, float *vecs) {
     __shared__ __align__(16) ChunkTable ct;
@@ -177,10 +178,16 @@ __global__ void chunk_coef_prepass_kernel(const float *alpha, const float *theta
     for (int t = 0; t < 64; t++) table[t * 64 + l] = table_scaled[t * 64 + l] = 0.f;
     __syncthreads();
     const int one = l & 15, four = 4 * (l >> 4);
+    const int other_L = L == 64 ? 21 : 64;
+    const bool other_in = l < other_L;
+    const float other_keep = other_in ? 0.75f : 1.f, other_et = other_in ? 0.5f : 0.f;
+    const ChunkVectors other = coef_vectors(other_keep, other_et, other_in);
+    chunk_table_build(ct, other, other_keep, other_et, other_in ? 3.f : 0.f, other_L);
     chunk_table_build(ct, cv, keep, et, in ? 1.f : 0.f, L);
     chunk_table_tiles<true, 0, 0>(ct, cv, [&](int T, int J, const cf32x4 &c) {
         for (int i = 0; i < 4; i++) table[(16 * T + four + i) * 64 + 16 * J + one] = c[i];
     });
+    chunk_table_build(ct, other, other_keep, other_et, other_in ? 3.f : 0.f, other_L);
     chunk_table_build(ct, cv, keep, et, nth, L);
     chunk_table_tiles<false, 0, 0>(ct, cv, [&](int T, int J, const cf32x4 &w) {
         for (int i = 0; i < 4; i++) table_scaled[(16 * T + one) * 64 + 16 * J + four + i] = w[i];

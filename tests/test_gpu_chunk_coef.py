@@ -78,7 +78,8 @@ def test_generated_coefficients_match_the_recurrences(kind, L):
 
 @pytest.mark.parametrize("kind,L", CASES)
 def test_prepass_helpers_match_the_recurrences(kind, L):
-    """coef_vectors and the tiles of chunk_table_tiles (what cw_coef_kernel / cw_coef_bwd_kernel are made of) on one chunk."""
+    """coef_vectors and the tiles of chunk_table_tiles (what cw_coef_kernel / cw_coef_bwd_kernel are made of) on one chunk,
+    behind one of another length in the same tables."""
     rs = np.random.default_rng(L * 11 + len(kind))
     sig = lambda x: 1 / (1 + np.exp(-x))
     al, th, et = (sig(rs.standard_normal(64)).astype(np.float32) for _ in range(3))
