@@ -65,6 +65,33 @@ def test_frequency_aware_adamw_under_scripted_pulses():
     assert host(dW[3]).max() <= 2.0
 
 
+@pytest.mark.parametrize("max_norm", [0.0, 1.0])
+def test_bounds_of_a_tensor_hold_behind_the_whole_update(max_norm):
+    """Bounds in the update's body of four elements a thread, its tail, the path of buffers that are not 16-byte aligned, and of a
+    tensor that takes many workgroups: the weights of the same step without bounds, cut off at them, bit for bit; gradients and
+    moments the same.  Bounds on both sides are crossed."""
+    sizes, shift = [1024, 513, 1027, 64, 5, 1, 300001, 256, 513], [0, 0, 0, 1, 2, 3, 0, 0, 1]
+    bounded = [0, 1, 2, 3, 4, 6, 8]
+    make = lambda a, o: dev(np.concatenate([np.zeros(o, np.float32), a]))[o:]
+    start = [[rnd(n), rnd(n), 0.1 * rnd(n), rnd(n) ** 2] for n in sizes]
+    results = []
+    for clamp in (True, False):
+        opt, t = FrequencyAwareAdamW(1, 0.9, 0.95, 1e-8, 0.1), [[make(a, o) for a in p] for p, o in zip(start, shift)]
+        ids = [opt.add_tensor(-1, w, g, m, v) for w, g, m, v in t]
+        if clamp:
+            for i in bounded:
+                opt.set_clamp(ids[i], -0.25, 0.5)
+        opt.step(Conductor(1, [1]).pulse(), 1e-2, max_norm, zeros(2))
+        torch.cuda.synchronize()
+        results.append([[host(x) for x in p] for p in t])
+    for i, (one, other) in enumerate(zip(*results)):
+        want = np.clip(other[0], np.float32(-0.25), np.float32(0.5)) if i in bounded else other[0]
+        assert np.array_equal(one[0], want), i
+        assert all(np.array_equal(a, b) for a, b in zip(one[1:], other[1:])), i
+        if sizes[i] > 5:
+            assert other[0].min() < -0.25 and other[0].max() > 0.5
+
+
 @pytest.mark.parametrize("k", [1, 2, 4])
 def test_combine_gate_and_backward(k):
     n = 5003
