@@ -582,7 +582,7 @@ class MagLayer:
 
     def backward(self, cache, d_out, grads=None):
         """-> (d_x [bs, s, d], grads: MagParams of gradients).  `grads`: a MagParams from new_grads() to write
-        into (zeroed here first); a new one is made otherwise."""
+        into, whatever it holds (cleared here unless every gradient is written); a new one is made otherwise."""
         x = cache["x"]
         bs, s, d = x.shape
         p, nh, hd = self.p, self.nh, self.hd
@@ -591,7 +591,7 @@ class MagLayer:
         do2 = d_out.reshape(n, d)
         if grads is None:
             grads = self.new_grads()
-        elif not (cache.get("bf16") and cache["na"] == self.k):   # with every level active each one is written
+        elif not (cache.get("bf16") and cache["na"] == self.k):   # there, with every level active, each one is written
             grads.flat.zero_()
         if cache.get("bf16"):
             return self._backward_bf16(cache, d_out, grads), grads

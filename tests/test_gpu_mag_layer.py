@@ -240,6 +240,29 @@ def test_decode_steps_reproduce_the_full_sequence_forward(frozen_second):
         assert m_err <= 1e-4 * max(full.m_state[lv].abs().max().item(), 1e-6), (lv, m_err)
 
 
+@pytest.mark.parametrize("bs,s,heads,k", [(1, 65, 4, 1), (2, 200, 4, 2), (1, 513, 8, 4)])
+def test_backward_writes_every_gradient_that_it_does_not_clear(bs, s, heads, k):
+    """With every level active a buffer of gradients handed in is not cleared first: what was there, NaN, is all gone, and the
+    gradients are those in a new buffer, bit for bit."""
+    d = 64 * heads
+    layer = MagLayer(d, heads, k, 64, [1, 1, 1, 1][:k], rule="chunkwise", chunk=64, seed=31, precision="bf16")
+    g = torch.Generator(device="cuda").manual_seed(s)
+    x, d_out = (torch.randn(bs, s, d, generator=g, device="cuda") for _ in range(2))
+    _, cache = layer.forward(x)
+    assert cache["bf16"] and cache["na"] == k
+    tensors = lambda m: [m.w_q, m.w_k, m.w_v, m.w_o] + [getattr(lv, n) for lv in m.levels for n in (
+        "w_k", "w_v", "w_q", "w_alpha", "b_alpha", "w_theta", "b_theta", "w_eta", "b_eta")]
+    given = layer.new_grads()
+    for t in tensors(given):
+        t.fill_(float("nan"))
+    d_x, got = layer.backward(cache, d_out, given)
+    want_x, want = layer.backward(cache, d_out)
+    torch.cuda.synchronize()
+    assert got is given and torch.equal(d_x, want_x)
+    for a, b in zip(tensors(got), tensors(want)):
+        assert torch.equal(a, b) and b.any()
+
+
 def test_failed_capture_restores_the_launch_stream_and_the_context_memories():
     """A warm-up that raises must not leave the library launching on the side stream, nor the context memories
     advanced: the next (eager) step then equals the step of a trainer that never tried to capture."""
