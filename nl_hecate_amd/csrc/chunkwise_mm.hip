@@ -322,8 +322,8 @@ __global__ __launch_bounds__(kThr) void cw_out_fwd_kernel(const TIn *__restrict_
 // other's products, taken where there are more chunks than compute units; a chunk by itself is faster with the registers.
 // Against one persistent workgroup a compute unit that asked for its next chunk ahead, forward and backward of the rule, us: 2048
 // chunks 617 -> 608, 768 296 -> 293 (this kernel 42 -> 38), 8192 2141 -> 2102; as pairs 40 and 252 chunks lose 2.
-template <class TIn, bool PAIR>
-__global__ __launch_bounds__(kThr, PAIR ? 4 : 2) void cw_local_bwd_kernel(const TIn *__restrict__ k, const TIn *__restrict__ q,
+template <bool PAIR>
+__global__ __launch_bounds__(kThr, PAIR ? 4 : 2) void cw_local_bwd_kernel(const float *__restrict__ k, const float *__restrict__ q,
                                                             const float *__restrict__ d_y,
                                                             const float *__restrict__ alpha,
                                                             const float *__restrict__ theta,
@@ -337,8 +337,7 @@ __global__ __launch_bounds__(kThr, PAIR ? 4 : 2) void cw_local_bwd_kernel(const 
     NLH_STRIP_ORIGIN();
     const int task = blockIdx.x, chain = task / nc, ci = task % nc, t0 = ci * C, L = min(C, s - t0);
     const size_t tok = (size_t)chain * s + t0;
-    Tile<TIn> tk, tq;
-    Tile<float> td;
+    Tile<float> tk, tq, td;
     const Gates gt = fetch_gates(alpha + tok, theta + tok, eta + tok, L, has_s != 0);
     fetch(tk, k + tok * HD, L);
     fetch(tq, q + tok * HD, L);
@@ -403,9 +402,9 @@ constexpr size_t kLocalBwdLds = 5 * MAT * sizeof(float), kLocalBwdPairLds = 4 * 
 // ── backward, main per-chunk pass: dQ, dK, dV, dtheta; exports for the gate pass ──
 //   pvec [chain][token][4] = p0, ps, -theta g1, -theta g2   xs [chain][chunk][j][t] = -theta_j (dy_t.e_j)(q_t.k_j)
 //   scal [chunk][4] = <M0, dMo>, <S0, dMo>, <S0, dSo> (dMo, dSo: adjoints of the chunk's end state)
-template <class TIn, bool TRACK>
+template <bool TRACK>
 __global__ __launch_bounds__(kThr) void cw_grads_bwd_kernel(
-    const TIn *__restrict__ k, const TIn *__restrict__ v, const TIn *__restrict__ q, const float *__restrict__ d_y,
+    const float *__restrict__ k, const float *__restrict__ v, const float *__restrict__ q, const float *__restrict__ d_y,
     const float *__restrict__ alpha, const float *__restrict__ theta, const float *__restrict__ eta,
     const float *__restrict__ m_states, const float *__restrict__ s_states, const float *__restrict__ dm_states,
     const float *__restrict__ ds_states, float *__restrict__ d_k, float *__restrict__ d_v, float *__restrict__ d_q,
@@ -419,8 +418,7 @@ __global__ __launch_bounds__(kThr) void cw_grads_bwd_kernel(
     __shared__ float dots[3][8];       // partial <M0, dMo>, <S0, dMo>, <S0, dSo> per wave (the gate pass's scalars)
     float *Ss = B5, *Cc = B6;
     NLH_STRIP_ORIGIN();
-    Tile<TIn> tk, tq, tv;
-    Tile<float> td, tm, ts;
+    Tile<float> tk, tq, tv, td, tm, ts;
     Gates gt;
     auto fetch_task = [&](int task) {
         const int chain = task / nc, ci = task % nc, t0 = ci * C, L = min(C, s - t0);
@@ -734,13 +732,10 @@ bool backward_mm(const char *fn, const TIn *k, const TIn *v, const TIn *q, const
     if (es.failed()) return true;
     static bool attr_set = false;
     if (!attr_set) {
-        set_lds(cw_local_bwd_kernel<float, false>, kLocalBwdLds);
-        set_lds(cw_local_bwd_kernel<uint16_t, false>, kLocalBwdLds);
-        set_lds(cw_local_bwd_kernel<float, true>, kLocalBwdPairLds);
-        set_lds(cw_local_bwd_kernel<uint16_t, true>, kLocalBwdPairLds);
-        set_lds(cw_grads_bwd_kernel<float, false>, kGradsBwdLds);
-        set_lds(cw_grads_bwd_kernel<float, true>, kGradsBwdLds);
-        set_lds(cw_grads_bwd_kernel<uint16_t, false>, kGradsBwdLds);
+        set_lds(cw_local_bwd_kernel<false>, kLocalBwdLds);
+        set_lds(cw_local_bwd_kernel<true>, kLocalBwdPairLds);
+        set_lds(cw_grads_bwd_kernel<false>, kGradsBwdLds);
+        set_lds(cw_grads_bwd_kernel<true>, kGradsBwdLds);
         attr_set = true;
     }
     if constexpr (sizeof(TIn) == 2) {
@@ -758,7 +753,7 @@ bool backward_mm(const char *fn, const TIn *k, const TIn *v, const TIn *q, const
                              persistent_grid(batch * nc), dy_rows, out16, guard ? &tracks : nullptr);
     } else {
         const bool pair = batch * nc > compute_units();
-        hipLaunchKernelGGL((pair ? cw_local_bwd_kernel<TIn, true> : cw_local_bwd_kernel<TIn, false>), dim3(batch * nc), dim3(kThr),
+        hipLaunchKernelGGL((pair ? cw_local_bwd_kernel<true> : cw_local_bwd_kernel<false>), dim3(batch * nc), dim3(kThr),
                            pair ? kLocalBwdPairLds : kLocalBwdLds, stream(), k, q, d_y, alpha, theta, eta, sc.loc, sc.locs, seq_len, chunk_size, nc,
                            (int)has_s);
         check_launch("cw_local_bwd_kernel");
@@ -766,16 +761,9 @@ bool backward_mm(const char *fn, const TIn *k, const TIn *v, const TIn *q, const
                            nullptr, nullptr, sc.loc, sc.locs, dm_states, ds_states, nc, batch);
         check_launch("cw_scan_kernel");
         KernelTimer kt("cw_grads_bwd_kernel");
-        if (guard)
-            hipLaunchKernelGGL((cw_grads_bwd_kernel<float, true>), dim3(batch * nc), dim3(kThr), kGradsBwdLds, stream(),
-                               reinterpret_cast<const float *>(k), reinterpret_cast<const float *>(v),
-                               reinterpret_cast<const float *>(q), d_y, alpha, theta, eta, m_states, s_states, dm_states,
-                               ds_states, d_k, d_v, d_q, d_theta, pvec, xs, scal, seq_len, chunk_size, nc, (int)has_s, batch * nc,
-                               tracks);
-        else
-            hipLaunchKernelGGL((cw_grads_bwd_kernel<TIn, false>), dim3(batch * nc), dim3(kThr), kGradsBwdLds, stream(), k, v,
-                               q, d_y, alpha, theta, eta, m_states, s_states, dm_states, ds_states, d_k, d_v, d_q, d_theta,
-                               pvec, xs, scal, seq_len, chunk_size, nc, (int)has_s, batch * nc, ChainTracks{nullptr, nullptr});
+        hipLaunchKernelGGL((guard ? cw_grads_bwd_kernel<true> : cw_grads_bwd_kernel<false>), dim3(batch * nc), dim3(kThr),
+                           kGradsBwdLds, stream(), k, v, q, d_y, alpha, theta, eta, m_states, s_states, dm_states, ds_states, d_k,
+                           d_v, d_q, d_theta, pvec, xs, scal, seq_len, chunk_size, nc, (int)has_s, batch * nc, tracks);
         check_launch("cw_grads_bwd_kernel");
     }
     const bool packed = sizeof(TIn) == 2;   // where the gradient of the initial state sits (see above)
