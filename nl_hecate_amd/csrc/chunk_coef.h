@@ -21,6 +21,7 @@
 
 #include <algorithm>
 
+#include "lane_ops.h"
 #include "runtime.h"
 
 namespace nlh {
@@ -275,10 +276,6 @@ __device__ __forceinline__ void diag_steps(float *dst, float keep, float et, flo
         dst[I * kDiagLd] = c;
         diag_steps<I + 1>(dst, keep, et, b, c);
     }
-}
-__device__ __forceinline__ void wave_lds_order() {   // LDS that the lanes of one wave exchange
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
 }
 // One wave, lane = token; keep and et are zero or the identity's beyond L, scale zero there.
 // A lane whose block has ended goes on with gates of zero: it writes zeros, and they land in the part of the next tile that is

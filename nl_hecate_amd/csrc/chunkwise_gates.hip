@@ -31,6 +31,7 @@
 #include <algorithm>
 
 #include "chunkwise_grads.h"
+#include "lane_ops.h"
 #include "runtime.h"
 
 namespace nlh {
@@ -93,11 +94,6 @@ __global__ __launch_bounds__(64 * kGateWaves, 2) void cw_gates_sweep_kernel(
     if (task >= ntask) return;   // no barrier below: waves are independent
     GateRows<T> &gr = reinterpret_cast<GateRows<T> *>(smem)[wv];
     float *U = smem + kGateWaves * sizeof(GateRows<T>) / sizeof(float) + (size_t)wv * (HAS_S ? 2 : 1) * GTRI, *V = U + GTRI;
-    // rows of LDS are written and read back by different lanes of one wave
-    auto lds_order = [] {
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-    };
     struct Chunk {
         size_t tok;
         int L;
@@ -141,7 +137,7 @@ __global__ __launch_bounds__(64 * kGateWaves, 2) void cw_gates_sweep_kernel(
         int own = lane;
         asm volatile("" : "+v"(own));   // as if new for each chunk: 64 comparisons kept for all of them would not fit the scalar registers
         if (after < ntask) coming = chunk_of(after);
-        lds_order();   // the chunk before has been read
+        wave_lds_order();   // the chunk before has been read
         gr.keep[lane] = in ? T(1) - T(c.alpha) : T(1);
         gr.eta[lane] = c.eta;
         gr.g1[lane] = c.pv.z;
@@ -153,7 +149,7 @@ __global__ __launch_bounds__(64 * kGateWaves, 2) void cw_gates_sweep_kernel(
         T pum = um, pvm = vm, pvs = vs;              // their values at s = lane - 1
         U[tri_row(0) + lane] = (float)u;
         if (HAS_S) V[tri_row(0) + lane] = (float)v;
-        lds_order();   // the gates for the sweep; and row 0 before the others
+        wave_lds_order();   // the gates for the sweep; and row 0 before the others
         Four<T> kpn = four_at(gr.keep);
         Four<float> etn = four_at(gr.eta), g1n = four_at(gr.g1), g2n = four_at(gr.g2);
 #pragma unroll
@@ -192,7 +188,7 @@ __global__ __launch_bounds__(64 * kGateWaves, 2) void cw_gates_sweep_kernel(
             if (s0 % 16 == 12 && after < ntask) request(after, s0 / 16);
             __builtin_amdgcn_sched_barrier(0);
         }
-        lds_order();
+        wave_lds_order();
 
         // ── sweep 2: lane = s; weights r[s][t], c[t][s], bb[s][t] advance with t and start, with the sums, at t = s: what the lane
         // reads before, other rows' values, leaves nothing behind ──

@@ -165,6 +165,13 @@ __device__ __forceinline__ void wave_reduce_scatter(float (&v)[N], float (&out)[
     for (int n = 0; n < N / 4; n++) out[n] = group_allreduce<16>(out[n]);
 }
 
+// LDS that the lanes of one wave exchange: what was written before is there for what reads behind it.  A wave's LDS instructions
+// take effect in their order; this keeps the compiler to it.
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // Which entry of a batch block blk belongs to: begin[0 .. count), ascending, at most 64; blk is the same for the whole wave and all
 // of its lanes are here.  One load for all entries; a walk over them was a chain of scalar loads.
 __device__ __forceinline__ int batch_entry(const int *begin, int count, int blk) {

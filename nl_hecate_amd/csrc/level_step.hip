@@ -212,11 +212,6 @@ __device__ __forceinline__ void project_block(const u16 *Xs, const u16 *wf, f32x
 // instruction stores eight complete 128-byte rows.  A compute unit's store path moved the 8-byte pieces at about
 // half the rate.  tb: the wave's own [8][72] bf16; row_ptr(R): where the wave's 64 columns of token R (0 .. 31 of
 // this tile) go, or null past the end.
-__device__ __forceinline__ void lanes_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 template <class RowPtr>
 __device__ __forceinline__ void store_tile_rows(const f32x16 (&t)[2], float scale, u16 *tb, RowPtr row_ptr) {
     const int lane = threadIdx.x & 63, l32 = lane & 31, hf = lane >> 5;
@@ -233,9 +228,9 @@ __device__ __forceinline__ void store_tile_rows(const f32x16 (&t)[2], float scal
         }
         // lanes exchange data here: to the compiler a lane that skipped the writes above has nothing to wait for and
         // its read may run before the other lanes' writes (it did); the wave barrier keeps the order for all lanes
-        lanes_sync();
+        wave_lds_order();
         const bf16x8 r = *reinterpret_cast<const bf16x8 *>(tb + (lane >> 3) * 72 + (lane & 7) * 8);
-        lanes_sync();
+        wave_lds_order();
         u16 *dst = row_ptr(8 * h + (lane >> 3));
         if (dst) *reinterpret_cast<bf16x8 *>(dst + (lane & 7) * 8) = r;
     }

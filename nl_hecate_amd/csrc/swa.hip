@@ -28,12 +28,6 @@ constexpr int kSwaWaves = 4;
 
 __device__ __forceinline__ float bf2f(unsigned short h) { return __uint_as_float(((unsigned)h) << 16); }
 
-// Orders one wave's LDS writes before reads by its other lanes.
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
-
 struct SwaGeom { int n_p, ls, ll; };
 __device__ __forceinline__ SwaGeom swa_geom(int t, int window, int n_persistent) {
     SwaGeom g;
@@ -93,7 +87,7 @@ __global__ __launch_bounds__(kSwaWaves * 64) void swa_forward_kernel(
     const float scale = 1.0f / sqrtf((float)head_dim);
 
     for (int d = lane; d < head_dim; d += 64) vec[d] = bf2f(qb[d]);
-    wave_sync();
+    wave_lds_order();
     // scores, one key per lane per round
     float mx = -INFINITY;
     for (int s = lane; s < aw; s += 64) {
@@ -122,7 +116,7 @@ __global__ __launch_bounds__(kSwaWaves * 64) void swa_forward_kernel(
         sc[s] = w;
         wr[s] = f32_to_bf16_rne(w);
     }
-    wave_sync();
+    wave_lds_order();
     // out[d] = sum_s w_s v[key_s][d]  (unrounded weights, as the reference)
     for (int d = lane; d < head_dim; d += 64) {
         float acc = 0.f;
@@ -160,7 +154,7 @@ __global__ __launch_bounds__(kSwaWaves * 64) void swa_backward_query_kernel(
     const float scale = 1.0f / sqrtf((float)head_dim);
 
     for (int d = lane; d < head_dim; d += 64) vec[d] = d_out[qo + d];
-    wave_sync();
+    wave_lds_order();
     float dot_pw = 0.f;
     for (int s = lane; s < aw; s += 64) {
         const bool valid = s < n_persistent ? s < g.n_p : (s - n_persistent) < g.ll;
@@ -178,7 +172,7 @@ __global__ __launch_bounds__(kSwaWaves * 64) void swa_backward_query_kernel(
         sc[s] = ds;
         dsr[s] = ds;
     }
-    wave_sync();
+    wave_lds_order();
     for (int d = lane; d < head_dim; d += 64) {
         float acc = 0.f;
         for (int s = 0; s < g.n_p; s++) acc += sc[s] * bf2f(kb[(size_t)s * td + d]);

@@ -63,11 +63,6 @@ __device__ __forceinline__ float groups_max(float x) {
     asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(a), "+v"(b));
     return fmaxf(a, b);
 }
-// LDS that the lanes of one wave exchange
-__device__ __forceinline__ void wave_lds_order() {
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
 // mask of elements e (low half) and e + 1 of those numbered first .. last
 __device__ __forceinline__ unsigned own_pair(int e, int first, int last) {
     return (e >= first && e <= last ? 0xffffu : 0u) | (e + 1 >= first && e + 1 <= last ? 0xffff0000u : 0u);
