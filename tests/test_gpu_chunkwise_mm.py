@@ -66,7 +66,8 @@ CASES = [  # B, s, C
     (2, 24, 1),
     (1, 1, 64),      # one token
     (5, 64, 7),      # odd chunk length, remainder of 1
-    (300, 70, 64),   # more chunk tasks (600) than compute units: the persistent kernels loop over ragged ranges
+    (300, 70, 64),   # more chunks (600) than compute units: the gradient kernel of bf16 tokens loops over ragged ranges, the local pass of
+                     # float tokens runs two workgroups a compute unit
 ]
 
 
