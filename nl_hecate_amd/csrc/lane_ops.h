@@ -166,10 +166,12 @@ __device__ __forceinline__ void wave_reduce_scatter(float (&v)[N], float (&out)[
 }
 
 // LDS that the lanes of one wave exchange: what was written before is there for what reads behind it.  A wave's LDS instructions
-// take effect in their order; this keeps the compiler to it.
+// take effect in their order; this keeps the compiler to it, on either side of the place where lanes that skipped a write meet
+// the others again (with one fence in front of it, a read behind may move up to it, and into the branch that skips the write).
 __device__ __forceinline__ void wave_lds_order() {
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 // Which entry of a batch block blk belongs to: begin[0 .. count), ascending, at most 64; blk is the same for the whole wave and all
