@@ -88,9 +88,11 @@ __device__ __forceinline__ void split_products(unsigned w01, unsigned w23, f32x4
     lo = make_uint2(pack2(fmaf(w[0], dw[0], -bf_lo(hi.x)), fmaf(w[1], dw[1], -bf_hi(hi.x))),
                     pack2(fmaf(w[2], dw[2], -bf_lo(hi.y)), fmaf(w[3], dw[3], -bf_hi(hi.y))));
 }
-// their sum
-__device__ __forceinline__ float sum_products(unsigned w01, unsigned w23, f32x4 dw, f32x4 x) {
-    return fmaf(bf_lo(w01), dw[0], x[1]) + fmaf(bf_lo(w23), dw[2], x[3]);
+// their sum; it is there before lo can be used, or factors of every tile would wait in registers for the stage's end
+__device__ __forceinline__ float sum_products(unsigned w01, unsigned w23, f32x4 dw, f32x4 x, uint2 &lo) {
+    float sum = fmaf(bf_lo(w01), dw[0], x[1]) + fmaf(bf_lo(w23), dw[2], x[3]);
+    asm("" : "+v"(sum), "+v"(lo.y));
+    return sum;
 }
 // Workgroup -> (block of the sequence, head * batch) with all blocks of one head on one XCD.
 // Workgroups go to the 8 XCDs round robin in linear order, and each XCD has its own L2; blocks
@@ -694,7 +696,7 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_q_stats_kernel(const unsigned 
                     wp[c][1] = pack2(w[2], w[3]);
                     f32x4 x;
                     split_products(wp[c][0], wp[c][1], dw, x, hi[c], lo[c]);
-                    const float d4 = sum_products(wp[c][0], wp[c][1], dw, x);
+                    const float d4 = sum_products(wp[c][0], wp[c][1], dw, x, lo[c]);
                     if constexpr (SPLIT) Dx[wave][qt][c][l] = d4;
                     else dpart[qt] += d4;
                 }
@@ -923,7 +925,7 @@ __global__ __launch_bounds__(256, 2) void swa_bwd_q_blocked_kernel(const unsigne
                     const uint2 wp = c ? make_uint2(wcur[half][qt].z, wcur[half][qt].w) : make_uint2(wcur[half][qt].x, wcur[half][qt].y);
                     f32x4 x;
                     split_products(wp.x, wp.y, dw, x, hi[c], lo[c]);
-                    const float d4 = sum_products(wp.x, wp.y, dw, x);
+                    const float d4 = sum_products(wp.x, wp.y, dw, x, lo[c]);
                     if constexpr (SPLIT) Dx[wave][qt][c][l] = d4;
                     else dpart[qt] += d4;
                 }
