@@ -33,7 +33,7 @@ hipStream_t stream();   // launch stream (the null stream unless nlh_set_stream 
 // a HIP graph captured earlier still holds the old address and must be dropped, not replayed.
 // While the launch stream is being captured a slot cannot grow: the call fails instead.
 float *scratch(int slot, size_t bytes);
-constexpr int kScratchSlots = 42;
+constexpr int kScratchSlots = 44;
 // Scratch for an entry point that can do without (slots of its own): null, and nothing said, while the launch stream is
 // being captured (a graph would keep the address), on another stream than the slot's first caller (until
 // nlh_release_workspace: two streams are not ordered against each other), or above kOptionalScratch bytes, which bounds

@@ -1132,7 +1132,7 @@ extern "C" void selfref_chunkwise_forward_f32_rocm(float *mems, const float *emb
         return;
     }
     // Longer chunks have no explicit form of the shared factors to read q and y from; at every chunk size up to the
-    // limit the three launches are the faster ones (times in selfref_chain.hip).
+    // limit that file's kernels are the faster ones (times in selfref_chain.hip).
     if (C <= kLrC) {
         selfref_forward_chain({mems, embedded, y, k_cache, v_cache, q_cache, alpha_cache, theta_cache, alpha_mean_cache,
                                eta_mean_cache, frozen, seq_len, d, batch_size, C, nc, sg});

@@ -1,4 +1,4 @@
-// HOPE self-referential memory, forward for chunks of up to 64 tokens, as three launches.
+// HOPE self-referential memory, forward for chunks of up to 64 tokens, as three launches or as the same work in one.
 //
 // With the snapshot F_c of the chunk's start every memory moves by one outer product a token,
 //     M_c <- (1-a_t) M_c + th_t w_c,t k_t^T,    w_c,t = v_t - F_c k_t   (self-generated values: F_c (v_t - k_t)),
@@ -9,6 +9,7 @@
 //   selfref_chain_kernel  one workgroup per chain:               k, v, gates, snapshots of M_k, M_v
 //   selfref_scan_kernel   one workgroup per (chain, memory):     M_q, M_eta, M_alpha, M_mem chunk by chunk
 //   selfref_read_kernel   one workgroup per (chain, chunk):      q and y from the snapshots
+//   selfref_forward_kernel   all of it, the others a chunk behind the chains: where these leave compute units idle
 #include <hip/hip_runtime.h>
 
 #include <utility>
@@ -51,6 +52,31 @@ __device__ __forceinline__ void while_true(Fn &f, std::integer_sequence<int, I..
     (void)(f(std::integral_constant<int, I>{}) && ...);
 }
 
+// ── chunks handed from workgroup to workgroup ────────────────────────────────────────────────────────────────────
+// A counter for each chain, a cache line of its own, says how many of its chunks are in memory.  The writer waits for its stores in
+// every wave, meets the others at a barrier, and one wave makes them visible to the device and moves the counter.
+constexpr int kTellStride = 32, kTellChunks = 4;
+__device__ __forceinline__ void stores_arrived() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+__device__ __forceinline__ void tell(unsigned *counter, int n) {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+    __builtin_amdgcn_wave_barrier();
+    if ((threadIdx.x & 63) == 0) __hip_atomic_store(counter, (unsigned)n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// The whole workgroup, n counters of the first wave's lanes at once; what their writers stored before they told `until` is read
+// behind this.
+__device__ __forceinline__ void wait_told(const unsigned *counter, int n, int until) {
+    if (threadIdx.x < 64) {
+        const unsigned *mine = counter + ((int)threadIdx.x < n ? threadIdx.x : 0) * kTellStride;
+        while (__builtin_amdgcn_ballot_w64(__hip_atomic_load(mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < (unsigned)until))
+            __builtin_amdgcn_s_sleep(8);
+    }
+    __syncthreads();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+}
+
 // ── the recurrence ───────────────────────────────────────────────────────────────────────────────────────────────
 // Tiles of 16 tokens.  At a tile's start P0_c = M_c X^T for the whole tile comes off the matrix cores; inside the tile
 // token t adds its outer product to the later columns only, P_c[t'] = (1-a_t) P_c[t'] + th_t w_c,t (k_t . x_t') from
@@ -77,15 +103,17 @@ __device__ __forceinline__ void while_true(Fn &f, std::integer_sequence<int, I..
 //
 // Bound by the issue rate of one wave per SIMD: 820 clocks a token (120 vector and LDS instructions of the first four waves,
 // the exchange), 4000 for a tile's start and end.  64 chains of 2048 tokens, head size 64, chunks of 64: 0.92 ms, 1.26 with the
-// means in every wave; with the two kernels below 1.14 ms; one kernel that formed all products of a token with all six
+// means in every wave; with the two kernels below 1.14 ms one after the other and 0.98 beside each other; one kernel that formed all products of a token with all six
 // memories in sequence (it serves longer chunks, selfref.hip) takes 2.29 ms.  Chunks of 1, 4, 8, 16 tokens at 64 chains of
 // 512: 6.64, 2.04, 1.27, 0.88 ms there, 3.84, 1.15, 0.70, 0.47 ms with the means in every wave.
 
-template <int D, bool SG>
-__global__ __launch_bounds__(4 * D + 64) void selfref_chain_kernel(
-    float *__restrict__ mems, const float *__restrict__ emb, float *__restrict__ k_cache, float *__restrict__ v_cache,
-    float *__restrict__ alpha_cache, float *__restrict__ theta_cache, float *__restrict__ amean_cache,
-    float *__restrict__ emean_cache, float *__restrict__ frozen, int s, int C, int nc) {
+// done: with others waiting for this chain's chunks (selfref_forward_kernel), how many of them there are.
+template <int D, bool SG, bool WAITED>
+__device__ __forceinline__ void chain_of(const SelfrefForward &a, size_t b, unsigned *done) {
+    float *const mems = a.mems, *const k_cache = a.k, *const v_cache = a.v, *const alpha_cache = a.alpha, *const theta_cache = a.theta,
+                 *const amean_cache = a.amean, *const emean_cache = a.emean, *const frozen = a.frozen;
+    const float *const emb = a.emb;
+    const int s = a.s, C = a.C, nc = a.nc;
     constexpr int KT = D / 16, NW = D / 16, DD = D * D, LD = D + 16, V4 = D / 4;
     __shared__ __align__(16) float xt[2][kTB * LD];
     __shared__ __align__(16) float Kt[2][kTB * LD], Vt[2][kTB * LD];  // the tile's k, v: exchange and operand
@@ -101,7 +129,7 @@ __global__ __launch_bounds__(4 * D + 64) void selfref_chain_kernel(
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, wr = 16 * wave;
     const int ml = lane & 15, kg = lane >> 4, r = lane >> 2, cq = lane & 3;
     const int to_quad = 4 * (r + 16 * cq), to_mm = 4 * (4 * ml + kg);  // source lanes of the two permutations, in bytes
-    const size_t b = blockIdx.x, tok0 = b * (size_t)s;
+    const size_t tok0 = b * (size_t)s;
     float *mb = mems + b * 6 * DD;
 
     for (int e = tid; e < 4 * D; e += 4 * D + 64) {
@@ -128,7 +156,7 @@ __global__ __launch_bounds__(4 * D + 64) void selfref_chain_kernel(
         const float scale = row == 0 ? -1.4426950408889634f : 1.4426950408889634f;   // exp(-x) of alpha's mean, exp(x) of eta's
         __syncthreads();
         f32x4 M = *reinterpret_cast<const f32x4 *>(&mean[row][c4]);
-        int chunk_t = 0;
+        int chunk_t = 0, whole = 0, told = 0;   // chunks in front of the tile before; as the others know
         for (int tb = 0, te, buf = 0; tb < s; tb = te, buf ^= 1) {
             te = tile_end(tb);
             const int nt = te - tb;
@@ -171,6 +199,13 @@ __global__ __launch_bounds__(4 * D + 64) void selfref_chain_kernel(
                 const f32x4 m = *reinterpret_cast<const f32x4 *>(other);
                 if (t + 2 < kTB) other += row == 3 ? LD : 0;
                 lds_barrier();
+                if (WAITED && t == 0) {
+                    if (whole >= told + kTellChunks || (whole > told && whole >= nc - kTellChunks)) {
+                        told = whole;
+                        tell(done, told);
+                    }
+                    whole = tb / C;
+                }
                 // row 3: x of the next token against k, the other rows the means against u
                 const f32x4 u = *reinterpret_cast<const f32x4 *>((SG && row < 3 ? Ub : Kb) + t * LD + c4);
                 float ps = 0.f;
@@ -208,12 +243,18 @@ __global__ __launch_bounds__(4 * D + 64) void selfref_chain_kernel(
             }
 #pragma unroll
             for (int v = 0; v < 4; v++) M[v] = fmaf((float)kept, M[v], add[v]);
+            if (WAITED) stores_arrived();
             if (col < nt) {
                 const size_t o = tok0 + tb + col;
                 const float e = 1.f + __builtin_amdgcn_exp2f(mine * scale);
                 if (row == 0) { alpha_cache[o] = sigmoid_of(mine, e); amean_cache[o] = mine; }
                 if (row == 1) { theta_cache[o] = softplus_of(mine, e); emean_cache[o] = mine; }
             }
+        }
+        if (WAITED) {
+            stores_arrived();
+            lds_barrier();
+            tell(done, nc);
         }
         return;
     }
@@ -390,6 +431,8 @@ __global__ __launch_bounds__(4 * D + 64) void selfref_chain_kernel(
                 for (int v = 0; v < 4; v++) M[c][kt][v] = fmaf(kept, M[c][kt][v], add[c][kt][v]);
             }
         }
+        // What this wave stored in earlier tiles has arrived long ago; behind the next tile's first barrier that holds for all.
+        if (WAITED) stores_arrived();
         if (stt < nt) {
             const size_t o = (tok0 + tb + stt) * D + sj;
             *reinterpret_cast<float4 *>(k_cache + o) = *reinterpret_cast<const float4 *>(Kb + stt * LD + sj);
@@ -402,28 +445,40 @@ __global__ __launch_bounds__(4 * D + 64) void selfref_chain_kernel(
         for (int kt = 0; kt < KT; kt++)
             *reinterpret_cast<f32x4 *>(mb + c * DD + (wr + ml) * D + 16 * kt + 4 * kg) = M[c][kt];
     }
+    if (WAITED) {
+        stores_arrived();
+        lds_barrier();
+    }
+}
+template <int D, bool SG>
+__global__ __launch_bounds__(4 * D + 64) void selfref_chain_kernel(SelfrefForward a) {
+    chain_of<D, SG, false>(a, blockIdx.x, nullptr);
 }
 
 // ── the other memories ───────────────────────────────────────────────────────────────────────────────────────────
 // Chunk by chunk F <- A_L F + sum_s c_s (v_s - F k_s) k_s^T with c_s = th_s prod_{r>s} (1-a_r), both products on the
 // fp32 matrix cores; a wave owns 16 rows, its lane (ml, kg) row ml, columns 16 kt + 4 kg + v, which serves as operand
 // and as result.  The next chunk's k, v, gates are requested before the products of the current one.
-template <int D, bool SG>
-__global__ __launch_bounds__(4 * D) void selfref_scan_kernel(
-    float *__restrict__ mems, const float *__restrict__ k_cache, const float *__restrict__ v_cache,
-    const float *__restrict__ alpha_cache, const float *__restrict__ theta_cache, float *__restrict__ frozen, int s,
-    int C, int nc, int batch) {
+// A workgroup takes N of the four memories, the first of them number `first`.  done, mine: the chain's chunks as they come, and
+// the snapshots that this workgroup has written (selfref_forward_kernel); a chunk is then requested when it is there.
+template <int D>
+constexpr int scan_lds_floats(bool waits) { return (waits ? 1 : 2) * (2 * kLrC * (D + 4) + kLrC + 4); }
+template <int D, bool SG, int N, bool WAITS>
+__device__ __forceinline__ void scan_of(const SelfrefForward &a, size_t b, int first, float *lds, const unsigned *done, unsigned *mine) {
     constexpr int KT = D / 16, ST = kLrC / 16, DD = D * D, NT = 4 * D, LD = D + 4, V4 = D / 4;
     constexpr int LOADS = kLrC * V4 / NT;  // 4 at every D
-    __shared__ __align__(16) float Ks[2][kLrC * LD], Us[2][kLrC * LD];  // k and v (self-generated values: k - v)
-    __shared__ float cs[2][kLrC], keep_chunk[2];
+    constexpr int SET = scan_lds_floats<D>(true);
+    const float *const k_cache = a.k, *const v_cache = a.v, *const alpha_cache = a.alpha, *const theta_cache = a.theta;
+    const int s = a.s, C = a.C, nc = a.nc;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, wr = 16 * wave, ml = lane & 15, kg = lane >> 4;
-    const size_t b = blockIdx.x % batch, tok0 = b * (size_t)s;  // the four memories of a chain share an XCD's L2
-    const int comp = 2 + blockIdx.x / batch;
-    float *mb = mems + (b * 6 + comp) * DD + (wr + ml) * D + 4 * kg;
-    f32x4 F[KT];
+    const size_t tok0 = b * (size_t)s, at = (size_t)(wr + ml) * D + 4 * kg;
+    float *mb = a.mems + (b * 6 + 2 + first) * DD + at;
+    f32x4 F[N][KT];
 #pragma unroll
-    for (int kt = 0; kt < KT; kt++) F[kt] = *reinterpret_cast<const f32x4 *>(mb + 16 * kt);
+    for (int m = 0; m < N; m++) {
+#pragma unroll
+        for (int kt = 0; kt < KT; kt++) F[m][kt] = *reinterpret_cast<const f32x4 *>(mb + m * DD + 16 * kt);
+    }
 
     float4 nk[LOADS], nv[LOADS];
     float nal = 0.f, nth = 0.f;
@@ -441,12 +496,13 @@ __global__ __launch_bounds__(4 * D) void selfref_scan_kernel(
             nth = lane < L ? theta_cache[tok0 + t0 + lane] : 0.f;
         }
     };
-    auto stage = [&](int buf) {
+    auto stage = [&](float *Ks) {   // k and v (self-generated values: k - v), the products, the chunk's retention
+        float *Us = Ks + kLrC * LD, *cs = Us + kLrC * LD;
 #pragma unroll
         for (int i = 0; i < LOADS; i++) {
             const int e = tid + i * NT, li = e / V4, j = (e % V4) * 4;
-            *reinterpret_cast<float4 *>(&Ks[buf][li * LD + j]) = nk[i];
-            *reinterpret_cast<float4 *>(&Us[buf][li * LD + j]) =
+            *reinterpret_cast<float4 *>(&Ks[li * LD + j]) = nk[i];
+            *reinterpret_cast<float4 *>(&Us[li * LD + j]) =
                 SG ? make_float4(nk[i].x - nv[i].x, nk[i].y - nv[i].y, nk[i].z - nv[i].z, nk[i].w - nv[i].w) : nv[i];
         }
         if (wave == 0) {  // products of the retentions behind each token
@@ -457,77 +513,124 @@ __global__ __launch_bounds__(4 * D) void selfref_scan_kernel(
                 if (lane + off < 64) x *= y;
             }
             const float behind = __shfl_down(x, 1, 64);
-            cs[buf][lane] = nth * (lane < 63 ? behind : 1.f);
-            if (lane == 0) keep_chunk[buf] = x;
+            cs[lane] = nth * (lane < 63 ? behind : 1.f);
+            if (lane == 0) cs[kLrC] = x;
         }
     };
-    request(0);
-    stage(0);
-    __syncthreads();
+    auto snapshot = [&](int ci) {
+        float *fb = a.frozen + ((b * nc + ci) * 6 + 2 + first) * (size_t)DD + at;
+#pragma unroll
+        for (int m = 0; m < N; m++) {
+#pragma unroll
+            for (int kt = 0; kt < KT; kt++) *reinterpret_cast<f32x4 *>(fb + m * DD + 16 * kt) = F[m][kt];
+        }
+    };
+    if (!WAITS) {
+        request(0);
+        stage(lds);
+        __syncthreads();
+    }
     for (int ci = 0; ci < nc; ci++) {
-        const int buf = ci & 1, L = min(C, s - ci * C);
-        if (ci + 1 < nc) request(ci + 1);
-        float *fb = frozen + ((b * nc + ci) * 6 + comp) * (size_t)DD + (wr + ml) * D + 4 * kg;
-#pragma unroll
-        for (int kt = 0; kt < KT; kt++) *reinterpret_cast<f32x4 *>(fb + 16 * kt) = F[kt];
-        const float *K = Ks[buf], *U = Us[buf];
-        f32x4 w[ST], N[KT], a[2][ST];
-        const float keep = keep_chunk[buf];
+        const int L = min(C, s - ci * C);
+        float *const K = lds + (WAITS ? 0 : ci & 1) * SET, *const U = K + kLrC * LD, *const cs = U + kLrC * LD;
+        snapshot(ci);
+        if (WAITS) {
+            stores_arrived();
+            wait_told(done, 1, ci + 1);   // everybody's snapshot has arrived
+            if (wave == 0) tell(mine, ci + 1);
+            request(ci);
+            stage(K);
+            __syncthreads();
+        } else if (ci + 1 < nc) {
+            request(ci + 1);
+        }
+        const float keep = cs[kLrC];
         // Tiles behind the chunk's last token hold zeros.  Operands are read one step ahead: left to the compiler, every
-        // read stands right before its use.
-        auto read_w = [&](int kt, int p) __attribute__((always_inline)) {
+        // read stands right before its use.  M memories at a time, so that their sums fit the registers.
+        constexpr int M = N > 2 ? 2 : N;
 #pragma unroll
-            for (int st = 0; st < ST; st++)
-                a[p][st] = *reinterpret_cast<const f32x4 *>((SG ? U : K) + (16 * st + ml) * LD + 16 * kt + 4 * kg);
-        };
-        float kb[2][KT];
-        auto read_n = [&](int i, int p) __attribute__((always_inline)) {
+        for (int m0 = 0; m0 < N; m0 += M) {
+            f32x4 w[M][ST], S[M][KT], x[2][ST];
+            auto read_w = [&](int kt, int p) __attribute__((always_inline)) {
 #pragma unroll
-            for (int kt = 0; kt < KT; kt++) kb[p][kt] = K[(16 * (i >> 2) + 4 * kg + (i & 3)) * LD + 16 * kt + ml];
-        };
-        read_w(0, 0);
+                for (int st = 0; st < ST; st++)
+                    x[p][st] = *reinterpret_cast<const f32x4 *>((SG ? U : K) + (16 * st + ml) * LD + 16 * kt + 4 * kg);
+            };
+            float kb[2][KT];
+            auto read_n = [&](int i, int p) __attribute__((always_inline)) {
 #pragma unroll
-        for (int st = 0; st < ST; st++) w[st] = f32x4{0.f, 0.f, 0.f, 0.f};
+                for (int kt = 0; kt < KT; kt++) kb[p][kt] = K[(16 * (i >> 2) + 4 * kg + (i & 3)) * LD + 16 * kt + ml];
+            };
+            read_w(0, 0);
 #pragma unroll
-        for (int kt = 0; kt < KT; kt++) {
-            N[kt] = f32x4{0.f, 0.f, 0.f, 0.f};   // the chunk's sum by itself: F rounds once a chunk
-            if (kt + 1 < KT) read_w(kt + 1, (kt + 1) & 1);
-            else read_n(0, 0);
-            __builtin_amdgcn_sched_barrier(0);
+            for (int m = 0; m < M; m++) {
 #pragma unroll
-            for (int v = 0; v < 4; v++) {
-#pragma unroll
-                for (int st = 0; st < ST; st++) w[st] = mfma4(a[kt & 1][st][v], F[kt][v], w[st]);
+                for (int st = 0; st < ST; st++) w[m][st] = f32x4{0.f, 0.f, 0.f, 0.f};
             }
-            __builtin_amdgcn_sched_barrier(0);
-        }
 #pragma unroll
-        for (int st = 0; st < ST; st++) {
+            for (int kt = 0; kt < KT; kt++) {
+                if (kt + 1 < KT) read_w(kt + 1, (kt + 1) & 1);
+                else read_n(0, 0);
+                __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int v = 0; v < 4; v++) {
-                const int t = 16 * st + 4 * kg + v;
-                w[st][v] = cs[buf][t] * ((SG ? 0.f : U[t * LD + wr + ml]) - w[st][v]);
+                for (int v = 0; v < 4; v++) {
+#pragma unroll
+                    for (int m = 0; m < M; m++) {
+#pragma unroll
+                        for (int st = 0; st < ST; st++) w[m][st] = mfma4(x[kt & 1][st][v], F[m0 + m][kt][v], w[m][st]);
+                    }
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+            for (int m = 0; m < M; m++) {
+#pragma unroll
+                for (int kt = 0; kt < KT; kt++) S[m][kt] = f32x4{0.f, 0.f, 0.f, 0.f};   // the chunk's sum by itself: F rounds once a chunk
+            }
+#pragma unroll
+            for (int st = 0; st < ST; st++) {
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    const int t = 16 * st + 4 * kg + v;
+#pragma unroll
+                    for (int m = 0; m < M; m++) w[m][st][v] = cs[t] * ((SG ? 0.f : U[t * LD + wr + ml]) - w[m][st][v]);
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < 4 * ST; i++) {
+                if (16 * (i >> 2) >= L) break;
+                if (i + 1 < 4 * ST) read_n(i + 1, (i + 1) & 1);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int m = 0; m < M; m++) {
+#pragma unroll
+                    for (int kt = 0; kt < KT; kt++) S[m][kt] = mfma4(kb[i & 1][kt], w[m][i >> 2][i & 3], S[m][kt]);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+            for (int m = 0; m < M; m++) {
+#pragma unroll
+                for (int kt = 0; kt < KT; kt++) {
+#pragma unroll
+                    for (int v = 0; v < 4; v++) F[m0 + m][kt][v] = fmaf(keep, F[m0 + m][kt][v], S[m][kt][v]);
+                }
             }
         }
-#pragma unroll
-        for (int i = 0; i < 4 * ST; i++) {
-            if (16 * (i >> 2) >= L) break;
-            if (i + 1 < 4 * ST) read_n(i + 1, (i + 1) & 1);
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int kt = 0; kt < KT; kt++) N[kt] = mfma4(kb[i & 1][kt], w[i >> 2][i & 3], N[kt]);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-#pragma unroll
-        for (int kt = 0; kt < KT; kt++) {
-#pragma unroll
-            for (int v = 0; v < 4; v++) F[kt][v] = fmaf(keep, F[kt][v], N[kt][v]);
-        }
-        if (ci + 1 < nc) stage(buf ^ 1);
+        if (!WAITS && ci + 1 < nc) stage(lds + ((ci + 1) & 1) * SET);
         __syncthreads();
     }
 #pragma unroll
-    for (int kt = 0; kt < KT; kt++) *reinterpret_cast<f32x4 *>(mb + 16 * kt) = F[kt];
+    for (int m = 0; m < N; m++) {
+#pragma unroll
+        for (int kt = 0; kt < KT; kt++) *reinterpret_cast<f32x4 *>(mb + m * DD + 16 * kt) = F[m][kt];
+    }
+}
+template <int D, bool SG>
+__global__ __launch_bounds__(4 * D) void selfref_scan_kernel(SelfrefForward a) {
+    __shared__ __align__(16) float lds[scan_lds_floats<D>(false)];
+    // the four memories of a chain share an XCD's L2
+    scan_of<D, SG, 1, false>(a, blockIdx.x % a.batch, blockIdx.x / a.batch, lds, nullptr, nullptr);
 }
 
 // ── reads ────────────────────────────────────────────────────────────────────────────────────────────────────────
@@ -536,31 +639,33 @@ __global__ __launch_bounds__(4 * D) void selfref_scan_kernel(
 // scaled, are the operand of G and H at once; its rows change layout through its own 16 rows of LDS without a barrier.
 // 116 us for 2048 chunks of 64 at head size 64, two workgroups per compute unit; 40 are matrix instructions, the rest the
 // tables at a chunk's start and the four waves' unequal numbers of earlier tokens.
+template <int D>
+constexpr int read_lds_floats() { return chunk_lds_floats<D>(0) + D / 16 * kTB * kWL; }
 template <int D, bool SG>
-__global__ __launch_bounds__(4 * D) void selfref_read_kernel(
-    const float *__restrict__ emb, const float *__restrict__ k_cache, const float *__restrict__ v_cache,
-    const float *__restrict__ alpha_cache, const float *__restrict__ theta_cache, const float *__restrict__ frozen,
-    float *__restrict__ q_cache, float *__restrict__ y, int s, int C, int nc) {
+__device__ __forceinline__ void read_of(const SelfrefForward &a, size_t b, int ci, float *chunk_lds) {
+    const float *const emb = a.emb, *const frozen = a.frozen;
+    float *const q_cache = a.q, *const y = a.y;
+    const int s = a.s, C = a.C, nc = a.nc;
     constexpr int KT = D / 16, NW = D / 16, DD = D * D, KL = D + 4;
-    extern __shared__ __align__(16) float chunk_lds[];
     const ChunkLds<D> m(chunk_lds);
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, ml = lane & 15, kg = lane >> 4;
+    int tid = threadIdx.x;   // an opaque copy: addresses made of it are not to live across the chunks of a workgroup
+    asm volatile("" : "+v"(tid));
+    const int wave = tid >> 6, lane = tid & 63, ml = lane & 15, kg = lane >> 4;
     float *row = m.tiles + wave * kTB * kWL;  // the wave's rows
-    const int ci = blockIdx.x % nc;
-    const size_t b = blockIdx.x / nc, chunk = blockIdx.x, tok0 = b * (size_t)s;
+    const size_t chunk = b * nc + ci, tok0 = b * (size_t)s;
     const int t0 = ci * C, L = min(C, s - t0);
-    chunk_setup<D, SG>(m, k_cache, v_cache, alpha_cache, theta_cache, tok0, t0, L, tid);
+    chunk_setup<D, SG>(m, a.k, a.v, a.alpha, a.theta, tok0, t0, L, tid);
     const float *UC = SG ? m.XC : m.KC;
 
     for (int tile = wave; tile * kTB < L; tile += NW) {
         const int li0 = tile * kTB, nt = min(kTB, L - li0);
         const size_t o0 = (tok0 + t0 + li0) * D;
-        f32x4 a[KT], in[KT];  // the read's argument: as operand, and row 4 kg + v, column 16 jt + ml
+        f32x4 op[KT], in[KT];  // the read's argument: as operand, and row 4 kg + v, column 16 jt + ml
 #pragma unroll
         for (int kt = 0; kt < KT; kt++) {
-            a[kt] = ml < nt ? *reinterpret_cast<const f32x4 *>(emb + o0 + (size_t)ml * D + 16 * kt + 4 * kg)
+            op[kt] = ml < nt ? *reinterpret_cast<const f32x4 *>(emb + o0 + (size_t)ml * D + 16 * kt + 4 * kg)
                             : f32x4{0.f, 0.f, 0.f, 0.f};
-            *reinterpret_cast<f32x4 *>(row + ml * kWL + 16 * kt + 4 * kg) = a[kt];
+            *reinterpret_cast<f32x4 *>(row + ml * kWL + 16 * kt + 4 * kg) = op[kt];
         }
         __builtin_amdgcn_wave_barrier();
 #pragma unroll
@@ -578,7 +683,7 @@ __global__ __launch_bounds__(4 * D) void selfref_read_kernel(
                 for (int kt = 0; kt < KT; kt++) {
                     const f32x4 kk = *reinterpret_cast<const f32x4 *>(m.KC + (16 * st + ml) * KL + 16 * kt + 4 * kg);
 #pragma unroll
-                    for (int v = 0; v < 4; v++) acc = mfma4(a[kt][v], kk[v], acc);
+                    for (int v = 0; v < 4; v++) acc = mfma4(op[kt][v], kk[v], acc);
                 }
 #pragma unroll
                 for (int v = 0; v < 4; v++) {
@@ -613,7 +718,7 @@ __global__ __launch_bounds__(4 * D) void selfref_read_kernel(
             }
             __builtin_amdgcn_wave_barrier();
 #pragma unroll
-            for (int kt = 0; kt < KT; kt++) a[kt] = *reinterpret_cast<const f32x4 *>(row + ml * kWL + 16 * kt + 4 * kg);
+            for (int kt = 0; kt < KT; kt++) op[kt] = *reinterpret_cast<const f32x4 *>(row + ml * kWL + 16 * kt + 4 * kg);
             f32x4 f[2][KT];  // the next 16 rows of the snapshot are requested before the products of the current ones
             auto request = [&](int jt, int w) __attribute__((always_inline)) {
 #pragma unroll
@@ -628,7 +733,7 @@ __global__ __launch_bounds__(4 * D) void selfref_read_kernel(
 #pragma unroll
                 for (int kt = 0; kt < KT; kt++) {
 #pragma unroll
-                    for (int v = 0; v < 4; v++) h[jt] = mfma4(a[kt][v], f[jt & 1][kt][v], h[jt]);
+                    for (int v = 0; v < 4; v++) h[jt] = mfma4(op[kt][v], f[jt & 1][kt][v], h[jt]);
                 }
                 float *dst = pass ? y : q_cache;
 #pragma unroll
@@ -647,7 +752,7 @@ __global__ __launch_bounds__(4 * D) void selfref_read_kernel(
                 __builtin_amdgcn_wave_barrier();
 #pragma unroll
                 for (int kt = 0; kt < KT; kt++)
-                    a[kt] = *reinterpret_cast<const f32x4 *>(row + ml * kWL + 16 * kt + 4 * kg);
+                    op[kt] = *reinterpret_cast<const f32x4 *>(row + ml * kWL + 16 * kt + 4 * kg);
             }
         }
         __builtin_amdgcn_wave_barrier();
@@ -655,19 +760,97 @@ __global__ __launch_bounds__(4 * D) void selfref_read_kernel(
 }
 
 template <int D, bool SG>
+__global__ __launch_bounds__(4 * D) void selfref_read_kernel(SelfrefForward a) {
+    extern __shared__ __align__(16) float lds[];
+    read_of<D, SG>(a, blockIdx.x / a.nc, blockIdx.x % a.nc, lds);
+}
+
+// ── all three at once ────────────────────────────────────────────────────────────────────────────────────────────
+// The chains leave most of the compute units idle and are followed by nothing but what hangs off their finished chunks.  So one
+// launch has workgroups for the chains, for the other memories of each chain, which follow it chunk by chunk, and for the reads, which
+// take the chunks in the order in which they are finished.  A workgroup waits only for those that started before it: what it does
+// follows from the number it draws when it starts, chains first, and a chain waits for nobody, so every wait ends whatever part of
+// the grid is resident.  The LDS keeps a chain's compute unit to itself.
+// 64 chains of 2048 tokens, head size 64, chunks of 64: 0.98 ms; the chains by themselves 0.92, telling of their chunks 0.01, their
+// company 0.03, and what follows the last chunk 0.02 (the three launches: 0.91 + 0.11 + 0.12).
+__global__ void selfref_counters_kernel(unsigned *counters, int n) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < n) counters[i] = 0;
+}
+constexpr int kAloneFloats = 81 * 256;   // more than half of a compute unit's LDS
+template <int D, bool SG, int N>
+__global__ __launch_bounds__(4 * D + 64) void selfref_forward_kernel(SelfrefForward a, unsigned *counters, int readers) {
+    extern __shared__ __align__(16) float lds[];
+    __shared__ int drawn;
+    if (threadIdx.x == 0) drawn = (int)__hip_atomic_fetch_add(counters, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    const int role = __builtin_amdgcn_readfirstlane(drawn);
+    constexpr int PARTS = 4 / N;   // workgroups for a chain's other memories; its counters: the chain's own, then theirs
+    auto counters_of = [&](size_t b) { return counters + (1 + b * (1 + PARTS)) * kTellStride; };
+    if (role < a.batch) {
+        chain_of<D, SG, true>(a, role, counters_of(role));
+        return;
+    }
+    if (threadIdx.x >= 4 * D) return;
+    const int followers = a.batch * (1 + PARTS);
+    if (role < followers) {
+        const size_t b = role % a.batch;
+        const int part = role / a.batch - 1;
+        scan_of<D, SG, N, true>(a, b, part * N, lds, counters_of(b), counters_of(b) + (1 + part) * kTellStride);
+        return;
+    }
+    for (int task = role - followers; task < a.batch * a.nc; task += readers) {
+        const int ci = task / a.batch;
+        const size_t b = task % a.batch;
+        wait_told(counters_of(b), 1 + PARTS, ci + 1);
+        read_of<D, SG>(a, b, ci, lds);
+        __syncthreads();   // the chunk's LDS is free
+    }
+}
+template <int D, bool SG, int N>
+bool launch_together(const SelfrefForward &a) {
+    const int n = (1 + (1 + 4 / N) * a.batch) * kTellStride, followers = (1 + 4 / N) * a.batch;
+    unsigned *counters = reinterpret_cast<unsigned *>(scratch_if_free(42, n * sizeof(unsigned)));
+    if (!counters) return false;
+    constexpr int most = scan_lds_floats<D>(true) > read_lds_floats<D>() ? scan_lds_floats<D>(true) : read_lds_floats<D>();
+    constexpr size_t lds = (most > kAloneFloats ? most : kAloneFloats) * sizeof(float);
+    const long long tasks = (long long)a.batch * a.nc, rest = compute_units() - followers;
+    const int readers = (int)(tasks < rest ? tasks : rest);
+    hipLaunchKernelGGL(selfref_counters_kernel, dim3(ceil_div(n, 256)), dim3(256), 0, stream(), counters, n);
+    check_launch("selfref_counters_kernel");
+    check_hip(hipFuncSetAttribute(reinterpret_cast<const void *>(selfref_forward_kernel<D, SG, N>),
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds), "dynamic LDS size");
+    KernelTimer kt("selfref_forward_kernel");
+    hipLaunchKernelGGL((selfref_forward_kernel<D, SG, N>), dim3(followers + readers), dim3(4 * D + 64), lds, stream(), a, counters, readers);
+    check_launch("selfref_forward_kernel");
+    return true;
+}
+
+template <int D, bool SG>
 void launch(const SelfrefForward &a) {
+    // Together where compute units stay idle beside the chains and those that follow them keep up with them: the other memories
+    // take 10 us a chunk of any length, a chain 7 us for 16 tokens.  64 chains of 512 tokens, head size 64, three launches / one:
+    // chunks of 8 0.57 / 0.73 ms, of 16 0.38 / 0.41, of 32 0.326 / 0.306, of 64 0.299 / 0.277; 4 chains of 100 tokens 82 / 75 us.
+    // As many workgroups for a chain's other memories as leave most of the chip to the reads, which are the slower ones.
+    const int cus = compute_units();
+    if (a.nc > 1 && a.C >= 2 * kTB && 4 * a.batch <= cus) {
+        if (16 * a.batch <= cus   ? launch_together<D, SG, 1>(a)
+            : 8 * a.batch <= cus ? launch_together<D, SG, 2>(a)
+                                 : launch_together<D, SG, 4>(a))
+            return;
+    }
     const dim3 block(4 * D);
-    hipLaunchKernelGGL((selfref_chain_kernel<D, SG>), dim3(a.batch), dim3(4 * D + 64), 0, stream(), a.mems, a.emb, a.k, a.v, a.alpha,
-                       a.theta, a.amean, a.emean, a.frozen, a.s, a.C, a.nc);
+    {
+        KernelTimer kt("selfref_chain_kernel");
+        hipLaunchKernelGGL((selfref_chain_kernel<D, SG>), dim3(a.batch), dim3(4 * D + 64), 0, stream(), a);
+    }
     check_launch("selfref_chain_kernel");
-    hipLaunchKernelGGL((selfref_scan_kernel<D, SG>), dim3(4 * a.batch), block, 0, stream(), a.mems, a.k, a.v, a.alpha,
-                       a.theta, a.frozen, a.s, a.C, a.nc, a.batch);
+    hipLaunchKernelGGL((selfref_scan_kernel<D, SG>), dim3(4 * a.batch), block, 0, stream(), a);
     check_launch("selfref_scan_kernel");
-    const size_t lds = (chunk_lds_floats<D>(0) + D / 16 * kTB * kWL) * sizeof(float);
+    const size_t lds = read_lds_floats<D>() * sizeof(float);
     check_hip(hipFuncSetAttribute(reinterpret_cast<const void *>(selfref_read_kernel<D, SG>),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds), "dynamic LDS size");
-    hipLaunchKernelGGL((selfref_read_kernel<D, SG>), dim3(a.batch * a.nc), block, lds, stream(), a.emb, a.k, a.v, a.alpha,
-                       a.theta, a.frozen, a.q, a.y, a.s, a.C, a.nc);
+    hipLaunchKernelGGL((selfref_read_kernel<D, SG>), dim3(a.batch * a.nc), block, lds, stream(), a);
     check_launch("selfref_read_kernel");
 }
 

@@ -106,7 +106,7 @@ template <int D>
 constexpr int chunk_lds_floats(int tiles) { return 2 * kLrC * (D + 4) + kLrC * kLrC + kTB * kWL + 5 * kLrC + tiles * kTB * (D + 4); }
 
 // Forward for chunks of up to kLrC tokens at head sizes 16, 32 and 64; arguments as in
-// selfref_chunkwise_forward_f32_rocm, nc chunks of C tokens.  Takes no scratch memory.
+// selfref_chunkwise_forward_f32_rocm, nc chunks of C tokens.  Scratch memory only where it is free to take.
 struct SelfrefForward {
     float *mems;
     const float *emb;

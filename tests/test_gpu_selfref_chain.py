@@ -1,10 +1,15 @@
 """The chain-resident forward of the self-referential memory (chunks of up to 64 tokens) at the edges of its 16-token
 tiles: chunks one token short of, at and behind a tile's end, last chunks of one token, every head size, both value
 modes, against the float32 oracle; gradients against the float64 oracle (1e-4, fp32 sums over a chain)."""
+import ctypes
+
 import numpy as np
 import pytest
+import torch
 
+from nl_hecate_amd.ffi import lib
 from tests.gpu_util import assert_close
+from tests.test_gpu_exact_mm import kernels_run
 from tests.test_gpu_selfref import gpu_run, inputs, oracle_run
 
 pytestmark = pytest.mark.gpu
@@ -89,3 +94,53 @@ def test_row_means_and_retentions_keep_their_float64_parts(C, sg):
     ratio = {n: round(float(np.exp(np.mean(e))), 2) for n, e in log.items()}
     print(sg, C, ratio)
     assert max(ratio["alpha"], ratio["theta"], ratio["k"]) <= 0.7 and ratio["y"] <= 0.85, ratio
+
+
+@pytest.fixture
+def side_stream():
+    """Launches on a second stream: the scratch that the kernels in one launch want belongs to the first."""
+    side = torch.cuda.Stream()
+
+    def run(call):
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            lib.nlh_set_stream(ctypes.c_void_p(side.cuda_stream))
+            try:
+                return call()
+            finally:
+                lib.nlh_set_stream(None)
+
+    lib.nlh_release_workspace()
+    yield run
+    lib.nlh_set_stream(None)
+    lib.nlh_release_workspace()
+
+
+# chains at the limits of the rules (a launch for all up to a quarter of the compute units, more workgroups a chain up to an
+# eighth and a sixteenth), chunks at the limit, last chunks of one token and of a partial tile, more chunks than readers
+@pytest.mark.parametrize("B,s,C", [(1, 65, 64), (2, 33, 32), (16, 100, 33), (17, 129, 64), (32, 200, 48), (33, 161, 32),
+                                   (64, 200, 64), (64, 610, 32), (65, 130, 64), (3, 1000, 64), (2, 64, 16)])
+@pytest.mark.parametrize("d", [16, 32, 64])
+@pytest.mark.parametrize("sg", [True, False])
+def test_in_one_launch_and_one_after_the_other(side_stream, B, s, C, d, sg):
+    mems, x, dy = inputs(B, s, d, seed=s * 100 + C + d)
+    print(f"selfref together B={B} s={s} d={d} C={C} sg={sg}", flush=True)
+    got = gpu_run(mems, x, dy, C, sg)
+    for i in range(2):   # the second run finds the counters of the first
+        again = gpu_run(mems, x, dy, C, sg)
+        assert all(np.array_equal(got[n], again[n]) for n in got)
+    apart = side_stream(lambda: gpu_run(mems, x, dy, C, sg))
+    for n in got:
+        assert np.array_equal(got[n], apart[n]), n
+
+
+def test_which_calls_run_in_one_launch(side_stream):
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    for B, s, C, one in ((2, 65, 64, True), (cus // 4, 65, 64, True), (cus // 4 + 1, 65, 64, False), (2, 65, 32, True),
+                         (2, 65, 31, False), (2, 64, 64, False)):
+        a = inputs(B, s, 16, seed=1)
+        ran = kernels_run(lambda: gpu_run(*a, C, True))
+        assert ("selfref_forward_kernel" in ran) == one and ("selfref_chain_kernel" in ran) != one, (B, s, C)
+    a = inputs(2, 130, 64, seed=2)
+    gpu_run(*a, 64, True)
+    assert "selfref_chain_kernel" in side_stream(lambda: kernels_run(lambda: gpu_run(*a, 64, True)))
