@@ -246,56 +246,6 @@ __global__ __launch_bounds__(4 * D) void selfref_fwd_kernel(
 // Staged tile arrays, [kTB][D] floats each.
 enum { A_K = 0, A_V, A_Q, A_X, A_DY, A_G, A_P, A_DQ, A_DP, A_DG, A_DH, A_HX, A_HQ, A_COUNT };
 
-// out_t = [A_t a1_t] + sum_{s<t} c_ts R_s ([l2_s . a2_t] - [l1_s . a1_t]) for the tokens of one tile, written
-// to dst[tt * dst_stride + j]; t = li0 + tt is the token's index in its chunk, the a1 terms exist with
-// HAS1, the a2 term with HAS2.  With L1 = u, R = k this is G_t^T a1 (plus H_t^T a2 for L2 = v); with
-// L1 = k, R = u it is G_t a1; with L2 = k, R = v it is H_t a2.  Two products on the fp32 matrix cores:
-// S = a2 L2^T - a1 L1^T (tokens x earlier tokens; wave w takes the earlier tokens 16 w ..), masked and
-// scaled by c into Wt, then Wt R (wave w takes columns 16 w ..).  Tile rows have stride TL, the chunk
-// arrays KL, Wt kWL (all = 4 mod 64, so the operand reads of a wave fall on 64 banks).  Rows of the
-// chunk arrays behind the chunk's last token are read (times zero) and must be finite.  Called by
-// every thread of the workgroup; one barrier inside, the caller synchronises before Wt, the tile or
-// dst (when it is in LDS) are touched again.
-template <int D, bool HAS1, bool HAS2>
-__device__ __forceinline__ void lowrank_tile(const float *a1, const float *L1, const float *a2, const float *L2,
-                                             const float *R, int li0, int nt, const float *CT, const float *cA,
-                                             float *Wt, float *dst, size_t dst_stride, int tid) {
-    constexpr int TL = D + 4, KL = D + 4, NW = D / 16;
-    const int lane = tid & 63, wave = tid >> 6, ml = lane & 15, kg = lane >> 4;
-    const int nprev = li0 + nt - 1;  // earlier tokens any token of the tile sees
-    for (int st = wave; st < kLrC / 16; st += NW) {
-        f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
-        if (16 * st < nprev) {
-#pragma unroll
-            for (int k0 = 0; k0 < D; k0 += 4) {
-                if (HAS1)
-                    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(-a1[ml * TL + k0 + kg],
-                                                               L1[(16 * st + ml) * KL + k0 + kg], acc, 0, 0, 0);
-                if (HAS2)
-                    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a2[ml * TL + k0 + kg],
-                                                               L2[(16 * st + ml) * KL + k0 + kg], acc, 0, 0, 0);
-            }
-        }
-#pragma unroll
-        for (int v = 0; v < 4; v++) {
-            const int tt = 4 * kg + v, li = li0 + tt, s1 = 16 * st + ml;
-            Wt[tt * kWL + s1] = (tt < nt && s1 < li) ? CT[li * kLrC + s1] * acc[v] : 0.f;
-        }
-    }
-    __syncthreads();
-    f32x4 o = f32x4{0.f, 0.f, 0.f, 0.f};
-    // all of Wt's columns: those behind the tile's last token are zero, and a fixed trip count lets the
-    // operand reads of the whole product be issued ahead of the first matrix instruction
-#pragma unroll
-    for (int k0 = 0; k0 < kLrC; k0 += 4)
-        o = __builtin_amdgcn_mfma_f32_16x16x4f32(Wt[ml * kWL + k0 + kg], R[(k0 + kg) * KL + 16 * wave + ml], o, 0, 0, 0);
-#pragma unroll
-    for (int v = 0; v < 4; v++) {
-        const int tt = 4 * kg + v, j = 16 * wave + ml;
-        if (tt < nt) dst[(size_t)tt * dst_stride + j] = HAS1 ? fmaf(cA[li0 + tt], a1[tt * TL + j], o[v]) : o[v];
-    }
-}
-
 // Chunk-parallel first pass of the backward (chunks of up to kLrC tokens): one workgroup per
 // (chain, chunk), without self-generated values (with them: selfref_sweep.hip).  Per token g = G x, p = G q,
 // dp = F_mem^T dy, dq = G^T dp + H^T dy, H x, H q into rp [B, s, RS, D]; per chunk the transposed F_k, F_v, F_q
@@ -425,35 +375,12 @@ __global__ __launch_bounds__(4 * D) void selfref_bwd_chunks_kernel(
     }
 }
 
-// Chunk-parallel last pass on the same path: d_x_t = G_t^T dg_t + H_t^T dh_t, in place on d_emb, which
-// holds dg [B, s, D] on entry (dh likewise in its own buffer without self-generated values).
 template <int D, bool SG>
 __global__ __launch_bounds__(4 * D) void selfref_bwd_dx_kernel(
     const float *__restrict__ k_cache, const float *__restrict__ v_cache, const float *__restrict__ alpha_cache,
     const float *__restrict__ theta_cache, float *d_emb, const float *__restrict__ dh, int s, int C, int nc) {
-    constexpr int V4 = D / 4, TL = D + 4;
     extern __shared__ __align__(16) float chunk_lds[];
-    const ChunkLds<D> m(chunk_lds);
-    float *tDG = m.tiles, *tDH = tDG + kTB * TL;
-    const int tid = threadIdx.x;
-    const int ci = blockIdx.x % nc;
-    const size_t b = blockIdx.x / nc, tok0 = b * (size_t)s;
-    const int t0 = ci * C, L = min(C, s - t0);
-    chunk_setup<D, SG>(m, k_cache, v_cache, alpha_cache, theta_cache, tok0, t0, L, tid);
-    const int stt = tid / V4, sj = (tid % V4) * 4;
-    const int ntile = (L + kTB - 1) / kTB;
-    for (int tile = 0; tile < ntile; tile++) {
-        const int tb = t0 + tile * kTB, nt = min(kTB, t0 + L - tb);
-        __syncthreads();
-        if (stt < nt) {
-            const size_t o = (tok0 + tb + stt) * D + sj;
-            *reinterpret_cast<float4 *>(tDG + stt * TL + sj) = *reinterpret_cast<const float4 *>(d_emb + o);
-            if (!SG) *reinterpret_cast<float4 *>(tDH + stt * TL + sj) = *reinterpret_cast<const float4 *>(dh + o);
-        }
-        __syncthreads();
-        lowrank_tile<D, true, !SG>(tDG, SG ? m.XC : m.KC, tDH, m.XC, m.KC, tb - t0, nt, m.CT, m.cA, m.Wt,
-                                   d_emb + (tok0 + tb) * D, (size_t)D, tid);
-    }
+    dx_of_chunk<D, SG>(chunk_lds, k_cache, v_cache, alpha_cache, theta_cache, d_emb, dh, blockIdx.x / nc, blockIdx.x % nc, s, C, [] {});
 }
 
 template <int D, bool SG, bool LR>
@@ -1068,8 +995,9 @@ void launch_bwd_sg(const BwdArgs &a) {
     if (a.lowrank) {
         const size_t lds3 = chunk_lds_floats<D>(2) * sizeof(float);
         if constexpr (SG) {
-            selfref_backward_sweep({a.emb, a.dy, a.kc, a.vc, a.qc, a.al, a.th, a.am, a.em, a.frozen, a.d_emb, a.d_mems,
-                                    a.gtraj, a.rp, a.ftt, a.csv, a.s, D, a.batch, a.C, a.nc});
+            if (selfref_backward_sweep({a.emb, a.dy, a.kc, a.vc, a.qc, a.al, a.th, a.am, a.em, a.frozen, a.d_emb, a.d_mems,
+                                    a.gtraj, a.rp, a.ftt, a.csv, a.s, D, a.batch, a.C, a.nc}))
+                return;
         } else {
             const size_t lds1 = chunk_lds_floats<D>(4) * sizeof(float);
             set_lds(selfref_bwd_chunks_kernel<D>, lds1);

@@ -15,6 +15,7 @@
 #include <utility>
 
 #include "../../include/nl_hecate_ffi.h"
+#include "handover.h"
 #include "lane_ops.h"
 #include "quad_rows.h"
 #include "runtime.h"
@@ -50,31 +51,6 @@ __device__ __forceinline__ void wave_lds_fence() { asm volatile("" ::: "memory")
 template <class Fn, int... I>
 __device__ __forceinline__ void while_true(Fn &f, std::integer_sequence<int, I...>) {
     (void)(f(std::integral_constant<int, I>{}) && ...);
-}
-
-// ── chunks handed from workgroup to workgroup ────────────────────────────────────────────────────────────────────
-// A counter for each chain, a cache line of its own, says how many of its chunks are in memory.  The writer waits for its stores in
-// every wave, meets the others at a barrier, and one wave makes them visible to the device and moves the counter.
-constexpr int kTellStride = 32, kTellChunks = 4;
-__device__ __forceinline__ void stores_arrived() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-}
-__device__ __forceinline__ void tell(unsigned *counter, int n) {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-    __builtin_amdgcn_wave_barrier();
-    if ((threadIdx.x & 63) == 0) __hip_atomic_store(counter, (unsigned)n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-// The whole workgroup, n counters of the first wave's lanes at once; what their writers stored before they told `until` is read
-// behind this.
-__device__ __forceinline__ void wait_told(const unsigned *counter, int n, int until) {
-    if (threadIdx.x < 64) {
-        const unsigned *mine = counter + ((int)threadIdx.x < n ? threadIdx.x : 0) * kTellStride;
-        while (__builtin_amdgcn_ballot_w64(__hip_atomic_load(mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < (unsigned)until))
-            __builtin_amdgcn_s_sleep(8);
-    }
-    __syncthreads();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
 }
 
 // ── the recurrence ───────────────────────────────────────────────────────────────────────────────────────────────
@@ -773,20 +749,12 @@ __global__ __launch_bounds__(4 * D) void selfref_read_kernel(SelfrefForward a) {
 // the grid is resident.  The LDS keeps a chain's compute unit to itself.
 // 64 chains of 2048 tokens, head size 64, chunks of 64: 0.98 ms; the chains by themselves 0.92, telling of their chunks 0.01, their
 // company 0.03, and what follows the last chunk 0.02 (the three launches: 0.91 + 0.11 + 0.12).
-__global__ void selfref_counters_kernel(unsigned *counters, int n) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i < n) counters[i] = 0;
-}
-constexpr int kAloneFloats = 81 * 256;   // more than half of a compute unit's LDS
 template <int D, bool SG, int N>
-__global__ __launch_bounds__(4 * D + 64) void selfref_forward_kernel(SelfrefForward a, unsigned *counters, int readers) {
+__global__ __launch_bounds__(4 * D + 64) void selfref_forward_kernel(SelfrefForward a, unsigned *counters) {
     extern __shared__ __align__(16) float lds[];
-    __shared__ int drawn;
-    if (threadIdx.x == 0) drawn = (int)__hip_atomic_fetch_add(counters, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __syncthreads();
-    const int role = __builtin_amdgcn_readfirstlane(drawn);
+    const int role = draw(counters);
     constexpr int PARTS = 4 / N;   // workgroups for a chain's other memories; its counters: the chain's own, then theirs
-    auto counters_of = [&](size_t b) { return counters + (1 + b * (1 + PARTS)) * kTellStride; };
+    auto counters_of = [&](size_t b) { return counters + (2 + b * (1 + PARTS)) * kTellStride; };
     if (role < a.batch) {
         chain_of<D, SG, true>(a, role, counters_of(role));
         return;
@@ -799,7 +767,7 @@ __global__ __launch_bounds__(4 * D + 64) void selfref_forward_kernel(SelfrefForw
         scan_of<D, SG, N, true>(a, b, part * N, lds, counters_of(b), counters_of(b) + (1 + part) * kTellStride);
         return;
     }
-    for (int task = role - followers; task < a.batch * a.nc; task += readers) {
+    for (int task = draw(counters + kTellStride); task < a.batch * a.nc; task = draw(counters + kTellStride)) {
         const int ci = task / a.batch;
         const size_t b = task % a.batch;
         wait_told(counters_of(b), 1 + PARTS, ci + 1);
@@ -809,19 +777,18 @@ __global__ __launch_bounds__(4 * D + 64) void selfref_forward_kernel(SelfrefForw
 }
 template <int D, bool SG, int N>
 bool launch_together(const SelfrefForward &a) {
-    const int n = (1 + (1 + 4 / N) * a.batch) * kTellStride, followers = (1 + 4 / N) * a.batch;
+    const int n = (2 + (1 + 4 / N) * a.batch) * kTellStride, followers = (1 + 4 / N) * a.batch;
     unsigned *counters = reinterpret_cast<unsigned *>(scratch_if_free(42, n * sizeof(unsigned)));
     if (!counters) return false;
     constexpr int most = scan_lds_floats<D>(true) > read_lds_floats<D>() ? scan_lds_floats<D>(true) : read_lds_floats<D>();
     constexpr size_t lds = (most > kAloneFloats ? most : kAloneFloats) * sizeof(float);
     const long long tasks = (long long)a.batch * a.nc, rest = compute_units() - followers;
     const int readers = (int)(tasks < rest ? tasks : rest);
-    hipLaunchKernelGGL(selfref_counters_kernel, dim3(ceil_div(n, 256)), dim3(256), 0, stream(), counters, n);
-    check_launch("selfref_counters_kernel");
+    clear_counters(counters, n);
     check_hip(hipFuncSetAttribute(reinterpret_cast<const void *>(selfref_forward_kernel<D, SG, N>),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds), "dynamic LDS size");
     KernelTimer kt("selfref_forward_kernel");
-    hipLaunchKernelGGL((selfref_forward_kernel<D, SG, N>), dim3(followers + readers), dim3(4 * D + 64), lds, stream(), a, counters, readers);
+    hipLaunchKernelGGL((selfref_forward_kernel<D, SG, N>), dim3(followers + readers), dim3(4 * D + 64), lds, stream(), a, counters);
     check_launch("selfref_forward_kernel");
     return true;
 }
@@ -829,11 +796,13 @@ bool launch_together(const SelfrefForward &a) {
 template <int D, bool SG>
 void launch(const SelfrefForward &a) {
     // Together where compute units stay idle beside the chains and those that follow them keep up with them: the other memories
-    // take 10 us a chunk of any length, a chain 7 us for 16 tokens.  64 chains of 512 tokens, head size 64, three launches / one:
-    // chunks of 8 0.57 / 0.73 ms, of 16 0.38 / 0.41, of 32 0.326 / 0.306, of 64 0.299 / 0.277; 4 chains of 100 tokens 82 / 75 us.
+    // take 10 us a chunk of any length, a chain 7 us for 16 tokens.  64 chains of 512 tokens, head size 64, apart / together:
+    // chunks of 8 0.57 / 0.73 ms, of 16 0.38 / 0.41, of 32 0.327 / 0.308, of 64 0.299 / 0.279.  Behind a short sequence follow the reads of
+    // its chunks on what the chains and their company leave of the chip: 64 chains of 200 tokens 0.94 times as fast together, of 300
+    // 1.04, of 400 1.03, 48 of 300 in chunks of 32 0.97; up to 8 chains every chunk has a workgroup of its own (4 of 100 tokens 82 / 75 us).
     // As many workgroups for a chain's other memories as leave most of the chip to the reads, which are the slower ones.
     const int cus = compute_units();
-    if (a.nc > 1 && a.C >= 2 * kTB && 4 * a.batch <= cus) {
+    if (a.nc > 1 && a.C >= 2 * kTB && 4 * a.batch <= cus && (a.s >= 400 || a.batch <= 8)) {
         if (16 * a.batch <= cus   ? launch_together<D, SG, 1>(a)
             : 8 * a.batch <= cus ? launch_together<D, SG, 2>(a)
                                  : launch_together<D, SG, 4>(a))

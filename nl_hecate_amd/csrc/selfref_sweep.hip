@@ -32,6 +32,7 @@
 #include <utility>
 
 #include "../../include/nl_hecate_ffi.h"
+#include "handover.h"
 #include "lane_ops.h"
 #include "quad_rows.h"
 #include "runtime.h"
@@ -79,22 +80,22 @@ __device__ __forceinline__ void store_columns(float *p, const float (&x)[N]) {
 // low-rank products wait and F_k, F_v, F_q are on their way.  2048 chunks at head size 64: 293 us; four waves, one for each tile, whose
 // column sums of F_eta and F_alpha were 64 loads one after the other, took 363.
 template <int D>
-__global__ __launch_bounds__(kPrepThr) void selfref_bwd_prepare_kernel(
-    const float *__restrict__ emb, const float *__restrict__ d_y, const float *__restrict__ k_cache,
-    const float *__restrict__ v_cache, const float *__restrict__ q_cache, const float *__restrict__ alpha_cache,
-    const float *__restrict__ theta_cache, const float *__restrict__ amean_cache,
-    const float *__restrict__ emean_cache, const float *__restrict__ frozen, float *__restrict__ gl,
-    float *__restrict__ tok, float *__restrict__ outer, float *__restrict__ csv, float *__restrict__ d_mems, int s, int C, int nc) {
+__device__ __forceinline__ void prepare_of(const SelfrefSweep &a, size_t b, int ci, float *lds) {
+    const float *const emb = a.emb, *const d_y = a.d_y, *const k_cache = a.k, *const v_cache = a.v, *const q_cache = a.q,
+                *const alpha_cache = a.alpha, *const theta_cache = a.theta, *const amean_cache = a.amean, *const emean_cache = a.emean,
+                *const frozen = a.frozen;
+    float *const gl = a.gl, *const tok = a.tok, *const outer = a.outer, *const csv = a.csv, *const d_mems = a.d_mems;
+    const int s = a.s, C = a.C, nc = a.nc;
     constexpr int KT = D / 16, DD = D * D, KL = D + 4, V4 = D / 4;
     constexpr int JH = KT > 1 ? KT / 2 : 1, CG = KT / JH;   // a wave's column tiles; groups of columns
     constexpr int TF = sweep_token_floats(D);
     using P = PrepareLds<D>;
-    extern __shared__ __align__(16) float lds[];
     const ChunkLds<D> m(lds);
     float *Wx = m.tiles + P::wx, *Wq = m.tiles + P::wq, *Wd = m.tiles + P::wd, *DP = m.tiles + P::dp, *sums = m.tiles + P::sums;
-    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, ml = lane & 15, kg = lane >> 4;
-    const int ci = blockIdx.x % nc;
-    const size_t b = blockIdx.x / nc, chunk = blockIdx.x, tok0 = b * (size_t)s;
+    int tid = threadIdx.x;   // an opaque copy: addresses made of it are not to live across the chunks of a workgroup
+    asm volatile("" : "+v"(tid));
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, ml = lane & 15, kg = lane >> 4;
+    const size_t chunk = b * nc + ci, tok0 = b * (size_t)s;
     const int t0 = ci * C, L = min(C, s - t0), ntile = (L + kTB - 1) / kTB;
     const float *fz = frozen + chunk * 6 * DD;
     const int half = wave >> 2, tile = half ? 7 - wave : wave, li0 = tile * kTB, nt = min(kTB, L - li0);
@@ -498,6 +499,14 @@ __global__ __launch_bounds__(kPrepThr) void selfref_bwd_prepare_kernel(
     }
 }
 
+template <int D>
+constexpr size_t prepare_lds_bytes() { return (chunk_lds_floats<D>(0) + PrepareLds<D>::floats) * sizeof(float); }
+template <int D>
+__global__ __launch_bounds__(kPrepThr) void selfref_bwd_prepare_kernel(SelfrefSweep a) {
+    extern __shared__ __align__(16) float lds[];
+    prepare_of<D>(a, blockIdx.x / a.nc, blockIdx.x % a.nc, lds);
+}
+
 // ── matrices ─────────────────────────────────────────────────────────────────────────────────────────────────────
 // What a chunk's tokens add to dF whatever the sweep finds: the lane's part of a wave's 16 rows.
 template <int D>
@@ -714,17 +723,20 @@ constexpr int sweep_lds_floats(int d) { return 2 * sweep_tile_floats(d) + kTB * 
 // over (i, kg)), and the coefficients of a product with a vector whose element CP kg + i is broadcast from lane i of
 // DPP row kg.  dG is kept a second time by columns (dGT).  Tokens of a tile are result rows in the order sigma, so that
 // lane kg owns the columns s = 4 v + kg of Y.
-template <int D>
-__global__ __launch_bounds__(8 * D) void selfref_bwd_sweep_kernel(
-    const float *__restrict__ emb, const float *__restrict__ k_cache, const float *__restrict__ v_cache,
-    const float *__restrict__ frozen, const float *__restrict__ gl, const float *__restrict__ tok,
-    const float *__restrict__ outer, const float *__restrict__ csv, float *__restrict__ d_emb,
-    float *__restrict__ d_mems, int s, int C, int nc) {
+// FOLLOWED: what a chunk needs comes from workgroups that work beside this one (selfref_backward_kernel): sh counts the chunks whose
+// share of dG_L is there (from the end of the chain), pr is 1 for a prepared chunk of the chain; done tells of the chunks whose dg is
+// stored.  The second half asks a chunk ahead, so that nobody waits for the answer, and tells behind a wait that it has anyway.
+template <int D, bool FOLLOWED>
+__device__ __forceinline__ void sweep_of(const SelfrefSweep &args, size_t b, float *raw, const unsigned *pr, const unsigned *sh,
+                                         unsigned *done) {
+    const float *const emb = args.emb, *const k_cache = args.k, *const v_cache = args.v, *const frozen = args.frozen,
+                *const gl = args.gl, *const tok = args.tok, *const outer = args.outer, *const csv = args.csv;
+    float *const d_emb = args.d_emb, *const d_mems = args.d_mems;
+    const int s = args.s, C = args.C, nc = args.nc;
     constexpr int CP = D / 4, KT = D / 16, JT = D / 16, NT = 4 * D, NW = D / 16, DD = D * D, V4 = D / 4, LD = D + 4;
     constexpr int TF = sweep_token_floats(D), TILE = kTB * LD;
     constexpr int LG = D + 16;                       // rows 4 v + kg of g fall on different banks for the four kg
     enum { A_K, A_U, A_X, A_DG0, A_FX };             // and g behind them
-    extern __shared__ __align__(16) float raw[];
     constexpr int SET = sweep_tile_floats(D);
     static_assert(SET >= D * LD, "dG_L in the place of a tile's inputs");
     float *const DG = raw + 2 * SET, *const GLT = DG + TILE, *const Fa = GLT + D * LD, *const Fb = Fa + D * LD;   // G_L^T, F_k, F_v
@@ -742,7 +754,15 @@ __global__ __launch_bounds__(8 * D) void selfref_bwd_sweep_kernel(
     const int tid = second ? threadIdx.x - NT : threadIdx.x, r = tid >> 2, cq = tid & 3, wave = tid >> 6, lane = tid & 63;
     const int ml = lane & 15, kg = lane >> 4, wr = 16 * wave, c0 = cq * CP;
     const int s_of = sigma(lane & 15), kg_of = lane >> 4;   // as my_s and kg, for masks that stay in scalar registers
-    const size_t b = blockIdx.x, tok0 = b * (size_t)s;
+    const size_t tok0 = b * (size_t)s;
+
+    if (FOLLOWED) {   // the last two chunks and the share between them
+        if (threadIdx.x < 64) {
+            while (!told(pr + nc - 1, 1) || !told(pr + nc - 2, 1) || !told(sh, 1)) __builtin_amdgcn_s_sleep(8);
+        }
+        __syncthreads();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    }
 
     f32x4 accEA = kZero;
     float dG[CP], dGT[CP], sig = 0.f;
@@ -800,10 +820,12 @@ __global__ __launch_bounds__(8 * D) void selfref_bwd_sweep_kernel(
         request(tid);
         stage(0, tid);
         request(tid);
+        int stored = 0, whole = 0, told_of = 0;   // chunks whose dg was stored before now, before the tile before; as the others know
         for (int ci = nc - 1, buf = 0; ci >= 0; ci--) {
             const int t0 = ci * C, L = min(C, s - t0), ntile = (L + kTB - 1) / kTB;
             const size_t chunk = b * nc + ci;
             const float *fz = frozen + chunk * 6 * DD;
+            unsigned ask_p = 1, ask_s = 1;   // answers of the chunk before the one before this
             int me = tid;
             asm volatile("" : "+v"(me));
             const int wave = me >> 6, lane = me & 63, ml = lane & 15, kg = lane >> 4;
@@ -812,6 +834,7 @@ __global__ __launch_bounds__(8 * D) void selfref_bwd_sweep_kernel(
                 put_rows<D>(Bb, dFm[1], me);
             }
             lds_barrier();
+            if (FOLLOWED) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
             if (ci < nc - 1) {
                 // accE <- G_L accE, accA <- G_L accA: rows 0 and 1 of one more product
                 f32x4 accV[KT];
@@ -876,6 +899,18 @@ __global__ __launch_bounds__(8 * D) void selfref_bwd_sweep_kernel(
                 const float *set = raw + buf * SET, *tg = set + 5 * TILE;
                 for (int i = 0; i < 3; i++) lds_barrier();   // top, W and Z, the first token
                 stage(buf ^ 1, me);
+                if (FOLLOWED) {   // no load is under way here, and stores of the tile before have arrived
+                    stores_arrived();
+                    if (wave == 0 && (whole >= told_of + kTellChunks || (whole > told_of && whole >= nc - kTellChunks))) {
+                        told_of = whole;
+                        tell(done, told_of);
+                    }
+                    whole = stored;
+                    if (tile == 0 && ci > 1) {
+                        ask_p = __hip_atomic_load(pr + ci - 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        ask_s = __hip_atomic_load(sh, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    }
+                }
                 request(me);
                 if (tile < ntile - 1) pending(tile + 1, integral_constant<int, 0>{});
                 lds_barrier();
@@ -914,6 +949,11 @@ __global__ __launch_bounds__(8 * D) void selfref_bwd_sweep_kernel(
             pending(0, integral_constant<int, 1>{});
             pending(0, integral_constant<int, 2>{});
             pending(0, integral_constant<int, 3>{});
+            stored++;
+            // the chunk after the next needs its preparation and its share; the other half meets this one at the next barrier
+            if (FOLLOWED && ci > 1 && (!ask_p || ask_s < (unsigned)(nc - ci + 1))) {
+                while (!told(pr + ci - 2, 1) || !told(sh, nc - ci + 1)) __builtin_amdgcn_s_sleep(2);
+            }
         }
 #pragma unroll
         for (int c = 0; c < 2; c++) {   // gradients of the initial memories
@@ -923,7 +963,9 @@ __global__ __launch_bounds__(8 * D) void selfref_bwd_sweep_kernel(
                 for (int v = 0; v < 4; v++) dmb[(size_t)c * DD + (wr + 4 * kg + v) * D + 16 * jt + ml] = dFm[c][jt][v];
             }
         }
+        if (FOLLOWED) stores_arrived();
         __syncthreads();
+        if (FOLLOWED && tid < 64) tell(done, nc);
         __syncthreads();
         return;
     }
@@ -957,6 +999,7 @@ __global__ __launch_bounds__(8 * D) void selfref_bwd_sweep_kernel(
         // LDS-only barriers from here on: requests and the stores of dg stay under way across them
         if (ci < nc - 1 && kg == 0) { av[0][wr + ml] = accEA[0]; av[1][wr + ml] = accEA[1]; }
         lds_barrier();
+        if (FOLLOWED) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
         sig = 0.f;
         if (ci < nc - 1) {
             // Chunk boundary: gradients of F'_c = F_c G_L flow into dG_L = sum_c F_c^T dF'_c and dF_c = dF'_c G_L^T, on
@@ -1212,14 +1255,181 @@ __global__ __launch_bounds__(8 * D) void selfref_bwd_sweep_kernel(
 }
 
 template <int D>
-void launch(const SelfrefSweep &a) {
-    constexpr size_t lds = (chunk_lds_floats<D>(0) + PrepareLds<D>::floats) * sizeof(float);
+__global__ __launch_bounds__(8 * D) void selfref_bwd_sweep_kernel(SelfrefSweep a) {
+    extern __shared__ __align__(16) float raw[];
+    sweep_of<D, false>(a, blockIdx.x, raw, nullptr, nullptr, nullptr);
+}
+
+// ── all of it at once ────────────────────────────────────────────────────────────────────────────────────────────
+// A chain's gradients of F_q and F_mem and their share of dG_L, as selfref_bwd_scan_kernel and selfref_bwd_share_kernel, chunk by
+// chunk as the chunks are prepared.  8 D threads: a wave has 16 rows of one of the two, and 16 rows and half of the columns of a share.
+template <int D>
+constexpr int passed_lds_floats() { return 4 * D * (D + 4); }
+template <int D>
+__device__ __forceinline__ void passed_of(const SelfrefSweep &a, size_t b, float *lds, const unsigned *prepared, unsigned *shares) {
+    constexpr int KT = D / 16, DD = D * D, LD = D + 4, NW = D / 16, JH = KT / 2, STEPS = D / 4;
+    static_assert(KT % 2 == 0, "two waves for 16 rows of a share");
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, ml = lane & 15, kg = lane >> 4, nc = a.nc;
+    const int c = wave / NW, row0 = 16 * (wave % NW);
+    float *const Fs = lds, *const Bm = lds + 2 * D * LD;   // F_q, F_mem; dF'_q, dF'_mem
+    float *const rows = a.outer + (b * nc * 4 + 2 + c) * DD + (row0 + ml) * D + 4 * kg;
+    const float *const g = a.gl + b * nc * DD + ml * D + 4 * kg;
+    f32x4 f[KT], G[KT][KT], sums[KT], F[KT];
+    auto request_F = [&](int ci) {   // half the threads for each matrix
+#pragma unroll
+        for (int i = 0; i < KT; i++)
+            F[i] = *reinterpret_cast<const f32x4 *>(a.frozen + ((b * nc + ci) * 6 + (c ? 5 : 2)) * DD + (tid % (4 * D) + i * 4 * D) * 4);
+    };
+    request_F(nc - 2);
+    wait_told(prepared + nc - 1, 1, 1);
+#pragma unroll
+    for (int kt = 0; kt < KT; kt++) f[kt] = *reinterpret_cast<const f32x4 *>(rows + (size_t)(nc - 1) * 4 * DD + 16 * kt);
+    for (int ci = nc - 2; ci >= 0; ci--) {
+        stage_matrix<D>(Fs + c * D * LD, F, tid % (4 * D));
+#pragma unroll
+        for (int kt = 0; kt < KT; kt++) *reinterpret_cast<f32x4 *>(Bm + c * D * LD + (row0 + ml) * LD + 16 * kt + 4 * kg) = f[kt];
+        __syncthreads();
+        request_F(max(ci - 1, 0));
+        {   // the same sums in the same order as a workgroup that takes one memory after the other
+            f32x4 acc[JH];
+#pragma unroll
+            for (int j = 0; j < JH; j++) acc[j] = kZero;
+            for (int m = 0; m < 2; m++) {
+                const float *Fm = Fs + m * D * LD + row0 + ml, *B = Bm + m * D * LD + 16 * JH * c + ml;
+#pragma unroll
+                for (int i = 0; i < STEPS; i++) {
+                    const int k = 16 * (i >> 2) + 4 * kg + (i & 3);
+#pragma unroll
+                    for (int j = 0; j < JH; j++) acc[j] = mfma4(Fm[k * LD], B[k * LD + 16 * j], acc[j]);
+                }
+            }
+            float *share = a.outer + ((b * nc + ci + 1) * 4 + 2) * DD;
+#pragma unroll
+            for (int j = 0; j < JH; j++)
+                *reinterpret_cast<f32x4 *>(share + ((size_t)(wave % NW * KT + JH * c + j) * 64 + lane) * 4) = acc[j];
+        }
+        stores_arrived();
+        wait_told(prepared + ci, 1, 1);   // everybody's part of the share has arrived
+        if (wave == 0) tell(shares, nc - 1 - ci);
+#pragma unroll
+        for (int kt = 0; kt < KT; kt++) {
+            sums[kt] = *reinterpret_cast<const f32x4 *>(rows + (size_t)ci * 4 * DD + 16 * kt);
+#pragma unroll
+            for (int jt = 0; jt < KT; jt++) G[kt][jt] = *reinterpret_cast<const f32x4 *>(g + (size_t)ci * DD + 16 * jt * D + 16 * kt);
+        }
+        f32x4 acc[KT];
+#pragma unroll
+        for (int jt = 0; jt < KT; jt++) acc[jt] = kZero;
+#pragma unroll
+        for (int kt = 0; kt < KT; kt++) {
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+#pragma unroll
+                for (int jt = 0; jt < KT; jt++) acc[jt] = mfma4(G[kt][jt][v], f[kt][v], acc[jt]);
+            }
+        }
+#pragma unroll
+        for (int jt = 0; jt < KT; jt++) f[jt] = acc[jt] + sums[jt];
+    }
+    float *out = a.d_mems + (b * 6 + (c ? 5 : 2)) * DD + (row0 + ml) * D + 4 * kg;
+#pragma unroll
+    for (int jt = 0; jt < KT; jt++) *reinterpret_cast<f32x4 *>(out + 16 * jt) = f[jt];
+}
+
+// Counters: the numbers drawn, by workgroups and for the chunks of the first and the last ones; a chain's shares, its chunks with dg; a
+// flag for each prepared chunk.
+struct BackwardCounters {
+    unsigned *drawn;
+    int batch, nc;
+    __host__ __device__ unsigned *next(int i) const { return drawn + (1 + i) * kTellStride; }
+    __host__ __device__ unsigned *shares(size_t b) const { return drawn + (3 + b) * kTellStride; }
+    __host__ __device__ unsigned *swept(size_t b) const { return drawn + (3 + batch + b) * kTellStride; }
+    __host__ __device__ unsigned *prepared(size_t b) const { return drawn + (3 + 2 * (size_t)batch) * kTellStride + b * nc; }
+    size_t floats() const { return (3 + 2 * (size_t)batch) * kTellStride + (size_t)batch * nc; }
+};
+// The sweeps leave most of the compute units idle, need one prepared chunk after the other, from the end, and their dg becomes d_x
+// chunk by chunk.  So one launch has workgroups that prepare chunks, in the order in which they are needed; for each chain one that
+// takes the gradients of F_q and F_mem through it, and the sweep; and those that form d_x, which start as the first ones end.  The
+// order of the numbers (handover.h) is that order.  A workgroup fills a compute unit's LDS.
+// 64 chains of 2048 tokens, head size 64, chunks of 64: 1.49 ms for 0.29 + 0.06 + 0.03 + 1.29 + 0.06 of five launches.  The
+// preparation ends at 0.69 ms, a sweep starts at 0.05 and is slower than alone by 5 % (its neighbours' code and traffic), the last
+// d_x is 8 us behind the last sweep.  With the chunks dealt out beforehand the last d_x was 170 us behind: some workgroups of the last
+// kind find no place before the sweeps end.
+template <int D>
+__global__ __launch_bounds__(8 * D) void selfref_backward_kernel(SelfrefSweep a, BackwardCounters n, int preparers) {
+    static_assert(8 * D == kPrepThr, "the same workgroup for all");
+    extern __shared__ __align__(16) float raw[];
+    int role = draw(n.drawn);
+    const int tasks = a.batch * a.nc;
+    if (role < preparers) {
+        for (int task = draw(n.next(0)); task < tasks; task = draw(n.next(0))) {
+            const int ci = a.nc - 1 - task / a.batch;
+            const size_t b = task % a.batch;
+            prepare_of<D>(a, b, ci, raw);
+            stores_arrived();
+            __syncthreads();
+            if (threadIdx.x < 64) tell(n.prepared(b) + ci, 1);
+        }
+        return;
+    }
+    role -= preparers;
+    if (role < a.batch) {
+        passed_of<D>(a, role, raw, n.prepared(role), n.shares(role));
+        return;
+    }
+    role -= a.batch;
+    if (role < a.batch) {
+        sweep_of<D, true>(a, role, raw, n.prepared(role), n.shares(role), n.swept(role));
+        return;
+    }
+    if (threadIdx.x >= 4 * D) return;
+    for (int task = draw(n.next(1)); task < tasks; task = draw(n.next(1))) {
+        const int ci = a.nc - 1 - task / a.batch;
+        const size_t b = task % a.batch;
+        dx_of_chunk<D, true>(raw, a.k, a.v, a.alpha, a.theta, a.d_emb, nullptr, b, ci, a.s, a.C,
+                             [&] { wait_told(n.swept(b), 1, a.nc - ci); });
+        __syncthreads();   // the chunk's LDS is free
+    }
+}
+
+template <int D>
+bool launch_together(const SelfrefSweep &a) {
+    const int cus = compute_units();
+    BackwardCounters n{nullptr, a.batch, a.nc};
+    n.drawn = reinterpret_cast<unsigned *>(scratch_if_free(43, n.floats() * sizeof(unsigned)));
+    if (!n.drawn) return false;
+    constexpr size_t sweep = sweep_lds_floats(D) * sizeof(float), lds = sweep > prepare_lds_bytes<D>() ? sweep : prepare_lds_bytes<D>();
+    static_assert(lds >= kAloneFloats * sizeof(float) && lds >= passed_lds_floats<D>() * sizeof(float) &&
+                  lds >= chunk_lds_floats<D>(2) * sizeof(float), "LDS");
+    const long long tasks = (long long)a.batch * a.nc, rest = cus - 2 * a.batch;
+    const int others = (int)(tasks < rest ? tasks : rest);
+    clear_counters(n.drawn, (int)n.floats());
+    check_hip(hipFuncSetAttribute(reinterpret_cast<const void *>(selfref_backward_kernel<D>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds),
+              "dynamic LDS size");
+    KernelTimer kt("selfref_backward_kernel");
+    hipLaunchKernelGGL((selfref_backward_kernel<D>), dim3(2 * a.batch + 2 * others), dim3(8 * D), lds, stream(), a, n, others);
+    check_launch("selfref_backward_kernel");
+    return true;
+}
+
+template <int D>
+bool launch(const SelfrefSweep &a) {
+    constexpr size_t lds = prepare_lds_bytes<D>();
     static_assert(5 * kLrC * (D + 4) <= chunk_lds_floats<D>(0) + PrepareLds<D>::sums, "operands of the outer products");
     static_assert(lds <= 160 * 1024, "LDS");
+    if constexpr (8 * D == kPrepThr) {
+        // Together where the chunks are more than the chip prepares in two rounds, beside chains that leave at least half of it to
+        // them.  Otherwise the preparation is over before the sweep is far, and what a sweep does here besides (0.9 us a chunk, and
+        // its first chunks to wait for) costs more than the launches behind each other.  Apart / together: 64 chains of 2048 tokens
+        // 1734 / 1484 us in chunks of 64 and 2081 / 1887 in chunks of 32, of 512 tokens 430 / 420 and 509 / 488; 24 of 1400 1.05, 32 of
+        // 1000 1.03, 48 of 400 1.03 times as fast; 16 of 1000 (256 chunks) 0.98, 64 of 200 0.87.  Chunks have two tiles at least, since
+        // the inputs of a tile are requested two tiles ahead and those of one chunk ahead are there.
+        const int cus = compute_units();
+        if (a.C >= 2 * kTB && 4 * a.batch <= cus && (long long)a.batch * a.nc >= 2 * cus && launch_together<D>(a)) return true;
+    }
     check_hip(hipFuncSetAttribute(reinterpret_cast<const void *>(selfref_bwd_prepare_kernel<D>),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds), "dynamic LDS size");
-    hipLaunchKernelGGL((selfref_bwd_prepare_kernel<D>), dim3(a.batch * a.nc), dim3(kPrepThr), lds, stream(), a.emb, a.d_y, a.k,
-                       a.v, a.q, a.alpha, a.theta, a.amean, a.emean, a.frozen, a.gl, a.tok, a.outer, a.csv, a.d_mems, a.s, a.C, a.nc);
+    hipLaunchKernelGGL((selfref_bwd_prepare_kernel<D>), dim3(a.batch * a.nc), dim3(kPrepThr), lds, stream(), a);
     check_launch("selfref_bwd_prepare_kernel");
     if (a.nc > 1) {
         hipLaunchKernelGGL((selfref_bwd_scan_kernel<D>), dim3(2 * (D / 16) * a.batch), dim3(64), 0, stream(), a.gl, a.outer, a.d_mems,
@@ -1233,17 +1443,15 @@ void launch(const SelfrefSweep &a) {
     check_hip(hipFuncSetAttribute(reinterpret_cast<const void *>(selfref_bwd_sweep_kernel<D>),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)sweep_lds), "dynamic LDS size");
     KernelTimer kt("selfref_bwd_kernel");
-    hipLaunchKernelGGL((selfref_bwd_sweep_kernel<D>), dim3(a.batch), dim3(8 * D), sweep_lds, stream(), a.emb, a.k, a.v, a.frozen,
-                       a.gl, a.tok, a.outer, a.csv, a.d_emb, a.d_mems, a.s, a.C, a.nc);
+    hipLaunchKernelGGL((selfref_bwd_sweep_kernel<D>), dim3(a.batch), dim3(8 * D), sweep_lds, stream(), a);
     check_launch("selfref_bwd_sweep_kernel");
+    return false;
 }
 
 }  // namespace
 
-void selfref_backward_sweep(const SelfrefSweep &a) {
-    if (a.d == 16) launch<16>(a);
-    else if (a.d == 32) launch<32>(a);
-    else launch<64>(a);
+bool selfref_backward_sweep(const SelfrefSweep &a) {
+    return a.d == 16 ? launch<16>(a) : a.d == 32 ? launch<32>(a) : launch<64>(a);
 }
 
 }  // namespace nlh
