@@ -62,12 +62,11 @@ __device__ __forceinline__ bf16x8 ld_op_tr(const u16 *X, int row0, int ks) {
     return tr_pair(p, p + 4 * STRIDE);
 }
 // ld_op and ld_op_tr of a matrix in the permuted layout
-__device__ __forceinline__ bf16x8 ld_perm(const u16 *X, int row0, int ks) {
-    const int l = threadIdx.x & 63;
+__device__ __forceinline__ bf16x8 ld_perm(const u16 *X, int row0, int ks, int l = threadIdx.x & 63) {
     return *reinterpret_cast<const bf16x8 *>(X + bf_at(row0 + (l & 15), 32 * ks + 8 * (l >> 4)));
 }
-__device__ __forceinline__ bf16x8 ld_perm_tr(const u16 *X, int row0, int ks) {   // row0 a multiple of 16
-    const int l = threadIdx.x & 63, sl = l & 15, k = 32 * ks + 8 * (l >> 4) + (sl >> 2), n = row0 + 4 * (sl & 3);
+__device__ __forceinline__ bf16x8 ld_perm_tr(const u16 *X, int row0, int ks, int l = threadIdx.x & 63) {   // row0 a multiple of 16
+    const int sl = l & 15, k = 32 * ks + 8 * (l >> 4) + (sl >> 2), n = row0 + 4 * (sl & 3);
     return tr_pair(X + bf_at(k, n), X + bf_at(k + 4, n));
 }
 // Two floats rounded to bf16 (nearest, even) in one dword, x in the low half, opaque to the compiler: where it sees a half

@@ -6,8 +6,15 @@
 #include <stdint.h>
 
 #include "head_rows.h"
+#include "runtime.h"
 
 namespace nlh {
+
+// Both halves of a chain in one workgroup: where the halves of all chains do not fit the chip at once.  Up to there a half a compute
+// unit is faster (one compute unit takes 5 us for a chunk of both, 3 us for a half).  Forward and backward, us, halves / whole: 128
+// chains of 4096 tokens 680 in halves; 136 960 / 840, 192 1164 / 1030, 256 1345 / 1233; 256 of 1000 375 / 346; 300 of 2048 933 / 907;
+// without momentum 256 of 4096 1168 / 1052.
+inline bool chain_in_one_workgroup(int batch) { return 2 * batch > compute_units(); }
 
 // What a test of the reference's couplings needs from the forward (chunkwise_guard.hip), left behind by the chain
 // kernel as it goes: e2 [batch, 2 halves, num_chunks * 64] = the sum over the half's 32 memory rows of the squared

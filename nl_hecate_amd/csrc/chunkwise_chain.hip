@@ -31,7 +31,7 @@
 namespace nlh {
 namespace {
 
-constexpr int kChainThr = 512;     // 8 waves
+constexpr int kChainThr = 512;     // 8 waves for 32 rows of a chain
 
 // Work split of the eight waves: a 64x64 product is four 32x32 blocks (2x2 tiles of 16x16; an
 // A or B operand read from LDS then serves two tiles).  Wave w works on block bi = w%4 with
@@ -100,31 +100,35 @@ __global__ __launch_bounds__(64) void cw_coef_kernel(const float *__restrict__ a
 // for K, Q and W).  Waves 0..3 (group X): E, then Y^T, one 16-token strip each.  Waves 4..7
 // (group Y): one 32x32 block of W.P each, then one 16-column strip of the transposed state
 // update; they hold the fp32 master state.
+// H = 2: one workgroup of sixteen waves has both halves, eight waves each, and its group Y waves a 32 x 16 block of W.P; K, Q and W
+// are fetched, and W.P formed, once, and four waves on a SIMD hide each other's latencies.  256 chains of 4096 tokens: 393 -> 313 us.
 // TRACK: also leaves the per-token error norms and the chunk-start state norms of ChainTracks behind.
-template <bool HAS_S, bool TRACK>
-__global__ __launch_bounds__(kChainThr) void cw_chain_fwd_kernel(
+template <bool HAS_S, bool TRACK, int H>
+__global__ __launch_bounds__(H *kChainThr) void cw_chain_fwd_kernel(
     const u16 *__restrict__ k, const u16 *__restrict__ v, const u16 *__restrict__ q,
     const float *__restrict__ table, const float *__restrict__ vecs, const float *m_initial, const float *s_initial,
     float *__restrict__ m_states, float *__restrict__ s_states,
     float *__restrict__ y, int s, int C, int nc, int batch, HeadRows yr, ChainTracks tr, ChainFinal fin) {
-    constexpr int HMAT = 32 * 64;   // a 32-row matrix
+    constexpr int HMAT = 32 * H * 64;   // this workgroup's rows of a matrix
+    constexpr int CT = 2 / H;           // 16-token tiles of a group Y wave's block of P^T
     extern __shared__ __align__(16) unsigned char smem_raw[];
     u16 *Kr = reinterpret_cast<u16 *>(smem_raw);   // K [t][c]
     u16 *Kt0 = Kr + kPerm, *Kt1 = Kt0 + kPerm;       // K^T [c][t] of this chunk / V [t][i] until K^T of the next lands
     u16 *Qr0 = Kt1 + kPerm, *Qr1 = Qr0 + kPerm;      // Q [t][c], alternating between chunks
     u16 *WPh = Qr1 + kPerm, *WPl = WPh + kPerm;      // W.P [t][j]
-    u16 *Mh = WPl + kPerm, *Ml = Mh + HMAT;         // chunk-start M [i][c], this workgroup's 32 rows, hi / lo
+    u16 *Mh = WPl + kPerm, *Ml = Mh + HMAT;         // chunk-start M [i][c], this workgroup's rows, hi / lo
     u16 *Sh = Ml + HMAT, *Sl = Sh + HMAT;          // chunk-start S
     u16 *Eh = Sl + HMAT, *El = Eh + HMAT;          // E^T [i][t]
     u16 *EMh = El + HMAT, *EMl = EMh + HMAT;       // (E.wM)^T
     u16 *ESh = EMl + HMAT, *ESl = ESh + HMAT;      // (E.wS)^T
     float *cvec = reinterpret_cast<float *>(ESl + HMAT);   // a, beta, wM, wS [64] each, then a_L, beta_L, h_L
 
-    const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, g = l >> 4, r16 = l & 15;
-    int chain, half;
-    chain_half_of_block(batch, chain, half);
-    const int i0 = 32 * half;
-    const bool grpX = w < 4;
+    const int tid = threadIdx.x, w = H == 1 ? tid >> 6 : __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63, g = l >> 4, r16 = l & 15, first_l = l;
+    int chain, half;   // of the wave's rows
+    if (H == 1) chain_half_of_block(batch, chain, half);
+    else { chain = blockIdx.x; half = (w >> 2) & 1; }
+    const int i0 = 32 * half, il = H == 1 ? 0 : i0;   // first row; and in LDS
+    const bool grpX = w < 4 * H;
     const int bi = w & 3, bm = 32 * (bi >> 1), bn = 32 * (bi & 1);   // group Y: 32x32 block of P^T; group X: strip bi
     const size_t chain_tok = (size_t)chain * s;
     const size_t state0 = (size_t)chain * (nc + 1) * HD * HD;
@@ -145,38 +149,51 @@ __global__ __launch_bounds__(kChainThr) void cw_chain_fwd_kernel(
     }
 
     // Registers of the next chunk.  K, Q: row st_t, 8-element block st_cb (16 rows x 64 bytes per
-    // wave instruction).  V (threads 0..255): row vt, block vcb of this half's 32 columns.  Group Y:
+    // wave instruction), with sixteen waves K by the first eight and Q by the others.  V: row vt, columns from vcb of this workgroup's,
+    // eight by each of the first 256 threads, or four by each of 1024.  Group Y:
     // W at the accumulator positions of its P^T block.  Threads 0..259: one float of the vectors.
-    const int st_t = 16 * (w & 3) + (l & 15), st_cb = 4 * (w >> 2) + (l >> 4);
-    const int vt = (tid >> 2) & 63, vcb = tid & 3;
-    uint4 sk, sq, sv;
-    f32x4 wn[2][2], wc[2][2];
+    const int st_t = 16 * (w & 3) + (l & 15), st_cb = 4 * ((w >> 2) & 1) + (l >> 4);
+    const int vt = H == 1 ? (tid >> 2) & 63 : tid >> 4, vcb = H == 1 ? (tid & 3) * 8 : (tid & 15) * 4;
+    const bool has_k = H == 1 || w < 8, has_q = H == 1 || w >= 8;
+    const int ct0 = H == 1 ? 0 : half;   // group Y: first 16-token tile of its block
+    uint4 sk, sq, sv;   // with sixteen waves sk is K or Q
+    f32x4 wn[2][CT], wc[2][CT];
     float vn = 0.f;
     auto fetch = [&](int c) {
         const int L = min(C, s - c * C);
         const size_t tok = chain_tok + (size_t)c * C;
         const size_t o = (tok + min(st_t, L - 1)) * HD + st_cb * 8;
-        sk = *reinterpret_cast<const uint4 *>(k + o);
-        sq = *reinterpret_cast<const uint4 *>(q + o);
-        sv = *reinterpret_cast<const uint4 *>(v + (tok + min(vt, L - 1)) * HD + i0 + vcb * 8);
+        if (H == 1) {
+            sk = *reinterpret_cast<const uint4 *>(k + o);
+            sq = *reinterpret_cast<const uint4 *>(q + o);
+        } else {
+            sk = *reinterpret_cast<const uint4 *>((has_k ? k : q) + o);
+        }
+        const u16 *vp = v + (tok + min(vt, L - 1)) * HD + (i0 - il) + vcb;
+        if (H == 1) {
+            sv = *reinterpret_cast<const uint4 *>(vp);
+        } else {
+            const uint2 x = *reinterpret_cast<const uint2 *>(vp);
+            sv = make_uint4(x.x, x.y, 0, 0);
+        }
         const size_t chunk = (size_t)chain * nc + c;
         const float *tb = table + chunk * kTableFloats, *vo = vecs + chunk * kVecFloats;
 #pragma unroll
         for (int rt = 0; rt < 2; rt++)
 #pragma unroll
-            for (int ct = 0; ct < 2; ct++)
+            for (int ct = 0; ct < CT; ct++)
                 wn[rt][ct] = *reinterpret_cast<const f32x4 *>(
-                    (!grpX && tile_live(bi, rt, ct)) ? tb + (((bi * 2 + rt) * 2 + ct) * 64 + l) * 4 : vo + 4 * CW + 4);
+                    (!grpX && tile_live(bi, rt, ct0 + ct)) ? tb + (((bi * 2 + rt) * 2 + ct0 + ct) * 64 + l) * 4 : vo + 4 * CW + 4);
         vn = vo[min(tid, 4 * CW + 3)];
     };
     auto land = [&](int c) {   // wait for the loads here; zero the rows beyond a short chunk
         const int L = min(C, s - c * C);
-        if (st_t >= L) { sk = make_uint4(0, 0, 0, 0); sq = sk; }
+        if (st_t >= L) { sk = make_uint4(0, 0, 0, 0); if (H == 1) sq = sk; }
         if (vt >= L) sv = make_uint4(0, 0, 0, 0);
 #pragma unroll
         for (int rt = 0; rt < 2; rt++)
 #pragma unroll
-            for (int ct = 0; ct < 2; ct++) wc[rt][ct] = wn[rt][ct];
+            for (int ct = 0; ct < CT; ct++) wc[rt][ct] = wn[rt][ct];
         // V and the vectors are written to LDS later, behind the stores of this step: pin their
         // arrival to this point
         asm volatile("" : "+v"(sv.x), "+v"(sv.y), "+v"(sv.z), "+v"(sv.w), "+v"(vn));
@@ -191,7 +208,12 @@ __global__ __launch_bounds__(kChainThr) void cw_chain_fwd_kernel(
         }
     };
     auto commit_v = [&](u16 *dst) {
-        if (tid < 256) *reinterpret_cast<uint4 *>(dst + bf_at(vt, vcb * 8)) = sv;
+        if (H == 2) *reinterpret_cast<uint2 *>(dst + bf_at(vt, vcb)) = make_uint2(sv.x, sv.y);
+        else if (tid < 256) *reinterpret_cast<uint4 *>(dst + bf_at(vt, vcb)) = sv;
+    };
+    auto commit_tokens = [&](u16 *Q, u16 *Kt) {
+        if (has_k) { commit_rows(Kr, sk); commit_kt(Kt); }
+        if (has_q) commit_rows(Q, H == 1 ? sq : sk);
     };
     auto commit_vecs = [&]() {
         if (tid < 4 * CW + 4) cvec[tid] = vn;
@@ -212,7 +234,7 @@ __global__ __launch_bounds__(kChainThr) void cw_chain_fwd_kernel(
     auto stage_state = [&]() {             // -> LDS operands of the next chunk
 #pragma unroll
         for (int ct = 0; ct < 2; ct++) {
-            const int off = bf_at(16 * ct + r16, 16 * bi + 4 * g);
+            const int off = bf_at(il + 16 * ct + r16, 16 * bi + 4 * g);
             split_store(Mh, Ml, off, Mm[ct]);
             if (HAS_S) split_store(Sh, Sl, off, Sm[ct]);
         }
@@ -230,9 +252,7 @@ __global__ __launch_bounds__(kChainThr) void cw_chain_fwd_kernel(
         stage_state();
     }
     land(0);
-    commit_rows(Kr, sk);
-    commit_rows(Qr0, sq);
-    commit_kt(Kt0);
+    commit_tokens(Qr0, Kt0);
     commit_v(Kt1);
     commit_vecs();
     __syncthreads();
@@ -240,6 +260,11 @@ __global__ __launch_bounds__(kChainThr) void cw_chain_fwd_kernel(
     for (int c = 0; c < nc; c++) {
         const int t0 = c * C, L = min(C, s - t0);
         const size_t tok = chain_tok + t0;
+        // The thread's place through an opaque copy, once per chunk: with sixteen waves the LDS addresses made of it do not fit
+        // the registers across the sequence.
+        int me = first_l;
+        if (H == 2) asm volatile("" : "+v"(me));
+        const int l = me, g = l >> 4, r16 = l & 15;
         // this chunk: Q in Qc, K^T in Kc, V in Kn (until K^T of the next chunk replaces it)
         u16 *Qc = (c & 1) ? Qr1 : Qr0, *Kc = (c & 1) ? Kt1 : Kt0;
         u16 *Qn = (c & 1) ? Qr0 : Qr1, *Kn = (c & 1) ? Kt0 : Kt1;
@@ -261,8 +286,8 @@ __global__ __launch_bounds__(kChainThr) void cw_chain_fwd_kernel(
         // ── first half: E^T, (E.wM)^T, (E.wS)^T (group X) and W.P (group Y) ──
         if (grpX) {
             // E[t][i]: rows t = 16 bi .., columns i = 16 ct ..
-            const bf16x8 aK[2] = {ld_perm(Kr, 16 * bi, 0), ld_perm(Kr, 16 * bi, 1)};
-            const bf16x8 aV = ld_perm(Kn, 16 * bi, 0);
+            const bf16x8 aK[2] = {ld_perm(Kr, 16 * bi, 0, l), ld_perm(Kr, 16 * bi, 1, l)};
+            const bf16x8 aV = ld_perm(Kn, 16 * bi, H == 1 ? 0 : half, l);
             const f32x4 wm = *reinterpret_cast<const f32x4 *>(cvec + 2 * CW + 16 * bi + 4 * g);
             const f32x4 wsv = *reinterpret_cast<const f32x4 *>(cvec + 3 * CW + 16 * bi + 4 * g);
             f32x4 esq = zero4();
@@ -271,12 +296,12 @@ __global__ __launch_bounds__(kChainThr) void cw_chain_fwd_kernel(
                 f32x4 e = zero4();
 #pragma unroll
                 for (int ks = 0; ks < 2; ks++) {
-                    e = mfma32(aK[ks], ld_perm(Mh, 16 * ct, ks), e);
-                    e = mfma32(aK[ks], ld_perm(Ml, 16 * ct, ks), e);
+                    e = mfma32(aK[ks], ld_perm(Mh, il + 16 * ct, ks, l), e);
+                    e = mfma32(aK[ks], ld_perm(Ml, il + 16 * ct, ks, l), e);
                 }
                 e = mfma32(aV, negI[ct], e);
                 if (TRACK) esq += e * e;
-                const int off = bf_at(16 * ct + r16, 16 * bi + 4 * g);   // [i][t .. t+3]
+                const int off = bf_at(il + 16 * ct + r16, 16 * bi + 4 * g);   // [i][t .. t+3]
                 split_store(Eh, El, off, e);
                 split_store(EMh, EMl, off, e * wm);
                 if (HAS_S) split_store(ESh, ESl, off, e * wsv);
@@ -292,13 +317,17 @@ __global__ __launch_bounds__(kChainThr) void cw_chain_fwd_kernel(
 #pragma unroll
             for (int rt = 0; rt < 2; rt++)
 #pragma unroll
-                for (int ks = 0; ks < 2; ks++) aK[rt][ks] = ld_perm(Kr, bm + 16 * rt, ks);
-            f32x4 acc[2][2] = {{zero4(), zero4()}, {zero4(), zero4()}};
+                for (int ks = 0; ks < 2; ks++) aK[rt][ks] = ld_perm(Kr, bm + 16 * rt, ks, l);
+            f32x4 acc[2][CT];
+#pragma unroll
+            for (int rt = 0; rt < 2; rt++)
+#pragma unroll
+                for (int ct = 0; ct < CT; ct++) acc[rt][ct] = zero4();
 #pragma unroll
             for (int ks = 0; ks < 2; ks++)
 #pragma unroll
-                for (int ct = 0; ct < 2; ct++) {
-                    const bf16x8 bq = ld_perm(Qc, bn + 16 * ct, ks);
+                for (int ct = 0; ct < CT; ct++) {
+                    const bf16x8 bq = ld_perm(Qc, bn + 16 * (ct0 + ct), ks, l);
 #pragma unroll
                     for (int rt = 0; rt < 2; rt++)     // P^T[j][t]: rows j, columns t
                         acc[rt][ct] = mfma32(aK[rt][ks], bq, acc[rt][ct]);
@@ -306,8 +335,8 @@ __global__ __launch_bounds__(kChainThr) void cw_chain_fwd_kernel(
 #pragma unroll
             for (int rt = 0; rt < 2; rt++)
 #pragma unroll
-                for (int ct = 0; ct < 2; ct++)         // [t][j .. j+3]
-                    split_store(WPh, WPl, bf_at(bn + 16 * ct + r16, bm + 16 * rt + 4 * g),
+                for (int ct = 0; ct < CT; ct++)         // [t][j .. j+3]
+                    split_store(WPh, WPl, bf_at(bn + 16 * (ct0 + ct) + r16, bm + 16 * rt + 4 * g),
                                 wc[rt][ct] * acc[rt][ct]);
         }
         __syncthreads();
@@ -320,18 +349,18 @@ __global__ __launch_bounds__(kChainThr) void cw_chain_fwd_kernel(
             y0[0] = y0[1] = y1[0] = y1[1] = zero4();
 #pragma unroll
             for (int ks = 0; ks < 2; ks++) {
-                const bf16x8 bQ = ld_perm(Qc, 16 * bi, ks), bWh = ld_perm(WPh, 16 * bi, ks), bWl = ld_perm(WPl, 16 * bi, ks);
+                const bf16x8 bQ = ld_perm(Qc, 16 * bi, ks, l), bWh = ld_perm(WPh, 16 * bi, ks, l), bWl = ld_perm(WPl, 16 * bi, ks, l);
 #pragma unroll
                 for (int rt = 0; rt < 2; rt++) {
-                    const bf16x8 eh = ld_perm(Eh, 16 * rt, ks);
-                    y0[rt] = mfma32(ld_perm(Mh, 16 * rt, ks), bQ, y0[rt]);
-                    y0[rt] = mfma32(ld_perm(Ml, 16 * rt, ks), bQ, y0[rt]);
+                    const bf16x8 eh = ld_perm(Eh, il + 16 * rt, ks, l);
+                    y0[rt] = mfma32(ld_perm(Mh, il + 16 * rt, ks, l), bQ, y0[rt]);
+                    y0[rt] = mfma32(ld_perm(Ml, il + 16 * rt, ks, l), bQ, y0[rt]);
                     y2[rt] = mfma32(eh, bWh, y2[rt]);
                     y2[rt] = mfma32(eh, bWl, y2[rt]);
-                    y2[rt] = mfma32(ld_perm(El, 16 * rt, ks), bWh, y2[rt]);
+                    y2[rt] = mfma32(ld_perm(El, il + 16 * rt, ks, l), bWh, y2[rt]);
                     if (HAS_S) {
-                        y1[rt] = mfma32(ld_perm(Sh, 16 * rt, ks), bQ, y1[rt]);
-                        y1[rt] = mfma32(ld_perm(Sl, 16 * rt, ks), bQ, y1[rt]);
+                        y1[rt] = mfma32(ld_perm(Sh, il + 16 * rt, ks, l), bQ, y1[rt]);
+                        y1[rt] = mfma32(ld_perm(Sl, il + 16 * rt, ks, l), bQ, y1[rt]);
                     }
                 }
             }
@@ -343,14 +372,14 @@ __global__ __launch_bounds__(kChainThr) void cw_chain_fwd_kernel(
             f32x4 am[2] = {zero4(), zero4()}, as[2] = {zero4(), zero4()};
 #pragma unroll
             for (int ks = 0; ks < 2; ks++) {
-                const bf16x8 aKt = ld_perm(Kc, 16 * bi, ks);
+                const bf16x8 aKt = ld_perm(Kc, 16 * bi, ks, l);
 #pragma unroll
                 for (int ct = 0; ct < 2; ct++) {
-                    am[ct] = mfma32(aKt, ld_perm(EMh, 16 * ct, ks), am[ct]);
-                    am[ct] = mfma32(aKt, ld_perm(EMl, 16 * ct, ks), am[ct]);
+                    am[ct] = mfma32(aKt, ld_perm(EMh, il + 16 * ct, ks, l), am[ct]);
+                    am[ct] = mfma32(aKt, ld_perm(EMl, il + 16 * ct, ks, l), am[ct]);
                     if (HAS_S) {
-                        as[ct] = mfma32(aKt, ld_perm(ESh, 16 * ct, ks), as[ct]);
-                        as[ct] = mfma32(aKt, ld_perm(ESl, 16 * ct, ks), as[ct]);
+                        as[ct] = mfma32(aKt, ld_perm(ESh, il + 16 * ct, ks, l), as[ct]);
+                        as[ct] = mfma32(aKt, ld_perm(ESl, il + 16 * ct, ks, l), as[ct]);
                     }
                 }
             }
@@ -363,9 +392,7 @@ __global__ __launch_bounds__(kChainThr) void cw_chain_fwd_kernel(
         }
         // tokens of the next chunk land: K and V of this one are no longer read
         land(min(c + 1, nc - 1));
-        commit_rows(Kr, sk);
-        commit_rows(Qn, sq);
-        commit_kt(Kn);
+        commit_tokens(Qn, Kn);
         // results of this chunk leave
         if (grpX) {
             const int t = 16 * bi + r16;
@@ -393,7 +420,22 @@ __global__ __launch_bounds__(kChainThr) void cw_chain_fwd_kernel(
     }
 }
 
-constexpr size_t kChainFwdLds = (7 * kPerm + 10 * 32 * 64) * sizeof(u16) + (4 * CW + 4) * sizeof(float);
+constexpr size_t chain_fwd_lds(int h) { return (7 * kPerm + 10 * 32 * h * 64) * sizeof(u16) + (4 * CW + 4) * sizeof(float); }
+
+template <bool HAS_S, bool TRACK, int H>
+void launch_chain(const u16 *k, const u16 *v, const u16 *q, const float *table, const float *vecs, const float *m_initial,
+                  const float *s_initial, float *m_states, float *s_states, float *y, int seq_len, int chunk_size, int nc, int batch,
+                  const HeadRows &yr, const ChainTracks &tr, const ChainFinal &fin) {
+    static bool attr_set = false;
+    if (!attr_set) {
+        check_hip(hipFuncSetAttribute(reinterpret_cast<const void *>(cw_chain_fwd_kernel<HAS_S, TRACK, H>),
+                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)chain_fwd_lds(H)), "dynamic LDS size");
+        attr_set = true;
+    }
+    KernelTimer kt("cw_chain_fwd_kernel");
+    hipLaunchKernelGGL((cw_chain_fwd_kernel<HAS_S, TRACK, H>), dim3(2 / H * batch), dim3(H * kChainThr), chain_fwd_lds(H), stream(), k, v, q,
+                       table, vecs, m_initial, s_initial, m_states, s_states, y, seq_len, chunk_size, nc, batch, yr, tr, fin);
+}
 
 template <bool HAS_S>
 void launch_forward(const char *fn, const u16 *k, const u16 *v, const u16 *q, const float *alpha, const float *theta,
@@ -404,16 +446,6 @@ void launch_forward(const char *fn, const u16 *k, const u16 *v, const u16 *q, co
     const int nc = ceil_div(seq_len, chunk_size), nchunks = batch * nc;
     float *table = scratch(3, (size_t)nchunks * kTableFloats * sizeof(float));
     float *vecs = scratch(4, (size_t)nchunks * kVecFloats * sizeof(float));
-    static bool attr_set = false;
-    if (!attr_set) {
-        check_hip(hipFuncSetAttribute(reinterpret_cast<const void *>(cw_chain_fwd_kernel<HAS_S, false>),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)kChainFwdLds),
-                  "dynamic LDS size");
-        check_hip(hipFuncSetAttribute(reinterpret_cast<const void *>(cw_chain_fwd_kernel<HAS_S, true>),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)kChainFwdLds),
-                  "dynamic LDS size");
-        attr_set = true;
-    }
     if (es.failed()) return;
     {
         KernelTimer kt("cw_coef_kernel");
@@ -422,17 +454,11 @@ void launch_forward(const char *fn, const u16 *k, const u16 *v, const u16 *q, co
                            coef_chunks_per_wave(nchunks));
     }
     check_launch("cw_coef_kernel");
-    {
-        KernelTimer kt("cw_chain_fwd_kernel");
-        if (tracks)
-            hipLaunchKernelGGL((cw_chain_fwd_kernel<HAS_S, true>), dim3(2 * batch), dim3(kChainThr), kChainFwdLds, stream(), k,
-                               v, q, table, vecs, m_initial, s_initial, m_states, s_states, y, seq_len, chunk_size, nc, batch,
-                               yr, *tracks, fin);
-        else
-            hipLaunchKernelGGL((cw_chain_fwd_kernel<HAS_S, false>), dim3(2 * batch), dim3(kChainThr), kChainFwdLds, stream(), k,
-                               v, q, table, vecs, m_initial, s_initial, m_states, s_states, y, seq_len, chunk_size, nc, batch,
-                               yr, ChainTracks{nullptr, nullptr}, fin);
-    }
+    const ChainTracks tr = tracks ? *tracks : ChainTracks{nullptr, nullptr};
+    const bool whole = chain_in_one_workgroup(batch);
+    auto launch = tracks ? (whole ? launch_chain<HAS_S, true, 2> : launch_chain<HAS_S, true, 1>)
+                         : (whole ? launch_chain<HAS_S, false, 2> : launch_chain<HAS_S, false, 1>);
+    launch(k, v, q, table, vecs, m_initial, s_initial, m_states, s_states, y, seq_len, chunk_size, nc, batch, yr, tr, fin);
     check_launch(fn);
 }
 

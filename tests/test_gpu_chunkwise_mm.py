@@ -13,6 +13,7 @@ from nl_hecate_amd import dispatch as D
 from nl_hecate_amd.ffi import lib
 from oracle import pyoracle as orc
 from tests.gpu_util import assert_close, dev, host, rule_inputs, zeros
+from tests.test_gpu_exact_mm import kernels_run
 
 pytestmark = pytest.mark.gpu
 
@@ -327,3 +328,62 @@ def test_gate_gradients_of_more_chunks_than_waves(rule, n, s, C):
         want = sum(p[1][i].double() for p in parts)
         size = sum(p[1][i].abs().double() for p in parts)
         assert ((t.double() - want).abs() <= 2 ** -24 * 2 * n * (size + 8 * size.mean())).all(), i
+
+
+def _in_parts(rule, n, s, C, step, seed):
+    """Forward and backward of n chains at once and of `step` at a time: outputs of each chain, sums over the chains."""
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    rnd = lambda *shape: torch.randn(*shape, generator=g, device="cuda")
+    mats, slots = (2, -(-s // C) + 1) if rule == "titans" else (1, -(-s // C) + 1)
+    kvq = [(rnd(n, s, 64) / 8).to(torch.bfloat16) for _ in range(3)]
+    gates = [torch.sigmoid(rnd(n, s)) for _ in range(mats + 1)]
+    initial, d_y = [rnd(n, 64, 64) * 0.1 for _ in range(mats)], rnd(n, s, 64)
+
+    def both(a, b):
+        cut = lambda t: t[a:b].contiguous()
+        x, first = [cut(t) for t in kvq + gates], [cut(t) for t in initial]
+        states, y = [zeros(b - a, slots, 64, 64) for _ in range(mats)], zeros(b - a, s, 64)
+        out = [zeros(b - a, s, 64) for _ in range(3)] + [zeros(b - a, s) for _ in gates]
+        d0 = [zeros(64, 64) for _ in range(mats)]
+        D.call(f"{rule}_chunkwise_forward_bf16_rocm", *x, *first, *states, y, s, 64, b - a, C)
+        D.call(f"{rule}_chunkwise_backward_bf16_rocm", *x, *states, cut(d_y), *out, *d0, s, 64, b - a, C)
+        torch.cuda.synchronize()
+        return [y, *states, *out], d0
+
+    parts = [both(a, min(a + step, n)) for a in range(0, n, step)]
+    return both(0, n), parts
+
+
+# chains whose halves are more than the compute units, by one and by many; a chunk of one token at the end, chunks below a tile,
+# one chunk alone
+@pytest.mark.parametrize("rule", ["titans", "delta"])
+@pytest.mark.parametrize("more,s,C", [(1, 193, 64), (9, 100, 64), (1, 64, 64), (72, 70, 17), (3, 33, 32), (130, 50, 64), (1, 5, 1)])
+def test_chains_in_one_workgroup_and_in_two(rule, more, s, C):
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    n = cus // 2 + more
+    (whole, d0), parts = _in_parts(rule, n, s, C, 8, seed=n + s + C)
+    for i, t in enumerate(whole):
+        assert torch.equal(t, torch.cat([p[0][i] for p in parts])), i
+    for i, t in enumerate(d0):   # n float terms in another order
+        want, size = (sum(f(p[1][i].double()) for p in parts) for f in (lambda x: x, torch.abs))
+        assert ((t.double() - want).abs() <= 2 ** -24 * 2 * n * (size + 8 * size.mean())).all(), i
+
+
+@pytest.mark.parametrize("fires", ["nothing", "norm", "clip"])
+def test_tracks_of_chains_in_one_workgroup(fires):
+    """What the last chain's second half of the rows leaves behind decides alone."""
+    B, s, C = torch.cuda.get_device_properties(0).multi_processor_count // 2 + 1, 130, 64
+    g = torch.Generator(device="cuda").manual_seed(5)
+    rnd = lambda *shape: torch.randn(*shape, generator=g, device="cuda")
+    kvq = [(rnd(B, s, 64) / 8).to(torch.bfloat16) for _ in range(3)]
+    gates = [torch.sigmoid(rnd(B, s) - 3) for _ in range(3)]
+    m0, s0 = rnd(B, 64, 64) * 0.01, rnd(B, 64, 64) * 0.01
+    if fires == "norm":
+        m0[-1, 50, 3] = 1000.0
+    if fires == "clip":
+        kvq[1][-1, 129, 50] = 1000.0   # in the chunk of two tokens
+    slots = -(-s // C) + 1
+    states, y = [zeros(B, slots, 64, 64) for _ in range(2)], zeros(B, s, 64)
+    ran = kernels_run(lambda: D.call("titans_chunkwise_forward_bf16_guarded_rocm", *kvq, *gates, m0, s0, *states, y, s, 64, B, C,
+                                     500.0, 500.0))
+    assert "cw_chain_fwd_kernel" in ran and ("rule_fwd_kernel" in ran) == (fires != "nothing"), ran
