@@ -40,7 +40,7 @@
 // rounded once: 0.6 to 1.0e-7, each output at or below its walk over spread gates, gates at a model's start and long-lived
 // states.  Left in fp32 are the products that do not show: the inverse, K K^T, K M^T, the maps
 // of the adjoint scan and the products with the adjoint at the chunk's end.  512 tokens of 32 chains, head size 64: first
-// kernel 38 -> 46 us, gradients 38 -> 65, scan 16 -> 23, gates 10 -> 15; head size 32, 777 tokens of 16: 21 -> 25, 24 -> 32,
+// kernel 38 -> 46 us, gradients 38 -> 48, scan 16 -> 23, gates 10 -> 15; head size 32, 777 tokens of 16: 21 -> 25, 24 -> 32,
 // 5 -> 8, 7 -> 9.  Head size 64 with checkpoints every 32 tokens and more keeps fp32 sums: there the form is the path that
 // there was, and its two kernels are bound by their products.
 //
@@ -489,7 +489,12 @@ __global__ __launch_bounds__(kThr) void ex_grads_kernel(
     int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     asm volatile("" : "+s"(w));
     NLH_STRIP_ORIGIN_OF(w);
-    auto MMA = [&](Strip &acc, auto fa, auto fb) { product<P64>(acc, fa, fb, l); };
+    // Float64 sums at head size 64: the scheduler, left alone, reads the operands of several products ahead and spills 119 registers
+    // (256 chunks 64 us with the spills, 48 without); the other forms have room for that.
+    auto MMA = [&](Strip &acc, auto fa, auto fb) {
+        product<P64>(acc, fa, fb, l);
+        if (P64 && D == 64) __builtin_amdgcn_sched_barrier(0);
+    };
     auto MMAR = [&](Strip &acc, auto fa, auto fb, int p0, int p1) { product_range<P64>(acc, fa, fb, p0, p1, l); };
     auto FORC = [&](Strip &acc, auto f) { for_c(acc, f, l); };
     auto MMD = [&](Strip &acc, auto fa, auto fb) { if constexpr (D == 64) MMA(acc, fa, fb); else MMAR(acc, fa, fb, 0, D / 32); };
