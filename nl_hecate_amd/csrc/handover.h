@@ -6,6 +6,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <mutex>
+
 #include "runtime.h"
 
 namespace nlh {
@@ -48,6 +50,10 @@ __device__ __forceinline__ int draw(unsigned *counter) {
 }
 
 constexpr int kAloneFloats = 81 * 256;   // more than half of a compute unit's LDS
+
+// Held from where the counters' memory is taken to where their kernel is launched: with two host threads on one stream, the first
+// one's kernel is not to come between the second one's cleared counters and its kernel.
+inline std::mutex counters_in_use;
 
 // A kernel and not a memset: the launch may be recorded.
 __global__ static void clear_counters_kernel(unsigned *counters, int n) {

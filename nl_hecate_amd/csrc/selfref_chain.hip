@@ -778,6 +778,7 @@ __global__ __launch_bounds__(4 * D + 64) void selfref_forward_kernel(SelfrefForw
 template <int D, bool SG, int N>
 bool launch_together(const SelfrefForward &a) {
     const int n = (2 + (1 + 4 / N) * a.batch) * kTellStride, followers = (1 + 4 / N) * a.batch;
+    const std::lock_guard<std::mutex> hold(counters_in_use);
     unsigned *counters = reinterpret_cast<unsigned *>(scratch_if_free(42, n * sizeof(unsigned)));
     if (!counters) return false;
     constexpr int most = scan_lds_floats<D>(true) > read_lds_floats<D>() ? scan_lds_floats<D>(true) : read_lds_floats<D>();

@@ -1396,6 +1396,7 @@ template <int D>
 bool launch_together(const SelfrefSweep &a) {
     const int cus = compute_units();
     BackwardCounters n{nullptr, a.batch, a.nc};
+    const std::lock_guard<std::mutex> hold(counters_in_use);
     n.drawn = reinterpret_cast<unsigned *>(scratch_if_free(43, n.floats() * sizeof(unsigned)));
     if (!n.drawn) return false;
     constexpr size_t sweep = sweep_lds_floats(D) * sizeof(float), lds = sweep > prepare_lds_bytes<D>() ? sweep : prepare_lds_bytes<D>();

@@ -2,11 +2,13 @@
 tiles: chunks one token short of, at and behind a tile's end, last chunks of one token, every head size, both value
 modes, against the float32 oracle; gradients against the float64 oracle (1e-4, fp32 sums over a chain)."""
 import ctypes
+import threading
 
 import numpy as np
 import pytest
 import torch
 
+from nl_hecate_amd import selfref as SR
 from nl_hecate_amd.ffi import lib
 from tests.gpu_util import assert_close
 from tests.test_gpu_exact_mm import kernels_run
@@ -150,3 +152,23 @@ def test_which_calls_run_in_one_launch(side_stream):
     a = inputs(n + 1, 13 * 32, 64, seed=2)
     ran = side_stream(lambda: kernels_run(lambda: gpu_run(*a, 32, True)))
     assert "selfref_chain_kernel" in ran and "selfref_backward_kernel" not in ran
+
+
+def test_two_host_threads_on_one_stream():
+    """Each call's counters are cleared and used without another thread's launch between them."""
+    calls = [[torch.from_numpy(a).cuda() for a in inputs(*size, seed=31)[:2]] for size in ((4, 300, 64), (8, 500, 32))]
+    got = [None, None]
+    forward = [lambda m=m, x=x: SR.chunkwise_self_ref_step(m.clone(), x, 64)[0] for m, x in calls]
+    want = [f() for f in forward]
+    torch.cuda.synchronize()
+
+    def repeat(i):
+        got[i] = [forward[i]() for _ in range(20)]
+
+    threads = [threading.Thread(target=repeat, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for w, runs in zip(want, got):
+        assert len(runs) == 20 and all(torch.equal(w, y) for y in runs)
