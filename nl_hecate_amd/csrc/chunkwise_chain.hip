@@ -212,8 +212,9 @@ __global__ __launch_bounds__(H *kChainThr) void cw_chain_fwd_kernel(
         else if (tid < 256) *reinterpret_cast<uint4 *>(dst + bf_at(vt, vcb)) = sv;
     };
     auto commit_tokens = [&](u16 *Q, u16 *Kt) {
-        if (has_k) { commit_rows(Kr, sk); commit_kt(Kt); }
-        if (has_q) commit_rows(Q, H == 1 ? sq : sk);
+        if (has_k) commit_rows(Kr, sk);
+        if (has_q) commit_rows(Q, H == 1 ? sq : sk);   // whole rows first: K^T leaves in single elements
+        if (has_k) commit_kt(Kt);
     };
     auto commit_vecs = [&]() {
         if (tid < 4 * CW + 4) cvec[tid] = vn;
