@@ -51,18 +51,24 @@ __device__ __forceinline__ int draw(unsigned *counter) {
 
 constexpr int kAloneFloats = 81 * 256;   // more than half of a compute unit's LDS
 
-// Held from where the counters' memory is taken to where their kernel is launched: with two host threads on one stream, the first
-// one's kernel is not to come between the second one's cleared counters and its kernel.
-inline std::mutex counters_in_use;
-
-// A kernel and not a memset: the launch may be recorded.
 __global__ static void clear_counters_kernel(unsigned *counters, int n) {
     const int i = blockIdx.x * 256 + threadIdx.x;
     if (i < n) counters[i] = 0;
 }
-inline void clear_counters(unsigned *counters, int n) {
-    hipLaunchKernelGGL(clear_counters_kernel, dim3(ceil_div(n, 256)), dim3(256), 0, stream(), counters, n);
-    check_launch("clear_counters_kernel");
-}
+
+// The counters of one launch, taken from a scratch slot and cleared; `at` is null where that is not free.  They are held until the
+// kernel is launched, and cleared on the stream on which it has to be launched, `on`: with other host threads beside this one,
+// nobody else's kernel comes between, and nlh_set_stream does not part the two.
+inline std::mutex counters_in_use;
+struct Counters {
+    const std::lock_guard<std::mutex> held{counters_in_use};
+    const hipStream_t on = stream();
+    unsigned *const at;
+    Counters(int slot, size_t n) : at(reinterpret_cast<unsigned *>(scratch_if_free(slot, n * sizeof(unsigned), on))) {
+        if (!at) return;
+        hipLaunchKernelGGL(clear_counters_kernel, dim3(ceil_div(n, 256)), dim3(256), 0, on, at, (int)n);
+        check_launch("clear_counters_kernel");
+    }
+};
 
 }  // namespace nlh

@@ -34,11 +34,11 @@ hipStream_t stream();   // launch stream (the null stream unless nlh_set_stream 
 // While the launch stream is being captured a slot cannot grow: the call fails instead.
 float *scratch(int slot, size_t bytes);
 constexpr int kScratchSlots = 44;
-// Scratch for an entry point that can do without (slots of its own): null, and nothing said, while the launch stream is
-// being captured (a graph would keep the address), on another stream than the slot's first caller (until
+// Scratch for an entry point that can do without (slots of its own), for launches on `on`: null, and nothing said, while
+// that stream is being captured (a graph would keep the address), on another stream than the slot's first caller's (until
 // nlh_release_workspace: two streams are not ordered against each other), or above kOptionalScratch bytes, which bounds
 // what stays allocated.
-float *scratch_if_free(int slot, size_t bytes);
+float *scratch_if_free(int slot, size_t bytes, hipStream_t on = stream());
 constexpr size_t kOptionalScratch = (size_t)256 << 20;
 
 // Optional per-kernel timing: while enabled (nlh_kernel_timer_enable), a

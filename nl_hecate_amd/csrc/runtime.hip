@@ -108,22 +108,22 @@ float *scratch(int slot, size_t bytes) {
     return (float *)s.ptr;
 }
 
-float *scratch_if_free(int slot, size_t bytes) {
+float *scratch_if_free(int slot, size_t bytes, hipStream_t on) {
     if (slot < 0 || slot >= kScratchSlots || bytes > kOptionalScratch) return nullptr;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(g_stream, &cap) != hipSuccess) {
+    if (hipStreamIsCapturing(on, &cap) != hipSuccess) {
         (void)hipGetLastError();   // a legacy stream while another one is being captured: not ours to use either
         return nullptr;
     }
     if (cap != hipStreamCaptureStatusNone) return nullptr;
     Slot &s = g_slots[slot];
-    if (s.owned && s.owner != g_stream) return nullptr;
+    if (s.owned && s.owner != on) return nullptr;
     int dev = 0;
     check_hip(hipGetDevice(&dev), "hipGetDevice");
     if (s.ptr && s.device != dev) return nullptr;
     if (s.bytes < bytes) {
         if (s.ptr) {   // no captured graph holds this address: the generation stays
-            check_hip(hipStreamSynchronize(g_stream), "scratch: hipStreamSynchronize");
+            check_hip(hipStreamSynchronize(on), "scratch: hipStreamSynchronize");
             check_hip(hipFree(s.ptr), "scratch: hipFree");
             s = Slot();
         }
@@ -136,7 +136,7 @@ float *scratch_if_free(int slot, size_t bytes) {
         s.device = dev;
     }
     s.owned = true;
-    s.owner = g_stream;
+    s.owner = on;
     return (float *)s.ptr;
 }
 

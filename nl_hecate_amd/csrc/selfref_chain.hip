@@ -778,18 +778,17 @@ __global__ __launch_bounds__(4 * D + 64) void selfref_forward_kernel(SelfrefForw
 template <int D, bool SG, int N>
 bool launch_together(const SelfrefForward &a) {
     const int n = (2 + (1 + 4 / N) * a.batch) * kTellStride, followers = (1 + 4 / N) * a.batch;
-    const std::lock_guard<std::mutex> hold(counters_in_use);
-    unsigned *counters = reinterpret_cast<unsigned *>(scratch_if_free(42, n * sizeof(unsigned)));
-    if (!counters) return false;
+    const Counters counters(42, n);
+    if (!counters.at) return false;
     constexpr int most = scan_lds_floats<D>(true) > read_lds_floats<D>() ? scan_lds_floats<D>(true) : read_lds_floats<D>();
     constexpr size_t lds = (most > kAloneFloats ? most : kAloneFloats) * sizeof(float);
     const long long tasks = (long long)a.batch * a.nc, rest = compute_units() - followers;
     const int readers = (int)(tasks < rest ? tasks : rest);
-    clear_counters(counters, n);
     check_hip(hipFuncSetAttribute(reinterpret_cast<const void *>(selfref_forward_kernel<D, SG, N>),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds), "dynamic LDS size");
     KernelTimer kt("selfref_forward_kernel");
-    hipLaunchKernelGGL((selfref_forward_kernel<D, SG, N>), dim3(followers + readers), dim3(4 * D + 64), lds, stream(), a, counters);
+    hipLaunchKernelGGL((selfref_forward_kernel<D, SG, N>), dim3(followers + readers), dim3(4 * D + 64), lds, counters.on, a,
+                       counters.at);
     check_launch("selfref_forward_kernel");
     return true;
 }

@@ -1345,7 +1345,7 @@ struct BackwardCounters {
     __host__ __device__ unsigned *shares(size_t b) const { return drawn + (3 + b) * kTellStride; }
     __host__ __device__ unsigned *swept(size_t b) const { return drawn + (3 + batch + b) * kTellStride; }
     __host__ __device__ unsigned *prepared(size_t b) const { return drawn + (3 + 2 * (size_t)batch) * kTellStride + b * nc; }
-    size_t floats() const { return (3 + 2 * (size_t)batch) * kTellStride + (size_t)batch * nc; }
+    size_t words() const { return (3 + 2 * (size_t)batch) * kTellStride + (size_t)batch * nc; }
 };
 // The sweeps leave most of the compute units idle, need one prepared chunk after the other, from the end, and their dg becomes d_x
 // chunk by chunk.  So one launch has workgroups that prepare chunks, in the order in which they are needed; for each chain one that
@@ -1396,19 +1396,19 @@ template <int D>
 bool launch_together(const SelfrefSweep &a) {
     const int cus = compute_units();
     BackwardCounters n{nullptr, a.batch, a.nc};
-    const std::lock_guard<std::mutex> hold(counters_in_use);
-    n.drawn = reinterpret_cast<unsigned *>(scratch_if_free(43, n.floats() * sizeof(unsigned)));
-    if (!n.drawn) return false;
+    const Counters counters(43, n.words());
+    if (!counters.at) return false;
+    n.drawn = counters.at;
     constexpr size_t sweep = sweep_lds_floats(D) * sizeof(float), lds = sweep > prepare_lds_bytes<D>() ? sweep : prepare_lds_bytes<D>();
     static_assert(lds >= kAloneFloats * sizeof(float) && lds >= passed_lds_floats<D>() * sizeof(float) &&
                   lds >= chunk_lds_floats<D>(2) * sizeof(float), "LDS");
     const long long tasks = (long long)a.batch * a.nc, rest = cus - 2 * a.batch;
     const int others = (int)(tasks < rest ? tasks : rest);
-    clear_counters(n.drawn, (int)n.floats());
     check_hip(hipFuncSetAttribute(reinterpret_cast<const void *>(selfref_backward_kernel<D>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds),
               "dynamic LDS size");
     KernelTimer kt("selfref_backward_kernel");
-    hipLaunchKernelGGL((selfref_backward_kernel<D>), dim3(2 * a.batch + 2 * others), dim3(8 * D), lds, stream(), a, n, others);
+    hipLaunchKernelGGL((selfref_backward_kernel<D>), dim3(2 * a.batch + 2 * others), dim3(8 * D), lds, counters.on, a, n,
+                       others);
     check_launch("selfref_backward_kernel");
     return true;
 }

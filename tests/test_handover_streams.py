@@ -1,0 +1,112 @@
+"""Which stream the self-referential kernels in one launch and the counters they share go to: the library's own entry points
+against a runtime that only writes down what it is asked for, so no GPU is needed."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+from nl_hecate_amd import ffi
+
+# A runtime in front of the real one: device memory is host memory that nobody reads, kernels are names.
+RUNTIME = r"""
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <map>
+#include <string>
+struct dim3 { unsigned x, y, z; };
+static std::map<const void *, std::string> names;
+static std::string said;
+static struct { dim3 grid, block; size_t lds; void *stream; } pushed;
+static const char *moment = nullptr;   // the next call of this name is followed by then(with)
+static void (*then)(void *) = nullptr;
+static void *with = nullptr;
+static void say(const char *what, const char *which, const void *stream) {
+    char line[1024];
+    snprintf(line, sizeof line, "%s %s %zu\n", what, which, (size_t)stream);
+    said += line;
+}
+static int answer(const char *call) {
+    if (moment && !strcmp(moment, call)) { moment = nullptr; then(with); }
+    return 0;
+}
+extern "C" {
+const char *what_was_said() { return said.c_str(); }
+void say_nothing() { said.clear(); }
+// As if another thread called f(stream) right behind the next call of that name.
+void behind_next(const char *call, void (*f)(void *), void *stream) { moment = strdup(call); then = f; with = stream; }
+
+void **__hipRegisterFatBinary(const void *) { static void *m; return &m; }
+void __hipUnregisterFatBinary(void **) {}
+void __hipRegisterFunction(void **, const void *f, char *, const char *name, unsigned, void *, void *, void *, void *, int *) { names[f] = name; }
+void __hipRegisterVar(void **, void *, char *, char *, int, size_t, int, int) {}
+int __hipPushCallConfiguration(dim3 g, dim3 b, size_t lds, void *s) { pushed = {g, b, lds, s}; return 0; }
+int __hipPopCallConfiguration(dim3 *g, dim3 *b, size_t *lds, void **s) { *g = pushed.grid; *b = pushed.block; *lds = pushed.lds; *s = pushed.stream; return 0; }
+int hipLaunchKernel(const void *f, dim3, dim3, void **, size_t, void *s) { say("launch", names[f].c_str(), s); return 0; }
+int hipGetDevice(int *d) { *d = 0; return 0; }
+int hipGetLastError() { return 0; }
+int hipFuncSetAttribute(const void *, int, int) { return answer("hipFuncSetAttribute"); }
+int hipMalloc(void **p, size_t n) { *p = malloc(n); say("alloc", "", nullptr); return 0; }
+int hipFree(void *p) { free(p); say("free", "", nullptr); return 0; }
+int hipStreamSynchronize(void *s) { say("synchronize", "", s); return 0; }
+int hipDeviceSynchronize() { say("synchronize", "device", nullptr); return 0; }
+int hipStreamIsCapturing(void *s, int *status) { *status = 0; say("query", "", s); return answer("hipStreamIsCapturing"); }
+}
+"""
+
+DRIVER = r"""
+import ctypes, sys
+fake = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+fake.what_was_said.restype = ctypes.c_char_p
+fake.behind_next.argtypes = [ctypes.c_char_p, ctypes.c_void_p, ctypes.c_void_p]
+from nl_hecate_amd.ffi import lib
+lib.load()
+some = 4096   # a device address that nobody reads
+forward = lambda B, s, C, d=64: lib.selfref_chunkwise_forward_f32_rocm(*[some] * 11, s, d, B, C, 1)
+backward = lambda B, s, C, d=64: lib.selfref_chunkwise_backward_f32_rocm(*[some] * 12, s, d, B, C, 1)
+ONE, OTHER = 0x1000, 0x2000
+on = lambda stream: lib.nlh_set_stream(ctypes.c_void_p(stream))
+switch_behind = lambda call, stream: fake.behind_next(call, ctypes.cast(lib.nlh_set_stream, ctypes.c_void_p), stream)
+def said():
+    out = [tuple(line.split(" ")) for line in fake.what_was_said().decode().splitlines()]
+    fake.say_nothing()
+    return [(what, which, int(stream)) for what, which, stream in out]
+def launches():
+    return [(which, stream) for what, which, stream in said() if what == "launch"]
+"""
+
+
+@pytest.fixture(scope="module")
+def on_host(tmp_path_factory):
+    at = tmp_path_factory.mktemp("runtime")
+    (at / "runtime.cpp").write_text(RUNTIME)
+    subprocess.check_call(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-o", str(at / "runtime.so"), str(at / "runtime.cpp")])
+    root = os.path.dirname(os.path.dirname(os.path.abspath(ffi.__file__)))
+
+    def run(body):
+        r = subprocess.run([sys.executable, "-c", DRIVER + body, str(at / "runtime.so")], cwd=root, capture_output=True, text=True,
+                           timeout=100)
+        assert r.returncode == 0, r.stdout + r.stderr
+
+    return run
+
+
+CALLS = [("forward", "2, 128, 64", "selfref_forward_kernel"), ("backward", "64, 1024, 64", "selfref_backward_kernel")]
+
+
+@pytest.mark.parametrize("moment", ["hipStreamIsCapturing", "hipFuncSetAttribute"])
+@pytest.mark.parametrize("call,sizes,kernel", CALLS)
+def test_counters_and_their_kernel_on_one_stream(on_host, call, sizes, kernel, moment):
+    """Another thread sets another stream while a call is under way."""
+    on_host(f"""
+on(ONE)
+{call}({sizes})       # what is allocated once
+said()
+switch_behind(b"{moment}", OTHER)
+{call}({sizes})
+ran = launches()
+clear = [s for name, s in ran if "clear_counters_kernel" in name]
+kernel = [s for name, s in ran if "{kernel}" in name]
+assert clear == kernel == [ONE], ran
+""")
