@@ -36,8 +36,8 @@ float *scratch(int slot, size_t bytes);
 constexpr int kScratchSlots = 44;
 // Scratch for an entry point that can do without (slots of its own), for launches on `on`: null, and nothing said, while
 // that stream is being captured (a graph would keep the address), on another stream than the slot's first caller's (until
-// nlh_release_workspace: two streams are not ordered against each other), or above kOptionalScratch bytes, which bounds
-// what stays allocated.
+// nlh_release_workspace: two streams are not ordered against each other), on hipStreamPerThread, which is another stream in
+// every thread, or above kOptionalScratch bytes, which bounds what stays allocated.
 float *scratch_if_free(int slot, size_t bytes, hipStream_t on = stream());
 constexpr size_t kOptionalScratch = (size_t)256 << 20;
 

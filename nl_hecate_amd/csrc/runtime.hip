@@ -110,6 +110,7 @@ float *scratch(int slot, size_t bytes) {
 
 float *scratch_if_free(int slot, size_t bytes, hipStream_t on) {
     if (slot < 0 || slot >= kScratchSlots || bytes > kOptionalScratch) return nullptr;
+    if (on == hipStreamPerThread) return nullptr;   // one handle, another stream in every thread
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(on, &cap) != hipSuccess) {
         (void)hipGetLastError();   // a legacy stream while another one is being captured: not ours to use either

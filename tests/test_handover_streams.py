@@ -110,3 +110,19 @@ clear = [s for name, s in ran if "clear_counters_kernel" in name]
 kernel = [s for name, s in ran if "{kernel}" in name]
 assert clear == kernel == [ONE], ran
 """)
+
+
+@pytest.mark.parametrize("call,sizes,kernel", CALLS)
+def test_one_handle_for_a_stream_in_every_thread(on_host, call, sizes, kernel):
+    """hipStreamPerThread: two threads' launches are not ordered, so they share no counters."""
+    on_host(f"""
+PER_THREAD = 2
+on(PER_THREAD)
+{call}({sizes})
+ran = launches()
+assert ran and not any("clear_counters_kernel" in name or "{kernel}" in name for name, _ in ran), ran
+assert {{stream for _, stream in ran}} == {{PER_THREAD}}
+on(ONE)      # which did not make it the owner
+{call}({sizes})
+assert any("{kernel}" in name for name, _ in launches())
+""")
