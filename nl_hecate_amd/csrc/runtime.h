@@ -39,6 +39,10 @@ constexpr int kScratchSlots = 44;
 // nlh_release_workspace: two streams are not ordered against each other), on hipStreamPerThread, which is another stream in
 // every thread, or above kOptionalScratch bytes, which bounds what stays allocated.
 float *scratch_if_free(int slot, size_t bytes, hipStream_t on = stream());
+// An event of the slot's own, or null, for a user who has to order the slot's launches by more than the handle of their
+// stream: a stream may be destroyed with work on it, and its handle come again for a stream that does not wait for that
+// work.  Recorded behind each launch and waited for in front of the next.
+hipEvent_t scratch_event(int slot);
 constexpr size_t kOptionalScratch = (size_t)256 << 20;
 
 // Optional per-kernel timing: while enabled (nlh_kernel_timer_enable), a

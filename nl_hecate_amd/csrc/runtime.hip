@@ -32,6 +32,7 @@ struct Slot {
     int device = -1;
     bool owned = false;            // scratch_if_free: by the stream that took it first
     hipStream_t owner = nullptr;
+    hipEvent_t used = nullptr;     // scratch_event
 };
 static Slot g_slots[kScratchSlots];
 
@@ -124,9 +125,13 @@ float *scratch_if_free(int slot, size_t bytes, hipStream_t on) {
     if (s.ptr && s.device != dev) return nullptr;
     if (s.bytes < bytes) {
         if (s.ptr) {   // no captured graph holds this address: the generation stays
-            check_hip(hipStreamSynchronize(on), "scratch: hipStreamSynchronize");
+            if (s.used)
+                check_hip(hipEventSynchronize(s.used), "scratch: hipEventSynchronize");
+            else
+                check_hip(hipStreamSynchronize(on), "scratch: hipStreamSynchronize");
             check_hip(hipFree(s.ptr), "scratch: hipFree");
-            s = Slot();
+            s.ptr = nullptr;
+            s.bytes = 0;
         }
         if (hipMalloc(&s.ptr, bytes) != hipSuccess) {
             (void)hipGetLastError();
@@ -139,6 +144,15 @@ float *scratch_if_free(int slot, size_t bytes, hipStream_t on) {
     s.owned = true;
     s.owner = on;
     return (float *)s.ptr;
+}
+
+hipEvent_t scratch_event(int slot) {
+    Slot &s = g_slots[slot];
+    if (!s.used && hipEventCreateWithFlags(&s.used, hipEventDisableTiming) != hipSuccess) {
+        (void)hipGetLastError();
+        s.used = nullptr;
+    }
+    return s.used;
 }
 
 KernelTimer::KernelTimer(const char *name) : slot(-1) {
@@ -182,6 +196,7 @@ void nlh_release_workspace(void) {
             (void)hipDeviceSynchronize();
             (void)hipFree(s.ptr);
         }
+        if (s.used) (void)hipEventDestroy(s.used);
         s = nlh::Slot();
     }
 }

@@ -154,6 +154,18 @@ def test_which_calls_run_in_one_launch(side_stream):
     assert "selfref_chain_kernel" in ran and "selfref_backward_kernel" not in ran
 
 
+def test_first_on_a_stream_of_the_callers(side_stream):
+    """The counters are then ordered by an event as well; the null stream comes second and takes the separate kernels."""
+    mems, x, dy = inputs(48, 720, 64, seed=8)
+    runs = [side_stream(lambda: gpu_run(mems, x, dy, 64, True)) for _ in range(3)]
+    ran = side_stream(lambda: kernels_run(lambda: gpu_run(mems, x, dy, 64, True)))
+    assert {"selfref_forward_kernel", "selfref_backward_kernel"} <= ran
+    apart = gpu_run(mems, x, dy, 64, True)
+    assert "selfref_chain_kernel" in kernels_run(lambda: gpu_run(mems, x, dy, 64, True))
+    for got in runs:
+        assert all(np.array_equal(got[n], apart[n]) for n in apart)
+
+
 def test_two_host_threads_on_one_stream():
     """Each call's counters are cleared and used without another thread's launch between them."""
     calls = [[torch.from_numpy(a).cuda() for a in inputs(*size, seed=31)[:2]] for size in ((4, 300, 64), (8, 500, 32))]

@@ -51,6 +51,11 @@ int hipMalloc(void **p, size_t n) { *p = malloc(n); say("alloc", "", nullptr); r
 int hipFree(void *p) { free(p); say("free", "", nullptr); return 0; }
 int hipStreamSynchronize(void *s) { say("synchronize", "", s); return 0; }
 int hipDeviceSynchronize() { say("synchronize", "device", nullptr); return 0; }
+int hipEventCreateWithFlags(void **e, unsigned) { static size_t n = 0; *e = (void *)(++n << 16); return 0; }
+int hipEventDestroy(void *) { return 0; }
+int hipEventSynchronize(void *) { say("synchronize", "event", nullptr); return 0; }
+int hipEventRecord(void *e, void *s) { say("record", std::to_string((size_t)e).c_str(), s); return 0; }
+int hipStreamWaitEvent(void *s, void *e, unsigned) { say("wait", std::to_string((size_t)e).c_str(), s); return 0; }
 int hipStreamIsCapturing(void *s, int *status) { *status = 0; say("query", "", s); return answer("hipStreamIsCapturing"); }
 }
 """
@@ -125,4 +130,37 @@ assert {{stream for _, stream in ran}} == {{PER_THREAD}}
 on(ONE)      # which did not make it the owner
 {call}({sizes})
 assert any("{kernel}" in name for name, _ in launches())
+""")
+
+
+@pytest.mark.parametrize("call,sizes,kernel", CALLS)
+def test_a_handle_that_comes_again(on_host, call, sizes, kernel):
+    """A stream destroyed with work on it, its handle given to another one: the counters are cleared behind the work."""
+    on_host(f"""
+on(ONE)
+{call}({sizes})
+for _ in range(3):
+    said()
+    {call}({sizes})
+    order = [(what, which) for what, which, stream in said() if stream == ONE and what != "query"]
+    what = [w for w, _ in order]
+    assert what == ["wait", "launch", "launch", "record"], order
+    assert order[0][1] == order[3][1] and "clear_counters_kernel" in order[1][1] and "{kernel}" in order[2][1], order
+lib.nlh_release_workspace()
+on(None)     # which cannot be destroyed
+{call}({sizes})
+said()
+{call}({sizes})
+assert [what for what, _, stream in said() if what in ("wait", "launch", "record")] == ["launch", "launch"]
+""")
+
+
+def test_counters_that_grow_wait_for_their_last_user(on_host):
+    on_host("""
+on(ONE)
+forward(2, 128, 64)
+said()
+forward(8, 128, 64)
+order = [(what, which) for what, which, _ in said() if what in ("synchronize", "free", "alloc")]
+assert order == [("synchronize", "event"), ("free", ""), ("alloc", "")], order
 """)
