@@ -793,21 +793,35 @@ bool launch_together(const SelfrefForward &a) {
     return true;
 }
 
+// Together where compute units stay idle beside the chains and those that follow them keep up with them: the other memories
+// take 10 us a chunk of any length, a chain 7 us for 16 tokens.  64 chains of 512 tokens, head size 64, apart / together:
+// chunks of 8 0.57 / 0.73 ms, of 16 0.38 / 0.41, of 32 0.327 / 0.308, of 64 0.299 / 0.279.  Behind a short sequence follow the reads of
+// its chunks on what the chains and their company leave of the chip, so the sequence has to be long enough; up to 8 chains every chunk
+// has a workgroup of its own.  Times as fast together, with self-generated values (without them at or above these), chains x tokens:
+//   head size 64, chunks of 32 / 64: 9 x 400 1.07 / 1.04, 33 x 400 0.99 / 1.01, 64 x 400 1.02 / 1.00, 64 x 2048 1.19 / 1.12;
+//     4 x 65 1.04 / 1.06, 8 x 65 0.99 / 1.02, 8 x 100 0.99 / 1.05
+//   32: 33 x 500 0.99 / 1.05, 64 x 500 0.98 / 1.01, 33 x 600 1.04 / 1.05, 64 x 600 1.04 / 1.03, 64 x 2048 1.13 / 1.11;
+//     4 x 65 0.97 / 1.04, 8 x 100 0.96 / 1.04, 8 x 200 1.01 / 1.04
+//   16: 32 x 500 1.02 / 1.01, 64 x 500 0.95 / 0.98, 33 x 600 1.03 / 1.02, 64 x 600 1.03 / 1.01, 64 x 2048 1.11 / 1.06;
+//     4 x 65 1.04 / 1.02, 8 x 65 1.03 / 1.01
+// On another stream than the null stream the counters' event adds 5 us: 4 x 100 0.96 / 1.01 there, 24 x 400 1.01 / 1.00, 64 x 600
+// 1.10 / 1.08 (head size 64).
+template <int D>
+bool together_pays(const SelfrefForward &a) {
+    if (a.nc < 2 || a.C < 2 * kTB || 4 * a.batch > compute_units()) return false;
+    if (a.s >= 600) return true;
+    if (stream()) return false;
+    if (a.batch > 8) return D == 64 && a.s >= 400;
+    return a.C >= 3 * kTB || a.s >= 200 || a.batch <= (D == 64 ? 4 : D == 32 ? 0 : 8);
+}
+
 template <int D, bool SG>
 void launch(const SelfrefForward &a) {
-    // Together where compute units stay idle beside the chains and those that follow them keep up with them: the other memories
-    // take 10 us a chunk of any length, a chain 7 us for 16 tokens.  64 chains of 512 tokens, head size 64, apart / together:
-    // chunks of 8 0.57 / 0.73 ms, of 16 0.38 / 0.41, of 32 0.327 / 0.308, of 64 0.299 / 0.279.  Behind a short sequence follow the reads of
-    // its chunks on what the chains and their company leave of the chip: 64 chains of 200 tokens 0.94 times as fast together, of 300
-    // 1.04, of 400 1.03, 48 of 300 in chunks of 32 0.97; up to 8 chains every chunk has a workgroup of its own (4 of 100 tokens 82 / 75 us).
-    // As many workgroups for a chain's other memories as leave most of the chip to the reads, which are the slower ones.
-    const int cus = compute_units();
-    if (a.nc > 1 && a.C >= 2 * kTB && 4 * a.batch <= cus && (a.s >= 400 || a.batch <= 8)) {
-        if (16 * a.batch <= cus   ? launch_together<D, SG, 1>(a)
-            : 8 * a.batch <= cus ? launch_together<D, SG, 2>(a)
-                                 : launch_together<D, SG, 4>(a))
-            return;
-    }
+    // One workgroup for a chain's other memories, as many as there are leave the more of the chip to the reads, or two where that is
+    // most of it anyway: head size 64, two / one: 16 chains of 2048 tokens 958 / 960 us, 32 of 500 in chunks of 32 289 / 297, 64 of
+    // 2048 1009 / 983; four, 16 of 2048 970.  At smaller head sizes one keeps up: 32, 16 of 2048 654 / 649 us; 16, 578 / 571.
+    const bool two = D == 64 && 8 * a.batch <= compute_units();
+    if (together_pays<D>(a) && (two ? launch_together<D, SG, D == 64 ? 2 : 4>(a) : launch_together<D, SG, 4>(a))) return;
     const dim3 block(4 * D);
     {
         KernelTimer kt("selfref_chain_kernel");

@@ -118,11 +118,12 @@ def side_stream():
     lib.nlh_release_workspace()
 
 
-# chains at the limits of the rules (a launch for all up to a quarter of the compute units, more workgroups a chain up to an
-# eighth and a sixteenth), chunks at the limit, last chunks of one token and of a partial tile, more chunks than readers; for the
+# chains at the limits of the rules (a launch for all up to a quarter of the compute units, two workgroups for a chain's other
+# memories up to an eighth), lengths at the limits, chunks at the limit, last chunks of one token and of a partial tile, more chunks than readers; for the
 # backward as many chunks as twice the compute units
 @pytest.mark.parametrize("B,s,C", [(1, 65, 64), (2, 33, 32), (8, 129, 33), (16, 400, 33), (17, 449, 64), (32, 1030, 64), (33, 513, 32),
-                                   (64, 449, 64), (64, 610, 32), (52, 400, 40), (65, 449, 64), (3, 1000, 64), (2, 64, 16)])
+                                   (64, 449, 64), (64, 610, 32), (52, 400, 40), (65, 449, 64), (3, 1000, 64), (2, 64, 16),
+                                   (16, 600, 33), (32, 601, 64), (33, 640, 32), (64, 705, 64)])
 @pytest.mark.parametrize("d", [16, 32, 64])
 @pytest.mark.parametrize("sg", [True, False])
 def test_in_one_launch_and_one_after_the_other(side_stream, B, s, C, d, sg):
@@ -139,12 +140,16 @@ def test_in_one_launch_and_one_after_the_other(side_stream, B, s, C, d, sg):
 
 def test_which_calls_run_in_one_launch(side_stream):
     cus = torch.cuda.get_device_properties(0).multi_processor_count
-    for B, s, C, one in ((2, 65, 64, True), (8, 65, 64, True), (9, 65, 64, False),
-                        (cus // 4, 400, 64, True), (cus // 4 + 1, 400, 64, False), (2, 65, 32, True),
-                         (2, 65, 31, False), (2, 64, 64, False)):
-        a = inputs(B, s, 16, seed=1)
+    for B, s, d, C, one in ((2, 65, 16, 64, True), (8, 65, 16, 64, True), (9, 65, 16, 64, False),
+                            (cus // 4, 400, 64, 64, True), (cus // 4 + 1, 400, 64, 64, False), (2, 65, 16, 32, True),
+                            (2, 65, 16, 31, False), (2, 64, 16, 64, False),
+                            # short sequences at the smaller head sizes
+                            (9, 599, 16, 64, False), (9, 600, 16, 64, True), (9, 599, 32, 64, False), (cus // 4, 600, 32, 32, True),
+                            (9, 399, 64, 64, False), (8, 65, 32, 64, True), (1, 199, 32, 32, False), (1, 200, 32, 32, True),
+                            (4, 65, 64, 32, True), (5, 199, 64, 32, False), (5, 65, 64, 48, True), (8, 199, 16, 32, True)):
+        a = inputs(B, s, d, seed=1)
         ran = kernels_run(lambda: gpu_run(*a, C, True))
-        assert ("selfref_forward_kernel" in ran) == one and ("selfref_chain_kernel" in ran) != one, (B, s, C)
+        assert ("selfref_forward_kernel" in ran) == one and ("selfref_chain_kernel" in ran) != one, (B, s, d, C)
     n = 2 * cus // 13
     for B, s, d, C, one in ((n + 1, 13 * 32, 64, 32, True), (n - 1, 13 * 32, 64, 32, False), (n + 1, 13 * 32, 32, 32, False)):
         a = inputs(B, s, d, seed=2)

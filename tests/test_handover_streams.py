@@ -97,7 +97,7 @@ def on_host(tmp_path_factory):
     return run
 
 
-CALLS = [("forward", "2, 128, 64", "selfref_forward_kernel"), ("backward", "64, 1024, 64", "selfref_backward_kernel")]
+CALLS = [("forward", "2, 640, 64", "selfref_forward_kernel"), ("backward", "64, 1024, 64", "selfref_backward_kernel")]
 
 
 @pytest.mark.parametrize("moment", ["hipStreamIsCapturing", "hipFuncSetAttribute"])
@@ -158,9 +158,9 @@ assert [what for what, _, stream in said() if what in ("wait", "launch", "record
 def test_counters_that_grow_wait_for_their_last_user(on_host):
     on_host("""
 on(ONE)
-forward(2, 128, 64)
+forward(2, 640, 64)
 said()
-forward(8, 128, 64)
+forward(8, 640, 64)
 order = [(what, which) for what, which, _ in said() if what in ("synchronize", "free", "alloc")]
 assert order == [("synchronize", "event"), ("free", ""), ("alloc", "")], order
 """)
