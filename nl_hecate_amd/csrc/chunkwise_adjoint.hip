@@ -13,7 +13,7 @@
 // adjoint of the state at the start of chunk c (slot num_chunks = 0), rounded as the gradient pass
 // would round it; slot 0, the gradient of the initial state, leaves in fp32 (dm_first).
 //
-// Where the halves of all chains are more than the compute units, one workgroup of sixteen waves has all rows of a chain (H = 2): K, Q
+// Where that takes the fewer rounds (chunkwise_chain.h), one workgroup of sixteen waves has all rows of a chain (H = 2): K, Q
 // and the coefficients are fetched, and W.P formed, once, and four waves on a SIMD hide each other's
 // latencies.  256 chains of 4096 tokens: 282 -> 243 us.
 //
@@ -290,7 +290,7 @@ bool chunkwise_adjoint_bf16(const uint16_t *k, const uint16_t *q, const float *d
     const int nc = ceil_div(seq_len, chunk_size);
     const HeadRows dyr = dy_rows ? *dy_rows : head_major_rows(seq_len, HD);
     if (es.failed()) return true;
-    const bool whole = chain_in_one_workgroup(batch);
+    const bool whole = adjoint_in_one_workgroup(batch, nc);
     auto launch = has_s ? (whole ? launch_adjoint<true, 2> : launch_adjoint<true, 1>)
                         : (whole ? launch_adjoint<false, 2> : launch_adjoint<false, 1>);
     launch(k, q, d_y, tab_b, vecs, dm_snap, has_s ? ds_snap : nullptr, dm_first, has_s ? ds_first : nullptr, seq_len, chunk_size, nc, batch,

@@ -12,9 +12,17 @@ namespace nlh {
 
 // Both halves of a chain in one workgroup: where the halves of all chains do not fit the chip at once.  Up to there a half a compute
 // unit is faster (one compute unit takes 5 us for a chunk of both, 3 us for a half).  Forward and backward, us, halves / whole: 128
-// chains of 4096 tokens 680 in halves; 136 960 / 840, 192 1164 / 1030, 256 1345 / 1233; 256 of 1000 375 / 346; 300 of 2048 933 / 907;
-// without momentum 256 of 4096 1168 / 1052.
+// chains of 4096 tokens 680 in halves; 136 960 / 840, 192 1164 / 1030, 256 1345 / 1233; 129 of 64 55 / 50; without momentum 256 of 4096
+// 1168 / 1052.  Forward kernel, 2048 tokens: 256 chains 211 / 157, 257 285 / 259, 320 287 / 265, 384 303 / 277, 385 386 / 271, 640 499 / 412.
 inline bool chain_in_one_workgroup(int batch) { return 2 * batch > compute_units(); }
+// The adjoint scan alike, unless the chip takes the halves in three rounds and the chains in two, 257 to 384 of them here: 2048 tokens
+// 257 chains 212 / 220 us, 320 205 / 225, 384 220 / 230, and 1000 in chunks of 32 188 / 206, 192 / 208, 195 / 210.  Four rounds against
+// two, 385 chains, 293 / 226, and five against three, 513 and 640, 380 / 334 and 359 / 349.  A short sequence is mostly the start and the
+// end of a workgroup: 64 tokens 18.5 / 17.3, 18.9 / 18.3, 20.3 / 17.9.
+inline bool adjoint_in_one_workgroup(int batch, int num_chunks) {
+    const int cus = compute_units(), halves = ceil_div(2LL * batch, cus), whole = ceil_div(batch, cus);
+    return chain_in_one_workgroup(batch) && (num_chunks < 8 || 5 * halves >= 8 * whole);
+}
 
 // What a test of the reference's couplings needs from the forward (chunkwise_guard.hip), left behind by the chain
 // kernel as it goes: e2 [batch, 2 halves, num_chunks * 64] = the sum over the half's 32 memory rows of the squared

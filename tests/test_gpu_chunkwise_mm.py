@@ -357,7 +357,8 @@ def _in_parts(rule, n, s, C, step, seed):
 # chains whose halves are more than the compute units, by one and by many; a chunk of one token at the end, chunks below a tile,
 # one chunk alone
 @pytest.mark.parametrize("rule", ["titans", "delta"])
-@pytest.mark.parametrize("more,s,C", [(1, 193, 64), (9, 100, 64), (1, 64, 64), (72, 70, 17), (3, 33, 32), (130, 50, 64), (1, 5, 1)])
+@pytest.mark.parametrize("more,s,C", [(1, 193, 64), (9, 100, 64), (1, 64, 64), (72, 70, 17), (3, 33, 32), (130, 50, 64), (1, 5, 1),
+                                      (132, 513, 64), (131, 100, 10)])   # the last two: the adjoint scan in halves
 def test_chains_in_one_workgroup_and_in_two(rule, more, s, C):
     cus = torch.cuda.get_device_properties(0).multi_processor_count
     n = cus // 2 + more
