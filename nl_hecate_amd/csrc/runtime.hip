@@ -109,6 +109,14 @@ float *scratch(int slot, size_t bytes) {
     return (float *)s.ptr;
 }
 
+// While it lives, this thread's calls do not disturb a capture of another stream: in the mode that a capture has by default an
+// allocation, a free or a synchronisation anywhere in the process ends it, as if it had been asked for in the capture.
+struct BesideCaptures {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    BesideCaptures() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+    ~BesideCaptures() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
 float *scratch_if_free(int slot, size_t bytes, hipStream_t on) {
     if (slot < 0 || slot >= kScratchSlots || bytes > kOptionalScratch) return nullptr;
     if (on == hipStreamPerThread) return nullptr;   // one handle, another stream in every thread
@@ -124,6 +132,7 @@ float *scratch_if_free(int slot, size_t bytes, hipStream_t on) {
     check_hip(hipGetDevice(&dev), "hipGetDevice");
     if (s.ptr && s.device != dev) return nullptr;
     if (s.bytes < bytes) {
+        const BesideCaptures relaxed;
         if (s.ptr) {   // no captured graph holds this address: the generation stays
             if (s.used)
                 check_hip(hipEventSynchronize(s.used), "scratch: hipEventSynchronize");

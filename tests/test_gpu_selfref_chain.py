@@ -171,6 +171,30 @@ def test_first_on_a_stream_of_the_callers(side_stream):
         assert all(np.array_equal(got[n], apart[n]) for n in apart)
 
 
+def test_first_call_beside_a_capture_of_another_stream():
+    """The counters are allocated while somebody else records a graph: neither notices."""
+    mems, x, _ = inputs(4, 640, 64, seed=9)
+    mine, other = torch.cuda.Stream(), torch.cuda.Stream()
+    m, x = (torch.from_numpy(a).cuda() for a in (mems, x))
+    want = SR.chunkwise_self_ref_step(m.clone(), x, 64, True)[0]
+    first = m.clone()
+    y = [torch.zeros(*sh, device="cuda") for sh in [(4, 640, 64)] * 4 + [(4, 640)] * 4 + [(4, 10, 6, 64, 64)]]
+    number = torch.zeros(1, device="cuda")
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    lib.nlh_release_workspace()
+    with torch.cuda.graph(graph, stream=other):
+        number += 1
+        lib.nlh_set_stream(ctypes.c_void_p(mine.cuda_stream))
+        lib.selfref_chunkwise_forward_f32_rocm(*[t.data_ptr() for t in (first, x, *y)], 640, 64, 4, 64, 1)
+        lib.nlh_set_stream(None)
+    lib.nlh_release_workspace()
+    for _ in range(3):
+        graph.replay()
+    torch.cuda.synchronize()
+    assert float(number) == 3 and torch.equal(y[0], want)
+
+
 def test_two_host_threads_on_one_stream():
     """Each call's counters are cleared and used without another thread's launch between them."""
     calls = [[torch.from_numpy(a).cuda() for a in inputs(*size, seed=31)[:2]] for size in ((4, 300, 64), (8, 500, 32))]

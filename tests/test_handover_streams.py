@@ -15,6 +15,7 @@ RUNTIME = r"""
 #include <cstring>
 #include <map>
 #include <string>
+#include <utility>
 struct dim3 { unsigned x, y, z; };
 static std::map<const void *, std::string> names;
 static std::string said;
@@ -47,6 +48,12 @@ int hipLaunchKernel(const void *f, dim3, dim3, void **, size_t, void *s) { say("
 int hipGetDevice(int *d) { *d = 0; return 0; }
 int hipGetLastError() { return 0; }
 int hipFuncSetAttribute(const void *, int, int) { return answer("hipFuncSetAttribute"); }
+int hipThreadExchangeStreamCaptureMode(int *mode) {   // 0 global, 2 relaxed
+    static int now = 0;
+    std::swap(now, *mode);
+    say("mode", now == 2 ? "relaxed" : "global", nullptr);
+    return 0;
+}
 int hipMalloc(void **p, size_t n) { *p = malloc(n); say("alloc", "", nullptr); return 0; }
 int hipFree(void *p) { free(p); say("free", "", nullptr); return 0; }
 int hipStreamSynchronize(void *s) { say("synchronize", "", s); return 0; }
@@ -163,4 +170,18 @@ said()
 forward(8, 640, 64)
 order = [(what, which) for what, which, _ in said() if what in ("synchronize", "free", "alloc")]
 assert order == [("synchronize", "event"), ("free", ""), ("alloc", "")], order
+""")
+
+
+def test_optional_scratch_is_allocated_beside_captures(on_host):
+    """A capture of another stream ends with an allocation, a free or a wait in the mode that it has by default."""
+    on_host("""
+on(ONE)
+inside = False
+for size in ((2, 640, 64), (8, 640, 64)):
+    forward(*size)
+    for what, which, _ in said():
+        inside = which == "relaxed" if what == "mode" else inside
+        assert inside or what not in ("alloc", "free", "synchronize"), what
+assert not inside
 """)
