@@ -172,7 +172,10 @@ def test_combine_gate_with_bf16_attention_matches_the_fp32_kernels():
     _close("d_y", dy2, dy1, 1e-6)
 
 
-@pytest.mark.parametrize("levels,bs,nh,s,C,per_level", [(3, 2, 4, 150, 64, False), (2, 1, 8, 70, 16, True)])
+# the last three: both halves of a chain in one workgroup (more chains than half the compute units; that form against fewer
+# chains: test_gpu_chunkwise_mm.py), the very last with its adjoint scan in halves
+@pytest.mark.parametrize("levels,bs,nh,s,C,per_level", [(3, 2, 4, 150, 64, False), (2, 1, 8, 70, 16, True), (3, 6, 8, 193, 64, False),
+                                                        (5, 4, 8, 70, 16, True), (4, 9, 8, 513, 64, False)])
 def test_chunkwise_rule_on_token_major_rows_equals_the_head_major_entry_points(levels, bs, nh, s, C, per_level):
     """titans_chunkwise_{forward,backward}_bf16_tokens_rocm write y / read d_y in [levels, bs, s, nh*64] (d_y
     optionally shared by the levels); same kernels, other addresses: bit-equal to the head-major pair."""

@@ -11,6 +11,7 @@ import numpy as np
 import pytest
 import torch
 
+from nl_hecate_amd import dispatch as D
 from nl_hecate_amd.ffi import lib
 from oracle import memory_level as OL
 from oracle import pyoracle as orc
@@ -218,6 +219,38 @@ def test_levels_forward_and_backward_through_the_c_abi(bs, s, nh, levels, chunk)
     worst["d_m_initial"] = rel_err(host(dm), dm_ref)
     print({k: f"{v:.1e}" for k, v in worst.items()}, flush=True)
     assert max(worst.values()) <= 2e-2, worst
+
+
+@pytest.mark.parametrize("bs,s,nh,levels,chunk", [(5, 193, 8, 4, 64), (9, 50, 8, 4, 17), (3, 130, 8, 6, 64)])
+def test_levels_forward_of_many_chains_carries_the_states(bs, s, nh, levels, chunk):
+    """More chains than half the compute units (and than all of them): y at token-major rows, the snapshots and the carried
+    memories, which are read and written in place, are the bits of the head-major entry point on eight chains at a time."""
+    hd, B, n_extra = 64, bs * nh, 1
+    x, w_extra, w_levels, gates = make_inputs(bs, s, nh, levels, n_extra, seed=s)
+    st = Step(bs, s, nh, levels, n_extra, chunk)
+    tx, twe, twl = dev(x), dev(w_extra), dev(w_levels)
+    tg = [[dev(g[nm]) for nm in GATE_NAMES] for g in gates]
+    g = torch.Generator(device="cuda").manual_seed(s)
+    m_ctx, s_ctx = (0.05 * torch.randn(levels * B, hd * hd, generator=g, device="cuda") for _ in range(2))
+    for turn in range(2):
+        m0, s0 = m_ctx.clone(), s_ctx.clone()
+        lib.titans_levels_forward_bf16_rocm(
+            tx.data_ptr(), twe.data_ptr(), n_extra, ptr_array(st.extra), twl.data_ptr(), ptr_array([t for g in tg for t in g]),
+            m_ctx.data_ptr(), s_ctx.data_ptr(), st.xb.data_ptr(), st.kh.data_ptr(), st.vh.data_ptr(), st.qh.data_ptr(),
+            st.ah.data_ptr(), st.th.data_ptr(), st.eh.data_ptr(), st.k_norms.data_ptr(), st.q_norms.data_ptr(),
+            st.alpha.data_ptr(), st.theta.data_ptr(), st.eta.data_ptr(), st.mc.data_ptr(), st.sc.data_ptr(), st.y.data_ptr(),
+            bs, s, nh, hd, levels, chunk, 1e-8)
+        slots = st.mc.shape[1]
+        for a in range(0, levels * B, 8):
+            cut = [t[a:a + 8] for t in (st.kh, st.vh, st.qh, st.ah, st.th, st.eh, m0, s0)]
+            mc, sc = (torch.zeros(8, slots, hd * hd, device="cuda") for _ in range(2))
+            y = torch.zeros(8, s, hd, device="cuda")
+            D.call("titans_chunkwise_forward_bf16_rocm", *cut, mc, sc, y, s, hd, 8, chunk)
+            lv, b = a // B, a % B // nh          # eight heads of one batch element
+            assert torch.equal(st.y[lv, b], y.permute(1, 0, 2).reshape(s, nh * hd)), (turn, a)
+            assert torch.equal(st.mc[a:a + 8], mc) and torch.equal(st.sc[a:a + 8], sc), (turn, a)
+            assert torch.equal(m_ctx[a:a + 8], mc[:, -1]) and torch.equal(s_ctx[a:a + 8], sc[:, -1]), (turn, a)
+        assert not torch.equal(m_ctx, m0)
 
 
 def test_linear_pair_and_combine_gate():
