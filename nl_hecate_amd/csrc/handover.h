@@ -6,8 +6,6 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
-#include <mutex>
-
 #include "runtime.h"
 
 namespace nlh {
@@ -57,11 +55,10 @@ __global__ static void clear_counters_kernel(unsigned *counters, int n) {
 }
 
 // The counters of one launch, taken from a scratch slot and cleared; `at` is null where that is not free.  They are held until the
-// kernel is launched, and cleared on the stream on which it has to be launched, `on`: with other host threads beside this one,
+// kernel is launched (they alone: other scratch of a call is for one host thread at a time), and cleared on the stream on which it has to be launched, `on`: with other host threads beside this one,
 // nobody else's kernel comes between, and nlh_set_stream does not part the two.  They are cleared behind their last user's
 // kernel, since a workgroup that waits for a count that is taken away never ends: on the null stream, which cannot be destroyed, by the
 // stream's order, on another by an event as well (scratch_event; 5 us between calls back to back).
-inline std::mutex counters_in_use;
 struct Counters {
     const std::lock_guard<std::mutex> held{counters_in_use};
     const hipStream_t on = stream();

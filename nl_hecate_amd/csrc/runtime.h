@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stddef.h>
 
+#include <mutex>
+
 namespace nlh {
 
 // Error policy.  Mode 0 (default) is the reference contract for void entry
@@ -43,6 +45,9 @@ float *scratch_if_free(int slot, size_t bytes, hipStream_t on = stream());
 // stream: a stream may be destroyed with work on it, and its handle come again for a stream that does not wait for that
 // work.  Recorded behind each launch and waited for in front of the next.
 hipEvent_t scratch_event(int slot);
+// Held by a call from where it takes counters (handover.h) to where it has launched their kernel, and by
+// nlh_release_workspace: with several host threads, the counters stay as long as somebody is about to use them.
+inline std::mutex counters_in_use;
 constexpr size_t kOptionalScratch = (size_t)256 << 20;
 
 // Optional per-kernel timing: while enabled (nlh_kernel_timer_enable), a

@@ -199,6 +199,7 @@ void nlh_set_stream(void *hip_stream) { nlh::g_stream = (hipStream_t)hip_stream;
 unsigned long long nlh_workspace_generation(void) { return nlh::g_arena_generation; }
 
 void nlh_release_workspace(void) {
+    const std::lock_guard<std::mutex> hold(nlh::counters_in_use);
     nlh::g_arena_generation++;
     for (auto &s : nlh::g_slots) {
         if (s.ptr) {

@@ -10,11 +10,13 @@ from nl_hecate_amd import ffi
 
 # A runtime in front of the real one: device memory is host memory that nobody reads, kernels are names.
 RUNTIME = r"""
+#include <chrono>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
 #include <map>
 #include <string>
+#include <thread>
 #include <utility>
 struct dim3 { unsigned x, y, z; };
 static std::map<const void *, std::string> names;
@@ -28,14 +30,19 @@ static void say(const char *what, const char *which, const void *stream) {
     snprintf(line, sizeof line, "%s %s %zu\n", what, which, (size_t)stream);
     said += line;
 }
+static std::thread other;
 static int answer(const char *call) {
-    if (moment && !strcmp(moment, call)) { moment = nullptr; then(with); }
+    if (!moment || strcmp(moment, call)) return 0;
+    moment = nullptr;
+    other = std::thread(then, with);
+    std::this_thread::sleep_for(std::chrono::milliseconds(200));   // it is done by then, or waits for this thread
     return 0;
 }
 extern "C" {
 const char *what_was_said() { return said.c_str(); }
 void say_nothing() { said.clear(); }
-// As if another thread called f(stream) right behind the next call of that name.
+// Another thread calls f(stream) right behind the next call of that name; join_other() waits for its end.
+void join_other() { if (other.joinable()) other.join(); }
 void behind_next(const char *call, void (*f)(void *), void *stream) { moment = strdup(call); then = f; with = stream; }
 
 void **__hipRegisterFatBinary(const void *) { static void *m; return &m; }
@@ -81,6 +88,7 @@ ONE, OTHER = 0x1000, 0x2000
 on = lambda stream: lib.nlh_set_stream(ctypes.c_void_p(stream))
 switch_behind = lambda call, stream: fake.behind_next(call, ctypes.cast(lib.nlh_set_stream, ctypes.c_void_p), stream)
 def said():
+    fake.join_other()
     out = [tuple(line.split(" ")) for line in fake.what_was_said().decode().splitlines()]
     fake.say_nothing()
     return [(what, which, int(stream)) for what, which, stream in out]
@@ -93,7 +101,7 @@ def launches():
 def on_host(tmp_path_factory):
     at = tmp_path_factory.mktemp("runtime")
     (at / "runtime.cpp").write_text(RUNTIME)
-    subprocess.check_call(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-o", str(at / "runtime.so"), str(at / "runtime.cpp")])
+    subprocess.check_call(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-pthread", "-o", str(at / "runtime.so"), str(at / "runtime.cpp")])
     root = os.path.dirname(os.path.dirname(os.path.abspath(ffi.__file__)))
 
     def run(body):
@@ -184,4 +192,19 @@ for size in ((2, 640, 64), (8, 640, 64)):
         inside = which == "relaxed" if what == "mode" else inside
         assert inside or what not in ("alloc", "free", "synchronize"), what
 assert not inside
+""")
+
+
+@pytest.mark.parametrize("call,sizes,kernel", CALLS)
+def test_a_release_waits_for_the_launch(on_host, call, sizes, kernel):
+    """nlh_release_workspace from another thread while a call has its counters and has not launched their kernel."""
+    on_host(f"""
+on(ONE)
+{call}({sizes})
+said()
+fake.behind_next(b"hipFuncSetAttribute", ctypes.cast(lib.nlh_release_workspace, ctypes.c_void_p), None)
+{call}({sizes})
+order = [which if what == "launch" else what for what, which, _ in said() if what in ("launch", "free")]
+assert "free" in order and [o for o in order if "{kernel}" in o], order
+assert max(i for i, o in enumerate(order) if "{kernel}" in o) < order.index("free"), order
 """)
