@@ -54,7 +54,7 @@ __global__ static void clear_counters_kernel(unsigned *counters, int n) {
     if (i < n) counters[i] = 0;
 }
 
-// The counters of one launch, taken from a scratch slot and cleared; `at` is null where that is not free.  They are held until the
+// The counters of one launch, taken from a scratch slot and cleared; `at` is null where that is not free, or an error was raised.  They are held until the
 // kernel is launched (they alone: other scratch of a call is for one host thread at a time), and cleared on the stream on which it has to be launched, `on`: with other host threads beside this one,
 // nobody else's kernel comes between, and nlh_set_stream does not part the two.  They are cleared behind their last user's
 // kernel, since a workgroup that waits for a count that is taken away never ends: on the null stream, which cannot be destroyed, by the
@@ -67,13 +67,15 @@ struct Counters {
     Counters(int slot, size_t n) : at(reinterpret_cast<unsigned *>(scratch_if_free(slot, n * sizeof(unsigned), on))) {
         if (at && on && !(used = scratch_event(slot))) at = nullptr;
         if (!at) return;
+        const ErrorScope es;
         if (used) check_hip(hipStreamWaitEvent(on, used, 0), "counters: hipStreamWaitEvent");
         hipLaunchKernelGGL(clear_counters_kernel, dim3(ceil_div(n, 256)), dim3(256), 0, on, at, (int)n);
         check_launch("clear_counters_kernel");
+        if (es.failed()) at = nullptr;
     }
     Counters(const Counters &) = delete;
     ~Counters() {
-        if (used) check_hip(hipEventRecord(used, on), "counters: hipEventRecord");
+        if (used && at) check_hip(hipEventRecord(used, on), "counters: hipEventRecord");
     }
 };
 

@@ -31,7 +31,9 @@ static void say(const char *what, const char *which, const void *stream) {
     said += line;
 }
 static std::thread other;
+static const char *failing = nullptr;   // the next call of this name fails
 static int answer(const char *call) {
+    if (failing && !strcmp(failing, call)) { failing = nullptr; return 1; }
     if (!moment || strcmp(moment, call)) return 0;
     moment = nullptr;
     other = std::thread(then, with);
@@ -42,6 +44,7 @@ extern "C" {
 const char *what_was_said() { return said.c_str(); }
 void say_nothing() { said.clear(); }
 // Another thread calls f(stream) right behind the next call of that name; join_other() waits for its end.
+void fail_next(const char *call) { failing = strdup(call); }
 void join_other() { if (other.joinable()) other.join(); }
 void behind_next(const char *call, void (*f)(void *), void *stream) { moment = strdup(call); then = f; with = stream; }
 
@@ -53,7 +56,8 @@ int __hipPushCallConfiguration(dim3 g, dim3 b, size_t lds, void *s) { pushed = {
 int __hipPopCallConfiguration(dim3 *g, dim3 *b, size_t *lds, void **s) { *g = pushed.grid; *b = pushed.block; *lds = pushed.lds; *s = pushed.stream; return 0; }
 int hipLaunchKernel(const void *f, dim3, dim3, void **, size_t, void *s) { say("launch", names[f].c_str(), s); return 0; }
 int hipGetDevice(int *d) { *d = 0; return 0; }
-int hipGetLastError() { return 0; }
+int hipGetLastError() { return answer("hipGetLastError"); }
+const char *hipGetErrorString(int) { return "failed on purpose"; }
 int hipFuncSetAttribute(const void *, int, int) { return answer("hipFuncSetAttribute"); }
 int hipThreadExchangeStreamCaptureMode(int *mode) {   // 0 global, 2 relaxed
     static int now = 0;
@@ -69,7 +73,7 @@ int hipEventCreateWithFlags(void **e, unsigned) { static size_t n = 0; *e = (voi
 int hipEventDestroy(void *) { return 0; }
 int hipEventSynchronize(void *) { say("synchronize", "event", nullptr); return 0; }
 int hipEventRecord(void *e, void *s) { say("record", std::to_string((size_t)e).c_str(), s); return 0; }
-int hipStreamWaitEvent(void *s, void *e, unsigned) { say("wait", std::to_string((size_t)e).c_str(), s); return 0; }
+int hipStreamWaitEvent(void *s, void *e, unsigned) { say("wait", std::to_string((size_t)e).c_str(), s); return answer("hipStreamWaitEvent"); }
 int hipStreamIsCapturing(void *s, int *status) { *status = 0; say("query", "", s); return answer("hipStreamIsCapturing"); }
 }
 """
@@ -207,4 +211,22 @@ fake.behind_next(b"hipFuncSetAttribute", ctypes.cast(lib.nlh_release_workspace, 
 order = [which if what == "launch" else what for what, which, _ in said() if what in ("launch", "free")]
 assert "free" in order and [o for o in order if "{kernel}" in o], order
 assert max(i for i, o in enumerate(order) if "{kernel}" in o) < order.index("free"), order
+""")
+
+
+@pytest.mark.parametrize("step", ["hipStreamWaitEvent", "hipGetLastError"])   # behind the launch that clears them
+@pytest.mark.parametrize("call,sizes,kernel", CALLS)
+def test_no_kernel_on_counters_that_were_not_cleared(on_host, call, sizes, kernel, step):
+    on_host(f"""
+lib.nlh_set_error_mode(1)
+on(ONE)
+{call}({sizes})
+said()
+fake.fail_next(b"{step}")
+{call}({sizes})
+assert b"failed on purpose" in ctypes.string_at(lib.nlh_last_error())
+assert not any("{kernel}" in name for name, _ in launches())
+lib.nlh_clear_error()
+{call}({sizes})
+assert any("{kernel}" in name for name, _ in launches()) and ctypes.string_at(lib.nlh_last_error()) == b""
 """)
