@@ -213,3 +213,33 @@ def test_two_host_threads_on_one_stream():
         t.join()
     for w, runs in zip(want, got):
         assert len(runs) == 20 and all(torch.equal(w, y) for y in runs)
+
+
+def test_two_host_threads_forward_and_backward():
+    """As above with kernels of two forms, and the backward, whose other scratch has its size before the threads start."""
+    sizes = ((64, 705, 64), (16, 640, 32)), ((48, 720, 64), (64, 640, 64))
+    for step, pair in zip((0, 1), sizes):
+        calls = []
+        for B, s, C in pair:
+            mems, x, dy = (torch.from_numpy(a).cuda() for a in inputs(B, s, 64, seed=s))
+            if step == 0:
+                calls.append(lambda m=mems, x=x, C=C: SR.chunkwise_self_ref_step(m.clone(), x, C, True)[0])
+            else:
+                cache = SR.chunkwise_self_ref_step(mems, x, C, True)[1]
+                calls.append(lambda c=cache, dy=dy: torch.cat([t.flatten() for t in SR.chunkwise_self_ref_step_backward(c, dy)]))
+        want = [f() for f in calls]
+        assert all(f"selfref_{('forward', 'backward')[step]}_kernel" in kernels_run(f) for f in calls)
+        torch.cuda.synchronize()
+        got = [None, None]
+
+        def repeat(i):
+            got[i] = [calls[i]() for _ in range(15)]
+
+        threads = [threading.Thread(target=repeat, args=(i,)) for i in range(2)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        torch.cuda.synchronize()
+        for w, runs in zip(want, got):
+            assert len(runs) == 15 and all(torch.equal(w, y) for y in runs)
