@@ -78,8 +78,8 @@ int nlh_selftest_chunk_coef_prepass(const float *alpha, const float *theta, cons
  * error_clip <= 0 and m_norm_max <= 0 or >= 1e30 disable clip / projection.
  * The forwards of the exact rule, and of the frozen rule at head size 32, need no scratch memory.  At head sizes 32 and 64
  * they take up to 256 MiB of it for few long chains, where it is free to take: not while the launch stream is being
- * captured, and on the first stream that took it only (until nlh_release_workspace); otherwise they walk the tokens.  So do
- * the *_final_states_f32_rocm. */
+ * captured, not on hipStreamPerThread, and on the first stream that took it only (until nlh_release_workspace; that stream
+ * must not be destroyed with such calls under way); otherwise they walk the tokens.  So do the *_final_states_f32_rocm. */
 /* core/src/cuda_ffi.rs:134 */
 void titans_forward_f32_cuda(const float *k_mem, const float *v_mem, const float *q_mem,
                              const float *alpha, const float *theta, const float *eta,
@@ -536,7 +536,12 @@ void memory_read_only_backward_f32_rocm(const float *d_y, const float *m, float 
  *   y, k/v/q_cache [batch, seq_len, d];  alpha/theta/alpha_mean/eta_mean_cache [batch, seq_len]
  *   frozen    [batch, num_chunks, 6, d*d], num_chunks = ceil(seq_len / chunk_size)
  * d = 16, 32, 64 run on the tiled kernels; every other d from 1 to 512 on general ones (the reference's own
- * tests use d = 4, core/src/chunkwise_self_ref.rs:662); larger d is an error. */
+ * tests use d = 4, core/src/chunkwise_self_ref.rs:662); larger d is an error.
+ * Chunks of 32 to 64 tokens, few chains and long sequences: each direction is one launch whose workgroups hand chunks over
+ * through counters.  The forward takes 17 KiB of scratch for them and no other; both run as separate launches, with the same
+ * results, where the counters are not free to take: while the launch stream is being captured, on hipStreamPerThread, and on
+ * any stream but the first that took them.  So a process whose first such call is the warm-up of a capture on a side stream
+ * has the separate launches on its other streams until nlh_release_workspace. */
 void selfref_chunkwise_forward_f32_rocm(float *mems, const float *embedded, float *y, float *k_cache,
                                         float *v_cache, float *q_cache, float *alpha_cache,
                                         float *theta_cache, float *alpha_mean_cache, float *eta_mean_cache,

@@ -40,7 +40,7 @@
 // rounded once: 0.6 to 1.0e-7, each output at or below its walk over spread gates, gates at a model's start and long-lived
 // states.  Left in fp32 are the products that do not show: the inverse, K K^T, K M^T, the maps
 // of the adjoint scan and the products with the adjoint at the chunk's end.  512 tokens of 32 chains, head size 64: first
-// kernel 38 -> 46 us, gradients 38 -> 48, scan 16 -> 23, gates 10 -> 15; head size 32, 777 tokens of 16: 21 -> 25, 24 -> 32,
+// kernel 38 -> 46 us, gradients 38 -> 49, scan 16 -> 23, gates 10 -> 15; head size 32, 777 tokens of 16: 21 -> 25, 24 -> 32,
 // 5 -> 8, 7 -> 9.  Head size 64 with checkpoints every 32 tokens and more keeps fp32 sums: there the form is the path that
 // there was, and its two kernels are bound by their products.
 //
@@ -490,7 +490,8 @@ __global__ __launch_bounds__(kThr) void ex_grads_kernel(
     asm volatile("" : "+s"(w));
     NLH_STRIP_ORIGIN_OF(w);
     // Float64 sums at head size 64: the scheduler, left alone, reads the operands of several products ahead and spills 119 registers
-    // (256 chunks 64 us with the spills, 48 without); the other forms have room for that.
+    // a lane, one with the barrier (256 chunks 64 -> 49 us).  At head size 32, where it spills two, the barrier leaves none and no
+    // time either (208 chunks 33.5 / 33.7 us between events); the other forms spill none.
     auto MMA = [&](Strip &acc, auto fa, auto fb) {
         product<P64>(acc, fa, fb, l);
         if (P64 && D == 64) __builtin_amdgcn_sched_barrier(0);
@@ -824,10 +825,13 @@ static int chunk_of(int C) { return C * (CW / C); }
 static bool wide_sums(int d, int C) { return d == 32 || C < 32; }
 
 // Cost models from measurements on one MI355X (us).  A chunk costs the two chunk-parallel kernels of the backward about
-// 65 us of a compute unit whatever its length (95 with float64 sums, 54 at head size 32), a scan step 2.0 (2.9, 0.65); the
+// 65 us of a compute unit whatever its length (95 with float64 sums, 46 + 49; the pass takes 92 more a round of chunks over
+// 2 to 16 rounds, intervals of 8; 54 at head size 32), a scan step 2.0 (2.9, 0.65); the
 // fused sequential kernel walks a chain's tokens at 0.6 each on a quarter of a compute unit's worth of workgroups (four per
 // chain, one at head size 32), the kernel that reads a whole trajectory at 1.1.  Under a clip or a bound the test on the
-// errors adds two launches to the matrix form where the fused kernel's only adds one on its maxima.
+// errors adds two launches to the matrix form where the fused kernel's only adds one on its maxima.  Matrix form / walk on
+// both sides of the line, intervals of 8: 128 chains of 64 tokens 110 / 97, 160 115 / 137; 64 of 128 105 / 89, of 200 120 / 132;
+// 192 of 96 202 / 194, 256 216 / 254.
 bool exact_backward_mm_pays(int seq_len, int batch, int d, int C, bool tested, bool frozen) {
     const int nc = ceil_div(seq_len, frozen ? C : chunk_of(C)), cus = compute_units();
     const bool wide = wide_sums(d, C);

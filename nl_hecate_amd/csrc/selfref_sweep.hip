@@ -1354,7 +1354,8 @@ struct BackwardCounters {
 // 64 chains of 2048 tokens, head size 64, chunks of 64: 1.49 ms for 0.29 + 0.06 + 0.03 + 1.29 + 0.06 of five launches.  The
 // preparation ends at 0.69 ms, a sweep starts at 0.05 and is slower than alone by 5 % (its neighbours' code and traffic), the last
 // d_x is 8 us behind the last sweep.  With the chunks dealt out beforehand the last d_x was 170 us behind: some workgroups of the last
-// kind find no place before the sweeps end.
+// kind find no place before the sweeps end.  Of 256 registers a lane six values are spilled (20 bytes of scratch; the sweep by itself
+// spills four).
 template <int D>
 __global__ __launch_bounds__(8 * D) void selfref_backward_kernel(SelfrefSweep a, BackwardCounters n, int preparers) {
     static_assert(8 * D == kPrepThr, "the same workgroup for all");
